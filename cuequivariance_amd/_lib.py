@@ -70,11 +70,14 @@ EXPORTED_SYMBOLS = (
     "cueq_layer_norm_fwd",
     "cueq_layer_norm_bwd_workspace",
     "cueq_layer_norm_bwd",
-    "cueq_gate_fwd",
-    "cueq_gate_bwd",
     "cueq_sum_cols",
     "cueq_sum_rows_workspace",
     "cueq_sum_rows",
+    "cueq_trimul_grads_values",
+    "cueq_trimul_saved_bytes",
+    "cueq_trimul_workspace_bytes",
+    "cueq_trimul_fwd",
+    "cueq_trimul_bwd",
 )
 
 
@@ -262,16 +265,22 @@ def load() -> C.CDLL:
         lib.cueq_layer_norm_bwd_workspace.restype = i64
         lib.cueq_layer_norm_bwd.argtypes = [i32, i64, i64, ptr, ptr, ptr, ptr, ptr, ptr, ptr, ptr, ptr, i64, ptr]
         lib.cueq_layer_norm_bwd.restype = C.c_int
-        lib.cueq_gate_fwd.argtypes = [i32, i64, i64, ptr, ptr, ptr, ptr, i32, ptr, i32, ptr, ptr]
-        lib.cueq_gate_fwd.restype = C.c_int
-        lib.cueq_gate_bwd.argtypes = [i32, i64, i64, ptr, ptr, ptr, ptr, ptr, i32, ptr, i32, ptr, ptr, ptr]
-        lib.cueq_gate_bwd.restype = C.c_int
         lib.cueq_sum_cols.argtypes = [i32, i64, i64, ptr, ptr, ptr]
         lib.cueq_sum_cols.restype = C.c_int
         lib.cueq_sum_rows_workspace.argtypes = [i64, i64]
         lib.cueq_sum_rows_workspace.restype = i64
         lib.cueq_sum_rows.argtypes = [i32, i64, i64, ptr, ptr, ptr, i64, ptr]
         lib.cueq_sum_rows.restype = C.c_int
+        lib.cueq_trimul_grads_values.argtypes = [i64, i64]
+        lib.cueq_trimul_grads_values.restype = i64
+        lib.cueq_trimul_saved_bytes.argtypes = [i32, i64, i64, i64, i64]
+        lib.cueq_trimul_saved_bytes.restype = i64
+        lib.cueq_trimul_workspace_bytes.argtypes = [i32, i64, i64, i64, i64, i32, i32]
+        lib.cueq_trimul_workspace_bytes.restype = i64
+        lib.cueq_trimul_fwd.argtypes = [i32, i64, i64, i64, i64, i32, C.c_double, ptr, ptr, ptr, ptr, ptr, ptr, i64, ptr]
+        lib.cueq_trimul_fwd.restype = C.c_int
+        lib.cueq_trimul_bwd.argtypes = [i32, i64, i64, i64, i64, i32, ptr, ptr, ptr, ptr, ptr, ptr, C.c_uint32, ptr, ptr, i64, ptr]
+        lib.cueq_trimul_bwd.restype = C.c_int
         # the library has read the environment itself at this point: remember what it saw, so that the first launch does
         # not push those values again over an option set by cueq_set_option in the meantime
         for env, _ in _ENV_OPTIONS:

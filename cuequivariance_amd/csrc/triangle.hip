@@ -1,11 +1,11 @@
 // Kernels of the triangle multiplicative update (AlphaFold-style pair update):
 //   LayerNorm over the hidden dimension, sigmoid-gated dual projection, the triangular contraction
 //   t[d,b,i,j] = sum_k a[d,b,i,k] b[d,b,j,k], LayerNorm across d with a layout change, output gate.
-// The stages are separate launches composed by the host (cuequivariance_amd/cuet/triangle.py):
+// The stages are separate launches:
 //   cueq_gemm_nt        batched C = alpha * A * B^T (+ C), both operands contraction-contiguous, MFMA
 //   cueq_transpose      batched 2-D transpose through LDS
 //   cueq_layer_norm_*   row LayerNorm forward / backward (one wavefront per row)
-//   cueq_gate_*         out = sigmoid(u + bu) * (v + bv) * mask and its backward
+//   cueq_trimul_*       all of them in order, forward and backward
 //   cueq_sum_rows/cols  reductions for the bias / affine gradients
 // Math is fp32 throughout; tensors are fp32 or bf16.
 //
@@ -108,6 +108,30 @@ __device__ __forceinline__ float ln_affine(float centered, float rs, float gm, f
   return __fadd_rn(__fmul_rn(__fmul_rn(centered, rs), gm), bt);
 }
 
+// Pair rows of a padded square.  The contraction moves its n x n matrices in 16-byte pieces, so an extent n that is no multiple
+// of such a piece is rounded up to np inside the update: what lives between the stages has B np^2 rows, what the caller holds
+// (x, mask, the update, the two gradients of the pair tensor) B n^2.  src(m) is the caller's row of padded row m, -1 for padding.
+// The division is a multiplication by floor(2^(31 + s) / np) + 1, exact for m < 2^31.
+struct PairRows {
+  int n = 0, np = 0;
+  uint32_t magic = 0;
+  int shift = 0;
+  __host__ static PairRows make(int n, int np) {
+    PairRows p;
+    p.n = n; p.np = np;
+    while ((1ll << p.shift) < np) ++p.shift;
+    p.magic = static_cast<uint32_t>((1ull << (31 + p.shift)) / static_cast<uint64_t>(np) + 1);
+    return p;
+  }
+  __device__ __forceinline__ int over(int m) const {
+    return static_cast<int>((static_cast<uint64_t>(static_cast<uint32_t>(m)) * magic) >> 31 >> shift);
+  }
+  __device__ __forceinline__ int src(int m) const {
+    const int q = over(m), k = m - q * np, b = over(q), i = q - b * np;
+    return (k < n && i < n) ? (b * n + i) * n + k : -1;
+  }
+};
+
 template <typename TO>
 __device__ __forceinline__ void stage_put(char* tile, int row_stride, int col, int h, const floatx16& acc, float alpha) {
   using F = TO;
@@ -145,10 +169,11 @@ __device__ __forceinline__ uint4 add_vec(uint4 a, uint4 b) {
 // nthreads threads (index t) move `rows` staged rows of NCOLS elements to C (row stride ldc elements)
 template <typename TO, int NCOLS>
 __device__ __forceinline__ void stage_flush(const char* tile, int row_stride, int rows, TO* __restrict__ C, int64_t ldc, int t, int nthreads,
-                                            bool accumulate) {
+                                            bool accumulate, int cols = NCOLS) {
   constexpr int EPV = 16 / sizeof(TO), VPR = NCOLS / EPV;
   for (int idx = t; idx < rows * VPR; idx += nthreads) {
     const int r = idx / VPR, cv = idx % VPR;
+    if (cv * EPV >= cols) continue;
     uint4 val = *reinterpret_cast<const uint4*>(tile + r * row_stride + cv * 16);
     uint4* g = reinterpret_cast<uint4*>(C + static_cast<int64_t>(r) * ldc + cv * EPV);
     if (accumulate) val = add_vec<TO>(val, *g);
@@ -352,7 +377,7 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_kernel(const TI* __restrict
     __syncthreads();  // every wavefront is done with the operand tiles, which become staging space
     // (parts addressed through a table: every part checks the alignment of its own result block)
     const bool vec_rows = gmode == 3 ? (reinterpret_cast<uintptr_t>(C) % 16 == 0 && (ldc * sizeof(TO)) % 16 == 0) : vec_out != 0;
-    if (vec_rows && m0 + wm * 64 + 64 <= M && n0 + wn * 64 + 64 <= N) {
+    if (vec_rows && N % 8 == 0) {  // (edge tiles too: whole vectors of the rows and columns that exist)
       constexpr int RS = 64 * sizeof(TO) + 16;
       static_assert(WM * WN * 32 * RS <= 2 * (ABYTES + BBYTES), "staging tiles must fit the operand buffers");
       char* tile = &smem[0][0] + wave * (32 * RS);
@@ -361,7 +386,8 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_kernel(const TI* __restrict
         stage_put<TO>(tile, RS, c, h, acc[i][0], alpha);
         stage_put<TO>(tile, RS, 32 + c, h, acc[i][1], alpha);
         __builtin_amdgcn_wave_barrier();
-        stage_flush<TO, 64>(tile, RS, 32, C + static_cast<int64_t>(m0 + wm * 64 + i * 32) * ldc + n0 + wn * 64, ldc, lane, 64, accumulate != 0);
+        stage_flush<TO, 64>(tile, RS, min(32, M - (m0 + wm * 64 + i * 32)), C + static_cast<int64_t>(m0 + wm * 64 + i * 32) * ldc + n0 + wn * 64, ldc, lane,
+                            64, accumulate != 0, N - (n0 + wn * 64));
         __builtin_amdgcn_wave_barrier();
       }
       return;
@@ -986,8 +1012,11 @@ __global__ void __launch_bounds__((gbi_threads<TI, SPLIT>()), (gbi_waves_per_sim
 // LNB (one-input form): X1 holds the rows of a LayerNorm whose input rows, mean and 1 / std are given, and the kernel
 // goes on to the gradient with respect to those input rows - the lane has half of the gradient row in registers, so the two
 // row sums of the LayerNorm backward are sums over its own values completed by one exchange - and writes that to dX1.
+//
+// PAD: the rows are those of a padded square (PairRows).  X and the gradients stay padded; dC by columns (the cotangent of
+// the update), the mask, the LayerNorm's input rows and, with LNB, the result `dres` are the caller's rows.
 // ------------------------------------------------------------------------------------------------
-template <typename F, int KT, bool SPLIT, bool DC_BY_ROW, bool LNB = false>
+template <typename F, int KT, bool SPLIT, bool DC_BY_ROW, bool LNB = false, bool PAD = false>
 __global__ void __launch_bounds__((SPLIT ? 256 : 512), (SPLIT ? 1 : 2))
     gate_bwd_input_res_kernel(const F* __restrict__ W1, const F* __restrict__ W2, int64_t ldw, const F* __restrict__ X1,
                               const F* __restrict__ X2, int64_t ldx, const F* __restrict__ bias1,
@@ -995,7 +1024,7 @@ __global__ void __launch_bounds__((SPLIT ? 256 : 512), (SPLIT ? 1 : 2))
                               int64_t ldc, F* __restrict__ dX1, F* __restrict__ dX2, int64_t lddx, int accumulate,
                               F* __restrict__ dU, F* __restrict__ dV, int C, int M, const F* __restrict__ ln_x = nullptr,
                               int64_t ldlx = 0, const float* __restrict__ ln_mean = nullptr, const float* __restrict__ ln_rstd = nullptr,
-                              const F* __restrict__ ln_gamma = nullptr) {
+                              const F* __restrict__ ln_gamma = nullptr, F* __restrict__ dres = nullptr, PairRows pairs = PairRows()) {
   static_assert(!(LNB && SPLIT), "the LayerNorm backward goes with the one-input form");
   using TI = F;
   constexpr int ES = 2, EPV = 8;
@@ -1045,6 +1074,7 @@ __global__ void __launch_bounds__((SPLIT ? 256 : 512), (SPLIT ? 1 : 2))
   // The loads run a chunk ahead of their use, across tile boundaries: (ptile, pci) is the next chunk to request.
   uint32_t dcr[8], dcn[8];
   auto dc_lane_offset = [&](int mld) -> uint32_t {
+    if constexpr (PAD && !DC_BY_ROW) mld = max(pairs.src(mld), 0);
     return DC_BY_ROW ? static_cast<uint32_t>(((4 * h + (lane & 1)) * ldc + (mld & ~1)) * ES) : static_cast<uint32_t>((mld * ldc + 4 * h) * ES);
   };
   int64_t ptile = static_cast<int64_t>(blockIdx.x) * NWAVES + wave;
@@ -1091,7 +1121,7 @@ __global__ void __launch_bounds__((SPLIT ? 256 : 512), (SPLIT ? 1 : 2))
         xf1[s2][q] = *reinterpret_cast<const uint4*>(X1 + o);
         if constexpr (SPLIT) xf2[s2][q] = *reinterpret_cast<const uint4*>(X2 + o);
       }
-    if (mask) mraw = raw16(mask[mld]);
+    if (mask) mraw = raw16(mask[PAD ? max(pairs.src(mld), 0) : mld]);  // (padding: its cotangent is zero)
   };
   int64_t tile = ptile;
   if (tile < ntiles) request_x(tile_row(tile));
@@ -1101,6 +1131,7 @@ __global__ void __launch_bounds__((SPLIT ? 256 : 512), (SPLIT ? 1 : 2))
     const int mrow0 = static_cast<int>(tile * 32);
     const int mcol = mrow0 + c;
     const float mk = mask ? lo16<F>(mraw) : 1.0f;
+    const uint32_t real = (PAD && !DC_BY_ROW && pairs.src(min(mcol, M - 1)) < 0) ? 0u : ~0u;  // (padding has no cotangent)
     floatx16 ax1[KT], ax2[SPLIT ? KT : 1];
 #pragma unroll
     for (int t = 0; t < KT; ++t) ax1[t] = floatx16{0};
@@ -1115,7 +1146,7 @@ __global__ void __launch_bounds__((SPLIT ? 256 : 512), (SPLIT ? 1 : 2))
           const uint32_t other = static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(dcn[v]), 0xB1, 0xF, 0xF, true));
           dcr[v] = __builtin_amdgcn_perm(other, dcn[v], pair_sel);
         } else {
-          dcr[v] = dcn[v];
+          dcr[v] = PAD ? (dcn[v] & real) : dcn[v];
         }
       }
       request_dc(dcn);
@@ -1261,7 +1292,8 @@ __global__ void __launch_bounds__((SPLIT ? 256 : 512), (SPLIT ? 1 : 2))
         // The float accumulators are swapped into row order (k = 16 j + 8 h + e per 32 columns), what is added to them
         // and the LayerNorm's input rows arrive in the same order.
         uint4 xr[KT][2];
-        const int64_t xrow = static_cast<int64_t>(min(mrow, M - 1)) * ldlx + (h * 16) / ES;
+        const int xsrc = PAD ? pairs.src(min(mrow, M - 1)) : min(mrow, M - 1);
+        const int64_t xrow = static_cast<int64_t>(max(xsrc, 0)) * ldlx + (h * 16) / ES;
 #pragma unroll
         for (int ds = 0; ds < KT; ++ds)
 #pragma unroll
@@ -1329,7 +1361,16 @@ __global__ void __launch_bounds__((SPLIT ? 256 : 512), (SPLIT ? 1 : 2))
       }
       }
       __builtin_amdgcn_sched_barrier(0);
-      if (mrow < M) {
+      if constexpr (LNB) {
+        const int dst = mrow < M ? (PAD ? pairs.src(mrow) : mrow) : -1;
+        if (dst >= 0) {
+          F* to = dres + static_cast<int64_t>(dst) * lddx + (h * 16) / ES;
+#pragma unroll
+          for (int ds = 0; ds < KT; ++ds)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) *reinterpret_cast<uint4*>(to + (ds * 64 + j * 32) / ES) = val[ds][j];
+        }
+      } else if (mrow < M) {
 #pragma unroll
         for (int ds = 0; ds < KT; ++ds)
 #pragma unroll
@@ -1353,14 +1394,18 @@ __global__ void __launch_bounds__((SPLIT ? 256 : 512), (SPLIT ? 1 : 2))
 // 32 further), so the statistics are sums over the lane's own values completed by one exchange; the rows are
 // normalised in the registers, rounded to the 2-byte type - the operand of the products, exactly what a separate
 // LayerNorm launch would have written - and stored with their mean and 1 / std for the later stages.
+//
+// PAD: the rows are those of a padded square (PairRows).  LN: X and the mask are the caller's rows, padding counts as a row of
+// zeros with mask 0.  ROWS: X and X2 are padded, the result goes to the caller's rows.
 // ------------------------------------------------------------------------------------------------
-template <typename F, int KT, bool LN, bool ROWS>
+template <typename F, int KT, bool LN, bool ROWS, bool PAD = false>
 __global__ void __launch_bounds__(512, 2)
     dual_gate_res_kernel(const F* __restrict__ W1, const F* __restrict__ W2, int64_t ldw, const F* __restrict__ X,
                          const F* __restrict__ X2, int64_t ldx, const F* __restrict__ bias1, const F* __restrict__ bias2, const F* __restrict__ mask,
                          F* __restrict__ out, int64_t ldc, int C, int M, const F* __restrict__ gamma,
                          const F* __restrict__ beta, float eps, F* __restrict__ xhat, int64_t ldxh, float* __restrict__ mean,
-                         float* __restrict__ rstd) {
+                         float* __restrict__ rstd, PairRows pairs = PairRows()) {
+  static_assert(!PAD || LN || ROWS, "padded rows go with the two stages of the triangle update");
   using TI = F;
   constexpr int ES = 2, EPV = 8;
   constexpr int K = 32 * KT, ROWB = K * ES, NS = ROWB / 64, VPR = ROWB / 16;
@@ -1405,10 +1450,16 @@ __global__ void __launch_bounds__(512, 2)
   // wavefront's next tile are requested while the current one is worked on
   uint4 xn[NT][NS][2], xn2[1][NS][2];
   uint32_t mraw[NT] = {};
+  bool pad_n[NT] = {};
   auto request_x = [&](int64_t tl) {
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      const int mld = static_cast<int>(min(tl * (32 * NT) + 32 * t + c, static_cast<int64_t>(M) - 1));
+      int mld = static_cast<int>(min(tl * (32 * NT) + 32 * t + c, static_cast<int64_t>(M) - 1));
+      if constexpr (PAD && LN) {
+        mld = pairs.src(mld);
+        pad_n[t] = mld < 0;
+        mld = max(mld, 0);
+      }
 #pragma unroll
       for (int s2 = 0; s2 < NS; ++s2)
 #pragma unroll
@@ -1436,9 +1487,15 @@ __global__ void __launch_bounds__(512, 2)
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
           xf[t][s2][q] = xn[t][s2][q];
+          if constexpr (PAD && LN) {
+            if (pad_n[t]) xf[t][s2][q] = make_uint4(0, 0, 0, 0);
+          }
           if constexpr (ROWS) xf2[t][s2][q] = xn2[t][s2][q];
         }
       mk[t] = mask ? lo16<F>(mraw[t]) : 1.0f;
+      if constexpr (PAD && LN) {
+        if (pad_n[t]) mk[t] = 0.0f;
+      }
     }
     request_x(min(tile + tstep, ntiles - 1));  // (past the end: the last tile again, so that the request is unconditional)
     if constexpr (LN) {
@@ -1535,6 +1592,7 @@ __global__ void __launch_bounds__(512, 2)
         // result by rows (M x C): the lane holds its own row m and, of this chunk, c = 8 (v >> 2) + 4 h + (v & 3); the lane
         // halves swap register pairs (v_permlane32_swap), after which each stores 16 contiguous bytes of its row
         uint32_t pk[8];
+        const int mdst = PAD ? (mcol[0] < M ? pairs.src(mcol[0]) : -1) : (mcol[0] < M ? mcol[0] : -1);
 #pragma unroll
         for (int a = 0; a < 4; ++a) {
           float g[4];
@@ -1550,8 +1608,8 @@ __global__ void __launch_bounds__(512, 2)
         for (int j = 0; j < 2; ++j) {
           const auto s0 = __builtin_amdgcn_permlane32_swap(pk[4 * j], pk[4 * j + 2], false, false);
           const auto s1 = __builtin_amdgcn_permlane32_swap(pk[4 * j + 1], pk[4 * j + 3], false, false);
-          if (mcol[0] < M)
-            *reinterpret_cast<uint4*>(out + static_cast<int64_t>(mcol[0]) * ldc + c0 + 16 * j + 8 * h) = make_uint4(s0[0], s1[0], s0[1], s1[1]);
+          if (mdst >= 0)
+            *reinterpret_cast<uint4*>(out + static_cast<int64_t>(mdst) * ldc + c0 + 16 * j + 8 * h) = make_uint4(s0[0], s1[0], s0[1], s1[1]);
         }
       } else {
 #pragma unroll
@@ -1815,10 +1873,11 @@ __global__ void __launch_bounds__(256) ln_fwd_rows8(const T* __restrict__ x, con
   }
 }
 
+// (pairs.np != 0: dy, mean and rstd are rows of a padded square, x and dx the caller's rows)
 template <typename T, int L>
 __global__ void __launch_bounds__(256) ln_bwd_rows8(const T* __restrict__ dy, const T* __restrict__ x, const float* __restrict__ mean,
                                                     const float* __restrict__ rstd, const T* __restrict__ gamma, T* __restrict__ dx,
-                                                    float* __restrict__ part, int64_t rows, int rows_per_block) {
+                                                    float* __restrict__ part, int64_t rows, int rows_per_block, PairRows pairs) {
   using F = T;
   constexpr int D = 8 * L, RPW = 64 / L;
   extern __shared__ float sred[];  // [4 waves][2][D]
@@ -1831,11 +1890,12 @@ __global__ void __launch_bounds__(256) ln_bwd_rows8(const T* __restrict__ dy, co
   const int64_t r_end = min(r_begin + rows_per_block, rows);
   for (int64_t r0 = r_begin + wave * RPW; r0 < r_end; r0 += 4 * RPW) {
     const int64_t row = r0 + sub;
-    const bool ok = row < r_end;
+    const int64_t xrow = row < r_end ? (pairs.np ? pairs.src(static_cast<int>(row)) : row) : -1;
+    const bool ok = xrow >= 0;
     float xh[8], g[8];
     float mu = 0.f, rs = 0.f;
     if (ok) {
-      tn_load8(x + row * D + col, xh);
+      tn_load8(x + xrow * D + col, xh);
       tn_load8(dy + row * D + col, g);
       mu = mean[row];
       rs = rstd[row];
@@ -1857,7 +1917,7 @@ __global__ void __launch_bounds__(256) ln_bwd_rows8(const T* __restrict__ dy, co
     s2 = group_sum<L>(s2) * (1.0f / D);
 #pragma unroll
     for (int e = 0; e < 8; ++e) g[e] = rs * (g[e] - s1 - xh[e] * s2);
-    if (ok) ln_store8(dx + row * D + col, g);
+    if (ok) ln_store8(dx + xrow * D + col, g);
   }
   // rows of one wavefront -> one lane group, then the four wavefronts through LDS
 #pragma unroll
@@ -2342,47 +2402,6 @@ __global__ void __launch_bounds__(256, 2) ln_t_bwd_cols_kernel(const F* __restri
   }
 }
 
-// ------------------------------------------------------------------------------------------------
-// gate: out[r][c] = sigmoid(u + bu) * (v + bv) * mask;  biases and mask are indexed by row (axis 0) or column (axis 1)
-// ------------------------------------------------------------------------------------------------
-template <typename T>
-__global__ void __launch_bounds__(256) gate_fwd_kernel(const float* __restrict__ u, const float* __restrict__ v, const T* __restrict__ bu,
-                                                       const T* __restrict__ bv, int bias_axis, const T* __restrict__ mask, int mask_axis,
-                                                       T* __restrict__ out, int64_t R, int64_t Ccols) {
-  const int64_t tid = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (tid >= R * Ccols) return;
-  const int64_t r = tid / Ccols, cc = tid - r * Ccols;
-  const int64_t ib = bias_axis == 0 ? r : cc;
-  const float uu = u[tid] + (bu ? tri_load(bu, ib) : 0.f);
-  const float vv = v[tid] + (bv ? tri_load(bv, ib) : 0.f);
-  float o = vv / (1.0f + __expf(-uu));
-  if (mask) o *= tri_load(mask, mask_axis == 0 ? r : cc);
-  tri_store(out, tid, o);
-}
-
-// du = dout * mask * (v + bv) * s * (1 - s),  dv = dout * mask * s,  s = sigmoid(u + bu)
-template <typename T>
-__global__ void __launch_bounds__(256) gate_bwd_kernel(const T* __restrict__ dout, const float* __restrict__ u, const float* __restrict__ v,
-                                                       const T* __restrict__ bu, const T* __restrict__ bv, int bias_axis,
-                                                       const T* __restrict__ mask, int mask_axis, T* __restrict__ du, T* __restrict__ dv,
-                                                       int64_t R, int64_t Ccols) {
-  const int64_t tid = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (tid >= R * Ccols) return;
-  const int64_t r = tid / Ccols, cc = tid - r * Ccols;
-  const int64_t ib = bias_axis == 0 ? r : cc;
-  const float uu = u[tid] + (bu ? tri_load(bu, ib) : 0.f);
-  const float vv = v[tid] + (bv ? tri_load(bv, ib) : 0.f);
-  const float s = 1.0f / (1.0f + __expf(-uu));
-  float d = tri_load(dout, tid);
-  if (mask) d *= tri_load(mask, mask_axis == 0 ? r : cc);
-  tri_store(du, tid, d * vv * s * (1.0f - s));
-  tri_store(dv, tid, d * s);
-}
-
-// ------------------------------------------------------------------------------------------------
-// reductions of an (R x C) array: sum over columns -> [R] (one wavefront per row);
-// sum over rows -> [C] (two stages through per-block partials)
-// ------------------------------------------------------------------------------------------------
 template <typename TI>
 __global__ void __launch_bounds__(256) sum_cols_kernel(const TI* __restrict__ in, float* __restrict__ out, int64_t R, int64_t Ccols) {
   const int lane = threadIdx.x & 63;
@@ -2438,15 +2457,57 @@ __global__ void __launch_bounds__(1024) sum_rows_lds_kernel(const TI* __restrict
   }
 }
 
-template <typename TO>
-__global__ void __launch_bounds__(256) fold_partials_kernel(const float* __restrict__ part, TO* __restrict__ out, int64_t nparts, int64_t n,
-                                                            int accumulate) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (i >= n) return;
+// the two halves of in (2 x R x Ccols) summed over their rows in one launch (grid.y = half; a null result is skipped): the
+// per-block partials of a LayerNorm's dgamma and dbeta.  (One thread per column over all rows took 243 us for 1024 rows of 128
+// columns - one load in flight at a time on one CU; sixteen row lanes with four loads each take 7.)
+__global__ void __launch_bounds__(1024) fold_two_kernel(const float* __restrict__ in, float* __restrict__ out0, float* __restrict__ out1, int64_t R,
+                                                        int64_t Ccols) {
+  __shared__ float s_acc[16][64];
+  float* out = blockIdx.y ? out1 : out0;
+  if (!out) return;
+  const float* p = in + static_cast<int64_t>(blockIdx.y) * R * Ccols;
+  const int cl = threadIdx.x & 63, rl = threadIdx.x >> 6;
+  const int64_t cc = static_cast<int64_t>(blockIdx.x) * 64 + cl;
   float s = 0;
-  for (int64_t p = 0; p < nparts; ++p) s += part[p * n + i];
-  if (accumulate) s += tri_load(out, i);
-  tri_store(out, i, s);
+  if (cc < Ccols) {
+    int64_t r = rl;
+    for (; r + 48 < R; r += 64) {
+      const float v0 = p[r * Ccols + cc], v1 = p[(r + 16) * Ccols + cc], v2 = p[(r + 32) * Ccols + cc], v3 = p[(r + 48) * Ccols + cc];
+      s += v0; s += v1; s += v2; s += v3;
+    }
+    for (; r < R; r += 16) s += p[r * Ccols + cc];
+  }
+  s_acc[rl][cl] = s;
+  __syncthreads();
+  if (rl == 0 && cc < Ccols) {
+    float total = 0;
+#pragma unroll
+    for (int t = 0; t < 16; ++t) total += s_acc[t][cl];
+    out[cc] = total;
+  }
+}
+
+// rows of a padded square from the caller's rows (TO_PAD; padding is zero) or back, in 16-byte vectors (V = uint4) or elements;
+// a null `in` stands for ones
+template <typename V, bool TO_PAD>
+__global__ void __launch_bounds__(256) pair_rows_kernel(const V* __restrict__ in, V* __restrict__ out, int vpr, int64_t total, PairRows pairs, V one) {
+  for (int64_t e = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; e < total; e += static_cast<int64_t>(gridDim.x) * 256) {
+    const int64_t m = e / vpr;
+    const int v = static_cast<int>(e - m * vpr), src = pairs.src(static_cast<int>(m));
+    if constexpr (TO_PAD) {
+      V val{};
+      if (src >= 0) val = in ? in[static_cast<int64_t>(src) * vpr + v] : one;
+      out[e] = val;
+    } else if (src >= 0) {
+      out[static_cast<int64_t>(src) * vpr + v] = in[e];
+    }
+  }
+}
+
+template <typename TO>
+__global__ void __launch_bounds__(256) round_values_kernel(const float* __restrict__ in, TO* __restrict__ out, int64_t n) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (i < n) tri_store(out, i, in[i]);
 }
 
 static bool is_io(int dt) { return dt == CUEQ_F32 || dt == CUEQ_BF16 || dt == CUEQ_F16; }
@@ -2668,19 +2729,25 @@ static bool dual_gate_res_fits(int64_t C, int64_t M, int64_t K, const void* out,
 }
 static int launch_dual_gate_res(int64_t C, int64_t M, int64_t K, const void* W1, const void* W2, int64_t ldw, const void* X, const void* X2,
                                 int64_t ldx, const void* bias1, const void* bias2, const void* mask, void* out, int64_t ldc, const void* gamma,
-                                const void* beta, float eps, void* xhat, int64_t ldxh, float* mean, float* rstd, bool half, hipStream_t stream) {
+                                const void* beta, float eps, void* xhat, int64_t ldxh, float* mean, float* rstd, bool half, hipStream_t stream,
+                                PairRows pairs = PairRows()) {
   const bool by_rows = X2 != nullptr;
   const size_t lds = dual_gate_res_lds(C, K, xhat != nullptr);
   const int64_t ntiles = (M + (by_rows ? 31 : 63)) / (by_rows ? 32 : 64);
   int64_t gx = (ntiles + 7) / 8;
   if (gx > device_cus()) gx = device_cus();
-#define DGR_F(FT, KT, LN, RW) do { auto kfn = dual_gate_res_kernel<FT, KT, LN, RW>; \
+#define DGR_F(FT, KT, LN, RW, PD) do { auto kfn = dual_gate_res_kernel<FT, KT, LN, RW, PD>; \
     CUEQ_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kfn), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds))); \
-    hipLaunchKernelGGL(kfn, dim3(static_cast<unsigned>(gx)), dim3(512), lds, stream, static_cast<const FT*>(W1), static_cast<const FT*>(W2), ldw, static_cast<const FT*>(X), static_cast<const FT*>(X2), ldx, static_cast<const FT*>(bias1), static_cast<const FT*>(bias2), static_cast<const FT*>(mask), static_cast<FT*>(out), ldc, static_cast<int>(C), static_cast<int>(M), static_cast<const FT*>(gamma), static_cast<const FT*>(beta), eps, static_cast<FT*>(xhat), ldxh, mean, rstd); } while (0)
-#define DGR(KT, LN, RW) do { if (half) DGR_F(f16bits, KT, LN, RW); else DGR_F(uint16_t, KT, LN, RW); } while (0)
+    hipLaunchKernelGGL(kfn, dim3(static_cast<unsigned>(gx)), dim3(512), lds, stream, static_cast<const FT*>(W1), static_cast<const FT*>(W2), ldw, static_cast<const FT*>(X), static_cast<const FT*>(X2), ldx, static_cast<const FT*>(bias1), static_cast<const FT*>(bias2), static_cast<const FT*>(mask), static_cast<FT*>(out), ldc, static_cast<int>(C), static_cast<int>(M), static_cast<const FT*>(gamma), static_cast<const FT*>(beta), eps, static_cast<FT*>(xhat), ldxh, mean, rstd, pairs); } while (0)
+#define DGR(KT, LN, RW) do { if (half) DGR_F(f16bits, KT, LN, RW, false); else DGR_F(uint16_t, KT, LN, RW, false); } while (0)
+#define DGP(KT, LN, RW) do { if (half) DGR_F(f16bits, KT, LN, RW, true); else DGR_F(uint16_t, KT, LN, RW, true); } while (0)
 #define DGR_K(LN, RW) do { switch (K / 32) { case 1: DGR(1, LN, RW); break; case 2: DGR(2, LN, RW); break; case 3: DGR(3, LN, RW); break; default: DGR(4, LN, RW); break; } } while (0)
-  if (by_rows) DGR_K(false, true); else if (xhat) DGR_K(true, false); else DGR_K(false, false);
+  if (pairs.np) {  // (K = 64 or 128: the caller checks)
+    if (by_rows) { if (K == 64) DGP(2, false, true); else DGP(4, false, true); }
+    else { if (K == 64) DGP(2, true, false); else DGP(4, true, false); }
+  } else if (by_rows) DGR_K(false, true); else if (xhat) DGR_K(true, false); else DGR_K(false, false);
 #undef DGR_K
+#undef DGP
 #undef DGR
 #undef DGR_F
   CUEQ_CHECK_HIP(hipGetLastError());
@@ -2762,7 +2829,8 @@ static int gate_bwd_input_impl(int32_t dtype, int64_t C, int64_t M, int64_t K, c
                                const void* X1, const void* X2, int64_t ldx,
                                const void* bias1, const void* bias2, const void* mask, const void* dC, int64_t ldc,
                                int32_t dc_by_row, void* dX1, void* dX2, int64_t lddx, int32_t accumulate, void* dU, void* dV,
-                               const void* ln_x, int64_t ldlx, const float* ln_mean, const float* ln_rstd, const void* ln_gamma, void* stream_) {
+                               const void* ln_x, int64_t ldlx, const float* ln_mean, const float* ln_rstd, const void* ln_gamma, void* stream_,
+                               void* dres = nullptr, PairRows pairs = PairRows()) {
   hipStream_t stream = static_cast<hipStream_t>(stream_);
   CUEQ_REQUIRE(is_io(dtype), CUEQ_ERR_UNSUPPORTED, "gate_bwd_input: dtype must be float32 or bfloat16");
   CUEQ_REQUIRE(C >= 0 && M >= 0 && K > 0, CUEQ_ERR_INVALID, "gate_bwd_input: bad extents");
@@ -2771,6 +2839,7 @@ static int gate_bwd_input_impl(int32_t dtype, int64_t C, int64_t M, int64_t K, c
   CUEQ_REQUIRE(C % 32 == 0 && C > 0, CUEQ_ERR_UNSUPPORTED, "gate_bwd_input: C must be a positive multiple of 32");
   CUEQ_REQUIRE(M < (1ll << 31) - kTile && C < (1ll << 31), CUEQ_ERR_TOO_LARGE, "gate_bwd_input: extent too large");
   CUEQ_REQUIRE(W1 && W2 && X1 && dC && dX1 && (!dU == !dV), CUEQ_ERR_INVALID, "gate_bwd_input: null operand");
+  if (ln_x && !dres) dres = dX1;  // (in place)
   const bool bf = dtype != CUEQ_F32, half = dtype == CUEQ_F16;
   const bool split = X2 != nullptr && X2 != X1;
   CUEQ_REQUIRE(!split || dX2, CUEQ_ERR_INVALID, "gate_bwd_input: two inputs need two gradients");
@@ -2811,26 +2880,33 @@ static int gate_bwd_input_impl(int32_t dtype, int64_t C, int64_t M, int64_t K, c
       const int64_t ntiles = (M + 31) / 32;
       int64_t gx = (ntiles + nwaves - 1) / nwaves;
       if (gx > device_cus()) gx = device_cus();
-#define GBR_F(FT, KT, SP) do { auto kfn = gate_bwd_input_res_kernel<FT, KT, SP, !SP, false>; \
+#define GBR_F(FT, KT, SP, PD) do { auto kfn = gate_bwd_input_res_kernel<FT, KT, SP, !SP, false, PD>; \
         CUEQ_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kfn), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds))); \
-        hipLaunchKernelGGL(kfn, dim3(static_cast<unsigned>(gx)), dim3(SP ? 256 : 512), lds, stream, static_cast<const FT*>(W1), static_cast<const FT*>(W2), ldw, static_cast<const FT*>(X1), static_cast<const FT*>(X2), ldx, static_cast<const FT*>(bias1), static_cast<const FT*>(bias2), static_cast<const FT*>(mask), static_cast<const FT*>(dC), ldc, static_cast<FT*>(dX1), static_cast<FT*>(dX2), lddx, accumulate, static_cast<FT*>(dU), static_cast<FT*>(dV), static_cast<int>(C), static_cast<int>(M), static_cast<const FT*>(nullptr), int64_t(0), static_cast<const float*>(nullptr), static_cast<const float*>(nullptr), static_cast<const FT*>(nullptr)); } while (0)
-#define GBR(KT, SP) do { if (half) GBR_F(f16bits, KT, SP); else GBR_F(uint16_t, KT, SP); } while (0)
+        hipLaunchKernelGGL(kfn, dim3(static_cast<unsigned>(gx)), dim3(SP ? 256 : 512), lds, stream, static_cast<const FT*>(W1), static_cast<const FT*>(W2), ldw, static_cast<const FT*>(X1), static_cast<const FT*>(X2), ldx, static_cast<const FT*>(bias1), static_cast<const FT*>(bias2), static_cast<const FT*>(mask), static_cast<const FT*>(dC), ldc, static_cast<FT*>(dX1), static_cast<FT*>(dX2), lddx, accumulate, static_cast<FT*>(dU), static_cast<FT*>(dV), static_cast<int>(C), static_cast<int>(M), static_cast<const FT*>(nullptr), int64_t(0), static_cast<const float*>(nullptr), static_cast<const float*>(nullptr), static_cast<const FT*>(nullptr), static_cast<FT*>(nullptr), pairs); } while (0)
+#define GBR(KT, SP) do { if (half) GBR_F(f16bits, KT, SP, false); else GBR_F(uint16_t, KT, SP, false); } while (0)
+#define GBP(KT, SP) do { if (half) GBR_F(f16bits, KT, SP, true); else GBR_F(uint16_t, KT, SP, true); } while (0)
 #define GBR_K(SP) do { switch (K / 32) { case 1: GBR(1, SP); break; case 2: GBR(2, SP); break; case 3: GBR(3, SP); break; default: GBR(4, SP); break; } } while (0)
-#define GBL_F(FT, KT) do { auto kfn = gate_bwd_input_res_kernel<FT, KT, false, true, true>; \
+#define GBL_F(FT, KT, PD) do { auto kfn = gate_bwd_input_res_kernel<FT, KT, false, true, true, PD>; \
         CUEQ_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kfn), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds))); \
-        hipLaunchKernelGGL(kfn, dim3(static_cast<unsigned>(gx)), dim3(512), lds, stream, static_cast<const FT*>(W1), static_cast<const FT*>(W2), ldw, static_cast<const FT*>(X1), static_cast<const FT*>(X2), ldx, static_cast<const FT*>(bias1), static_cast<const FT*>(bias2), static_cast<const FT*>(mask), static_cast<const FT*>(dC), ldc, static_cast<FT*>(dX1), static_cast<FT*>(dX2), lddx, accumulate, static_cast<FT*>(dU), static_cast<FT*>(dV), static_cast<int>(C), static_cast<int>(M), static_cast<const FT*>(ln_x), ldlx, ln_mean, ln_rstd, static_cast<const FT*>(ln_gamma)); } while (0)
-#define GBL(KT) do { if (half) GBL_F(f16bits, KT); else GBL_F(uint16_t, KT); } while (0)
-      if (ln_x) { switch (K / 32) { case 1: GBL(1); break; case 2: GBL(2); break; case 3: GBL(3); break; default: GBL(4); break; } }
+        hipLaunchKernelGGL(kfn, dim3(static_cast<unsigned>(gx)), dim3(512), lds, stream, static_cast<const FT*>(W1), static_cast<const FT*>(W2), ldw, static_cast<const FT*>(X1), static_cast<const FT*>(X2), ldx, static_cast<const FT*>(bias1), static_cast<const FT*>(bias2), static_cast<const FT*>(mask), static_cast<const FT*>(dC), ldc, static_cast<FT*>(dX1), static_cast<FT*>(dX2), lddx, accumulate, static_cast<FT*>(dU), static_cast<FT*>(dV), static_cast<int>(C), static_cast<int>(M), static_cast<const FT*>(ln_x), ldlx, ln_mean, ln_rstd, static_cast<const FT*>(ln_gamma), static_cast<FT*>(dres), pairs); } while (0)
+#define GBL(KT, PD) do { if (half) GBL_F(f16bits, KT, PD); else GBL_F(uint16_t, KT, PD); } while (0)
+      if (pairs.np) {  // (K = 64 or 128: the caller checks)
+        if (ln_x) { if (K == 64) GBL(2, true); else GBL(4, true); }
+        else if (split) { if (K == 64) GBP(2, true); else GBP(4, true); }
+        else { if (K == 64) GBP(2, false); else GBP(4, false); }
+      } else if (ln_x) { switch (K / 32) { case 1: GBL(1, false); break; case 2: GBL(2, false); break; case 3: GBL(3, false); break; default: GBL(4, false); break; } }
       else if (split) GBR_K(true); else GBR_K(false);
 #undef GBL
 #undef GBL_F
 #undef GBR_K
+#undef GBP
 #undef GBR
 #undef GBR_F
       CUEQ_CHECK_HIP(hipGetLastError());
       return CUEQ_OK;
     }
   }
+  CUEQ_REQUIRE(!pairs.np, CUEQ_ERR_UNSUPPORTED, "gate_bwd_input: padded rows need the resident weights");
   CUEQ_REQUIRE(!ln_x, CUEQ_ERR_UNSUPPORTED, "gate_bwd_input_ln: needs bfloat16, the weights fitting the local data share, an even M and ldc (compose cueq_gate_bwd_input and cueq_layer_norm_bwd otherwise)");
 #define GBI(TI, KT, SP) hipLaunchKernelGGL((gate_bwd_input_kernel<TI, KT, SP, !SP>), dim3(static_cast<unsigned>((M + gbi_threads<TI, SP>() / 2 - 1) / (gbi_threads<TI, SP>() / 2))), dim3(gbi_threads<TI, SP>()), 0, stream, static_cast<const TI*>(W1), static_cast<const TI*>(W2), ldw, static_cast<const TI*>(X1), static_cast<const TI*>(X2), ldx, static_cast<const TI*>(bias1), static_cast<const TI*>(bias2), static_cast<const TI*>(mask), static_cast<const TI*>(dC), ldc, static_cast<TI*>(dX1), static_cast<TI*>(dX2), lddx, accumulate, static_cast<TI*>(dU), static_cast<TI*>(dV), static_cast<int>(C), static_cast<int>(M))
 #define GBI_K(TI, SP) do { switch (K / 32) { case 1: GBI(TI, 1, SP); break; case 2: GBI(TI, 2, SP); break; case 3: GBI(TI, 3, SP); break; default: GBI(TI, 4, SP); break; } } while (0)
@@ -2862,6 +2938,30 @@ extern "C" int cueq_gate_bwd_input_ln(int32_t dtype, int64_t C, int64_t M, int64
                "gate_bwd_input_ln: the LayerNorm input rows must be 16-byte aligned");
   return gate_bwd_input_impl(dtype, C, M, K, W1, W2, ldw, X, nullptr, ldx, bias1, bias2, mask, dC, ldc, 1, dX, nullptr, lddx, accumulate, nullptr, nullptr,
                              ln_x, ldlx, ln_mean, ln_rstd, ln_gamma, stream_);
+}
+
+// Partial products of a long contraction in the input type's matrix instructions: chunk i of `chunks` covers k in
+// [i kc, (i + 1) kc), kc = long_k_chunk(...); partials[i][part] (float32, M x N) = A_part[:, chunk] B_part[:, chunk]^T.  A is M x K, or
+// K x M with trans_a; B is K x N; part p of A / B starts p * stride_a / stride_b elements further.  The caller sums the chunks.
+static int64_t long_k_chunk(int64_t K, int64_t M, int64_t N, int64_t nparts) {
+  const int64_t tiles = ((M + kTile - 1) / kTile) * ((N + kTile - 1) / kTile) * nparts;
+  int64_t chunks = std::max<int64_t>(1, 2 * device_cus() / tiles);
+  chunks = std::min(chunks, std::max<int64_t>(1, K / 512));
+  return ((K + chunks - 1) / chunks + 63) & ~int64_t(63);
+}
+static int gemm_long_k(int32_t dtype, bool trans_a, int64_t M, int64_t N, int64_t K, const void* A, int64_t lda, int64_t stride_a, const void* B,
+                       int64_t ldb, int64_t stride_b, int64_t nparts, float* partials, hipStream_t stream) {
+  const int64_t kc = long_k_chunk(K, M, N, nparts), chunks = (K + kc - 1) / kc;
+  CUEQ_REQUIRE(chunks * nparts < 65536 && M < (1 << 20) && N < (1 << 20), CUEQ_ERR_TOO_LARGE, "gemm_long_k: too many parts");
+  const dim3 grid(static_cast<unsigned>((N + kTile - 1) / kTile), static_cast<unsigned>((M + kTile - 1) / kTile), static_cast<unsigned>(chunks * nparts));
+  KernelTimer timer("gemm_long_k", stream);
+#define LK(TI, TA) hipLaunchKernelGGL((gemm_kernel<TI, float, TA, true>), grid, dim3(256), 0, stream, static_cast<const TI*>(A), lda, TA ? kc * lda : kc, static_cast<const TI*>(B), ldb, kc * ldb, partials, N, nparts * M * N, static_cast<int>(M), static_cast<int>(N), static_cast<int>(kc), 1.0f, 0, 0, K, static_cast<int>(nparts), stride_a, stride_b, M * N, nullptr, 0, 0, 0, 0)
+#define LK_T(TI) do { if (trans_a) LK(TI, true); else LK(TI, false); } while (0)
+  TRI_DISPATCH(dtype, LK_T(float), LK_T(uint16_t), LK_T(f16bits));
+#undef LK_T
+#undef LK
+  CUEQ_CHECK_HIP(hipGetLastError());
+  return CUEQ_OK;
 }
 
 extern "C" int64_t cueq_gemm_tn_items(int64_t rows, int32_t nparts) {
@@ -2983,9 +3083,9 @@ static int64_t ln_bwd_blocks(int64_t rows) {
 extern "C" int64_t cueq_layer_norm_bwd_workspace(int64_t rows, int64_t D) { return ln_bwd_blocks(rows) * 2 * D * static_cast<int64_t>(sizeof(float)); }
 
 // dgamma / dbeta (float32, length D) may be null; workspace as sized by cueq_layer_norm_bwd_workspace.
-extern "C" int cueq_layer_norm_bwd(int32_t dtype, int64_t rows, int64_t D, const void* dy, const void* x, const float* mean, const float* rstd,
-                                   const void* gamma, void* dx, float* dgamma, float* dbeta, void* workspace, int64_t workspace_bytes,
-                                   void* stream_) {
+static int layer_norm_bwd_impl(int32_t dtype, int64_t rows, int64_t D, const void* dy, const void* x, const float* mean, const float* rstd,
+                               const void* gamma, void* dx, float* dgamma, float* dbeta, void* workspace, int64_t workspace_bytes,
+                               void* stream_, PairRows pairs) {
   hipStream_t stream = static_cast<hipStream_t>(stream_);
   CUEQ_REQUIRE(is_io(dtype), CUEQ_ERR_UNSUPPORTED, "layer_norm: dtype must be float32 or bfloat16");
   CUEQ_REQUIRE(D > 0 && D <= 64 * kLnMaxPerLane, CUEQ_ERR_UNSUPPORTED, "layer_norm: hidden size must be in [1, %d]", 64 * kLnMaxPerLane);
@@ -3006,12 +3106,13 @@ extern "C" int cueq_layer_norm_bwd(int32_t dtype, int64_t rows, int64_t D, const
     const int nq = static_cast<int>((D + 63) / 64);
     if (al16 && (D == 32 || D == 64 || D == 128 || D == 256 || D == 512)) {
       const int L = static_cast<int>(D / 8);
-#define LNB8(T, LL) hipLaunchKernelGGL((ln_bwd_rows8<T, LL>), dim3(static_cast<unsigned>(nb)), dim3(256), sh, stream, static_cast<const T*>(dy), static_cast<const T*>(x), mean, rstd, static_cast<const T*>(gamma), static_cast<T*>(dx), part, rows, rpb)
+#define LNB8(T, LL) hipLaunchKernelGGL((ln_bwd_rows8<T, LL>), dim3(static_cast<unsigned>(nb)), dim3(256), sh, stream, static_cast<const T*>(dy), static_cast<const T*>(x), mean, rstd, static_cast<const T*>(gamma), static_cast<T*>(dx), part, rows, rpb, pairs)
 #define LNB8_L(T) do { switch (L) { case 4: LNB8(T, 4); break; case 8: LNB8(T, 8); break; case 16: LNB8(T, 16); break; case 32: LNB8(T, 32); break; default: LNB8(T, 64); } } while (0)
       TRI_DISPATCH(dtype, LNB8_L(float), LNB8_L(uint16_t), LNB8_L(f16bits));
 #undef LNB8_L
 #undef LNB8
     } else {
+      CUEQ_REQUIRE(!pairs.np, CUEQ_ERR_UNSUPPORTED, "layer_norm: padded rows need D = 32, 64, 128, 256 or 512");
 #define LN_BWD(T, NQ) hipLaunchKernelGGL((ln_bwd_kernel<T, NQ>), dim3(static_cast<unsigned>(nb)), dim3(256), sh, stream, static_cast<const T*>(dy), static_cast<const T*>(x), mean, rstd, static_cast<const T*>(gamma), static_cast<T*>(dx), part, rows, static_cast<int>(D), rpb)
 #define LN_BWD_NQ(T) do { if (nq <= 1) LN_BWD(T, 1); else if (nq <= 2) LN_BWD(T, 2); else if (nq <= 4) LN_BWD(T, 4); else if (nq <= 8) LN_BWD(T, 8); else LN_BWD(T, 16); } while (0)
     TRI_DISPATCH(dtype, LN_BWD_NQ(float), LN_BWD_NQ(uint16_t), LN_BWD_NQ(f16bits));
@@ -3020,12 +3121,15 @@ extern "C" int cueq_layer_norm_bwd(int32_t dtype, int64_t rows, int64_t D, const
     }
   }
   CUEQ_CHECK_HIP(hipGetLastError());
-  const unsigned g = static_cast<unsigned>((D + 255) / 256);
-  if (dgamma) hipLaunchKernelGGL(fold_partials_kernel<float>, dim3(g), dim3(256), 0, stream, part, dgamma, nb, D, 0);
-  CUEQ_CHECK_HIP(hipGetLastError());
-  if (dbeta) hipLaunchKernelGGL(fold_partials_kernel<float>, dim3(g), dim3(256), 0, stream, part + nb * D, dbeta, nb, D, 0);
+  if (dgamma || dbeta) hipLaunchKernelGGL(fold_two_kernel, dim3(static_cast<unsigned>((D + 63) / 64), 2), dim3(1024), 0, stream, part, dgamma, dbeta, nb, D);
   CUEQ_CHECK_HIP(hipGetLastError());
   return CUEQ_OK;
+}
+
+extern "C" int cueq_layer_norm_bwd(int32_t dtype, int64_t rows, int64_t D, const void* dy, const void* x, const float* mean, const float* rstd,
+                                   const void* gamma, void* dx, float* dgamma, float* dbeta, void* workspace, int64_t workspace_bytes,
+                                   void* stream_) {
+  return layer_norm_bwd_impl(dtype, rows, D, dy, x, mean, rstd, gamma, dx, dgamma, dbeta, workspace, workspace_bytes, stream_, PairRows());
 }
 
 static bool ln_t_ok(int32_t dtype, int64_t M, int64_t D, const void* a, const void* b, const void* c) {
@@ -3140,51 +3244,11 @@ extern "C" int cueq_layer_norm_t_bwd(int32_t dtype, int64_t M, int64_t D, const 
                  hipLaunchKernelGGL(ln_t_bwd_kernel<f16bits>, dim3(static_cast<unsigned>(nb)), dim3(256), bwd_lds, stream, static_cast<const f16bits*>(dy), static_cast<const f16bits*>(x_t), mean, rstd, static_cast<const f16bits*>(gamma), static_cast<f16bits*>(dx_t), part, M, static_cast<int>(D), ntiles, need_affine));
   }
   CUEQ_CHECK_HIP(hipGetLastError());
-  const unsigned g = static_cast<unsigned>((D + 255) / 256);
-  if (dgamma) hipLaunchKernelGGL(fold_partials_kernel<float>, dim3(g), dim3(256), 0, stream, part, dgamma, nb, D, 0);
-  CUEQ_CHECK_HIP(hipGetLastError());
-  if (dbeta) hipLaunchKernelGGL(fold_partials_kernel<float>, dim3(g), dim3(256), 0, stream, part + nb * D, dbeta, nb, D, 0);
+  if (dgamma || dbeta) hipLaunchKernelGGL(fold_two_kernel, dim3(static_cast<unsigned>((D + 63) / 64), 2), dim3(1024), 0, stream, part, dgamma, dbeta, nb, D);
   CUEQ_CHECK_HIP(hipGetLastError());
   return CUEQ_OK;
 }
 
-extern "C" int cueq_gate_fwd(int32_t dtype, int64_t rows, int64_t cols, const float* u, const float* v, const void* bias_u, const void* bias_v,
-                             int32_t bias_axis, const void* mask, int32_t mask_axis, void* out, void* stream_) {
-  hipStream_t stream = static_cast<hipStream_t>(stream_);
-  CUEQ_REQUIRE(is_io(dtype), CUEQ_ERR_UNSUPPORTED, "gate: dtype must be float32 or bfloat16");
-  const int64_t n = rows * cols;
-  if (n <= 0) return CUEQ_OK;
-  CUEQ_REQUIRE(u && v && out, CUEQ_ERR_INVALID, "gate: null operand");
-  CUEQ_REQUIRE((n + 255) / 256 < (1ll << 31), CUEQ_ERR_TOO_LARGE, "gate: too many elements");
-  const dim3 grid(static_cast<unsigned>((n + 255) / 256));
-  KernelTimer timer("gate_fwd", stream);
-  TRI_DISPATCH(dtype,
-               hipLaunchKernelGGL(gate_fwd_kernel<float>, grid, dim3(256), 0, stream, u, v, static_cast<const float*>(bias_u), static_cast<const float*>(bias_v), bias_axis, static_cast<const float*>(mask), mask_axis, static_cast<float*>(out), rows, cols),
-               hipLaunchKernelGGL(gate_fwd_kernel<uint16_t>, grid, dim3(256), 0, stream, u, v, static_cast<const uint16_t*>(bias_u), static_cast<const uint16_t*>(bias_v), bias_axis, static_cast<const uint16_t*>(mask), mask_axis, static_cast<uint16_t*>(out), rows, cols),
-               hipLaunchKernelGGL(gate_fwd_kernel<f16bits>, grid, dim3(256), 0, stream, u, v, static_cast<const f16bits*>(bias_u), static_cast<const f16bits*>(bias_v), bias_axis, static_cast<const f16bits*>(mask), mask_axis, static_cast<f16bits*>(out), rows, cols));
-  CUEQ_CHECK_HIP(hipGetLastError());
-  return CUEQ_OK;
-}
-
-extern "C" int cueq_gate_bwd(int32_t dtype, int64_t rows, int64_t cols, const void* dout, const float* u, const float* v, const void* bias_u,
-                             const void* bias_v, int32_t bias_axis, const void* mask, int32_t mask_axis, void* du, void* dv, void* stream_) {
-  hipStream_t stream = static_cast<hipStream_t>(stream_);
-  CUEQ_REQUIRE(is_io(dtype), CUEQ_ERR_UNSUPPORTED, "gate: dtype must be float32 or bfloat16");
-  const int64_t n = rows * cols;
-  if (n <= 0) return CUEQ_OK;
-  CUEQ_REQUIRE(dout && u && v && du && dv, CUEQ_ERR_INVALID, "gate: null operand");
-  CUEQ_REQUIRE((n + 255) / 256 < (1ll << 31), CUEQ_ERR_TOO_LARGE, "gate: too many elements");
-  const dim3 grid(static_cast<unsigned>((n + 255) / 256));
-  KernelTimer timer("gate_bwd", stream);
-  TRI_DISPATCH(dtype,
-               hipLaunchKernelGGL(gate_bwd_kernel<float>, grid, dim3(256), 0, stream, static_cast<const float*>(dout), u, v, static_cast<const float*>(bias_u), static_cast<const float*>(bias_v), bias_axis, static_cast<const float*>(mask), mask_axis, static_cast<float*>(du), static_cast<float*>(dv), rows, cols),
-               hipLaunchKernelGGL(gate_bwd_kernel<uint16_t>, grid, dim3(256), 0, stream, static_cast<const uint16_t*>(dout), u, v, static_cast<const uint16_t*>(bias_u), static_cast<const uint16_t*>(bias_v), bias_axis, static_cast<const uint16_t*>(mask), mask_axis, static_cast<uint16_t*>(du), static_cast<uint16_t*>(dv), rows, cols),
-               hipLaunchKernelGGL(gate_bwd_kernel<f16bits>, grid, dim3(256), 0, stream, static_cast<const f16bits*>(dout), u, v, static_cast<const f16bits*>(bias_u), static_cast<const f16bits*>(bias_v), bias_axis, static_cast<const f16bits*>(mask), mask_axis, static_cast<f16bits*>(du), static_cast<f16bits*>(dv), rows, cols));
-  CUEQ_CHECK_HIP(hipGetLastError());
-  return CUEQ_OK;
-}
-
-// out[r] = sum_c in[r][c]   (float32 result)
 extern "C" int cueq_sum_cols(int32_t dtype, int64_t rows, int64_t cols, const void* in, float* out, void* stream_) {
   hipStream_t stream = static_cast<hipStream_t>(stream_);
   CUEQ_REQUIRE(is_io(dtype), CUEQ_ERR_UNSUPPORTED, "sum_cols: dtype must be float32 or bfloat16");
@@ -3241,7 +3305,314 @@ extern "C" int cueq_sum_rows(int32_t dtype, int64_t rows, int64_t cols, const vo
                hipLaunchKernelGGL(sum_rows_partial_kernel<uint16_t>, grid, dim3(256), 0, stream, static_cast<const uint16_t*>(in), part, rows, cols, rpb),
                hipLaunchKernelGGL(sum_rows_partial_kernel<f16bits>, grid, dim3(256), 0, stream, static_cast<const f16bits*>(in), part, rows, cols, rpb));
   CUEQ_CHECK_HIP(hipGetLastError());
-  hipLaunchKernelGGL(fold_partials_kernel<float>, dim3(static_cast<unsigned>((cols + 255) / 256)), dim3(256), 0, stream, part, out, nb, cols, 0);
+  hipLaunchKernelGGL(sum_rows_lds_kernel<float>, dim3(static_cast<unsigned>((cols + 63) / 64)), dim3(1024), 0, stream, part, out, nb, cols);
   CUEQ_CHECK_HIP(hipGetLastError());
   return CUEQ_OK;
 }
+
+// ------------------------------------------------------------------------------------------------
+// The whole update, forward and backward, as one call each: the stages above in order on one stream, what lives between them in
+// one buffer.  (The host needs about 4 us per stage when every stage is a call from Python with its own allocations - 190 us for
+// the eleven launches of a step, more than they take on the GPU below 256 x 256 pairs.)
+//
+// The pair rows between the stages are those of a square of np x np, np = n rounded up to a whole number of 16-byte pieces: with
+// an odd n no row of the contraction's matrices is aligned, and the products would run one element at a time (391 x 391 x 128
+// bfloat16 training step 196 ms).  The stages that touch the caller's rows map them (`PairRows`, `mapped`); where those stages
+// are not the ones with resident weights the rows are copied in and out instead (`copies`).
+// ------------------------------------------------------------------------------------------------
+namespace {
+
+enum { kNinW, kNinB, kPinW, kPinB, kGinW, kGinB, kNoutW, kNoutB, kPoutW, kPoutB, kGoutW, kGoutB, kWeights };
+
+struct TriPlan {
+  int32_t dt;
+  int64_t B, N, Np, D, Do, M, es;
+  bool resident, mapped, copies;
+  PairRows pairs;
+
+  TriPlan(int32_t dt_, int64_t B_, int64_t N_, int64_t D_, int64_t Do_) : dt(dt_), B(B_), N(N_), D(D_), Do(Do_) {
+    es = dt == CUEQ_F32 ? 4 : 2;
+    const int64_t epv = 16 / es;
+    Np = (N + epv - 1) / epv * epv;
+    M = B * Np * Np;
+    // LayerNorm inside the input stage; the gate kernels with the weights in LDS for all four passes over the pair rows
+    resident = dt != CUEQ_F32 && D % 32 == 0 && D <= 128 && M % 2 == 0 && M >= 4096 && M <= kRowSlab && dual_gate_res_lds(2 * D, D, true) <= 160 * 1024;
+    const size_t bwd_out = static_cast<size_t>(2 * Do * (D == 128 ? 2 * D : 2 * D + 16) + 8 * Do + 32 * (2 * D + 16));
+    const size_t bwd_in = static_cast<size_t>(4 * D * (D == 128 ? 2 * D : 2 * D + 16) + 16 * D + 4 * D);
+    mapped = Np != N && resident && (D == 64 || D == 128) && Do % 32 == 0 && dual_gate_res_lds(Do, D, false) <= 160 * 1024 && bwd_out <= 160 * 1024 &&
+             bwd_in <= 160 * 1024 && (M * Do + 8) * es < (1ll << 32) && 5 * M * es < (1ll << 32);
+    copies = Np != N && !mapped;
+    if (Np != N && M < (1ll << 31)) pairs = PairRows::make(static_cast<int>(N), static_cast<int>(Np));
+  }
+};
+
+struct Carve {  // consecutive pieces of a buffer, each on a 256-byte boundary
+  char* base;
+  int64_t used = 0;
+  explicit Carve(void* p) : base(static_cast<char*>(p)) {}
+  char* take(int64_t bytes) {
+    char* p = base ? base + used : nullptr;
+    used += (bytes + 255) & ~int64_t(255);
+    return p;
+  }
+};
+
+struct TriSaved {  // what the backward reads again
+  char *xh, *y, *ab, *t, *xp, *maskp;
+  float *mean1, *rstd1, *mean2, *rstd2;
+  int64_t bytes;
+  TriSaved(const TriPlan& p, void* buf) {
+    Carve c(buf);
+    const int64_t rows = p.M * p.D * p.es;
+    xh = c.take(rows);
+    y = c.take(rows);
+    ab = c.take(2 * rows);
+    t = c.take(rows);
+    mean1 = reinterpret_cast<float*>(c.take(4 * p.M));
+    rstd1 = reinterpret_cast<float*>(c.take(4 * p.M));
+    mean2 = reinterpret_cast<float*>(c.take(4 * p.M));
+    rstd2 = reinterpret_cast<float*>(c.take(4 * p.M));
+    xp = p.copies ? c.take(rows) : nullptr;
+    maskp = p.copies ? c.take(p.M * p.es) : nullptr;
+    bytes = c.used;
+  }
+};
+
+struct TriFwdWork {
+  char *outp, *tT;
+  int64_t bytes;
+  TriFwdWork(const TriPlan& p, void* buf) {
+    Carve c(buf);
+    outp = p.copies ? c.take(p.M * p.Do * p.es) : nullptr;
+    tT = p.D > kLnTMaxD ? c.take(p.M * p.D * p.es) : nullptr;
+    bytes = c.used;
+  }
+};
+
+struct TriBwdWork {
+  char *dxh, *dy, *dt, *dab, *du2, *du1, *doutp, *dxp, *tT, *part, *ln;
+  float* grads;
+  int64_t part_bytes, ln_bytes, bytes;
+  TriBwdWork(const TriPlan& p, bool weights, void* buf) {
+    Carve c(buf);
+    const int64_t rows = p.M * p.D * p.es;
+    dxh = c.take(rows);
+    dy = c.take(rows);
+    dt = c.take(rows);
+    dab = c.take(2 * rows);
+    doutp = p.copies ? c.take(p.M * p.Do * p.es) : nullptr;
+    dxp = p.copies ? c.take(rows) : nullptr;
+    tT = p.D > kLnTMaxD ? c.take(2 * rows) : nullptr;
+    // the gate gradients: needed for the weight gradients, and where the fused input gradient does not take the shape
+    const bool fused_out = p.D <= 128 && p.Do % 32 == 0, fused_in = p.D <= 128;
+    du2 = weights || !fused_out ? c.take(2 * p.M * p.Do * p.es) : nullptr;
+    du1 = weights || !fused_in ? c.take(4 * rows) : nullptr;
+    auto partial = [&](int64_t m, int64_t n, int64_t parts) {
+      const int64_t kc = long_k_chunk(p.M, m, n, parts), chunks = (p.M + kc - 1) / kc;
+      return chunks * parts * m * n * 4 + 256 + cueq_sum_rows_workspace(chunks, parts * m * n);
+    };
+    part_bytes = weights ? std::max({partial(4 * p.D, p.D, 1), partial(p.Do, p.D, 2), cueq_sum_rows_workspace(p.M, p.Do)}) : 0;
+    part = c.take(part_bytes);
+    ln_bytes = std::max(cueq_layer_norm_bwd_workspace(p.M, p.D), weights ? cueq_layer_norm_t_bwd_workspace(p.dt, p.M, p.D) : int64_t(0));
+    ln = c.take(ln_bytes);
+    grads = reinterpret_cast<float*>(c.take(weights ? 4 * cueq_trimul_grads_values(p.D, p.Do) : 0));
+    bytes = c.used;
+  }
+};
+
+int pair_copy(const TriPlan& p, const void* in, void* out, int64_t width, bool to_pad, hipStream_t stream) {
+  const int64_t bytes = width * p.es;
+  const bool vec = bytes % 16 == 0 && ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 15) == 0;
+  const int vpr = static_cast<int>(vec ? bytes / 16 : width);
+  const int64_t total = p.M * vpr;
+  const dim3 grid(static_cast<unsigned>(std::min<int64_t>((total + 255) / 256, 16ll * device_cus())));
+#define PC(V, ONE) do { if (to_pad) hipLaunchKernelGGL((pair_rows_kernel<V, true>), grid, dim3(256), 0, stream, static_cast<const V*>(in), static_cast<V*>(out), vpr, total, p.pairs, ONE); \
+    else hipLaunchKernelGGL((pair_rows_kernel<V, false>), grid, dim3(256), 0, stream, static_cast<const V*>(in), static_cast<V*>(out), vpr, total, p.pairs, ONE); } while (0)
+  if (vec) PC(uint4, uint4{});
+  else if (p.es == 4) PC(float, 1.0f);
+  else PC(uint16_t, static_cast<uint16_t>(p.dt == CUEQ_BF16 ? 0x3f80 : 0x3c00));
+#undef PC
+  CUEQ_CHECK_HIP(hipGetLastError());
+  return CUEQ_OK;
+}
+
+#define TRI_STEP(expr) do { const int rc_ = (expr); if (rc_ != CUEQ_OK) return rc_; } while (0)
+
+int tri_check(const TriPlan& p) {
+  CUEQ_REQUIRE(is_io(p.dt), CUEQ_ERR_UNSUPPORTED, "trimul: dtype must be float32, bfloat16 or half");
+  CUEQ_REQUIRE(p.B >= 0 && p.N >= 0 && p.D > 0 && p.D % 32 == 0 && p.Do > 0, CUEQ_ERR_INVALID, "trimul: bad extents");
+  CUEQ_REQUIRE(p.M < (1ll << 31) - 256, CUEQ_ERR_TOO_LARGE, "trimul: too many pair rows");
+  return CUEQ_OK;
+}
+
+}  // namespace
+
+extern "C" int64_t cueq_trimul_grads_values(int64_t D, int64_t Do) { return 4 * D + 4 * D * D + 2 * Do * D + 4 * D + 2 * Do; }
+extern "C" int64_t cueq_trimul_saved_bytes(int32_t dtype, int64_t B, int64_t N, int64_t D, int64_t Do) { return TriSaved(TriPlan(dtype, B, N, D, Do), nullptr).bytes; }
+extern "C" int64_t cueq_trimul_workspace_bytes(int32_t dtype, int64_t B, int64_t N, int64_t D, int64_t Do, int32_t backward, int32_t weight_grads) {
+  const TriPlan p(dtype, B, N, D, Do);
+  return backward ? TriBwdWork(p, weight_grads != 0, nullptr).bytes : TriFwdWork(p, nullptr).bytes;
+}
+
+extern "C" int cueq_trimul_fwd(int32_t dtype, int64_t B, int64_t N, int64_t D, int64_t Do, int32_t outgoing, double eps, const void* x, const void* mask,
+                               const void* const* w, void* out, void* saved, void* workspace, int64_t workspace_bytes, void* stream_) {
+  hipStream_t stream = static_cast<hipStream_t>(stream_);
+  const TriPlan p(dtype, B, N, D, Do);
+  TRI_STEP(tri_check(p));
+  if (p.M == 0) return CUEQ_OK;
+  CUEQ_REQUIRE(x && w && w[kPinW] && w[kGinW] && w[kPoutW] && w[kGoutW] && out && saved, CUEQ_ERR_INVALID, "trimul: null operand");
+  const TriSaved s(p, saved);
+  const TriFwdWork k(p, workspace);
+  CUEQ_REQUIRE(workspace_bytes >= k.bytes && (workspace || k.bytes == 0), CUEQ_ERR_INVALID, "trimul: workspace too small");
+  const int64_t M = p.M;
+  if (p.copies) {
+    TRI_STEP(pair_copy(p, x, s.xp, D, true, stream));
+    TRI_STEP(pair_copy(p, mask, s.maskp, 1, true, stream));
+    x = s.xp;
+    mask = s.maskp;
+  }
+  if (p.resident) {
+    KernelTimer timer("ln_dual_gate_fwd", stream);
+    TRI_STEP(launch_dual_gate_res(2 * D, M, D, w[kGinW], w[kPinW], D, x, nullptr, D, w[kGinB], w[kPinB], mask, s.ab, M, w[kNinW], w[kNinB],
+                                  static_cast<float>(eps), s.xh, D, s.mean1, s.rstd1, dtype == CUEQ_F16, stream, p.mapped ? p.pairs : PairRows()));
+  } else {
+    TRI_STEP(cueq_layer_norm_fwd(dtype, M, D, x, w[kNinW], w[kNinB], eps, s.xh, s.mean1, s.rstd1, stream_));
+    TRI_STEP(cueq_dual_gate(dtype, 0, 2 * D, M, D, w[kGinW], w[kPinW], D, s.xh, nullptr, D, w[kGinB], w[kPinB], 0, mask, 1, nullptr, s.ab, nullptr, M,
+                            stream_));
+  }
+  const int64_t np = p.Np, sq = np * np;
+  char* b = s.ab + M * D * p.es;
+  // t[i, j] = sum_k a[i, k] b[j, k]  /  sum_k a[k, i] b[k, j]
+  TRI_STEP(cueq_gemm(dtype, dtype, outgoing ? 0 : 1, outgoing ? 0 : 1, np, np, np, s.ab, np, sq, b, np, sq, s.t, np, sq, D * B, 1.0, 0, stream_));
+  if (D <= kLnTMaxD) {
+    TRI_STEP(cueq_layer_norm_t_fwd(dtype, M, D, s.t, w[kNoutW], w[kNoutB], eps, s.y, s.mean2, s.rstd2, stream_));
+  } else {
+    TRI_STEP(cueq_transpose(dtype, 1, D, M, s.t, k.tT, stream_));
+    TRI_STEP(cueq_layer_norm_fwd(dtype, M, D, k.tT, w[kNoutW], w[kNoutB], eps, s.y, s.mean2, s.rstd2, stream_));
+  }
+  if (p.mapped) {
+    KernelTimer timer("dual_gate_fwd", stream);
+    TRI_STEP(launch_dual_gate_res(Do, M, D, w[kGoutW], w[kPoutW], D, s.xh, s.y, D, w[kGoutB], w[kPoutB], nullptr, out, Do, nullptr, nullptr, 0.f, nullptr, 0,
+                                  nullptr, nullptr, dtype == CUEQ_F16, stream, p.pairs));
+    return CUEQ_OK;
+  }
+  void* to = p.copies ? k.outp : out;
+  TRI_STEP(cueq_dual_gate(dtype, 0, M, Do, D, s.xh, s.y, D, w[kGoutW], w[kPoutW], D, w[kGoutB], w[kPoutB], 1, nullptr, 0, nullptr, to, nullptr, Do, stream_));
+  if (p.copies) TRI_STEP(pair_copy(p, to, out, Do, false, stream));
+  return CUEQ_OK;
+}
+
+extern "C" int cueq_trimul_bwd(int32_t dtype, int64_t B, int64_t N, int64_t D, int64_t Do, int32_t outgoing, const void* x, const void* mask,
+                               const void* const* w, void* saved, const void* dout, void* dx, uint32_t need, void* grads, void* workspace,
+                               int64_t workspace_bytes, void* stream_) {
+  hipStream_t stream = static_cast<hipStream_t>(stream_);
+  const TriPlan p(dtype, B, N, D, Do);
+  TRI_STEP(tri_check(p));
+  const int64_t nv = cueq_trimul_grads_values(D, Do);
+  if (p.M == 0) return CUEQ_OK;  // (the caller returns zeros)
+  CUEQ_REQUIRE(x && w && saved && dout && dx && (grads || !need), CUEQ_ERR_INVALID, "trimul: null operand");
+  const TriSaved s(p, saved);
+  const TriBwdWork k(p, need != 0, workspace);
+  CUEQ_REQUIRE(workspace && workspace_bytes >= k.bytes, CUEQ_ERR_INVALID, "trimul: workspace too small");
+  const int64_t M = p.M, es = p.es, np = p.Np, sq = np * np;
+  auto wants = [&](int i) { return (need >> i & 1u) != 0; };
+  const bool w_out = wants(kPoutW) || wants(kPoutB) || wants(kGoutW) || wants(kGoutB);
+  const bool w_in = wants(kPinW) || wants(kPinB) || wants(kGinW) || wants(kGinB);
+  // the float32 gradients: norms, the input projections (gate, then value), the output projections, the biases
+  float* gf = dtype == CUEQ_F32 ? static_cast<float*>(grads) : k.grads;
+  float *g_nin = gf, *g_nout = gf + 2 * D, *g_in = gf + 4 * D, *g_out = g_in + 4 * D * D, *g_in_b = g_out + 2 * Do * D, *g_out_b = g_in_b + 4 * D;
+  if (p.copies) {
+    TRI_STEP(pair_copy(p, dout, k.doutp, Do, true, stream));
+    x = s.xp;
+    mask = s.maskp;
+    dout = k.doutp;
+  }
+  const PairRows pairs = p.mapped ? p.pairs : PairRows();
+  void* dxt = p.copies ? k.dxp : dx;
+
+  // output gate
+  char *du2 = k.du2, *dv2 = k.du2 ? k.du2 + M * Do * es : nullptr;
+  if (D <= 128 && Do % 32 == 0) {
+    TRI_STEP(gate_bwd_input_impl(dtype, Do, M, D, w[kGoutW], w[kPoutW], D, s.xh, s.y, D, w[kGoutB], w[kPoutB], nullptr, dout, Do, 0, k.dxh, k.dy, D, 0,
+                                 w_out ? du2 : nullptr, w_out ? dv2 : nullptr, nullptr, 0, nullptr, nullptr, nullptr, stream_, nullptr, pairs));
+  } else {
+    TRI_STEP(cueq_dual_gate(dtype, 1, M, Do, D, s.xh, s.y, D, w[kGoutW], w[kPoutW], D, w[kGoutB], w[kPoutB], 1, nullptr, 0, dout, du2, dv2, Do, stream_));
+    TRI_STEP(cueq_gemm(dtype, dtype, 0, 1, M, D, Do, du2, Do, 0, w[kGoutW], D, 0, k.dxh, D, 0, 1, 1.0, 0, stream_));
+    TRI_STEP(cueq_gemm(dtype, dtype, 0, 1, M, D, Do, dv2, Do, 0, w[kPoutW], D, 0, k.dy, D, 0, 1, 1.0, 0, stream_));
+  }
+  const int64_t epv = 16 / es;
+  // sums of the partial products of a long contraction straight into the gradient
+  auto long_k = [&](bool trans_a, int64_t m, const char* A, int64_t lda, int64_t sa, const char* Bm, int64_t sb, int64_t parts, float* to) -> int {
+    const int64_t kc = long_k_chunk(M, m, D, parts), chunks = (M + kc - 1) / kc;
+    float* part = reinterpret_cast<float*>(k.part);
+    TRI_STEP(gemm_long_k(dtype, trans_a, m, D, M, A, lda, sa, Bm, D, sb, parts, part, stream));
+    char* ws = k.part + ((chunks * parts * m * D * 4 + 255) & ~int64_t(255));
+    return cueq_sum_rows(CUEQ_F32, chunks, parts * m * D, part, to, ws, k.part + k.part_bytes - ws, stream_);
+  };
+  if (wants(kGoutW) || wants(kPoutW)) {
+    if (Do % epv == 0) {
+      TRI_STEP(long_k(true, Do, du2, Do, M * Do, s.xh, (s.y - s.xh) / es, 2, g_out));
+    } else {  // (rows of Do elements are not 16-byte aligned: the element-wise product)
+      TRI_STEP(cueq_gemm(dtype, CUEQ_F32, 1, 1, Do, D, M, du2, Do, 0, s.xh, D, 0, g_out, D, 0, 1, 1.0, 0, stream_));
+      TRI_STEP(cueq_gemm(dtype, CUEQ_F32, 1, 1, Do, D, M, dv2, Do, 0, s.y, D, 0, g_out + Do * D, D, 0, 1, 1.0, 0, stream_));
+    }
+  }
+  if (wants(kGoutB)) TRI_STEP(cueq_sum_rows(dtype, M, Do, du2, g_out_b, k.part, k.part_bytes, stream_));
+  if (wants(kPoutB)) TRI_STEP(cueq_sum_rows(dtype, M, Do, dv2, g_out_b + Do, k.part, k.part_bytes, stream_));
+
+  // LayerNorm across d
+  float *dgo = wants(kNoutW) ? g_nout : nullptr, *dbo = wants(kNoutB) ? g_nout + D : nullptr;
+  if (D <= kLnTMaxD) {
+    TRI_STEP(cueq_layer_norm_t_bwd(dtype, M, D, k.dy, s.t, s.mean2, s.rstd2, w[kNoutW], k.dt, dgo, dbo, k.ln, k.ln_bytes, stream_));
+  } else {
+    char* dtT = k.tT + M * D * es;
+    TRI_STEP(cueq_transpose(dtype, 1, D, M, s.t, k.tT, stream_));
+    TRI_STEP(cueq_layer_norm_bwd(dtype, M, D, k.dy, k.tT, s.mean2, s.rstd2, w[kNoutW], dtT, dgo, dbo, k.ln, k.ln_bytes, stream_));
+    TRI_STEP(cueq_transpose(dtype, 1, M, D, dtT, k.dt, stream_));
+  }
+
+  // triangular contraction
+  char *a = s.ab, *b = s.ab + M * D * es, *da = k.dab, *db = k.dab + M * D * es;
+  if (outgoing) {  // t = a b^T: da[i, k] = sum_j dt[i, j] b[j, k], db[j, k] = sum_i dt[i, j] a[i, k]
+    TRI_STEP(cueq_gemm(dtype, dtype, 0, 1, np, np, np, k.dt, np, sq, b, np, sq, da, np, sq, D * B, 1.0, 0, stream_));
+    TRI_STEP(cueq_gemm(dtype, dtype, 1, 1, np, np, np, k.dt, np, sq, a, np, sq, db, np, sq, D * B, 1.0, 0, stream_));
+  } else {  // t = a^T b: da[k, i] = sum_j b[k, j] dt[i, j], db[k, j] = sum_i a[k, i] dt[i, j]
+    TRI_STEP(cueq_gemm(dtype, dtype, 0, 0, np, np, np, b, np, sq, k.dt, np, sq, da, np, sq, D * B, 1.0, 0, stream_));
+    TRI_STEP(cueq_gemm(dtype, dtype, 0, 1, np, np, np, a, np, sq, k.dt, np, sq, db, np, sq, D * B, 1.0, 0, stream_));
+  }
+
+  // input gate and projections - and, when neither their weights nor the LayerNorm's ask for a gradient, the input LayerNorm in
+  // the same kernel
+  const bool affine_in = wants(kNinW) || wants(kNinB);
+  char *du1 = k.du1, *dv1 = k.du1 ? k.du1 + 2 * M * D * es : nullptr;
+  const bool ln_fused = dtype != CUEQ_F32 && D <= 128 && M % 2 == 0 && (4 * M + M) * es < (1ll << 32) &&
+                        4 * D * (D == 128 ? 2 * D : 2 * D + 16) + 20 * D <= 160 * 1024;  // (what cueq_gate_bwd_input_ln takes, however many rows)
+  if (!w_in && !affine_in && ln_fused) {
+    TRI_STEP(gate_bwd_input_impl(dtype, 2 * D, M, D, w[kGinW], w[kPinW], D, s.xh, nullptr, D, w[kGinB], w[kPinB], mask, k.dab, M, 1,
+                                 k.dxh, nullptr, D, 1, nullptr, nullptr, x, D, s.mean1, s.rstd1, w[kNinW], stream_, dxt, pairs));
+    if (p.copies) TRI_STEP(pair_copy(p, dxt, dx, D, false, stream));
+  } else {
+    if (D <= 128) {
+      TRI_STEP(gate_bwd_input_impl(dtype, 2 * D, M, D, w[kGinW], w[kPinW], D, s.xh, nullptr, D, w[kGinB], w[kPinB], mask, k.dab, M, 1, k.dxh, nullptr, D,
+                                   1, w_in ? du1 : nullptr, w_in ? dv1 : nullptr, nullptr, 0, nullptr, nullptr, nullptr, stream_, nullptr, pairs));
+    } else {
+      TRI_STEP(cueq_dual_gate(dtype, 1, 2 * D, M, D, w[kGinW], w[kPinW], D, s.xh, nullptr, D, w[kGinB], w[kPinB], 0, mask, 1, k.dab, du1, dv1, M, stream_));
+      TRI_STEP(cueq_gemm(dtype, dtype, 1, 1, M, D, 2 * D, du1, M, 0, w[kGinW], D, 0, k.dxh, D, 0, 1, 1.0, 1, stream_));
+      TRI_STEP(cueq_gemm(dtype, dtype, 1, 1, M, D, 2 * D, dv1, M, 0, w[kPinW], D, 0, k.dxh, D, 0, 1, 1.0, 1, stream_));
+    }
+    if (wants(kGinW) || wants(kPinW)) TRI_STEP(long_k(false, 4 * D, du1, M, 0, s.xh, 0, 1, g_in));  // (gate rows, then value rows)
+    if (wants(kGinB)) TRI_STEP(cueq_sum_cols(dtype, 2 * D, M, du1, g_in_b, stream_));
+    if (wants(kPinB)) TRI_STEP(cueq_sum_cols(dtype, 2 * D, M, dv1, g_in_b + 2 * D, stream_));
+    TRI_STEP(layer_norm_bwd_impl(dtype, M, D, k.dxh, x, s.mean1, s.rstd1, w[kNinW], dxt, wants(kNinW) ? g_nin : nullptr, wants(kNinB) ? g_nin + D : nullptr,
+                                 k.ln, k.ln_bytes, stream_, pairs));
+    if (p.copies) TRI_STEP(pair_copy(p, dxt, dx, D, false, stream));
+  }
+  if (need && dtype != CUEQ_F32) {
+    const dim3 grid(static_cast<unsigned>((nv + 255) / 256));
+    if (dtype == CUEQ_F16) hipLaunchKernelGGL(round_values_kernel<f16bits>, grid, dim3(256), 0, stream, gf, static_cast<f16bits*>(grads), nv);
+    else hipLaunchKernelGGL(round_values_kernel<uint16_t>, grid, dim3(256), 0, stream, gf, static_cast<uint16_t*>(grads), nv);
+    CUEQ_CHECK_HIP(hipGetLastError());
+  }
+  return CUEQ_OK;
+}
+#undef TRI_STEP

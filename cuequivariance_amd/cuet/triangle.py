@@ -11,14 +11,16 @@ reference states in the open
     y   = LayerNorm over d of t, stored (B, N, N, D)
     out = sigmoid(xh G_out^T + b) * (y P_out^T + b)       -- the output gate reads the normalised input xh
 
-Every stage is a HIP kernel reached through the C ABI (``cueq_gemm_nt``, ``cueq_layer_norm_*``, ``cueq_gate_*``,
-``cueq_transpose``, ``cueq_sum_*``); torch only owns the buffers.  Inputs float32 or bfloat16, fp32 accumulation;
-intermediate tensors are kept in the input dtype like the reference does; the projection accumulators stay in registers
-(``cueq_dual_gate`` fuses both projections with the gate and recomputes them in the backward).
+Forward and backward are one call of the C library each (``cueq_trimul_fwd`` / ``cueq_trimul_bwd``: the stages in order, what
+lives between them in one buffer); torch only owns the buffers.  Inputs float32, bfloat16 or half, fp32 accumulation;
+intermediate tensors are kept in the input dtype like the reference does; the projection accumulators stay in registers (both
+projections fused with the gate and recomputed in the backward).  The wrappers of the single stages below are what the stages'
+own tests call.
 """
 
 from __future__ import annotations
 
+import ctypes
 import enum
 import math
 from typing import List, Optional
@@ -162,28 +164,6 @@ def layer_norm_t_bwd(dy: torch.Tensor, xt: torch.Tensor, mean, rstd, gamma, need
     return dxt, dgamma, dbeta
 
 
-def gate_fwd(u, v, bias_u, bias_v, bias_axis: int, mask, mask_axis: int, dtype) -> torch.Tensor:
-    rows, cols = u.shape
-    out = torch.empty(rows, cols, dtype=dtype, device=u.device)
-    _lib.check(
-        _lib.load().cueq_gate_fwd(_CODE[dtype], rows, cols, u.data_ptr(), v.data_ptr(), _ptr(bias_u), _ptr(bias_v), bias_axis,
-                                  _ptr(mask), mask_axis, out.data_ptr(), _stream(u)),
-        "cueq_gate_fwd",
-    )
-    return out
-
-
-def gate_bwd(dout, u, v, bias_u, bias_v, bias_axis: int, mask, mask_axis: int):
-    rows, cols = u.shape
-    du, dv = torch.empty_like(dout), torch.empty_like(dout)
-    _lib.check(
-        _lib.load().cueq_gate_bwd(_CODE[dout.dtype], rows, cols, dout.data_ptr(), u.data_ptr(), v.data_ptr(), _ptr(bias_u),
-                                  _ptr(bias_v), bias_axis, _ptr(mask), mask_axis, du.data_ptr(), dv.data_ptr(), _stream(u)),
-        "cueq_gate_bwd",
-    )
-    return du, dv
-
-
 def _fusable(*tensors) -> bool:
     """The fused projection + gate kernel moves 16-byte vectors: row strides and addresses must allow it."""
     for t in tensors:
@@ -196,7 +176,7 @@ def _fusable(*tensors) -> bool:
 
 def dual_gate_fwd(A1, A2, B1, B2, bias1, bias2, bias_axis: int, mask, mask_axis: int) -> torch.Tensor:
     """``sigmoid(A1 B1^T + bias1) * (A2 B2^T + bias2) * mask`` (``B2 is None``: same as ``B1``); the two products stay
-    in registers when the operands allow the fused kernel, otherwise they go through float32 buffers."""
+    in registers."""
     M, K = A1.shape
     N = B1.shape[0]
     T = A1.dtype
@@ -209,9 +189,7 @@ def dual_gate_fwd(A1, A2, B1, B2, bias1, bias2, bias_axis: int, mask, mask_axis:
             "cueq_dual_gate",
         )
         return out
-    u = gemm_nt(A1, B1, torch.float32)
-    v = gemm_nt(A2, B1 if B2 is None else B2, torch.float32)
-    return gate_fwd(u, v, bias1, bias2, bias_axis, mask, mask_axis, T)
+    raise NotImplementedError("dual_gate_fwd: operands must be 16-byte aligned")
 
 
 def ln_dual_gate_fwd(x, gamma, beta, eps: float, W1, W2, bias1, bias2, mask):
@@ -235,25 +213,6 @@ def ln_dual_gate_fwd(x, gamma, beta, eps: float, W1, W2, bias1, bias2, mask):
         "cueq_ln_dual_gate",
     )
     return out, xh, mean, rstd
-
-
-def dual_gate_bwd(dout, A1, A2, B1, B2, bias1, bias2, bias_axis: int, mask, mask_axis: int):
-    """Gradients of the two products of :func:`dual_gate_fwd` (they are recomputed, not read back)."""
-    M, K = A1.shape
-    N = B1.shape[0]
-    T = A1.dtype
-    if _fusable(A1, A2, B1, B2, dout) and (K * A1.element_size()) % 16 == 0:
-        du, dv = torch.empty(M, N, dtype=T, device=A1.device), torch.empty(M, N, dtype=T, device=A1.device)
-        _lib.check(
-            _lib.load().cueq_dual_gate(_CODE[T], 1, M, N, K, A1.data_ptr(), A2.data_ptr(), A1.stride(0), B1.data_ptr(), _ptr(B2),
-                                       B1.stride(0), _ptr(bias1), _ptr(bias2), bias_axis, _ptr(mask), mask_axis, dout.data_ptr(),
-                                       du.data_ptr(), dv.data_ptr(), N, _stream(A1)),
-            "cueq_dual_gate",
-        )
-        return du, dv
-    u = gemm_nt(A1, B1, torch.float32)
-    v = gemm_nt(A2, B1 if B2 is None else B2, torch.float32)
-    return gate_bwd(dout, u, v, bias1, bias2, bias_axis, mask, mask_axis)
 
 
 def gate_bwd_input(dC, dc_by_row: bool, W1, W2, X1, X2, bias1, bias2, mask, dX1=None, want_gate_grads: bool = False):
@@ -310,13 +269,6 @@ def gate_bwd_input_ln(dC, W1, W2, X, bias1, bias2, mask, dX, ln_x, ln_mean, ln_r
     return dX
 
 
-def sum_cols(x: torch.Tensor) -> torch.Tensor:
-    rows, cols = x.shape
-    out = torch.empty(rows, dtype=torch.float32, device=x.device)
-    _lib.check(_lib.load().cueq_sum_cols(_CODE[x.dtype], rows, cols, x.data_ptr(), out.data_ptr(), _stream(x)), "cueq_sum_cols")
-    return out
-
-
 def sum_rows(x: torch.Tensor) -> torch.Tensor:
     rows, cols = x.shape
     lib = _lib.load()
@@ -327,168 +279,77 @@ def sum_rows(x: torch.Tensor) -> torch.Tensor:
     return out
 
 
-def _split_k_chunks(K: int, align: int) -> int:
-    """Number of equal chunks (each a multiple of ``align``) to split a long contraction into."""
-    for n in range(min(512, max(1, K // 512)), 1, -1):
-        if K % n == 0 and (K // n) % align == 0:
-            return n
-    return 1
-
-
-def gemm_long_k(A: torch.Tensor, B: torch.Tensor) -> torch.Tensor:
-    """``A (P, K) @ B (Q, K)^T`` in float32 for a very long ``K``: equal k-chunks as a batched GEMM, then an ordered
-    sum of the partial products (no atomics)."""
-    P, K = A.shape
-    Q = B.shape[0]
-    n = _split_k_chunks(K, 8 if A.dtype in _TWO_BYTE else 4)
-    if n == 1:
-        return gemm_nt(A, B, torch.float32)
-    ck = K // n
-    Ab = A.as_strided((n, P, ck), (ck, A.stride(0), 1))
-    Bb = B.as_strided((n, Q, ck), (ck, B.stride(0), 1))
-    part = gemm_nt(Ab, Bb, torch.float32)
-    return sum_rows(part.view(n, P * Q)).view(P, Q)
-
-
 # ---------------------------------------------------------------------------------------------
 # autograd
 # ---------------------------------------------------------------------------------------------
-def _trimul_fwd(x, mask, nin_w, nin_b, p_in_w, p_in_b, g_in_w, g_in_b, nout_w, nout_b, p_out_w, p_out_b, g_out_w, g_out_b,
-                outgoing: bool, eps: float):
-    """Forward of the update on ``x (B, N, N, D)``: returns the output, the tensors the backward reads (inputs first,
-    then the eight computed ones) and the extents."""
-    if True:
-        T = x.dtype
-        Bsz, N, _, D = x.shape
-        M = Bsz * N * N
-        Do = p_out_w.shape[0]
-        x2 = x.reshape(M, D)
-        mflat = None if mask is None else mask.reshape(M)
-        # (2D, M) == (2D, B, N, N): the "transposed output" of the reference comes for free with the weights as rows
-        fused = ln_dual_gate_fwd(x2, nin_w, nin_b, eps, g_in_w, p_in_w, g_in_b, p_in_b, mflat)
-        if fused is not None:
-            ab, xh, mean1, rstd1 = fused
-        else:
-            xh, mean1, rstd1 = layer_norm_fwd(x2, nin_w, nin_b, eps)
-            ab = dual_gate_fwd(g_in_w, p_in_w, xh, None, g_in_b, p_in_b, 0, mflat, 1)
-        a = ab[:D].view(D * Bsz, N, N)
-        b = ab[D:].view(D * Bsz, N, N)
-        if outgoing:
-            t = gemm_nt(a, b, T)  # t[i, j] = sum_k a[i, k] b[j, k]
-        else:
-            t = gemm_nt(a, b, T, trans_a=True, trans_b=True)  # t[i, j] = sum_k a[k, i] b[k, j]
-        t2 = t.view(D, M)
-        if _ln_t_ok(t2):
-            y, mean2, rstd2 = layer_norm_t_fwd(t2, nout_w, nout_b, eps)  # (M, D)
-        else:
-            y, mean2, rstd2 = layer_norm_fwd(transpose(t2), nout_w, nout_b, eps)
-        out = dual_gate_fwd(xh, y, g_out_w, p_out_w, g_out_b, p_out_b, 1, None, 0)  # (M, Do)
-        saved = (x2, mflat, nin_w, p_in_w, p_in_b, g_in_w, g_in_b, nout_w, p_out_w, p_out_b, g_out_w, g_out_b,
-                 xh, mean1, rstd1, ab, t2, mean2, rstd2, y)
-        has = (nin_w is not None, nin_b is not None, nout_w is not None, nout_b is not None)
-        return out.view(Bsz, N, N, Do), saved, (Bsz, N, D, Do), has
+def _aligned(t: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
+    """``t`` on a 16-byte boundary (a copy when a view starts elsewhere)."""
+    return t.clone() if t is not None and t.data_ptr() % 16 else t
 
 
-def _cast(g, like, have):
-    return g.to(like.dtype) if (g is not None and have) else None
+def _pointers(weights):
+    return (ctypes.c_void_p * 12)(*[_ptr(t) for t in weights])
 
 
-def _trimul_bwd(saved, dims, has, outgoing: bool, need, dout):
-    """Gradients for the 16 arguments of :func:`_trimul_fwd` (``need[k]``: whether argument ``k`` wants one)."""
-    if True:
-        (x2, mflat, nin_w, p_in_w, p_in_b, g_in_w, g_in_b, nout_w, p_out_w, p_out_b, g_out_w, g_out_b,
-         xh, mean1, rstd1, ab, t2, mean2, rstd2, y) = saved
-        Bsz, N, D, Do = dims
-        M = Bsz * N * N
-        T = x2.dtype
-        dout = dout.contiguous().view(M, Do).to(T)
+def _trimul_fwd(x, mask, weights, outgoing: bool, eps: float):
+    """Forward of the update on ``x (B, N, N, D)`` with the twelve weights (norm_in w, b, p_in w, b, g_in w, b, norm_out w, b,
+    p_out w, b, g_out w, b; ``None`` where absent): the output and the buffer the backward reads (``cueq_trimul_fwd``)."""
+    lib = _lib.load()
+    Bsz, N, _, D = x.shape
+    Do = weights[8].shape[0]
+    code, dev = _CODE[x.dtype], x.device
+    x, weights = _aligned(x), [_aligned(w) for w in weights]
+    out = torch.empty((Bsz, N, N, Do), dtype=x.dtype, device=dev)
+    saved = torch.empty(lib.cueq_trimul_saved_bytes(code, Bsz, N, D, Do), dtype=torch.uint8, device=dev)
+    ws_bytes = lib.cueq_trimul_workspace_bytes(code, Bsz, N, D, Do, 0, 0)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
+    _lib.check(lib.cueq_trimul_fwd(code, Bsz, N, D, Do, int(outgoing), float(eps), x.data_ptr(), _ptr(mask), _pointers(weights), out.data_ptr(),
+                                   saved.data_ptr(), _ptr(ws), ws_bytes, _stream(x)), "cueq_trimul_fwd")
+    return out, saved
 
-        # output gate
-        w_out = need[10] or need[11] or need[12] or need[13]
-        fused = gate_bwd_input(dout, False, g_out_w, p_out_w, xh, y, g_out_b, p_out_b, None, None, w_out)
-        if fused is not None:
-            dxh, dy, du2, dv2 = fused
-        else:
-            du2, dv2 = dual_gate_bwd(dout, xh, y, g_out_w, p_out_w, g_out_b, p_out_b, 1, None, 0)  # (M, Do)
-            dxh = gemm_nt(du2, transpose(g_out_w), T)  # (M, D)
-            dy = gemm_nt(dv2, transpose(p_out_w), T)
-        w_in = need[4] or need[5] or need[6] or need[7]
-        xhT = transpose(xh) if (w_in or need[12]) else None  # (D, M)
-        d_g_out_w = d_p_out_w = d_g_out_b = d_p_out_b = None
-        if need[12]:
-            d_g_out_w = gemm_long_k(transpose(du2), xhT).to(g_out_w.dtype)
-        if need[10]:
-            d_p_out_w = gemm_long_k(transpose(dv2), transpose(y)).to(p_out_w.dtype)
-        if g_out_b is not None and need[13]:
-            d_g_out_b = sum_rows(du2).to(g_out_b.dtype)
-        if p_out_b is not None and need[11]:
-            d_p_out_b = sum_rows(dv2).to(p_out_b.dtype)
 
-        # LayerNorm across d
-        affine_out = (has[2] and need[8]) or (has[3] and need[9])
-        if _ln_t_ok(t2):
-            dt, d_nout_w, d_nout_b = layer_norm_t_bwd(dy, t2, mean2, rstd2, nout_w, affine_out)  # (D, M)
-        else:
-            dtT, d_nout_w, d_nout_b = layer_norm_bwd(dy, transpose(t2), mean2, rstd2, nout_w, affine_out)
-            dt = transpose(dtT)
-        dt = dt.view(D * Bsz, N, N)  # (D, M) viewed per (d, b)
-
-        # triangular contraction
-        a = ab[:D].view(D * Bsz, N, N)
-        b = ab[D:].view(D * Bsz, N, N)
-        dab = torch.empty_like(ab)
-        da = dab[:D].view(D * Bsz, N, N)
-        db = dab[D:].view(D * Bsz, N, N)
-        if outgoing:  # t = a b^T
-            gemm_nt(dt, b, T, out=da, trans_b=True)  # da[i, k] = sum_j dt[i, j] b[j, k]
-            gemm_nt(dt, a, T, out=db, trans_a=True, trans_b=True)  # db[j, k] = sum_i dt[i, j] a[i, k]
-        else:  # t = a^T b
-            gemm_nt(b, dt, T, out=da)  # da[k, i] = sum_j b[k, j] dt[i, j]
-            gemm_nt(a, dt, T, out=db, trans_b=True)  # db[k, j] = sum_i a[k, i] dt[i, j]
-
-        # input gate and projections - and, when neither their weights nor the LayerNorm's ask for a gradient, the input
-        # LayerNorm in the same kernel
-        affine_in = (has[0] and need[2]) or (has[1] and need[3])
-        if not w_in and not affine_in and need[0]:
-            dx = gate_bwd_input_ln(dab, g_in_w, p_in_w, xh, g_in_b, p_in_b, mflat, dxh, x2, mean1, rstd1, nin_w)
-            if dx is not None:
-                return (dx.view(Bsz, N, N, D), None, None, None, None, None, None, None, _cast(d_nout_w, x2, has[2]), _cast(d_nout_b, x2, has[3]),
-                        d_p_out_w, d_p_out_b, d_g_out_w, d_g_out_b, None, None)
-        fused = gate_bwd_input(dab, True, g_in_w, p_in_w, xh, None, g_in_b, p_in_b, mflat, dxh, w_in)
-        if fused is not None:
-            du1, dv1 = fused[2], fused[3]
-        else:
-            du1, dv1 = dual_gate_bwd(dab, g_in_w, p_in_w, xh, None, g_in_b, p_in_b, 0, mflat, 1)  # (2D, M)
-            gemm_nt(transpose(du1), transpose(g_in_w), T, out=dxh, accumulate=True)
-            gemm_nt(transpose(dv1), transpose(p_in_w), T, out=dxh, accumulate=True)
-        d_g_in_w = d_p_in_w = d_g_in_b = d_p_in_b = None
-        if need[6]:
-            d_g_in_w = gemm_long_k(du1, xhT).to(g_in_w.dtype)
-        if need[4]:
-            d_p_in_w = gemm_long_k(dv1, xhT).to(p_in_w.dtype)
-        if g_in_b is not None and need[7]:
-            d_g_in_b = sum_cols(du1).to(g_in_b.dtype)
-        if p_in_b is not None and need[5]:
-            d_p_in_b = sum_cols(dv1).to(p_in_b.dtype)
-
-        # input LayerNorm
-        dx, d_nin_w, d_nin_b = layer_norm_bwd(dxh, x2, mean1, rstd1, nin_w, affine_in)
-        dx = dx.view(Bsz, N, N, D) if need[0] else None
-        return (dx, None, _cast(d_nin_w, x2, has[0]), _cast(d_nin_b, x2, has[1]), d_p_in_w, d_p_in_b, d_g_in_w, d_g_in_b,
-                _cast(d_nout_w, x2, has[2]), _cast(d_nout_b, x2, has[3]), d_p_out_w, d_p_out_b, d_g_out_w, d_g_out_b, None, None)
+def _trimul_bwd(x, mask, weights, saved, outgoing: bool, need, dout):
+    """``[dx, None (mask), the twelve weight gradients]`` (``need[k]``: whether argument ``k`` of the list wants one)."""
+    lib = _lib.load()
+    Bsz, N, _, D = x.shape
+    Do = weights[8].shape[0]
+    code, dev, T = _CODE[x.dtype], x.device, x.dtype
+    x, weights = _aligned(x), [_aligned(w) for w in weights]
+    wanted = [bool(n) and w is not None for n, w in zip(need[2:14], weights)]
+    bits = sum(1 << i for i, n in enumerate(wanted) if n)
+    dx = torch.empty_like(x)
+    grads = torch.empty(lib.cueq_trimul_grads_values(D, Do), dtype=T, device=dev) if bits else None
+    if x.numel() == 0:
+        if grads is not None:
+            grads.zero_()
+    else:
+        dout = _aligned(dout.to(T).contiguous())
+        ws_bytes = lib.cueq_trimul_workspace_bytes(code, Bsz, N, D, Do, 1, int(bits != 0))
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+        _lib.check(lib.cueq_trimul_bwd(code, Bsz, N, D, Do, int(outgoing), x.data_ptr(), _ptr(mask), _pointers(weights), saved.data_ptr(),
+                                       dout.data_ptr(), dx.data_ptr(), bits, _ptr(grads), ws.data_ptr(), ws_bytes, _stream(x)), "cueq_trimul_bwd")
+    out: list = [dx if need[0] else None, None] + [None] * 12
+    if grads is not None:
+        # the order of the gradients in the buffer: norms, input projections (gate, value), output projections, biases
+        sizes = ((0, D), (1, D), (6, D), (7, D), (4, 2 * D * D), (2, 2 * D * D), (10, Do * D), (8, Do * D), (5, 2 * D), (3, 2 * D), (11, Do), (9, Do))
+        for (i, _), g in zip(sizes, grads.split([n for _, n in sizes])):
+            if wanted[i]:
+                out[2 + i] = g.view(weights[i].shape)
+    return out
 
 
 class _TriMul(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, *args):
-        out, saved, dims, has = _trimul_fwd(*args)
-        ctx.save_for_backward(*saved)
-        ctx.outgoing, ctx.dims, ctx.has = args[14], dims, has
+    def forward(ctx, outgoing, eps, x, mask, *weights):
+        out, saved = _trimul_fwd(x, mask, weights, outgoing, eps)
+        ctx.save_for_backward(x, mask, saved, *weights)
+        ctx.outgoing = outgoing
         return out
 
     @staticmethod
     def backward(ctx, dout):
-        return _trimul_bwd(ctx.saved_tensors, ctx.dims, ctx.has, ctx.outgoing, ctx.needs_input_grad, dout)
+        x, mask, saved, *weights = ctx.saved_tensors
+        return (None, None, *_trimul_bwd(x, mask, weights, saved, ctx.outgoing, ctx.needs_input_grad[2:], dout))
 
 
 # ---------------------------------------------------------------------- traced execution (torch.compile / export)
@@ -502,36 +363,27 @@ def _placeholders(ref: torch.Tensor, tensors):
 @torch.library.custom_op("cuequivariance_amd::trimul_fwd", mutates_args=(), device_types="cuda")
 def _trimul_fwd_op(x: torch.Tensor, tensors: List[torch.Tensor], present: List[int], outgoing: bool, eps: float) -> List[torch.Tensor]:
     args = [t if p else None for t, p in zip(tensors, present)]  # mask, then the 12 weights
-    out, saved, _, _ = _trimul_fwd(x, *args, outgoing, eps)
-    return [out, *saved[12:]]  # + xh, mean1, rstd1, ab, t2, mean2, rstd2, y
+    return list(_trimul_fwd(x, args[0], args[1:], outgoing, eps))
 
 
 @_trimul_fwd_op.register_fake
 def _trimul_fwd_fake(x, tensors, present, outgoing, eps):
     Bsz, N, _, D = x.shape
-    M = Bsz * N * N
     Do = tensors[9].shape[0]  # p_out_weight
-    f32 = dict(dtype=torch.float32)
-    return [x.new_empty(Bsz, N, N, Do), x.new_empty(M, D), x.new_empty(M, **f32), x.new_empty(M, **f32), x.new_empty(2 * D, M),
-            x.new_empty(D, M), x.new_empty(M, **f32), x.new_empty(M, **f32), x.new_empty(M, D)]
+    return [x.new_empty(Bsz, N, N, Do),
+            x.new_empty(_lib.load().cueq_trimul_saved_bytes(_CODE[x.dtype], int(Bsz), int(N), int(D), int(Do)), dtype=torch.uint8)]
 
 
 @torch.library.custom_op("cuequivariance_amd::trimul_bwd", mutates_args=(), device_types="cuda")
-def _trimul_bwd_op(dout: torch.Tensor, x: torch.Tensor, tensors: List[torch.Tensor], computed: List[torch.Tensor], present: List[int],
+def _trimul_bwd_op(dout: torch.Tensor, x: torch.Tensor, tensors: List[torch.Tensor], saved: torch.Tensor, present: List[int],
                    need: List[bool], outgoing: bool) -> List[torch.Tensor]:
-    mask, nin_w, nin_b, p_in_w, p_in_b, g_in_w, g_in_b, nout_w, nout_b, p_out_w, p_out_b, g_out_w, g_out_b = [
-        t if p else None for t, p in zip(tensors, present)]
-    Bsz, N, _, D = x.shape
-    M = Bsz * N * N
-    saved = (x.reshape(M, D), None if mask is None else mask.reshape(M), nin_w, p_in_w, p_in_b, g_in_w, g_in_b, nout_w, p_out_w, p_out_b,
-             g_out_w, g_out_b, *computed)
-    has = (nin_w is not None, nin_b is not None, nout_w is not None, nout_b is not None)
-    grads = _trimul_bwd(saved, (Bsz, N, D, p_out_w.shape[0]), has, outgoing, [*need, False, False], dout)
-    return [x.new_empty(0) if (g is None or not n) else g.contiguous() for g, n in zip(grads[:14], need)]
+    args = [t if p else None for t, p in zip(tensors, present)]
+    grads = _trimul_bwd(x, args[0], args[1:], saved, outgoing, need, dout)
+    return [x.new_empty(0) if (g is None or not n) else g.clone() if k > 0 else g for k, (g, n) in enumerate(zip(grads, need))]
 
 
 @_trimul_bwd_op.register_fake
-def _trimul_bwd_fake(dout, x, tensors, computed, present, need, outgoing):
+def _trimul_bwd_fake(dout, x, tensors, saved, present, need, outgoing):
     like = [x, *tensors]
     return [torch.empty_like(t) if (n and (k == 0 or present[k - 1]) and k != 1) else x.new_empty(0) for k, (t, n) in enumerate(zip(like, need))]
 
@@ -539,23 +391,22 @@ def _trimul_bwd_fake(dout, x, tensors, computed, present, need, outgoing):
 def _trimul_setup_context(ctx, inputs, output):
     x, tensors, present, outgoing, eps = inputs
     ctx.present, ctx.outgoing, ctx.ntensors = list(present), outgoing, len(tensors)
-    ctx.save_for_backward(x, *tensors, *output[1:])
+    ctx.save_for_backward(x, *tensors, output[1])
 
 
 def _trimul_autograd(ctx, grads):
     saved = ctx.saved_tensors
-    x, tensors, computed = saved[0], list(saved[1: 1 + ctx.ntensors]), list(saved[1 + ctx.ntensors:])
+    x, tensors = saved[0], list(saved[1: 1 + ctx.ntensors])
     flags = ctx.needs_input_grad[1]
     if isinstance(flags, bool):
         flags = [flags] * len(tensors)
     need = [bool(ctx.needs_input_grad[0]), *[bool(f) for f in flags]]
-    got = _trimul_bwd_op(grads[0], x, tensors, computed, ctx.present, need, ctx.outgoing)
+    got = _trimul_bwd_op(grads[0], x, tensors, saved[1 + ctx.ntensors], ctx.present, need, ctx.outgoing)
     pick = [g if g.numel() > 0 else None for g in got]
     return pick[0], pick[1:], None, None, None
 
 
 torch.library.register_autograd("cuequivariance_amd::trimul_fwd", _trimul_autograd, setup_context=_trimul_setup_context)
-
 
 
 def _lecun_normal(shape, device, dtype) -> torch.Tensor:
@@ -655,5 +506,5 @@ def triangle_multiplicative_update(
         tensors, present = _placeholders(xf, [mf, *args])
         out = _trimul_fwd_op(xf, tensors, present, direction == "outgoing", float(eps))[0]
     else:
-        out = _TriMul.apply(xf, mf, *args, direction == "outgoing", float(eps))
+        out = _TriMul.apply(direction == "outgoing", float(eps), xf, mf, *args)
     return out.view(tuple(lead) + (N, N, Do))

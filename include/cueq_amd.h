@@ -439,22 +439,30 @@ int cueq_layer_norm_t_bwd(int32_t dtype, int64_t M, int64_t D, const void* dy, c
                           const void* gamma, void* dx_t, float* dgamma, float* dbeta, void* workspace, int64_t workspace_bytes,
                           void* stream);
 
-/* out = sigmoid(u + bias_u) * (v + bias_v) * mask on a rows x cols array (u, v float32 accumulators of the two
- * projections); biases (may be NULL) are indexed by row (bias_axis 0) or column (1), the mask (may be NULL)
- * likewise (_sigmoid_gated_dual_gemm.py:135-150).  cueq_gate_bwd returns the gradients of u and v
- * (_sigmoid_gated_dual_gemm.py:153-218). */
-int cueq_gate_fwd(int32_t dtype, int64_t rows, int64_t cols, const float* u, const float* v, const void* bias_u,
-                  const void* bias_v, int32_t bias_axis, const void* mask, int32_t mask_axis, void* out, void* stream);
-int cueq_gate_bwd(int32_t dtype, int64_t rows, int64_t cols, const void* dout, const float* u, const float* v,
-                  const void* bias_u, const void* bias_v, int32_t bias_axis, const void* mask, int32_t mask_axis,
-                  void* du, void* dv, void* stream);
-
 /* Deterministic reductions of a rows x cols array into float32: over columns (one value per row) and over rows
  * (one value per column; workspace of cueq_sum_rows_workspace bytes).  Used for bias and affine gradients. */
 int cueq_sum_cols(int32_t dtype, int64_t rows, int64_t cols, const void* in, float* out, void* stream);
 int64_t cueq_sum_rows_workspace(int64_t rows, int64_t cols);
 int cueq_sum_rows(int32_t dtype, int64_t rows, int64_t cols, const void* in, float* out, void* workspace,
                   int64_t workspace_bytes, void* stream);
+
+/* The whole triangle multiplicative update of pair tensors x (B, N, N, D) -> out (B, N, N, Do), any N, in one call per
+ * direction (cuequivariance_torch/primitives/triangle.py:138-262).  `weights`: host array of 12 device pointers - input
+ * norm weight, bias; value projection p_in weight (2D, D), bias; gate g_in weight, bias; output norm weight, bias; p_out weight
+ * (Do, D), bias; g_out weight, bias; norms and biases may be NULL, and so may `mask` (B, N, N).  x and the weights contiguous and
+ * 16-byte aligned.  `saved` (cueq_trimul_saved_bytes) carries what the backward reads again.  The backward writes dx and, for
+ * the bits set in `need` (bit i = weights[i]), gradients in the element type into `grads` (cueq_trimul_grads_values elements):
+ * norm_in weight, bias, norm_out weight, bias (D each), g_in, p_in (2D x D), g_out, p_out (Do x D), g_in bias, p_in bias (2D),
+ * g_out bias, p_out bias (Do); what was not asked for is left undefined. */
+int64_t cueq_trimul_grads_values(int64_t D, int64_t Do);
+int64_t cueq_trimul_saved_bytes(int32_t dtype, int64_t B, int64_t N, int64_t D, int64_t Do);
+int64_t cueq_trimul_workspace_bytes(int32_t dtype, int64_t B, int64_t N, int64_t D, int64_t Do, int32_t backward, int32_t weight_grads);
+int cueq_trimul_fwd(int32_t dtype, int64_t B, int64_t N, int64_t D, int64_t Do, int32_t outgoing, double eps, const void* x,
+                    const void* mask, const void* const* weights, void* out, void* saved, void* workspace, int64_t workspace_bytes,
+                    void* stream);
+int cueq_trimul_bwd(int32_t dtype, int64_t B, int64_t N, int64_t D, int64_t Do, int32_t outgoing, const void* x, const void* mask,
+                    const void* const* weights, void* saved, const void* dout, void* dx, uint32_t need, void* grads, void* workspace,
+                    int64_t workspace_bytes, void* stream);
 
 #ifdef __cplusplus
 }
