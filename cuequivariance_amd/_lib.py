@@ -289,6 +289,28 @@ def load() -> C.CDLL:
     return _lib
 
 
+_host = None
+
+
+def host():
+    """The host module (``csrc/host``: launch paths and autograd functions in native code), bound to the loaded library."""
+    global _host
+    if _host is None:
+        import torch  # noqa: F401  (the module links against it)
+
+        load()
+        with _lock:
+            if _host is None:
+                try:
+                    from . import _host as module
+                except ImportError as e:
+                    raise ImportError("cuequivariance_amd/_host.so is missing or does not match this PyTorch: build it with "
+                                      f"`python -m cuequivariance_amd.build` ({e})") from e
+                module.load(str(LIB_PATH), CueqError)
+                _host = module
+    return _host
+
+
 _ENV_OPTIONS = (("CUEQ_DETERMINISTIC", b"deterministic"), ("CUEQ_FORCE_GENERIC", b"force_generic"))
 _env_seen: dict = {}
 

@@ -1,0 +1,130 @@
+// The host side of the hot launch paths in native code.  A forward and backward of a small batch costs a few launches; resolving
+// the call, allocating the results and entering the backward in Python took several times as long (and the backward, which
+// PyTorch runs on a thread of its own, had to wait for the interpreter): the step of 622 edges, 50 us of kernels, took 176 us.
+// Everything here falls back to the Python path (by returning None) for calls that are not plain eager ones.
+#include "host.h"
+
+#include <dlfcn.h>
+
+#include <cstdlib>
+#include <list>
+#include <mutex>
+
+#include <torch/csrc/jit/frontend/tracer.h>
+
+namespace cueq_host {
+
+Library& lib() {
+  static Library l;
+  return l;
+}
+
+namespace {
+PyObject* g_error_class = nullptr;
+
+struct EnvOption {
+  const char *env, *option;
+  std::string seen;
+  bool set = false;
+} g_env[] = {{"CUEQ_DETERMINISTIC", "deterministic"}, {"CUEQ_FORCE_GENERIC", "force_generic"}};
+
+void load(const std::string& path, pybind11::object error_class) {
+  void* handle = dlopen(path.c_str(), RTLD_NOW | RTLD_LOCAL);
+  if (!handle) throw std::runtime_error(std::string("cannot load ") + path + ": " + dlerror());
+#define X(name)                                                                  \
+  lib().name = reinterpret_cast<decltype(&::name)>(dlsym(handle, #name));        \
+  if (!lib().name) throw std::runtime_error(path + " has no entry point " #name);
+  CUEQ_HOST_ENTRIES(X)
+#undef X
+  g_error_class = error_class.release().ptr();
+  for (auto& o : g_env) {  // (the library has read the environment itself when it was loaded)
+    const char* v = std::getenv(o.env);
+    o.set = v != nullptr;
+    o.seen = v ? v : "";
+  }
+}
+
+struct CsrEntry {
+  at::Tensor index, offsets, perm;
+  uint32_t version;
+  int64_t nrows;
+};
+std::mutex g_csr_mutex;
+std::list<CsrEntry> g_csr;  // most recently used first
+}  // namespace
+
+void sync_options() {
+  for (auto& o : g_env) {
+    const char* v = std::getenv(o.env);
+    if ((v != nullptr) == o.set && (!v || o.seen == v)) continue;
+    o.set = v != nullptr;
+    o.seen = v ? v : "";
+    lib().cueq_set_option(o.option, v && v[0] == '1' ? 1 : 0);
+  }
+}
+
+bool unwatched() { return !torch::jit::tracer::isTracing() && !c10::impl::TorchDispatchModeTLS::any_modes_set(); }
+
+bool wants_graph(const std::vector<at::Tensor>& tensors) {
+  if (!at::GradMode::is_enabled()) return false;
+  for (const auto& t : tensors)
+    if (t.defined() && t.requires_grad()) return true;
+  return false;
+}
+
+// Eager mode: built once per index tensor and cached (the build checks on the host that the ids are in range and skips the sort when
+// they are sorted already).  While the current stream is being captured into a HIP graph the grouping is recorded into the graph
+// instead (device-side work only, nothing cached), so every replay regroups from whatever the index buffer holds then.  Index
+// tensors made under torch.inference_mode() carry no version counter and are not cached either.
+std::pair<at::Tensor, at::Tensor> segment_csr(const at::Tensor& index, int64_t nrows) {
+  const bool capturing = c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None;
+  const bool cacheable = !capturing && !index.is_inference();
+  const int64_t n = index.numel();
+  if (cacheable) {
+    std::lock_guard<std::mutex> lock(g_csr_mutex);
+    for (auto it = g_csr.begin(); it != g_csr.end(); ++it) {
+      if (it->nrows == nrows && it->version == index._version() && it->index.data_ptr() == index.data_ptr() && it->index.numel() == n &&
+          it->index.scalar_type() == index.scalar_type() && it->index.device() == index.device()) {
+        g_csr.splice(g_csr.begin(), g_csr, it);
+        return {it->offsets, it->perm};
+      }
+    }
+  }
+  const c10::DeviceGuard guard(index.device());
+  at::Tensor offsets = new_tensor({nrows + 1}, at::kLong, index.device()), perm = new_tensor({std::max<int64_t>(n, 1)}, at::kLong, index.device());
+  const int64_t bytes = lib().cueq_segment_csr_workspace(n, nrows);
+  at::Tensor ws = new_tensor({bytes}, at::kByte, index.device());
+  std::optional<pybind11::gil_scoped_release> release;  // (the build waits for two flags)
+  if (PyGILState_Check()) release.emplace();
+  const auto build = capturing ? lib().cueq_segment_csr_build_async : lib().cueq_segment_csr_build;
+  check(build(index.data_ptr(), index.scalar_type() == at::kLong ? 1 : 0, n, nrows, offsets.data_ptr<int64_t>(), perm.data_ptr<int64_t>(), ws.data_ptr(), bytes,
+              stream_of(index.device().index())),
+        "cueq_segment_csr_build");
+  release.reset();
+  if (cacheable) {
+    // (the index tensor is kept alive with the entry so that its address cannot be reused meanwhile)
+    std::list<CsrEntry> old;
+    std::lock_guard<std::mutex> lock(g_csr_mutex);
+    g_csr.push_front({index, offsets, perm, index._version(), nrows});
+    if (g_csr.size() > 32) old.splice(old.begin(), g_csr, std::prev(g_csr.end()));
+  }
+  return {offsets, perm};
+}
+
+}  // namespace cueq_host
+
+PYBIND11_MODULE(_host, m) {
+  namespace py = pybind11;
+  using namespace cueq_host;
+  py::register_exception_translator([](std::exception_ptr p) {
+    try {
+      if (p) std::rethrow_exception(p);
+    } catch (const CueqError& e) {
+      PyErr_SetString(g_error_class ? g_error_class : PyExc_RuntimeError, e.what());
+    }
+  });
+  m.def("load", &load);
+  m.def("segment_csr", &segment_csr);
+  bind_uniform_1d(m);
+  bind_triangle(m);
+}

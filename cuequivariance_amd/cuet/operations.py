@@ -54,6 +54,11 @@ def _transposition_moves(irreps) -> bool:
     return any(mul > 1 and ir.dim > 1 for mul, ir in irreps)
 
 
+def _operator(module: torch.nn.Module):
+    """The host module's operator behind ``module.f`` (a uniform-1d ``SegmentedPolynomial``), or ``None`` while a graph is traced."""
+    return None if torch.compiler.is_compiling() else module._modules["f"]._modules["m"].operator
+
+
 def _default_layout(layout) -> cue.IrrepsLayout:
     if layout is None:
         assumed = cue.get_layout_scope(raising=False)  # (inside ``with cue.assume(layout):``)
@@ -178,6 +183,8 @@ class ChannelWiseTensorProduct(torch.nn.Module):
         self.f = SegmentedPolynomial(
             e.polynomial, method=self.method, math_dtype=math_dtype, options={"segment_groups": groups} if groups else None
         )
+        self._direct = (self.method == "uniform_1d" and self.transpose_in1.is_identity and self.transpose_in2.is_identity
+                        and self.transpose_out.is_identity)
 
     def extra_repr(self) -> str:
         return (
@@ -198,6 +205,13 @@ class ChannelWiseTensorProduct(torch.nn.Module):
         """Arguments as in the reference (``operations/tp_channel_wise.py:186-258``).  Row ids outside ``[0, size_out)`` in ``indices_out`` raise an error in eager mode; while the current stream is being
         captured into a HIP graph the grouping of the batch rows by output row is recorded as device work that cannot report
         them: such batch rows are left out of every output row, at capture and at every replay."""
+        # the whole call in native code when it is a plain one; anything else, and every error, takes the way below
+        w = weight if self.weight is None else (self.weight if weight is None else None)
+        if self._direct and w is not None:
+            op = _operator(self)
+            out = op.product(w, x1, x2, indices_1, indices_2, indices_out, size_out) if op is not None else None
+            if out is not None:
+                return out
         x1 = apply_layout(self.transpose_in1, x1)
         x2 = apply_layout(self.transpose_in2, x2)
         indices_in: Dict[int, torch.Tensor] = {}
@@ -282,6 +296,7 @@ class ChannelWiseSphericalTensorProduct(torch.nn.Module):
         if groups:
             options["segment_groups"] = groups
         self.f = SegmentedPolynomial(polynomial, method="uniform_1d", math_dtype=math_dtype, options=options)
+        self._direct = self.transpose_in1.is_identity and self.transpose_out.is_identity
 
     def extra_repr(self) -> str:
         return f"ls={self.ls}, normalize={self.normalize}, shared_weights={self.shared_weights}, weight_numel={self.weight_numel}"
@@ -298,6 +313,12 @@ class ChannelWiseSphericalTensorProduct(torch.nn.Module):
         torch._assert(vectors.ndim == 2 and vectors.shape[1] == 3, f"vectors must have shape (batch, 3) - got {vectors.shape}")
         if self.normalize:
             vectors = torch.nn.functional.normalize(vectors, dim=1)
+        w = weight if self.weight is None else (self.weight if weight is None else None)
+        if self._direct and w is not None:
+            op = _operator(self)
+            out = op.product(w, x1, vectors, indices_1, None, indices_out, size_out) if op is not None else None
+            if out is not None:
+                return out
         x1 = apply_layout(self.transpose_in1, x1)
         indices_in: Dict[int, torch.Tensor] = {} if indices_1 is None else {1: indices_1}
         indices_o: Dict[int, torch.Tensor] = {}
@@ -590,12 +611,19 @@ class SymmetricContraction(torch.nn.Module):
         )
         self.f = SegmentedPolynomial(self.etp.polynomial, method=self.method, math_dtype=math_dtype,
                                      options={"segment_groups": groups} if groups else None)
+        self._direct = (self.method == "uniform_1d" and self.projection is None and self.transpose_in.is_identity
+                        and self.transpose_out.is_identity)
 
     def extra_repr(self) -> str:
         return f"contraction_degree={self.contraction_degree}, weight_shape={self.weight_shape}"
 
     def forward(self, x: torch.Tensor, indices: torch.Tensor) -> torch.Tensor:
         """``x``: ``(batch, irreps_in.dim)``; ``indices``: ``(batch,)``; returns ``(batch, irreps_out.dim)``."""
+        if self._direct:
+            op = _operator(self)
+            out = op.indexed(self.weight, x, indices) if op is not None else None
+            if out is not None:
+                return out
         if self.projection is not None:
             weight = torch.einsum("zau,ab->zbu", self.weight, self.projection)
         else:
@@ -624,6 +652,10 @@ class SphericalHarmonics(torch.nn.Module):
         torch._assert(vectors.ndim == 2, f"Input must have shape (batch, 3) - got {vectors.shape}")
         if self.normalize:
             vectors = torch.nn.functional.normalize(vectors, dim=1)
+        op = _operator(self)
+        outs = op.call([vectors], [None], [None], [-1]) if op is not None and type(vectors) is torch.Tensor else None
+        if outs is not None:
+            return outs[0]
         [output] = self.f([vectors])
         return output
 

@@ -18,7 +18,7 @@ from typing import Any, Dict, List, Optional
 import torch
 import torch.nn as nn
 
-from .. import cue
+from .. import _lib, cue
 from ..tables import U1dTables
 from . import uniform_1d as u1d
 from .script import scriptable
@@ -122,6 +122,15 @@ class SegmentedPolynomialFromUniform1d(nn.Module):
             plan.polynomial = polynomial  # (lets kernels for symmetric contractions be generated at first use)
             plan.origin = (options or {}).get("origin")  # (the descriptor a flattened fully connected product came from)
 
+    @property
+    def operator(self):
+        """The operator as the host module runs it (``csrc/host/uniform_1d.cpp``); ``None`` for a call it does not take."""
+        op = self.__dict__.get("_operator")
+        if op is None:
+            fixed = {None: -1, torch.float32: 0, torch.float64: 1}[self.math_dtype]
+            op = self.__dict__["_operator"] = _lib.host().U1dOperator(self._plans[torch.float32].native, self._plans[torch.float64].native, fixed)
+        return op
+
     def __reduce__(self):
         return (
             SegmentedPolynomial,
@@ -143,6 +152,14 @@ class SegmentedPolynomialFromUniform1d(nn.Module):
         output_shapes: Dict[int, torch.Tensor],
         output_indices: Dict[int, torch.Tensor],
     ):
+        if not torch.compiler.is_compiling() and all(type(t) in u1d._PLAIN_TENSORS for t in inputs):
+            rows = [-1] * self.num_outputs
+            for pos, shape in output_shapes.items():
+                rows[pos] = shape.size(0)
+            outs = self.operator.call(inputs, [input_indices.get(b) for b in range(self.num_inputs)],
+                                      [output_indices.get(o) for o in range(self.num_outputs)], rows)
+            if outs is not None:
+                return outs
         num_index = 0
         batch_dim = [self.BATCH_DIM_AUTO] * (self.num_inputs + self.num_outputs)
         index_buffer = [-1] * (self.num_inputs + self.num_outputs)

@@ -12,7 +12,7 @@ reference states in the open
     out = sigmoid(xh G_out^T + b) * (y P_out^T + b)       -- the output gate reads the normalised input xh
 
 Forward and backward are one call of the C library each (``cueq_trimul_fwd`` / ``cueq_trimul_bwd``: the stages in order, what
-lives between them in one buffer); torch only owns the buffers.  Inputs float32, bfloat16 or half, fp32 accumulation;
+lives between them in one buffer), made by the host module (``csrc/host/triangle.cpp``); torch only owns the buffers.  Inputs float32, bfloat16 or half, fp32 accumulation;
 intermediate tensors are kept in the input dtype like the reference does; the projection accumulators stay in registers (both
 projections fused with the gate and recomputed in the backward).  The wrappers of the single stages below are what the stages'
 own tests call.
@@ -20,7 +20,6 @@ own tests call.
 
 from __future__ import annotations
 
-import ctypes
 import enum
 import math
 from typing import List, Optional
@@ -282,76 +281,6 @@ def sum_rows(x: torch.Tensor) -> torch.Tensor:
 # ---------------------------------------------------------------------------------------------
 # autograd
 # ---------------------------------------------------------------------------------------------
-def _aligned(t: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
-    """``t`` on a 16-byte boundary (a copy when a view starts elsewhere)."""
-    return t.clone() if t is not None and t.data_ptr() % 16 else t
-
-
-def _pointers(weights):
-    return (ctypes.c_void_p * 12)(*[_ptr(t) for t in weights])
-
-
-def _trimul_fwd(x, mask, weights, outgoing: bool, eps: float):
-    """Forward of the update on ``x (B, N, N, D)`` with the twelve weights (norm_in w, b, p_in w, b, g_in w, b, norm_out w, b,
-    p_out w, b, g_out w, b; ``None`` where absent): the output and the buffer the backward reads (``cueq_trimul_fwd``)."""
-    lib = _lib.load()
-    Bsz, N, _, D = x.shape
-    Do = weights[8].shape[0]
-    code, dev = _CODE[x.dtype], x.device
-    x, weights = _aligned(x), [_aligned(w) for w in weights]
-    out = torch.empty((Bsz, N, N, Do), dtype=x.dtype, device=dev)
-    saved = torch.empty(lib.cueq_trimul_saved_bytes(code, Bsz, N, D, Do), dtype=torch.uint8, device=dev)
-    ws_bytes = lib.cueq_trimul_workspace_bytes(code, Bsz, N, D, Do, 0, 0)
-    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
-    _lib.check(lib.cueq_trimul_fwd(code, Bsz, N, D, Do, int(outgoing), float(eps), x.data_ptr(), _ptr(mask), _pointers(weights), out.data_ptr(),
-                                   saved.data_ptr(), _ptr(ws), ws_bytes, _stream(x)), "cueq_trimul_fwd")
-    return out, saved
-
-
-def _trimul_bwd(x, mask, weights, saved, outgoing: bool, need, dout):
-    """``[dx, None (mask), the twelve weight gradients]`` (``need[k]``: whether argument ``k`` of the list wants one)."""
-    lib = _lib.load()
-    Bsz, N, _, D = x.shape
-    Do = weights[8].shape[0]
-    code, dev, T = _CODE[x.dtype], x.device, x.dtype
-    x, weights = _aligned(x), [_aligned(w) for w in weights]
-    wanted = [bool(n) and w is not None for n, w in zip(need[2:14], weights)]
-    bits = sum(1 << i for i, n in enumerate(wanted) if n)
-    dx = torch.empty_like(x)
-    grads = torch.empty(lib.cueq_trimul_grads_values(D, Do), dtype=T, device=dev) if bits else None
-    if x.numel() == 0:
-        if grads is not None:
-            grads.zero_()
-    else:
-        dout = _aligned(dout.to(T).contiguous())
-        ws_bytes = lib.cueq_trimul_workspace_bytes(code, Bsz, N, D, Do, 1, int(bits != 0))
-        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-        _lib.check(lib.cueq_trimul_bwd(code, Bsz, N, D, Do, int(outgoing), x.data_ptr(), _ptr(mask), _pointers(weights), saved.data_ptr(),
-                                       dout.data_ptr(), dx.data_ptr(), bits, _ptr(grads), ws.data_ptr(), ws_bytes, _stream(x)), "cueq_trimul_bwd")
-    out: list = [dx if need[0] else None, None] + [None] * 12
-    if grads is not None:
-        # the order of the gradients in the buffer: norms, input projections (gate, value), output projections, biases
-        sizes = ((0, D), (1, D), (6, D), (7, D), (4, 2 * D * D), (2, 2 * D * D), (10, Do * D), (8, Do * D), (5, 2 * D), (3, 2 * D), (11, Do), (9, Do))
-        for (i, _), g in zip(sizes, grads.split([n for _, n in sizes])):
-            if wanted[i]:
-                out[2 + i] = g.view(weights[i].shape)
-    return out
-
-
-class _TriMul(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, outgoing, eps, x, mask, *weights):
-        out, saved = _trimul_fwd(x, mask, weights, outgoing, eps)
-        ctx.save_for_backward(x, mask, saved, *weights)
-        ctx.outgoing = outgoing
-        return out
-
-    @staticmethod
-    def backward(ctx, dout):
-        x, mask, saved, *weights = ctx.saved_tensors
-        return (None, None, *_trimul_bwd(x, mask, weights, saved, ctx.outgoing, ctx.needs_input_grad[2:], dout))
-
-
 # ---------------------------------------------------------------------- traced execution (torch.compile / export)
 # Two opaque operators, forward and backward, around the same two functions.  Optional tensors travel as empty
 # placeholders plus a presence list (operator schemas have no optional entries inside tensor lists; the list holds
@@ -363,7 +292,7 @@ def _placeholders(ref: torch.Tensor, tensors):
 @torch.library.custom_op("cuequivariance_amd::trimul_fwd", mutates_args=(), device_types="cuda")
 def _trimul_fwd_op(x: torch.Tensor, tensors: List[torch.Tensor], present: List[int], outgoing: bool, eps: float) -> List[torch.Tensor]:
     args = [t if p else None for t, p in zip(tensors, present)]  # mask, then the 12 weights
-    return list(_trimul_fwd(x, args[0], args[1:], outgoing, eps))
+    return list(_lib.host().trimul_fwd(x, args[0], args[1:], outgoing, eps))
 
 
 @_trimul_fwd_op.register_fake
@@ -378,7 +307,9 @@ def _trimul_fwd_fake(x, tensors, present, outgoing, eps):
 def _trimul_bwd_op(dout: torch.Tensor, x: torch.Tensor, tensors: List[torch.Tensor], saved: torch.Tensor, present: List[int],
                    need: List[bool], outgoing: bool) -> List[torch.Tensor]:
     args = [t if p else None for t, p in zip(tensors, present)]
-    grads = _trimul_bwd(x, args[0], args[1:], saved, outgoing, need, dout)
+    bits = sum(1 << i for i, n in enumerate([need[0], *need[2:14]]) if n)
+    dx, *grads = _lib.host().trimul_bwd(x, args[0], args[1:], saved, outgoing, bits, dout)
+    grads = [dx, None, *grads]
     return [x.new_empty(0) if (g is None or not n) else g.clone() if k > 0 else g for k, (g, n) in enumerate(zip(grads, need))]
 
 
@@ -447,6 +378,12 @@ def triangle_multiplicative_update(
     """
     if direction not in ("outgoing", "incoming"):
         raise ValueError("direction must be either 'outgoing' or 'incoming'")
+    if not torch.compiler.is_compiling() and type(x) in (torch.Tensor, torch.nn.Parameter) and (precision is None or isinstance(precision, int)):
+        # the whole call in native code when every tensor is as the kernels take it; anything else, and every error, below
+        out = _lib.host().trimul_direct(x, mask, [norm_in_weight, norm_in_bias, p_in_weight, p_in_bias, g_in_weight, g_in_bias, norm_out_weight,
+                                                  norm_out_bias, p_out_weight, p_out_bias, g_out_weight, g_out_bias], direction == "outgoing", eps)
+        if out is not None:
+            return out
     if precision is not None and not isinstance(precision, (TriMulPrecision, int)):
         raise ValueError("precision must be a TriMulPrecision or None")
     if x.dim() < 3:
@@ -506,5 +443,5 @@ def triangle_multiplicative_update(
         tensors, present = _placeholders(xf, [mf, *args])
         out = _trimul_fwd_op(xf, tensors, present, direction == "outgoing", float(eps))[0]
     else:
-        out = _TriMul.apply(direction == "outgoing", float(eps), xf, mf, *args)
+        out = _lib.host().trimul(xf, mf, list(args), direction == "outgoing", float(eps))
     return out.view(tuple(lead) + (N, N, Do))

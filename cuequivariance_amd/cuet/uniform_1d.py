@@ -84,7 +84,8 @@ class Uniform1dPlan:
         self.name = name
         self.math_dtype = math_dtype
         self.widths = tuple(tables.width(b) for b in range(tables.num_inputs + tables.num_outputs))
-        self._configs: dict = {}  # resolved call configurations by call shape
+        self._records: dict = {}  # resolved calls by call shape
+        self._native = None
         self._handles: dict[int, int] = {}
         self._backward: dict[tuple, "Uniform1dPlan"] = {}
         self._choice: dict = {}
@@ -111,6 +112,17 @@ class Uniform1dPlan:
     def key(self) -> tuple:
         return (self.math_dtype, self.tables)
 
+    @property
+    def native(self):
+        """The plan as the host module knows it (it owns the device plans)."""
+        if self._native is None:
+            nin = self.num_inputs
+            self._native = _lib.host().U1dPlan(nin, self.num_outputs, list(self.widths), [int(self.dtypes[nin + o]) for o in range(self.num_outputs)],
+                                               self.math_dtype == torch.float64, self)
+        return self._native
+
+    def backward_choice(self, needs: tuple, device: torch.device) -> tuple:
+        return _backward_choice(self, tuple(bool(n) for n in needs), device)
 
     def specialised(self, device: torch.device) -> bool:
         """True when kernels generated for exactly these tables are linked into the library."""
@@ -135,6 +147,7 @@ class Uniform1dPlan:
             out = C.c_void_p()
             with torch.cuda.device(idx):
                 _lib.check(lib.cueq_u1d_plan_create(C.byref(desc), C.byref(out)), "cueq_u1d_plan_create")
+            self.native.adopt(out.value)
             self._handles[idx] = out.value
             if (not _jit.enabled() and self.jit_root is None and not lib.cueq_u1d_plan_info(out.value, None)
                     and (_jit.is_channelwise(self.tables) or _jit.is_symmetric_contraction(self.polynomial))):
@@ -162,14 +175,6 @@ class Uniform1dPlan:
     def serves(self, dtype: torch.dtype) -> bool:
         """True when kernels generated for exactly these tables and buffers of ``dtype`` are registered with the library."""
         return _jit._has_spec(self.tables, _DTYPE_CODE[self.math_dtype], _DTYPE_CODE[dtype])
-
-    def __del__(self):
-        try:
-            lib = _lib.load()
-            for h in self._handles.values():
-                lib.cueq_u1d_plan_destroy(h)
-        except Exception:
-            pass
 
     # ------------------------------------------------------------------ transposition
     def backward_plan(self, needs_grad: tuple) -> "Uniform1dPlan":
@@ -226,219 +231,32 @@ def _cached_plan(plan: Uniform1dPlan) -> Uniform1dPlan:
         return plan
 
 
-# ---------------------------------------------------------------------- CSR cache
-_csr_cache: "OrderedDict[tuple, tuple]" = OrderedDict()
-
-
 def _segment_csr(index: torch.Tensor, nrows: int):
-    """(offsets[nrows+1], perm[n]) grouping batch ids by output row.
-
-    Eager mode: built once per index tensor and cached (the build checks on the host that the ids are in range and
-    skips the sort when they are sorted already).  While the current stream is being captured into a HIP graph the
-    grouping is recorded into the graph instead (device-side work only, nothing cached), so every replay regroups from
-    whatever the index buffer holds then.  Index tensors made under ``torch.inference_mode()`` carry no version counter
-    and are not cached either."""
-    lib = _lib.load()
-    n = index.numel()
-    capturing = torch.cuda.is_current_stream_capturing()
-    cacheable = not capturing and not index.is_inference()
-    if cacheable:
-        key = (index.data_ptr(), index._version, n, int(nrows), index.dtype, index.device)
-        hit = _csr_cache.get(key)
-        if hit is not None:
-            _csr_cache.move_to_end(key)
-            return hit[1], hit[2]
-    offsets = torch.empty(nrows + 1, dtype=torch.int64, device=index.device)
-    perm = torch.empty(max(n, 1), dtype=torch.int64, device=index.device)
-    ws_bytes = lib.cueq_segment_csr_workspace(n, nrows)
-    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=index.device)
-    stream = torch.cuda.current_stream(index.device).cuda_stream
-    build = lib.cueq_segment_csr_build_async if capturing else lib.cueq_segment_csr_build
-    _lib.check(
-        build(index.data_ptr(), 1 if index.dtype == torch.int64 else 0, n, nrows,
-              offsets.data_ptr(), perm.data_ptr(), ws.data_ptr(), ws_bytes, stream),
-        "cueq_segment_csr_build",
-    )
-    if cacheable:
-        # the index tensor is kept alive with the entry so its address cannot be reused meanwhile
-        _csr_cache[key] = (index, offsets, perm)
-        while len(_csr_cache) > 32:
-            _csr_cache.popitem(last=False)
-    return offsets, perm
+    """(offsets[nrows+1], perm[n]) grouping batch ids by output row: cached per index tensor in eager mode, recorded into the
+    graph while the current stream is being captured (``csrc/host/module.cpp``)."""
+    return _lib.host().segment_csr(index, int(nrows))
 
 
 # ---------------------------------------------------------------------- execution
-class _CallConfig:
-    """Resolved batching of one call: per buffer the mode, the index tensor slot and the row count.  Also holds what the
-    launches of this call shape reuse: prepared argument records (by dtype signature) and the configurations of its
-    backward calls."""
-
-    __slots__ = ("modes", "index_of", "rows", "batch", "records", "backward")
-
-    def __init__(self, modes, index_of, rows, batch):
-        self.modes = tuple(modes)
-        self.index_of = tuple(index_of)
-        self.rows = tuple(rows)
-        self.batch = int(batch)
-        self.records: dict = {}
-        self.backward: dict = {}
-
-    def backward_config(self, computed: tuple) -> "_CallConfig":
-        """The configuration of the gradient call for the inputs flagged in ``computed`` (its outputs are their gradients)."""
-        hit = self.backward.get(computed)
-        if hit is None:
-            flagged = [i for i, n in enumerate(computed) if n]
-            hit = self.backward[computed] = _CallConfig(
-                list(self.modes) + [self.modes[i] for i in flagged], list(self.index_of) + [self.index_of[i] for i in flagged],
-                list(self.rows) + [self.rows[i] for i in flagged], self.batch)
-        return hit
+def _record(plan: Uniform1dPlan, modes, index_of, rows, batch: int, tensors: Sequence[torch.Tensor]):
+    """The resolved call for tensors of these shapes and types (inputs, then indices), checked and made once."""
+    nin = plan.num_inputs
+    for b in range(nin):
+        t = tensors[b]
+        if t.dim() != 2 or t.shape[1] != plan.widths[b]:
+            raise ValueError(f"uniform_1d: input {b} has shape {tuple(t.shape)}, expected (rows, {plan.widths[b]})")
+        if t.dtype not in _DTYPE_CODE:
+            raise ValueError(f"uniform_1d: unsupported dtype {t.dtype} for input {b}")
+    for t in tensors:
+        if t.device.type != "cuda":
+            raise RuntimeError("uniform_1d runs on the GPU only; got tensors on " + str(t.device))
+    return _lib.host().U1dRecord(plan.native, [int(m) for m in modes], [int(i) for i in index_of], [int(r) for r in rows], int(batch), list(tensors))
 
 
-class _LaunchRecord:
-    """The argument array of ``cueq_u1d_run`` for one call shape and dtype signature, with every field that does not change
-    from call to call filled in once; a launch writes the data / index / grouping pointers only."""
-
-    __slots__ = ("bufs", "proxies", "out_dtypes")
-
-    def __init__(self, plan: "Uniform1dPlan", cfg: _CallConfig, in_dtypes, idx_dtypes):
-        nin, nout = plan.num_inputs, plan.num_outputs
-        self.bufs = (_lib.U1dBuffer * (nin + nout))()
-        self.proxies = [self.bufs[b] for b in range(nin + nout)]  # (one ctypes proxy per buffer, made once)
-        self.out_dtypes = []
-        for b in range(nin + nout):
-            bb = self.proxies[b]
-            if b < nin:
-                dtype = in_dtypes[b]
-                if dtype not in _DTYPE_CODE:
-                    raise ValueError(f"uniform_1d: unsupported dtype {dtype} for input {b}")
-            else:
-                src = plan.dtypes[b]
-                dtype = plan.math_dtype if src < 0 else in_dtypes[src]
-                self.out_dtypes.append(dtype)
-            bb.rows = cfg.rows[b]
-            bb.dtype = _DTYPE_CODE[dtype]
-            bb.batch_dim = cfg.modes[b]
-            if cfg.modes[b] == BATCH_DIM_INDEXED:
-                bb.index_is_64 = 1 if idx_dtypes[cfg.index_of[b]] == torch.int64 else 0
-
-
-class _NoSwitch:
-    def __enter__(self):
-        return None
-
-    def __exit__(self, *exc):
-        return False
-
-
-_NO_SWITCH = _NoSwitch()
-
-
-def _on_device(device: torch.device):
-    """Context that makes ``device`` current; nothing to do (and nothing to pay) when it already is."""
-    if device.index is None or device.index == torch.cuda.current_device():
-        return _NO_SWITCH
-    return torch.cuda.device(device)
-
-
-def _launch(plan: Uniform1dPlan, cfg: _CallConfig, inputs: Sequence[torch.Tensor],
-            indices: Sequence[torch.Tensor]) -> List[torch.Tensor]:
-    nin, nout = plan.num_inputs, plan.num_outputs
-    device = inputs[0].device if nin else indices[0].device
-    if device.type != "cuda":
-        raise RuntimeError("uniform_1d runs on the GPU only; got tensors on " + str(device))
-    lib = _lib.load()
-    _lib.sync_options_from_env()
-    sig = (tuple([t.dtype for t in inputs]), tuple([i.dtype for i in indices]))
-    pool = cfg.records.get(sig)
-    if pool is None:
-        pool = cfg.records[sig] = []
-    try:
-        rec = pool.pop()  # (a record is used by one launch at a time: list.pop / append are atomic)
-    except IndexError:
-        rec = _LaunchRecord(plan, cfg, sig[0], sig[1])
-        if nin and sig[0][0].itemsize == 2 and all(d == sig[0][0] for d in sig[0]):
-            plan.ensure_io(sig[0][0])
-    modes, widths = cfg.modes, plan.widths
-    with _on_device(device):
-        handle = plan._handles.get(device.index)
-        if handle is None:
-            handle = plan.handle(device)
-        proxies = rec.proxies
-        keep = []
-        for b in range(nin):
-            t = inputs[b]
-            if t.dim() != 2 or t.shape[1] != widths[b]:
-                raise ValueError(f"uniform_1d: input {b} has shape {tuple(t.shape)}, expected (rows, {widths[b]})")
-            if not t.is_contiguous():
-                t = t.contiguous()
-                keep.append(t)
-            bb = proxies[b]
-            bb.data = t.data_ptr()
-            if modes[b] == BATCH_DIM_INDEXED:
-                bb.index = indices[cfg.index_of[b]].data_ptr()
-        outputs = []
-        for o in range(nout):
-            b = nin + o
-            out = torch.empty((cfg.rows[b], widths[b]), dtype=rec.out_dtypes[o], device=device)
-            outputs.append(out)
-            bb = proxies[b]
-            bb.data = out.data_ptr()
-            if modes[b] == BATCH_DIM_INDEXED:
-                idx = indices[cfg.index_of[b]]
-                bb.index = idx.data_ptr()
-                offsets, perm = _segment_csr(idx, cfg.rows[b])
-                keep += [offsets, perm]
-                bb.csr_offsets = offsets.data_ptr()
-                bb.csr_perm = perm.data_ptr()
-        ws_bytes = lib.cueq_u1d_workspace_size(handle, rec.bufs, cfg.batch)
-        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=device) if ws_bytes > 0 else None
-        stream = torch._C._cuda_getCurrentRawStream(device.index if device.index is not None else torch.cuda.current_device())
-        status = lib.cueq_u1d_run(handle, rec.bufs, cfg.batch, ws.data_ptr() if ws is not None else None, ws_bytes, stream)
-        if status != 0:
-            _lib.check(status, f"cueq_u1d_run[{plan.name}]")
-    pool.append(rec)
-    return outputs
-
-
-class _Uniform1dFunction(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, plan: Uniform1dPlan, cfg: _CallConfig, num_index: int, *tensors):
-        nin = plan.num_inputs
-        inputs, indices = tensors[:nin], tensors[nin: nin + num_index]
-        ctx.plan, ctx.cfg, ctx.num_index = plan, cfg, num_index
-        ctx.save_for_backward(*tensors)
-        outs = _launch(plan, cfg, [t.detach() for t in inputs], indices)
-        return tuple(outs)
-
-    @staticmethod
-    def backward(ctx, *grad_outputs):
-        plan, cfg, num_index = ctx.plan, ctx.cfg, ctx.num_index
-        nin, nout = plan.num_inputs, plan.num_outputs
-        tensors = ctx.saved_tensors
-        inputs, indices = tensors[:nin], tensors[nin:]
-        needs = tuple(ctx.needs_input_grad[3: 3 + nin])
-        if not any(needs):
-            return (None,) * (3 + len(tensors))
-        bplan, computed = _backward_choice(plan, needs, inputs[0].device)
-        cots = []
-        for o, g in enumerate(grad_outputs):
-            b = nin + o
-            if g is None:
-                src = plan.dtypes[b]
-                g = torch.zeros((cfg.rows[b], plan.width(b)), device=inputs[0].device,
-                                dtype=plan.math_dtype if src < 0 else inputs[src].dtype)
-            cots.append(g)
-        flagged = [i for i, n in enumerate(computed) if n]
-        bcfg = cfg.backward_config(computed)
-        if torch.is_grad_enabled():  # (create_graph: the gradient call is recorded, derivatives of any order)
-            grads = _Uniform1dFunction.apply(bplan, bcfg, num_index, *inputs, *cots, *indices)
-        else:
-            grads = _launch(bplan, bcfg, [t.detach() for t in inputs] + cots, indices)
-        out = [None, None, None] + [None] * len(tensors)
-        for g, i in zip(grads, flagged):
-            if needs[i]:
-                out[3 + i] = g
-        return tuple(out)
+def _remember(plan: Uniform1dPlan, key, record) -> None:
+    if len(plan._records) >= 64:  # (call shapes of a module are few; a stream of ever new batch sizes starts over)
+        plan._records.clear()
+    plan._records[key] = record
 
 
 # ---------------------------------------------------------------------- traced execution
@@ -448,9 +266,12 @@ class _Uniform1dFunction(torch.autograd.Function):
 def _u1d_launch_op(plan_key: str, modes: List[int], index_of: List[int], rows: List[int], batch: int,
                    tensors: List[torch.Tensor]) -> List[torch.Tensor]:
     plan = _plan_by_key(plan_key)
-    nin = plan.num_inputs
-    outs = _launch(plan, _CallConfig(modes, index_of, rows, batch), [t.detach() for t in tensors[:nin]], tensors[nin:])
-    return list(outs)
+    key = (tuple(modes), tuple(index_of), tuple(rows), batch, tuple([(t.shape, t.dtype, t.device) for t in tensors]))
+    record = plan._records.get(key)
+    if record is None:
+        record = _record(plan, modes, index_of, rows, batch, tensors)
+        _remember(plan, key, record)
+    return record.run([t.detach() for t in tensors])
 
 
 @_u1d_launch_op.register_fake
@@ -515,10 +336,12 @@ def run_plan(plan: Uniform1dPlan, batch_dim: Sequence[int], index_buffer: Sequen
         if not idx.is_contiguous():
             indices[k] = idx.contiguous()
     # the resolution below depends on these numbers only: resolved once per call shape
-    key = (tuple(batch_dim), tuple(index_buffer), batch_size, tuple([t.shape[0] for t in inputs]), tuple([i.shape[0] for i in indices]))
-    cfg = plan._configs.get(key) if not torch.compiler.is_compiling() else None
-    if cfg is not None and inputs and type(inputs[0]) in _PLAIN_TENSORS:
-        return list(_Uniform1dFunction.apply(plan, cfg, num_index, *inputs, *indices))
+    eager = not (torch.compiler.is_compiling() or torch.jit.is_tracing() or (inputs and type(inputs[0]) not in _PLAIN_TENSORS))
+    if eager:
+        key = (tuple(batch_dim), tuple(index_buffer), batch_size, tuple([(t.shape, t.dtype, t.device) for t in (*inputs, *indices)]))
+        record = plan._records.get(key)
+        if record is not None:
+            return record.run([*inputs, *indices])
     modes = list(batch_dim)
     batch = batch_size
     # batch size: the common length of index tensors and of batched (multi-row) inputs
@@ -555,14 +378,11 @@ def run_plan(plan: Uniform1dPlan, batch_dim: Sequence[int], index_buffer: Sequen
     # (traced: under Dynamo, or called with the tracer's tensor subclasses when a composite operator is decomposed)
     if torch.jit.is_tracing():  # (the tracer hands out sizes as tensors: row counts become constants of the trace)
         rows, batch = [int(r) for r in rows], int(batch)
-    if torch.compiler.is_compiling() or torch.jit.is_tracing() or (inputs and type(inputs[0]) not in _PLAIN_TENSORS):
+    if not eager:
         return list(_u1d_launch_op(plan.traced_key, modes, list(index_buffer[: nin + nout]), rows, batch, [*inputs, *indices]))
-    cfg = _CallConfig(modes, list(index_buffer[: nin + nout]), rows, batch)
-    if len(plan._configs) >= 64:  # (call shapes of a module are few; a stream of ever new batch sizes starts over)
-        plan._configs.clear()
-    plan._configs[key] = cfg
-    outs = _Uniform1dFunction.apply(plan, cfg, num_index, *inputs, *indices)
-    return list(outs)
+    record = _record(plan, modes, index_buffer[: nin + nout], rows, batch, [*inputs, *indices])
+    _remember(plan, key, record)
+    return record.run([*inputs, *indices])
 
 
 def uniform_1d(
