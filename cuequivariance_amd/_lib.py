@@ -73,6 +73,10 @@ EXPORTED_SYMBOLS = (
     "cueq_sum_cols",
     "cueq_sum_rows_workspace",
     "cueq_sum_rows",
+    "cueq_linear_flex",
+    "cueq_linear_flex_dw_chunks",
+    "cueq_linear_flex_dw",
+    "cueq_sum_runs",
     "cueq_trimul_grads_values",
     "cueq_trimul_saved_bytes",
     "cueq_trimul_workspace_bytes",
@@ -271,6 +275,14 @@ def load() -> C.CDLL:
         lib.cueq_sum_rows_workspace.restype = i64
         lib.cueq_sum_rows.argtypes = [i32, i64, i64, ptr, ptr, ptr, i64, ptr]
         lib.cueq_sum_rows.restype = C.c_int
+        lib.cueq_linear_flex.argtypes = [i32, i32, i64, ptr, i64, ptr, ptr, i64, ptr, i32, ptr, i32, i32, ptr]
+        lib.cueq_linear_flex.restype = C.c_int
+        lib.cueq_linear_flex_dw_chunks.argtypes = [i64, i32]
+        lib.cueq_linear_flex_dw_chunks.restype = i64
+        lib.cueq_linear_flex_dw.argtypes = [i32, i64, ptr, i64, ptr, i64, ptr, i32, i32, i64, ptr, i32, i32, ptr, ptr]
+        lib.cueq_linear_flex_dw.restype = C.c_int
+        lib.cueq_sum_runs.argtypes = [ptr, i32, i32, ptr, ptr, i32, ptr, ptr]
+        lib.cueq_sum_runs.restype = C.c_int
         lib.cueq_trimul_grads_values.argtypes = [i64, i64]
         lib.cueq_trimul_grads_values.restype = i64
         lib.cueq_trimul_saved_bytes.argtypes = [i32, i64, i64, i64, i64]

@@ -127,4 +127,5 @@ PYBIND11_MODULE(_host, m) {
   m.def("segment_csr", &segment_csr);
   bind_uniform_1d(m);
   bind_triangle(m);
+  bind_linear(m);
 }

@@ -18,6 +18,7 @@ from __future__ import annotations
 
 import ctypes as C
 import json
+import struct
 import threading
 from collections import OrderedDict
 from typing import Dict, List, Optional
@@ -191,32 +192,123 @@ def _merged_weight_gradient(mod: "SegmentedPolynomialDense"):
     return out
 
 
-def _merged_tables(mod: "SegmentedPolynomialDense", device: torch.device):
-    """For the 3-operand form: the column blocks of all paths as parts of table-driven launches, one launch per distinct
-    (K, N, coefficient).  ``fwd``: rows (x offset, weight offset, out offset); ``dx``: rows (g offset, weight offset, dx
-    offset); ``None`` when two parts of one launch would write the same columns (those take the per-group launches)."""
-    key = (device.type, device.index)
-    hit = mod._merged.get(key)
-    if hit is None:
+def _flex_tables(mod: "SegmentedPolynomialDense", mul_ir: bool):
+    """Packed tables of ``csrc/linear_flex.hip`` for the 3-operand form: ``((forward blocks, parts, input-gradient blocks, parts, weight
+    gradients), (column tiles of the two, tiles of the third), element sizes served)``, or ``None``.  Every weight block is used by one
+    run of components: separate blocks at constant strides (``ir_mul``) or one block with the components innermost (``mul_ir``)."""
+    groups = mod.fwd_groups
+    if len({p.w_off for p, *_ in groups}) != len(groups) or sum(K * N for _, K, N in mod.weight_blocks) != mod.input_sizes[0]:
+        return None
+    units = []  # (a0, c0, w_off, K, N, D, coefficient)
+    for p, count, da, dc in groups:
+        if mul_ir:
+            if count not in (1, 3, 5, 7) or (count > 1 and (da != p.K or dc != p.N)):
+                return None
+            units.append((p.a_off, p.c_off, p.w_off, p.K, p.N, count, p.coeff))
+        else:
+            units += [(p.a_off + t * da, p.c_off + t * dc, p.w_off, p.K, p.N, 1, p.coeff) for t in range(count)]
+    served = 0
+    for bit, epv, step in ((1, 4, 8), (2, 8, 16)):  # (float / 2-byte: elements of a 16-byte piece, channels of a step)
+        if (all(v % epv == 0 for u in units for v in u[:3]) and all(u[3] % step == 0 and u[4] % step == 0 for u in units)
+                and mod.input_sizes[1] % epv == 0 and mod.out_size % epv == 0):
+            served |= bit
+    if not served:
+        return None
+
+    def side(result, extent, source, contraction):
         by = {}
-        for p in mod.paths:
-            by.setdefault((p.K, p.N, p.coeff), []).append(p)
-        ok = all(len({p.c_off for p in plist}) == len(plist) and len({p.a_off for p in plist}) == len(plist) for plist in by.values())
-        outs = [p.c_off for p in mod.paths]
-        ins = [p.a_off for p in mod.paths]
-        ok = ok and len(set(outs)) == len(outs) and len(set(ins)) == len(ins)
-        # the table-driven launch moves 16-byte vectors: extents and offsets in multiples of 8 elements
-        ok = ok and all(v % 8 == 0 for p in mod.paths for v in (p.K, p.N, p.a_off, p.c_off, p.w_off))
-        hit = None
-        if ok:
-            hit = [(K, N, coeff,
-                    torch.tensor([(p.a_off, p.w_off, p.c_off) for p in plist], dtype=torch.int64, device=device),
-                    torch.tensor([(p.c_off, p.w_off, p.a_off) for p in plist], dtype=torch.int64, device=device),
-                    _rows_tables(K, N, plist))
-                   for (K, N, coeff), plist in by.items()]
-        mod._merged[key] = hit if hit is not None else False
-        return hit
-    return hit or None
+        for u in units:
+            by.setdefault((u[result], u[extent], u[5]), []).append(u)
+        if len({k[0] for k in by}) != len(by):
+            return None
+        blocks, parts, tiles = b"", b"", 0
+        for (c0, n, d), us in by.items():
+            nt = -(-n // 32)
+            blocks += struct.pack("<q6i", c0, n, d, len(parts) // 24, len(us), nt, 0)
+            tiles += nt
+            for u in us:
+                parts += struct.pack("<qqif", u[source], u[2], u[contraction], u[6])
+        return blocks, parts, tiles
+
+    fwd, dx = side(1, 4, 0, 3), side(0, 3, 1, 4)
+    if fwd is None or dx is None:
+        return None
+    grads, tiles = b"", 0
+    for p, count, da, dc in groups:
+        ntv = -(-p.N // 64)
+        nt = ntv * -(-p.K // 64)
+        d, comps = (count, 1) if mul_ir else (1, count)
+        grads += struct.pack("<3q8ifi", p.a_off, p.c_off, p.w_off, p.K, p.N, d, comps, da, dc, nt, ntv, p.coeff, 0)
+        tiles += nt
+    return (fwd[0], fwd[1], dx[0], dx[1], grads), (fwd[2], dx[2], tiles), served
+
+
+def _rows_launches(mod: "SegmentedPolynomialDense", es: int):
+    """``(forward, input gradient, whether all stream rows)`` launches for rows in ``ir_mul``, or ``None``: one or more launches of
+    ``cueq_linear_rows`` per distinct (K, N, coefficient) - of the tiled ``cueq_gemm_table`` for other extents -, no two parts
+    writing the same columns."""
+    paths = mod.paths
+    if len({p.c_off for p in paths}) != len(paths) or len({p.a_off for p in paths}) != len(paths):
+        return None
+    if any(v % 8 for p in paths for v in (p.K, p.N, p.a_off, p.c_off, p.w_off)):
+        return None
+    by = {}
+    for p in paths:
+        by.setdefault((p.K, p.N, p.coeff), []).append(p)
+    fwd, dx, streaming = [], [], True
+    for (K, N, coeff), plist in by.items():
+        tables = _rows_tables(K, N, plist)
+        if tables is None:
+            streaming = False
+            flat = lambda rows: [v for r in rows for v in r]
+            fwd.append((0, N, K, flat([(p.a_off, p.w_off, p.c_off) for p in plist]), len(plist), coeff))
+            dx.append((0, K, N, flat([(p.c_off, p.w_off, p.a_off) for p in plist]), len(plist), coeff))
+            continue
+        for fwd_host, dx_host, nparts in tables[es]:
+            fwd.append((1, N, K, list(fwd_host), nparts, coeff))
+            dx.append((1, K, N, list(dx_host), nparts, coeff))
+    return fwd, dx, streaming
+
+
+# Rows from which on the row-streaming launches (weights in LDS) are the faster ones for forward and input gradient, by (rows in
+# mul_ir, element size) and multiplicity (up to 32, up to 64, above): where the measured times of the two cross.  Below, a launch is
+# bound by the chain of one wavefront, above by what one CU keeps in flight (128x0e+128x1o+128x2e, 4 000 rows of float: 27 us
+# against 72; 200 000: 804 against 623).  The weight gradient's row launches win from the first row on, but for float in mul_ir.
+_ROWS_FROM = {(False, 4): (15_000, 10_000, 35_000), (False, 2): (30_000, 3_000, 6_000), (True, 4): (50_000, 30_000, 22_000),
+              (True, 2): (50_000, 22_000, 15_000)}
+_GRADS_FROM = {(False, 4): 0, (False, 2): 0, (True, 4): 5_000, (True, 2): 0}
+
+
+def _linear_op(mod: "SegmentedPolynomialDense"):
+    """The 3-operand form as the host module runs it (``csrc/host/linear.cpp``), or ``None`` for shapes its launches do not take."""
+    if mod.has_x2 or mod.method != "fused_tp":
+        return None
+    tables = _flex_tables(mod, mod.rows_mul_ir)
+    if tables is None:
+        return None
+    op = _lib.host().LinearOp(mod.input_sizes[1], mod.out_size, mod.input_sizes[0], mod.rows_mul_ir, mod.dx1_covers_input, mod.fwd_covers_output,
+                              tables[2], tables[0], tables[1])
+    most = max(max(p.K, p.N) for p in mod.paths)
+    for es in (4, 2):
+        rows_from, grads_from = _ROWS_FROM[(mod.rows_mul_ir, es)][0 if most <= 32 else 1 if most <= 64 else 2], _GRADS_FROM[(mod.rows_mul_ir, es)]
+        if mod.rows_mul_ir:
+            if mod.mul_ir is not None and mod.mul_ir.accepts({4: torch.float32, 2: torch.bfloat16}[es]):
+                fwd, dx, dw = mod.mul_ir.tables(es)
+                op.add_rows(es, rows_from, [(d, n, k, list(t), parts, c) for d, n, k, t, parts, c in fwd],
+                            [(d, n, k, list(t), parts, c) for d, n, k, t, parts, c in dx])
+                op.add_grads(es, grads_from, [(K, N, c, 0, 0, 0, 0, list(t), list(w), [1] * len(w)) for K, N, c, t, _, w in dw])
+            continue
+        launches = _rows_launches(mod, es)
+        if launches is not None:
+            fwd, dx, streaming = launches
+            op.add_rows(es, rows_from if streaming else 2_000, fwd, dx)
+        merged = _merged_weight_gradient(mod)
+        if merged is not None:
+            K, N, coeff, a0, c0, da, dc, runs = merged
+            op.add_grads(es, grads_from, [(K, N, coeff, a0, c0, da, dc, [], [w for w, _ in runs], [n for _, n in runs])])
+        else:
+            op.add_grads(es, grads_from, [(p.K, p.N, p.coeff, p.a_off, p.c_off, da, dc, [], [p.w_off], [count]) for p, count, da, dc in mod.fwd_groups])
+    return op
 
 
 def _rows_tables(K: int, N: int, plist):
@@ -341,72 +433,6 @@ class _MulIrPlan:
         return self._tables[es]
 
 
-def _run_mul_ir(dtype, A, W, Cout, launches, forward: bool):
-    """Forward (``W`` blocks ``K x N`` as they lie) or input gradient (the same blocks read as ``N x K``) of the ``mul_ir``
-    parts: ``Cout[z, c0 + v d + i] = coeff * sum_u A[z, a0 + u d + i] W[u, v]``."""
-    lib = _lib.load()
-    stream = torch.cuda.current_stream(A.device).cuda_stream
-    code = _DTYPE_CODE[dtype]
-    for d, n_res, k_con, table, nparts, coeff in launches:
-        if d == 1:
-            _lib.check(lib.cueq_linear_rows(code, 1 if forward else 0, A.shape[0], n_res, k_con, A.data_ptr(), A.stride(0), W.data_ptr(), W.numel(),
-                                            Cout.data_ptr(), Cout.stride(0), table, nparts, coeff, stream), "cueq_linear_rows")
-        else:
-            _lib.check(lib.cueq_linear_rows_mul_ir(code, 1 if forward else 0, A.shape[0], n_res, k_con, A.data_ptr(), A.stride(0), W.data_ptr(),
-                                                   W.numel(), Cout.data_ptr(), Cout.stride(0), table, nparts, coeff, stream),
-                       "cueq_linear_rows_mul_ir")
-
-
-def _weight_gradient_mul_ir(dtype, x, g, numel, launches):
-    """``dW`` (float32, flat) of the ``mul_ir`` parts: chunked partial products, then one ordered row sum per block."""
-    lib = _lib.load()
-    stream = torch.cuda.current_stream(x.device).cuda_stream
-    code = _DTYPE_CODE[dtype]
-    gw32 = torch.zeros(numel, dtype=torch.float32, device=x.device)
-    for K, N, coeff, table, nparts, w_offs in launches:
-        first = (C.c_int32 * (nparts + 1))()
-        items = lib.cueq_linear_dw_mul_ir_items(x.shape[0], table, nparts, first)
-        part = torch.empty(items, K * N, dtype=torch.float32, device=x.device)
-        _lib.check(lib.cueq_linear_dw_mul_ir(code, K, N, x.shape[0], x.data_ptr(), x.stride(0), g.data_ptr(), g.stride(0), table, nparts,
-                                             part.data_ptr(), coeff, stream), "cueq_linear_dw_mul_ir")
-        ws_bytes = max(lib.cueq_sum_rows_workspace(first[p + 1] - first[p], K * N) for p in range(nparts))
-        ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=x.device)
-        for p, w_off in enumerate(w_offs):
-            rows = part[first[p]: first[p + 1]]
-            _lib.check(lib.cueq_sum_rows(_lib.F32, rows.shape[0], K * N, rows.data_ptr(), gw32[w_off: w_off + K * N].data_ptr(), ws.data_ptr(),
-                                         ws_bytes, stream), "cueq_sum_rows")
-    return gw32
-
-
-def _vector_rows(*tensors) -> bool:
-    return all(t.data_ptr() % 16 == 0 and (t.dim() < 2 or (t.stride(0) * t.element_size()) % 16 == 0) for t in tensors)
-
-
-def _run_merged(dtype, A, B, Cout, launches, forward: bool):
-    """``Cout[:, c : c + N] = coeff * A[:, a : a + K] @ W_p`` (forward, W_p is K x N as it lies) or
-    ``Cout[:, a : a + K] = coeff * A[:, c : c + N] @ W_p^T`` (input gradient) for all parts of a launch at once."""
-    lib = _lib.load()
-    stream = torch.cuda.current_stream(A.device).cuda_stream
-    code = _DTYPE_CODE[dtype]
-    for K, N, coeff, fwd_tab, dx_tab, rows in launches:
-        if rows is not None and dtype in _MATRIX_CORE:
-            for fwd_host, dx_host, nparts in rows[A.element_size()]:
-                if forward:
-                    _lib.check(lib.cueq_linear_rows(code, 1, A.shape[0], N, K, A.data_ptr(), A.stride(0), B.data_ptr(), B.numel(), Cout.data_ptr(),
-                                                    Cout.stride(0), fwd_host, nparts, coeff, stream), "cueq_linear_rows")
-                else:
-                    _lib.check(lib.cueq_linear_rows(code, 0, A.shape[0], K, N, A.data_ptr(), A.stride(0), B.data_ptr(), B.numel(), Cout.data_ptr(),
-                                                    Cout.stride(0), dx_host, nparts, coeff, stream), "cueq_linear_rows")
-        elif forward:
-            _lib.check(lib.cueq_gemm_table(code, code, 0, 1, A.shape[0], N, K, A.data_ptr(), A.stride(0), B.data_ptr(), N,
-                                           Cout.data_ptr(), Cout.stride(0), fwd_tab.data_ptr(), fwd_tab.shape[0], 1, 0, coeff, 0, stream),
-                       "cueq_gemm_table")
-        else:
-            _lib.check(lib.cueq_gemm_table(code, code, 0, 0, A.shape[0], K, N, A.data_ptr(), A.stride(0), B.data_ptr(), N,
-                                           Cout.data_ptr(), Cout.stride(0), dx_tab.data_ptr(), dx_tab.shape[0], 1, 0, coeff, 0, stream),
-                       "cueq_gemm_table")
-
-
 def _run_tiled(dtype, A, a_key, B_of, Cout, c_key, groups, Kdim, Ndim):
     """``Cout[:, c : c + N] (+)= coeff * A[:, a : a + K] @ B^T`` per group through the 128 x 128 tiled MFMA kernel
     (``cueq_gemm_nt``; ``B_of(path)`` gives the pointer of the ``N x K`` block)."""
@@ -439,16 +465,9 @@ class _DenseFunction(torch.autograd.Function):
         wd = w.detach().to(dtype).contiguous()
         x1d = x1.detach().contiguous()
         x2d = x2.detach().contiguous() if x2 is not None else None
-        if Z > 0 and mod.rows_mul_ir:
-            x1d, wd = _aligned(x1d), _aligned(wd)
+        if Z > 0:
             with torch.cuda.device(x1.device):
-                _run_mul_ir(dtype, x1d, wd, out, mod.mul_ir.tables(x1d.element_size())[0], True)
-        elif Z > 0:
-            with torch.cuda.device(x1.device):
-                merged = _merged_tables(mod, x1.device) if (mod.tiled(dtype, x1d, out) and _vector_rows(x1d, wd, out)) else None
-                if merged is not None:
-                    _run_merged(dtype, x1d, wd, out, merged, True)
-                elif mod.tiled(dtype, x1d, out):
+                if mod.tiled(dtype, x1d, out):
                     # out[:, k_seg] (+)= c * x1[:, i_seg] @ W_p: the kernel wants W_p^T (N x K, contraction contiguous)
                     wt = mod.transposed_weights(wd)
                     es = wd.element_size()
@@ -497,13 +516,8 @@ class _DenseFunction(torch.autograd.Function):
             if needs_input_grad[2]:
                 # dx1[:, i_seg] += c * x2[:, j] * g[:, k_seg] @ W_p^T
                 gx1 = (torch.empty_like if mod.dx1_covers_input else torch.zeros_like)(x1d)
-                if Z > 0 and mod.rows_mul_ir:
-                    _run_mul_ir(dtype, _aligned(g), _aligned(wd), gx1, mod.mul_ir.tables(g.element_size())[1], False)
-                elif Z > 0:
-                    merged = _merged_tables(mod, x1.device) if (mod.tiled(dtype, g, gx1) and _vector_rows(g, wd, gx1)) else None
-                    if merged is not None:
-                        _run_merged(dtype, g, wd, gx1, merged, False)
-                    elif mod.tiled(dtype, g, gx1):
+                if Z > 0:
+                    if mod.tiled(dtype, g, gx1):
                         # dx1[:, i_seg] (+)= c * g[:, k_seg] @ W_p^T: W_p (K x N) is already "N x K" for this product
                         es = wd.element_size()
                         _run_tiled(dtype, g, lambda p: p.c_off, lambda p: wd.data_ptr() + p.w_off * es, gx1, lambda p: p.a_off,
@@ -512,35 +526,13 @@ class _DenseFunction(torch.autograd.Function):
                         _run_gemms(dtype, g, wd, x2d, gx1, tables.dx1)
             if needs_input_grad[1]:
                 gwd = None
-                if Z > 0 and mod.rows_mul_ir:
-                    gwd = _weight_gradient_mul_ir(dtype, _aligned(x1d), _aligned(g), wd.numel(), mod.mul_ir.tables(x1d.element_size())[2]).view(wd.shape)
-                elif Z > 0 and mod.tiled(dtype, x1d, g):
+                if Z > 0 and mod.tiled(dtype, x1d, g):
                     # dW_p[k][n] += c * sum_z x1[z, i_seg + k] g[z, k_seg + n]: chunked partial products, ordered sum
                     # straight into a float32 image of the weights (a block met a second time is added)
                     code, es = _DTYPE_CODE[dtype], x1d.element_size()
                     gw32 = torch.zeros(wd.numel(), dtype=torch.float32, device=x1.device)
                     written = set()
-                    merged = _merged_weight_gradient(mod)
-                    if merged is not None:
-                        # every component of every block in one launch (the partial products of a block's components are
-                        # consecutive rows of `part`), then one ordered row sum per block
-                        K, N, coeff, a0, c0, da, dc, runs = merged
-                        nparts = sum(n for _, n in runs)
-                        items = lib.cueq_gemm_tn_items(Z, nparts)
-                        chunks = items // nparts
-                        part = torch.empty(items, K * N, dtype=torch.float32, device=x1.device)
-                        _lib.check(
-                            lib.cueq_gemm_tn(code, K, N, Z, x1d.data_ptr() + a0 * es, x1d.stride(0), da, g.data_ptr() + c0 * es,
-                                             g.stride(0), dc, nparts, part.data_ptr(), coeff, stream), "cueq_gemm_tn")
-                        first_part = 0
-                        for w_off, n in runs:
-                            rows = part[first_part * chunks: (first_part + n) * chunks]
-                            ws_bytes = lib.cueq_sum_rows_workspace(n * chunks, K * N)
-                            ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=x1.device)
-                            _lib.check(lib.cueq_sum_rows(_lib.F32, n * chunks, K * N, rows.data_ptr(), gw32[w_off: w_off + K * N].data_ptr(),
-                                                         ws.data_ptr(), ws_bytes, stream), "cueq_sum_rows")
-                            first_part += n
-                    for p, count, da, dc in (mod.fwd_groups if merged is None else []):
+                    for p, count, da, dc in mod.fwd_groups:
                         items = lib.cueq_gemm_tn_items(Z, count)
                         part = torch.empty(items, p.K * p.N, dtype=torch.float32, device=x1.device)
                         _lib.check(
@@ -1153,7 +1145,10 @@ def _remember_traced(key: str, mod: "SegmentedPolynomialDense") -> None:
 
 @torch.library.custom_op("cuequivariance_amd::dense_fwd", mutates_args=(), device_types="cuda")
 def _dense_fwd_op(mod_key: str, kind: int, w: torch.Tensor, x1: torch.Tensor, x2: Optional[torch.Tensor]) -> torch.Tensor:
-    return _FUNCTIONS[kind].forward(_PlainContext(), _module_by_key(mod_key), w, x1, x2)
+    mod = _module_by_key(mod_key)
+    if mod.linear_takes(x1, x2):
+        return mod.linear.forward(w.detach(), x1.detach())
+    return _FUNCTIONS[kind].forward(_PlainContext(), mod, w, x1, x2)
 
 
 @_dense_fwd_op.register_fake
@@ -1168,7 +1163,10 @@ def _dense_bwd_op(mod_key: str, kind: int, w: torch.Tensor, x1: torch.Tensor, x2
     ctx.mod, ctx.has_x2 = _module_by_key(mod_key), x2 is not None
     ctx.saved_tensors = (w, x1, x2 if (x2 is not None or kind == 1) else torch.empty(0))
     ctx.needs_input_grad = (False, *need)
-    if kind == 0:
+    if ctx.mod.linear_takes(x1, x2):
+        op, g = ctx.mod.linear, g.detach()
+        grads = (op.dw(x1.detach(), g, w) if need[0] else None, op.dx(w.detach(), g, x1) if need[1] else None, None)
+    elif kind == 0:
         grads = _DenseFunction._backward_impl(ctx, g, ctx.needs_input_grad)[1:4]
     else:
         grads = _FcFunction.grads(ctx.mod, w, x1, x2, g, *ctx.needs_input_grad[1:4])
@@ -1253,11 +1251,13 @@ class SegmentedPolynomialDense(nn.Module):
         # 4-operand form: `row_blocks` = ([(mul, d)] of the first operand, [(mul, d)] of the output); the generated fused kernels
         # take such rows apart / put them together in registers, other executors of this module do not take them.
         self.mul_ir, self.fc_blocks = None, None
+        self.rows_mul_ir = rows == "mul_ir"
+        self._linear = False
         if rows == "mul_ir" and not self.has_x2:
             self.mul_ir = _MulIrPlan.build(self)
-            if self.mul_ir is None:
+            if self.mul_ir is None and _flex_tables(self, True) is None:
                 raise NotImplementedError("fused_tp: rows='mul_ir' needs a Linear-like polynomial with blocks of 1, 3, 5 or 7 components "
-                                          "and multiplicities 32, 64, 96 or 128")
+                                          "and multiplicities that are multiples of 8")
         elif rows == "mul_ir":
             def starts(blocks, size):
                 out, off = [], 0
@@ -1271,7 +1271,6 @@ class SegmentedPolynomialDense(nn.Module):
             if row_blocks is None:
                 raise NotImplementedError("fused_tp: rows='mul_ir' of a 4-operand contraction needs row_blocks")
             self.fc_blocks = (starts(row_blocks[0], self.input_sizes[1]), starts(row_blocks[1], self.out_size))
-        self.rows_mul_ir = rows == "mul_ir"
         # the text under which a traced graph names this module: the arguments it was built from
         self.traced_key = json.dumps({
             "polynomial": polynomial.pack(), "math_dtype": None if math_dtype is None else str(math_dtype).split(".")[-1],
@@ -1296,12 +1295,26 @@ class SegmentedPolynomialDense(nn.Module):
                                                           _FC_ELEMENT[dtype], blocks[0], blocks[1])
         return self._fused[key]
 
+    @property
+    def linear(self):
+        """The 3-operand form as the host module runs it, or ``None``."""
+        if self._linear is False:
+            self._linear = _linear_op(self)
+        return self._linear
+
+    def linear_takes(self, x1, x2) -> bool:
+        return x2 is None and x1.dtype in _MATRIX_CORE and self.linear is not None and self.linear.takes(x1)
+
+    def rows_accepted(self, dtype) -> bool:
+        """``rows="mul_ir"`` of the 3-operand form: whether rows of this type are taken as they lie."""
+        return dtype in _MATRIX_CORE and self.linear is not None and self.linear.takes(torch.empty(0, dtype=dtype))
+
     def mul_ir_ready(self, dtype) -> bool:
         """Whether rows in ``mul_ir`` can be taken as they lie for this dtype."""
         if not self.rows_mul_ir:
             return False
-        if self.mul_ir is not None:
-            return self.mul_ir.accepts(dtype)
+        if not self.has_x2:
+            return self.rows_accepted(dtype)
         if dtype not in _MATRIX_CORE or not self.fc_plan.ok:
             return False
         from .. import jit
@@ -1380,7 +1393,7 @@ class SegmentedPolynomialDense(nn.Module):
             raise NotImplementedError("fused_tp: weights must be shared over the batch (one row)")
         if x1.dtype not in _DTYPE_CODE:
             raise ValueError(f"fused_tp: unsupported dtype {x1.dtype}")
-        if self.rows_mul_ir and self.mul_ir is not None and not self.mul_ir.accepts(x1.dtype):
+        if self.rows_mul_ir and not self.has_x2 and not self.rows_accepted(x1.dtype):
             raise NotImplementedError(f"fused_tp: rows='mul_ir' does not take {x1.dtype} with these multiplicities")
         if self.rows_mul_ir and self.fc_blocks is not None and not self.mul_ir_ready(x1.dtype):
             raise NotImplementedError("fused_tp: rows='mul_ir' of a fully connected product runs on the generated fused kernels only "
@@ -1400,4 +1413,8 @@ class SegmentedPolynomialDense(nn.Module):
             return [self.forward([w.float(), x1.float(), x2.float()], input_indices, output_shapes, output_indices)[0].to(torch.float16)]
         if x2 is not None and self.fc_plan.ok and x1.dtype in _MATRIX_CORE:
             return [_apply_dense(1, self, w, x1, x2)]
+        if x2 is None and not torch.compiler.is_compiling() and self.linear_takes(x1, x2):
+            out = self.linear.direct(w, x1)
+            if out is not None:
+                return [out]
         return [_apply_dense(0, self, w, x1, x2)]

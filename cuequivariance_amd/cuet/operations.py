@@ -514,6 +514,17 @@ class Linear(torch.nn.Module):
             except NotImplementedError:
                 self.f_rows = None
 
+    def _linear_op(self):
+        """The host module's operator for rows in this module's layouts, or ``None``."""
+        if self.method != "fused_tp":
+            return None
+        if self.f_rows is not None:
+            return self.f_rows._modules["m"].dense.linear
+        if not (self.transpose_in.is_identity and self.transpose_out.is_identity):
+            return None
+        dense = getattr(self.f._modules["m"], "dense", None)
+        return dense.linear if dense is not None else None
+
     def extra_repr(self) -> str:
         return (
             f"shared_weights={self.shared_weights}, internal_weights={self.internal_weights}, "
@@ -534,8 +545,14 @@ class Linear(torch.nn.Module):
             input_indices[0] = weight_indices
         if weight is None:
             raise ValueError("Weights should not be None")
+        if not input_indices and not torch.compiler.is_compiling():
+            # the whole call in native code when it is a plain one; anything else, and every error, takes the way below
+            op = self._linear_op()
+            out = op.direct(weight, x) if op is not None else None
+            if out is not None:
+                return out
         if (self.f_rows is not None and not input_indices and weight.shape[0] == 1 and x.is_cuda and x.dtype == weight.dtype
-                and self.f_rows.m.dense.mul_ir.accepts(x.dtype)):
+                and self.f_rows.m.dense.rows_accepted(x.dtype)):
             return self.f_rows([weight, x])[0]
         if self.method != "indexed_linear" and (input_indices or weight.shape[0] != 1):
             out = self.f_per_sample([weight, apply_layout(self.transpose_in, x)], input_indices)

@@ -446,6 +446,26 @@ int64_t cueq_sum_rows_workspace(int64_t rows, int64_t cols);
 int cueq_sum_rows(int32_t dtype, int64_t rows, int64_t cols, const void* in, float* out, void* workspace,
                   int64_t workspace_bytes, void* stream);
 
+/* Equivariant Linear for batches that do not fill the chip with the row-streaming launches, any number of input blocks per block
+ * of the result: C[z, c0 + v D + i] = sum over the block's parts of coeff sum_u A[z, a0 + u D + i] W[w0 + u N + v] - with
+ * transposed_weights W[w0 + v K + u], K the contraction length.  `blocks` and `parts` are device tables (FlexBlock, FlexPart of csrc/linear_flex.hip:
+ * {int64 c0; int32 N, D, first part, parts, column tiles of 32, unused} and {int64 a0, w0; int32 contraction length; float coeff});
+ * contraction lengths multiples of 8 (float32) / 16, N of 4, D 1, 3, 5 or 7, offsets of 16 bytes.  mul_ir only names the timer. */
+int cueq_linear_flex(int32_t dtype, int32_t transposed_weights, int64_t rows, const void* A, int64_t lda, const void* W, void* C,
+                     int64_t ldc, const void* blocks, int32_t nblocks, const void* parts, int32_t column_tiles, int32_t mul_ir,
+                     void* stream);
+/* Its weight gradient, dW[w0 + u N + v] = coeff sum_z sum_i x[z, a0 + ..] g[z, c0 + ..] for every entry of the device table
+ * `grads` ({int64 a0, c0, w0; int32 K, N, D, components, stride in x, stride in g, tiles of 64 x 64, tiles along N; float coeff}),
+ * partial products per row chunk (float32, chunks x numel in `partial`) summed in order and rounded to out_dtype. */
+int64_t cueq_linear_flex_dw_chunks(int64_t rows, int32_t tiles);
+int cueq_linear_flex_dw(int32_t dtype, int64_t rows, const void* X, int64_t ldx, const void* G, int64_t ldg, const void* grads,
+                        int32_t ngrads, int32_t tiles, int64_t numel, float* partial, int32_t mul_ir, int32_t out_dtype, void* dW,
+                        void* stream);
+/* Ordered sums of consecutive rows of `partial` (float32, `per` values a row): out[w0[b] .. + per) = rows first[b] ..
+ * first[b + 1] (first: nruns + 1 host integers), rounded to out_dtype. */
+int cueq_sum_runs(const float* partial, int32_t per, int32_t nruns, const int32_t* first, const int64_t* w0, int32_t out_dtype,
+                  void* out, void* stream);
+
 /* The whole triangle multiplicative update of pair tensors x (B, N, N, D) -> out (B, N, N, Do), any N, in one call per
  * direction (cuequivariance_torch/primitives/triangle.py:138-262).  `weights`: host array of 12 device pointers - input
  * norm weight, bias; value projection p_in weight (2D, D), bias; gate g_in weight, bias; output norm weight, bias; p_out weight
