@@ -77,6 +77,10 @@ EXPORTED_SYMBOLS = (
     "cueq_linear_flex_dw_chunks",
     "cueq_linear_flex_dw",
     "cueq_sum_runs",
+    "cueq_fc_flex",
+    "cueq_fc_flex_dw_chunks",
+    "cueq_fc_flex_dw",
+    "cueq_fc_factors",
     "cueq_trimul_grads_values",
     "cueq_trimul_saved_bytes",
     "cueq_trimul_workspace_bytes",
@@ -283,6 +287,14 @@ def load() -> C.CDLL:
         lib.cueq_linear_flex_dw.restype = C.c_int
         lib.cueq_sum_runs.argtypes = [ptr, i32, i32, ptr, ptr, i32, ptr, ptr]
         lib.cueq_sum_runs.restype = C.c_int
+        lib.cueq_fc_flex.argtypes = [i32, i32, i32, i64, ptr, i64, ptr, ptr, i64, ptr, i64, ptr, i64, ptr, i32, ptr, ptr, i32, i32, i32, ptr, ptr, ptr]
+        lib.cueq_fc_flex.restype = C.c_int
+        lib.cueq_fc_flex_dw_chunks.argtypes = [i64, i32]
+        lib.cueq_fc_flex_dw_chunks.restype = i64
+        lib.cueq_fc_flex_dw.argtypes = [i32, i32, i64, ptr, i64, ptr, i64, ptr, i64, ptr, i32, ptr, i32, i64, ptr, ptr]
+        lib.cueq_fc_flex_dw.restype = C.c_int
+        lib.cueq_fc_factors.argtypes = [i32, i32, i64, ptr, i64, ptr, i64, ptr, i64, ptr, i32, ptr, ptr, i32, i32, ptr, i64, ptr, ptr]
+        lib.cueq_fc_factors.restype = C.c_int
         lib.cueq_trimul_grads_values.argtypes = [i64, i64]
         lib.cueq_trimul_grads_values.restype = i64
         lib.cueq_trimul_saved_bytes.argtypes = [i32, i64, i64, i64, i64]

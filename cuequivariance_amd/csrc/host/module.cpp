@@ -128,4 +128,5 @@ PYBIND11_MODULE(_host, m) {
   bind_uniform_1d(m);
   bind_triangle(m);
   bind_linear(m);
+  bind_fully_connected(m);
 }

@@ -180,29 +180,35 @@ struct FlexGrad {
   float coeff;
 };
 
-template <typename TI, int D>
+// NT x NT tiles of 32 x 32: one for blocks of at most 32 channels (a 64 x 64 tile would be three quarters padding), four otherwise
+template <typename TI, int D, int NT>
 __device__ __forceinline__ void flex_grad_tile(const FlexGrad& q, int tile, const TI* __restrict__ X, int64_t ldx, const TI* __restrict__ G, int64_t ldg,
                                                float* __restrict__ P, int64_t zb, int64_t ze) {
   constexpr int ES = sizeof(TI), ROWS = ES == 4 ? 2 : 16;  // rows (contraction) per matrix instruction
   const int lane = threadIdx.x & 63, c = lane & 31, h = lane >> 5;
   const int u0 = (tile / q.ntv) * 64, v0 = (tile % q.ntv) * 64;
-  fx16 acc[2][2];
+  fx16 acc[NT][NT];
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
+  for (int a = 0; a < NT; ++a)
 #pragma unroll
-    for (int b = 0; b < 2; ++b) acc[a][b] = fx16{0};
-  const int u[2] = {min(u0 + c, q.K - 1), min(u0 + 32 + c, q.K - 1)}, v[2] = {min(v0 + c, q.N - 1), min(v0 + 32 + c, q.N - 1)};
+    for (int b = 0; b < NT; ++b) acc[a][b] = fx16{0};
+  int u[NT], v[NT];
+#pragma unroll
+  for (int a = 0; a < NT; ++a) {
+    u[a] = min(u0 + 32 * a + c, q.K - 1);
+    v[a] = min(v0 + 32 * a + c, q.N - 1);
+  }
   for (int comp = 0; comp < q.comps; ++comp) {
     const TI *xp = X + q.a0 + static_cast<int64_t>(comp) * q.sa, *gp = G + q.c0 + static_cast<int64_t>(comp) * q.sc;
     if constexpr (ES == 4) {
       constexpr int U = D == 1 ? 8 : D == 3 ? 4 : 2;  // row pairs in flight
       for (int64_t z = zb; z < ze; z += 2 * U) {
-        float xa[U][2][D], ga[U][2][D];
+        float xa[U][NT][D], ga[U][NT][D];
 #pragma unroll
         for (int s = 0; s < U; ++s) {
           const int64_t zz = z + 2 * s + h, zr = min(zz, ze - 1);
 #pragma unroll
-          for (int a = 0; a < 2; ++a)
+          for (int a = 0; a < NT; ++a)
 #pragma unroll
             for (int i = 0; i < D; ++i) {
               const float xv = xp[zr * ldx + u[a] * D + i], gv = gp[zr * ldg + v[a] * D + i];
@@ -215,18 +221,18 @@ __device__ __forceinline__ void flex_grad_tile(const FlexGrad& q, int tile, cons
 #pragma unroll
           for (int i = 0; i < D; ++i)
 #pragma unroll
-            for (int a = 0; a < 2; ++a)
+            for (int a = 0; a < NT; ++a)
 #pragma unroll
-              for (int b = 0; b < 2; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(xa[s][a][i], ga[s][b][i], acc[a][b], 0, 0, 0);
+              for (int b = 0; b < NT; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(xa[s][a][i], ga[s][b][i], acc[a][b], 0, 0, 0);
       }
     } else {
       const uint16_t *xq = reinterpret_cast<const uint16_t*>(xp), *gq = reinterpret_cast<const uint16_t*>(gp);
       for (int64_t z = zb; z < ze; z += ROWS) {
 #pragma unroll 1
         for (int i = 0; i < D; ++i) {
-          uint4 xa[2], ga[2];
+          uint4 xa[NT], ga[NT];
 #pragma unroll
-          for (int a = 0; a < 2; ++a) {
+          for (int a = 0; a < NT; ++a) {
             uint32_t ex[8], eg[8];
 #pragma unroll
             for (int s = 0; s < 8; ++s) {
@@ -239,17 +245,17 @@ __device__ __forceinline__ void flex_grad_tile(const FlexGrad& q, int tile, cons
             ga[a] = make_uint4(eg[0] | eg[1] << 16, eg[2] | eg[3] << 16, eg[4] | eg[5] << 16, eg[6] | eg[7] << 16);
           }
 #pragma unroll
-          for (int a = 0; a < 2; ++a)
+          for (int a = 0; a < NT; ++a)
 #pragma unroll
-            for (int b = 0; b < 2; ++b) acc[a][b] = mm_32x32x16<TI>(xa[a], ga[b], acc[a][b]);
+            for (int b = 0; b < NT; ++b) acc[a][b] = mm_32x32x16<TI>(xa[a], ga[b], acc[a][b]);
         }
       }
     }
   }
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
+  for (int a = 0; a < NT; ++a)
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
+    for (int b = 0; b < NT; ++b) {
       const int vv = v0 + 32 * b + c;
       if (vv >= q.N) continue;
 #pragma unroll
@@ -274,12 +280,14 @@ __global__ void __launch_bounds__(256, 2) flex_grad_kernel(const FlexGrad* __res
   const FlexGrad q = grads[b];
   const int64_t zb = chunk * rows_per_chunk, ze = min(zb + rows_per_chunk, Z);
   float* P = partial + chunk * numel;
+#define FLEX_TILE(D) do { if (q.K <= 32 && q.N <= 32) flex_grad_tile<TI, D, 1>(q, tile, X, ldx, G, ldg, P, zb, ze); else flex_grad_tile<TI, D, 2>(q, tile, X, ldx, G, ldg, P, zb, ze); } while (0)
   switch (q.D) {
-    case 1: flex_grad_tile<TI, 1>(q, tile, X, ldx, G, ldg, P, zb, ze); break;
-    case 3: flex_grad_tile<TI, 3>(q, tile, X, ldx, G, ldg, P, zb, ze); break;
-    case 5: flex_grad_tile<TI, 5>(q, tile, X, ldx, G, ldg, P, zb, ze); break;
-    default: flex_grad_tile<TI, 7>(q, tile, X, ldx, G, ldg, P, zb, ze);
+    case 1: FLEX_TILE(1); break;
+    case 3: FLEX_TILE(3); break;
+    case 5: FLEX_TILE(5); break;
+    default: FLEX_TILE(7);
   }
+#undef FLEX_TILE
 }
 
 // out[w] = sum over the chunks, in order, rounded once to the weights' type; 16 chunk lanes x 64 weights per block

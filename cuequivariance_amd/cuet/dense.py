@@ -273,10 +273,13 @@ def _rows_launches(mod: "SegmentedPolynomialDense", es: int):
 # Rows from which on the row-streaming launches (weights in LDS) are the faster ones for forward and input gradient, by (rows in
 # mul_ir, element size) and multiplicity (up to 32, up to 64, above): where the measured times of the two cross.  Below, a launch is
 # bound by the chain of one wavefront, above by what one CU keeps in flight (128x0e+128x1o+128x2e, 4 000 rows of float: 27 us
-# against 72; 200 000: 804 against 623).  The weight gradient's row launches win from the first row on, but for float in mul_ir.
-_ROWS_FROM = {(False, 4): (15_000, 10_000, 35_000), (False, 2): (30_000, 3_000, 6_000), (True, 4): (50_000, 30_000, 22_000),
-              (True, 2): (50_000, 22_000, 15_000)}
-_GRADS_FROM = {(False, 4): 0, (False, 2): 0, (True, 4): 5_000, (True, 2): 0}
+# against 72; 200 000: 804 against 623).
+_NEVER = 1 << 60
+_ROWS_FROM = {(False, 4): (15_000, 10_000, 35_000), (False, 2): (_NEVER, 3_000, 6_000), (True, 4): (60_000, 30_000, 22_000),
+              (True, 2): (_NEVER, 22_000, 15_000)}
+# ... and for the weight gradient, whose row launches win from the first row on but for float in mul_ir and for up to 32 channels (their
+# 128 x 128 tiles are padding then: 200 000 rows of 32x0e+32x1o+32x2e, float: 485 us against 274)
+_GRADS_FROM = {(False, 4): (_NEVER, 0, 0), (False, 2): (15_000, 0, 0), (True, 4): (150_000, 5_000, 5_000), (True, 2): (0, 0, 0)}
 
 
 def _linear_op(mod: "SegmentedPolynomialDense"):
@@ -290,7 +293,8 @@ def _linear_op(mod: "SegmentedPolynomialDense"):
                               tables[2], tables[0], tables[1])
     most = max(max(p.K, p.N) for p in mod.paths)
     for es in (4, 2):
-        rows_from, grads_from = _ROWS_FROM[(mod.rows_mul_ir, es)][0 if most <= 32 else 1 if most <= 64 else 2], _GRADS_FROM[(mod.rows_mul_ir, es)]
+        size = 0 if most <= 32 else 1 if most <= 64 else 2
+        rows_from, grads_from = _ROWS_FROM[(mod.rows_mul_ir, es)][size], _GRADS_FROM[(mod.rows_mul_ir, es)][size]
         if mod.rows_mul_ir:
             if mod.mul_ir is not None and mod.mul_ir.accepts({4: torch.float32, 2: torch.bfloat16}[es]):
                 fwd, dx, dw = mod.mul_ir.tables(es)
@@ -308,6 +312,80 @@ def _linear_op(mod: "SegmentedPolynomialDense"):
             op.add_grads(es, grads_from, [(K, N, coeff, a0, c0, da, dc, [], [w for w, _ in runs], [n for _, n in runs])])
         else:
             op.add_grads(es, grads_from, [(p.K, p.N, p.coeff, p.a_off, p.c_off, da, dc, [], [p.w_off], [count]) for p, count, da, dc in mod.fwd_groups])
+    return op
+
+
+def _fc_tables(mod: "SegmentedPolynomialDense"):
+    """Packed tables of ``csrc/fc_flex.hip`` for ``uvw,iu,jv,kw+ijk`` with ``v = 1``: ``((blocks and parts forward, of the input
+    gradient, weight gradients, coefficients), tiles, element sizes served, most components)``, or ``None``."""
+    ope, stp = mod._polynomial_orig.operations[0]
+    if str(stp.subscripts) not in ("uvw,iu,jv,kw+ijk", "uw,iu,j,kw+ijk") or not stp.paths:
+        return None
+    offs = [o.segment_offsets() for o in stp.operands]
+    coef: list = []
+    paths = []  # (w0, a0, K, D1, c0, N, D3, coefficients as [i, k, j], as [k, i, j], j0, d2)
+    for p in stp.paths:
+        sw, s1, s2, so = p.indices
+        (d1, K), d2, (d3, N) = stp.operands[1][s1], stp.operands[2][s2][0], stp.operands[3][so]
+        c = p.coefficients
+        if d1 not in (1, 3, 5) or d3 not in (1, 3, 5):
+            return None
+        at = len(coef)
+        coef += [float(v) for v in c.transpose(0, 2, 1).reshape(-1)]
+        back = len(coef)
+        coef += [float(v) for v in c.transpose(2, 0, 1).reshape(-1)]
+        paths.append((offs[0][sw], offs[1][s1], K, d1, offs[3][so], N, d3, at, back, offs[2][s2], d2))
+    if len({p[0] for p in paths}) != len(paths) or sum(p[2] * p[5] for p in paths) != mod.input_sizes[0] or mod.input_sizes[2] > 64:
+        return None
+    served = 0
+    for bit, epv, step in ((1, 4, 8), (2, 8, 16)):
+        if (all(v % epv == 0 for p in paths for v in (p[0], p[1], p[4])) and all(p[2] % step == 0 and p[5] % step == 0 for p in paths)
+                and mod.input_sizes[1] % epv == 0 and mod.out_size % epv == 0):
+            served |= bit
+    if not served:
+        return None
+
+    def side(block, part):
+        by = {}
+        for p in paths:
+            by.setdefault(block(p), []).append(p)
+        blocks, parts, tiles = b"", b"", 0
+        for (c0, n, d), ps in sorted(by.items(), key=lambda kv: -sum(part(p)[3] for p in kv[1])):  # (the longest units first)
+            nt = -(-n // 32)
+            blocks += struct.pack("<6i", c0, n, d, len(parts) // 40, len(ps), nt)
+            tiles += nt
+            for p in ps:
+                parts += struct.pack("<q8i", *part(p), 0)
+        return blocks, parts, tiles
+
+    fwd = side(lambda p: (p[4], p[5], p[6]), lambda p: (p[0], p[1], p[2], p[3], p[7], p[9], p[10], p[5]))
+    dx = side(lambda p: (p[1], p[2], p[3]), lambda p: (p[0], p[4], p[5], p[6], p[8], p[9], p[10], p[5]))
+    grads, tiles = b"", 0
+    for p in sorted(paths, key=lambda p: -p[3]):
+        ntv = -(-p[5] // 64)
+        nt = ntv * -(-p[2] // 64)
+        grads += struct.pack("<q12i", p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7], p[9], p[10], nt, ntv, 0)
+        tiles += nt
+    return ((fwd[0], fwd[1], dx[0], dx[1], grads, struct.pack(f"<{len(coef)}f", *coef)), (fwd[2], dx[2], tiles), served,
+            max(max(p[3], p[6]) for p in paths), [(p[0], p[1], p[2], p[3], p[5], p[6]) for p in sorted(paths, key=lambda p: -p[3])])
+
+
+# Rows from which on the generated kernels are the faster ones (forward, input gradients, weight gradient), by element size: always,
+# but for the float forward, whose unit is a wavefront's 19 us (64 channels, 3 000 rows: 27 us against 17).
+_FC_FROM = {4: (15_000, 0, 0), 2: (0, 0, 0)}
+
+
+def _fc_op(mod: "SegmentedPolynomialDense"):
+    """The 4-operand form as the host module runs it (``csrc/host/fully_connected.cpp``), or ``None``."""
+    if not mod.has_x2 or mod.method != "fused_tp":
+        return None
+    tables = _fc_tables(mod)
+    if tables is None:
+        return None
+    op = _lib.host().FcOp(mod.input_sizes[1], mod.input_sizes[2], mod.out_size, mod.input_sizes[0], mod.rows_mul_ir, mod.dx1_covers_input,
+                          mod.fwd_covers_output, tables[2], tables[3], tables[0], tables[1])
+    # from these rows on (float, 2-byte) the weight gradient's factors go through memory to the tiled product (measured crossings)
+    op.add_tiled_dw(tables[4], 13_000, 6_000)
     return op
 
 
@@ -1148,6 +1226,8 @@ def _dense_fwd_op(mod_key: str, kind: int, w: torch.Tensor, x1: torch.Tensor, x2
     mod = _module_by_key(mod_key)
     if mod.linear_takes(x1, x2):
         return mod.linear.forward(w.detach(), x1.detach())
+    if mod.fc_takes(x1, x2):
+        return mod.fully_connected.forward(w.detach(), x1.detach(), x2.detach())
     return _FUNCTIONS[kind].forward(_PlainContext(), mod, w, x1, x2)
 
 
@@ -1166,6 +1246,8 @@ def _dense_bwd_op(mod_key: str, kind: int, w: torch.Tensor, x1: torch.Tensor, x2
     if ctx.mod.linear_takes(x1, x2):
         op, g = ctx.mod.linear, g.detach()
         grads = (op.dw(x1.detach(), g, w) if need[0] else None, op.dx(w.detach(), g, x1) if need[1] else None, None)
+    elif ctx.mod.fc_takes(x1, x2):
+        grads = ctx.mod.fully_connected.gradients(w, x1.detach(), x2.detach(), g.detach(), *need)
     elif kind == 0:
         grads = _DenseFunction._backward_impl(ctx, g, ctx.needs_input_grad)[1:4]
     else:
@@ -1252,7 +1334,7 @@ class SegmentedPolynomialDense(nn.Module):
         # take such rows apart / put them together in registers, other executors of this module do not take them.
         self.mul_ir, self.fc_blocks = None, None
         self.rows_mul_ir = rows == "mul_ir"
-        self._linear = False
+        self._linear, self._fc = False, {}
         if rows == "mul_ir" and not self.has_x2:
             self.mul_ir = _MulIrPlan.build(self)
             if self.mul_ir is None and _flex_tables(self, True) is None:
@@ -1286,14 +1368,7 @@ class SegmentedPolynomialDense(nn.Module):
             return None
         if any(t.data_ptr() % 16 or (t.stride(0) * t.element_size()) % 16 or t.stride(1) != 1 for t in row_tensors):
             return None
-        from .. import jit
-
-        key = (dtype, jit.enabled())
-        if key not in self._fused:
-            blocks = self.fc_blocks or (None, None)
-            self._fused[key] = jit.fully_connected_unit(self.paths, self.input_sizes[2], self.input_sizes[1], self.out_size,
-                                                          _FC_ELEMENT[dtype], blocks[0], blocks[1])
-        return self._fused[key]
+        return self._generated(dtype)
 
     @property
     def linear(self):
@@ -1301,6 +1376,45 @@ class SegmentedPolynomialDense(nn.Module):
         if self._linear is False:
             self._linear = _linear_op(self)
         return self._linear
+
+    @property
+    def fully_connected(self):
+        """The 4-operand form as the host module runs it, or ``None`` (one with and one without generated kernels, as compilation
+        at first use is switched on or off)."""
+        from .. import jit
+
+        on = jit.enabled()
+        if on not in self._fc:
+            self._fc[on] = _fc_op(self)
+        return self._fc[on]
+
+    def fc_takes(self, x1, x2) -> bool:
+        """Whether the host module runs this 4-operand product for rows of this type (the generated kernels, where they are the
+        faster ones, are looked for at the first call of a type)."""
+        if x2 is None or x1.dtype not in _MATRIX_CORE:
+            return False
+        op = self.fully_connected
+        if op is None or not op.takes(x1):
+            return False
+        from .. import jit
+
+        if (x1.dtype, jit.enabled()) not in self._fused and self.fc_plan.ok:
+            unit = self._generated(x1.dtype)
+            if unit is not None:
+                address = lambda f: C.cast(f, C.c_void_p).value
+                op.add_unit(_DTYPE_CODE[x1.dtype], [address(f) for f in (unit.fcj_fwd, unit.fcj_dx1, unit.fcj_dx2, unit.fcj_dx12, unit.fcj_dw_blocks,
+                                                                         unit.fcj_dw)], *_FC_FROM[x1.dtype.itemsize])
+        return True
+
+    def _generated(self, dtype):
+        """The kernels generated for this product (``codegen/fullyconnected.py``; compiled at first use), or ``None``."""
+        from .. import jit
+
+        key = (dtype, jit.enabled())
+        if key not in self._fused:
+            blocks = self.fc_blocks or (None, None)
+            self._fused[key] = jit.fully_connected_unit(self.paths, self.input_sizes[2], self.input_sizes[1], self.out_size, _FC_ELEMENT[dtype], *blocks)
+        return self._fused[key]
 
     def linear_takes(self, x1, x2) -> bool:
         return x2 is None and x1.dtype in _MATRIX_CORE and self.linear is not None and self.linear.takes(x1)
@@ -1315,15 +1429,11 @@ class SegmentedPolynomialDense(nn.Module):
             return False
         if not self.has_x2:
             return self.rows_accepted(dtype)
+        if self.fc_takes(torch.empty(0, dtype=dtype), ()):
+            return True
         if dtype not in _MATRIX_CORE or not self.fc_plan.ok:
             return False
-        from .. import jit
-
-        key = (dtype, jit.enabled())
-        if key not in self._fused:
-            self._fused[key] = jit.fully_connected_unit(self.paths, self.input_sizes[2], self.input_sizes[1], self.out_size,
-                                                          _FC_ELEMENT[dtype], *self.fc_blocks)
-        return self._fused[key] is not None
+        return self._generated(dtype) is not None
 
     def tiled(self, dtype, A: torch.Tensor, Cout: torch.Tensor) -> bool:
         """The tiled kernel serves fp32 / bf16 contractions without a per-row scale."""
@@ -1407,7 +1517,11 @@ class SegmentedPolynomialDense(nn.Module):
                 x2 = x2.expand(x1.shape[0], x2.shape[1])
             elif x1.shape[0] == 1 and x2.shape[0] != 1:
                 x1 = x1.expand(x2.shape[0], x1.shape[1])
-        if x2 is not None and x1.dtype == torch.float16 and not (self.fc_plan.ok and self.fused_unit(torch.float16, _aligned(x1.detach())) is not None):
+        if x2 is not None and not torch.compiler.is_compiling() and not torch.jit.is_tracing() and type(x1) in (torch.Tensor, torch.nn.Parameter) and self.fc_takes(x1, x2):
+            out = self.fully_connected.direct(w, x1, x2)
+            if out is not None:
+                return [out]
+        if x2 is not None and x1.dtype == torch.float16 and not (self.fc_takes(x1, x2) or self.fc_plan.ok and self.fused_unit(torch.float16, _aligned(x1.detach())) is not None):
             # half runs on the generated fused kernels only (the table-driven kernels behind them know float32 and bfloat16):
             # anything else is computed in float32 - every half is a float - and rounded once
             return [self.forward([w.float(), x1.float(), x2.float()], input_indices, output_shapes, output_indices)[0].to(torch.float16)]

@@ -183,8 +183,8 @@ class ChannelWiseTensorProduct(torch.nn.Module):
         self.f = SegmentedPolynomial(
             e.polynomial, method=self.method, math_dtype=math_dtype, options={"segment_groups": groups} if groups else None
         )
-        self._direct = (self.method == "uniform_1d" and self.transpose_in1.is_identity and self.transpose_in2.is_identity
-                        and self.transpose_out.is_identity)
+        self._direct = (self.method == "uniform_1d" and self.transpose_in1.moves_nothing and self.transpose_in2.moves_nothing
+                        and self.transpose_out.moves_nothing)
 
     def extra_repr(self) -> str:
         return (
@@ -296,7 +296,7 @@ class ChannelWiseSphericalTensorProduct(torch.nn.Module):
         if groups:
             options["segment_groups"] = groups
         self.f = SegmentedPolynomial(polynomial, method="uniform_1d", math_dtype=math_dtype, options=options)
-        self._direct = self.transpose_in1.is_identity and self.transpose_out.is_identity
+        self._direct = self.transpose_in1.moves_nothing and self.transpose_out.moves_nothing
 
     def extra_repr(self) -> str:
         return f"ls={self.ls}, normalize={self.normalize}, shared_weights={self.shared_weights}, weight_numel={self.weight_numel}"
@@ -428,6 +428,13 @@ class FullyConnectedTensorProduct(torch.nn.Module):
             weight = self.weight
         elif weight is None:
             raise ValueError("Internal weights are not used, weight should not be None")
+        if indices_1 is None and indices_out is None and not torch.compiler.is_compiling() and type(x1) is torch.Tensor:
+            # the whole call in native code when it is a plain one; anything else, and every error, takes the way below
+            dense = self._dense()
+            if dense is not None and dense.fc_takes(x1, x2):
+                out = dense.fully_connected.direct(weight, x1, x2)
+                if out is not None:
+                    return out
         if indices_1 is None and indices_out is None and self._rows_ready(x1, x2, weight):
             return self.f_rows([weight, x1, apply_layout(self.transpose_in2, x2)])[0]
         x1 = apply_layout(self.transpose_in1, x1)
@@ -443,6 +450,16 @@ class FullyConnectedTensorProduct(torch.nn.Module):
         if weight.shape[0] != 1 or self.f is None:
             return apply_layout(self.transpose_out, self.f_per_sample([weight, x1, x2])[0])
         return apply_layout(self.transpose_out, self.f([weight, x1, x2])[0])
+
+    def _dense(self):
+        """The executor of the 4-operand form for rows in this module's layouts, or ``None``."""
+        if self.method != "fused_tp" or not self.transpose_in2.moves_nothing:
+            return None
+        if self.f_rows is not None:
+            return self.f_rows._modules["m"].dense
+        if self.f is None or not (self.transpose_in1.moves_nothing and self.transpose_out.moves_nothing):
+            return None
+        return getattr(self.f._modules["m"], "dense", None)
 
     def _rows_ready(self, x1, x2, weight) -> bool:
         dense = self.f_rows.m.dense if self.f_rows is not None else None
@@ -520,7 +537,7 @@ class Linear(torch.nn.Module):
             return None
         if self.f_rows is not None:
             return self.f_rows._modules["m"].dense.linear
-        if not (self.transpose_in.is_identity and self.transpose_out.is_identity):
+        if not (self.transpose_in.moves_nothing and self.transpose_out.moves_nothing):
             return None
         dense = getattr(self.f._modules["m"], "dense", None)
         return dense.linear if dense is not None else None
@@ -628,8 +645,8 @@ class SymmetricContraction(torch.nn.Module):
         )
         self.f = SegmentedPolynomial(self.etp.polynomial, method=self.method, math_dtype=math_dtype,
                                      options={"segment_groups": groups} if groups else None)
-        self._direct = (self.method == "uniform_1d" and self.projection is None and self.transpose_in.is_identity
-                        and self.transpose_out.is_identity)
+        self._direct = (self.method == "uniform_1d" and self.projection is None and self.transpose_in.moves_nothing
+                        and self.transpose_out.moves_nothing)
 
     def extra_repr(self) -> str:
         return f"contraction_degree={self.contraction_degree}, weight_shape={self.weight_shape}"

@@ -104,6 +104,7 @@ class TransposeIrrepsLayout(torch.nn.Module):
             self.f = torch.nn.Identity()
         self.source, self.target = source, target
         self.is_identity = isinstance(self.f, torch.nn.Identity)  # callers skip the module call then (see `apply_layout`)
+        self.moves_nothing = self.is_identity or self.f.trivial  # (every block has multiplicity or dimension one)
 
     def __repr__(self):
         return f"TransposeIrrepsLayout({self.source} -> {self.target})"

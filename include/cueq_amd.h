@@ -466,6 +466,26 @@ int cueq_linear_flex_dw(int32_t dtype, int64_t rows, const void* X, int64_t ldx,
 int cueq_sum_runs(const float* partial, int32_t per, int32_t nruns, const int32_t* first, const int64_t* w0, int32_t out_dtype,
                   void* out, void* stream);
 
+/* Fully connected product with shared weights and a second operand of multiplicity one, table-driven, for batches that do not
+ * fill the chip with the generated kernels and for extents those do not take.  gradient == 0: rows of x1 against the weights;
+ * 1: rows of the cotangent against the weights read transposed - with X1, partial (column_tiles x rows x n2 floats) and dX2
+ * given also the gradient of x2 from the same products.  `blocks`, `parts`, `grads` are device tables (FcBlock, FcPart, FcGrad of
+ * csrc/fc_flex.hip), `coef` the path coefficients; multiplicities multiples of 8 (float32) / 16, components 1, 3 or 5. */
+int cueq_fc_flex(int32_t dtype, int32_t gradient, int32_t mul_ir, int64_t rows, const void* A, int64_t lda, const void* W,
+                 const void* X2, int64_t ldx2, const void* X1, int64_t ldx1, void* C, int64_t ldc, const void* blocks,
+                 int32_t nblocks, const void* parts, const float* coef, int32_t column_tiles, int32_t most_components, int32_t n2,
+                 float* partial, void* dX2, void* stream);
+/* Partial products of the weight gradient, cueq_fc_flex_dw_chunks x numel floats to be summed in order (cueq_sum_runs). */
+int64_t cueq_fc_flex_dw_chunks(int64_t rows, int32_t tiles);
+int cueq_fc_flex_dw(int32_t dtype, int32_t mul_ir, int64_t rows, const void* X1, int64_t ldx1, const void* X2, int64_t ldx2,
+                    const void* G, int64_t ldg, const void* grads, int32_t ngrads, const float* coef, int32_t tiles, int64_t numel,
+                    float* partial, void* stream);
+/* For many rows: H (rows x ldh: for every path of `grads`, in order, D1 x N columns sum_k s_ik g_k), which the weight gradient then
+ * contracts with x1 (cueq_gemm_table); x1 in mul_ir is also written with its components apart (X1T, blocks as in `blocks1`).  nfactors: D1 x D3 summed over the paths. */
+int cueq_fc_factors(int32_t dtype, int32_t mul_ir, int64_t rows, const void* X1, int64_t ldx1, const void* X2, int64_t ldx2,
+                    const void* G, int64_t ldg, const void* grads, int32_t ngrads, const float* coef, const void* blocks1,
+                    int32_t nblocks1, int32_t nfactors, void* H, int64_t ldh, void* X1T, void* stream);
+
 /* The whole triangle multiplicative update of pair tensors x (B, N, N, D) -> out (B, N, N, Do), any N, in one call per
  * direction (cuequivariance_torch/primitives/triangle.py:138-262).  `weights`: host array of 12 device pointers - input
  * norm weight, bias; value projection p_in weight (2D, D), bias; gate g_in weight, bias; output norm weight, bias; p_out weight
