@@ -80,6 +80,7 @@ EXPORTED_SYMBOLS = (
     "cueq_fc_flex",
     "cueq_fc_flex_dw_chunks",
     "cueq_fc_flex_dw",
+    "cueq_fc_pack",
     "cueq_fc_factors",
     "cueq_trimul_grads_values",
     "cueq_trimul_saved_bytes",
@@ -287,11 +288,13 @@ def load() -> C.CDLL:
         lib.cueq_linear_flex_dw.restype = C.c_int
         lib.cueq_sum_runs.argtypes = [ptr, i32, i32, ptr, ptr, i32, ptr, ptr]
         lib.cueq_sum_runs.restype = C.c_int
-        lib.cueq_fc_flex.argtypes = [i32, i32, i32, i64, ptr, i64, ptr, ptr, i64, ptr, i64, ptr, i64, ptr, i32, ptr, ptr, i32, i32, i32, ptr, ptr, ptr]
+        lib.cueq_fc_flex.argtypes = [i32, i32, i32, i32, i64, ptr, i64, ptr, ptr, i64, ptr, i64, ptr, i64, ptr, i32, ptr, ptr, i32, i32, i32, ptr, ptr, ptr]
         lib.cueq_fc_flex.restype = C.c_int
-        lib.cueq_fc_flex_dw_chunks.argtypes = [i64, i32]
+        lib.cueq_fc_pack.argtypes = [i32, ptr, ptr, ptr, i32, i64, ptr]
+        lib.cueq_fc_pack.restype = C.c_int
+        lib.cueq_fc_flex_dw_chunks.argtypes = [i64, i32, i32]
         lib.cueq_fc_flex_dw_chunks.restype = i64
-        lib.cueq_fc_flex_dw.argtypes = [i32, i32, i64, ptr, i64, ptr, i64, ptr, i64, ptr, i32, ptr, i32, i64, ptr, ptr]
+        lib.cueq_fc_flex_dw.argtypes = [i32, i32, i32, i64, ptr, i64, ptr, i64, ptr, i64, ptr, i32, ptr, i32, i64, ptr, ptr]
         lib.cueq_fc_flex_dw.restype = C.c_int
         lib.cueq_fc_factors.argtypes = [i32, i32, i64, ptr, i64, ptr, i64, ptr, i64, ptr, i32, ptr, ptr, i32, i32, ptr, i64, ptr, ptr]
         lib.cueq_fc_factors.restype = C.c_int

@@ -1,7 +1,9 @@
-// Fully connected product with shared weights and a second operand of multiplicity one (uvw,iu,jv,kw+ijk, v = 1), table-driven:
+// Fully connected product with shared weights (uvw,iu,jv,kw+ijk, any v), table-driven:
 //
-//   out[z, k, w] = sum over the paths p of the block   sum_ij C_p[i, j, k] x2[z, j] sum_u x1[z, i, u] W_p[u, w]
+//   out[z, k, w] = sum over the paths p of the block and the channels v of its x2 block
+//                  sum_ij C_p[i, j, k] x2[z, j, v] sum_u x1[z, i, u] W_p[u, v, w]
 //
+// First for one channel v (a second operand of multiplicity one, and float rows of any): a channel is a part of its own.
 // In the manner of linear_flex.hip: a wavefront takes 32 rows x 32 columns of one result block (all its components), weights and
 // rows straight from the caches, no LDS for operands, no barriers.  The products are issued as W-columns x rows, so a lane holds one
 // row: T_i = x1_i W_p stays in registers, and the factors s_ik = sum_j C_p[i, j, k] x2[z, j] are scalars of the lane:
@@ -22,11 +24,18 @@
 namespace cueq {
 namespace {
 
-struct FcPart {          // one path: its weights, the source block it contracts, its factors
+struct FcPart {            // one path: its weights, the source block it contracts, its factors
   int64_t w0;
   int32_t a0, K, D, coef;  // source block: offset, multiplicity, components; coef: offset of the D x DR x d2 factors
-  int32_t j0, d2;
-  int32_t stride, unused;  // elements between weight rows as stored
+  int32_t j0, d2;          // x2 block: offset, components
+  int32_t stride, V, js, vs, wv;  // elements between weight rows as stored; multiplicity of the x2 block, elements between its
+                                  // components / its channels, and between the weights of two channels
+  uint32_t mask;           // bit i * DR + k: some factor of (i, k) is not zero
+};
+struct FcPack {  // the weights of one path put into the order of the matrix instructions' operands
+  int64_t src, dst;
+  int32_t K, N, sk, sn, V, vs, pieces, steps;  // contracted / result extent and their strides, channels of x2 and their stride;
+                                               // steps of 16 contracted values written (zeros past K)
 };
 struct FcBlock {  // one block of the result
   int32_t c0, N, D, first, parts, nt;
@@ -47,9 +56,34 @@ __device__ __forceinline__ uint32_t fc_pick(const uint4* run, int i0, int i1) {
   return __builtin_amdgcn_perm(w[i1 >> 1], w[i0 >> 1], sel);
 }
 
-// T[i] = source_i W (32 columns from n0) for the DS components of one source block; n: this lane's column, clamped
-template <typename TI, int DS, bool WT, bool MI>
-__device__ __forceinline__ void fc_products(fx16 (&T)[DS], const FcPart& part, const TI* __restrict__ row, const TI* __restrict__ W, int n) {
+// component i of eight channels: x is DS pieces of one component each (ir_mul) or of eight channels with their components adjacent
+template <int DS, bool MI>
+__device__ __forceinline__ uint4 fc_component(const uint4 (&x)[DS], int i) {
+  if constexpr (DS == 1 || !MI) return x[i];
+  else return make_uint4(fc_pick<DS>(&x[0], i, DS + i), fc_pick<DS>(&x[0], 2 * DS + i, 3 * DS + i), fc_pick<DS>(&x[0], 4 * DS + i, 5 * DS + i),
+                         fc_pick<DS>(&x[0], 6 * DS + i, 7 * DS + i));
+}
+
+// The coefficients of one path (at most 64), a lane each: short products would wait for a memory request for each of them.
+struct FcCoefs {
+  float mine;
+  __device__ __forceinline__ FcCoefs(const float* from, int n) : mine(0.f) {
+    const int lane = threadIdx.x & 63;
+    if (lane < n) mine = from[lane];
+  }
+  __device__ __forceinline__ float operator[](int i) const {  // i: the same in all lanes
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, mine), i));
+  }
+};
+
+// How the weights lie: as given, contracted over their first or their last extent, or packed by fc_pack_kernel
+enum FcWeights { kPlain = 0, kTransposed = 1, kPacked = 2 };
+constexpr int kFragment = 512;  // 2-byte elements of one packed operand: 64 lanes x 8
+
+// T[i] = source_i W (32 columns from n0) for the DS components of one source block; n: this lane's column, clamped; W: the weights of
+// the path and the channel of x2
+template <typename TI, int DS, int WM, bool MI>
+__device__ __forceinline__ void fc_products(fx16 (&T)[DS], const FcPart& part, const TI* __restrict__ row, const TI* __restrict__ W, int n, int n0) {
   constexpr int ES = sizeof(TI), EPV = 16 / ES, STEP = 2 * EPV;
   const int h = (threadIdx.x >> 5) & 1;
 #pragma unroll
@@ -59,17 +93,19 @@ __device__ __forceinline__ void fc_products(fx16 (&T)[DS], const FcPart& part, c
     const int k = k0 + EPV * h;
 #pragma unroll
     for (int i = 0; i < DS; ++i) xx[i] = *reinterpret_cast<const uint4*>(row + part.a0 + (MI ? k * DS + i * EPV : i * part.K + k));
-    if constexpr (WT) {
-      ww = *reinterpret_cast<const uint4*>(W + part.w0 + static_cast<int64_t>(n) * part.stride + k);
+    if constexpr (WM == kPacked) {
+      ww = *reinterpret_cast<const uint4*>(W + ((k0 / STEP) * part.stride + n0 / 32) * kFragment + (threadIdx.x & 63) * 8);
+    } else if constexpr (WM == kTransposed) {
+      ww = *reinterpret_cast<const uint4*>(W + static_cast<int64_t>(n) * part.stride + k);
     } else if constexpr (ES == 4) {
       uint32_t e[4];
 #pragma unroll
-      for (int s = 0; s < 4; ++s) e[s] = reinterpret_cast<const uint32_t*>(W)[part.w0 + static_cast<int64_t>(k + s) * part.stride + n];
+      for (int s = 0; s < 4; ++s) e[s] = reinterpret_cast<const uint32_t*>(W)[static_cast<int64_t>(k + s) * part.stride + n];
       ww = make_uint4(e[0], e[1], e[2], e[3]);
     } else {
       uint32_t e[8];
 #pragma unroll
-      for (int s = 0; s < 8; ++s) e[s] = reinterpret_cast<const uint16_t*>(W)[part.w0 + static_cast<int64_t>(k + s) * part.stride + n];
+      for (int s = 0; s < 8; ++s) e[s] = reinterpret_cast<const uint16_t*>(W)[static_cast<int64_t>(k + s) * part.stride + n];
       ww = make_uint4(e[0] | e[1] << 16, e[2] | e[3] << 16, e[4] | e[5] << 16, e[6] | e[7] << 16);
     }
   };
@@ -86,11 +122,7 @@ __device__ __forceinline__ void fc_products(fx16 (&T)[DS], const FcPart& part, c
     } else {
 #pragma unroll
       for (int i = 0; i < DS; ++i) {
-        uint4 op;
-        if constexpr (DS == 1 || !MI) op = x[i];
-        else op = make_uint4(fc_pick<DS>(&x[0], i, DS + i), fc_pick<DS>(&x[0], 2 * DS + i, 3 * DS + i), fc_pick<DS>(&x[0], 4 * DS + i, 5 * DS + i),
-                             fc_pick<DS>(&x[0], 6 * DS + i, 7 * DS + i));
-        T[i] = mm_32x32x16<TI>(wv, op, T[i]);
+        T[i] = mm_32x32x16<TI>(wv, fc_component<DS, MI>(x, i), T[i]);
       }
     }
 #pragma unroll
@@ -122,21 +154,21 @@ __device__ __forceinline__ void fc_load4(float (&v)[4][DR], const TI* __restrict
   }
 }
 
-template <typename TI, int DS, int DR, bool WT, bool MI, bool DX2>
+// (a channel of x2 is a part of its own here: a loop over them costs the registers of straight code)
+template <typename TI, int DS, int DR, int WM, bool MI, bool DX2>
 __device__ __forceinline__ void fc_part(fx16 (&acc)[DR], const FcPart& part, const FcBlock& blk, const TI* __restrict__ row, const TI* __restrict__ W,
-                                        const float* __restrict__ coef, const TI* __restrict__ x2row, const TI* __restrict__ x1row, float* lsum, int n2, int n0,
-                                        int n) {
-  const int lane = threadIdx.x & 63, c = lane & 31, h = lane >> 5;
-  fx16 T[DS];
-  fc_products<TI, DS, WT, MI>(T, part, row, W, n);
+                                        const float* __restrict__ coef, const TI* __restrict__ x2row, const TI* __restrict__ x1row, float* sums, int n0, int n) {
+  const int lane = threadIdx.x & 63, h = lane >> 5;
   const float* __restrict__ cf = coef + part.coef;
+  fx16 T[DS];
+  fc_products<TI, DS, WM, MI>(T, part, row, W + part.w0, n, n0);
   float s[DS][DR];
 #pragma unroll
   for (int i = 0; i < DS; ++i)
 #pragma unroll
     for (int k = 0; k < DR; ++k) s[i][k] = 0.f;
   for (int j = 0; j < part.d2; ++j) {
-    const float xj = fc_widen(x2row + part.j0 + j);
+    const float xj = fc_widen(x2row + part.j0 + j * part.js);
 #pragma unroll
     for (int i = 0; i < DS; ++i)
 #pragma unroll
@@ -147,7 +179,7 @@ __device__ __forceinline__ void fc_part(fx16 (&acc)[DR], const FcPart& part, con
 #pragma unroll
     for (int i = 0; i < DS; ++i)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) acc[k][v] = fmaf(s[i][k], T[i][v], acc[k][v]);
+      for (int r = 0; r < 16; ++r) acc[k][r] = fmaf(s[i][k], T[i][r], acc[k][r]);
   if constexpr (DX2) {
     float y[DS][DR];
 #pragma unroll
@@ -179,34 +211,207 @@ __device__ __forceinline__ void fc_part(fx16 (&acc)[DR], const FcPart& part, con
       for (int i = 0; i < DS; ++i)
 #pragma unroll
         for (int k = 0; k < DR; ++k) d = fmaf(cf[(i * DR + k) * part.d2 + j], y[i][k], d);
-      lsum[c * n2 + part.j0 + j] += d;
+      sums[part.j0 + j * part.js] += d;
     }
   }
 }
 
-template <typename TI, int DR, bool WT, bool MI, bool DX2, int MAXD>
+// The components that a product of irreps of degree 0 and 1 couples (d1 x d2 -> d3 with d <= 3, and 3 x 5 -> 3): which (i, k) have a
+// coefficient at all is known when the kernel is compiled, and its loops are straight code.
+template <int DS, int DR, int D2>
+constexpr bool fc_couples(int i, int k) {
+  return DS != 3 || DR != 3 || (D2 == 1 ? i == k : D2 == 3 ? i != k : true);
+}
+
+// 2-byte elements where x2 has several channels, packed weights, K <= 16 KT and the couplings above: the source block of the row stays in registers over
+// the channels of x2, and the weights of 16 / KT channels go through LDS for the four wavefronts of the workgroup (four row tiles under
+// one column tile), the next ones requested meanwhile.  Straight code is what counts: with the extents, the components of x2 and the
+// couplings tested in the loop, every fragment was waited for by itself and a channel took some 3 000 cycles of latency.
+// Bound by the issue of vector instructions (a product of 32 x 32 x K is scaled and added component by component); 12 501 rows of
+// 64x0e+64x1o (x) 16x0e+16x1o, bfloat16: forward 38.7 us, both input gradients 82 us (the tests in the loop: 45 / 172, x2 read from
+// memory: 46), where the products of the operands went through memory 160 and 340 us.
+template <typename TI, int DS, int DR, int D2, bool MI, bool DX2, int KT>
+__device__ __forceinline__ void fc_part_channels(fx16 (&acc)[DR], const FcPart& part, const FcBlock& blk, const TI* __restrict__ row, const TI* __restrict__ W,
+                                                 const float* __restrict__ coef, const TI* x2row, const TI* __restrict__ x1row, float* sums, uint4* wl,
+                                                 int n0) {
+  constexpr int VC = 16 / KT;
+  const int lane = threadIdx.x & 63, h = lane >> 5, wave = threadIdx.x >> 6;
+  uint4 x[KT][DS], wn[4];
+  auto request = [&](int v0) {  // (fragments past K are packed as zeros; past the last channel the last one is read again)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int f = wave + 4 * e, v = min(v0 + f / KT, part.V - 1), t = f % KT;
+      wn[e] = *reinterpret_cast<const uint4*>(W + part.w0 + static_cast<int64_t>(v) * part.wv + (t * part.stride + n0 / 32) * kFragment + lane * 8);
+    }
+  };
+  request(0);
+#pragma unroll
+  for (int t = 0; t < KT; ++t) {
+    const int k = 16 * t + 8 * h, kk = min(k, part.K - 8);
+    uint4 raw[DS];
+#pragma unroll
+    for (int i = 0; i < DS; ++i) raw[i] = *reinterpret_cast<const uint4*>(row + part.a0 + (MI ? kk * DS + i * 8 : i * part.K + kk));
+#pragma unroll
+    for (int i = 0; i < DS; ++i) x[t][i] = k < part.K ? fc_component<DS, MI>(raw, i) : make_uint4(0, 0, 0, 0);
+  }
+  uint2 x1[DX2 ? 4 : 1][DR];
+  if constexpr (DX2) {
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+      const int m = min(n0 + 8 * a + 4 * h, blk.N - 4);
+#pragma unroll
+      for (int q = 0; q < DR; ++q) x1[a][q] = *reinterpret_cast<const uint2*>(x1row + blk.c0 + (MI ? m * DR + 4 * q : q * blk.N + m));
+    }
+  }
+  const FcCoefs cf(coef + part.coef, DS * DR * D2);
+#pragma unroll 1
+  for (int v0 = 0; v0 < part.V; v0 += VC) {
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 4; ++e) wl[(wave + 4 * e) * 64 + lane] = wn[e];
+    __syncthreads();
+    request(v0 + VC);
+    const int end = min(VC, part.V - v0);
+#pragma unroll 1
+    for (int g = 0; g < end; ++g) {
+      const int y0 = part.j0 + (v0 + g) * part.vs;
+      float xj[D2];
+#pragma unroll
+      for (int j = 0; j < D2; ++j) xj[j] = fc_widen(x2row + y0 + j * part.js);
+      uint4 wv[KT];
+#pragma unroll
+      for (int t = 0; t < KT; ++t) wv[t] = wl[(g * KT + t) * 64 + lane];
+      fx16 T[DS];
+#pragma unroll
+      for (int i = 0; i < DS; ++i) T[i] = fx16{0};
+#pragma unroll
+      for (int t = 0; t < KT; ++t)
+#pragma unroll
+        for (int i = 0; i < DS; ++i) T[i] = mm_32x32x16<TI>(wv[t], x[t][i], T[i]);
+      float s[DS][DR];
+#pragma unroll
+      for (int i = 0; i < DS; ++i)
+#pragma unroll
+        for (int k = 0; k < DR; ++k) {
+          s[i][k] = 0.f;
+          if (fc_couples<DS, DR, D2>(i, k))
+#pragma unroll
+            for (int j = 0; j < D2; ++j) s[i][k] = fmaf(cf[(i * DR + k) * D2 + j], xj[j], s[i][k]);
+        }
+#pragma unroll
+      for (int k = 0; k < DR; ++k)
+#pragma unroll
+        for (int i = 0; i < DS; ++i)
+          if (fc_couples<DS, DR, D2>(i, k))
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[k][r] = fmaf(s[i][k], T[i][r], acc[k][r]);
+      if constexpr (DX2) {
+        float y[DS][DR];
+#pragma unroll
+        for (int i = 0; i < DS; ++i)
+#pragma unroll
+          for (int k = 0; k < DR; ++k) y[i][k] = 0.f;
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+          const bool in = n0 + 8 * a + 4 * h < blk.N;
+          float xv[4][DR];
+#pragma unroll
+          for (int q = 0; q < DR; ++q) {
+            uint32_t w[2] = {x1[a][q].x, x1[a][q].y};
+            asm volatile("" : "+v"(w[0]), "+v"(w[1]));  // (widened here, not kept widened over the channels: 48 registers)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const float f = mm_widen<TI>(static_cast<uint16_t>(e & 1 ? w[e >> 1] >> 16 : w[e >> 1] & 0xffffu));
+              if constexpr (MI) xv[(4 * q + e) / DR][(4 * q + e) % DR] = f;
+              else xv[e][q] = f;
+            }
+          }
+#pragma unroll
+          for (int i = 0; i < DS; ++i)
+#pragma unroll
+            for (int k = 0; k < DR; ++k)
+              if (fc_couples<DS, DR, D2>(i, k)) {
+                float f = 0.f;
+#pragma unroll
+                for (int b = 0; b < 4; ++b) f = fmaf(T[i][4 * a + b], xv[b][k], f);
+                y[i][k] += in ? f : 0.f;
+              }
+        }
+#pragma unroll
+        for (int i = 0; i < DS; ++i)
+#pragma unroll
+          for (int k = 0; k < DR; ++k)
+            if (fc_couples<DS, DR, D2>(i, k)) y[i][k] += __shfl_xor(y[i][k], 32, 64);
+        // (the two halves hold the same sums: each adds every other column)
+#pragma unroll
+        for (int j = 0; j < D2; ++j) {
+          float d = 0.f;
+#pragma unroll
+          for (int i = 0; i < DS; ++i)
+#pragma unroll
+            for (int k = 0; k < DR; ++k)
+              if (fc_couples<DS, DR, D2>(i, k)) d = fmaf(cf[(i * DR + k) * D2 + j], y[i][k], d);
+          if ((j & 1) == h) sums[y0 + j * part.js] += d;
+        }
+      }
+    }
+  }
+}
+
+// 32-bit words from row to row of x2 in LDS
+__host__ __device__ constexpr int fc_x2_words(int n2) { return (n2 + 1) / 2 | 1; }
+
+template <typename TI, int DR, int WM, bool MI, bool DX2, int MAXD, int KT>
 __device__ __forceinline__ void fc_tile(const FcBlock& blk, const FcPart* __restrict__ parts, const float* __restrict__ coef, const TI* __restrict__ A, int64_t lda,
                                         const TI* __restrict__ W, const TI* __restrict__ X2, int64_t ldx2, const TI* __restrict__ X1, int64_t ldx1,
-                                        TI* __restrict__ C, int64_t ldc, float* __restrict__ partial, float* lsum, int n2, int64_t Z, int64_t z0, int n0) {
+                                        TI* __restrict__ C, int64_t ldc, float* __restrict__ partial, float* lsum, uint4* wl, int n2, int64_t Z, int64_t z0, int n0) {
   constexpr int ES = sizeof(TI);
   const int lane = threadIdx.x & 63, c = lane & 31, h = lane >> 5;
   const int64_t z = min(z0 + c, Z - 1);
   fx16 acc[DR];
 #pragma unroll
   for (int k = 0; k < DR; ++k) acc[k] = fx16{0};
+  const int n2p = n2 | 1;  // (sums of the lanes' rows an odd number of words apart)
   if constexpr (DX2) {
-    for (int e = lane; e < 32 * n2; e += 64) lsum[e] = 0.f;
+    for (int e = lane; e < 32 * n2p; e += 64) lsum[e] = 0.f;
     __builtin_amdgcn_wave_barrier();
   }
   const int n = min(n0 + c, blk.N - 1);
   const TI *row = A + z * lda, *x2row = X2 + z * ldx2, *x1row = DX2 ? X1 + z * ldx1 : nullptr;
+  if constexpr (KT > 0) {  // the rows of x2 are read channel by channel: from LDS, an odd number of words apart
+    const int words = fc_x2_words(n2);
+    uint32_t* x2l = reinterpret_cast<uint32_t*>(wl + 16 * 64) + (DX2 ? 4 * 32 * n2p : 0) + (threadIdx.x >> 6) * 32 * words;
+    const int used = (n2 + 1) / 2;
+#pragma unroll 8
+    for (int e = lane; e < 32 * used; e += 64) {
+      const int r = e / used, j = 2 * (e - r * used);
+      const uint16_t* from = reinterpret_cast<const uint16_t*>(X2 + min(z0 + r, Z - 1) * ldx2 + j);
+      x2l[r * words + e - r * used] = static_cast<uint32_t>(from[0]) | static_cast<uint32_t>(from[j + 1 < n2 ? 1 : 0]) << 16;
+    }
+    __builtin_amdgcn_wave_barrier();
+    x2row = reinterpret_cast<const TI*>(x2l + c * words);
+  }
+  float* sums = lsum + c * n2p;
+  auto one = [&](auto ds, const FcPart& part) {
+    constexpr int DS = decltype(ds)::value;
+    auto channels = [&](auto d2) { fc_part_channels<TI, DS, DR, decltype(d2)::value, MI, DX2, KT>(acc, part, blk, row, W, coef, x2row, x1row, sums, wl, n0); };
+    if constexpr (KT > 0 && DS == 3 && DR == 3) {
+      if (part.d2 == 1) channels(std::integral_constant<int, 1>{});
+      else if (part.d2 == 3) channels(std::integral_constant<int, 3>{});
+      else channels(std::integral_constant<int, 5>{});
+    } else if constexpr (KT > 0) {
+      channels(std::integral_constant<int, (DS == 1 && DR == 1 ? 1 : 3)>{});
+    } else {
+      fc_part<TI, DS, DR, WM, MI, DX2>(acc, part, blk, row, W, coef, x2row, x1row, sums, n0, n);
+    }
+  };
   for (int p = 0; p < blk.parts; ++p) {
     const FcPart part = parts[blk.first + p];
     switch (part.D) {
-      case 1: fc_part<TI, 1, DR, WT, MI, DX2>(acc, part, blk, row, W, coef, x2row, x1row, lsum, n2, n0, n); break;
-      case 3: fc_part<TI, 3, DR, WT, MI, DX2>(acc, part, blk, row, W, coef, x2row, x1row, lsum, n2, n0, n); break;
+      case 1: one(std::integral_constant<int, 1>{}, part); break;
+      case 3: one(std::integral_constant<int, 3>{}, part); break;
       default:
-        if constexpr (MAXD > 3) fc_part<TI, 5, DR, WT, MI, DX2>(acc, part, blk, row, W, coef, x2row, x1row, lsum, n2, n0, n);
+        if constexpr (MAXD > 3) one(std::integral_constant<int, 5>{}, part);
     }
   }
   if (z0 + c < Z) {
@@ -229,34 +434,64 @@ __device__ __forceinline__ void fc_tile(const FcBlock& blk, const FcPart* __rest
   if constexpr (DX2) {
     __builtin_amdgcn_wave_barrier();
     const int64_t rows = min<int64_t>(32, Z - z0);
-    for (int e = lane; e < rows * n2; e += 64) partial[z0 * n2 + e] = lsum[e];
+    for (int e = lane; e < rows * n2; e += 64) partial[z0 * n2 + e] = lsum[e / n2 * n2p + e % n2];
   }
 }
 
-// MAXD: the most components of any block (3 or 5): what the register budget has to hold
-template <typename TI, bool WT, bool MI, bool DX2, int MAXD>
-__global__ void __launch_bounds__(256, (MAXD > 3 ? 2 : 3)) fc_rows_kernel(const FcBlock* __restrict__ blocks, const FcPart* __restrict__ parts, const float* __restrict__ coef, int nblocks,
+// MAXD: the most components of any block (3 or 5): what the register budget has to hold.
+template <typename TI, int WM, bool MI, bool DX2, int MAXD, int KT>
+__global__ void __launch_bounds__(256, (MAXD > 3 || KT > 0 ? 2 : 3)) fc_rows_kernel(const FcBlock* __restrict__ blocks, const FcPart* __restrict__ parts, const float* __restrict__ coef, int nblocks,
                                                          int tiles_n, const TI* __restrict__ A, int64_t lda, const TI* __restrict__ W, const TI* __restrict__ X2,
                                                          int64_t ldx2, const TI* __restrict__ X1, int64_t ldx1, TI* __restrict__ C, int64_t ldc,
                                                          float* __restrict__ partial, int n2, int64_t Z) {
-  extern __shared__ float fc_lsum[];
+  extern __shared__ __align__(16) float fc_lsum[];  // 16 fragments of weights (KT > 0), the sums of every wavefront, its rows of x2 (KT > 0)
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-  const int64_t unit = static_cast<int64_t>(blockIdx.x) * 4 + wave;
-  const int64_t zt = unit / tiles_n;
-  const int column = static_cast<int>(unit - zt * tiles_n);
+  // four tiles of one row of tiles to a workgroup; with packed weights four rows of tiles under one column: they read the same weights
+  // at about the same time
+  int64_t zt;
+  int column;
+  if constexpr (WM == kPacked) {
+    const int64_t group = blockIdx.x / tiles_n;
+    column = static_cast<int>(blockIdx.x - group * tiles_n);
+    zt = group * 4 + wave;
+  } else {
+    const int64_t unit = static_cast<int64_t>(blockIdx.x) * 4 + wave;
+    zt = unit / tiles_n;
+    column = static_cast<int>(unit - zt * tiles_n);
+  }
   int tile = column, b = 0;
   while (b < nblocks && tile >= blocks[b].nt) tile -= blocks[b++].nt;
   const int64_t z0 = zt * 32;
-  if (b == nblocks || z0 >= Z) return;
+  // (with weights through LDS a wavefront past the last row stays for the barriers: it reads the last row and stores nothing)
+  if (b == nblocks || (KT == 0 && z0 >= Z)) return;
   const FcBlock blk = blocks[b];
-  float* lsum = fc_lsum + wave * 32 * n2;
+  uint4* wl = reinterpret_cast<uint4*>(fc_lsum);
+  float* lsum = fc_lsum + (KT > 0 ? 16 * 64 * 4 : 0) + wave * 32 * (n2 | 1);
   float* part = DX2 ? partial + static_cast<int64_t>(column) * Z * n2 : nullptr;
   switch (blk.D) {
-    case 1: fc_tile<TI, 1, WT, MI, DX2, MAXD>(blk, parts, coef, A, lda, W, X2, ldx2, X1, ldx1, C, ldc, part, lsum, n2, Z, z0, tile * 32); break;
-    case 3: fc_tile<TI, 3, WT, MI, DX2, MAXD>(blk, parts, coef, A, lda, W, X2, ldx2, X1, ldx1, C, ldc, part, lsum, n2, Z, z0, tile * 32); break;
+    case 1: fc_tile<TI, 1, WM, MI, DX2, MAXD, KT>(blk, parts, coef, A, lda, W, X2, ldx2, X1, ldx1, C, ldc, part, lsum, wl, n2, Z, z0, tile * 32); break;
+    case 3: fc_tile<TI, 3, WM, MI, DX2, MAXD, KT>(blk, parts, coef, A, lda, W, X2, ldx2, X1, ldx1, C, ldc, part, lsum, wl, n2, Z, z0, tile * 32); break;
     default:
-      if constexpr (MAXD > 3) fc_tile<TI, 5, WT, MI, DX2, MAXD>(blk, parts, coef, A, lda, W, X2, ldx2, X1, ldx1, C, ldc, part, lsum, n2, Z, z0, tile * 32);
+      if constexpr (MAXD > 3) fc_tile<TI, 5, WM, MI, DX2, MAXD, KT>(blk, parts, coef, A, lda, W, X2, ldx2, X1, ldx1, C, ldc, part, lsum, wl, n2, Z, z0, tile * 32);
   }
+}
+
+// The weights of every path in the order the matrix instructions take them: fragment (channel of x2, 16 contracted values, 32 columns),
+// 16 bytes per lane.
+template <typename TI>
+__global__ void __launch_bounds__(256) fc_pack_kernel(const FcPack* __restrict__ packs, int npacks, const TI* __restrict__ W, TI* __restrict__ out, int64_t pieces) {
+  int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (i >= pieces) return;
+  int b = 0;
+  while (b + 1 < npacks && i >= packs[b].pieces) i -= packs[b++].pieces;
+  const FcPack q = packs[b];
+  const int nt = (q.N + 31) / 32, lane = static_cast<int>(i & 63), f = static_cast<int>(i >> 6), n = min(f % nt * 32 + (lane & 31), q.N - 1);
+  const int kt = f / nt % q.steps, v = f / nt / q.steps;
+  const uint16_t* __restrict__ src = reinterpret_cast<const uint16_t*>(W) + q.src + static_cast<int64_t>(v) * q.vs + static_cast<int64_t>(n) * q.sn;
+  uint32_t e[8];
+#pragma unroll
+  for (int s = 0; s < 8; ++s) e[s] = kt * 16 < q.K ? src[static_cast<int64_t>(kt * 16 + (lane >> 5) * 8 + s) * q.sk] : 0;
+  *reinterpret_cast<uint4*>(out + q.dst + i * 8) = make_uint4(e[0] | e[1] << 16, e[2] | e[3] << 16, e[4] | e[5] << 16, e[6] | e[7] << 16);
 }
 
 // dx2[z, j] = sum of the partial rows of all column tiles, in order
@@ -272,7 +507,9 @@ __global__ void __launch_bounds__(256) fc_fold_kernel(const float* __restrict__ 
 
 struct FcGrad {  // weight gradient of one path
   int64_t w0;
-  int32_t a0, K, D1, c0, N, D3, coef, j0, d2, nt, ntv, unused;
+  int32_t a0, K, D1, c0, N, D3, coef, j0, d2, nt, ntv;  // nt: 64 x 64 tiles, those of every channel of x2; ntv: across the columns
+  int32_t stride, V, js, vs;                            // as in FcPart
+  uint32_t mask;
 };
 
 template <typename TI, int D1, int D3, bool MI>
@@ -281,6 +518,8 @@ __device__ __forceinline__ void fc_grad_tile(const FcGrad& q, int tile, const fl
                                              int64_t ze) {
   constexpr int ES = sizeof(TI);
   const int lane = threadIdx.x & 63, c = lane & 31, h = lane >> 5;
+  const int per = q.nt / q.V, channel = tile / per;
+  tile -= channel * per;
   const int u0 = (tile / q.ntv) * 64, v0 = (tile % q.ntv) * 64;
   const float* __restrict__ cf = coef + q.coef;
   fx16 acc[2][2];
@@ -300,14 +539,14 @@ __device__ __forceinline__ void fc_grad_tile(const FcGrad& q, int tile, const fl
     constexpr int NI = decltype(ni)::value;
     const int64_t zr = min(z, ze - 1);
     const bool in = z < ze;
-    const TI *xr = X1 + zr * ldx1 + q.a0, *gr = G + zr * ldg + q.c0, *yr = X2 + zr * ldx2 + q.j0;
+    const TI *xr = X1 + zr * ldx1 + q.a0, *gr = G + zr * ldg + q.c0, *yr = X2 + zr * ldx2 + q.j0 + channel * q.vs;
     float s[NI][D3];
 #pragma unroll
     for (int i = 0; i < NI; ++i)
 #pragma unroll
       for (int k = 0; k < D3; ++k) s[i][k] = 0.f;
     for (int j = 0; j < q.d2; ++j) {
-      const float xj = fc_widen(yr + j);
+      const float xj = fc_widen(yr + j * q.js);
 #pragma unroll
       for (int i = 0; i < NI; ++i)
 #pragma unroll
@@ -375,7 +614,7 @@ __device__ __forceinline__ void fc_grad_tile(const FcGrad& q, int tile, const fl
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int uu = u0 + 32 * a + 8 * (r >> 2) + 4 * h + (r & 3);
-        if (uu < q.K) P[q.w0 + static_cast<int64_t>(uu) * q.N + vv] = acc[a][b][r];
+        if (uu < q.K) P[q.w0 + channel * q.N + static_cast<int64_t>(uu) * q.stride + vv] = acc[a][b][r];
       }
     }
 }
@@ -405,6 +644,179 @@ __global__ void __launch_bounds__(256, 2) fc_grad_kernel(const FcGrad* __restric
     case 41: FC_TILE(5, 1); break;
     case 43: FC_TILE(5, 3); break;
     default: FC_TILE(5, 5);
+  }
+#undef FC_TILE
+}
+
+// Weight gradient of 2-byte rows where the x2 blocks have several channels: a workgroup takes 64 x 64 of one path for four channels,
+// one per wavefront, so that the rows of x1 and of the cotangent - transposed into LDS, 32 at a time, the next ones requested
+// meanwhile - serve four channels, and every H_i of a channel serves 64 columns of x1.  54 us for 12 501 rows of 64x0e+64x1o (x)
+// 16x0e+16x1o in bfloat16 (73 with the components tested in the loop; 194 with the products of the operands in memory), bound by the
+// vector instructions that form H.
+constexpr int kDvRows = 32, kDvPad = kDvRows + 8;  // (rows of 80 bytes: 16-byte pieces stay aligned)
+template <typename TI, int D1, int D3, int D2, bool MI>
+__device__ __forceinline__ void fc_grad_channels(const FcGrad& q, int tile, const float* __restrict__ coef, const TI* __restrict__ X1, int64_t ldx1,
+                                                 const TI* __restrict__ X2, int64_t ldx2, const TI* __restrict__ G, int64_t ldg, float* __restrict__ P, int64_t zb,
+                                                 int64_t ze, uint16_t* lds) {
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c = lane & 31, h = lane >> 5;
+  const int per = q.nt / ((q.V + 3) / 4), v0 = tile / per * 4;  // (nt of this table: 64 x 64 tiles times groups of four channels)
+  tile %= per;
+  const int u0 = tile / q.ntv * 64, w0 = tile % q.ntv * 64;
+  uint16_t *xs = lds, *gs = lds + 3 * 64 * kDvPad;
+  float* ys = reinterpret_cast<float*>(lds + 6 * 64 * kDvPad);  // [channel][component][32 rows]
+  const FcCoefs cf(coef + q.coef, D1 * D3 * D2);
+  fx16 acc[2][2];
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b) acc[a][b] = fx16{0};
+
+  // staging: this thread's two rows and four columns of every component
+  const int pair = tid >> 4, col = 4 * (tid & 15);
+  const int uc = min(u0 + col, q.K - 4), wc = min(w0 + col, q.N - 4);
+  uint2 rx[2][D1], rg[2][D3];
+  float ry[3];  // (4 channels x up to 5 components x 32 rows over 256 threads)
+  const int ny = 4 * D2 * kDvRows;
+  auto request = [&](int64_t z) {
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+      const int64_t zr = z + 2 * pair + r;
+      const bool in = zr < ze;
+      const TI *xr = X1 + min(zr, ze - 1) * ldx1 + q.a0, *gr = G + min(zr, ze - 1) * ldg + q.c0;
+#pragma unroll
+      for (int i = 0; i < D1; ++i) {
+        const uint2 t = *reinterpret_cast<const uint2*>(xr + (MI ? uc * D1 + 4 * i : i * q.K + uc));
+        rx[r][i] = in ? t : make_uint2(0, 0);
+      }
+#pragma unroll
+      for (int k = 0; k < D3; ++k) {
+        const uint2 t = *reinterpret_cast<const uint2*>(gr + (MI ? wc * D3 + 4 * k : k * q.N + wc));
+        rg[r][k] = in ? t : make_uint2(0, 0);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 3; ++e) {
+      const int at = tid + 256 * e;
+      ry[e] = 0.f;
+      if (at < ny) {  // a row's values are adjacent threads' (rows slowest)
+        const int row = at / (4 * D2), vj = at - row * (4 * D2), v = vj / D2, j = vj - v * D2;
+        if (z + row < ze && v0 + v < q.V) ry[e] = fc_widen(X2 + (z + row) * ldx2 + q.j0 + (v0 + v) * q.vs + j * q.js);
+      }
+    }
+  };
+  auto stage = [&](auto dc, uint16_t* to, const auto& regs) {
+    constexpr int D = decltype(dc)::value;
+    const uint16_t *e0 = reinterpret_cast<const uint16_t*>(&regs[0][0]), *e1 = reinterpret_cast<const uint16_t*>(&regs[1][0]);
+#pragma unroll
+    for (int m = 0; m < 4 * D; ++m) {
+      const int comp = MI ? m % D : m / 4, cc = col + (MI ? m / D : m % 4);
+      *reinterpret_cast<uint32_t*>(to + (comp * 64 + cc) * kDvPad + 2 * pair) = static_cast<uint32_t>(e0[m]) | static_cast<uint32_t>(e1[m]) << 16;
+    }
+  };
+  request(zb);
+  for (int64_t z = zb; z < ze; z += kDvRows) {
+    __syncthreads();
+    stage(std::integral_constant<int, D1>{}, xs, rx);
+    stage(std::integral_constant<int, D3>{}, gs, rg);
+#pragma unroll
+    for (int e = 0; e < 3; ++e) {
+      const int at = tid + 256 * e;
+      if (at < ny) {
+        const int row = at / (4 * D2), vj = at - row * (4 * D2);
+        ys[vj * kDvRows + row] = ry[e];
+      }
+    }
+    __syncthreads();
+    if (z + kDvRows < ze) request(z + kDvRows);
+    if (v0 + wave < q.V) {
+#pragma unroll 1
+      for (int t = 0; t < kDvRows; t += 16) {
+        uint4 graw[2][D3];
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int k = 0; k < D3; ++k) graw[b][k] = *reinterpret_cast<const uint4*>(gs + (k * 64 + 32 * b + c) * kDvPad + t + 8 * h);
+        const float* yv = ys + wave * D2 * kDvRows + t + 8 * h;
+#pragma unroll
+        for (int i = 0; i < D1; ++i) {
+          float H[2][8];
+#pragma unroll
+          for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) H[b][e] = 0.f;
+#pragma unroll
+          for (int k = 0; k < D3; ++k) {
+            if (!fc_couples<D1, D3, D2>(i, k)) continue;
+            float s[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) s[e] = 0.f;
+#pragma unroll
+            for (int j = 0; j < D2; ++j) {
+              const float f = cf[(i * D3 + k) * D2 + j];
+              const float4 lo = *reinterpret_cast<const float4*>(yv + j * kDvRows), hi = *reinterpret_cast<const float4*>(yv + j * kDvRows + 4);
+              s[0] = fmaf(f, lo.x, s[0]); s[1] = fmaf(f, lo.y, s[1]); s[2] = fmaf(f, lo.z, s[2]); s[3] = fmaf(f, lo.w, s[3]);
+              s[4] = fmaf(f, hi.x, s[4]); s[5] = fmaf(f, hi.y, s[5]); s[6] = fmaf(f, hi.z, s[6]); s[7] = fmaf(f, hi.w, s[7]);
+            }
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+              const uint32_t words[4] = {graw[b][k].x, graw[b][k].y, graw[b][k].z, graw[b][k].w};
+#pragma unroll
+              for (int e = 0; e < 8; ++e)
+                H[b][e] = fmaf(s[e], mm_widen<TI>(static_cast<uint16_t>(e & 1 ? words[e >> 1] >> 16 : words[e >> 1] & 0xffffu)), H[b][e]);
+            }
+          }
+          uint4 hp[2];
+#pragma unroll
+          for (int b = 0; b < 2; ++b) hp[b] = make_uint4(mm_pack<TI>(H[b][0], H[b][1]), mm_pack<TI>(H[b][2], H[b][3]), mm_pack<TI>(H[b][4], H[b][5]), mm_pack<TI>(H[b][6], H[b][7]));
+#pragma unroll
+          for (int a = 0; a < 2; ++a) {
+            const uint4 xf = *reinterpret_cast<const uint4*>(xs + (i * 64 + 32 * a + c) * kDvPad + t + 8 * h);
+#pragma unroll
+            for (int b = 0; b < 2; ++b) acc[a][b] = mm_32x32x16<TI>(xf, hp[b], acc[a][b]);
+          }
+        }
+      }
+    }
+  }
+  if (v0 + wave >= q.V) return;
+  P += q.w0 + static_cast<int64_t>(v0 + wave) * q.N;
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const int w = w0 + 32 * b + c;
+      if (w >= q.N) continue;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int u = u0 + 32 * a + 8 * (r >> 2) + 4 * h + (r & 3);
+        if (u < q.K) P[static_cast<int64_t>(u) * q.stride + w] = acc[a][b][r];
+      }
+    }
+}
+
+template <typename TI, bool MI>
+__global__ void __launch_bounds__(256, 2) fc_grad_channels_kernel(const FcGrad* __restrict__ grads, const float* __restrict__ coef, int ngrads, int tiles,
+                                                                  const TI* __restrict__ X1, int64_t ldx1, const TI* __restrict__ X2, int64_t ldx2,
+                                                                  const TI* __restrict__ G, int64_t ldg, float* __restrict__ partial, int64_t numel, int64_t Z,
+                                                                  int64_t rows_per_chunk, int64_t chunks) {
+  __shared__ __align__(16) uint16_t lds[6 * 64 * kDvPad + 2 * 4 * 5 * kDvRows];
+  const int64_t chunk = blockIdx.x / tiles;
+  int tile = static_cast<int>(blockIdx.x - chunk * tiles), b = 0;
+  if (chunk >= chunks) return;
+  while (b < ngrads && tile >= grads[b].nt) tile -= grads[b++].nt;
+  if (b == ngrads) return;
+  const FcGrad q = grads[b];
+  const int64_t zb = chunk * rows_per_chunk, ze = min(zb + rows_per_chunk, Z);
+  float* P = partial + chunk * numel;
+#define FC_TILE(A, B, C) fc_grad_channels<TI, A, B, C, MI>(q, tile, coef, X1, ldx1, X2, ldx2, G, ldg, P, zb, ze, lds)
+  switch (q.D1 * 8 + q.D3) {
+    case 9: FC_TILE(1, 1, 1); break;
+    case 11: FC_TILE(1, 3, 3); break;
+    case 25: FC_TILE(3, 1, 3); break;
+    default:
+      if (q.d2 == 1) FC_TILE(3, 3, 1);
+      else if (q.d2 == 3) FC_TILE(3, 3, 3);
+      else FC_TILE(3, 3, 5);
   }
 #undef FC_TILE
 }
@@ -484,7 +896,7 @@ __global__ void __launch_bounds__(256) fc_factors_kernel(const FcGrad* __restric
 
 using namespace cueq;
 
-static_assert(sizeof(FcPart) == 40 && sizeof(FcBlock) == 24 && sizeof(FcGrad) == 56, "the tables the host uploads");
+static_assert(sizeof(FcPart) == 56 && sizeof(FcBlock) == 24 && sizeof(FcGrad) == 72 && sizeof(FcPack) == 48, "the tables the host uploads");
 
 #define FC_DISPATCH(dt, CALL)                                      \
   do {                                                             \
@@ -494,34 +906,61 @@ static_assert(sizeof(FcPart) == 40 && sizeof(FcBlock) == 24 && sizeof(FcGrad) ==
   } while (0)
 
 // gradient == 0: rows of x1 against W; 1: rows of the cotangent against W^T, and with X1, partial and dX2 given also the gradient of x2
-extern "C" int cueq_fc_flex(int32_t dtype, int32_t gradient, int32_t mul_ir, int64_t rows, const void* A, int64_t lda, const void* W, const void* X2, int64_t ldx2,
+// packed > 0: W holds the packed weights (2-byte elements) in groups of 2 or 4 steps of 16 contracted values (blocks held in registers, the
+// couplings of fc_couples only), or - 5 - in as many as every block has
+extern "C" int cueq_fc_flex(int32_t dtype, int32_t gradient, int32_t mul_ir, int32_t packed, int64_t rows, const void* A, int64_t lda, const void* W, const void* X2, int64_t ldx2,
                             const void* X1, int64_t ldx1, void* C, int64_t ldc, const void* blocks, int32_t nblocks, const void* parts, const float* coef,
                             int32_t column_tiles, int32_t most_components, int32_t n2, float* partial, void* dX2, void* stream_) {
   hipStream_t stream = static_cast<hipStream_t>(stream_);
   CUEQ_REQUIRE(dtype == CUEQ_F32 || dtype == CUEQ_BF16 || dtype == CUEQ_F16, CUEQ_ERR_UNSUPPORTED, "fc_flex: dtype must be float32, bfloat16 or half");
-  CUEQ_REQUIRE(rows >= 0 && nblocks > 0 && column_tiles > 0 && n2 > 0 && n2 <= 64, CUEQ_ERR_INVALID, "fc_flex: bad extents");
+  CUEQ_REQUIRE(rows >= 0 && nblocks > 0 && column_tiles > 0 && n2 > 0 && n2 <= 128, CUEQ_ERR_INVALID, "fc_flex: bad extents");
+  CUEQ_REQUIRE(!packed || dtype != CUEQ_F32, CUEQ_ERR_UNSUPPORTED, "fc_flex: packed weights are 2-byte elements");
   if (rows == 0) return CUEQ_OK;
   CUEQ_REQUIRE(A && W && X2 && C && blocks && parts && coef && (!dX2 || (gradient && X1 && partial)), CUEQ_ERR_INVALID, "fc_flex: null operand");
   const int64_t epv = dtype == CUEQ_F32 ? 4 : 8;
   CUEQ_REQUIRE(((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(C) | reinterpret_cast<uintptr_t>(W) | reinterpret_cast<uintptr_t>(X1)) & 15) == 0 &&
                    lda % epv == 0 && ldc % epv == 0 && ldx1 % epv == 0,
                CUEQ_ERR_UNSUPPORTED, "fc_flex: rows must be 16-byte aligned");
-  const int64_t units = (rows + 31) / 32 * column_tiles, grid = (units + 3) / 4;
+  const int64_t row_tiles = (rows + 31) / 32;
+  const int64_t grid = packed ? (row_tiles + 3) / 4 * column_tiles : (row_tiles * column_tiles + 3) / 4;
   CUEQ_REQUIRE(grid < (1ll << 31), CUEQ_ERR_TOO_LARGE, "fc_flex: too many rows");
-  const size_t lds = dX2 ? 4 * 32 * n2 * sizeof(float) : 0;
+  const size_t lds = (dX2 ? 4 * 32 * (n2 | 1) * sizeof(float) : 0) + (packed && packed <= 4 && most_components <= 3 ? 16 * 1024 + 4 * 32 * fc_x2_words(n2) * sizeof(uint32_t) : 0);
   KernelTimer timer(gradient ? "fc_flex_dx" : "fc_flex_fwd", stream);
-#define FC_GO(TI, WT, MI, DX) do { if (most_components <= 3) FC_GD(TI, WT, MI, DX, 3); else FC_GD(TI, WT, MI, DX, 5); } while (0)
-#define FC_GD(TI, WT, MI, DX, MD) hipLaunchKernelGGL((fc_rows_kernel<TI, WT, MI, DX, MD>), dim3(static_cast<unsigned>(grid)), dim3(256), lds, stream, static_cast<const FcBlock*>(blocks), static_cast<const FcPart*>(parts), coef, nblocks, column_tiles, static_cast<const TI*>(A), lda, static_cast<const TI*>(W), static_cast<const TI*>(X2), ldx2, static_cast<const TI*>(X1), ldx1, static_cast<TI*>(C), ldc, partial, n2, rows)
-#define FC(TI)                                                                                     \
-  do {                                                                                             \
-    if (!gradient) { if (mul_ir) FC_GO(TI, false, true, false); else FC_GO(TI, false, false, false); } \
-    else if (dX2) { if (mul_ir) FC_GO(TI, true, true, true); else FC_GO(TI, true, false, true); }  \
-    else { if (mul_ir) FC_GO(TI, true, true, false); else FC_GO(TI, true, false, false); }         \
+#define FC_GD(TI, WM, MI, DX, MD, KT)                                                                                                            \
+  do {                                                                                                                                         \
+    if (lds > 64 * 1024)                                                                                                                       \
+      CUEQ_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(fc_rows_kernel<TI, WM, MI, DX, MD, KT>),                                \
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));                                  \
+    FC_GL(TI, WM, MI, DX, MD, KT);                                                                                                             \
+  } while (0)
+#define FC_GL(TI, WM, MI, DX, MD, KT) hipLaunchKernelGGL((fc_rows_kernel<TI, WM, MI, DX, MD, KT>), dim3(static_cast<unsigned>(grid)), dim3(256), lds, stream, static_cast<const FcBlock*>(blocks), static_cast<const FcPart*>(parts), coef, nblocks, column_tiles, static_cast<const TI*>(A), lda, static_cast<const TI*>(W), static_cast<const TI*>(X2), ldx2, static_cast<const TI*>(X1), ldx1, static_cast<TI*>(C), ldc, partial, n2, rows)
+#define FC_GK(TI, MI, DX)                                              \
+  do {                                                                 \
+    if constexpr (sizeof(TI) == 2) {                                   \
+      if (most_components > 3) FC_GD(TI, kPacked, MI, DX, 5, 0);       \
+      else if (packed > 4) FC_GD(TI, kPacked, MI, DX, 3, 0);           \
+      else if (packed > 2) FC_GD(TI, kPacked, MI, DX, 3, 4);           \
+      else FC_GD(TI, kPacked, MI, DX, 3, 2);                           \
+    }                                                                  \
+  } while (0)
+#define FC_GO(TI, WM, MI, DX)                                          \
+  do {                                                                 \
+    if (packed) FC_GK(TI, MI, DX);                                     \
+    else if (most_components <= 3) FC_GD(TI, WM, MI, DX, 3, 0);        \
+    else FC_GD(TI, WM, MI, DX, 5, 0);                                  \
+  } while (0)
+#define FC(TI)                                                                                                    \
+  do {                                                                                                            \
+    if (!gradient) { if (mul_ir) FC_GO(TI, kPlain, true, false); else FC_GO(TI, kPlain, false, false); }          \
+    else if (dX2) { if (mul_ir) FC_GO(TI, kTransposed, true, true); else FC_GO(TI, kTransposed, false, true); }   \
+    else { if (mul_ir) FC_GO(TI, kTransposed, true, false); else FC_GO(TI, kTransposed, false, false); }          \
   } while (0)
   FC_DISPATCH(dtype, FC);
 #undef FC
-#undef FC_GD
 #undef FC_GO
+#undef FC_GK
+#undef FC_GD
+#undef FC_GL
   CUEQ_CHECK_HIP(hipGetLastError());
   if (dX2) {
     const int64_t values = rows * n2;
@@ -533,29 +972,54 @@ extern "C" int cueq_fc_flex(int32_t dtype, int32_t gradient, int32_t mul_ir, int
   return CUEQ_OK;
 }
 
-// partial products of every path's weight gradient: cueq_fc_flex_dw_chunks x numel floats, to be summed in order (cueq_sum_runs)
-static int64_t fc_rows_per_chunk(int64_t rows, int32_t tiles) {
-  int64_t chunks = std::min<int64_t>(8ll * device_cus() / std::max(1, tiles), (rows + 15) / 16);
-  chunks = std::max<int64_t>(1, chunks);
-  return ((rows + chunks - 1) / chunks + 15) / 16 * 16;
+// the weights as cueq_fc_flex takes them with `packed`: pieces of 16 bytes, those of all paths of the table
+extern "C" int cueq_fc_pack(int32_t dtype, const void* W, void* out, const void* packs, int32_t npacks, int64_t pieces, void* stream_) {
+  hipStream_t stream = static_cast<hipStream_t>(stream_);
+  CUEQ_REQUIRE(dtype == CUEQ_BF16 || dtype == CUEQ_F16, CUEQ_ERR_UNSUPPORTED, "fc_pack: dtype must be bfloat16 or half");
+  CUEQ_REQUIRE(npacks > 0 && pieces > 0 && pieces < (1ll << 31) && W && out && packs, CUEQ_ERR_INVALID, "fc_pack: bad extents or null operand");
+  KernelTimer timer("fc_pack", stream);
+  hipLaunchKernelGGL(fc_pack_kernel<uint16_t>, dim3(static_cast<unsigned>((pieces + 255) / 256)), dim3(256), 0, stream, static_cast<const FcPack*>(packs), npacks,
+                     static_cast<const uint16_t*>(W), static_cast<uint16_t*>(out), pieces);
+  CUEQ_CHECK_HIP(hipGetLastError());
+  return CUEQ_OK;
 }
-extern "C" int64_t cueq_fc_flex_dw_chunks(int64_t rows, int32_t tiles) {
-  const int64_t rpc = fc_rows_per_chunk(rows, tiles);
+
+// partial products of every path's weight gradient: cueq_fc_flex_dw_chunks x numel floats, to be summed in order (cueq_sum_runs)
+// (by_channels: fc_grad_channels_kernel, a workgroup per tile and chunk - two for every CU -, else a wavefront)
+static int64_t fc_rows_per_chunk(int64_t rows, int32_t tiles, bool by_channels) {
+  const int64_t step = by_channels ? kDvRows : 16;
+  int64_t chunks = std::min<int64_t>((by_channels ? 2ll : 8ll) * device_cus() / std::max(1, tiles), (rows + step - 1) / step);
+  chunks = std::max<int64_t>(1, chunks);
+  return ((rows + chunks - 1) / chunks + step - 1) / step * step;
+}
+extern "C" int64_t cueq_fc_flex_dw_chunks(int64_t rows, int32_t tiles, int32_t by_channels) {
+  const int64_t rpc = fc_rows_per_chunk(rows, tiles, by_channels != 0);
   return (rows + rpc - 1) / rpc;
 }
-extern "C" int cueq_fc_flex_dw(int32_t dtype, int32_t mul_ir, int64_t rows, const void* X1, int64_t ldx1, const void* X2, int64_t ldx2, const void* G, int64_t ldg,
-                               const void* grads, int32_t ngrads, const float* coef, int32_t tiles, int64_t numel, float* partial, void* stream_) {
+extern "C" int cueq_fc_flex_dw(int32_t dtype, int32_t mul_ir, int32_t by_channels, int64_t rows, const void* X1, int64_t ldx1, const void* X2, int64_t ldx2,
+                               const void* G, int64_t ldg, const void* grads, int32_t ngrads, const float* coef, int32_t tiles, int64_t numel, float* partial,
+                               void* stream_) {
   hipStream_t stream = static_cast<hipStream_t>(stream_);
   CUEQ_REQUIRE(dtype == CUEQ_F32 || dtype == CUEQ_BF16 || dtype == CUEQ_F16, CUEQ_ERR_UNSUPPORTED, "fc_flex_dw: dtype must be float32, bfloat16 or half");
   CUEQ_REQUIRE(rows > 0 && ngrads > 0 && tiles > 0 && numel > 0, CUEQ_ERR_INVALID, "fc_flex_dw: bad extents");
   CUEQ_REQUIRE(X1 && X2 && G && grads && coef && partial, CUEQ_ERR_INVALID, "fc_flex_dw: null operand");
-  const int64_t rpc = fc_rows_per_chunk(rows, tiles), chunks = (rows + rpc - 1) / rpc, grid = (chunks * tiles + 3) / 4;
+  CUEQ_REQUIRE(!by_channels || (dtype != CUEQ_F32 && ((reinterpret_cast<uintptr_t>(X1) | reinterpret_cast<uintptr_t>(G)) & 7) == 0 && ldx1 % 4 == 0 && ldg % 4 == 0),
+               CUEQ_ERR_UNSUPPORTED, "fc_flex_dw: channels together need 2-byte rows in 8-byte pieces");
+  const int64_t rpc = fc_rows_per_chunk(rows, tiles, by_channels != 0), chunks = (rows + rpc - 1) / rpc;
+  const int64_t grid = by_channels ? chunks * tiles : (chunks * tiles + 3) / 4;
   CUEQ_REQUIRE(grid < (1ll << 31), CUEQ_ERR_TOO_LARGE, "fc_flex_dw: too many tiles");
   KernelTimer timer("fc_flex_dw", stream);
-#define FC_GO(TI, MI) hipLaunchKernelGGL((fc_grad_kernel<TI, MI>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, static_cast<const FcGrad*>(grads), coef, ngrads, tiles, static_cast<const TI*>(X1), ldx1, static_cast<const TI*>(X2), ldx2, static_cast<const TI*>(G), ldg, partial, numel, rows, rpc, chunks)
-#define FC(TI) do { if (mul_ir) FC_GO(TI, true); else FC_GO(TI, false); } while (0)
-  FC_DISPATCH(dtype, FC);
+#define FC_GO(KERNEL, TI, MI) hipLaunchKernelGGL((KERNEL<TI, MI>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, static_cast<const FcGrad*>(grads), coef, ngrads, tiles, static_cast<const TI*>(X1), ldx1, static_cast<const TI*>(X2), ldx2, static_cast<const TI*>(G), ldg, partial, numel, rows, rpc, chunks)
+#define FC_CHANNELS(TI) do { if (mul_ir) FC_GO(fc_grad_channels_kernel, TI, true); else FC_GO(fc_grad_channels_kernel, TI, false); } while (0)
+#define FC(TI) do { if (mul_ir) FC_GO(fc_grad_kernel, TI, true); else FC_GO(fc_grad_kernel, TI, false); } while (0)
+  if (by_channels) {
+    if (dtype == CUEQ_F16) FC_CHANNELS(f16bits);
+    else FC_CHANNELS(uint16_t);
+  } else {
+    FC_DISPATCH(dtype, FC);
+  }
 #undef FC
+#undef FC_CHANNELS
 #undef FC_GO
   CUEQ_CHECK_HIP(hipGetLastError());
   return CUEQ_OK;

@@ -1,4 +1,4 @@
-// Fully connected product with shared weights, second operand of multiplicity one: the family of functions product / gradient of
+// Fully connected product with shared weights: the family of functions product / gradient of
 // x1 / of x2 / of the weights, each differentiable in terms of the others, on csrc/fc_flex.hip and - from the measured crossings on -
 // the kernels generated for the descriptor (codegen/fullyconnected.py).
 #include "host.h"
@@ -31,6 +31,15 @@ struct GradShape {  // the weight blocks of one extent: parts (path, component) 
   std::vector<int32_t> first{0};
 };
 
+// 2-byte rows where the second operand has several channels: weights packed for each direction (cueq_fc_pack), weight gradient by
+// groups of four channels
+struct Packed {
+  std::string fwd_blocks, fwd_parts, dx_blocks, dx_parts, fwd_packs, dx_packs, grads;
+  int fwd_longest = 0, dx_longest = 0, grad_tiles = 0;  // grad_tiles == 0: the weight gradient takes the tables of the other types
+  int64_t fwd_pieces = 0, dx_pieces = 0;
+  bool any() const { return fwd_longest > 0; }
+};
+
 struct FcOp {
   int64_t width1 = 0, n2 = 0, width_out = 0, numel = 0;
   bool mul_ir = false, covers_in = true, covers_out = true;
@@ -39,6 +48,7 @@ struct FcOp {
   int fwd_tiles = 0, dx_tiles = 0, grad_tiles = 0;
   std::unordered_map<int, Unit> units;  // by element type code
   std::vector<GradShape> shapes;
+  Packed packed;
   int64_t h_width = 0;
   int factors = 0;
   int64_t tiled_dw_from[2] = {1 << 30, 1 << 30};  // rows, by element size (4, 2)
@@ -47,6 +57,7 @@ struct FcOp {
   struct OnDevice {
     at::Tensor fwd_blocks, fwd_parts, dx_blocks, dx_parts, grads, coef;
     std::vector<at::Tensor> tables;
+    at::Tensor packed_fwd_blocks, packed_fwd_parts, packed_dx_blocks, packed_dx_parts, fwd_packs, dx_packs, packed_grads;
   };
   std::unordered_map<int, OnDevice> devices;
   const OnDevice& on(at::Device device) {
@@ -56,7 +67,13 @@ struct FcOp {
       auto up = [&](const std::string& s) {
         return at::from_blob(const_cast<char*>(s.data()), {static_cast<int64_t>(s.size())}, at::TensorOptions().dtype(at::kByte)).clone().to(device);
       };
-      it = devices.emplace(device.index(), OnDevice{up(fwd_blocks), up(fwd_parts), up(dx_blocks), up(dx_parts), up(grads), up(coef), {}}).first;
+      it = devices.emplace(device.index(), OnDevice{up(fwd_blocks), up(fwd_parts), up(dx_blocks), up(dx_parts), up(grads), up(coef), {}, {}, {}, {}, {}, {}, {}, {}}).first;
+      if (packed.any()) {
+        auto& d = it->second;
+        d.packed_fwd_blocks = up(packed.fwd_blocks), d.packed_dx_blocks = up(packed.dx_blocks);
+        d.packed_fwd_parts = up(packed.fwd_parts), d.packed_dx_parts = up(packed.dx_parts);
+        d.fwd_packs = up(packed.fwd_packs), d.dx_packs = up(packed.dx_packs), d.packed_grads = up(packed.grads);
+      }
       for (const auto& q : shapes) it->second.tables.push_back(at::tensor(q.table, at::kLong).to(device));
     }
     return it->second;
@@ -77,6 +94,16 @@ void launched(int status, const char* what) {
   if (status != 0) throw CueqError(std::string(what) + ": launch failed");
 }
 
+// the weights as the rows kernels read them: as they are, or packed
+at::Tensor weights_for(FcOp& op, const FcOp::OnDevice& t, const at::Tensor& w, bool packed, bool gradient, int code, hipStream_t stream) {
+  if (!packed) return w;
+  const at::Tensor& packs = gradient ? t.dx_packs : t.fwd_packs;
+  const int64_t pieces = gradient ? op.packed.dx_pieces : op.packed.fwd_pieces;
+  at::Tensor out = at::empty({pieces * 8}, w.options());
+  check(lib().cueq_fc_pack(code, w.data_ptr(), out.data_ptr(), packs.data_ptr(), static_cast<int>(packs.numel() / 48), pieces, stream), "cueq_fc_pack");
+  return out;
+}
+
 at::Tensor product(FcOp& op, const at::Tensor& w_, const at::Tensor& x1_, const at::Tensor& x2_, at::ScalarType dtype) {
   const at::Device device = x1_.device();
   const c10::DeviceGuard guard(device);
@@ -94,8 +121,10 @@ at::Tensor product(FcOp& op, const at::Tensor& w_, const at::Tensor& x1_, const 
     return out;
   }
   const auto& t = op.on(device);
-  check(lib().cueq_fc_flex(code, 0, op.mul_ir, Z, x1.data_ptr(), op.width1, w.data_ptr(), x2.data_ptr(), op.n2, nullptr, 0, out.data_ptr(), op.width_out,
-                           t.fwd_blocks.data_ptr(), static_cast<int>(t.fwd_blocks.numel() / 24), t.fwd_parts.data_ptr(),
+  const bool packed = op.packed.any() && dtype != at::kFloat;
+  const at::Tensor ww = weights_for(op, t, w, packed, false, code, stream);
+  check(lib().cueq_fc_flex(code, 0, op.mul_ir, packed ? op.packed.fwd_longest : 0, Z, x1.data_ptr(), op.width1, ww.data_ptr(), x2.data_ptr(), op.n2, nullptr, 0, out.data_ptr(), op.width_out,
+                           (packed ? t.packed_fwd_blocks : t.fwd_blocks).data_ptr(), static_cast<int>(t.fwd_blocks.numel() / 24), (packed ? t.packed_fwd_parts : t.fwd_parts).data_ptr(),
                            static_cast<const float*>(t.coef.data_ptr()), op.fwd_tiles, op.most, static_cast<int>(op.n2), nullptr, nullptr, stream),
         "cueq_fc_flex");
   return out;
@@ -150,9 +179,11 @@ Grads gradients(FcOp& op, const at::Tensor& w_, const at::Tensor& x1_, const at:
       at::Tensor part, dx1 = r.x1;
       if (need_2) part = new_tensor({op.dx_tiles, Z, op.n2}, at::kFloat, device);
       if (!dx1.defined()) dx1 = at::empty({Z, op.width1}, options);  // (the gradient of x2 comes from the same products)
-      check(lib().cueq_fc_flex(code, 1, op.mul_ir, Z, g.data_ptr(), op.width_out, w.data_ptr(), second.data_ptr(), op.n2, need_2 ? x1.data_ptr() : nullptr,
-                               need_2 ? op.width1 : 0, dx1.data_ptr(), op.width1, t.dx_blocks.data_ptr(), static_cast<int>(t.dx_blocks.numel() / 24),
-                               t.dx_parts.data_ptr(), static_cast<const float*>(t.coef.data_ptr()), op.dx_tiles, op.most, static_cast<int>(op.n2),
+      const bool packed = op.packed.any() && dtype != at::kFloat;
+      const at::Tensor ww = weights_for(op, t, w, packed, true, code, stream);
+      check(lib().cueq_fc_flex(code, 1, op.mul_ir, packed ? op.packed.dx_longest : 0, Z, g.data_ptr(), op.width_out, ww.data_ptr(), second.data_ptr(), op.n2, need_2 ? x1.data_ptr() : nullptr,
+                               need_2 ? op.width1 : 0, dx1.data_ptr(), op.width1, (packed ? t.packed_dx_blocks : t.dx_blocks).data_ptr(), static_cast<int>(t.dx_blocks.numel() / 24),
+                               (packed ? t.packed_dx_parts : t.dx_parts).data_ptr(), static_cast<const float*>(t.coef.data_ptr()), op.dx_tiles, op.most, static_cast<int>(op.n2),
                                need_2 ? part.data_ptr<float>() : nullptr, need_2 ? r.x2.data_ptr() : nullptr, stream),
             "cueq_fc_flex");
     }
@@ -165,7 +196,7 @@ Grads gradients(FcOp& op, const at::Tensor& w_, const at::Tensor& x1_, const at:
       const auto& t = op.on(device);
       at::Tensor H = at::empty({Z, op.h_width}, options), x1t = op.mul_ir ? at::empty({Z, op.width1}, options) : x1;
       check(lib().cueq_fc_factors(code, op.mul_ir, Z, x1.data_ptr(), op.width1, x2.data_ptr(), op.n2, g.data_ptr(), op.width_out, t.grads.data_ptr(),
-                                  static_cast<int>(t.grads.numel() / 56), static_cast<const float*>(t.coef.data_ptr()), t.dx_blocks.data_ptr(),
+                                  static_cast<int>(t.grads.numel() / 72), static_cast<const float*>(t.coef.data_ptr()), t.dx_blocks.data_ptr(),
                                   static_cast<int>(t.dx_blocks.numel() / 24), op.factors, H.data_ptr(), op.h_width, op.mul_ir ? x1t.data_ptr() : nullptr, stream),
             "cueq_fc_factors");
       for (size_t i = 0; i < op.shapes.size(); ++i) {
@@ -182,15 +213,18 @@ Grads gradients(FcOp& op, const at::Tensor& w_, const at::Tensor& x1_, const at:
       r.w = w_dtype == out_dtype ? gw : gw.to(w_dtype);
       return r;
     }
-    const int64_t chunks = u ? u->dw_blocks(Z) : lib().cueq_fc_flex_dw_chunks(Z, op.grad_tiles);
+    const bool by_channels = op.packed.grad_tiles > 0 && dtype != at::kFloat;
+    const int grad_tiles = by_channels ? op.packed.grad_tiles : op.grad_tiles;
+    const int64_t chunks = u ? u->dw_blocks(Z) : lib().cueq_fc_flex_dw_chunks(Z, grad_tiles, by_channels);
     at::Tensor part = new_tensor({chunks, op.numel}, at::kFloat, device);
     if (u) {
       launched(u->dw(Z, x1.data_ptr(), op.width1, x2.data_ptr(), op.n2, g.data_ptr(), op.width_out, part.data_ptr<float>(), op.numel, stream),
                "fully connected weight gradient");
     } else {
       const auto& t = op.on(device);
-      check(lib().cueq_fc_flex_dw(code, op.mul_ir, Z, x1.data_ptr(), op.width1, x2.data_ptr(), op.n2, g.data_ptr(), op.width_out, t.grads.data_ptr(),
-                                  static_cast<int>(t.grads.numel() / 56), static_cast<const float*>(t.coef.data_ptr()), op.grad_tiles, op.numel,
+      const at::Tensor& table = by_channels ? t.packed_grads : t.grads;
+      check(lib().cueq_fc_flex_dw(code, op.mul_ir, by_channels, Z, x1.data_ptr(), op.width1, x2.data_ptr(), op.n2, g.data_ptr(), op.width_out, table.data_ptr(),
+                                  static_cast<int>(table.numel() / 72), static_cast<const float*>(t.coef.data_ptr()), grad_tiles, op.numel,
                                   part.data_ptr<float>(), stream),
             "cueq_fc_flex_dw");
     }
@@ -384,6 +418,14 @@ void bind_fully_connected(py::module_& m) {
           op.factors += d * t[5].cast<int>();
         }
         op.h_width = h;
+      })
+      .def("add_packed", [](FcOp& op, const py::tuple& tables, const py::tuple& longest, const py::tuple& pieces, int grad_tiles) {
+        auto& p = op.packed;
+        p.fwd_blocks = tables[0].cast<std::string>(), p.fwd_parts = tables[1].cast<std::string>();
+        p.dx_blocks = tables[2].cast<std::string>(), p.dx_parts = tables[3].cast<std::string>();
+        p.fwd_packs = tables[4].cast<std::string>(), p.dx_packs = tables[5].cast<std::string>(), p.grads = tables[6].cast<std::string>();
+        p.fwd_longest = longest[0].cast<int>(), p.dx_longest = longest[1].cast<int>(), p.grad_tiles = grad_tiles;
+        p.fwd_pieces = pieces[0].cast<int64_t>(), p.dx_pieces = pieces[1].cast<int64_t>();
       })
       .def("takes", [](const FcOp& op, const at::Tensor& x) { return op.takes(x.scalar_type()); })
       .def("direct", &direct)

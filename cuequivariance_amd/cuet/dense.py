@@ -19,6 +19,7 @@ from __future__ import annotations
 import ctypes as C
 import json
 import struct
+from types import SimpleNamespace
 import threading
 from collections import OrderedDict
 from typing import Dict, List, Optional
@@ -315,18 +316,21 @@ def _linear_op(mod: "SegmentedPolynomialDense"):
     return op
 
 
-def _fc_tables(mod: "SegmentedPolynomialDense"):
-    """Packed tables of ``csrc/fc_flex.hip`` for ``uvw,iu,jv,kw+ijk`` with ``v = 1``: ``((blocks and parts forward, of the input
-    gradient, weight gradients, coefficients), tiles, element sizes served, most components)``, or ``None``."""
+def _fc_tables(mod, x2_mul_ir: bool = False):
+    """Packed tables of ``csrc/fc_flex.hip`` for a product ``uvw,iu,jv,kw+ijk`` (any ``v``; ``uw,iu,j,kw+ijk`` is ``v = 1``), the second
+    operand's rows in ``ir_mul`` or ``mul_ir``: ``((blocks and parts forward, of the input gradient, weight gradients, coefficients),
+    tiles, element sizes served, most components, paths, packed tables)``, or ``None``."""
     ope, stp = mod._polynomial_orig.operations[0]
     if str(stp.subscripts) not in ("uvw,iu,jv,kw+ijk", "uw,iu,j,kw+ijk") or not stp.paths:
         return None
     offs = [o.segment_offsets() for o in stp.operands]
+    sizes = [o.size for o in stp.operands]
     coef: list = []
-    paths = []  # (w0, a0, K, D1, c0, N, D3, coefficients as [i, k, j], as [k, i, j], j0, d2)
+    paths = []
     for p in stp.paths:
         sw, s1, s2, so = p.indices
         (d1, K), d2, (d3, N) = stp.operands[1][s1], stp.operands[2][s2][0], stp.operands[3][so]
+        V = stp.operands[0][sw][1] if len(stp.operands[0][sw]) == 3 else 1
         c = p.coefficients
         if d1 not in (1, 3, 5) or d3 not in (1, 3, 5):
             return None
@@ -334,40 +338,74 @@ def _fc_tables(mod: "SegmentedPolynomialDense"):
         coef += [float(v) for v in c.transpose(0, 2, 1).reshape(-1)]
         back = len(coef)
         coef += [float(v) for v in c.transpose(2, 0, 1).reshape(-1)]
-        paths.append((offs[0][sw], offs[1][s1], K, d1, offs[3][so], N, d3, at, back, offs[2][s2], d2))
-    if len({p[0] for p in paths}) != len(paths) or sum(p[2] * p[5] for p in paths) != mod.input_sizes[0] or mod.input_sizes[2] > 64:
+        used = (c != 0).any(axis=1)  # (i, k)
+        mask = sum(1 << (i * d3 + k) for i in range(d1) for k in range(d3) if used[i, k])
+        mask_back = sum(1 << (k * d1 + i) for i in range(d1) for k in range(d3) if used[i, k])
+        paths.append(SimpleNamespace(w0=offs[0][sw], a0=offs[1][s1], K=K, d1=d1, c0=offs[3][so], N=N, d3=d3, coef=at, coef_back=back, j0=offs[2][s2],
+                                     d2=d2, V=V, js=1 if x2_mul_ir else V, vs=d2 if x2_mul_ir else 1, mask=mask, mask_back=mask_back))
+    if len({p.w0 for p in paths}) != len(paths) or sum(p.K * p.V * p.N for p in paths) != sizes[0] or sizes[2] > 128:
         return None
     served = 0
     for bit, epv, step in ((1, 4, 8), (2, 8, 16)):
-        if (all(v % epv == 0 for p in paths for v in (p[0], p[1], p[4])) and all(p[2] % step == 0 and p[5] % step == 0 for p in paths)
-                and mod.input_sizes[1] % epv == 0 and mod.out_size % epv == 0):
+        if (all(v % epv == 0 for p in paths for v in (p.w0, p.a0, p.c0)) and all(p.K % step == 0 and p.N % step == 0 for p in paths)
+                and sizes[1] % epv == 0 and sizes[3] % epv == 0):
             served |= bit
     if not served:
         return None
 
-    def side(block, part):
+    # the couplings that the kernels with straight loops over the channels of x2 know (fc_couples); blocks held in registers there
+    # have up to 64 values
+    diagonal, all9 = 0b100010001, 0b111111111
+    allowed = {(1, 1, 1): 1, (1, 3, 3): 7, (3, 3, 1): 7, (3, 1, 3): diagonal, (3, 3, 3): all9 & ~diagonal, (3, 5, 3): all9}  # (d1, d2, d3)
+    straight = all((p.d1, p.d2, p.d3) in allowed and not (p.mask | p.mask_back) & ~allowed[p.d1, p.d2, p.d3] for p in paths)
+    resident = straight and all(p.K <= 64 and p.N <= 64 for p in paths)
+    steps = {True: 2 if all(p.N <= 32 for p in paths) else 4, False: 2 if all(p.K <= 32 for p in paths) else 4}  # (by direction: of 16 values)
+
+    def side(gradient, packed=None):
+        """Blocks (of the result; ``gradient``: of x1), parts - one per path, or per path and channel of x2 -, column tiles, and,
+        ``packed``, where every path's weights are put."""
         by = {}
         for p in paths:
-            by.setdefault(block(p), []).append(p)
-        blocks, parts, tiles = b"", b"", 0
-        for (c0, n, d), ps in sorted(by.items(), key=lambda kv: -sum(part(p)[3] for p in kv[1])):  # (the longest units first)
+            by.setdefault((p.a0, p.K, p.d1) if gradient else (p.c0, p.N, p.d3), []).append(p)
+        blocks, parts, tiles, packs, at = b"", b"", 0, b"", 0
+        components = lambda p: p.d3 if gradient else p.d1
+        for (c0, n, d), ps in sorted(by.items(), key=lambda kv: -sum(components(p) * p.V for p in kv[1])):  # (the longest units first)
             nt = -(-n // 32)
-            blocks += struct.pack("<6i", c0, n, d, len(parts) // 40, len(ps), nt)
+            together = packed and resident
+            blocks += struct.pack("<6i", c0, n, d, len(parts) // 56, sum(1 if together else p.V for p in ps), nt)
             tiles += nt
             for p in ps:
-                parts += struct.pack("<q8i", *part(p), 0)
-        return blocks, parts, tiles
+                source, K, co, mask = (p.c0, p.N, p.coef_back, p.mask_back) if gradient else (p.a0, p.K, p.coef, p.mask)
+                w0, stride, wv = p.w0, p.V * p.N, p.N
+                if packed:  # (fragments of 512 elements: channel, 16 contracted values, 32 columns)
+                    ks = steps[gradient] if resident else K // 16
+                    pieces = p.V * ks * nt * 64
+                    sk, sn = (1, p.V * p.N) if gradient else (p.V * p.N, 1)
+                    packs += struct.pack("<2q8i", p.w0, at, K, n, sk, sn, p.V, p.N, pieces, ks)
+                    w0, stride, wv = at, nt, ks * nt * 512
+                    at += pieces * 8
+                for v in range(1 if together else p.V):
+                    parts += struct.pack("<q11iI", w0 + v * wv, source, K, components(p), co, p.j0 + v * p.vs, p.d2, stride, p.V if together else 1,
+                                         p.js, p.vs, wv, mask)
+        return blocks, parts, tiles, packs, at // 8
 
-    fwd = side(lambda p: (p[4], p[5], p[6]), lambda p: (p[0], p[1], p[2], p[3], p[7], p[9], p[10], p[5]))
-    dx = side(lambda p: (p[1], p[2], p[3]), lambda p: (p[0], p[4], p[5], p[6], p[8], p[9], p[10], p[5]))
-    grads, tiles = b"", 0
-    for p in sorted(paths, key=lambda p: -p[3]):
-        ntv = -(-p[5] // 64)
-        nt = ntv * -(-p[2] // 64)
-        grads += struct.pack("<q12i", p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7], p[9], p[10], nt, ntv, 0)
-        tiles += nt
-    return ((fwd[0], fwd[1], dx[0], dx[1], grads, struct.pack(f"<{len(coef)}f", *coef)), (fwd[2], dx[2], tiles), served,
-            max(max(p[3], p[6]) for p in paths), [(p[0], p[1], p[2], p[3], p[5], p[6]) for p in sorted(paths, key=lambda p: -p[3])])
+    def grads(by_channels):
+        table, tiles = b"", 0
+        for p in sorted(paths, key=lambda p: -p.d1):
+            ntv = -(-p.N // 64)
+            nt = ntv * -(-p.K // 64) * (-(-p.V // 4) if by_channels else p.V)
+            table += struct.pack("<q15iI", p.w0, p.a0, p.K, p.d1, p.c0, p.N, p.d3, p.coef, p.j0, p.d2, nt, ntv, p.V * p.N, p.V, p.js, p.vs, p.mask)
+            tiles += nt
+        return table, tiles
+
+    fwd, dx, dw = side(False), side(True), grads(False)
+    packed = None
+    if served & 2 and any(p.V > 1 for p in paths):
+        pf, px = side(False, True), side(True, True)
+        pw = grads(True) if straight else (b"", 0)
+        packed = ((pf[0], pf[1], px[0], px[1], pf[3], px[3], pw[0]), (steps[False], steps[True]) if resident else (5, 5), (pf[4], px[4]), pw[1])
+    return ((fwd[0], fwd[1], dx[0], dx[1], dw[0], struct.pack(f"<{len(coef)}f", *coef)), (fwd[2], dx[2], dw[1]), served,
+            max(max(p.d1, p.d3) for p in paths), [(p.w0, p.a0, p.K, p.d1, p.N, p.d3) for p in sorted(paths, key=lambda p: -p.d1)], packed)
 
 
 # Rows from which on the generated kernels are the faster ones (forward, input gradients, weight gradient), by element size: always,
@@ -387,6 +425,62 @@ def _fc_op(mod: "SegmentedPolynomialDense"):
     # from these rows on (float, 2-byte) the weight gradient's factors go through memory to the tiled product (measured crossings)
     op.add_tiled_dw(tables[4], 13_000, 6_000)
     return op
+
+
+class GeneralFullyConnected:
+    """``uvw,iu,jv,kw+ijk`` with shared weights and a second operand of any multiplicity on the rows kernels of ``csrc/fc_flex.hip``, as
+    the host module runs it: the products of the two operands are formed in registers.  Rows of the first operand and of the
+    result in ``ir_mul`` or ``mul_ir`` (``rows_mul_ir``), rows of the second in either (``x2_mul_ir``)."""
+
+    def __init__(self, polynomial: cue.SegmentedPolynomial, rows_mul_ir: bool = False, x2_mul_ir: bool = False):
+        self._polynomial_orig, self.rows_mul_ir, self.x2_mul_ir = polynomial, rows_mul_ir, x2_mul_ir
+        self._op = False
+
+    @staticmethod
+    def build(polynomial: cue.SegmentedPolynomial, rows_mul_ir: bool = False, x2_mul_ir: bool = False):
+        """``None`` for other forms; what of this form the kernels do not take is found out at the first call."""
+        if len(polynomial.operations) != 1 or polynomial.num_inputs != 3 or polynomial.num_outputs != 1:
+            return None
+        ope, stp = polynomial.operations[0]
+        if tuple(ope.buffers) != (0, 1, 2, 3) or str(stp.subscripts) != "uvw,iu,jv,kw+ijk":
+            return None
+        return GeneralFullyConnected(polynomial, rows_mul_ir, x2_mul_ir)
+
+    def __reduce__(self):
+        return (GeneralFullyConnected, (self._polynomial_orig, self.rows_mul_ir, self.x2_mul_ir))
+
+    @property
+    def op(self):
+        if self._op is False:
+            stp = self._polynomial_orig.operations[0][1]
+            tables = _fc_tables(self, self.x2_mul_ir)
+            if tables is None:
+                self._op = None
+                return None
+            self._long = max(max(stp.operands[1][p.indices[1]][1], stp.operands[3][p.indices[3]][1]) for p in stp.paths) > 64
+            covered = [{p.indices[i] for p in stp.paths} == set(range(stp.operands[i].num_segments)) for i in (1, 3)]
+            op = _lib.host().FcOp(stp.operands[1].size, stp.operands[2].size, stp.operands[3].size, stp.operands[0].size, self.rows_mul_ir, *covered,
+                                  tables[2], tables[3], tables[0], tables[1])
+            if tables[5] is not None:
+                op.add_packed(*tables[5])
+            self._op = op
+        return self._op
+
+    def __call__(self, w: torch.Tensor, x1: torch.Tensor, x2: torch.Tensor):
+        """The product, or ``None`` unless it is a plain eager call of shapes and types the kernels take."""
+        if (torch.compiler.is_compiling() or torch.jit.is_tracing() or not w.is_cuda or not (w.dtype == x1.dtype == x2.dtype) or x1.dtype not in _MATRIX_CORE
+                or any(type(t) not in (torch.Tensor, torch.nn.Parameter) for t in (w, x1, x2))):
+            return None
+        if self.op is None:
+            return None
+        # Blocks of up to 64 values: always (64x0e+64x1o (x) 16x0e+16x1o, 50 000 rows, a training step: bfloat16 596 us against 2 879 with
+        # the products in memory, float 3 107 against 5 108).  Longer ones do not stay in registers, and the tiled products of the
+        # other way overtake: with 128x0e (x) 128x0e from 1 000 rows on (bfloat16 853 against 721 us); with ten channels 2-byte rows
+        # do at 20 000 (128x0e+128x1o+128x2e (x) 10x0e: 327 against 618 us for 1 000 rows, 2 575 against 2 081), float rows do not
+        # (50 000 rows: 7.4 against 8.3 ms).
+        if self._long and (x2.shape[-1] > 16 or (x1.element_size() == 2 and x1.shape[0] > 4000)):
+            return None
+        return self.op.direct(w, x1, x2)
 
 
 def _rows_tables(K: int, N: int, plist):

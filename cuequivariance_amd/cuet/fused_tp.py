@@ -377,7 +377,7 @@ class SegmentedPolynomialFusedTP(nn.Module):
     def __init__(self, polynomial: cue.SegmentedPolynomial, math_dtype=None, output_dtype_map: Optional[List[int]] = None,
                  name: str = "segmented_polynomial", rows: str = "ir_mul", row_blocks=None):
         super().__init__()
-        from .dense import SegmentedPolynomialDense
+        from .dense import GeneralFullyConnected, SegmentedPolynomialDense
 
         self._rows_orig, self._row_blocks_orig = rows, row_blocks
 
@@ -431,6 +431,10 @@ class SegmentedPolynomialFusedTP(nn.Module):
                 self.composed = _MatrixWithElementwiseStage(polynomial, math_dtype, name)
             except NotImplementedError:
                 self.composed = None
+        # (the fully connected form with a second operand of any multiplicity, products formed in registers: no stage in memory)
+        self.general = None
+        if self.dense is None and rows != "mul_ir" and self.composed is not None and math_dtype in (None, torch.float32) and self.dtypes[-1] >= 0:
+            self.general = GeneralFullyConnected.build(polynomial)
         if rows == "mul_ir" and self.dense is None:
             raise NotImplementedError("fused_tp: rows='mul_ir' is served by the matrix-core executor only")
         # one flattened executor per operation: (module, input buffers it reads, output it adds to)
@@ -470,6 +474,10 @@ class SegmentedPolynomialFusedTP(nn.Module):
                 and inputs[self.dense_perm[0]].shape[0] == 1 and inputs[0].dtype in (torch.float32, torch.float64, torch.bfloat16, torch.float16)
                 and all(t.dtype == inputs[0].dtype for t in inputs)):
             return self.dense([inputs[i] for i in self.dense_perm], input_indices, output_shapes, output_indices)
+        if self.general is not None and not input_indices and not output_indices and not output_shapes and len(inputs) == 3:
+            out = self.general(*inputs)
+            if out is not None:
+                return [out]
         if (self.composed is not None and self.composed.scalar_paths >= self.stages_from and not input_indices and not output_indices and not output_shapes and inputs[0].is_cuda
                 and inputs[self.composed.iw].shape[0] == 1 and inputs[0].dtype in (torch.float32, torch.float64, torch.bfloat16, torch.float16)
                 and all(t.dtype == inputs[0].dtype for t in inputs)

@@ -23,6 +23,7 @@ import torch
 
 from .. import cue
 from ..cue import descriptors
+from .dense import GeneralFullyConnected
 from .script import scriptable
 from .segmented_polynomial import SegmentedPolynomial
 from .transpose import TransposeIrrepsLayout, apply_layout
@@ -408,6 +409,13 @@ class FullyConnectedTensorProduct(torch.nn.Module):
             except (NotImplementedError, ValueError):
                 self.f_rows = None
 
+        # a second operand of multiplicity above one: rows in either layout as they lie (first operand and result in the same one)
+        self.general = None
+        if self.f is not None and getattr(self.f.m, "general", None) is not None:
+            mul_ir = [t.source == cue.mul_ir for t in (self.transpose_in1, self.transpose_in2)] + [self.transpose_out.target == cue.mul_ir]
+            if mul_ir[0] == mul_ir[2] and all(x.layout == cue.ir_mul for x in (e.inputs[1], e.inputs[2], e.outputs[0])):
+                self.general = GeneralFullyConnected.build(e.polynomial, mul_ir[0], mul_ir[1])
+
     def extra_repr(self) -> str:
         return (
             f"shared_weights={self.shared_weights}, internal_weights={self.internal_weights}, "
@@ -430,6 +438,10 @@ class FullyConnectedTensorProduct(torch.nn.Module):
             raise ValueError("Internal weights are not used, weight should not be None")
         if indices_1 is None and indices_out is None and not torch.compiler.is_compiling() and type(x1) is torch.Tensor:
             # the whole call in native code when it is a plain one; anything else, and every error, takes the way below
+            if self.general is not None:
+                out = self.general(weight, x1, x2)
+                if out is not None:
+                    return out
             dense = self._dense()
             if dense is not None and dense.fc_takes(x1, x2):
                 out = dense.fully_connected.direct(weight, x1, x2)

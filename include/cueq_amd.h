@@ -470,14 +470,19 @@ int cueq_sum_runs(const float* partial, int32_t per, int32_t nruns, const int32_
  * fill the chip with the generated kernels and for extents those do not take.  gradient == 0: rows of x1 against the weights;
  * 1: rows of the cotangent against the weights read transposed - with X1, partial (column_tiles x rows x n2 floats) and dX2
  * given also the gradient of x2 from the same products.  `blocks`, `parts`, `grads` are device tables (FcBlock, FcPart, FcGrad of
- * csrc/fc_flex.hip), `coef` the path coefficients; multiplicities multiples of 8 (float32) / 16, components 1, 3 or 5. */
-int cueq_fc_flex(int32_t dtype, int32_t gradient, int32_t mul_ir, int64_t rows, const void* A, int64_t lda, const void* W,
+ * csrc/fc_flex.hip), `coef` the path coefficients; multiplicities multiples of 8 (float32) / 16, components 1, 3 or 5; blocks of x2
+ * of any multiplicity, n2 <= 128.  packed (2-byte elements): W as cueq_fc_pack lays it, `packed` the steps
+ * of 16 contracted values of every fragment group (2 or 4, zeros past the block), or 5: as many as the block has. */
+int cueq_fc_flex(int32_t dtype, int32_t gradient, int32_t mul_ir, int32_t packed, int64_t rows, const void* A, int64_t lda, const void* W,
                  const void* X2, int64_t ldx2, const void* X1, int64_t ldx1, void* C, int64_t ldc, const void* blocks,
                  int32_t nblocks, const void* parts, const float* coef, int32_t column_tiles, int32_t most_components, int32_t n2,
                  float* partial, void* dX2, void* stream);
-/* Partial products of the weight gradient, cueq_fc_flex_dw_chunks x numel floats to be summed in order (cueq_sum_runs). */
-int64_t cueq_fc_flex_dw_chunks(int64_t rows, int32_t tiles);
-int cueq_fc_flex_dw(int32_t dtype, int32_t mul_ir, int64_t rows, const void* X1, int64_t ldx1, const void* X2, int64_t ldx2,
+/* The weights of all paths in the order of the matrix instructions' operands (table of FcPack), `pieces` of 16 bytes. */
+int cueq_fc_pack(int32_t dtype, const void* W, void* out, const void* packs, int32_t npacks, int64_t pieces, void* stream);
+/* Partial products of the weight gradient, cueq_fc_flex_dw_chunks x numel floats to be summed in order (cueq_sum_runs).  by_channels
+ * (2-byte elements): four channels of an x2 block to a workgroup, `tiles` and the table's counts for groups of four. */
+int64_t cueq_fc_flex_dw_chunks(int64_t rows, int32_t tiles, int32_t by_channels);
+int cueq_fc_flex_dw(int32_t dtype, int32_t mul_ir, int32_t by_channels, int64_t rows, const void* X1, int64_t ldx1, const void* X2, int64_t ldx2,
                     const void* G, int64_t ldg, const void* grads, int32_t ngrads, const float* coef, int32_t tiles, int64_t numel,
                     float* partial, void* stream);
 /* For many rows: H (rows x ldh: for every path of `grads`, in order, D1 x N columns sum_k s_ik g_k), which the weight gradient then
