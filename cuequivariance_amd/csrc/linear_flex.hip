@@ -41,11 +41,15 @@ __device__ __forceinline__ uint32_t pick2(const uint4* run, int i0, int i1) {  /
 }
 
 // one tile: rows z0 .. z0 + 32 ZT, columns n0 .. n0 + 32 of the block.  WT: the weights are read transposed (input gradient).
-template <typename TI, int D, int ZT, bool WT>
+// SK: wavefronts that share the tile, each with its part of every contraction; the first adds the others' sums, in order, through
+// LDS and stores (SK > 1: all SK wavefronts of the workgroup are here).
+template <typename TI, int D, int ZT, bool WT, int SK>
 __device__ __forceinline__ void flex_tile(const FlexBlock& blk, const FlexPart* __restrict__ parts, const TI* __restrict__ A, int64_t lda, const TI* __restrict__ W,
                                           TI* __restrict__ C, int64_t ldc, int64_t Z, int64_t z0, int n0) {
   constexpr int ES = sizeof(TI), EPV = 16 / ES, STEP = 2 * EPV;  // channels per step: 4 + 4 (float), 8 + 8
+  static_assert(SK == 1 || ZT == 1, "a shared tile has 32 rows");
   const int lane = threadIdx.x & 63, c = lane & 31, h = lane >> 5;
+  const int share = SK > 1 ? __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)) : 0;
   fx16 acc[ZT][D];
 #pragma unroll
   for (int t = 0; t < ZT; ++t)
@@ -88,9 +92,11 @@ __device__ __forceinline__ void flex_tile(const FlexBlock& blk, const FlexPart* 
         ww = make_uint4(e[0] | e[1] << 16, e[2] | e[3] << 16, e[4] | e[5] << 16, e[6] | e[7] << 16);
       }
     };
-    load(0, x, wv);
-    for (int k0 = 0; k0 < part.K; k0 += STEP) {
-      load(min(k0 + STEP, part.K - STEP), xn, wn);
+    const int steps = part.K / STEP, first = SK > 1 ? steps * share / SK * STEP : 0, last = SK > 1 ? steps * (share + 1) / SK * STEP : part.K;
+    if (SK > 1 && first == last) continue;
+    load(first, x, wv);
+    for (int k0 = first; k0 < last; k0 += STEP) {
+      load(min(k0 + STEP, last - STEP), xn, wn);
 #pragma unroll
       for (int t = 0; t < ZT; ++t) {
         if constexpr (ES == 4) {
@@ -117,6 +123,23 @@ __device__ __forceinline__ void flex_tile(const FlexBlock& blk, const FlexPart* 
         for (int i = 0; i < D; ++i) x[t][i] = xn[t][i];
       wv = wn;
     }
+  }
+  if constexpr (SK > 1) {
+    __shared__ float others[SK - 1][16][64];
+#pragma unroll
+    for (int i = 0; i < D; ++i) {
+      if (share)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) others[share - 1][r][lane] = acc[0][i][r];
+      __syncthreads();
+      if (!share)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+#pragma unroll
+          for (int o = 0; o < SK - 1; ++o) acc[0][i][r] += others[o][r][lane];
+      __syncthreads();
+    }
+    if (share) return;
   }
 #pragma unroll
   for (int t = 0; t < ZT; ++t) {
@@ -145,12 +168,13 @@ __device__ __forceinline__ void flex_tile(const FlexBlock& blk, const FlexPart* 
 }
 
 // unit = (column tiles of the blocks one after the other) x (row tile); the column tile runs fastest, so a block's wavefronts share rows
-template <typename TI, bool WT, int ZBIG>
+// (SK > 1: a workgroup per unit)
+template <typename TI, bool WT, int ZBIG, int SK>
 __global__ void __launch_bounds__(256, 2) flex_rows_kernel(const FlexBlock* __restrict__ blocks, const FlexPart* __restrict__ parts, int nblocks, int tiles_n,
                                                            const TI* __restrict__ A, int64_t lda, const TI* __restrict__ W, TI* __restrict__ C, int64_t ldc,
                                                            int64_t Z) {
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-  const int64_t unit = static_cast<int64_t>(blockIdx.x) * 4 + wave;
+  const int64_t unit = SK > 1 ? static_cast<int64_t>(blockIdx.x) : static_cast<int64_t>(blockIdx.x) * 4 + wave;
   const int64_t zt = unit / tiles_n;
   int tile = static_cast<int>(unit - zt * tiles_n);
   int b = 0;
@@ -160,15 +184,15 @@ __global__ void __launch_bounds__(256, 2) flex_rows_kernel(const FlexBlock* __re
   if (b == nblocks || z0 >= Z) return;
   const FlexBlock blk = blocks[b];
   switch (blk.D) {
-    case 1: flex_tile<TI, 1, ZBIG, WT>(blk, parts, A, lda, W, C, ldc, Z, z0, tile * 32); break;
+    case 1: flex_tile<TI, 1, ZBIG, WT, SK>(blk, parts, A, lda, W, C, ldc, Z, z0, tile * 32); break;
     case 3:
-      for (int t = 0; t < ZBIG && z0 + 32 * t < Z; ++t) flex_tile<TI, 3, 1, WT>(blk, parts, A, lda, W, C, ldc, Z, z0 + 32 * t, tile * 32);
+      for (int t = 0; t < ZBIG && z0 + 32 * t < Z; ++t) flex_tile<TI, 3, 1, WT, SK>(blk, parts, A, lda, W, C, ldc, Z, z0 + 32 * t, tile * 32);
       break;
     case 5:
-      for (int t = 0; t < ZBIG && z0 + 32 * t < Z; ++t) flex_tile<TI, 5, 1, WT>(blk, parts, A, lda, W, C, ldc, Z, z0 + 32 * t, tile * 32);
+      for (int t = 0; t < ZBIG && z0 + 32 * t < Z; ++t) flex_tile<TI, 5, 1, WT, SK>(blk, parts, A, lda, W, C, ldc, Z, z0 + 32 * t, tile * 32);
       break;
     default:
-      for (int t = 0; t < ZBIG && z0 + 32 * t < Z; ++t) flex_tile<TI, 7, 1, WT>(blk, parts, A, lda, W, C, ldc, Z, z0 + 32 * t, tile * 32);
+      for (int t = 0; t < ZBIG && z0 + 32 * t < Z; ++t) flex_tile<TI, 7, 1, WT, SK>(blk, parts, A, lda, W, C, ldc, Z, z0 + 32 * t, tile * 32);
   }
 }
 
@@ -375,18 +399,23 @@ extern "C" int cueq_linear_flex(int32_t dtype, int32_t transposed_weights, int64
   // two row tiles per wavefront halve the weight loads once there are units enough for two per SIMD
   const int64_t zt1 = (rows + 31) / 32;
   const bool big = zt1 * column_tiles >= 8 * 4ll * device_cus();
-  const int64_t units = (big ? (rows + 63) / 64 : zt1) * column_tiles, grid = (units + 3) / 4;
+  // four wavefronts share a tile where all tiles, four wavefronts each, still run at once (two workgroups to a CU): 300 rows of
+  // 128x0e+128x1o+128x2e in mul_ir, float, forward 21.8 -> 9.7 us, 1 000 rows 22.1 -> 12.6 (1 400 rows, past the line: 22.5 either way)
+  const bool shared = zt1 * column_tiles <= 2ll * device_cus();
+  const int64_t units = (big ? (rows + 63) / 64 : zt1) * column_tiles, grid = shared ? units : (units + 3) / 4;
   CUEQ_REQUIRE(grid < (1ll << 31), CUEQ_ERR_TOO_LARGE, "linear_flex: too many rows");
   KernelTimer timer(mul_ir ? "linear_rows_mul_ir" : "linear_rows", stream);
 #define FLEX_ARGS(TI) static_cast<const FlexBlock*>(blocks), static_cast<const FlexPart*>(parts), nblocks, column_tiles, static_cast<const TI*>(A), lda, static_cast<const TI*>(W), static_cast<TI*>(C), ldc, rows
 #define FLEX(TI)                                                                                                                                                       \
   do {                                                                                                                                                                 \
     if (transposed_weights) {                                                                                                                                          \
-      if (big) hipLaunchKernelGGL((flex_rows_kernel<TI, true, 2>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, FLEX_ARGS(TI));                            \
-      else hipLaunchKernelGGL((flex_rows_kernel<TI, true, 1>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, FLEX_ARGS(TI));                                \
+      if (shared) hipLaunchKernelGGL((flex_rows_kernel<TI, true, 1, 4>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, FLEX_ARGS(TI));                    \
+      else if (big) hipLaunchKernelGGL((flex_rows_kernel<TI, true, 2, 1>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, FLEX_ARGS(TI));                            \
+      else hipLaunchKernelGGL((flex_rows_kernel<TI, true, 1, 1>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, FLEX_ARGS(TI));                                \
     } else {                                                                                                                                                           \
-      if (big) hipLaunchKernelGGL((flex_rows_kernel<TI, false, 2>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, FLEX_ARGS(TI));                           \
-      else hipLaunchKernelGGL((flex_rows_kernel<TI, false, 1>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, FLEX_ARGS(TI));                               \
+      if (shared) hipLaunchKernelGGL((flex_rows_kernel<TI, false, 1, 4>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, FLEX_ARGS(TI));                    \
+      else if (big) hipLaunchKernelGGL((flex_rows_kernel<TI, false, 2, 1>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, FLEX_ARGS(TI));                           \
+      else hipLaunchKernelGGL((flex_rows_kernel<TI, false, 1, 1>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, FLEX_ARGS(TI));                               \
     }                                                                                                                                                                  \
   } while (0)
   FLEX_DISPATCH(dtype, FLEX);
