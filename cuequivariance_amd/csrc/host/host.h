@@ -59,7 +59,8 @@ inline bool ordinary(const at::Tensor& t) {
   static const c10::DispatchKeySet odd = c10::DispatchKeySet(
       {c10::DispatchKey::Python, c10::DispatchKey::PythonTLSSnapshot, c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
        c10::DispatchKey::Functionalize, c10::DispatchKey::Conjugate, c10::DispatchKey::Negative, c10::DispatchKey::ZeroTensor});
-  return t.defined() && t.is_cuda() && t.layout() == at::kStrided && !t.key_set().has_any(odd);
+  // (with a tangent of forward-mode differentiation it goes the way that refuses it: the launches here would drop the tangent)
+  return t.defined() && t.is_cuda() && t.layout() == at::kStrided && !t.key_set().has_any(odd) && !t._fw_grad(/*level=*/0).defined();
 }
 // nothing watches the calls (torch.jit.trace, dispatch modes): the direct path may be taken
 bool unwatched();

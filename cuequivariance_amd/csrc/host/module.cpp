@@ -66,6 +66,8 @@ void sync_options() {
 bool unwatched() { return !torch::jit::tracer::isTracing() && !c10::impl::TorchDispatchModeTLS::any_modes_set(); }
 
 bool wants_graph(const std::vector<at::Tensor>& tensors) {
+  for (const auto& t : tensors)  // (a call without a graph would drop the tangent)
+    TORCH_CHECK_NOT_IMPLEMENTED(!t.defined() || !t._fw_grad(/*level=*/0).defined(), "cuequivariance_amd: forward-mode differentiation is not implemented");
   if (!at::GradMode::is_enabled()) return false;
   for (const auto& t : tensors)
     if (t.defined() && t.requires_grad()) return true;

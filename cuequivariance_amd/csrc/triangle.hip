@@ -3354,7 +3354,7 @@ struct Carve {  // consecutive pieces of a buffer, each on a 256-byte boundary
     char* p = base ? base + used : nullptr;
     // (large pieces a few pages apart: extents that are powers of two would put all streams of a kernel on the same channels at
     // once - 512 x 512 x 128 in bfloat16, input gradient, against a separate allocation per tensor: 0.6 - 1.0 % slower without the
-    // distance, 0.5 % slower to 0.5 % faster with it over three boxes)
+    // distance, 0.5 % slower to 0.5 % faster with it, measured three times)
     used += ((bytes + 255) & ~int64_t(255)) + (bytes >= (1 << 20) ? 5 * 4096 + 7 * 256 : 0);
     return p;
   }
