@@ -111,14 +111,18 @@ __device__ __forceinline__ float ln_affine(float centered, float rs, float gm, f
 // Pair rows of a padded square.  The contraction moves its n x n matrices in 16-byte pieces, so an extent n that is no multiple
 // of such a piece is rounded up to np inside the update: what lives between the stages has B np^2 rows, what the caller holds
 // (x, mask, the update, the two gradients of the pair tensor) B n^2.  src(m) is the caller's row of padded row m, -1 for padding.
+// Padding holds copies of the last real row and column (near), so that it is as finite as the caller's rows in every stage - a row
+// of zeros has no deviation, and the reciprocal of it under a vanishing eps is infinite -, except where the contraction runs over it
+// (not live): the two factors are zero there.  Its cotangent is zero, and with it every gradient.
 // The division is a multiplication by floor(2^(31 + s) / np) + 1, exact for m < 2^31.
 struct PairRows {
   int n = 0, np = 0;
+  int over_rows = 0;  // the contraction runs over the row index of the matrices (incoming) instead of the column index
   uint32_t magic = 0;
   int shift = 0;
-  __host__ static PairRows make(int n, int np) {
+  __host__ static PairRows make(int n, int np, bool over_rows) {
     PairRows p;
-    p.n = n; p.np = np;
+    p.n = n; p.np = np; p.over_rows = over_rows ? 1 : 0;
     while ((1ll << p.shift) < np) ++p.shift;
     p.magic = static_cast<uint32_t>((1ull << (31 + p.shift)) / static_cast<uint64_t>(np) + 1);
     return p;
@@ -129,6 +133,11 @@ struct PairRows {
   __device__ __forceinline__ int src(int m) const {
     const int q = over(m), k = m - q * np, b = over(q), i = q - b * np;
     return (k < n && i < n) ? (b * n + i) * n + k : -1;
+  }
+  __device__ __forceinline__ int near(int m, bool& live) const {
+    const int q = over(m), k = m - q * np, b = over(q), i = q - b * np;
+    live = (over_rows ? i : k) < n;
+    return (b * n + min(i, n - 1)) * n + min(k, n - 1);
   }
 };
 
@@ -1121,7 +1130,8 @@ __global__ void __launch_bounds__((SPLIT ? 256 : 512), (SPLIT ? 1 : 2))
         xf1[s2][q] = *reinterpret_cast<const uint4*>(X1 + o);
         if constexpr (SPLIT) xf2[s2][q] = *reinterpret_cast<const uint4*>(X2 + o);
       }
-    if (mask) mraw = raw16(mask[PAD ? max(pairs.src(mld), 0) : mld]);  // (padding: its cotangent is zero)
+    bool live;  // (padding: its cotangent is zero)
+    if (mask) mraw = raw16(mask[PAD ? pairs.near(mld, live) : mld]);
   };
   int64_t tile = ptile;
   if (tile < ntiles) request_x(tile_row(tile));
@@ -1395,8 +1405,8 @@ __global__ void __launch_bounds__((SPLIT ? 256 : 512), (SPLIT ? 1 : 2))
 // normalised in the registers, rounded to the 2-byte type - the operand of the products, exactly what a separate
 // LayerNorm launch would have written - and stored with their mean and 1 / std for the later stages.
 //
-// PAD: the rows are those of a padded square (PairRows).  LN: X and the mask are the caller's rows, padding counts as a row of
-// zeros with mask 0.  ROWS: X and X2 are padded, the result goes to the caller's rows.
+// PAD: the rows are those of a padded square (PairRows).  LN: X and the mask are the caller's rows, padding takes the nearest one,
+// and its result is zero where the contraction runs over it.  ROWS: X and X2 are padded, the result goes to the caller's rows.
 // ------------------------------------------------------------------------------------------------
 template <typename F, int KT, bool LN, bool ROWS, bool PAD = false>
 __global__ void __launch_bounds__(512, 2)
@@ -1450,16 +1460,12 @@ __global__ void __launch_bounds__(512, 2)
   // wavefront's next tile are requested while the current one is worked on
   uint4 xn[NT][NS][2], xn2[1][NS][2];
   uint32_t mraw[NT] = {};
-  bool pad_n[NT] = {};
+  bool live_n[NT] = {};
   auto request_x = [&](int64_t tl) {
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
       int mld = static_cast<int>(min(tl * (32 * NT) + 32 * t + c, static_cast<int64_t>(M) - 1));
-      if constexpr (PAD && LN) {
-        mld = pairs.src(mld);
-        pad_n[t] = mld < 0;
-        mld = max(mld, 0);
-      }
+      if constexpr (PAD && LN) mld = pairs.near(mld, live_n[t]);
 #pragma unroll
       for (int s2 = 0; s2 < NS; ++s2)
 #pragma unroll
@@ -1478,6 +1484,7 @@ __global__ void __launch_bounds__(512, 2)
   for (int64_t tile = tile0; tile < ntiles; tile += tstep) {
     uint4 xf[NT][NS][2], xf2[1][NS][2];
     float mk[NT];
+    uint32_t keep[NT];  // padding that the contraction runs over: selected away (a product with 0 would keep what is not finite)
     int mcol[NT];
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
@@ -1487,15 +1494,10 @@ __global__ void __launch_bounds__(512, 2)
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
           xf[t][s2][q] = xn[t][s2][q];
-          if constexpr (PAD && LN) {
-            if (pad_n[t]) xf[t][s2][q] = make_uint4(0, 0, 0, 0);
-          }
           if constexpr (ROWS) xf2[t][s2][q] = xn2[t][s2][q];
         }
       mk[t] = mask ? lo16<F>(mraw[t]) : 1.0f;
-      if constexpr (PAD && LN) {
-        if (pad_n[t]) mk[t] = 0.0f;
-      }
+      keep[t] = !(PAD && LN) || live_n[t] ? ~0u : 0u;
     }
     request_x(min(tile + tstep, ntiles - 1));  // (past the end: the last tile again, so that the request is unconditional)
     if constexpr (LN) {
@@ -1622,7 +1624,8 @@ __global__ void __launch_bounds__(512, 2)
             const int v = 4 * a + b;
             g[b] = __builtin_amdgcn_rcpf(1.0f + __expf(-au[t][v])) * av[t][v] * mk[t];
           }
-          const uint32_t own[2] = {pack16<F>(g[0], g[1]), pack16<F>(g[2], g[3])};
+          uint32_t own[2] = {pack16<F>(g[0], g[1]), pack16<F>(g[2], g[3])};
+          if constexpr (PAD) own[0] &= keep[t], own[1] &= keep[t];
 #pragma unroll
           for (int j = 0; j < 2; ++j) {
             const uint32_t other = static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(own[j]), 0xB1, 0xF, 0xF, true));
@@ -2487,19 +2490,29 @@ __global__ void __launch_bounds__(1024) fold_two_kernel(const float* __restrict_
   }
 }
 
-// rows of a padded square from the caller's rows (TO_PAD; padding is zero) or back, in 16-byte vectors (V = uint4) or elements;
-// a null `in` stands for ones
-template <typename V, bool TO_PAD>
+// rows of a padded square from the caller's rows - the pair tensor and the mask (a null `in`: ones) as PairRows says, or with zeros
+// for padding (the cotangent) - or back, in 16-byte vectors (V = uint4) or elements
+enum PairCopy { kPairNear, kPairMask, kPairZero, kPairBack };
+template <typename V, int MODE>
 __global__ void __launch_bounds__(256) pair_rows_kernel(const V* __restrict__ in, V* __restrict__ out, int vpr, int64_t total, PairRows pairs, V one) {
   for (int64_t e = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; e < total; e += static_cast<int64_t>(gridDim.x) * 256) {
     const int64_t m = e / vpr;
-    const int v = static_cast<int>(e - m * vpr), src = pairs.src(static_cast<int>(m));
-    if constexpr (TO_PAD) {
+    const int v = static_cast<int>(e - m * vpr);
+    if constexpr (MODE == kPairNear || MODE == kPairMask) {
+      bool live;
+      const int src = pairs.near(static_cast<int>(m), live);
       V val{};
-      if (src >= 0) val = in ? in[static_cast<int64_t>(src) * vpr + v] : one;
+      if (MODE == kPairNear || live) val = in ? in[static_cast<int64_t>(src) * vpr + v] : one;
       out[e] = val;
-    } else if (src >= 0) {
-      out[static_cast<int64_t>(src) * vpr + v] = in[e];
+    } else {
+      const int src = pairs.src(static_cast<int>(m));
+      if constexpr (MODE == kPairZero) {
+        V val{};
+        if (src >= 0) val = in[static_cast<int64_t>(src) * vpr + v];
+        out[e] = val;
+      } else if (src >= 0) {
+        out[static_cast<int64_t>(src) * vpr + v] = in[e];
+      }
     }
   }
 }
@@ -3330,7 +3343,7 @@ struct TriPlan {
   bool resident, mapped, copies;
   PairRows pairs;
 
-  TriPlan(int32_t dt_, int64_t B_, int64_t N_, int64_t D_, int64_t Do_) : dt(dt_), B(B_), N(N_), D(D_), Do(Do_) {
+  TriPlan(int32_t dt_, int64_t B_, int64_t N_, int64_t D_, int64_t Do_, bool outgoing = true) : dt(dt_), B(B_), N(N_), D(D_), Do(Do_) {
     es = dt == CUEQ_F32 ? 4 : 2;
     const int64_t epv = 16 / es;
     Np = (N + epv - 1) / epv * epv;
@@ -3342,7 +3355,7 @@ struct TriPlan {
     mapped = Np != N && resident && (D == 64 || D == 128) && Do % 32 == 0 && dual_gate_res_lds(Do, D, false) <= 160 * 1024 && bwd_out <= 160 * 1024 &&
              bwd_in <= 160 * 1024 && (M * Do + 8) * es < (1ll << 32) && 5 * M * es < (1ll << 32);
     copies = Np != N && !mapped;
-    if (Np != N && M < (1ll << 31)) pairs = PairRows::make(static_cast<int>(N), static_cast<int>(Np));
+    if (Np != N && M < (1ll << 31)) pairs = PairRows::make(static_cast<int>(N), static_cast<int>(Np), !outgoing);
   }
 };
 
@@ -3423,18 +3436,20 @@ struct TriBwdWork {
   }
 };
 
-int pair_copy(const TriPlan& p, const void* in, void* out, int64_t width, bool to_pad, hipStream_t stream) {
+int pair_copy(const TriPlan& p, const void* in, void* out, int64_t width, PairCopy mode, hipStream_t stream) {
   const int64_t bytes = width * p.es;
   const bool vec = bytes % 16 == 0 && ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 15) == 0;
   const int vpr = static_cast<int>(vec ? bytes / 16 : width);
   const int64_t total = p.M * vpr;
   const dim3 grid(static_cast<unsigned>(std::min<int64_t>((total + 255) / 256, 16ll * device_cus())));
-#define PC(V, ONE) do { if (to_pad) hipLaunchKernelGGL((pair_rows_kernel<V, true>), grid, dim3(256), 0, stream, static_cast<const V*>(in), static_cast<V*>(out), vpr, total, p.pairs, ONE); \
-    else hipLaunchKernelGGL((pair_rows_kernel<V, false>), grid, dim3(256), 0, stream, static_cast<const V*>(in), static_cast<V*>(out), vpr, total, p.pairs, ONE); } while (0)
+#define PC_M(V, MODE, ONE) hipLaunchKernelGGL((pair_rows_kernel<V, MODE>), grid, dim3(256), 0, stream, static_cast<const V*>(in), static_cast<V*>(out), vpr, total, p.pairs, ONE)
+#define PC(V, ONE) do { switch (mode) { case kPairNear: PC_M(V, kPairNear, ONE); break; case kPairMask: PC_M(V, kPairMask, ONE); break; \
+    case kPairZero: PC_M(V, kPairZero, ONE); break; default: PC_M(V, kPairBack, ONE); } } while (0)
   if (vec) PC(uint4, uint4{});
   else if (p.es == 4) PC(float, 1.0f);
   else PC(uint16_t, static_cast<uint16_t>(p.dt == CUEQ_BF16 ? 0x3f80 : 0x3c00));
 #undef PC
+#undef PC_M
   CUEQ_CHECK_HIP(hipGetLastError());
   return CUEQ_OK;
 }
@@ -3460,7 +3475,7 @@ extern "C" int64_t cueq_trimul_workspace_bytes(int32_t dtype, int64_t B, int64_t
 extern "C" int cueq_trimul_fwd(int32_t dtype, int64_t B, int64_t N, int64_t D, int64_t Do, int32_t outgoing, double eps, const void* x, const void* mask,
                                const void* const* w, void* out, void* saved, void* workspace, int64_t workspace_bytes, void* stream_) {
   hipStream_t stream = static_cast<hipStream_t>(stream_);
-  const TriPlan p(dtype, B, N, D, Do);
+  const TriPlan p(dtype, B, N, D, Do, outgoing != 0);
   TRI_STEP(tri_check(p));
   if (p.M == 0) return CUEQ_OK;
   CUEQ_REQUIRE(x && w && w[kPinW] && w[kGinW] && w[kPoutW] && w[kGoutW] && out && saved, CUEQ_ERR_INVALID, "trimul: null operand");
@@ -3469,8 +3484,8 @@ extern "C" int cueq_trimul_fwd(int32_t dtype, int64_t B, int64_t N, int64_t D, i
   CUEQ_REQUIRE(workspace_bytes >= k.bytes && (workspace || k.bytes == 0), CUEQ_ERR_INVALID, "trimul: workspace too small");
   const int64_t M = p.M;
   if (p.copies) {
-    TRI_STEP(pair_copy(p, x, s.xp, D, true, stream));
-    TRI_STEP(pair_copy(p, mask, s.maskp, 1, true, stream));
+    TRI_STEP(pair_copy(p, x, s.xp, D, kPairNear, stream));
+    TRI_STEP(pair_copy(p, mask, s.maskp, 1, kPairMask, stream));
     x = s.xp;
     mask = s.maskp;
   }
@@ -3501,7 +3516,7 @@ extern "C" int cueq_trimul_fwd(int32_t dtype, int64_t B, int64_t N, int64_t D, i
   }
   void* to = p.copies ? k.outp : out;
   TRI_STEP(cueq_dual_gate(dtype, 0, M, Do, D, s.xh, s.y, D, w[kGoutW], w[kPoutW], D, w[kGoutB], w[kPoutB], 1, nullptr, 0, nullptr, to, nullptr, Do, stream_));
-  if (p.copies) TRI_STEP(pair_copy(p, to, out, Do, false, stream));
+  if (p.copies) TRI_STEP(pair_copy(p, to, out, Do, kPairBack, stream));
   return CUEQ_OK;
 }
 
@@ -3509,7 +3524,7 @@ extern "C" int cueq_trimul_bwd(int32_t dtype, int64_t B, int64_t N, int64_t D, i
                                const void* const* w, void* saved, const void* dout, void* dx, uint32_t need, void* grads, void* workspace,
                                int64_t workspace_bytes, void* stream_) {
   hipStream_t stream = static_cast<hipStream_t>(stream_);
-  const TriPlan p(dtype, B, N, D, Do);
+  const TriPlan p(dtype, B, N, D, Do, outgoing != 0);
   TRI_STEP(tri_check(p));
   const int64_t nv = cueq_trimul_grads_values(D, Do);
   if (p.M == 0) return CUEQ_OK;  // (the caller returns zeros)
@@ -3525,7 +3540,7 @@ extern "C" int cueq_trimul_bwd(int32_t dtype, int64_t B, int64_t N, int64_t D, i
   float* gf = dtype == CUEQ_F32 ? static_cast<float*>(grads) : k.grads;
   float *g_nin = gf, *g_nout = gf + 2 * D, *g_in = gf + 4 * D, *g_out = g_in + 4 * D * D, *g_in_b = g_out + 2 * Do * D, *g_out_b = g_in_b + 4 * D;
   if (p.copies) {
-    TRI_STEP(pair_copy(p, dout, k.doutp, Do, true, stream));
+    TRI_STEP(pair_copy(p, dout, k.doutp, Do, kPairZero, stream));
     x = s.xp;
     mask = s.maskp;
     dout = k.doutp;
@@ -3593,7 +3608,7 @@ extern "C" int cueq_trimul_bwd(int32_t dtype, int64_t B, int64_t N, int64_t D, i
   if (!w_in && !affine_in && ln_fused) {
     TRI_STEP(gate_bwd_input_impl(dtype, 2 * D, M, D, w[kGinW], w[kPinW], D, s.xh, nullptr, D, w[kGinB], w[kPinB], mask, k.dab, M, 1,
                                  k.dxh, nullptr, D, 1, nullptr, nullptr, x, D, s.mean1, s.rstd1, w[kNinW], stream_, dxt, pairs));
-    if (p.copies) TRI_STEP(pair_copy(p, dxt, dx, D, false, stream));
+    if (p.copies) TRI_STEP(pair_copy(p, dxt, dx, D, kPairBack, stream));
   } else {
     if (D <= 128) {
       TRI_STEP(gate_bwd_input_impl(dtype, 2 * D, M, D, w[kGinW], w[kPinW], D, s.xh, nullptr, D, w[kGinB], w[kPinB], mask, k.dab, M, 1, k.dxh, nullptr, D,
@@ -3608,7 +3623,7 @@ extern "C" int cueq_trimul_bwd(int32_t dtype, int64_t B, int64_t N, int64_t D, i
     if (wants(kPinB)) TRI_STEP(cueq_sum_cols(dtype, 2 * D, M, dv1, g_in_b + 2 * D, stream_));
     TRI_STEP(layer_norm_bwd_impl(dtype, M, D, k.dxh, x, s.mean1, s.rstd1, w[kNinW], dxt, wants(kNinW) ? g_nin : nullptr, wants(kNinB) ? g_nin + D : nullptr,
                                  k.ln, k.ln_bytes, stream_, pairs));
-    if (p.copies) TRI_STEP(pair_copy(p, dxt, dx, D, false, stream));
+    if (p.copies) TRI_STEP(pair_copy(p, dxt, dx, D, kPairBack, stream));
   }
   if (need && dtype != CUEQ_F32) {
     const dim3 grid(static_cast<unsigned>((nv + 255) / 256));
