@@ -52,6 +52,7 @@ struct FcOp {
   int64_t h_width = 0;
   int factors = 0;
   int64_t tiled_dw_from[2] = {1 << 30, 1 << 30};  // rows, by element size (4, 2)
+  bool float_factors = false;  // bfloat16 rows: the weight gradient's factors H stay float32 (half rows: always)
 
   std::mutex mutex;
   struct OnDevice {
@@ -191,11 +192,17 @@ Grads gradients(FcOp& op, const at::Tensor& w_, const at::Tensor& x1_, const at:
   if (need_w) {
     const at::ScalarType out_dtype = w_dtype == at::kDouble ? at::kFloat : w_dtype;
     const Unit* u = unit && Z >= unit->dw_from ? unit : nullptr;
+    // The factors H_i = sum_k s_ik g_k are operands of a product, rounded to its type.  In half they leave its range long before the
+    // gradient does (65 504: a scaled loss), and bfloat16 calls that were float32 throughout would lose a rounding's worth: both
+    // contract float copies of their rows.  (Generated kernels: a product's own, in its own type.)
+    const at::ScalarType dw_dtype = !u && (dtype == at::kHalf || (dtype == at::kBFloat16 && op.float_factors)) ? at::kFloat : dtype;
+    const at::Tensor a1 = x1.to(dw_dtype), a2 = x2.to(dw_dtype), ag = g.to(dw_dtype);
+    const int dw_code = dtype_code(dw_dtype);
     at::Tensor gw = new_tensor(w_sizes, out_dtype, device);
-    if (!u && Z >= op.tiled_dw_from[dtype == at::kFloat ? 0 : 1]) {
+    if (!u && Z >= op.tiled_dw_from[dw_dtype == at::kFloat ? 0 : 1]) {
       const auto& t = op.on(device);
-      at::Tensor H = at::empty({Z, op.h_width}, options), x1t = op.mul_ir ? at::empty({Z, op.width1}, options) : x1;
-      check(lib().cueq_fc_factors(code, op.mul_ir, Z, x1.data_ptr(), op.width1, x2.data_ptr(), op.n2, g.data_ptr(), op.width_out, t.grads.data_ptr(),
+      at::Tensor H = at::empty({Z, op.h_width}, ag.options()), x1t = op.mul_ir ? at::empty({Z, op.width1}, ag.options()) : a1;
+      check(lib().cueq_fc_factors(dw_code, op.mul_ir, Z, a1.data_ptr(), op.width1, a2.data_ptr(), op.n2, ag.data_ptr(), op.width_out, t.grads.data_ptr(),
                                   static_cast<int>(t.grads.numel() / 72), static_cast<const float*>(t.coef.data_ptr()), t.dx_blocks.data_ptr(),
                                   static_cast<int>(t.dx_blocks.numel() / 24), op.factors, H.data_ptr(), op.h_width, op.mul_ir ? x1t.data_ptr() : nullptr, stream),
             "cueq_fc_factors");
@@ -203,7 +210,7 @@ Grads gradients(FcOp& op, const at::Tensor& w_, const at::Tensor& x1_, const at:
         const GradShape& q = op.shapes[i];
         const int64_t per = int64_t(q.K) * q.N;
         at::Tensor part = new_tensor({q.parts * kChunks, per}, at::kFloat, device);
-        check(lib().cueq_gemm_table(code, CUEQ_F32, 1, 1, q.K, q.N, Z, x1t.data_ptr(), op.width1, H.data_ptr(), op.h_width, part.data_ptr(), q.N,
+        check(lib().cueq_gemm_table(dw_code, CUEQ_F32, 1, 1, q.K, q.N, Z, x1t.data_ptr(), op.width1, H.data_ptr(), op.h_width, part.data_ptr(), q.N,
                                     t.tables[i].data_ptr<int64_t>(), q.parts, kChunks, per, 1.0, 0, stream),
               "cueq_gemm_table");
         check(lib().cueq_sum_runs(part.data_ptr<float>(), static_cast<int>(per), static_cast<int>(q.w0.size()), q.first.data(), q.w0.data(),
@@ -213,7 +220,7 @@ Grads gradients(FcOp& op, const at::Tensor& w_, const at::Tensor& x1_, const at:
       r.w = w_dtype == out_dtype ? gw : gw.to(w_dtype);
       return r;
     }
-    const bool by_channels = op.packed.grad_tiles > 0 && dtype != at::kFloat;
+    const bool by_channels = op.packed.grad_tiles > 0 && dw_dtype != at::kFloat;
     const int grad_tiles = by_channels ? op.packed.grad_tiles : op.grad_tiles;
     const int64_t chunks = u ? u->dw_blocks(Z) : lib().cueq_fc_flex_dw_chunks(Z, grad_tiles, by_channels);
     at::Tensor part = new_tensor({chunks, op.numel}, at::kFloat, device);
@@ -223,7 +230,7 @@ Grads gradients(FcOp& op, const at::Tensor& w_, const at::Tensor& x1_, const at:
     } else {
       const auto& t = op.on(device);
       const at::Tensor& table = by_channels ? t.packed_grads : t.grads;
-      check(lib().cueq_fc_flex_dw(code, op.mul_ir, by_channels, Z, x1.data_ptr(), op.width1, x2.data_ptr(), op.n2, g.data_ptr(), op.width_out, table.data_ptr(),
+      check(lib().cueq_fc_flex_dw(dw_code, op.mul_ir, by_channels, Z, a1.data_ptr(), op.width1, a2.data_ptr(), op.n2, ag.data_ptr(), op.width_out, table.data_ptr(),
                                   static_cast<int>(table.numel() / 72), static_cast<const float*>(t.coef.data_ptr()), grad_tiles, op.numel,
                                   part.data_ptr<float>(), stream),
             "cueq_fc_flex_dw");
@@ -427,6 +434,7 @@ void bind_fully_connected(py::module_& m) {
         p.fwd_longest = longest[0].cast<int>(), p.dx_longest = longest[1].cast<int>(), p.grad_tiles = grad_tiles;
         p.fwd_pieces = pieces[0].cast<int64_t>(), p.dx_pieces = pieces[1].cast<int64_t>();
       })
+      .def("keep_float_factors", [](FcOp& op) { op.float_factors = true; })
       .def("takes", [](const FcOp& op, const at::Tensor& x) { return op.takes(x.scalar_type()); })
       .def("direct", &direct)
       .def("forward", [](const OpPtr& op, const at::Tensor& w, const at::Tensor& x1, const at::Tensor& x2) { return forward(op, w, x1, x2, x1.scalar_type()); })

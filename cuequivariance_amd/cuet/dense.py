@@ -18,6 +18,7 @@ from __future__ import annotations
 
 import ctypes as C
 import json
+import math
 import struct
 from types import SimpleNamespace
 import threading
@@ -427,6 +428,11 @@ def _fc_op(mod: "SegmentedPolynomialDense"):
     return op
 
 
+# Scalar paths of the flattened operation from which on products with a matrix shape run as a Linear map with an element-wise stage
+# (``cuet/fused_tp.py``) instead of flattened on the uniform-1d kernels.
+STAGES_FROM = 2048
+
+
 class GeneralFullyConnected:
     """``uvw,iu,jv,kw+ijk`` with shared weights and a second operand of any multiplicity on the rows kernels of ``csrc/fc_flex.hip``, as
     the host module runs it: the products of the two operands are formed in registers.  Rows of the first operand and of the
@@ -463,6 +469,11 @@ class GeneralFullyConnected:
                                   tables[2], tables[3], tables[0], tables[1])
             if tables[5] is not None:
                 op.add_packed(*tables[5])
+            # (2-byte products with fewer scalar paths have their other form in float32 throughout - the flattened kernels; here the
+            # products and sums are float32 too, but for the factors of the weight gradient, which stay so as well then: relative
+            # error of a bfloat16 weight gradient 2.3e-3 -> 1.6e-3, its own rounding)
+            if sum(int((p.coefficients != 0).sum()) * math.prod(stp.operands[0][p.indices[0]][:2]) for p in stp.paths) < STAGES_FROM:
+                op.keep_float_factors()
             self._op = op
         return self._op
 

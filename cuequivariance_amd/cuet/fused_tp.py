@@ -377,7 +377,7 @@ class SegmentedPolynomialFusedTP(nn.Module):
     def __init__(self, polynomial: cue.SegmentedPolynomial, math_dtype=None, output_dtype_map: Optional[List[int]] = None,
                  name: str = "segmented_polynomial", rows: str = "ir_mul", row_blocks=None):
         super().__init__()
-        from .dense import GeneralFullyConnected, SegmentedPolynomialDense
+        from .dense import STAGES_FROM, GeneralFullyConnected, SegmentedPolynomialDense
 
         self._rows_orig, self._row_blocks_orig = rows, row_blocks
 
@@ -424,7 +424,7 @@ class SegmentedPolynomialFusedTP(nn.Module):
         # flattened operation would have `stages_from` scalar paths or more (small multiplicities are one cheap launch of a
         # generated uniform-1d kernel; beyond a few thousand paths that kernel takes minutes to compile and the matrix
         # cores are far ahead)
-        self.stages_from = 2048
+        self.stages_from = STAGES_FROM
         self.composed = None
         if self.dense is None and rows != "mul_ir":
             try:
