@@ -2,6 +2,7 @@
 // x1 / of x2 / of the weights, each differentiable in terms of the others, on csrc/fc_flex.hip and - from the measured crossings on -
 // the kernels generated for the descriptor (codegen/fullyconnected.py).
 #include "host.h"
+#include "shared_map.h"
 
 #include <mutex>
 #include <unordered_map>
@@ -46,7 +47,7 @@ struct FcOp {
   int epv_ok = 0, most = 1;
   std::string fwd_blocks, fwd_parts, dx_blocks, dx_parts, grads, coef;
   int fwd_tiles = 0, dx_tiles = 0, grad_tiles = 0;
-  std::unordered_map<int, Unit> units;  // by element type code
+  SharedMap<Unit> units;  // by element type code
   std::vector<GradShape> shapes;
   Packed packed;
   int64_t h_width = 0;
@@ -80,10 +81,6 @@ struct FcOp {
     return it->second;
   }
   bool takes(at::ScalarType t) const { return (t == at::kFloat && (epv_ok & 1)) || ((t == at::kBFloat16 || t == at::kHalf) && (epv_ok & 2)); }
-  const Unit* unit(int code) const {
-    auto it = units.find(code);
-    return it == units.end() ? nullptr : &it->second;
-  }
 };
 using OpPtr = std::shared_ptr<FcOp>;
 
@@ -112,8 +109,8 @@ at::Tensor product(FcOp& op, const at::Tensor& w_, const at::Tensor& x1_, const 
   const int64_t Z = x1.size(0);
   const auto options = at::TensorOptions().dtype(dtype).device(device);
   const int code = dtype_code(dtype);
-  const Unit* u = op.unit(code);
-  if (u && Z < u->fwd_from) u = nullptr;
+  const std::optional<Unit> unit = op.units.find(code);
+  const Unit* u = unit && Z >= unit->fwd_from ? &*unit : nullptr;
   at::Tensor out = op.covers_out || u ? at::empty({Z, op.width_out}, options) : at::zeros({Z, op.width_out}, options);
   if (Z == 0) return out;
   hipStream_t stream = stream_of(device.index());
@@ -153,9 +150,9 @@ Grads gradients(FcOp& op, const at::Tensor& w_, const at::Tensor& x1_, const at:
   }
   const int code = dtype_code(dtype);
   hipStream_t stream = stream_of(device.index());
-  const Unit* unit = op.unit(code);
+  const std::optional<Unit> unit = op.units.find(code);
   if (need_1 || need_2) {
-    const Unit* u = unit && Z >= unit->dx_from ? unit : nullptr;
+    const Unit* u = unit && Z >= unit->dx_from ? &*unit : nullptr;
     // (without x2 - the gradient of x2 alone does not use it - any values do: what they scale is not asked for)
     const at::Tensor second = x2.defined() ? x2 : at::zeros({Z, op.n2}, options);
     if (need_1) r.x1 = op.covers_in || u ? at::empty({Z, op.width1}, options) : at::zeros({Z, op.width1}, options);
@@ -191,7 +188,7 @@ Grads gradients(FcOp& op, const at::Tensor& w_, const at::Tensor& x1_, const at:
   }
   if (need_w) {
     const at::ScalarType out_dtype = w_dtype == at::kDouble ? at::kFloat : w_dtype;
-    const Unit* u = unit && Z >= unit->dw_from ? unit : nullptr;
+    const Unit* u = unit && Z >= unit->dw_from ? &*unit : nullptr;
     // The factors H_i = sum_k s_ik g_k are operands of a product, rounded to its type.  In half they leave its range long before the
     // gradient does (65 504: a scaled loss), and bfloat16 calls that were float32 throughout would lose a rounding's worth: both
     // contract float copies of their rows.  (Generated kernels: a product's own, in its own type.)
@@ -396,7 +393,7 @@ void bind_fully_connected(py::module_& m) {
         u.dx12 = reinterpret_cast<decltype(u.dx12)>(f.at(3)), u.dw_blocks = reinterpret_cast<decltype(u.dw_blocks)>(f.at(4));
         u.dw = reinterpret_cast<decltype(u.dw)>(f.at(5));
         u.fwd_from = fwd_from, u.dx_from = dx_from, u.dw_from = dw_from;
-        op.units[code] = u;
+        op.units.set(code, u);
       })
       // paths in the order of the weight-gradient table: (w0, a0, K, components, N, components of the result)
       .def("add_tiled_dw", [](FcOp& op, const py::list& paths, int64_t from4, int64_t from2) {
