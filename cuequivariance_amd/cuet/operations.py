@@ -23,10 +23,11 @@ import torch
 
 from .. import cue
 from ..cue import descriptors
-from .dense import GeneralFullyConnected
+from .dense import GeneralFullyConnected, SegmentedPolynomialDense
+from .fused_tp import SegmentedPolynomialFusedTP, _FlattenedOperation, _MatrixWithElementwiseStage
 from .script import scriptable
-from .segmented_polynomial import SegmentedPolynomial
-from .transpose import TransposeIrrepsLayout, apply_layout
+from .segmented_polynomial import SegmentedPolynomial, SegmentedPolynomialFromUniform1d
+from .transpose import TransposeIrrepsLayout, TransposeSegments, apply_layout
 
 __all__ = ["ChannelWiseTensorProduct", "FullyConnectedTensorProduct", "Linear", "SymmetricContraction", "SphericalHarmonics",
            "Rotation", "Inversion", "encode_rotation_angle", "vector_to_euler_angles"]
@@ -55,9 +56,34 @@ def _transposition_moves(irreps) -> bool:
     return any(mul > 1 and ir.dim > 1 for mul, ir in irreps)
 
 
+def _untouched(module: torch.nn.Module) -> bool:
+    """Whether the children of ``module`` are of the classes it was built with and a call of one runs its ``forward`` and nothing else:
+    a replaced child (a wrapper, ``torch.compile``), a hook on one (profilers, operation counters) or a ``forward`` put in its place
+    is to be called."""
+    for child in module._modules.values():
+        if child is not None:
+            d = child.__dict__
+            if (type(child) not in _BUILT or d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"] or d["_backward_pre_hooks"]
+                    or "forward" in d or "_compiled_call_impl" in d):
+                return False
+    return True
+
+
+def _executor(module: torch.nn.Module, name: str, kind: type):
+    """The executor (of type ``kind``) that a call of the child ``name`` ends in, when it may be run without those calls; else ``None``."""
+    if torch.compiler.is_compiling() or torch.nn.modules.module._has_any_global_hook() or not _untouched(module):
+        return None
+    f = module._modules[name]
+    if type(f) is not SegmentedPolynomial or not _untouched(f):
+        return None
+    m = f._modules["m"]
+    return m if type(m) is kind and _untouched(m) else None
+
+
 def _operator(module: torch.nn.Module):
-    """The host module's operator behind ``module.f`` (a uniform-1d ``SegmentedPolynomial``), or ``None`` while a graph is traced."""
-    return None if torch.compiler.is_compiling() else module._modules["f"]._modules["m"].operator
+    """The host module's operator behind ``module.f`` (a uniform-1d ``SegmentedPolynomial``), or ``None``: see ``_executor``."""
+    m = _executor(module, "f", SegmentedPolynomialFromUniform1d)
+    return None if m is None else m.operator
 
 
 def _default_layout(layout) -> cue.IrrepsLayout:
@@ -105,6 +131,11 @@ class _FlattenedUniform(torch.nn.Module):
             self.f = SegmentedPolynomial(q, method="uniform_1d", math_dtype=self._math_dtype, options={"origin": self._polynomial})
         return self.f(inputs, input_indices=input_indices or {}, output_shapes=output_shapes or {},
                       output_indices=output_indices or {})
+
+
+_BUILT = frozenset([SegmentedPolynomial, SegmentedPolynomialFromUniform1d, SegmentedPolynomialFusedTP, SegmentedPolynomialDense,
+                    _MatrixWithElementwiseStage, _FlattenedOperation, _FlattenedUniform, TransposeIrrepsLayout, TransposeSegments, torch.nn.ModuleList,
+                    torch.nn.Identity])
 
 
 @scriptable("with_weight")
@@ -438,7 +469,7 @@ class FullyConnectedTensorProduct(torch.nn.Module):
             raise ValueError("Internal weights are not used, weight should not be None")
         if indices_1 is None and indices_out is None and not torch.compiler.is_compiling() and type(x1) is torch.Tensor:
             # the whole call in native code when it is a plain one; anything else, and every error, takes the way below
-            if self.general is not None:
+            if self.general is not None and _executor(self, "f", SegmentedPolynomialFusedTP) is not None:
                 out = self.general(weight, x1, x2)
                 if out is not None:
                     return out
@@ -467,14 +498,14 @@ class FullyConnectedTensorProduct(torch.nn.Module):
         """The executor of the 4-operand form for rows in this module's layouts, or ``None``."""
         if self.method != "fused_tp" or not self.transpose_in2.moves_nothing:
             return None
-        if self.f_rows is not None:
-            return self.f_rows._modules["m"].dense
-        if self.f is None or not (self.transpose_in1.moves_nothing and self.transpose_out.moves_nothing):
+        if self.f_rows is None and (self.f is None or not (self.transpose_in1.moves_nothing and self.transpose_out.moves_nothing)):
             return None
-        return getattr(self.f._modules["m"], "dense", None)
+        m = _executor(self, "f" if self.f_rows is None else "f_rows", SegmentedPolynomialFusedTP)
+        return None if m is None else m.dense
 
     def _rows_ready(self, x1, x2, weight) -> bool:
-        dense = self.f_rows.m.dense if self.f_rows is not None else None
+        # (a wrapper in the place of f_rows that does not show its executor is not asked: the rows are transposed then)
+        dense = getattr(getattr(self.f_rows, "m", None), "dense", None)
         return (dense is not None and weight is not None and weight.shape[0] == 1 and x1.is_cuda and x1.dtype == x2.dtype == weight.dtype
                 and x1.shape[0] == x2.shape[0] and dense.mul_ir_ready(x1.dtype))
 
@@ -547,12 +578,10 @@ class Linear(torch.nn.Module):
         """The host module's operator for rows in this module's layouts, or ``None``."""
         if self.method != "fused_tp":
             return None
-        if self.f_rows is not None:
-            return self.f_rows._modules["m"].dense.linear
-        if not (self.transpose_in.moves_nothing and self.transpose_out.moves_nothing):
+        if self.f_rows is None and not (self.transpose_in.moves_nothing and self.transpose_out.moves_nothing):
             return None
-        dense = getattr(self.f._modules["m"], "dense", None)
-        return dense.linear if dense is not None else None
+        m = _executor(self, "f" if self.f_rows is None else "f_rows", SegmentedPolynomialFusedTP)
+        return None if m is None or m.dense is None else m.dense.linear
 
     def extra_repr(self) -> str:
         return (
@@ -580,8 +609,8 @@ class Linear(torch.nn.Module):
             out = op.direct(weight, x) if op is not None else None
             if out is not None:
                 return out
-        if (self.f_rows is not None and not input_indices and weight.shape[0] == 1 and x.is_cuda and x.dtype == weight.dtype
-                and self.f_rows.m.dense.rows_accepted(x.dtype)):
+        rows = getattr(getattr(self.f_rows, "m", None), "dense", None)  # (see FullyConnectedTensorProduct._rows_ready)
+        if rows is not None and not input_indices and weight.shape[0] == 1 and x.is_cuda and x.dtype == weight.dtype and rows.rows_accepted(x.dtype):
             return self.f_rows([weight, x])[0]
         if self.method != "indexed_linear" and (input_indices or weight.shape[0] != 1):
             out = self.f_per_sample([weight, apply_layout(self.transpose_in, x)], input_indices)
