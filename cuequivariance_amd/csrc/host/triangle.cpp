@@ -30,14 +30,17 @@ variable_list aligned(at::TensorList ts) {
 }
 void* pointer(const at::Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
 
-// x (B, N, N, D), mask (B, N, N) or undefined, weights as above (undefined where absent), all contiguous in x's type
-std::pair<at::Tensor, at::Tensor> trimul_fwd(const at::Tensor& x_, const at::Tensor& mask, at::TensorList weights, bool outgoing, double eps) {
+// x (B, N, N, D), mask (B, N, N) or undefined, weights as above (undefined where absent), all contiguous in x's type; saved_bytes: a
+// size of what is kept for the backward that the caller has promised (a traced graph), 0: as much as is needed
+std::pair<at::Tensor, at::Tensor> trimul_fwd(const at::Tensor& x_, const at::Tensor& mask, at::TensorList weights, bool outgoing, double eps, int64_t saved_bytes = 0) {
   const at::Tensor x = aligned(x_);
   const variable_list w = aligned(weights);
   const Call c(x, w);
   const c10::DeviceGuard guard(c.device);
   at::Tensor out = new_tensor({c.B, c.N, c.N, c.Do}, x.scalar_type(), c.device);
-  at::Tensor saved = new_tensor({lib().cueq_trimul_saved_bytes(c.code, c.B, c.N, c.D, c.Do)}, at::kByte, c.device), ws;
+  const int64_t needed = lib().cueq_trimul_saved_bytes(c.code, c.B, c.N, c.D, c.Do);
+  TORCH_CHECK(!saved_bytes || saved_bytes >= needed, "triangle update: ", saved_bytes, " bytes promised for the backward, ", needed, " needed");
+  at::Tensor saved = new_tensor({saved_bytes ? saved_bytes : needed}, at::kByte, c.device), ws;
   const int64_t bytes = lib().cueq_trimul_workspace_bytes(c.code, c.B, c.N, c.D, c.Do, 0, 0);
   if (bytes > 0) ws = new_tensor({bytes}, at::kByte, c.device);
   check(lib().cueq_trimul_fwd(c.code, c.B, c.N, c.D, c.Do, outgoing, eps, x.data_ptr(), pointer(mask), c.w, out.data_ptr(), saved.data_ptr(), pointer(ws), bytes,
@@ -164,8 +167,8 @@ void bind_triangle(py::module_& m) {
   using OptionalList = std::vector<std::optional<at::Tensor>>;
   m.def("trimul", &run);
   m.def("trimul_direct", &direct);
-  m.def("trimul_fwd", [](const at::Tensor& x, const std::optional<at::Tensor>& mask, const OptionalList& weights, bool outgoing, double eps) {
-    return trimul_fwd(x, mask.value_or(at::Tensor()), given(weights), outgoing, eps);
+  m.def("trimul_fwd", [](const at::Tensor& x, const std::optional<at::Tensor>& mask, const OptionalList& weights, bool outgoing, double eps, int64_t saved_bytes) {
+    return trimul_fwd(x, mask.value_or(at::Tensor()), given(weights), outgoing, eps, saved_bytes);
   });
   m.def("trimul_bwd", [](const at::Tensor& x, const std::optional<at::Tensor>& mask, const OptionalList& weights, const at::Tensor& saved, bool outgoing,
                          uint32_t need, const at::Tensor& dout) {

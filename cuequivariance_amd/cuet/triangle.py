@@ -289,18 +289,29 @@ def _placeholders(ref: torch.Tensor, tensors):
     return [ref.new_empty(0) if t is None else t for t in tensors], [int(t is not None) for t in tensors]
 
 
+def _saved_bytes(x: torch.Tensor):
+    """An upper bound of ``cueq_trimul_saved_bytes`` that takes a symbolic side: the pair rows of a square whose side is rounded up to
+    whole 16-byte pieces, what the forward keeps of them (x hat, y, the two factors, t; four statistics; with a ragged side the
+    padded input and mask), and the most that the pieces' alignment adds."""
+    B, N, _, D = x.shape
+    size = x.element_size()
+    piece = 16 // size
+    padding = N * (piece - 1) % piece  # (-N modulo a piece; no term of what follows can be negative, so no guard is needed for the size)
+    ragged = (padding + piece - 1) // piece  # 0 or 1
+    rows = B * (N + padding) * (N + padding)
+    return rows * (5 * D * size + 16) + ragged * rows * (D + 1) * size + 10 * 22528
+
+
 @torch.library.custom_op("cuequivariance_amd::trimul_fwd", mutates_args=(), device_types="cuda")
 def _trimul_fwd_op(x: torch.Tensor, tensors: List[torch.Tensor], present: List[int], outgoing: bool, eps: float) -> List[torch.Tensor]:
     args = [t if p else None for t, p in zip(tensors, present)]  # mask, then the 12 weights
-    return list(_lib.host().trimul_fwd(x, args[0], args[1:], outgoing, eps))
+    return list(_lib.host().trimul_fwd(x, args[0], args[1:], outgoing, eps, _saved_bytes(x)))
 
 
 @_trimul_fwd_op.register_fake
 def _trimul_fwd_fake(x, tensors, present, outgoing, eps):
-    Bsz, N, _, D = x.shape
-    Do = tensors[9].shape[0]  # p_out_weight
-    return [x.new_empty(Bsz, N, N, Do),
-            x.new_empty(_lib.load().cueq_trimul_saved_bytes(_CODE[x.dtype], int(Bsz), int(N), int(D), int(Do)), dtype=torch.uint8)]
+    Bsz, N = x.shape[:2]
+    return [x.new_empty(Bsz, N, N, tensors[9].shape[0]), x.new_empty(_saved_bytes(x), dtype=torch.uint8)]  # (tensors[9]: p_out_weight)
 
 
 @torch.library.custom_op("cuequivariance_amd::trimul_bwd", mutates_args=(), device_types="cuda")
