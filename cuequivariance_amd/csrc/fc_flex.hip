@@ -154,6 +154,10 @@ __device__ __forceinline__ void fc_load4(float (&v)[4][DR], const TI* __restrict
   }
 }
 
+// c x + s, and s where there is no coupling (c, the same in all lanes, is zero): an infinite or undefined x reaches only the
+// components that it is coupled to.  (By its bits, so that the test is a scalar one; the host writes no negative zero.)
+__device__ __forceinline__ float fc_coupled(float c, float x, float s) { return fmaf(c, __builtin_bit_cast(uint32_t, c) == 0 ? 0.f : x, s); }
+
 // (a channel of x2 is a part of its own here: a loop over them costs the registers of straight code)
 template <typename TI, int DS, int DR, int WM, bool MI, bool DX2>
 __device__ __forceinline__ void fc_part(fx16 (&acc)[DR], const FcPart& part, const FcBlock& blk, const TI* __restrict__ row, const TI* __restrict__ W,
@@ -172,14 +176,15 @@ __device__ __forceinline__ void fc_part(fx16 (&acc)[DR], const FcPart& part, con
 #pragma unroll
     for (int i = 0; i < DS; ++i)
 #pragma unroll
-      for (int k = 0; k < DR; ++k) s[i][k] = fmaf(cf[(i * DR + k) * part.d2 + j], xj, s[i][k]);
+      for (int k = 0; k < DR; ++k) s[i][k] = fc_coupled(cf[(i * DR + k) * part.d2 + j], xj, s[i][k]);
   }
 #pragma unroll
   for (int k = 0; k < DR; ++k)
 #pragma unroll
     for (int i = 0; i < DS; ++i)
+      if (part.mask >> (i * DR + k) & 1)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[k][r] = fmaf(s[i][k], T[i][r], acc[k][r]);
+        for (int r = 0; r < 16; ++r) acc[k][r] = fmaf(s[i][k], T[i][r], acc[k][r]);
   if constexpr (DX2) {
     float y[DS][DR];
 #pragma unroll
@@ -196,8 +201,9 @@ __device__ __forceinline__ void fc_part(fx16 (&acc)[DR], const FcPart& part, con
         for (int i = 0; i < DS; ++i)
 #pragma unroll
           for (int k = 0; k < DR; ++k)
+            if (part.mask >> (i * DR + k) & 1)
 #pragma unroll
-            for (int b = 0; b < 4; ++b) y[i][k] = fmaf(T[i][4 * a + b], xv[b][k], y[i][k]);
+              for (int b = 0; b < 4; ++b) y[i][k] = fmaf(T[i][4 * a + b], xv[b][k], y[i][k]);
       }
     }
 #pragma unroll
@@ -210,17 +216,29 @@ __device__ __forceinline__ void fc_part(fx16 (&acc)[DR], const FcPart& part, con
 #pragma unroll
       for (int i = 0; i < DS; ++i)
 #pragma unroll
-        for (int k = 0; k < DR; ++k) d = fmaf(cf[(i * DR + k) * part.d2 + j], y[i][k], d);
+        for (int k = 0; k < DR; ++k) d = fc_coupled(cf[(i * DR + k) * part.d2 + j], y[i][k], d);
       sums[part.j0 + j * part.js] += d;
     }
   }
 }
 
-// The components that a product of irreps of degree 0 and 1 couples (d1 x d2 -> d3 with d <= 3, and 3 x 5 -> 3): which (i, k) have a
-// coefficient at all is known when the kernel is compiled, and its loops are straight code.
+// The components that a product of irreps of degree 0 and 1 couples (d1 x d2 -> d3 with d <= 3, and 3 x 5 -> 3, symmetric in the
+// two threes): which (i, j, k) have a coefficient at all is known when the kernel is compiled, and its loops are straight code
+// that touches nothing else.  The host tests its coefficients against the same rule (_couples in dense.py).
+template <int DS, int DR, int D2>
+constexpr bool fc_couples(int i, int k, int j) {
+  if (DS == 1 && DR == 1) return true;
+  if (DS == 1) return j == k;
+  if (DR == 1) return j == i;
+  if (D2 == 1) return i == k;
+  if (D2 == 3) return i != k && j == 3 - i - k;
+  return j == 0 ? i + k == 2 && i != k : j == 1 ? i + k == 1 : j == 2 ? i == k : j == 3 ? i + k == 3 : i == k && i != 1;
+}
 template <int DS, int DR, int D2>
 constexpr bool fc_couples(int i, int k) {
-  return DS != 3 || DR != 3 || (D2 == 1 ? i == k : D2 == 3 ? i != k : true);
+  for (int j = 0; j < D2; ++j)
+    if (fc_couples<DS, DR, D2>(i, k, j)) return true;
+  return false;
 }
 
 // 2-byte elements where x2 has several channels, packed weights, K <= 16 KT and the couplings above: the source block of the row stays in registers over
@@ -296,7 +314,8 @@ __device__ __forceinline__ void fc_part_channels(fx16 (&acc)[DR], const FcPart& 
           s[i][k] = 0.f;
           if (fc_couples<DS, DR, D2>(i, k))
 #pragma unroll
-            for (int j = 0; j < D2; ++j) s[i][k] = fmaf(cf[(i * DR + k) * D2 + j], xj[j], s[i][k]);
+            for (int j = 0; j < D2; ++j)
+              if (fc_couples<DS, DR, D2>(i, k, j)) s[i][k] = fmaf(cf[(i * DR + k) * D2 + j], xj[j], s[i][k]);
         }
 #pragma unroll
       for (int k = 0; k < DR; ++k)
@@ -350,7 +369,7 @@ __device__ __forceinline__ void fc_part_channels(fx16 (&acc)[DR], const FcPart& 
           for (int i = 0; i < DS; ++i)
 #pragma unroll
             for (int k = 0; k < DR; ++k)
-              if (fc_couples<DS, DR, D2>(i, k)) d = fmaf(cf[(i * DR + k) * D2 + j], y[i][k], d);
+              if (fc_couples<DS, DR, D2>(i, k, j)) d = fmaf(cf[(i * DR + k) * D2 + j], y[i][k], d);
           if ((j & 1) == h) sums[y0 + j * part.js] += d;
         }
       }
@@ -550,7 +569,7 @@ __device__ __forceinline__ void fc_grad_tile(const FcGrad& q, int tile, const fl
 #pragma unroll
       for (int i = 0; i < NI; ++i)
 #pragma unroll
-        for (int k = 0; k < D3; ++k) s[i][k] = fmaf(cf[((i0 + i) * D3 + k) * q.d2 + j], xj, s[i][k]);
+        for (int k = 0; k < D3; ++k) s[i][k] = fc_coupled(cf[((i0 + i) * D3 + k) * q.d2 + j], xj, s[i][k]);
     }
 #pragma unroll
     for (int a = 0; a < 2; ++a) {
@@ -563,7 +582,8 @@ __device__ __forceinline__ void fc_grad_tile(const FcGrad& q, int tile, const fl
         x[a][i] = in ? xv : 0.f;
         float t = 0.f;
 #pragma unroll
-        for (int k = 0; k < D3; ++k) t = fmaf(s[i][k], g[k], t);
+        for (int k = 0; k < D3; ++k)
+          if (q.mask >> ((i0 + i) * D3 + k) & 1) t = fmaf(s[i][k], g[k], t);
         hv[a][i] = in ? t : 0.f;
       }
     }
@@ -752,6 +772,7 @@ __device__ __forceinline__ void fc_grad_channels(const FcGrad& q, int tile, cons
             for (int e = 0; e < 8; ++e) s[e] = 0.f;
 #pragma unroll
             for (int j = 0; j < D2; ++j) {
+              if (!fc_couples<D1, D3, D2>(i, k, j)) continue;
               const float f = cf[(i * D3 + k) * D2 + j];
               const float4 lo = *reinterpret_cast<const float4*>(yv + j * kDvRows), hi = *reinterpret_cast<const float4*>(yv + j * kDvRows + 4);
               s[0] = fmaf(f, lo.x, s[0]); s[1] = fmaf(f, lo.y, s[1]); s[2] = fmaf(f, lo.z, s[2]); s[3] = fmaf(f, lo.w, s[3]);
@@ -846,7 +867,7 @@ __global__ void __launch_bounds__(256) fc_factors_kernel(const FcGrad* __restric
       const int n = q.D1 * q.D3;
       if (lane < n) {
         float f = 0.f;
-        for (int j = 0; j < q.d2; ++j) f = fmaf(coef[q.coef + lane * q.d2 + j], fc_widen(yr + j), f);
+        for (int j = 0; j < q.d2; ++j) f = fc_coupled(coef[q.coef + lane * q.d2 + j], fc_widen(yr + j), f);
         s[off + lane] = f;
       }
       off += n;
@@ -868,7 +889,7 @@ __global__ void __launch_bounds__(256) fc_factors_kernel(const FcGrad* __restric
           float a = 0.f, b = 0.f;
 #pragma unroll
           for (int k = 0; k < 5; ++k)
-            if (k < q.D3) {
+            if (k < q.D3 && (q.mask >> (i * q.D3 + k) & 1)) {
               const float f = s[off + i * q.D3 + k];
               a = fmaf(f, ga[k], a);
               b = fmaf(f, gb[k], b);

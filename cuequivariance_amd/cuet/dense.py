@@ -317,6 +317,19 @@ def _linear_op(mod: "SegmentedPolynomialDense"):
     return op
 
 
+def _couples(d1, d2, d3, i, j, k) -> bool:
+    """Whether the straight kernels of ``csrc/fc_flex.hip`` (``fc_couples`` there) take the coefficient ``(i, j, k)`` of a path."""
+    if (d1, d2, d3) not in ((1, 1, 1), (1, 3, 3), (3, 3, 1), (3, 1, 3), (3, 3, 3), (3, 5, 3)):
+        return False
+    if d1 == 1 or d3 == 1:
+        return j == (k if d1 == 1 else i)
+    if d2 == 1:
+        return i == k
+    if d2 == 3:
+        return i != k and j == 3 - i - k
+    return (i + k == 2 and i != k, i + k == 1, i == k, i + k == 3, i == k and i != 1)[j]
+
+
 def _fc_tables(mod, x2_mul_ir: bool = False):
     """Packed tables of ``csrc/fc_flex.hip`` for a product ``uvw,iu,jv,kw+ijk`` (any ``v``; ``uw,iu,j,kw+ijk`` is ``v = 1``), the second
     operand's rows in ``ir_mul`` or ``mul_ir``: ``((blocks and parts forward, of the input gradient, weight gradients, coefficients),
@@ -336,13 +349,14 @@ def _fc_tables(mod, x2_mul_ir: bool = False):
         if d1 not in (1, 3, 5) or d3 not in (1, 3, 5):
             return None
         at = len(coef)
-        coef += [float(v) for v in c.transpose(0, 2, 1).reshape(-1)]
+        coef += [float(v) + 0.0 for v in c.transpose(0, 2, 1).reshape(-1)]  # (no negative zeros: the kernels test for zero by the bits)
         back = len(coef)
-        coef += [float(v) for v in c.transpose(2, 0, 1).reshape(-1)]
+        coef += [float(v) + 0.0 for v in c.transpose(2, 0, 1).reshape(-1)]
         used = (c != 0).any(axis=1)  # (i, k)
         mask = sum(1 << (i * d3 + k) for i in range(d1) for k in range(d3) if used[i, k])
         mask_back = sum(1 << (k * d1 + i) for i in range(d1) for k in range(d3) if used[i, k])
-        paths.append(SimpleNamespace(w0=offs[0][sw], a0=offs[1][s1], K=K, d1=d1, c0=offs[3][so], N=N, d3=d3, coef=at, coef_back=back, j0=offs[2][s2],
+        coupled = all(_couples(d1, d2, d3, i, j, k) for i, j, k in zip(*c.nonzero()))
+        paths.append(SimpleNamespace(coupled=coupled, w0=offs[0][sw], a0=offs[1][s1], K=K, d1=d1, c0=offs[3][so], N=N, d3=d3, coef=at, coef_back=back, j0=offs[2][s2],
                                      d2=d2, V=V, js=1 if x2_mul_ir else V, vs=d2 if x2_mul_ir else 1, mask=mask, mask_back=mask_back))
     if len({p.w0 for p in paths}) != len(paths) or sum(p.K * p.V * p.N for p in paths) != sizes[0] or sizes[2] > 128:
         return None
@@ -354,11 +368,8 @@ def _fc_tables(mod, x2_mul_ir: bool = False):
     if not served:
         return None
 
-    # the couplings that the kernels with straight loops over the channels of x2 know (fc_couples); blocks held in registers there
-    # have up to 64 values
-    diagonal, all9 = 0b100010001, 0b111111111
-    allowed = {(1, 1, 1): 1, (1, 3, 3): 7, (3, 3, 1): 7, (3, 1, 3): diagonal, (3, 3, 3): all9 & ~diagonal, (3, 5, 3): all9}  # (d1, d2, d3)
-    straight = all((p.d1, p.d2, p.d3) in allowed and not (p.mask | p.mask_back) & ~allowed[p.d1, p.d2, p.d3] for p in paths)
+    # the couplings that the kernels with straight loops over the channels of x2 know; blocks held in registers there have up to 64 values
+    straight = all(p.coupled for p in paths)
     resident = straight and all(p.K <= 64 and p.N <= 64 for p in paths)
     steps = {True: 2 if all(p.N <= 32 for p in paths) else 4, False: 2 if all(p.K <= 32 for p in paths) else 4}  # (by direction: of 16 values)
 
