@@ -31,6 +31,7 @@ COMMON_FLAGS = [
     "-fPIC",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-command-line-argument",
+    "-Werror=return-type",  # (device code that runs off the end of a function goes on into whatever follows it)
     f"-I{ROOT / 'include'}",
     f"-I{CSRC}",
 ]

@@ -154,9 +154,96 @@ __device__ __forceinline__ void fc_load4(float (&v)[4][DR], const TI* __restrict
   }
 }
 
-// c x + s, and s where there is no coupling (c, the same in all lanes, is zero): an infinite or undefined x reaches only the
-// components that it is coupled to.  (By its bits, so that the test is a scalar one; the host writes no negative zero.)
-__device__ __forceinline__ float fc_coupled(float c, float x, float s) { return fmaf(c, __builtin_bit_cast(uint32_t, c) == 0 ? 0.f : x, s); }
+// Structural zeros.  The plain kernels multiply every pair of components by its factor, those that no coefficient couples among
+// them: with finite values a factor of zero adds nothing, but 0 * inf would make the whole row NaN where one component has
+// overflowed.  Results that are all finite have met finite values only; a wavefront that finds one of its results infinite or undefined
+// leaves the tile to fc_tile_coupled / fc_grad_coupled, which touch coupled components alone, in a simple loop of few registers
+// behind the straight code.  Tests for couplings in the straight code instead: forward of 3 000 rows of
+// 64 channels up to l = 2 (x) 8, float, 234 -> 280 us.
+__device__ __forceinline__ float fc_coupled(float c, float x, float s) { return fmaf(c, c == 0.f ? 0.f : x, s); }
+__device__ __forceinline__ float fc_probe(const fx16& v, float probe) {  // stays 0 while everything is finite
+#pragma unroll
+  for (int r = 0; r < 16; ++r) probe = fmaf(v[r], 0.f, probe);
+  return probe;
+}
+
+// one tile: a row and half of the columns a lane, four at a time; with X1 also the row sums of the gradient of x2
+template <typename TI>
+__device__ __forceinline__ void fc_tile_coupled(const FcBlock* __restrict__ block, const FcPart* __restrict__ parts, const float* __restrict__ coef,
+                                                          const TI* __restrict__ A, int64_t lda, const TI* __restrict__ W, const TI* __restrict__ X2,
+                                                          int64_t ldx2, const TI* __restrict__ X1, int64_t ldx1, TI* __restrict__ C, int64_t ldc,
+                                                          float* __restrict__ partial, float* lsum, int wm, bool mi, int n2, int64_t Z, int64_t z0, int n0) {
+  const FcBlock blk = *block;
+  const int lane = threadIdx.x & 63, c = lane & 31, h = lane >> 5, DR = blk.D, n2p = n2 | 1;
+  const int64_t z = min(z0 + c, Z - 1);
+  const TI *row = A + z * lda, *x2row = X2 + z * ldx2, *x1row = X1 ? X1 + z * ldx1 : nullptr;
+  float* sums = lsum + c * n2p;
+  if (x1row && h == 0)
+    for (int j = 0; j < n2; ++j) sums[j] = 0.f;
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll 1
+  for (int m0 = n0 + 16 * h; m0 < n0 + 16 * h + 16; m0 += 4) {
+    float acc[5][4];
+#pragma unroll
+    for (int k = 0; k < 5; ++k)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[k][e] = 0.f;
+#pragma unroll 1
+    for (int p = 0; p < blk.parts; ++p) {
+      const FcPart part = parts[blk.first + p];
+#pragma unroll 1
+      for (int i = 0; i < part.D; ++i) {
+        float t[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+        for (int u = 0; u < part.K; ++u) {
+          const float x = fc_widen(row + part.a0 + (mi ? u * part.D + i : i * part.K + u));
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int n = min(m0 + e, blk.N - 1);
+            const int64_t at = wm == kPacked ? static_cast<int64_t>((u >> 4) * part.stride + (n >> 5)) * kFragment + ((u >> 3 & 1) * 32 + (n & 31)) * 8 + (u & 7)
+                               : wm == kTransposed ? static_cast<int64_t>(n) * part.stride + u : static_cast<int64_t>(u) * part.stride + n;
+            t[e] = fmaf(x, fc_widen(W + part.w0 + at), t[e]);
+          }
+        }
+#pragma unroll
+        for (int k = 0; k < 5; ++k) {
+          if (k >= DR || !(part.mask >> (i * DR + k) & 1)) continue;
+          const float* cf = coef + part.coef + (i * DR + k) * part.d2;
+          float s = 0.f;
+#pragma unroll 1
+          for (int j = 0; j < part.d2; ++j) s = fc_coupled(cf[j], fc_widen(x2row + part.j0 + j * part.js), s);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[k][e] = fmaf(s, t[e], acc[k][e]);
+          if (!x1row) continue;
+          float y = 0.f;
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (m0 + e < blk.N) y = fmaf(t[e], fc_widen(x1row + blk.c0 + (mi ? (m0 + e) * DR + k : k * blk.N + m0 + e)), y);
+          y += __shfl_xor(y, 32, 64);
+          if (h == 0)
+#pragma unroll 1
+            for (int j = 0; j < part.d2; ++j) sums[part.j0 + j * part.js] = fc_coupled(cf[j], y, sums[part.j0 + j * part.js]);
+        }
+      }
+    }
+    if (z0 + c >= Z) continue;
+    TI* out = C + z * ldc + blk.c0;
+#pragma unroll
+    for (int k = 0; k < 5; ++k)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (k >= DR || m0 + e >= blk.N) continue;
+        TI* to = out + (mi ? (m0 + e) * DR + k : k * blk.N + m0 + e);
+        if constexpr (sizeof(TI) == 4) *to = acc[k][e];
+        else *reinterpret_cast<uint16_t*>(to) = mm_round<TI>(acc[k][e]);
+      }
+  }
+  if (x1row) {
+    __builtin_amdgcn_wave_barrier();
+    const int64_t rows = min<int64_t>(32, Z - z0);
+    for (int e = lane; e < rows * n2; e += 64) partial[z0 * n2 + e] = lsum[e / n2 * n2p + e % n2];
+  }
+}
 
 // (a channel of x2 is a part of its own here: a loop over them costs the registers of straight code)
 template <typename TI, int DS, int DR, int WM, bool MI, bool DX2>
@@ -176,15 +263,14 @@ __device__ __forceinline__ void fc_part(fx16 (&acc)[DR], const FcPart& part, con
 #pragma unroll
     for (int i = 0; i < DS; ++i)
 #pragma unroll
-      for (int k = 0; k < DR; ++k) s[i][k] = fc_coupled(cf[(i * DR + k) * part.d2 + j], xj, s[i][k]);
+      for (int k = 0; k < DR; ++k) s[i][k] = fmaf(cf[(i * DR + k) * part.d2 + j], xj, s[i][k]);
   }
 #pragma unroll
   for (int k = 0; k < DR; ++k)
 #pragma unroll
     for (int i = 0; i < DS; ++i)
-      if (part.mask >> (i * DR + k) & 1)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[k][r] = fmaf(s[i][k], T[i][r], acc[k][r]);
+      for (int r = 0; r < 16; ++r) acc[k][r] = fmaf(s[i][k], T[i][r], acc[k][r]);
   if constexpr (DX2) {
     float y[DS][DR];
 #pragma unroll
@@ -201,9 +287,8 @@ __device__ __forceinline__ void fc_part(fx16 (&acc)[DR], const FcPart& part, con
         for (int i = 0; i < DS; ++i)
 #pragma unroll
           for (int k = 0; k < DR; ++k)
-            if (part.mask >> (i * DR + k) & 1)
 #pragma unroll
-              for (int b = 0; b < 4; ++b) y[i][k] = fmaf(T[i][4 * a + b], xv[b][k], y[i][k]);
+            for (int b = 0; b < 4; ++b) y[i][k] = fmaf(T[i][4 * a + b], xv[b][k], y[i][k]);
       }
     }
 #pragma unroll
@@ -216,7 +301,7 @@ __device__ __forceinline__ void fc_part(fx16 (&acc)[DR], const FcPart& part, con
 #pragma unroll
       for (int i = 0; i < DS; ++i)
 #pragma unroll
-        for (int k = 0; k < DR; ++k) d = fc_coupled(cf[(i * DR + k) * part.d2 + j], y[i][k], d);
+        for (int k = 0; k < DR; ++k) d = fmaf(cf[(i * DR + k) * part.d2 + j], y[i][k], d);
       sums[part.j0 + j * part.js] += d;
     }
   }
@@ -380,8 +465,9 @@ __device__ __forceinline__ void fc_part_channels(fx16 (&acc)[DR], const FcPart& 
 // 32-bit words from row to row of x2 in LDS
 __host__ __device__ constexpr int fc_x2_words(int n2) { return (n2 + 1) / 2 | 1; }
 
+// false: some result is not finite, nothing is stored
 template <typename TI, int DR, int WM, bool MI, bool DX2, int MAXD, int KT>
-__device__ __forceinline__ void fc_tile(const FcBlock& blk, const FcPart* __restrict__ parts, const float* __restrict__ coef, const TI* __restrict__ A, int64_t lda,
+__device__ __forceinline__ bool fc_tile(const FcBlock& blk, const FcPart* __restrict__ parts, const float* __restrict__ coef, const TI* __restrict__ A, int64_t lda,
                                         const TI* __restrict__ W, const TI* __restrict__ X2, int64_t ldx2, const TI* __restrict__ X1, int64_t ldx1,
                                         TI* __restrict__ C, int64_t ldc, float* __restrict__ partial, float* lsum, uint4* wl, int n2, int64_t Z, int64_t z0, int n0) {
   constexpr int ES = sizeof(TI);
@@ -433,6 +519,16 @@ __device__ __forceinline__ void fc_tile(const FcBlock& blk, const FcPart* __rest
         if constexpr (MAXD > 3) one(std::integral_constant<int, 5>{}, part);
     }
   }
+  if constexpr (KT == 0) {  // (the straight kernels touch coupled components only)
+    float probe = 0.f;
+#pragma unroll
+    for (int k = 0; k < DR; ++k) probe = fc_probe(acc[k], probe);
+    if constexpr (DX2) {
+      __builtin_amdgcn_wave_barrier();
+      for (int e = h; e < n2; e += 2) probe = fmaf(sums[e], 0.f, probe);
+    }
+    if (__any(!(probe == 0.f))) return false;
+  }
   if (z0 + c < Z) {
     TI* out = C + z * ldc + blk.c0;
 #pragma unroll
@@ -455,6 +551,7 @@ __device__ __forceinline__ void fc_tile(const FcBlock& blk, const FcPart* __rest
     const int64_t rows = min<int64_t>(32, Z - z0);
     for (int e = lane; e < rows * n2; e += 64) partial[z0 * n2 + e] = lsum[e / n2 * n2p + e % n2];
   }
+  return true;
 }
 
 // MAXD: the most components of any block (3 or 5): what the register budget has to hold.
@@ -487,11 +584,15 @@ __global__ void __launch_bounds__(256, (MAXD > 3 || KT > 0 ? 2 : 3)) fc_rows_ker
   uint4* wl = reinterpret_cast<uint4*>(fc_lsum);
   float* lsum = fc_lsum + (KT > 0 ? 16 * 64 * 4 : 0) + wave * 32 * (n2 | 1);
   float* part = DX2 ? partial + static_cast<int64_t>(column) * Z * n2 : nullptr;
+  bool whole = true;
   switch (blk.D) {
-    case 1: fc_tile<TI, 1, WM, MI, DX2, MAXD, KT>(blk, parts, coef, A, lda, W, X2, ldx2, X1, ldx1, C, ldc, part, lsum, wl, n2, Z, z0, tile * 32); break;
-    case 3: fc_tile<TI, 3, WM, MI, DX2, MAXD, KT>(blk, parts, coef, A, lda, W, X2, ldx2, X1, ldx1, C, ldc, part, lsum, wl, n2, Z, z0, tile * 32); break;
+    case 1: whole = fc_tile<TI, 1, WM, MI, DX2, MAXD, KT>(blk, parts, coef, A, lda, W, X2, ldx2, X1, ldx1, C, ldc, part, lsum, wl, n2, Z, z0, tile * 32); break;
+    case 3: whole = fc_tile<TI, 3, WM, MI, DX2, MAXD, KT>(blk, parts, coef, A, lda, W, X2, ldx2, X1, ldx1, C, ldc, part, lsum, wl, n2, Z, z0, tile * 32); break;
     default:
-      if constexpr (MAXD > 3) fc_tile<TI, 5, WM, MI, DX2, MAXD, KT>(blk, parts, coef, A, lda, W, X2, ldx2, X1, ldx1, C, ldc, part, lsum, wl, n2, Z, z0, tile * 32);
+      if constexpr (MAXD > 3) whole = fc_tile<TI, 5, WM, MI, DX2, MAXD, KT>(blk, parts, coef, A, lda, W, X2, ldx2, X1, ldx1, C, ldc, part, lsum, wl, n2, Z, z0, tile * 32);
+  }
+  if constexpr (KT == 0) {
+    if (!whole) fc_tile_coupled<TI>(blocks + b, parts, coef, A, lda, W, X2, ldx2, DX2 ? X1 : nullptr, ldx1, C, ldc, part, lsum, WM, MI, n2, Z, z0, tile * 32);
   }
 }
 
@@ -531,8 +632,49 @@ struct FcGrad {  // weight gradient of one path
   uint32_t mask;
 };
 
+// one 64 x 64 tile of the weight gradient of one path and channel of x2, coupled components alone: a column and every other row a lane
+template <typename TI>
+__device__ __forceinline__ void fc_grad_coupled(const FcGrad* __restrict__ grad, const float* __restrict__ coef, const TI* __restrict__ X1, int64_t ldx1,
+                                                          const TI* __restrict__ X2, int64_t ldx2, const TI* __restrict__ G, int64_t ldg, float* __restrict__ P,
+                                                          bool mi, int tile, int64_t zb, int64_t ze) {
+  const FcGrad q = *grad;
+  const int per = q.nt / q.V, channel = tile / per, u0 = tile % per / q.ntv * 64, v0 = tile % per % q.ntv * 64;
+  const int c = threadIdx.x & 31, h = (threadIdx.x >> 5) & 1;
+#pragma unroll 1
+  for (int part = 0; part < 8; ++part) {
+    const int v = v0 + 32 * (part & 1) + c, vr = min(v, q.N - 1), ub = u0 + 16 * (part >> 1) + 8 * h;
+    float acc[8];
+#pragma unroll
+    for (int r = 0; r < 8; ++r) acc[r] = 0.f;
+#pragma unroll 1
+    for (int64_t z = zb; z < ze; ++z) {
+      const TI *xr = X1 + z * ldx1 + q.a0, *gr = G + z * ldg + q.c0, *yr = X2 + z * ldx2 + q.j0 + channel * q.vs;
+#pragma unroll 1
+      for (int i = 0; i < q.D1; ++i) {
+        float hv = 0.f;
+        for (int k = 0; k < q.D3; ++k) {
+          if (!(q.mask >> (i * q.D3 + k) & 1)) continue;
+          const float* cf = coef + q.coef + (i * q.D3 + k) * q.d2;
+          float s = 0.f;
+          for (int j = 0; j < q.d2; ++j) s = fc_coupled(cf[j], fc_widen(yr + j * q.js), s);
+          hv = fmaf(s, fc_widen(gr + (mi ? vr * q.D3 + k : k * q.N + vr)), hv);
+        }
+        if constexpr (sizeof(TI) == 2) hv = mm_widen<TI>(mm_round<TI>(hv));  // (an operand of a product there: of the rows' type)
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+          const int u = min(ub + r, q.K - 1);
+          acc[r] = fmaf(fc_widen(xr + (mi ? u * q.D1 + i : i * q.K + u)), hv, acc[r]);
+        }
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < 8; ++r)
+      if (v < q.N && ub + r < q.K) P[q.w0 + channel * q.N + static_cast<int64_t>(ub + r) * q.stride + v] = acc[r];
+  }
+}
+
 template <typename TI, int D1, int D3, bool MI>
-__device__ __forceinline__ void fc_grad_tile(const FcGrad& q, int tile, const float* __restrict__ coef, const TI* __restrict__ X1, int64_t ldx1,
+__device__ __forceinline__ bool fc_grad_tile(const FcGrad& q, int tile, const float* __restrict__ coef, const TI* __restrict__ X1, int64_t ldx1,
                                              const TI* __restrict__ X2, int64_t ldx2, const TI* __restrict__ G, int64_t ldg, float* __restrict__ P, int64_t zb,
                                              int64_t ze) {
   constexpr int ES = sizeof(TI);
@@ -569,7 +711,7 @@ __device__ __forceinline__ void fc_grad_tile(const FcGrad& q, int tile, const fl
 #pragma unroll
       for (int i = 0; i < NI; ++i)
 #pragma unroll
-        for (int k = 0; k < D3; ++k) s[i][k] = fc_coupled(cf[((i0 + i) * D3 + k) * q.d2 + j], xj, s[i][k]);
+        for (int k = 0; k < D3; ++k) s[i][k] = fmaf(cf[((i0 + i) * D3 + k) * q.d2 + j], xj, s[i][k]);
     }
 #pragma unroll
     for (int a = 0; a < 2; ++a) {
@@ -582,8 +724,7 @@ __device__ __forceinline__ void fc_grad_tile(const FcGrad& q, int tile, const fl
         x[a][i] = in ? xv : 0.f;
         float t = 0.f;
 #pragma unroll
-        for (int k = 0; k < D3; ++k)
-          if (q.mask >> ((i0 + i) * D3 + k) & 1) t = fmaf(s[i][k], g[k], t);
+        for (int k = 0; k < D3; ++k) t = fmaf(s[i][k], g[k], t);
         hv[a][i] = in ? t : 0.f;
       }
     }
@@ -625,6 +766,12 @@ __device__ __forceinline__ void fc_grad_tile(const FcGrad& q, int tile, const fl
             acc[a][b] = mm_32x32x16<TI>(make_uint4(xp[a][0], xp[a][1], xp[a][2], xp[a][3]), make_uint4(hp[b][0], hp[b][1], hp[b][2], hp[b][3]), acc[a][b]);
       }
   }
+  float probe = 0.f;
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b) probe = fc_probe(acc[a][b], probe);
+  if (__any(!(probe == 0.f))) return false;
 #pragma unroll
   for (int a = 0; a < 2; ++a)
 #pragma unroll
@@ -637,6 +784,7 @@ __device__ __forceinline__ void fc_grad_tile(const FcGrad& q, int tile, const fl
         if (uu < q.K) P[q.w0 + channel * q.N + static_cast<int64_t>(uu) * q.stride + vv] = acc[a][b][r];
       }
     }
+  return true;
 }
 
 template <typename TI, bool MI>
@@ -653,7 +801,8 @@ __global__ void __launch_bounds__(256, 2) fc_grad_kernel(const FcGrad* __restric
   const FcGrad q = grads[b];
   const int64_t zb = chunk * rows_per_chunk, ze = min(zb + rows_per_chunk, Z);
   float* P = partial + chunk * numel;
-#define FC_TILE(A, B) fc_grad_tile<TI, A, B, MI>(q, tile, coef, X1, ldx1, X2, ldx2, G, ldg, P, zb, ze)
+#define FC_TILE(A, B) whole = fc_grad_tile<TI, A, B, MI>(q, tile, coef, X1, ldx1, X2, ldx2, G, ldg, P, zb, ze)
+  bool whole = true;
   switch (q.D1 * 8 + q.D3) {
     case 9: FC_TILE(1, 1); break;
     case 11: FC_TILE(1, 3); break;
@@ -666,6 +815,7 @@ __global__ void __launch_bounds__(256, 2) fc_grad_kernel(const FcGrad* __restric
     default: FC_TILE(5, 5);
   }
 #undef FC_TILE
+  if (!whole) fc_grad_coupled<TI>(grads + b, coef, X1, ldx1, X2, ldx2, G, ldg, P, MI, tile, zb, ze);
 }
 
 // Weight gradient of 2-byte rows where the x2 blocks have several channels: a workgroup takes 64 x 64 of one path for four channels,
@@ -858,47 +1008,62 @@ __global__ void __launch_bounds__(256) fc_factors_kernel(const FcGrad* __restric
     else *reinterpret_cast<uint32_t*>(to) = mm_pack<TI>(a, b);
   };
   for (int64_t z = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6); z < Z; z += static_cast<int64_t>(gridDim.x) * 4) {
-    TI* h = H + z * ldh;
-    int off = 0;
-    __builtin_amdgcn_wave_barrier();
-    for (int p = 0; p < ngrads; ++p) {  // the factors of the row, a lane each
-      const FcGrad q = grads[p];
-      const TI* yr = X2 + z * ldx2 + q.j0;
-      const int n = q.D1 * q.D3;
-      if (lane < n) {
-        float f = 0.f;
-        for (int j = 0; j < q.d2; ++j) f = fc_coupled(coef[q.coef + lane * q.d2 + j], fc_widen(yr + j), f);
-        s[off + lane] = f;
-      }
-      off += n;
-    }
-    __builtin_amdgcn_wave_barrier();
-    off = 0;
-    for (int p = 0; p < ngrads; ++p) {
-      const FcGrad q = grads[p];
-      const TI* gr = G + z * ldg + q.c0;
-      for (int w = 2 * lane; w < q.N; w += 128) {
-        float ga[5], gb[5];
-#pragma unroll
-        for (int k = 0; k < 5; ++k)
-          if (k < q.D3) {
-            ga[k] = fc_widen(gr + (MI ? w * q.D3 + k : k * q.N + w));
-            gb[k] = fc_widen(gr + (MI ? (w + 1) * q.D3 + k : k * q.N + w + 1));
+    auto factors = [&](auto coupled) {  // of the row, a lane each
+      int off = 0;
+      __builtin_amdgcn_wave_barrier();
+      for (int p = 0; p < ngrads; ++p) {
+        const FcGrad q = grads[p];
+        const TI* yr = X2 + z * ldx2 + q.j0;
+        const int n = q.D1 * q.D3;
+        if (lane < n) {
+          float f = 0.f;
+          for (int j = 0; j < q.d2; ++j) {
+            const float cj = coef[q.coef + lane * q.d2 + j], xj = fc_widen(yr + j);
+            f = decltype(coupled)::value ? fc_coupled(cj, xj, f) : fmaf(cj, xj, f);
           }
-        for (int i = 0; i < q.D1; ++i) {
-          float a = 0.f, b = 0.f;
+          s[off + lane] = f;
+        }
+        off += n;
+      }
+      __builtin_amdgcn_wave_barrier();
+    };
+    float probe = 0.f;
+    auto write = [&](auto coupled) {
+      TI* h = H + z * ldh;
+      int off = 0;
+      for (int p = 0; p < ngrads; ++p) {
+        const FcGrad q = grads[p];
+        const TI* gr = G + z * ldg + q.c0;
+        for (int w = 2 * lane; w < q.N; w += 128) {
+          float ga[5], gb[5];
 #pragma unroll
           for (int k = 0; k < 5; ++k)
-            if (k < q.D3 && (q.mask >> (i * q.D3 + k) & 1)) {
-              const float f = s[off + i * q.D3 + k];
-              a = fmaf(f, ga[k], a);
-              b = fmaf(f, gb[k], b);
+            if (k < q.D3) {
+              ga[k] = fc_widen(gr + (MI ? w * q.D3 + k : k * q.N + w));
+              gb[k] = fc_widen(gr + (MI ? (w + 1) * q.D3 + k : k * q.N + w + 1));
             }
-          store2(h + i * q.N + w, a, b);
+          for (int i = 0; i < q.D1; ++i) {
+            float a = 0.f, b = 0.f;
+#pragma unroll
+            for (int k = 0; k < 5; ++k)
+              if (k < q.D3 && (!decltype(coupled)::value || (q.mask >> (i * q.D3 + k) & 1))) {
+                const float f = s[off + i * q.D3 + k];
+                a = fmaf(f, ga[k], a);
+                b = fmaf(f, gb[k], b);
+              }
+            probe = fmaf(a, 0.f, fmaf(b, 0.f, probe));
+            store2(h + i * q.N + w, a, b);
+          }
         }
+        h += q.D1 * q.N;
+        off += q.D1 * q.D3;
       }
-      h += q.D1 * q.N;
-      off += q.D1 * q.D3;
+    };
+    factors(std::false_type{});
+    write(std::false_type{});
+    if (__any(!(probe == 0.f))) {  // (not finite: again, coupled components alone)
+      factors(std::true_type{});
+      write(std::true_type{});
     }
     if constexpr (MI) {
       for (int b = 0; b < nblocks1; ++b) {

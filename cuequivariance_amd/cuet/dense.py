@@ -349,9 +349,9 @@ def _fc_tables(mod, x2_mul_ir: bool = False):
         if d1 not in (1, 3, 5) or d3 not in (1, 3, 5):
             return None
         at = len(coef)
-        coef += [float(v) + 0.0 for v in c.transpose(0, 2, 1).reshape(-1)]  # (no negative zeros: the kernels test for zero by the bits)
+        coef += [float(v) for v in c.transpose(0, 2, 1).reshape(-1)]
         back = len(coef)
-        coef += [float(v) + 0.0 for v in c.transpose(2, 0, 1).reshape(-1)]
+        coef += [float(v) for v in c.transpose(2, 0, 1).reshape(-1)]
         used = (c != 0).any(axis=1)  # (i, k)
         mask = sum(1 << (i * d3 + k) for i in range(d1) for k in range(d3) if used[i, k])
         mask_back = sum(1 << (k * d1 + i) for i in range(d1) for k in range(d3) if used[i, k])
