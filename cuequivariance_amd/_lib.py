@@ -70,6 +70,8 @@ EXPORTED_SYMBOLS = (
     "cueq_layer_norm_fwd",
     "cueq_layer_norm_bwd_workspace",
     "cueq_layer_norm_bwd",
+    "cueq_gate_fwd",
+    "cueq_gate_bwd",
     "cueq_sum_cols",
     "cueq_sum_rows_workspace",
     "cueq_sum_rows",
@@ -274,6 +276,10 @@ def load() -> C.CDLL:
         lib.cueq_layer_norm_bwd_workspace.restype = i64
         lib.cueq_layer_norm_bwd.argtypes = [i32, i64, i64, ptr, ptr, ptr, ptr, ptr, ptr, ptr, ptr, ptr, i64, ptr]
         lib.cueq_layer_norm_bwd.restype = C.c_int
+        lib.cueq_gate_fwd.argtypes = [i32, i64, i64, ptr, ptr, ptr, ptr, i32, ptr, i32, ptr, ptr]
+        lib.cueq_gate_fwd.restype = C.c_int
+        lib.cueq_gate_bwd.argtypes = [i32, i64, i64, ptr, ptr, ptr, ptr, ptr, i32, ptr, i32, ptr, ptr, ptr]
+        lib.cueq_gate_bwd.restype = C.c_int
         lib.cueq_sum_cols.argtypes = [i32, i64, i64, ptr, ptr, ptr]
         lib.cueq_sum_cols.restype = C.c_int
         lib.cueq_sum_rows_workspace.argtypes = [i64, i64]

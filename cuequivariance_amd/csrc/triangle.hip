@@ -5,6 +5,7 @@
 //   cueq_gemm_nt        batched C = alpha * A * B^T (+ C), both operands contraction-contiguous, MFMA
 //   cueq_transpose      batched 2-D transpose through LDS
 //   cueq_layer_norm_*   row LayerNorm forward / backward (one wavefront per row)
+//   cueq_gate_*         out = sigmoid(u + bu) * (v + bv) * mask and its backward, of products that are in memory
 //   cueq_trimul_*       all of them in order, forward and backward
 //   cueq_sum_rows/cols  reductions for the bias / affine gradients
 // Math is fp32 throughout; tensors are fp32 or bf16.
@@ -2405,6 +2406,47 @@ __global__ void __launch_bounds__(256, 2) ln_t_bwd_cols_kernel(const F* __restri
   }
 }
 
+// ------------------------------------------------------------------------------------------------
+// gate: out[r][c] = sigmoid(u + bu) * (v + bv) * mask;  biases and mask are indexed by row (axis 0) or column (axis 1)
+// ------------------------------------------------------------------------------------------------
+template <typename T>
+__global__ void __launch_bounds__(256) gate_fwd_kernel(const float* __restrict__ u, const float* __restrict__ v, const T* __restrict__ bu,
+                                                       const T* __restrict__ bv, int bias_axis, const T* __restrict__ mask, int mask_axis,
+                                                       T* __restrict__ out, int64_t R, int64_t Ccols) {
+  const int64_t tid = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (tid >= R * Ccols) return;
+  const int64_t r = tid / Ccols, cc = tid - r * Ccols;
+  const int64_t ib = bias_axis == 0 ? r : cc;
+  const float uu = u[tid] + (bu ? tri_load(bu, ib) : 0.f);
+  const float vv = v[tid] + (bv ? tri_load(bv, ib) : 0.f);
+  float o = vv / (1.0f + __expf(-uu));
+  if (mask) o *= tri_load(mask, mask_axis == 0 ? r : cc);
+  tri_store(out, tid, o);
+}
+
+// du = dout * mask * (v + bv) * s * (1 - s),  dv = dout * mask * s,  s = sigmoid(u + bu)
+template <typename T>
+__global__ void __launch_bounds__(256) gate_bwd_kernel(const T* __restrict__ dout, const float* __restrict__ u, const float* __restrict__ v,
+                                                       const T* __restrict__ bu, const T* __restrict__ bv, int bias_axis,
+                                                       const T* __restrict__ mask, int mask_axis, T* __restrict__ du, T* __restrict__ dv,
+                                                       int64_t R, int64_t Ccols) {
+  const int64_t tid = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (tid >= R * Ccols) return;
+  const int64_t r = tid / Ccols, cc = tid - r * Ccols;
+  const int64_t ib = bias_axis == 0 ? r : cc;
+  const float uu = u[tid] + (bu ? tri_load(bu, ib) : 0.f);
+  const float vv = v[tid] + (bv ? tri_load(bv, ib) : 0.f);
+  const float s = 1.0f / (1.0f + __expf(-uu));
+  float d = tri_load(dout, tid);
+  if (mask) d *= tri_load(mask, mask_axis == 0 ? r : cc);
+  tri_store(du, tid, d * vv * s * (1.0f - s));
+  tri_store(dv, tid, d * s);
+}
+
+// ------------------------------------------------------------------------------------------------
+// reductions of an (R x C) array: sum over columns -> [R] (one wavefront per row);
+// sum over rows -> [C] (two stages through per-block partials)
+// ------------------------------------------------------------------------------------------------
 template <typename TI>
 __global__ void __launch_bounds__(256) sum_cols_kernel(const TI* __restrict__ in, float* __restrict__ out, int64_t R, int64_t Ccols) {
   const int lane = threadIdx.x & 63;
@@ -3262,6 +3304,43 @@ extern "C" int cueq_layer_norm_t_bwd(int32_t dtype, int64_t M, int64_t D, const 
   return CUEQ_OK;
 }
 
+extern "C" int cueq_gate_fwd(int32_t dtype, int64_t rows, int64_t cols, const float* u, const float* v, const void* bias_u, const void* bias_v,
+                             int32_t bias_axis, const void* mask, int32_t mask_axis, void* out, void* stream_) {
+  hipStream_t stream = static_cast<hipStream_t>(stream_);
+  CUEQ_REQUIRE(is_io(dtype), CUEQ_ERR_UNSUPPORTED, "gate: dtype must be float32 or bfloat16");
+  const int64_t n = rows * cols;
+  if (n <= 0) return CUEQ_OK;
+  CUEQ_REQUIRE(u && v && out, CUEQ_ERR_INVALID, "gate: null operand");
+  CUEQ_REQUIRE((n + 255) / 256 < (1ll << 31), CUEQ_ERR_TOO_LARGE, "gate: too many elements");
+  const dim3 grid(static_cast<unsigned>((n + 255) / 256));
+  KernelTimer timer("gate_fwd", stream);
+  TRI_DISPATCH(dtype,
+               hipLaunchKernelGGL(gate_fwd_kernel<float>, grid, dim3(256), 0, stream, u, v, static_cast<const float*>(bias_u), static_cast<const float*>(bias_v), bias_axis, static_cast<const float*>(mask), mask_axis, static_cast<float*>(out), rows, cols),
+               hipLaunchKernelGGL(gate_fwd_kernel<uint16_t>, grid, dim3(256), 0, stream, u, v, static_cast<const uint16_t*>(bias_u), static_cast<const uint16_t*>(bias_v), bias_axis, static_cast<const uint16_t*>(mask), mask_axis, static_cast<uint16_t*>(out), rows, cols),
+               hipLaunchKernelGGL(gate_fwd_kernel<f16bits>, grid, dim3(256), 0, stream, u, v, static_cast<const f16bits*>(bias_u), static_cast<const f16bits*>(bias_v), bias_axis, static_cast<const f16bits*>(mask), mask_axis, static_cast<f16bits*>(out), rows, cols));
+  CUEQ_CHECK_HIP(hipGetLastError());
+  return CUEQ_OK;
+}
+
+extern "C" int cueq_gate_bwd(int32_t dtype, int64_t rows, int64_t cols, const void* dout, const float* u, const float* v, const void* bias_u,
+                             const void* bias_v, int32_t bias_axis, const void* mask, int32_t mask_axis, void* du, void* dv, void* stream_) {
+  hipStream_t stream = static_cast<hipStream_t>(stream_);
+  CUEQ_REQUIRE(is_io(dtype), CUEQ_ERR_UNSUPPORTED, "gate: dtype must be float32 or bfloat16");
+  const int64_t n = rows * cols;
+  if (n <= 0) return CUEQ_OK;
+  CUEQ_REQUIRE(dout && u && v && du && dv, CUEQ_ERR_INVALID, "gate: null operand");
+  CUEQ_REQUIRE((n + 255) / 256 < (1ll << 31), CUEQ_ERR_TOO_LARGE, "gate: too many elements");
+  const dim3 grid(static_cast<unsigned>((n + 255) / 256));
+  KernelTimer timer("gate_bwd", stream);
+  TRI_DISPATCH(dtype,
+               hipLaunchKernelGGL(gate_bwd_kernel<float>, grid, dim3(256), 0, stream, static_cast<const float*>(dout), u, v, static_cast<const float*>(bias_u), static_cast<const float*>(bias_v), bias_axis, static_cast<const float*>(mask), mask_axis, static_cast<float*>(du), static_cast<float*>(dv), rows, cols),
+               hipLaunchKernelGGL(gate_bwd_kernel<uint16_t>, grid, dim3(256), 0, stream, static_cast<const uint16_t*>(dout), u, v, static_cast<const uint16_t*>(bias_u), static_cast<const uint16_t*>(bias_v), bias_axis, static_cast<const uint16_t*>(mask), mask_axis, static_cast<uint16_t*>(du), static_cast<uint16_t*>(dv), rows, cols),
+               hipLaunchKernelGGL(gate_bwd_kernel<f16bits>, grid, dim3(256), 0, stream, static_cast<const f16bits*>(dout), u, v, static_cast<const f16bits*>(bias_u), static_cast<const f16bits*>(bias_v), bias_axis, static_cast<const f16bits*>(mask), mask_axis, static_cast<f16bits*>(du), static_cast<f16bits*>(dv), rows, cols));
+  CUEQ_CHECK_HIP(hipGetLastError());
+  return CUEQ_OK;
+}
+
+// out[r] = sum_c in[r][c]   (float32 result)
 extern "C" int cueq_sum_cols(int32_t dtype, int64_t rows, int64_t cols, const void* in, float* out, void* stream_) {
   hipStream_t stream = static_cast<hipStream_t>(stream_);
   CUEQ_REQUIRE(is_io(dtype), CUEQ_ERR_UNSUPPORTED, "sum_cols: dtype must be float32 or bfloat16");

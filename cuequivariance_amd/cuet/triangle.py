@@ -163,6 +163,28 @@ def layer_norm_t_bwd(dy: torch.Tensor, xt: torch.Tensor, mean, rstd, gamma, need
     return dxt, dgamma, dbeta
 
 
+def gate_fwd(u, v, bias_u, bias_v, bias_axis: int, mask, mask_axis: int, dtype) -> torch.Tensor:
+    rows, cols = u.shape
+    out = torch.empty(rows, cols, dtype=dtype, device=u.device)
+    _lib.check(
+        _lib.load().cueq_gate_fwd(_CODE[dtype], rows, cols, u.data_ptr(), v.data_ptr(), _ptr(bias_u), _ptr(bias_v), bias_axis,
+                                  _ptr(mask), mask_axis, out.data_ptr(), _stream(u)),
+        "cueq_gate_fwd",
+    )
+    return out
+
+
+def gate_bwd(dout, u, v, bias_u, bias_v, bias_axis: int, mask, mask_axis: int):
+    rows, cols = u.shape
+    du, dv = torch.empty_like(dout), torch.empty_like(dout)
+    _lib.check(
+        _lib.load().cueq_gate_bwd(_CODE[dout.dtype], rows, cols, dout.data_ptr(), u.data_ptr(), v.data_ptr(), _ptr(bias_u),
+                                  _ptr(bias_v), bias_axis, _ptr(mask), mask_axis, du.data_ptr(), dv.data_ptr(), _stream(u)),
+        "cueq_gate_bwd",
+    )
+    return du, dv
+
+
 def _fusable(*tensors) -> bool:
     """The fused projection + gate kernel moves 16-byte vectors: row strides and addresses must allow it."""
     for t in tensors:
@@ -175,7 +197,7 @@ def _fusable(*tensors) -> bool:
 
 def dual_gate_fwd(A1, A2, B1, B2, bias1, bias2, bias_axis: int, mask, mask_axis: int) -> torch.Tensor:
     """``sigmoid(A1 B1^T + bias1) * (A2 B2^T + bias2) * mask`` (``B2 is None``: same as ``B1``); the two products stay
-    in registers."""
+    in registers when the operands allow the fused kernel, otherwise they go through float32 buffers."""
     M, K = A1.shape
     N = B1.shape[0]
     T = A1.dtype
@@ -188,7 +210,9 @@ def dual_gate_fwd(A1, A2, B1, B2, bias1, bias2, bias_axis: int, mask, mask_axis:
             "cueq_dual_gate",
         )
         return out
-    raise NotImplementedError("dual_gate_fwd: operands must be 16-byte aligned")
+    u = gemm_nt(A1, B1, torch.float32)
+    v = gemm_nt(A2, B1 if B2 is None else B2, torch.float32)
+    return gate_fwd(u, v, bias1, bias2, bias_axis, mask, mask_axis, T)
 
 
 def ln_dual_gate_fwd(x, gamma, beta, eps: float, W1, W2, bias1, bias2, mask):
@@ -212,6 +236,25 @@ def ln_dual_gate_fwd(x, gamma, beta, eps: float, W1, W2, bias1, bias2, mask):
         "cueq_ln_dual_gate",
     )
     return out, xh, mean, rstd
+
+
+def dual_gate_bwd(dout, A1, A2, B1, B2, bias1, bias2, bias_axis: int, mask, mask_axis: int):
+    """Gradients of the two products of :func:`dual_gate_fwd` (they are recomputed, not read back)."""
+    M, K = A1.shape
+    N = B1.shape[0]
+    T = A1.dtype
+    if _fusable(A1, A2, B1, B2, dout) and (K * A1.element_size()) % 16 == 0:
+        du, dv = torch.empty(M, N, dtype=T, device=A1.device), torch.empty(M, N, dtype=T, device=A1.device)
+        _lib.check(
+            _lib.load().cueq_dual_gate(_CODE[T], 1, M, N, K, A1.data_ptr(), A2.data_ptr(), A1.stride(0), B1.data_ptr(), _ptr(B2),
+                                       B1.stride(0), _ptr(bias1), _ptr(bias2), bias_axis, _ptr(mask), mask_axis, dout.data_ptr(),
+                                       du.data_ptr(), dv.data_ptr(), N, _stream(A1)),
+            "cueq_dual_gate",
+        )
+        return du, dv
+    u = gemm_nt(A1, B1, torch.float32)
+    v = gemm_nt(A2, B1 if B2 is None else B2, torch.float32)
+    return gate_bwd(dout, u, v, bias1, bias2, bias_axis, mask, mask_axis)
 
 
 def gate_bwd_input(dC, dc_by_row: bool, W1, W2, X1, X2, bias1, bias2, mask, dX1=None, want_gate_grads: bool = False):

@@ -439,6 +439,16 @@ int cueq_layer_norm_t_bwd(int32_t dtype, int64_t M, int64_t D, const void* dy, c
                           const void* gamma, void* dx_t, float* dgamma, float* dbeta, void* workspace, int64_t workspace_bytes,
                           void* stream);
 
+/* out = sigmoid(u + bias_u) * (v + bias_v) * mask on a rows x cols array (u, v float32 accumulators of the two
+ * projections); biases (may be NULL) are indexed by row (bias_axis 0) or column (1), the mask (may be NULL)
+ * likewise (_sigmoid_gated_dual_gemm.py:135-150).  cueq_gate_bwd returns the gradients of u and v
+ * (_sigmoid_gated_dual_gemm.py:153-218). */
+int cueq_gate_fwd(int32_t dtype, int64_t rows, int64_t cols, const float* u, const float* v, const void* bias_u,
+                  const void* bias_v, int32_t bias_axis, const void* mask, int32_t mask_axis, void* out, void* stream);
+int cueq_gate_bwd(int32_t dtype, int64_t rows, int64_t cols, const void* dout, const float* u, const float* v,
+                  const void* bias_u, const void* bias_v, int32_t bias_axis, const void* mask, int32_t mask_axis,
+                  void* du, void* dv, void* stream);
+
 /* Deterministic reductions of a rows x cols array into float32: over columns (one value per row) and over rows
  * (one value per column; workspace of cueq_sum_rows_workspace bytes).  Used for bias and affine gradients. */
 int cueq_sum_cols(int32_t dtype, int64_t rows, int64_t cols, const void* in, float* out, void* stream);
