@@ -350,8 +350,8 @@ _env_seen: dict = {}
 
 def sync_options_from_env() -> None:
     """The library reads CUEQ_DETERMINISTIC / CUEQ_FORCE_GENERIC once, when it is loaded; a process that changes them
-    afterwards (``os.environ[...] = "1"``) is followed here: called by the Python launch paths, two dictionary lookups
-    when nothing changed.  Only a *change* of a variable is pushed, so an option set with ``set_option`` stays as set
+    afterwards (``os.environ[...] = "1"``) is followed here, for programs that call the C entry points themselves (the modules'
+    launches follow it in the host module, ``csrc/host/module.cpp``).  Only a *change* of a variable is pushed, so an option set with ``set_option`` stays as set
     until the variable of the same name is assigned a different value."""
     lib = load()
     for env, name in _ENV_OPTIONS:

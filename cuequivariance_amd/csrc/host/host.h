@@ -37,7 +37,7 @@ inline void check(int status, const char* what) {
   if (status != CUEQ_OK) throw CueqError(std::string(what) + " failed (status " + std::to_string(status) + "): " + lib().cueq_last_error());
 }
 
-// follows CUEQ_DETERMINISTIC / CUEQ_FORCE_GENERIC of the process's environment (called with the GIL held)
+// follows CUEQ_DETERMINISTIC / CUEQ_FORCE_GENERIC of the process's environment, at every uniform-1d launch (called with the GIL held)
 void sync_options();
 
 inline int dtype_code(at::ScalarType t) {

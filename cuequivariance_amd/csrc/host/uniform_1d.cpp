@@ -115,6 +115,10 @@ RecordPtr make_record(const std::shared_ptr<Plan>& plan, std::vector<int> modes,
 
 variable_list launch(const Record& r, const at::Tensor* inputs, const at::Tensor* indices) {
   const Plan& p = *r.plan;
+  {
+    py::gil_scoped_acquire gil;  // (a backward runs without it, and the program may be assigning to the environment)
+    sync_options();
+  }
   const at::Device device(at::kCUDA, r.device);
   const c10::DeviceGuard guard(device);
   c10::SmallVector<cueq_u1d_buffer, 12> bufs(r.buffers.begin(), r.buffers.end());
@@ -312,7 +316,6 @@ struct Operator {
     for (const auto& i : out_index)
       if (!add_index(i)) return {};
     for (int64_t r : out_rows) key.v.push_back(r);
-    sync_options();
     auto hit = records.find(key);
     RecordPtr rec;
     if (hit != records.end()) {
@@ -402,10 +405,7 @@ void bind_uniform_1d(py::module_& m) {
         for (size_t i = 0; i < tensors.size(); ++i) (static_cast<int>(i) < plan->nin ? types : index_types).push_back(tensors[i].scalar_type());
         return make_record(plan, std::move(modes), std::move(index_of), std::move(rows), batch, types, index_types, tensors.at(0).device().index());
       }))
-      .def("run", [](const RecordPtr& r, const variable_list& tensors) {
-        sync_options();
-        return Uniform1d::run(r, tensors);
-      });
+      .def("run", [](const RecordPtr& r, const variable_list& tensors) { return Uniform1d::run(r, tensors); });
   py::class_<Operator, std::shared_ptr<Operator>>(m, "U1dOperator")
       .def(py::init([](std::shared_ptr<Plan> plan32, std::shared_ptr<Plan> plan64, int fixed) {
         auto o = std::make_shared<Operator>();
