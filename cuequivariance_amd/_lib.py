@@ -89,6 +89,7 @@ EXPORTED_SYMBOLS = (
     "cueq_trimul_workspace_bytes",
     "cueq_trimul_fwd",
     "cueq_trimul_bwd",
+    "cueq_trimul_bwd_parts",
 )
 
 
@@ -313,7 +314,9 @@ def load() -> C.CDLL:
         lib.cueq_trimul_fwd.argtypes = [i32, i64, i64, i64, i64, i32, C.c_double, ptr, ptr, ptr, ptr, ptr, ptr, i64, ptr]
         lib.cueq_trimul_fwd.restype = C.c_int
         lib.cueq_trimul_bwd.argtypes = [i32, i64, i64, i64, i64, i32, ptr, ptr, ptr, ptr, ptr, ptr, C.c_uint32, ptr, ptr, i64, ptr]
+        lib.cueq_trimul_bwd_parts.argtypes = [i32, i64, i64, i64, i64, i32, ptr, ptr, ptr, ptr, ptr, ptr, C.c_uint32, ptr, ptr, i64, ptr]
         lib.cueq_trimul_bwd.restype = C.c_int
+        lib.cueq_trimul_bwd_parts.restype = C.c_int
         # the library has read the environment itself at this point: remember what it saw, so that the first launch does
         # not push those values again over an option set by cueq_set_option in the meantime
         for env, _ in _ENV_OPTIONS:

@@ -16,8 +16,8 @@ namespace cueq_host {
 
 #define CUEQ_HOST_ENTRIES(X)                                                                                                     \
   X(cueq_last_error) X(cueq_set_option) X(cueq_u1d_plan_destroy) X(cueq_u1d_workspace_size) X(cueq_u1d_run)                      \
-  X(cueq_segment_csr_workspace) X(cueq_segment_csr_build) X(cueq_segment_csr_build_async) X(cueq_trimul_grads_values)             \
-  X(cueq_trimul_saved_bytes) X(cueq_trimul_workspace_bytes) X(cueq_trimul_fwd) X(cueq_trimul_bwd)                      \
+  X(cueq_segment_csr_workspace) X(cueq_segment_csr_build) X(cueq_segment_csr_build_async) X(cueq_trimul_bwd_parts)                \
+  X(cueq_trimul_saved_bytes) X(cueq_trimul_workspace_bytes) X(cueq_trimul_fwd)                                         \
   X(cueq_linear_flex) X(cueq_linear_flex_dw_chunks) X(cueq_linear_flex_dw) X(cueq_sum_runs) X(cueq_linear_rows) X(cueq_linear_rows_mul_ir) \
   X(cueq_linear_dw_mul_ir_items) X(cueq_linear_dw_mul_ir) X(cueq_gemm_tn_items) X(cueq_gemm_tn) X(cueq_gemm_table) \
   X(cueq_fc_flex) X(cueq_fc_flex_dw_chunks) X(cueq_fc_flex_dw) X(cueq_fc_factors) X(cueq_fc_pack)

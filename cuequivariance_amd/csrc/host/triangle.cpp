@@ -59,31 +59,24 @@ variable_list trimul_bwd(const at::Tensor& x_, const at::Tensor& mask, at::Tenso
   uint32_t bits = need >> 1;
   for (int i = 0; i < kWeights; ++i)
     if (!weights[i].defined()) bits &= ~(1u << i);
-  at::Tensor dx = new_tensor(x.sizes(), x.scalar_type(), c.device), grads;
-  if (bits) grads = new_tensor({lib().cueq_trimul_grads_values(c.D, c.Do)}, x.scalar_type(), c.device);
-  if (x.numel() == 0) {
-    if (grads.defined()) grads.zero_();
-  } else {
+  at::Tensor dx = new_tensor(x.sizes(), x.scalar_type(), c.device);
+  variable_list out(1 + kWeights);
+  void* grads[kWeights] = {};
+  for (int i = 0; i < kWeights; ++i) {
+    if (!(bits >> i & 1)) continue;
+    out[1 + i] = new_tensor(weights[i].sizes(), x.scalar_type(), c.device);
+    grads[i] = out[1 + i].data_ptr();
+    if (x.numel() == 0) out[1 + i].zero_();
+  }
+  if (x.numel() != 0) {
     const at::Tensor dout = aligned(dout_.to(x.scalar_type()).contiguous());
     const int64_t bytes = lib().cueq_trimul_workspace_bytes(c.code, c.B, c.N, c.D, c.Do, 1, bits != 0);
     at::Tensor ws = new_tensor({bytes}, at::kByte, c.device);
-    check(lib().cueq_trimul_bwd(c.code, c.B, c.N, c.D, c.Do, outgoing, x.data_ptr(), pointer(mask), c.w, saved.data_ptr(), dout.data_ptr(), dx.data_ptr(), bits,
-                                pointer(grads), ws.data_ptr(), bytes, stream_of(c.device.index())),
-          "cueq_trimul_bwd");
+    check(lib().cueq_trimul_bwd_parts(c.code, c.B, c.N, c.D, c.Do, outgoing, x.data_ptr(), pointer(mask), c.w, saved.data_ptr(), dout.data_ptr(), dx.data_ptr(),
+                                      bits, grads, ws.data_ptr(), bytes, stream_of(c.device.index())),
+          "cueq_trimul_bwd_parts");
   }
-  variable_list out(1 + kWeights);
   if (need & 1) out[0] = dx;
-  if (grads.defined()) {  // the order of the gradients in the buffer: norms, projections (gate, value), biases
-    static const int order[kWeights] = {0, 1, 6, 7, 4, 2, 10, 8, 5, 3, 11, 9};
-    const int64_t D = c.D, Do = c.Do;
-    const int64_t sizes[kWeights] = {D, D, D, D, 2 * D * D, 2 * D * D, Do * D, Do * D, 2 * D, 2 * D, Do, Do};
-    int64_t at = 0;
-    for (int k = 0; k < kWeights; ++k) {
-      const int i = order[k];
-      if (bits >> i & 1) out[1 + i] = grads.narrow(0, at, sizes[k]).view(weights[i].sizes());
-      at += sizes[k];
-    }
-  }
   return out;
 }
 

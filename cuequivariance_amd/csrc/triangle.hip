@@ -2559,10 +2559,21 @@ __global__ void __launch_bounds__(256) pair_rows_kernel(const V* __restrict__ in
   }
 }
 
+// consecutive runs of float32 values, each rounded into a tensor of its own (null: not wanted)
+struct ValueRuns {
+  static constexpr int kMax = 12;
+  void* out[kMax];
+  int64_t first[kMax + 1];
+};
 template <typename TO>
-__global__ void __launch_bounds__(256) round_values_kernel(const float* __restrict__ in, TO* __restrict__ out, int64_t n) {
+__global__ void __launch_bounds__(256) round_runs_kernel(const float* __restrict__ in, ValueRuns runs) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (i < n) tri_store(out, i, in[i]);
+  if (i >= runs.first[ValueRuns::kMax]) return;
+  int r = 0;
+#pragma unroll
+  for (int k = 1; k < ValueRuns::kMax; ++k) r += i >= runs.first[k] ? 1 : 0;
+  TO* out = static_cast<TO*>(runs.out[r]);
+  if (out) tri_store(out, i - runs.first[r], in[i]);
 }
 
 static bool is_io(int dt) { return dt == CUEQ_F32 || dt == CUEQ_BF16 || dt == CUEQ_F16; }
@@ -3535,6 +3546,19 @@ int pair_copy(const TriPlan& p, const void* in, void* out, int64_t width, PairCo
 
 #define TRI_STEP(expr) do { const int rc_ = (expr); if (rc_ != CUEQ_OK) return rc_; } while (0)
 
+// the gradients in the order in which they are formed: norms, input projections (gate, then value), output projections, biases
+constexpr int kGradOrder[ValueRuns::kMax] = {kNinW, kNinB, kNoutW, kNoutB, kGinW, kPinW, kGoutW, kPoutW, kGinB, kPinB, kGoutB, kPoutB};
+ValueRuns tri_gradients(int64_t D, int64_t Do, uint32_t need, void* const* grads) {
+  const int64_t size[ValueRuns::kMax] = {D, D, D, D, 2 * D * D, 2 * D * D, Do * D, Do * D, 2 * D, 2 * D, Do, Do};
+  ValueRuns r;
+  r.first[0] = 0;
+  for (int k = 0; k < ValueRuns::kMax; ++k) {
+    r.out[k] = (need >> kGradOrder[k] & 1u) && grads ? grads[kGradOrder[k]] : nullptr;
+    r.first[k + 1] = r.first[k] + size[k];
+  }
+  return r;
+}
+
 int tri_check(const TriPlan& p) {
   CUEQ_REQUIRE(is_io(p.dt), CUEQ_ERR_UNSUPPORTED, "trimul: dtype must be float32, bfloat16 or half");
   CUEQ_REQUIRE(p.B >= 0 && p.N >= 0 && p.D > 0 && p.D % 32 == 0 && p.Do > 0, CUEQ_ERR_INVALID, "trimul: bad extents");
@@ -3602,12 +3626,23 @@ extern "C" int cueq_trimul_fwd(int32_t dtype, int64_t B, int64_t N, int64_t D, i
 extern "C" int cueq_trimul_bwd(int32_t dtype, int64_t B, int64_t N, int64_t D, int64_t Do, int32_t outgoing, const void* x, const void* mask,
                                const void* const* w, void* saved, const void* dout, void* dx, uint32_t need, void* grads, void* workspace,
                                int64_t workspace_bytes, void* stream_) {
+  void* parts[kWeights] = {};
+  const ValueRuns r = tri_gradients(D, Do, 0, nullptr);
+  for (int k = 0; k < kWeights; ++k)
+    if (grads) parts[kGradOrder[k]] = static_cast<char*>(grads) + r.first[k] * (dtype == CUEQ_F32 ? 4 : 2);
+  return cueq_trimul_bwd_parts(dtype, B, N, D, Do, outgoing, x, mask, w, saved, dout, dx, need, grads ? parts : nullptr, workspace, workspace_bytes, stream_);
+}
+
+extern "C" int cueq_trimul_bwd_parts(int32_t dtype, int64_t B, int64_t N, int64_t D, int64_t Do, int32_t outgoing, const void* x, const void* mask,
+                                     const void* const* w, void* saved, const void* dout, void* dx, uint32_t need, void* const* grads, void* workspace,
+                                     int64_t workspace_bytes, void* stream_) {
   hipStream_t stream = static_cast<hipStream_t>(stream_);
   const TriPlan p(dtype, B, N, D, Do, outgoing != 0);
   TRI_STEP(tri_check(p));
   const int64_t nv = cueq_trimul_grads_values(D, Do);
   if (p.M == 0) return CUEQ_OK;  // (the caller returns zeros)
   CUEQ_REQUIRE(x && w && saved && dout && dx && (grads || !need), CUEQ_ERR_INVALID, "trimul: null operand");
+  for (int i = 0; i < kWeights; ++i) CUEQ_REQUIRE(!(need >> i & 1u) || grads[i], CUEQ_ERR_INVALID, "trimul: null gradient");
   const TriSaved s(p, saved);
   const TriBwdWork k(p, need != 0, workspace);
   CUEQ_REQUIRE(workspace && workspace_bytes >= k.bytes, CUEQ_ERR_INVALID, "trimul: workspace too small");
@@ -3615,8 +3650,7 @@ extern "C" int cueq_trimul_bwd(int32_t dtype, int64_t B, int64_t N, int64_t D, i
   auto wants = [&](int i) { return (need >> i & 1u) != 0; };
   const bool w_out = wants(kPoutW) || wants(kPoutB) || wants(kGoutW) || wants(kGoutB);
   const bool w_in = wants(kPinW) || wants(kPinB) || wants(kGinW) || wants(kGinB);
-  // the float32 gradients: norms, the input projections (gate, then value), the output projections, the biases
-  float* gf = dtype == CUEQ_F32 ? static_cast<float*>(grads) : k.grads;
+  float* gf = k.grads;  // (float32, in the order of tri_gradients)
   float *g_nin = gf, *g_nout = gf + 2 * D, *g_in = gf + 4 * D, *g_out = g_in + 4 * D * D, *g_in_b = g_out + 2 * Do * D, *g_out_b = g_in_b + 4 * D;
   if (p.copies) {
     TRI_STEP(pair_copy(p, dout, k.doutp, Do, kPairZero, stream));
@@ -3704,10 +3738,12 @@ extern "C" int cueq_trimul_bwd(int32_t dtype, int64_t B, int64_t N, int64_t D, i
                                  k.ln, k.ln_bytes, stream_, pairs));
     if (p.copies) TRI_STEP(pair_copy(p, dxt, dx, D, kPairBack, stream));
   }
-  if (need && dtype != CUEQ_F32) {
+  if (need) {
     const dim3 grid(static_cast<unsigned>((nv + 255) / 256));
-    if (dtype == CUEQ_F16) hipLaunchKernelGGL(round_values_kernel<f16bits>, grid, dim3(256), 0, stream, gf, static_cast<f16bits*>(grads), nv);
-    else hipLaunchKernelGGL(round_values_kernel<uint16_t>, grid, dim3(256), 0, stream, gf, static_cast<uint16_t*>(grads), nv);
+    const ValueRuns runs = tri_gradients(D, Do, need, grads);
+    TRI_DISPATCH(dtype, hipLaunchKernelGGL(round_runs_kernel<float>, grid, dim3(256), 0, stream, gf, runs),
+                 hipLaunchKernelGGL(round_runs_kernel<uint16_t>, grid, dim3(256), 0, stream, gf, runs),
+                 hipLaunchKernelGGL(round_runs_kernel<f16bits>, grid, dim3(256), 0, stream, gf, runs));
     CUEQ_CHECK_HIP(hipGetLastError());
   }
   return CUEQ_OK;

@@ -364,7 +364,7 @@ def _trimul_bwd_op(dout: torch.Tensor, x: torch.Tensor, tensors: List[torch.Tens
     bits = sum(1 << i for i, n in enumerate([need[0], *need[2:14]]) if n)
     dx, *grads = _lib.host().trimul_bwd(x, args[0], args[1:], saved, outgoing, bits, dout)
     grads = [dx, None, *grads]
-    return [x.new_empty(0) if (g is None or not n) else g.clone() if k > 0 else g for k, (g, n) in enumerate(zip(grads, need))]
+    return [x.new_empty(0) if (g is None or not n) else g for g, n in zip(grads, need)]
 
 
 @_trimul_bwd_op.register_fake

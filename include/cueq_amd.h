@@ -518,6 +518,10 @@ int cueq_trimul_fwd(int32_t dtype, int64_t B, int64_t N, int64_t D, int64_t Do, 
 int cueq_trimul_bwd(int32_t dtype, int64_t B, int64_t N, int64_t D, int64_t Do, int32_t outgoing, const void* x, const void* mask,
                     const void* const* weights, void* saved, const void* dout, void* dx, uint32_t need, void* grads, void* workspace,
                     int64_t workspace_bytes, void* stream);
+/* The same with every gradient in a tensor of its own: `grads` is a host array of 12 device pointers in the order of `weights`. */
+int cueq_trimul_bwd_parts(int32_t dtype, int64_t B, int64_t N, int64_t D, int64_t Do, int32_t outgoing, const void* x, const void* mask,
+                          const void* const* weights, void* saved, const void* dout, void* dx, uint32_t need, void* const* grads,
+                          void* workspace, int64_t workspace_bytes, void* stream);
 
 #ifdef __cplusplus
 }
