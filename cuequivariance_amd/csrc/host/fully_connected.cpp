@@ -80,6 +80,11 @@ struct FcOp {
     }
     return it->second;
   }
+  // (as LinearOp::tables_at_hand: the generated kernels have no tables)
+  bool tables_at_hand(at::Device device) {
+    std::lock_guard<std::mutex> lock(mutex);
+    return devices.count(device.index()) || !capturing();
+  }
   bool takes(at::ScalarType t) const { return (t == at::kFloat && (epv_ok & 1)) || ((t == at::kBFloat16 || t == at::kHalf) && (epv_ok & 2)); }
 };
 using OpPtr = std::shared_ptr<FcOp>;
@@ -110,7 +115,7 @@ at::Tensor product(FcOp& op, const at::Tensor& w_, const at::Tensor& x1_, const 
   const auto options = at::TensorOptions().dtype(dtype).device(device);
   const int code = dtype_code(dtype);
   const std::optional<Unit> unit = op.units.find(code);
-  const Unit* u = unit && Z >= unit->fwd_from ? &*unit : nullptr;
+  const Unit* u = unit && (Z >= unit->fwd_from || !op.tables_at_hand(device)) ? &*unit : nullptr;
   at::Tensor out = op.covers_out || u ? at::empty({Z, op.width_out}, options) : at::zeros({Z, op.width_out}, options);
   if (Z == 0) return out;
   hipStream_t stream = stream_of(device.index());
@@ -152,7 +157,7 @@ Grads gradients(FcOp& op, const at::Tensor& w_, const at::Tensor& x1_, const at:
   hipStream_t stream = stream_of(device.index());
   const std::optional<Unit> unit = op.units.find(code);
   if (need_1 || need_2) {
-    const Unit* u = unit && Z >= unit->dx_from ? &*unit : nullptr;
+    const Unit* u = unit && (Z >= unit->dx_from || !op.tables_at_hand(device)) ? &*unit : nullptr;
     // (without x2 - the gradient of x2 alone does not use it - any values do: what they scale is not asked for)
     const at::Tensor second = x2.defined() ? x2 : at::zeros({Z, op.n2}, options);
     if (need_1) r.x1 = op.covers_in || u ? at::empty({Z, op.width1}, options) : at::zeros({Z, op.width1}, options);
@@ -188,7 +193,7 @@ Grads gradients(FcOp& op, const at::Tensor& w_, const at::Tensor& x1_, const at:
   }
   if (need_w) {
     const at::ScalarType out_dtype = w_dtype == at::kDouble ? at::kFloat : w_dtype;
-    const Unit* u = unit && Z >= unit->dw_from ? &*unit : nullptr;
+    const Unit* u = unit && (Z >= unit->dw_from || !op.tables_at_hand(device)) ? &*unit : nullptr;
     // The factors H_i = sum_k s_ik g_k are operands of a product, rounded to its type.  In half they leave its range long before the
     // gradient does (65 504: a scaled loss), and bfloat16 calls that were float32 throughout would lose a rounding's worth: both
     // contract float copies of their rows.  (Generated kernels: a product's own, in its own type.)

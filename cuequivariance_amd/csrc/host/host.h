@@ -67,6 +67,8 @@ bool unwatched();
 
 bool wants_graph(const std::vector<at::Tensor>& tensors);  // gradients are recorded and some tensor asks for one
 
+inline bool capturing() { return c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None; }  // a HIP graph
+
 // (offsets[nrows + 1], perm[n]) grouping batch ids by output row; cached per index tensor in eager mode
 std::pair<at::Tensor, at::Tensor> segment_csr(const at::Tensor& index, int64_t nrows);
 

@@ -58,6 +58,12 @@ struct LinearOp {
     }
     return it->second;
   }
+  // Whether the device tables are there or may be uploaded now: a first call that is captured into a HIP graph runs on the launches whose
+  // tables travel as arguments, where there are such, whatever the number of rows.
+  bool tables_at_hand(at::Device device) {
+    std::lock_guard<std::mutex> lock(mutex);
+    return devices.count(device.index()) || !capturing();
+  }
   bool takes(at::ScalarType t) const { return (t == at::kFloat && (epv_ok & 1)) || ((t == at::kBFloat16 || t == at::kHalf) && (epv_ok & 2)); }
 };
 using OpPtr = std::shared_ptr<LinearOp>;
@@ -79,7 +85,7 @@ at::Tensor apply_rows(LinearOp& op, const at::Tensor& w_, const at::Tensor& x_, 
   const int e = dtype == at::kFloat ? 0 : 1, code = dtype_code(dtype);
   const auto& launches = forward ? op.fwd_rows[e] : op.dx_rows[e];
   hipStream_t stream = stream_of(device.index());
-  if (!launches.empty() && Z >= op.rows_from[e]) {
+  if (!launches.empty() && (Z >= op.rows_from[e] || !op.tables_at_hand(device))) {
     for (size_t i = 0; i < launches.size(); ++i) {
       const RowsLaunch& l = launches[i];
       if (l.d == 0)  // result columns n, contraction k; the weight block is contraction-major in the forward
@@ -117,7 +123,7 @@ at::Tensor weight_gradient(LinearOp& op, const at::Tensor& x_, const at::Tensor&
   const int e = dtype == at::kFloat ? 0 : 1, code = dtype_code(dtype), out_code = dtype_code(out_dtype);
   const int64_t es = dtype == at::kFloat ? 4 : 2;
   hipStream_t stream = stream_of(device.index());
-  if (!op.grad_rows[e].empty() && Z >= op.grad_rows_from[e]) {
+  if (!op.grad_rows[e].empty() && (Z >= op.grad_rows_from[e] || !op.tables_at_hand(device))) {
     for (const auto& l : op.grad_rows[e]) {
       const int n = static_cast<int>(l.w_off.size());
       std::vector<int32_t> first(n + 1, 0);

@@ -79,8 +79,7 @@ bool wants_graph(const std::vector<at::Tensor>& tensors) {
 // instead (device-side work only, nothing cached), so every replay regroups from whatever the index buffer holds then.  Index
 // tensors made under torch.inference_mode() carry no version counter and are not cached either.
 std::pair<at::Tensor, at::Tensor> segment_csr(const at::Tensor& index, int64_t nrows) {
-  const bool capturing = c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None;
-  const bool cacheable = !capturing && !index.is_inference();
+  const bool recorded = capturing(), cacheable = !recorded && !index.is_inference();
   const int64_t n = index.numel();
   if (cacheable) {
     std::lock_guard<std::mutex> lock(g_csr_mutex);
@@ -98,7 +97,7 @@ std::pair<at::Tensor, at::Tensor> segment_csr(const at::Tensor& index, int64_t n
   at::Tensor ws = new_tensor({bytes}, at::kByte, index.device());
   std::optional<pybind11::gil_scoped_release> release;  // (the build waits for two flags)
   if (PyGILState_Check()) release.emplace();
-  const auto build = capturing ? lib().cueq_segment_csr_build_async : lib().cueq_segment_csr_build;
+  const auto build = recorded ? lib().cueq_segment_csr_build_async : lib().cueq_segment_csr_build;
   check(build(index.data_ptr(), index.scalar_type() == at::kLong ? 1 : 0, n, nrows, offsets.data_ptr<int64_t>(), perm.data_ptr<int64_t>(), ws.data_ptr(), bytes,
               stream_of(index.device().index())),
         "cueq_segment_csr_build");
