@@ -1,11 +1,8 @@
 // Fully connected product with shared weights: the family of functions product / gradient of
 // x1 / of x2 / of the weights, each differentiable in terms of the others, on csrc/fc_flex.hip and - from the measured crossings on -
 // the kernels generated for the descriptor (codegen/fullyconnected.py).
-#include "host.h"
 #include "shared_map.h"
-
-#include <mutex>
-#include <unordered_map>
+#include "tables.h"
 
 namespace cueq_host {
 namespace py = pybind11;
@@ -29,13 +26,15 @@ constexpr int64_t kChunks = 64;  // row chunks of the weight gradient's tiled pr
 struct GradShape {  // the weight blocks of one extent: parts (path, component) of the tiled products, components per block
   int K, N, parts = 0;
   std::vector<int64_t> table, w0;
+  int on_device = -1;
   std::vector<int32_t> first{0};
 };
 
 // 2-byte rows where the second operand has several channels: weights packed for each direction (cueq_fc_pack), weight gradient by
 // groups of four channels
 struct Packed {
-  std::string fwd_blocks, fwd_parts, dx_blocks, dx_parts, fwd_packs, dx_packs, grads;
+  enum { kBlocks, kParts, kPacks, kCoef, kGrads };
+  DeviceTables fwd, back;  // in this order (kGrads: back)
   int fwd_longest = 0, dx_longest = 0, grad_tiles = 0;  // grad_tiles == 0: the weight gradient takes the tables of the other types
   int64_t fwd_pieces = 0, dx_pieces = 0;
   bool any() const { return fwd_longest > 0; }
@@ -45,7 +44,9 @@ struct FcOp {
   int64_t width1 = 0, n2 = 0, width_out = 0, numel = 0;
   bool mul_ir = false, covers_in = true, covers_out = true;
   int epv_ok = 0, most = 1;
-  std::string fwd_blocks, fwd_parts, dx_blocks, dx_parts, grads, coef;
+  enum { kBlocks, kParts, kCoef, kGrads };
+  DeviceTables fwd, back;  // in this order (kGrads and the tiled products': back)
+  std::string coef;
   int fwd_tiles = 0, dx_tiles = 0, grad_tiles = 0;
   SharedMap<Unit> units;  // by element type code
   std::vector<GradShape> shapes;
@@ -55,55 +56,22 @@ struct FcOp {
   int64_t tiled_dw_from[2] = {1 << 30, 1 << 30};  // rows, by element size (4, 2)
   bool float_factors = false;  // bfloat16 rows: the weight gradient's factors H stay float32 (half rows: always)
 
-  std::mutex mutex;
-  struct OnDevice {
-    at::Tensor fwd_blocks, fwd_parts, dx_blocks, dx_parts, grads, coef;
-    std::vector<at::Tensor> tables;
-    at::Tensor packed_fwd_blocks, packed_fwd_parts, packed_dx_blocks, packed_dx_parts, fwd_packs, dx_packs, packed_grads;
-  };
-  std::unordered_map<int, OnDevice> devices;
-  const OnDevice& on(at::Device device) {
-    std::lock_guard<std::mutex> lock(mutex);
-    auto it = devices.find(device.index());
-    if (it == devices.end()) {
-      auto up = [&](const std::string& s) {
-        return at::from_blob(const_cast<char*>(s.data()), {static_cast<int64_t>(s.size())}, at::TensorOptions().dtype(at::kByte)).clone().to(device);
-      };
-      it = devices.emplace(device.index(), OnDevice{up(fwd_blocks), up(fwd_parts), up(dx_blocks), up(dx_parts), up(grads), up(coef), {}, {}, {}, {}, {}, {}, {}, {}}).first;
-      if (packed.any()) {
-        auto& d = it->second;
-        d.packed_fwd_blocks = up(packed.fwd_blocks), d.packed_dx_blocks = up(packed.dx_blocks);
-        d.packed_fwd_parts = up(packed.fwd_parts), d.packed_dx_parts = up(packed.dx_parts);
-        d.fwd_packs = up(packed.fwd_packs), d.dx_packs = up(packed.dx_packs), d.packed_grads = up(packed.grads);
-      }
-      for (const auto& q : shapes) it->second.tables.push_back(at::tensor(q.table, at::kLong).to(device));
-    }
-    return it->second;
-  }
-  // (as LinearOp::tables_at_hand: the generated kernels have no tables)
-  bool tables_at_hand(at::Device device) {
-    std::lock_guard<std::mutex> lock(mutex);
-    return devices.count(device.index()) || !capturing();
-  }
   bool takes(at::ScalarType t) const { return (t == at::kFloat && (epv_ok & 1)) || ((t == at::kBFloat16 || t == at::kHalf) && (epv_ok & 2)); }
 };
 using OpPtr = std::shared_ptr<FcOp>;
 
-at::Tensor rows_of(const at::Tensor& t, at::ScalarType dtype) {
-  at::Tensor r = t.to(dtype).contiguous();
-  return reinterpret_cast<uintptr_t>(r.data_ptr()) % 16 ? r.clone() : r;
-}
 void launched(int status, const char* what) {
   if (status != 0) throw CueqError(std::string(what) + ": launch failed");
 }
 
 // the weights as the rows kernels read them: as they are, or packed
-at::Tensor weights_for(FcOp& op, const FcOp::OnDevice& t, const at::Tensor& w, bool packed, bool gradient, int code, hipStream_t stream) {
+at::Tensor weights_for(FcOp& op, const at::Tensor& w, bool packed, bool gradient, int code, hipStream_t stream) {
   if (!packed) return w;
-  const at::Tensor& packs = gradient ? t.dx_packs : t.fwd_packs;
+  DeviceTables& tables = gradient ? op.packed.back : op.packed.fwd;
   const int64_t pieces = gradient ? op.packed.dx_pieces : op.packed.fwd_pieces;
   at::Tensor out = at::empty({pieces * 8}, w.options());
-  check(lib().cueq_fc_pack(code, w.data_ptr(), out.data_ptr(), packs.data_ptr(), static_cast<int>(packs.numel() / 48), pieces, stream), "cueq_fc_pack");
+  check(lib().cueq_fc_pack(code, w.data_ptr(), out.data_ptr(), tables.on(w.device(), Packed::kPacks), tables.count(Packed::kPacks, 48), pieces, stream),
+        "cueq_fc_pack");
   return out;
 }
 
@@ -115,7 +83,8 @@ at::Tensor product(FcOp& op, const at::Tensor& w_, const at::Tensor& x1_, const 
   const auto options = at::TensorOptions().dtype(dtype).device(device);
   const int code = dtype_code(dtype);
   const std::optional<Unit> unit = op.units.find(code);
-  const Unit* u = unit && (Z >= unit->fwd_from || !op.tables_at_hand(device)) ? &*unit : nullptr;
+  // (a first call that is captured into a HIP graph: the generated kernels have no tables to upload)
+  const Unit* u = unit && (Z >= unit->fwd_from || !op.fwd.at_hand(device)) ? &*unit : nullptr;
   at::Tensor out = op.covers_out || u ? at::empty({Z, op.width_out}, options) : at::zeros({Z, op.width_out}, options);
   if (Z == 0) return out;
   hipStream_t stream = stream_of(device.index());
@@ -123,12 +92,12 @@ at::Tensor product(FcOp& op, const at::Tensor& w_, const at::Tensor& x1_, const 
     launched(u->fwd(Z, w.data_ptr(), x1.data_ptr(), op.width1, x2.data_ptr(), op.n2, out.data_ptr(), op.width_out, stream), "fully connected product");
     return out;
   }
-  const auto& t = op.on(device);
   const bool packed = op.packed.any() && dtype != at::kFloat;
-  const at::Tensor ww = weights_for(op, t, w, packed, false, code, stream);
+  const at::Tensor ww = weights_for(op, w, packed, false, code, stream);
+  DeviceTables& t = packed ? op.packed.fwd : op.fwd;
   check(lib().cueq_fc_flex(code, 0, op.mul_ir, packed ? op.packed.fwd_longest : 0, Z, x1.data_ptr(), op.width1, ww.data_ptr(), x2.data_ptr(), op.n2, nullptr, 0, out.data_ptr(), op.width_out,
-                           (packed ? t.packed_fwd_blocks : t.fwd_blocks).data_ptr(), static_cast<int>(t.fwd_blocks.numel() / 24), (packed ? t.packed_fwd_parts : t.fwd_parts).data_ptr(),
-                           static_cast<const float*>(t.coef.data_ptr()), op.fwd_tiles, op.most, static_cast<int>(op.n2), nullptr, nullptr, stream),
+                           t.on(device, FcOp::kBlocks), t.count(FcOp::kBlocks, 24), t.on(device, FcOp::kParts), t.on<float>(device, packed ? int(Packed::kCoef) : int(FcOp::kCoef)),
+                           op.fwd_tiles, op.most, static_cast<int>(op.n2), nullptr, nullptr, stream),
         "cueq_fc_flex");
   return out;
 }
@@ -157,7 +126,7 @@ Grads gradients(FcOp& op, const at::Tensor& w_, const at::Tensor& x1_, const at:
   hipStream_t stream = stream_of(device.index());
   const std::optional<Unit> unit = op.units.find(code);
   if (need_1 || need_2) {
-    const Unit* u = unit && (Z >= unit->dx_from || !op.tables_at_hand(device)) ? &*unit : nullptr;
+    const Unit* u = unit && (Z >= unit->dx_from || !op.back.at_hand(device)) ? &*unit : nullptr;
     // (without x2 - the gradient of x2 alone does not use it - any values do: what they scale is not asked for)
     const at::Tensor second = x2.defined() ? x2 : at::zeros({Z, op.n2}, options);
     if (need_1) r.x1 = op.covers_in || u ? at::empty({Z, op.width1}, options) : at::zeros({Z, op.width1}, options);
@@ -178,22 +147,22 @@ Grads gradients(FcOp& op, const at::Tensor& w_, const at::Tensor& x1_, const at:
                    "fully connected gradient");
       }
     } else {
-      const auto& t = op.on(device);
       at::Tensor part, dx1 = r.x1;
       if (need_2) part = new_tensor({op.dx_tiles, Z, op.n2}, at::kFloat, device);
       if (!dx1.defined()) dx1 = at::empty({Z, op.width1}, options);  // (the gradient of x2 comes from the same products)
       const bool packed = op.packed.any() && dtype != at::kFloat;
-      const at::Tensor ww = weights_for(op, t, w, packed, true, code, stream);
+      const at::Tensor ww = weights_for(op, w, packed, true, code, stream);
+      DeviceTables& t = packed ? op.packed.back : op.back;
       check(lib().cueq_fc_flex(code, 1, op.mul_ir, packed ? op.packed.dx_longest : 0, Z, g.data_ptr(), op.width_out, ww.data_ptr(), second.data_ptr(), op.n2, need_2 ? x1.data_ptr() : nullptr,
-                               need_2 ? op.width1 : 0, dx1.data_ptr(), op.width1, (packed ? t.packed_dx_blocks : t.dx_blocks).data_ptr(), static_cast<int>(t.dx_blocks.numel() / 24),
-                               (packed ? t.packed_dx_parts : t.dx_parts).data_ptr(), static_cast<const float*>(t.coef.data_ptr()), op.dx_tiles, op.most, static_cast<int>(op.n2),
+                               need_2 ? op.width1 : 0, dx1.data_ptr(), op.width1, t.on(device, FcOp::kBlocks), t.count(FcOp::kBlocks, 24),
+                               t.on(device, FcOp::kParts), t.on<float>(device, packed ? int(Packed::kCoef) : int(FcOp::kCoef)), op.dx_tiles, op.most, static_cast<int>(op.n2),
                                need_2 ? part.data_ptr<float>() : nullptr, need_2 ? r.x2.data_ptr() : nullptr, stream),
             "cueq_fc_flex");
     }
   }
   if (need_w) {
     const at::ScalarType out_dtype = w_dtype == at::kDouble ? at::kFloat : w_dtype;
-    const Unit* u = unit && (Z >= unit->dw_from || !op.tables_at_hand(device)) ? &*unit : nullptr;
+    const Unit* u = unit && (Z >= unit->dw_from || !op.back.at_hand(device)) ? &*unit : nullptr;
     // The factors H_i = sum_k s_ik g_k are operands of a product, rounded to its type.  In half they leave its range long before the
     // gradient does (65 504: a scaled loss), and bfloat16 calls that were float32 throughout would lose a rounding's worth: both
     // contract float copies of their rows.  (Generated kernels: a product's own, in its own type.)
@@ -202,18 +171,17 @@ Grads gradients(FcOp& op, const at::Tensor& w_, const at::Tensor& x1_, const at:
     const int dw_code = dtype_code(dw_dtype);
     at::Tensor gw = new_tensor(w_sizes, out_dtype, device);
     if (!u && Z >= op.tiled_dw_from[dw_dtype == at::kFloat ? 0 : 1]) {
-      const auto& t = op.on(device);
+      DeviceTables& t = op.back;
       at::Tensor H = at::empty({Z, op.h_width}, ag.options()), x1t = op.mul_ir ? at::empty({Z, op.width1}, ag.options()) : a1;
-      check(lib().cueq_fc_factors(dw_code, op.mul_ir, Z, a1.data_ptr(), op.width1, a2.data_ptr(), op.n2, ag.data_ptr(), op.width_out, t.grads.data_ptr(),
-                                  static_cast<int>(t.grads.numel() / 72), static_cast<const float*>(t.coef.data_ptr()), t.dx_blocks.data_ptr(),
-                                  static_cast<int>(t.dx_blocks.numel() / 24), op.factors, H.data_ptr(), op.h_width, op.mul_ir ? x1t.data_ptr() : nullptr, stream),
+      check(lib().cueq_fc_factors(dw_code, op.mul_ir, Z, a1.data_ptr(), op.width1, a2.data_ptr(), op.n2, ag.data_ptr(), op.width_out, t.on(device, FcOp::kGrads),
+                                  t.count(FcOp::kGrads, 72), t.on<float>(device, FcOp::kCoef), t.on(device, FcOp::kBlocks), t.count(FcOp::kBlocks, 24), op.factors, H.data_ptr(), op.h_width, op.mul_ir ? x1t.data_ptr() : nullptr, stream),
             "cueq_fc_factors");
       for (size_t i = 0; i < op.shapes.size(); ++i) {
         const GradShape& q = op.shapes[i];
         const int64_t per = int64_t(q.K) * q.N;
         at::Tensor part = new_tensor({q.parts * kChunks, per}, at::kFloat, device);
         check(lib().cueq_gemm_table(dw_code, CUEQ_F32, 1, 1, q.K, q.N, Z, x1t.data_ptr(), op.width1, H.data_ptr(), op.h_width, part.data_ptr(), q.N,
-                                    t.tables[i].data_ptr<int64_t>(), q.parts, kChunks, per, 1.0, 0, stream),
+                                    t.on<int64_t>(device, q.on_device), q.parts, kChunks, per, 1.0, 0, stream),
               "cueq_gemm_table");
         check(lib().cueq_sum_runs(part.data_ptr<float>(), static_cast<int>(per), static_cast<int>(q.w0.size()), q.first.data(), q.w0.data(),
                                   dtype_code(out_dtype), gw.data_ptr(), stream),
@@ -230,10 +198,10 @@ Grads gradients(FcOp& op, const at::Tensor& w_, const at::Tensor& x1_, const at:
       launched(u->dw(Z, x1.data_ptr(), op.width1, x2.data_ptr(), op.n2, g.data_ptr(), op.width_out, part.data_ptr<float>(), op.numel, stream),
                "fully connected weight gradient");
     } else {
-      const auto& t = op.on(device);
-      const at::Tensor& table = by_channels ? t.packed_grads : t.grads;
-      check(lib().cueq_fc_flex_dw(dw_code, op.mul_ir, by_channels, Z, a1.data_ptr(), op.width1, a2.data_ptr(), op.n2, ag.data_ptr(), op.width_out, table.data_ptr(),
-                                  static_cast<int>(table.numel() / 72), static_cast<const float*>(t.coef.data_ptr()), grad_tiles, op.numel,
+      DeviceTables& t = by_channels ? op.packed.back : op.back;
+      const int table = by_channels ? int(Packed::kGrads) : int(FcOp::kGrads);
+      check(lib().cueq_fc_flex_dw(dw_code, op.mul_ir, by_channels, Z, a1.data_ptr(), op.width1, a2.data_ptr(), op.n2, ag.data_ptr(), op.width_out, t.on(device, table),
+                                  t.count(table, 72), t.on<float>(device, by_channels ? int(Packed::kCoef) : int(FcOp::kCoef)), grad_tiles, op.numel,
                                   part.data_ptr<float>(), stream),
             "cueq_fc_flex_dw");
     }
@@ -386,9 +354,9 @@ void bind_fully_connected(py::module_& m) {
         auto op = std::make_shared<FcOp>();
         op->width1 = width1, op->n2 = n2, op->width_out = width_out, op->numel = numel;
         op->mul_ir = mul_ir, op->covers_in = covers_in, op->covers_out = covers_out, op->epv_ok = epv_ok, op->most = most;
-        op->fwd_blocks = tables[0].cast<std::string>(), op->fwd_parts = tables[1].cast<std::string>();
-        op->dx_blocks = tables[2].cast<std::string>(), op->dx_parts = tables[3].cast<std::string>();
-        op->grads = tables[4].cast<std::string>(), op->coef = tables[5].cast<std::string>();
+        op->coef = tables[5].cast<std::string>();
+        for (int t : {0, 1, 5}) op->fwd.add(tables[t].cast<std::string>());
+        for (int t : {2, 3, 5, 4}) op->back.add(tables[t].cast<std::string>());
         op->fwd_tiles = tiles[0].cast<int>(), op->dx_tiles = tiles[1].cast<int>(), op->grad_tiles = tiles[2].cast<int>();
         return op;
       }))
@@ -426,13 +394,15 @@ void bind_fully_connected(py::module_& m) {
           h += int64_t(d) * N;
           op.factors += d * t[5].cast<int>();
         }
+        for (auto& q : op.shapes) q.on_device = op.back.add(q.table);
         op.h_width = h;
       })
       .def("add_packed", [](FcOp& op, const py::tuple& tables, const py::tuple& longest, const py::tuple& pieces, int grad_tiles) {
         auto& p = op.packed;
-        p.fwd_blocks = tables[0].cast<std::string>(), p.fwd_parts = tables[1].cast<std::string>();
-        p.dx_blocks = tables[2].cast<std::string>(), p.dx_parts = tables[3].cast<std::string>();
-        p.fwd_packs = tables[4].cast<std::string>(), p.dx_packs = tables[5].cast<std::string>(), p.grads = tables[6].cast<std::string>();
+        for (int t : {0, 1, 4}) p.fwd.add(tables[t].cast<std::string>());
+        for (int t : {2, 3, 5}) p.back.add(tables[t].cast<std::string>());
+        p.fwd.add(op.coef), p.back.add(op.coef);
+        p.back.add(tables[6].cast<std::string>());
         p.fwd_longest = longest[0].cast<int>(), p.dx_longest = longest[1].cast<int>(), p.grad_tiles = grad_tiles;
         p.fwd_pieces = pieces[0].cast<int64_t>(), p.dx_pieces = pieces[1].cast<int64_t>();
       })

@@ -1,9 +1,6 @@
 // Equivariant Linear with shared weights (uv,iu,iv): choice of the launches and the family of functions forward / input gradient /
 // weight gradient, each differentiable in terms of the others.
-#include "host.h"
-
-#include <mutex>
-#include <unordered_map>
+#include "tables.h"
 
 namespace cueq_host {
 namespace py = pybind11;
@@ -17,6 +14,7 @@ struct RowsLaunch {  // cueq_linear_rows (d == 1 or ir_mul), cueq_linear_rows_mu
   int d, n, k, parts;
   double coeff;
   std::vector<int64_t> table;
+  int on_device = -1;  // (d == 0) its number among the device tables
 };
 struct GradLaunch {  // one weight-gradient launch over strided components, or over mul_ir parts (table non-empty)
   int K, N;
@@ -31,47 +29,16 @@ struct LinearOp {
   int64_t width_in = 0, width_out = 0, numel = 0;
   bool mul_ir = false, covers_in = true, covers_out = true;
   int epv_ok = 0;  // bit 0: float, bit 1: 2-byte elements
-  std::string fwd_blocks, fwd_parts, dx_blocks, dx_parts, grads;  // packed tables
+  enum { kBlocks, kParts, kGrads };
+  DeviceTables fwd, back;  // the packed tables in this order (back: input gradient, then weight gradient), then those of tiled launches
   int fwd_tiles = 0, dx_tiles = 0, grad_tiles = 0;
   std::vector<RowsLaunch> fwd_rows[2], dx_rows[2];  // by element size (4, 2); empty: not for this shape
   std::vector<GradLaunch> grad_rows[2];
   int64_t rows_from[2] = {0, 0}, grad_rows_from[2] = {0, 0};  // from so many rows on the row-streaming launches are the faster ones
 
-  std::mutex mutex;
-  struct OnDevice {
-    at::Tensor fwd_blocks, fwd_parts, dx_blocks, dx_parts, grads;
-    std::vector<at::Tensor> tables[4];  // of the tiled launches: fwd_rows[0], [1], dx_rows[0], [1]
-  };
-  std::unordered_map<int, OnDevice> devices;
-
-  const OnDevice& on(at::Device device) {
-    std::lock_guard<std::mutex> lock(mutex);
-    auto it = devices.find(device.index());
-    if (it == devices.end()) {
-      auto up = [&](const std::string& s) {
-        return at::from_blob(const_cast<char*>(s.data()), {static_cast<int64_t>(s.size())}, at::TensorOptions().dtype(at::kByte)).clone().to(device);
-      };
-      it = devices.emplace(device.index(), OnDevice{up(fwd_blocks), up(fwd_parts), up(dx_blocks), up(dx_parts), up(grads), {}}).first;
-      for (int k = 0; k < 4; ++k)
-        for (const auto& l : (k < 2 ? fwd_rows : dx_rows)[k & 1])
-          it->second.tables[k].push_back(l.d ? at::Tensor() : at::tensor(l.table, at::kLong).to(device));
-    }
-    return it->second;
-  }
-  // Whether the device tables are there or may be uploaded now: a first call that is captured into a HIP graph runs on the launches whose
-  // tables travel as arguments, where there are such, whatever the number of rows.
-  bool tables_at_hand(at::Device device) {
-    std::lock_guard<std::mutex> lock(mutex);
-    return devices.count(device.index()) || !capturing();
-  }
   bool takes(at::ScalarType t) const { return (t == at::kFloat && (epv_ok & 1)) || ((t == at::kBFloat16 || t == at::kHalf) && (epv_ok & 2)); }
 };
 using OpPtr = std::shared_ptr<LinearOp>;
-
-at::Tensor rows_of(const at::Tensor& t, at::ScalarType dtype) {  // contiguous, 16-byte aligned, of that type
-  at::Tensor r = t.to(dtype).contiguous();
-  return reinterpret_cast<uintptr_t>(r.data_ptr()) % 16 ? r.clone() : r;
-}
 
 // forward: x (Z, width_in) -> (Z, width_out); otherwise the input gradient, g (Z, width_out) -> (Z, width_in)
 at::Tensor apply_rows(LinearOp& op, const at::Tensor& w_, const at::Tensor& x_, at::ScalarType dtype, bool forward) {
@@ -85,12 +52,14 @@ at::Tensor apply_rows(LinearOp& op, const at::Tensor& w_, const at::Tensor& x_, 
   const int e = dtype == at::kFloat ? 0 : 1, code = dtype_code(dtype);
   const auto& launches = forward ? op.fwd_rows[e] : op.dx_rows[e];
   hipStream_t stream = stream_of(device.index());
-  if (!launches.empty() && (Z >= op.rows_from[e] || !op.tables_at_hand(device))) {
+  DeviceTables& tables = forward ? op.fwd : op.back;
+  // (a first call that is captured into a HIP graph: the launches whose tables are arguments, however few the rows)
+  if (!launches.empty() && (Z >= op.rows_from[e] || !tables.at_hand(device))) {
     for (size_t i = 0; i < launches.size(); ++i) {
       const RowsLaunch& l = launches[i];
       if (l.d == 0)  // result columns n, contraction k; the weight block is contraction-major in the forward
         check(lib().cueq_gemm_table(code, code, 0, forward ? 1 : 0, Z, l.n, l.k, x.data_ptr(), lda, w.data_ptr(), forward ? l.n : l.k, out.data_ptr(), width,
-                                    op.on(device).tables[(forward ? 0 : 2) + e][i].data_ptr<int64_t>(), l.parts, 1, 0, l.coeff, 0, stream),
+                                    tables.on<int64_t>(device, l.on_device), l.parts, 1, 0, l.coeff, 0, stream),
               "cueq_gemm_table");
       else if (l.d == 1)
         check(lib().cueq_linear_rows(code, forward ? 1 : 0, Z, l.n, l.k, x.data_ptr(), lda, w.data_ptr(), op.numel, out.data_ptr(), width, l.table.data(), l.parts,
@@ -103,10 +72,8 @@ at::Tensor apply_rows(LinearOp& op, const at::Tensor& w_, const at::Tensor& x_, 
     }
     return out;
   }
-  const auto& t = op.on(device);
-  const at::Tensor &blocks = forward ? t.fwd_blocks : t.dx_blocks, &parts = forward ? t.fwd_parts : t.dx_parts;
-  check(lib().cueq_linear_flex(code, forward ? 0 : 1, Z, x.data_ptr(), lda, w.data_ptr(), out.data_ptr(), width, blocks.data_ptr(),
-                               static_cast<int>(blocks.numel() / 32), parts.data_ptr(), forward ? op.fwd_tiles : op.dx_tiles, op.mul_ir, stream),
+  check(lib().cueq_linear_flex(code, forward ? 0 : 1, Z, x.data_ptr(), lda, w.data_ptr(), out.data_ptr(), width, tables.on(device, LinearOp::kBlocks),
+                               tables.count(LinearOp::kBlocks, 32), tables.on(device, LinearOp::kParts), forward ? op.fwd_tiles : op.dx_tiles, op.mul_ir, stream),
         "cueq_linear_flex");
   return out;
 }
@@ -123,7 +90,7 @@ at::Tensor weight_gradient(LinearOp& op, const at::Tensor& x_, const at::Tensor&
   const int e = dtype == at::kFloat ? 0 : 1, code = dtype_code(dtype), out_code = dtype_code(out_dtype);
   const int64_t es = dtype == at::kFloat ? 4 : 2;
   hipStream_t stream = stream_of(device.index());
-  if (!op.grad_rows[e].empty() && (Z >= op.grad_rows_from[e] || !op.tables_at_hand(device))) {
+  if (!op.grad_rows[e].empty() && (Z >= op.grad_rows_from[e] || !op.back.at_hand(device))) {
     for (const auto& l : op.grad_rows[e]) {
       const int n = static_cast<int>(l.w_off.size());
       std::vector<int32_t> first(n + 1, 0);
@@ -147,10 +114,9 @@ at::Tensor weight_gradient(LinearOp& op, const at::Tensor& x_, const at::Tensor&
       check(lib().cueq_sum_runs(part.data_ptr<float>(), l.K * l.N, n, first.data(), l.w_off.data(), out_code, gw.data_ptr(), stream), "cueq_sum_runs");
     }
   } else {
-    const auto& t = op.on(device);
     const int64_t chunks = lib().cueq_linear_flex_dw_chunks(Z, op.grad_tiles);
     at::Tensor part = new_tensor({chunks, op.numel}, at::kFloat, device);
-    check(lib().cueq_linear_flex_dw(code, Z, x.data_ptr(), op.width_in, g.data_ptr(), op.width_out, t.grads.data_ptr(), static_cast<int>(t.grads.numel() / 64),
+    check(lib().cueq_linear_flex_dw(code, Z, x.data_ptr(), op.width_in, g.data_ptr(), op.width_out, op.back.on(device, LinearOp::kGrads), op.back.count(LinearOp::kGrads, 64),
                                     op.grad_tiles, op.numel, part.data_ptr<float>(), op.mul_ir, out_code, gw.data_ptr(), stream),
           "cueq_linear_flex_dw");
   }
@@ -245,11 +211,12 @@ py::object direct(const OpPtr& op, const at::Tensor& w, const at::Tensor& x) {
   return py::cast(forward(op, w, x));
 }
 
-std::vector<RowsLaunch> rows_launches(const py::list& l) {
+std::vector<RowsLaunch> rows_launches(const py::list& l, DeviceTables& tables) {
   std::vector<RowsLaunch> out;
   for (const auto& item : l) {
     const py::tuple t = py::reinterpret_borrow<py::tuple>(item);
     out.push_back({t[0].cast<int>(), t[1].cast<int>(), t[2].cast<int>(), t[4].cast<int>(), t[5].cast<double>(), t[3].cast<std::vector<int64_t>>()});
+    if (out.back().d == 0) out.back().on_device = tables.add(out.back().table);
   }
   return out;
 }
@@ -263,16 +230,15 @@ void bind_linear(py::module_& m) {
         auto op = std::make_shared<LinearOp>();
         op->width_in = width_in, op->width_out = width_out, op->numel = numel;
         op->mul_ir = mul_ir, op->covers_in = covers_in, op->covers_out = covers_out, op->epv_ok = epv_ok;
-        op->fwd_blocks = tables[0].cast<std::string>(), op->fwd_parts = tables[1].cast<std::string>();
-        op->dx_blocks = tables[2].cast<std::string>(), op->dx_parts = tables[3].cast<std::string>(), op->grads = tables[4].cast<std::string>();
+        for (int t = 0; t < 5; ++t) (t < 2 ? op->fwd : op->back).add(tables[t].cast<std::string>());
         op->fwd_tiles = tiles[0].cast<int>(), op->dx_tiles = tiles[1].cast<int>(), op->grad_tiles = tiles[2].cast<int>();
         return op;
       }))
       // launches for many rows, elements of `es` bytes: lists of (d, columns, contraction, table, parts, coefficient)
       .def("add_rows", [](LinearOp& op, int es, int64_t from, const py::list& fwd, const py::list& dx) {
         const int e = es == 4 ? 0 : 1;
-        op.fwd_rows[e] = rows_launches(fwd);
-        op.dx_rows[e] = rows_launches(dx);
+        op.fwd_rows[e] = rows_launches(fwd, op.fwd);
+        op.dx_rows[e] = rows_launches(dx, op.back);
         op.rows_from[e] = from;
       })
       // lists of (K, N, coefficient, a0, c0, da, dc, table, weight offsets, components per weight block)
