@@ -337,26 +337,27 @@ def _fc_tables(mod, x2_mul_ir: bool = False):
     ope, stp = mod._polynomial_orig.operations[0]
     if str(stp.subscripts) not in ("uvw,iu,jv,kw+ijk", "uw,iu,j,kw+ijk") or not stp.paths:
         return None
-    offs = [o.segment_offsets() for o in stp.operands]
-    sizes = [o.size for o in stp.operands]
+    operands = stp.operands
+    offs = [o.segment_offsets() for o in operands]
+    sizes = [o.size for o in operands]
     coef: list = []
     paths = []
     for p in stp.paths:
         sw, s1, s2, so = p.indices
-        (d1, K), d2, (d3, N) = stp.operands[1][s1], stp.operands[2][s2][0], stp.operands[3][so]
-        V = stp.operands[0][sw][1] if len(stp.operands[0][sw]) == 3 else 1
+        (d1, K), d2, (d3, N) = operands[1][s1], operands[2][s2][0], operands[3][so]
+        V = operands[0][sw][1] if len(operands[0][sw]) == 3 else 1
         c = p.coefficients
         if d1 not in (1, 3, 5) or d3 not in (1, 3, 5):
             return None
         at = len(coef)
-        coef += [float(v) for v in c.transpose(0, 2, 1).reshape(-1)]
+        coef += c.transpose(0, 2, 1).ravel().tolist()
         back = len(coef)
-        coef += [float(v) for v in c.transpose(2, 0, 1).reshape(-1)]
-        used = (c != 0).any(axis=1)  # (i, k)
-        mask = sum(1 << (i * d3 + k) for i in range(d1) for k in range(d3) if used[i, k])
-        mask_back = sum(1 << (k * d1 + i) for i in range(d1) for k in range(d3) if used[i, k])
-        coupled = all(_couples(d1, d2, d3, i, j, k) for i, j, k in zip(*c.nonzero()))
-        paths.append(SimpleNamespace(coupled=coupled, w0=offs[0][sw], a0=offs[1][s1], K=K, d1=d1, c0=offs[3][so], N=N, d3=d3, coef=at, coef_back=back, j0=offs[2][s2],
+        coef += c.transpose(2, 0, 1).ravel().tolist()
+        mask = mask_back = 0
+        for i, j, k in zip(*(v.tolist() for v in c.nonzero())):
+            mask |= 1 << (i * d3 + k)
+            mask_back |= 1 << (k * d1 + i)
+        paths.append(SimpleNamespace(c=c, w0=offs[0][sw], a0=offs[1][s1], K=K, d1=d1, c0=offs[3][so], N=N, d3=d3, coef=at, coef_back=back, j0=offs[2][s2],
                                      d2=d2, V=V, js=1 if x2_mul_ir else V, vs=d2 if x2_mul_ir else 1, mask=mask, mask_back=mask_back))
     if len({p.w0 for p in paths}) != len(paths) or sum(p.K * p.V * p.N for p in paths) != sizes[0] or sizes[2] > 128:
         return None
@@ -369,7 +370,8 @@ def _fc_tables(mod, x2_mul_ir: bool = False):
         return None
 
     # the couplings that the kernels with straight loops over the channels of x2 know; blocks held in registers there have up to 64 values
-    straight = all(p.coupled for p in paths)
+    several = any(p.V > 1 for p in paths)
+    straight = several and all(_couples(p.d1, p.d2, p.d3, *t) for p in paths for t in zip(*(v.tolist() for v in p.c.nonzero())))
     resident = straight and all(p.K <= 64 and p.N <= 64 for p in paths)
     steps = {True: 2 if all(p.N <= 32 for p in paths) else 4, False: 2 if all(p.K <= 32 for p in paths) else 4}  # (by direction: of 16 values)
 
@@ -412,7 +414,7 @@ def _fc_tables(mod, x2_mul_ir: bool = False):
 
     fwd, dx, dw = side(False), side(True), grads(False)
     packed = None
-    if served & 2 and any(p.V > 1 for p in paths):
+    if served & 2 and several:
         pf, px = side(False, True), side(True, True)
         pw = grads(True) if straight else (b"", 0)
         packed = ((pf[0], pf[1], px[0], px[1], pf[3], px[3], pw[0]), (steps[False], steps[True]) if resident else (5, 5), (pf[4], px[4]), pw[1])
