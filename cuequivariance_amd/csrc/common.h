@@ -52,6 +52,12 @@ typedef _Float16 mm_f16x2 __attribute__((ext_vector_type(2)));
 template <typename TI> struct is_half_bits { static constexpr bool value = false; };
 template <> struct is_half_bits<f16bits> { static constexpr bool value = true; };
 
+// elements i0 (low half) and i1 (high half) of a run of 2-byte elements in registers
+__device__ __forceinline__ uint32_t mm_pick(const uint4* run, int i0, int i1) {
+  const uint32_t* w = reinterpret_cast<const uint32_t*>(run);
+  const uint32_t sel = static_cast<uint32_t>((i0 & 1) * 2 | ((i0 & 1) * 2 + 1) << 8 | (4 + (i1 & 1) * 2) << 16 | (4 + (i1 & 1) * 2 + 1) << 24);
+  return __builtin_amdgcn_perm(w[i1 >> 1], w[i0 >> 1], sel);
+}
 // acc += A (32 x 16) B (16 x 32), eight 2-byte elements per lane and operand
 template <typename TI>
 __device__ __forceinline__ mm_floatx16 mm_32x32x16(uint4 a, uint4 b, mm_floatx16 acc) {

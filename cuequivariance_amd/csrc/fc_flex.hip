@@ -49,19 +49,12 @@ __device__ __forceinline__ float fc_widen(const TI* p) {
   else return mm_widen<TI>(*reinterpret_cast<const uint16_t*>(p));
 }
 
-template <int D>
-__device__ __forceinline__ uint32_t fc_pick(const uint4* run, int i0, int i1) {
-  const uint32_t* w = reinterpret_cast<const uint32_t*>(run);
-  const uint32_t sel = static_cast<uint32_t>((i0 & 1) * 2 | ((i0 & 1) * 2 + 1) << 8 | (4 + (i1 & 1) * 2) << 16 | (4 + (i1 & 1) * 2 + 1) << 24);
-  return __builtin_amdgcn_perm(w[i1 >> 1], w[i0 >> 1], sel);
-}
-
 // component i of eight channels: x is DS pieces of one component each (ir_mul) or of eight channels with their components adjacent
 template <int DS, bool MI>
 __device__ __forceinline__ uint4 fc_component(const uint4 (&x)[DS], int i) {
   if constexpr (DS == 1 || !MI) return x[i];
-  else return make_uint4(fc_pick<DS>(&x[0], i, DS + i), fc_pick<DS>(&x[0], 2 * DS + i, 3 * DS + i), fc_pick<DS>(&x[0], 4 * DS + i, 5 * DS + i),
-                         fc_pick<DS>(&x[0], 6 * DS + i, 7 * DS + i));
+  else return make_uint4(mm_pick(&x[0], i, DS + i), mm_pick(&x[0], 2 * DS + i, 3 * DS + i), mm_pick(&x[0], 4 * DS + i, 5 * DS + i),
+                         mm_pick(&x[0], 6 * DS + i, 7 * DS + i));
 }
 
 // The coefficients of one path (at most 64), a lane each: short products would wait for a memory request for each of them.

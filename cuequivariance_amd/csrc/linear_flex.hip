@@ -33,13 +33,6 @@ struct FlexBlock {  // one block of the result
 
 typedef float fx16 __attribute__((ext_vector_type(16)));
 
-template <int D>
-__device__ __forceinline__ uint32_t pick2(const uint4* run, int i0, int i1) {  // elements i0 (low), i1 (high) of a run of 2-byte elements
-  const uint32_t* w = reinterpret_cast<const uint32_t*>(run);
-  const uint32_t sel = static_cast<uint32_t>((i0 & 1) * 2 | ((i0 & 1) * 2 + 1) << 8 | (4 + (i1 & 1) * 2) << 16 | (4 + (i1 & 1) * 2 + 1) << 24);
-  return __builtin_amdgcn_perm(w[i1 >> 1], w[i0 >> 1], sel);
-}
-
 // one tile: rows z0 .. z0 + 32 ZT, columns n0 .. n0 + 32 of the block.  WT: the weights are read transposed (input gradient).
 // SK: wavefronts that share the tile, each with its part of every contraction; the first adds the others' sums, in order, through
 // LDS and stores (SK > 1: all SK wavefronts of the workgroup are here).
@@ -111,8 +104,8 @@ __device__ __forceinline__ void flex_tile(const FlexBlock& blk, const FlexPart* 
           for (int i = 0; i < D; ++i) {
             uint4 op;
             if constexpr (D == 1) op = x[t][0];
-            else op = make_uint4(pick2<D>(&x[t][0], i, D + i), pick2<D>(&x[t][0], 2 * D + i, 3 * D + i), pick2<D>(&x[t][0], 4 * D + i, 5 * D + i),
-                                 pick2<D>(&x[t][0], 6 * D + i, 7 * D + i));
+            else op = make_uint4(mm_pick(&x[t][0], i, D + i), mm_pick(&x[t][0], 2 * D + i, 3 * D + i), mm_pick(&x[t][0], 4 * D + i, 5 * D + i),
+                                 mm_pick(&x[t][0], 6 * D + i, 7 * D + i));
             acc[t][i] = mm_32x32x16<TI>(wv, op, acc[t][i]);
           }
         }

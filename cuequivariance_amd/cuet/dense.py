@@ -1442,7 +1442,6 @@ class SegmentedPolynomialDense(nn.Module):
         self.dx1_groups = _batched_groups(self.paths, lambda p: p.c_off, lambda p: p.a_off)
         self.weight_blocks = sorted({(p.w_off, p.K, p.N) for p in self.paths})
         self.fc_plan = _FcPlan(self.paths, self.input_sizes[2]) if self.has_x2 else None
-        self._merged: dict = {}
         self._fused: dict = {}
         self._dw_shapes: dict = {}
         # rows="mul_ir": the irreps operands (input 1 and the output of the 3-operand form) keep the component index
