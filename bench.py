@@ -245,8 +245,8 @@ def secondary(torch, cue, cuet, _lib, dev, wl: str, dtype_name, steps: int, warm
         if wl == "cfg4fcmi":
             desc += "; rows in mul_ir, taken as they lie by the fused kernels (no transposition pass)"
     elif wl == "fcgen":
-        # a fully connected product whose second operand has multiplicity above one (no BASELINE config; sizes chosen here): the
-        # products of the two operands in HBM, then a Linear map on the matrix cores
+        # a fully connected product whose second operand has multiplicity above one (sizes chosen here): products of the two operands
+        # formed in registers, contracted on the matrix cores
         Z = 50_000
         dtype = getattr(torch, _DTYPES[dtype_name])
         i1, i2 = cue.Irreps("O3", "64x0e+64x1o"), cue.Irreps("O3", "16x0e+16x1o")
@@ -268,9 +268,8 @@ def secondary(torch, cue, cuet, _lib, dev, wl: str, dtype_name, steps: int, warm
         f = 2 * Z * 64 * 16 * 64 * 10
         flops = {"fwd": f, "bwd": 2 * f}
         flop_roof, flop_peak = "mfma", MFMA_PEAK[dt]
-        desc = ("next row (the general fully connected form u_v_uvw_w): FullyConnectedTensorProduct 64x0e+64x1o (x) 16x0e+16x1o -> "
-                "64x0e+64x1o, batch 50000, shared weights, fwd + bwd (dw, dx1, dx2); products of the two operands in HBM (10240 values per "
-                "row), then a Linear map on the matrix cores")
+        desc = ("the general fully connected form u_v_uvw_w: FullyConnectedTensorProduct 64x0e+64x1o (x) 16x0e+16x1o -> 64x0e+64x1o, "
+                "batch 50000, shared weights, fwd + bwd (dw, dx1, dx2); products of the two operands (10240 per row) in registers")
     elif wl == "cfg2sh":
         # configs[1] with the spherical harmonics of the edge vectors evaluated inside the edge kernels (the step before the
         # product in a MACE interaction block): inputs are the raw edge vectors, gradients also with respect to them
@@ -298,7 +297,7 @@ def secondary(torch, cue, cuet, _lib, dev, wl: str, dtype_name, steps: int, warm
                 "100000 edges, inputs node features / edge vectors / per-edge weights, fwd + bwd (dw, dx1, d vectors)")
     elif wl == "fcconv":
         # the product inside FullyConnectedTensorProductConv: a weight row per edge, x1 gathered by source, output summed by
-        # destination (no BASELINE config; sizes chosen here)
+        # destination (sizes chosen here)
         E, N = 20_000, 2_000
         i1, i2 = cue.Irreps("O3", "64x0e+64x1o"), cue.Irreps("O3", "0e+1o+2e")
         m = cuet.FullyConnectedTensorProduct(i1, i2, i1, layout=cue.ir_mul, shared_weights=False, internal_weights=False,
@@ -322,7 +321,7 @@ def secondary(torch, cue, cuet, _lib, dev, wl: str, dtype_name, steps: int, warm
         f = 2 * E * 64 * 64 * 11
         flops = {"fwd": f, "bwd": 2 * f}
         flop_roof, flop_peak = "valu", VALU_PEAK_F32
-        desc = ("next row (FullyConnectedTensorProductConv's product): 64x0e+64x1o (x) 0e+1o+2e -> 64x0e+64x1o, a weight row per edge, "
+        desc = ("FullyConnectedTensorProductConv's product: 64x0e+64x1o (x) 0e+1o+2e -> 64x0e+64x1o, a weight row per edge, "
                 "20000 edges, 2000 nodes, x1 gathered by source, output summed by destination, fwd + bwd (dw, dx1, dx2)")
     elif wl == "cfg5":
         dtype = getattr(torch, _DTYPES[dtype_name or "bf16"])
