@@ -1485,7 +1485,6 @@ __global__ void __launch_bounds__(512, 2)
   for (int64_t tile = tile0; tile < ntiles; tile += tstep) {
     uint4 xf[NT][NS][2], xf2[1][NS][2];
     float mk[NT];
-    uint32_t keep[NT];  // padding that the contraction runs over: selected away (a product with 0 would keep what is not finite)
     int mcol[NT];
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
@@ -1498,7 +1497,9 @@ __global__ void __launch_bounds__(512, 2)
           if constexpr (ROWS) xf2[t][s2][q] = xn2[t][s2][q];
         }
       mk[t] = mask ? lo16<F>(mraw[t]) : 1.0f;
-      keep[t] = !(PAD && LN) || live_n[t] ? ~0u : 0u;
+      if constexpr (PAD && LN) {
+        if (!live_n[t]) mk[t] = 0.0f;  // (what it multiplies is as finite as the row that the padding repeats)
+      }
     }
     request_x(min(tile + tstep, ntiles - 1));  // (past the end: the last tile again, so that the request is unconditional)
     if constexpr (LN) {
@@ -1625,8 +1626,7 @@ __global__ void __launch_bounds__(512, 2)
             const int v = 4 * a + b;
             g[b] = __builtin_amdgcn_rcpf(1.0f + __expf(-au[t][v])) * av[t][v] * mk[t];
           }
-          uint32_t own[2] = {pack16<F>(g[0], g[1]), pack16<F>(g[2], g[3])};
-          if constexpr (PAD) own[0] &= keep[t], own[1] &= keep[t];
+          const uint32_t own[2] = {pack16<F>(g[0], g[1]), pack16<F>(g[2], g[3])};
 #pragma unroll
           for (int j = 0; j < 2; ++j) {
             const uint32_t other = static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(own[j]), 0xB1, 0xF, 0xF, true));

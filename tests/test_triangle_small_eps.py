@@ -43,3 +43,23 @@ def test_no_eps_on_ragged_squares(device, batch, n, d, outgoing, dtype, masked):
     for name, a, b in zip(["out", *wanted], [out, *got], [ref, *want]):
         err = (a.detach().cpu().double() - b.detach()).abs().max().item()
         assert err <= TOL[dtype] * max(b.detach().abs().max().item(), 1e-3), (name, err, b.abs().max().item())
+
+
+@pytest.mark.parametrize("n,d,outgoing,dtype", [(9, 32, True, torch.float32), (13, 64, False, torch.bfloat16), (67, 64, False, torch.bfloat16),
+                                                (71, 128, True, torch.float16)])
+@pytest.mark.parametrize("row,column", [(-1, -1), (2, -1), (-1, 3), (4, 5)])
+def test_an_infinite_value_stays_in_its_rows(device, n, d, outgoing, dtype, row, column):
+    """Padding repeats the last row and column: what is infinite there must not reach rows that it does not reach without padding."""
+    from cuequivariance_amd import cuet
+
+    g = torch.Generator().manual_seed(6)
+    r = lambda *shape, scale=1.0: (torch.randn(*shape, generator=g, dtype=torch.float64) * scale).to(dtype).double()
+    p = dict(x=r(1, n, n, d), p_in_weight=r(2 * d, d, scale=d ** -0.5), g_in_weight=r(2 * d, d, scale=d ** -0.5), p_out_weight=r(d, d, scale=d ** -0.5),
+             g_out_weight=r(d, d, scale=d ** -0.5), p_in_bias=r(2 * d), g_in_bias=r(2 * d))
+    p["x"][0, row, column, 7] = float("inf")
+    options = dict(direction="outgoing" if outgoing else "incoming")
+    want = oracle(**options, **p)
+    got = cuet.triangle_multiplicative_update(**options, **{k: v.to(dtype).to(device) for k, v in p.items()}).cpu().double()
+    keep = torch.isfinite(want)
+    assert keep.any() and not keep.all() and torch.equal(torch.isfinite(got), keep)
+    assert (got[keep] - want[keep]).abs().max().item() <= TOL[dtype] * want[keep].abs().max().item()
