@@ -74,6 +74,60 @@ bool wants_graph(const std::vector<at::Tensor>& tensors) {
   return false;
 }
 
+namespace {
+PyObject* key(const char* name) { return PyUnicode_InternFromString(name); }
+
+PyObject* dict_of(PyObject* object) {  // borrowed: the attributes of an instance
+  PyObject** d = _PyObject_GetDictPtr(object);
+  return d ? *d : nullptr;
+}
+bool empty(PyObject* dict, PyObject* name) {  // there and without an entry
+  PyObject* hooks = PyDict_GetItem(dict, name);
+  return hooks && PyDict_Check(hooks) && PyDict_Size(hooks) == 0;
+}
+
+// The children of a module are of the classes it was built with, and a call of one runs its `forward` and nothing else.
+bool untouched(PyObject* module, PyObject* built) {
+  static PyObject* const modules = key("_modules");
+  static PyObject* const hooks[] = {key("_forward_hooks"), key("_forward_pre_hooks"), key("_backward_hooks"), key("_backward_pre_hooks")};
+  static PyObject* const replaced[] = {key("forward"), key("_compiled_call_impl")};
+  PyObject* own = dict_of(module);
+  PyObject* children = own ? PyDict_GetItem(own, modules) : nullptr;
+  if (!children || !PyDict_Check(children)) return false;
+  PyObject *name, *child;
+  Py_ssize_t at = 0;
+  while (PyDict_Next(children, &at, &name, &child)) {
+    if (child == Py_None) continue;
+    if (PySet_Contains(built, reinterpret_cast<PyObject*>(Py_TYPE(child))) != 1) return false;
+    PyObject* d = dict_of(child);
+    if (!d) return false;
+    for (PyObject* h : hooks)
+      if (!empty(d, h)) return false;
+    for (PyObject* r : replaced)
+      if (PyDict_Contains(d, r)) return false;
+  }
+  return true;
+}
+
+// The executor of class `kind` that a call of `module`'s child `name` (of class `outer`) ends in, None unless it may be run without those
+// calls: nothing replaced, wrapped or hooked on the way, no hook on all modules.
+pybind11::object executor(const pybind11::object& module, const pybind11::str& name, const pybind11::type& outer, const pybind11::type& kind,
+                          const pybind11::object& built) {
+  static PyObject* const global[] = {key("_global_backward_pre_hooks"), key("_global_backward_hooks"),        key("_global_forward_pre_hooks"),
+                                     key("_global_forward_hooks"),      key("_global_forward_hooks_always_called"), key("_global_forward_hooks_with_kwargs")};
+  static PyObject* const torch_module = PyModule_GetDict(PyImport_ImportModule("torch.nn.modules.module"));
+  static PyObject *const modules = key("_modules"), *const inner = key("m");
+  for (PyObject* g : global)
+    if (!empty(torch_module, g)) return pybind11::none();
+  if (!untouched(module.ptr(), built.ptr())) return pybind11::none();
+  PyObject* f = PyDict_GetItem(PyDict_GetItem(dict_of(module.ptr()), modules), name.ptr());
+  if (!f || reinterpret_cast<PyObject*>(Py_TYPE(f)) != outer.ptr() || !untouched(f, built.ptr())) return pybind11::none();
+  PyObject* m = PyDict_GetItem(PyDict_GetItem(dict_of(f), modules), inner);
+  if (!m || reinterpret_cast<PyObject*>(Py_TYPE(m)) != kind.ptr() || !untouched(m, built.ptr())) return pybind11::none();
+  return pybind11::reinterpret_borrow<pybind11::object>(m);
+}
+}  // namespace
+
 // Eager mode: built once per index tensor and cached (the build checks on the host that the ids are in range and skips the sort when
 // they are sorted already).  While the current stream is being captured into a HIP graph the grouping is recorded into the graph
 // instead (device-side work only, nothing cached), so every replay regroups from whatever the index buffer holds then.  Index
@@ -126,6 +180,7 @@ PYBIND11_MODULE(_host, m) {
   });
   m.def("load", &load);
   m.def("segment_csr", &segment_csr);
+  m.def("executor", &executor);
   bind_uniform_1d(m);
   bind_triangle(m);
   bind_linear(m);

@@ -21,7 +21,7 @@ from typing import Dict, List, Optional, Sequence
 
 import torch
 
-from .. import cue
+from .. import _lib, cue
 from ..cue import descriptors
 from .dense import GeneralFullyConnected, SegmentedPolynomialDense
 from .fused_tp import SegmentedPolynomialFusedTP, _FlattenedOperation, _MatrixWithElementwiseStage
@@ -56,28 +56,13 @@ def _transposition_moves(irreps) -> bool:
     return any(mul > 1 and ir.dim > 1 for mul, ir in irreps)
 
 
-def _untouched(module: torch.nn.Module) -> bool:
-    """Whether the children of ``module`` are of the classes it was built with and a call of one runs its ``forward`` and nothing else:
-    a replaced child (a wrapper, ``torch.compile``), a hook on one (profilers, operation counters) or a ``forward`` put in its place
-    is to be called."""
-    for child in module._modules.values():
-        if child is not None:
-            d = child.__dict__
-            if (type(child) not in _BUILT or d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"] or d["_backward_pre_hooks"]
-                    or "forward" in d or "_compiled_call_impl" in d):
-                return False
-    return True
-
-
 def _executor(module: torch.nn.Module, name: str, kind: type):
-    """The executor (of type ``kind``) that a call of the child ``name`` ends in, when it may be run without those calls; else ``None``."""
-    if torch.compiler.is_compiling() or torch.nn.modules.module._has_any_global_hook() or not _untouched(module):
+    """The executor (of type ``kind``) that a call of the child ``name`` ends in, when it may be run without those calls; ``None`` while a
+    graph is traced, and where the calls are to be seen: a child of ``module`` or of ``name`` was replaced (a wrapper, ``torch.compile``),
+    has hooks (profilers, operation counters) or another ``forward``, or there are hooks on all modules."""
+    if torch.compiler.is_compiling():
         return None
-    f = module._modules[name]
-    if type(f) is not SegmentedPolynomial or not _untouched(f):
-        return None
-    m = f._modules["m"]
-    return m if type(m) is kind and _untouched(m) else None
+    return _lib.host().executor(module, name, SegmentedPolynomial, kind, _BUILT)
 
 
 def _operator(module: torch.nn.Module):
