@@ -411,6 +411,51 @@ def emit_forward(st: ChannelwiseStructure, T: str, nsplit: int, waves_per_eu: in
 # ---------------------------------------------------------------------------------------------
 # backward
 # ---------------------------------------------------------------------------------------------
+def _fold_plan(n: int, lanes: int):
+    """Lane bits that halve ``n`` sums (as (bit, sums before the step)) and those left for plain steps, for sums over the lane
+    bits below ``lanes``."""
+    halving, plain, bit = [], [], lanes // 2
+    while bit:
+        if n > 1:
+            halving.append((bit, n))
+            n = (n + 1) // 2
+        else:
+            plain.append(bit)
+        bit //= 2
+    assert n == 1
+    return halving, plain
+
+
+def emit_lane_sums(A, ind: str, T: str, values: Sequence[str], lanes: int, prefix: str) -> str:
+    """Sums of up to ``lanes`` registers over groups of ``lanes`` lanes, each left in the lane ``_slot_of_lane`` says; returns the
+    register's name."""
+    halving, plain = _fold_plan(len(values), lanes)
+    cur = list(values)
+    for level, (bit, n) in enumerate(halving):
+        assert n == len(cur)
+        nxt = []
+        for p in range(0, n, 2):
+            nxt.append(f"{prefix}{level}_{p // 2}")
+            A(f"{ind}const {T} {nxt[-1]} = " + (f"lane_fold<{bit}>({cur[p]}, {cur[p + 1]}, lane);" if p + 1 < n else f"lane_fold<{bit}>({cur[p]});"))
+        cur = nxt
+    for bit in plain:
+        A(f"{ind}const {T} {prefix}p{bit} = lane_fold<{bit}>({cur[0]});")
+        cur = [f"{prefix}p{bit}"]
+    return cur[0]
+
+
+def emit_slot_of_lane(A, ind: str, name: str, n: int, lanes: int):
+    """``const int name``: which of the ``n`` sums of ``emit_lane_sums`` this lane holds and stores, -1 where it stores none."""
+    halving, plain = _fold_plan(n, lanes)
+    A(f"{ind}int {name} = 0;")
+    A(f"{ind}{{")
+    A(f"{ind}  bool mine = (lane & {sum(plain)}) == 0;")
+    for bit, before in reversed(halving):
+        A(f"{ind}  {name} = 2 * {name} + ((lane & {bit}) ? 1 : 0); mine = mine && {name} < {before};")
+    A(f"{ind}  if (!mine) {name} = -1;")
+    A(f"{ind}}}")
+
+
 def emit_backward(st: ChannelwiseStructure, T: str, waves_per_eu: int, chunk: int, prefetch: bool = False, nsplit: int = 1) -> str:
     """HIP source of the fused backward kernel (dw, dx1, dx2 in one pass).
 
@@ -448,6 +493,10 @@ def emit_backward(st: ChannelwiseStructure, T: str, waves_per_eu: int, chunk: in
                 staged.append((first, d))
             first += d
         staged_segments = {i for i0, d in staged for i in range(i0, i0 + d)}
+
+        # the second operand's gradient, in pieces of at most 64 sums over the lanes
+        d2_names = [f"dv{a}" for a in range(3)] if st.harmonics else [f"pj{j}" if j in j_used else f"{fp}(0)" for j in range(st.nseg_x2)]
+        d2_pieces = [(c0, d2_names[c0: c0 + 64]) for c0 in range(0, len(d2_names), 64)]
 
         def load(S: str, zz: str, ind: str):
             A(f"{ind}{{")
@@ -548,12 +597,12 @@ def emit_backward(st: ChannelwiseStructure, T: str, waves_per_eu: int, chunk: in
                 A(f"{ind}    io_st(" + (f"dxa{i}" if i in i_used else f"{fp}(0)") + f", dp + ({st.x1_at(i)}));")
             A(f"{ind}  }}")
             A(f"{ind}}}")
-            # dx2: reduce over the 64 lanes; channel chunks and wavefronts of one batch row are folded afterwards
+            # dx2: reduced over the 64 lanes, the sums halved among them (16 sums over 64 lanes: 15 halving steps and 2 plain
+            # ones, one store of 16 lanes, where 16 butterflies take 96 steps and one lane 16 stores; forward + backward, fp32:
+            # 32 ch l <= 2, 60 000 edges 124.5 -> 118.6 us, 128 ch l <= 3, 1 000 edges 102.2 -> 99.0 us); channel chunks and wavefronts of one batch row are folded afterwards
             A(f"{ind}if (!active) {{" + " ".join(f"pj{j} = 0;" for j in j_used) + "}")
-            for j in j_used:
-                A(f"{ind}pj{j} = wave_sum(pj{j});")
             if st.harmonics:
-                # dv[a] = sum_j pj[j] dY_j/dv[a] (this wavefront's share: the sum over its channels and blocks is linear)
+                # dv[a] = sum_j pj[j] dY_j/dv[a] (this lane's share: the sums over channels and blocks are linear)
                 rests = set()
                 for j in j_used:
                     for vi, _ in st.harmonics[j]:
@@ -571,23 +620,20 @@ def emit_backward(st: ChannelwiseStructure, T: str, waves_per_eu: int, chunk: in
                             rest.remove(a)
                             A(f"{ind}  dv{a} = fma({_lit(c * vi.count(a), T)} * pj{j}, {_mono_name(tuple(rest))}, dv{a});")
                 A(f"{ind}}}")
-            A(f"{ind}if (lane == 0) {{")
             if nparts == 1:
-                A(f"{ind}  TI* __restrict__ d2 = dx2 + z * {st.x2_width}ll;")
+                A(f"{ind}TI* __restrict__ d2 = dx2 + z * {st.x2_width}ll;")
             else:
-                A(f"{ind}  {fp}* __restrict__ d2 = dx2_partial + (z * {nparts} + ch * {nsplit} + {q}) * {st.x2_width}ll;")
-            if st.harmonics:
-                for a in range(3):
-                    A(f"{ind}  io_st(dv{a}, d2 + {a});")
-            else:
-                for j in range(st.nseg_x2):
-                    A(f"{ind}  io_st(" + (f"pj{j}" if j in j_used else f"{fp}(0)") + f", d2 + {j});")
-            A(f"{ind}}}")
+                A(f"{ind}{fp}* __restrict__ d2 = dx2_partial + (z * {nparts} + ch * {nsplit} + {q}) * {st.x2_width}ll;")
+            for c0, names in d2_pieces:
+                total = emit_lane_sums(A, ind, fp, names, 64, f"r{c0}_")
+                A(f"{ind}if (slot{len(names)} >= 0) io_st({total}, d2 + {c0} + slot{len(names)});")
 
         A("template <bool X1_IDX, bool G_IDX, bool ATOMIC_DX1>")
         A(f"__device__ __forceinline__ void bwd_group{q}(BWD_PARAMS, int64_t z0, int64_t z1, int lane, int uu, bool active, int ch) {{")
         if staged:
             A(f"  __shared__ {fp} dxs[{64 * max(d for _, d in staged)}];")
+        for n in sorted({len(names) for _, names in d2_pieces}):
+            emit_slot_of_lane(A, "  ", f"slot{n}", n, 64)
         for k in ks:
             A(f"  {fp} gr{k} = 0;")
         A("  int64_t grow_cur = -1;")

@@ -20,16 +20,79 @@ __device__ __forceinline__ double dpp_move(double v) {
   return __builtin_bit_cast(double, (static_cast<uint64_t>(hi) << 32) | lo);
 }
 
+// ---- sums over lanes -----------------------------------------------------------------------------
+// v_permlane32_swap / v_permlane16_swap (32-bit words): lanes whose bit 32 (16) is set in the first register change places with
+// the lanes of the second whose bit is clear.  (The words are named before they are cast back: a bit cast of an element of the
+// builtin's result reads element 0.)
+template <int BIT>
+__device__ __forceinline__ void lane_swap(uint32_t& a, uint32_t& b) {
+  static_assert(BIT == 32 || BIT == 16, "lane bits that v_permlane*_swap moves");
+  if constexpr (BIT == 32) {
+    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    const uint32_t r0 = r[0], r1 = r[1];
+    a = r0; b = r1;
+  } else {
+    const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    const uint32_t r0 = r[0], r1 = r[1];
+    a = r0; b = r1;
+  }
+}
+template <int BIT>
+__device__ __forceinline__ void lane_swap(float& a, float& b) {
+  uint32_t x = __builtin_bit_cast(uint32_t, a), y = __builtin_bit_cast(uint32_t, b);
+  lane_swap<BIT>(x, y);
+  a = __builtin_bit_cast(float, x); b = __builtin_bit_cast(float, y);
+}
+template <int BIT>
+__device__ __forceinline__ void lane_swap(double& a, double& b) {
+  const uint64_t p = __builtin_bit_cast(uint64_t, a), q = __builtin_bit_cast(uint64_t, b);
+  uint32_t pl = static_cast<uint32_t>(p), ph = static_cast<uint32_t>(p >> 32), ql = static_cast<uint32_t>(q), qh = static_cast<uint32_t>(q >> 32);
+  lane_swap<BIT>(pl, ql);
+  lane_swap<BIT>(ph, qh);
+  a = __builtin_bit_cast(double, (static_cast<uint64_t>(ph) << 32) | pl);
+  b = __builtin_bit_cast(double, (static_cast<uint64_t>(qh) << 32) | ql);
+}
+
+// the value of this lane's partner across lane bit BIT (8: the lane 8 further in its row of 16, 4: the mirrored lane of its 8)
+template <int BIT, typename T>
+__device__ __forceinline__ T lane_partner(T v) {
+  static_assert(BIT == 8 || BIT == 4 || BIT == 2 || BIT == 1, "lane bits inside a row of 16");
+  return dpp_move<BIT == 8 ? 0x128 : BIT == 4 ? 0x141 : BIT == 2 ? 0x4E : 0xB1>(v);
+}
+
+// One halving step of a sum over lanes: every lane holds its share of two sums before, of one after it - of `a` where lane bit
+// BIT is clear, of `b` where it is set.  n sums over 64 lanes take n - 1 such steps and, with fewer than 64, the plain steps
+// below for the lane bits that are left, where a butterfly per sum takes 6 n.
+template <int BIT, typename T>
+__device__ __forceinline__ T lane_fold(T a, T b, int lane) {
+  if constexpr (BIT >= 16) {
+    lane_swap<BIT>(a, b);
+    return a + b;
+  } else {
+    const bool set = lane & BIT;
+    return (set ? b : a) + lane_partner<BIT>(set ? a : b);
+  }
+}
+template <int BIT, typename T>
+__device__ __forceinline__ T lane_fold(T a) {
+  if constexpr (BIT >= 16) {
+    T b = a;
+    lane_swap<BIT>(a, b);
+    return a + b;
+  } else {
+    return a + lane_partner<BIT>(a);
+  }
+}
+
 // Sum over the 64 lanes, result valid in every lane.  Fixed butterfly: bit-reproducible.
 template <typename T>
 __device__ __forceinline__ T wave_sum(T v) {
-  v += dpp_move<0xB1>(v);   // quad_perm [1,0,3,2]
-  v += dpp_move<0x4E>(v);   // quad_perm [2,3,0,1]
-  v += dpp_move<0x141>(v);  // row_half_mirror
+  v = lane_fold<1>(v);
+  v = lane_fold<2>(v);
+  v = lane_fold<4>(v);
   v += dpp_move<0x140>(v);  // row_mirror: every lane holds its row's sum
-  v += __shfl_xor(v, 16, 64);
-  v += __shfl_xor(v, 32, 64);
-  return v;
+  v = lane_fold<16>(v);
+  return lane_fold<32>(v);
 }
 
 // ---- element types of the buffers ----------------------------------------------------------------
