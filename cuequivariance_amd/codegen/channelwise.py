@@ -8,15 +8,16 @@ tensor product takes after flattening the Clebsch-Gordan modes — i.e. for ever
 
 Output: HIP source with the path table unrolled into the instruction stream.
 
-Forward kernel (one wavefront = one output row x 64 channels):
+Forward kernel (one wavefront = one output row x 64 channels; where there are few rows, four or eight wavefronts of a block share
+the list of a row, ``fwd_parts`` in ``cw_common.h``, and add their sums in LDS):
   * channels across lanes, so every HBM access is a contiguous 256-byte (fp32) line;
   * the uniform factor ``c_p * x2[j_p]`` of each path lives in a table register: lane ``n`` of each
     16-lane row holds the factor of a path whose ``x2`` index is ``n``; the FMA reads it with the DPP
     ``row_newbcast:n`` modifier, which broadcasts lane ``n`` of every row to the row - no LDS traffic,
     no scalar float arithmetic, one VALU instruction per path;
   * ``w[b] * x1[i]`` is formed once per (block, i) and reused by all paths of the block;
-  * the batch rows that scatter into one output row are summed in registers in CSR order, then
-    stored once: deterministic, nothing of batch size is materialised.
+  * the batch rows that scatter into one output row are summed in registers in CSR order (parts of the list among
+    themselves in order), then stored once: deterministic, nothing of batch size is materialised.
 
 Backward kernel (one wavefront per resident slot, each owning a contiguous range of batch rows x 64
 channels) computes the three gradients in one pass over the inputs.  With ``G[b][i][j] = sum_k C[i,j,k] g[k]`` (literal
@@ -250,6 +251,10 @@ def _tables_for(blocks: Sequence[Block]):
     return slots, tables
 
 
+FWD_PARTS = 8   # most wavefronts that share the batch rows of one output row
+FWD_FOLD = 16   # segments of the output that meet in LDS at a time
+
+
 def emit_forward(st: ChannelwiseStructure, T: str, nsplit: int, waves_per_eu: int, ns: str, prefetch: bool = True) -> str:
     """HIP source of the forward kernels (one ``__device__`` body per block group) in namespace ``ns``."""
     fp = T
@@ -334,11 +339,15 @@ def emit_forward(st: ChannelwiseStructure, T: str, nsplit: int, waves_per_eu: in
                 A(f"{ind}}}")
 
         A(f"template <bool X1_IDX, bool W_SHARED>")
-        A(f"__device__ __forceinline__ void fwd_group{q}(FWD_PARAMS, const {fp}* s_c, const {fp}* s_sh, int64_t r, int lane, int uu, bool active) {{")
+        A(f"__device__ __forceinline__ void fwd_group{q}(FWD_PARAMS, const {fp}* s_c, const {fp}* s_sh, {fp}* s_fold, int64_t r, int lane, int uu, bool active, int part, int nparts) {{")
         for k in ks:
             A(f"  {fp} acc{k} = 0;")
         A("  int64_t z0, z1;")
         A("  if (csr_offsets) { z0 = csr_offsets[r]; z1 = csr_offsets[r + 1]; } else { z0 = r; z1 = r + 1; }")
+        A("  if (nparts > 1) {")
+        A("    const int64_t first = z0, count = z1 - z0;")
+        A("    z0 = first + count * part / nparts; z1 = first + count * (part + 1) / nparts;")
+        A("  }")
         A("  const int n16 = lane & 15;")
         sets = ("a", "b") if prefetch else ("a",)
         for S in sets:
@@ -371,23 +380,45 @@ def emit_forward(st: ChannelwiseStructure, T: str, nsplit: int, waves_per_eu: in
             load("a", "zz", "    ")
             body("a", "    ")
             A("  }")
-        A("  if (active) {")
-        A(f"    TI* __restrict__ op = out + r * {st.nseg_out * st.extent}ll;")
+        A(f"  TI* __restrict__ op = out + r * {st.nseg_out * st.extent}ll;")
+        A("  if (nparts == 1) {")
+        A("    if (active) {")
         for k in ks:
-            A(f"    io_stnt(acc{k}, op + ({st.out_at(k)}));")
+            A(f"      io_stnt(acc{k}, op + ({st.out_at(k)}));")
+        A("    }")
+        A("    return;")
         A("  }")
+        # the parts' sums meet in LDS, FWD_FOLD segments at a time; the wavefronts share the segments among them and add the
+        # parts in order
+        for c0 in range(0, len(ks), FWD_FOLD):
+            piece = ks[c0: c0 + FWD_FOLD]
+            if c0:
+                A("  __syncthreads();")
+            for n, k in enumerate(piece):
+                A(f"  s_fold[(part * {FWD_FOLD} + {n}) * 64 + lane] = acc{k};")
+            A("  __syncthreads();")
+            A("  if (nparts == 4) {")
+            for parts in (4, FWD_PARTS):
+                if parts == FWD_PARTS:
+                    A("  } else {")
+                for n, k in enumerate(piece):
+                    A(f"    if (part == {n % parts}) {{ const {fp} sum = fold_sum<{parts}>(s_fold + {n * 64} + lane, {FWD_FOLD * 64}); if (active) io_stnt(sum, op + ({st.out_at(k)})); }}")
+            A("  }")
         A("}")
         A("")
     # kernel
     nch = (st.extent + 63) // 64
     A("template <bool X1_IDX, bool W_SHARED>")
-    A(f"__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu({waves_per_eu}))) fwd_kernel(FWD_PARAMS) {{")
+    most = min(FWD_PARTS, 4 * waves_per_eu)  # wavefronts of a block that are resident together
+    A(f"__global__ void __launch_bounds__({64 * most}) __attribute__((amdgpu_waves_per_eu({waves_per_eu}))) fwd_kernel(FWD_PARAMS) {{")
+    A(f"  extern __shared__ __align__(16) unsigned char fwd_shared[];  // (blocks of one wavefront have none)")
+    A(f"  {fp}* s_fold = reinterpret_cast<{fp}*>(fwd_shared);")
     A(f"  __shared__ {fp} s_c[{max(1, len(all_tables)) * 16}];")
-    A("  const int lane = threadIdx.x;")
-    A(f"  for (int i = lane; i < {len(all_tables) * 16}; i += 64) s_c[i] = fwd_ctab[i];")
+    A("  const int lane = threadIdx.x & 63, nparts = blockDim.x >> 6, part = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);")
+    A(f"  for (int i = threadIdx.x; i < {len(all_tables) * 16}; i += blockDim.x) s_c[i] = fwd_ctab[i];")
     if st.harmonics:
         A(f"  __shared__ {fp} s_sh[{npad * NM}];")
-        A(f"  for (int i = lane; i < {npad * NM}; i += 64) s_sh[i] = fwd_shtab[i];")
+        A(f"  for (int i = threadIdx.x; i < {npad * NM}; i += blockDim.x) s_sh[i] = fwd_shtab[i];")
     else:
         A(f"  const {fp}* s_sh = nullptr;")
     A("  __syncthreads();")
@@ -400,10 +431,12 @@ def emit_forward(st: ChannelwiseStructure, T: str, nsplit: int, waves_per_eu: in
         A(f"  const int u = ch * 64 + lane; const bool active = u < {st.extent}; const int uu = active ? u : 0;")
     A("  switch (q) {")
     for q in range(nsplit):
-        A(f"    case {q}: fwd_group{q}<X1_IDX, W_SHARED>(FWD_ARGS, s_c, s_sh, r, lane, uu, active); break;")
+        A(f"    case {q}: fwd_group{q}<X1_IDX, W_SHARED>(FWD_ARGS, s_c, s_sh, s_fold, r, lane, uu, active, part, nparts); break;")
     A("  }")
     A("}")
     A(f"constexpr int kFwdSplit = {nsplit};")
+    A(f"constexpr int kFwdWaves = {waves_per_eu};")
+    A(f"constexpr int kFwdParts = {most};          // most wavefronts that share the list of a row")
     A(f"constexpr int kChunks = {nch};")
     return "\n".join(L)
 
@@ -456,7 +489,7 @@ def emit_slot_of_lane(A, ind: str, name: str, n: int, lanes: int):
     A(f"{ind}}}")
 
 
-def emit_backward(st: ChannelwiseStructure, T: str, waves_per_eu: int, chunk: int, prefetch: bool = False, nsplit: int = 1) -> str:
+def emit_backward(st: ChannelwiseStructure, T: str, waves_per_eu: int, prefetch: bool = False, nsplit: int = 1) -> str:
     """HIP source of the fused backward kernel (dw, dx1, dx2 in one pass).
 
     ``nsplit`` > 1 deals the blocks out to that many wavefronts per (range of batch rows, 64 channels) with disjoint x1
@@ -688,7 +721,6 @@ def emit_backward(st: ChannelwiseStructure, T: str, waves_per_eu: int, chunk: in
         A(f"    case {q}: bwd_group{q}<X1_IDX, G_IDX, ATOMIC_DX1>(BWD_ARGS, z0, z1, lane, uu, active, ch); break;")
     A("  }")
     A("}")
-    A(f"constexpr int kBwdMinRange = {chunk};   // fewest batch rows worth a wavefront of their own")
     A(f"constexpr int kBwdWaves = {waves_per_eu};")
     A(f"constexpr int kBwdSplit = {nsplit};")
     A(f"constexpr int kBwdParts = {nparts};     // partial rows of the x2 gradient per batch row")
@@ -725,7 +757,7 @@ def io_type(T: str, io) -> tuple:
 
 
 def emit_unit(st: ChannelwiseStructure, T: str, name: str, fwd_hash: int, bwd_hash: int, *, fwd_split: int = 1,
-              fwd_waves: int = 2, fwd_prefetch: bool = True, bwd_waves: int = 2, bwd_chunk: int = 16,
+              fwd_waves: int = 2, fwd_prefetch: bool = True, bwd_waves: int = 2,
               bwd_prefetch: bool = False, bwd_split: int = 1, io=None) -> str:
     """Complete .hip translation unit: kernels, host launchers, registration under both table hashes.  ``io``: element type
     of the buffers when it is not the arithmetic type ``T`` ("bf16" / "f16" with ``T`` = float)."""
@@ -754,7 +786,7 @@ def emit_unit(st: ChannelwiseStructure, T: str, name: str, fwd_hash: int, bwd_ha
     A("")
     A(emit_forward(st, T, fwd_split, fwd_waves, ns, fwd_prefetch))
     A("")
-    A(emit_backward(st, T, bwd_waves, bwd_chunk, bwd_prefetch, bwd_split))
+    A(emit_backward(st, T, bwd_waves, bwd_prefetch, bwd_split))
     A("")
     same = "true" if io is None else "false"
     A(f"""
@@ -780,9 +812,11 @@ static int run_fwd(const SpecCall& c) {{
   TI* o = static_cast<TI*>(b[3].data);
   const int64_t* offs = out_idx ? b[3].csr_offsets : nullptr;
   const int64_t* perm = out_idx ? b[3].csr_perm : nullptr;
-  const dim3 g(static_cast<unsigned>(grid)), t(64);
+  const int nparts = out_idx ? fwd_parts(grid, c.batch, rows, kFwdWaves, kFwdParts) : 1;
+  const dim3 g(static_cast<unsigned>(grid)), t(64 * nparts);
+  const unsigned shared = nparts > 1 ? nparts * {FWD_FOLD * 64}u * sizeof({T}) : 0u;
   KernelTimer timer("{name}_fwd_{tag}", c.stream);
-#define LAUNCH_FWD(XI, WS) hipLaunchKernelGGL((fwd_kernel<XI, WS>), g, t, 0, c.stream, w, x1, x2, o, b[1].index, b[1].index_is_64, offs, perm)
+#define LAUNCH_FWD(XI, WS) hipLaunchKernelGGL((fwd_kernel<XI, WS>), g, t, shared, c.stream, w, x1, x2, o, b[1].index, b[1].index_is_64, offs, perm)
   if (x1_idx && w_shared) LAUNCH_FWD(true, true);
   else if (x1_idx) LAUNCH_FWD(true, false);
   else if (w_shared) LAUNCH_FWD(false, true);
@@ -844,10 +878,12 @@ static int run_bwd(const SpecCall& c) {{
     CUEQ_CHECK_HIP(hipGetLastError());
   }}
   if (batch > 0) {{
-    // one launch round of resident wavefronts; short batches get fewer, not shorter than kBwdMinRange rows
+    // one launch round of resident wavefronts, or a wavefront per batch row where there are fewer: a row more in the same
+    // wavefront costs 1.5 us, loading the cotangent row once more next to nothing (us with ranges of at least 16 / 8 / 2 / 1 rows,
+    // fp32: 32 ch l <= 2, 622 rows 24.3 / 13.2 / 5.4 / 4.4, 5 000 rows 30 / 17 / 12 / 12; 128 ch l <= 3, 1 000 rows 56 / 31 / 17 / 18,
+    // 12 000 rows 100 / 104 / 103 / 103)
     int64_t nranges = wave_slots(kBwdWaves) / kBwdParts;
-    const int64_t most = (batch + kBwdMinRange - 1) / kBwdMinRange;
-    if (nranges > most) nranges = most;
+    if (nranges > batch) nranges = batch;
     if (nranges < 1) nranges = 1;
     const int64_t grid = nranges * kBwdParts;
     const dim3 gd(static_cast<unsigned>(grid)), t(64);
