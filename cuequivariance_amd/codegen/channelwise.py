@@ -8,7 +8,7 @@ tensor product takes after flattening the Clebsch-Gordan modes — i.e. for ever
 
 Output: HIP source with the path table unrolled into the instruction stream.
 
-Forward kernel (one wavefront = one output row x 64 channels; where there are few rows, four or eight wavefronts of a block share
+Forward kernel (one wavefront = one output row x 64 channels, for 32 channels and fewer two or four batch rows at a time; where there are few rows, four or eight wavefronts of a block share
 the list of a row, ``fwd_parts`` in ``cw_common.h``, and add their sums in LDS):
   * channels across lanes, so every HBM access is a contiguous 256-byte (fp32) line;
   * the uniform factor ``c_p * x2[j_p]`` of each path lives in a table register: lane ``n`` of each
@@ -116,6 +116,14 @@ class ChannelwiseStructure:
     @property
     def num_paths(self):
         return sum(len(b.entries) for b in self.blocks)
+
+    @property
+    def packed(self) -> int:
+        """Batch rows a wavefront works on at a time: two (four) where 32 (16) lanes hold every channel of a row.  Each takes a whole
+        number of the 16-lane rows that DPP works in, so broadcasts and sums stay among its own lanes.  (With one batch row per
+        wavefront half the lanes or more were idle, and the masks around them cost registers: 32 ch, forward + backward,
+        l <= 2 fp32 60 000 edges 119 -> 102 us, l <= 3 fp64 30 000 edges 1 532 (spills) -> 228, l <= 3 bfloat16 2 517 edges 93 -> 79.)"""
+        return 4 if self.extent <= 16 else 2 if self.extent <= 32 else 1
 
     def _at(self, layout, seg: int) -> str:
         """Element offset of (segment, this lane's channel ``uu``) inside a row, as a C expression."""
@@ -252,12 +260,28 @@ def _tables_for(blocks: Sequence[Block]):
 
 
 FWD_PARTS = 8   # most wavefronts that share the batch rows of one output row
-FWD_FOLD = 16   # segments of the output that meet in LDS at a time
+FWD_FOLD = 16   # registers of output sums that meet in LDS at a time
+
+
+def emit_lanes(A, st: ChannelwiseStructure):
+    """The lane's channel ``uu``, whether it has one (``active``), and which of the wavefront's batch rows it works on (``sub``)."""
+    if st.packed > 1:
+        lanes = 64 // st.packed
+        A(f"  const int sub = lane / {lanes};")
+        if st.extent == lanes:
+            A(f"  const int uu = lane & {lanes - 1}; constexpr bool active = true;")
+        else:
+            A(f"  const int u = lane & {lanes - 1}; const bool active = u < {st.extent}; const int uu = active ? u : 0;")
+    elif st.extent % 64 == 0:
+        A("  constexpr int sub = 0; const int uu = ch * 64 + lane; constexpr bool active = true;")
+    else:
+        A(f"  constexpr int sub = 0; const int u = ch * 64 + lane; const bool active = u < {st.extent}; const int uu = active ? u : 0;")
 
 
 def emit_forward(st: ChannelwiseStructure, T: str, nsplit: int, waves_per_eu: int, ns: str, prefetch: bool = True) -> str:
     """HIP source of the forward kernels (one ``__device__`` body per block group) in namespace ``ns``."""
     fp = T
+    P = st.packed
     dpp = "v_fmac_f32_dpp" if T == "float" else "v_fmac_f64_dpp"
     groups = _split_blocks(st, nsplit)
     nsplit = len(groups)
@@ -339,14 +363,16 @@ def emit_forward(st: ChannelwiseStructure, T: str, nsplit: int, waves_per_eu: in
                 A(f"{ind}}}")
 
         A(f"template <bool X1_IDX, bool W_SHARED>")
-        A(f"__device__ __forceinline__ void fwd_group{q}(FWD_PARAMS, const {fp}* s_c, const {fp}* s_sh, {fp}* s_fold, int64_t r, int lane, int uu, bool active, int part, int nparts) {{")
+        A(f"__device__ __forceinline__ void fwd_group{q}(FWD_PARAMS, const {fp}* s_c, const {fp}* s_sh, {fp}* s_fold, int64_t r, int lane, int sub, int uu, bool active, int part, int nparts) {{")
         for k in ks:
             A(f"  {fp} acc{k} = 0;")
         A("  int64_t z0, z1;")
         A("  if (csr_offsets) { z0 = csr_offsets[r]; z1 = csr_offsets[r + 1]; } else { z0 = r; z1 = r + 1; }")
-        A("  if (nparts > 1) {")
+        A("  if (nparts > 1) {" if P == 1 else "  {")
         A("    const int64_t first = z0, count = z1 - z0;")
-        A("    z0 = first + count * part / nparts; z1 = first + count * (part + 1) / nparts;")
+        share = "part" if P == 1 else f"(part * {P} + sub)"
+        A(f"    const int shift = 31 - __builtin_clz(nparts * {P});  // (a power of two)")
+        A(f"    z0 = first + ((count * {share}) >> shift); z1 = first + ((count * ({share} + 1)) >> shift);")
         A("  }")
         A("  const int n16 = lane & 15;")
         sets = ("a", "b") if prefetch else ("a",)
@@ -381,28 +407,49 @@ def emit_forward(st: ChannelwiseStructure, T: str, nsplit: int, waves_per_eu: in
             body("a", "    ")
             A("  }")
         A(f"  TI* __restrict__ op = out + r * {st.nseg_out * st.extent}ll;")
+        # registers to store: a segment each; with several batch rows per wavefront, the sums over them are halved among their
+        # lanes, so that a register ends with a segment per group of lanes
+        totals = [(f"acc{k}", [k]) for k in ks]
+        for bit in {1: (), 2: (32,), 4: (16, 32)}[P]:  # (segment n of a register ends in the lanes of group n)
+            nxt = []
+            for n in range(0, len(totals), 2):
+                name = f"sum{bit}_{n // 2}"
+                pair = totals[n: n + 2]
+                A(f"  const {fp} {name} = lane_fold<{bit}>(" + ", ".join(t for t, _ in pair) + (", lane);" if len(pair) == 2 else ");"))
+                pad = [None] * len(pair[0][1])
+                nxt.append((name, pair[0][1] + (pair[1][1] if len(pair) == 2 else pad)))
+            totals = nxt
+
+        def store(value: str, segs: list) -> str:
+            """The store of a register by the group(s) of lanes that hold a segment."""
+            where, guard = st.out_at(segs[0]), ["active"]
+            for n in range(1, len(segs)):  # (segment n of a register is in the lanes of group n)
+                if segs[n] is not None:
+                    where = f"(sub == {n} ? {st.out_at(segs[n])} : {where})"
+            missing = [n for n in range(len(segs)) if segs[n] is None]
+            guard += [f"sub != {n}" for n in missing]
+            return f"if ({' && '.join(guard)}) io_stnt({value}, op + ({where}));"
+
         A("  if (nparts == 1) {")
-        A("    if (active) {")
-        for k in ks:
-            A(f"      io_stnt(acc{k}, op + ({st.out_at(k)}));")
-        A("    }")
+        for name, segs in totals:
+            A(f"    {store(name, segs)}")
         A("    return;")
         A("  }")
-        # the parts' sums meet in LDS, FWD_FOLD segments at a time; the wavefronts share the segments among them and add the
+        # the parts' sums meet in LDS, FWD_FOLD registers at a time; the wavefronts share the registers among them and add the
         # parts in order
-        for c0 in range(0, len(ks), FWD_FOLD):
-            piece = ks[c0: c0 + FWD_FOLD]
+        for c0 in range(0, len(totals), FWD_FOLD):
+            piece = totals[c0: c0 + FWD_FOLD]
             if c0:
                 A("  __syncthreads();")
-            for n, k in enumerate(piece):
-                A(f"  s_fold[(part * {FWD_FOLD} + {n}) * 64 + lane] = acc{k};")
+            for n, (name, _) in enumerate(piece):
+                A(f"  s_fold[(part * {FWD_FOLD} + {n}) * 64 + lane] = {name};")
             A("  __syncthreads();")
             A("  if (nparts == 4) {")
             for parts in (4, FWD_PARTS):
                 if parts == FWD_PARTS:
                     A("  } else {")
-                for n, k in enumerate(piece):
-                    A(f"    if (part == {n % parts}) {{ const {fp} sum = fold_sum<{parts}>(s_fold + {n * 64} + lane, {FWD_FOLD * 64}); if (active) io_stnt(sum, op + ({st.out_at(k)})); }}")
+                for n, (_, segs) in enumerate(piece):
+                    A(f"    if (part == {n % parts}) {{ const {fp} sum = fold_sum<{parts}>(s_fold + {n * 64} + lane, {FWD_FOLD * 64}); {store('sum', segs)} }}")
             A("  }")
         A("}")
         A("")
@@ -425,15 +472,13 @@ def emit_forward(st: ChannelwiseStructure, T: str, nsplit: int, waves_per_eu: in
     A("  int64_t wid = blockIdx.x;")
     A(f"  const int q = static_cast<int>(wid % {nsplit}); wid /= {nsplit};")
     A(f"  const int ch = static_cast<int>(wid % {nch}); const int64_t r = wid / {nch};")
-    if st.extent % 64 == 0:
-        A("  const int uu = ch * 64 + lane; constexpr bool active = true;")
-    else:
-        A(f"  const int u = ch * 64 + lane; const bool active = u < {st.extent}; const int uu = active ? u : 0;")
+    emit_lanes(A, st)
     A("  switch (q) {")
     for q in range(nsplit):
-        A(f"    case {q}: fwd_group{q}<X1_IDX, W_SHARED>(FWD_ARGS, s_c, s_sh, s_fold, r, lane, uu, active, part, nparts); break;")
+        A(f"    case {q}: fwd_group{q}<X1_IDX, W_SHARED>(FWD_ARGS, s_c, s_sh, s_fold, r, lane, sub, uu, active, part, nparts); break;")
     A("  }")
     A("}")
+    A(f"constexpr int kPacked = {P};             // batch rows a wavefront works on at a time")
     A(f"constexpr int kFwdSplit = {nsplit};")
     A(f"constexpr int kFwdWaves = {waves_per_eu};")
     A(f"constexpr int kFwdParts = {most};          // most wavefronts that share the list of a row")
@@ -507,6 +552,7 @@ def emit_backward(st: ChannelwiseStructure, T: str, waves_per_eu: int, prefetch:
     groups = _split_blocks(st, nsplit)
     nsplit = len(groups)
     nparts = nch * nsplit
+    P, lanes = st.packed, 64 // st.packed
     i_all = sorted({i for blk in st.blocks for i in blk.i_list})
     w_all = sorted({blk.b for blk in st.blocks})
     A(f"// backward: fused dw / dx1 / dx2; every wavefront owns one contiguous, equally sized range of batch rows; the blocks are")
@@ -527,9 +573,9 @@ def emit_backward(st: ChannelwiseStructure, T: str, waves_per_eu: int, prefetch:
             first += d
         staged_segments = {i for i0, d in staged for i in range(i0, i0 + d)}
 
-        # the second operand's gradient, in pieces of at most 64 sums over the lanes
+        # the second operand's gradient, in pieces of as many sums as a batch row has lanes
         d2_names = [f"dv{a}" for a in range(3)] if st.harmonics else [f"pj{j}" if j in j_used else f"{fp}(0)" for j in range(st.nseg_x2)]
-        d2_pieces = [(c0, d2_names[c0: c0 + 64]) for c0 in range(0, len(d2_names), 64)]
+        d2_pieces = [(c0, d2_names[c0: c0 + lanes]) for c0 in range(0, len(d2_names), lanes)]
 
         def load(S: str, zz: str, ind: str):
             A(f"{ind}{{")
@@ -614,9 +660,10 @@ def emit_backward(st: ChannelwiseStructure, T: str, waves_per_eu: int, prefetch:
                 for c in range(d):
                     A(f"{ind}  dxs[lane * {d} + {c}] = dxa{i0 + c};")
                 A(f"{ind}  __builtin_amdgcn_wave_barrier();")
+                own, base = ("lane", "") if P == 1 else (f"(lane & {lanes - 1})", f"sub * {lanes * d} + ")
                 for k in range(d):
-                    guard = "" if st.extent % 64 == 0 else f"if (ch * {64 * d} + {k * 64} + lane < {st.extent * d}) "
-                    A(f"{ind}  {guard}unsafeAtomicAdd(dp + {k * 64} + lane, dxs[{k * 64} + lane]);")
+                    guard = "" if st.extent % lanes == 0 else f"if (ch * {64 * d} + {k * lanes} + {own} < {st.extent * d}) "
+                    A(f"{ind}  {guard}unsafeAtomicAdd(dp + {k * lanes} + {own}, dxs[{base}{k * lanes} + {own}]);")
                 A(f"{ind}}}")
             A(f"{ind}if (active) {{")
             A(f"{ind}  if (ATOMIC_DX1) {{")
@@ -658,15 +705,15 @@ def emit_backward(st: ChannelwiseStructure, T: str, waves_per_eu: int, prefetch:
             else:
                 A(f"{ind}{fp}* __restrict__ d2 = dx2_partial + (z * {nparts} + ch * {nsplit} + {q}) * {st.x2_width}ll;")
             for c0, names in d2_pieces:
-                total = emit_lane_sums(A, ind, fp, names, 64, f"r{c0}_")
+                total = emit_lane_sums(A, ind, fp, names, lanes, f"r{c0}_")
                 A(f"{ind}if (slot{len(names)} >= 0) io_st({total}, d2 + {c0} + slot{len(names)});")
 
         A("template <bool X1_IDX, bool G_IDX, bool ATOMIC_DX1>")
-        A(f"__device__ __forceinline__ void bwd_group{q}(BWD_PARAMS, int64_t z0, int64_t z1, int lane, int uu, bool active, int ch) {{")
+        A(f"__device__ __forceinline__ void bwd_group{q}(BWD_PARAMS, int64_t z0, int64_t z1, int lane, int sub, int uu, bool active, int ch) {{")
         if staged:
             A(f"  __shared__ {fp} dxs[{64 * max(d for _, d in staged)}];")
         for n in sorted({len(names) for _, names in d2_pieces}):
-            emit_slot_of_lane(A, "  ", f"slot{n}", n, 64)
+            emit_slot_of_lane(A, "  ", f"slot{n}", n, lanes)
         for k in ks:
             A(f"  {fp} gr{k} = 0;")
         A("  int64_t grow_cur = -1;")
@@ -710,15 +757,13 @@ def emit_backward(st: ChannelwiseStructure, T: str, waves_per_eu: int, prefetch:
     A("  int64_t wid = blockIdx.x;")
     A(f"  const int q = static_cast<int>(wid % {nsplit}); wid /= {nsplit};")
     A(f"  const int ch = static_cast<int>(wid % {nch}); const int64_t cid = wid / {nch};")
-    if st.extent % 64 == 0:
-        A("  const int uu = ch * 64 + lane; constexpr bool active = true;")
-    else:
-        A(f"  const int u = ch * 64 + lane; const bool active = u < {st.extent}; const int uu = active ? u : 0;")
-    A(f"  const int64_t nranges = gridDim.x / {nparts};")
-    A("  const int64_t z0 = cid * batch / nranges, z1 = (cid + 1) * batch / nranges;")
+    emit_lanes(A, st)
+    A("  // (ranges of `range` batch rows, the first `longer` of them one row longer)")
+    A(f"  const int64_t rid = cid{'' if P == 1 else f' * {P} + sub'};")
+    A("  const int64_t z0 = rid * range + (rid < longer ? rid : longer), z1 = z0 + range + (rid < longer ? 1 : 0);")
     A("  switch (q) {")
     for q in range(nsplit):
-        A(f"    case {q}: bwd_group{q}<X1_IDX, G_IDX, ATOMIC_DX1>(BWD_ARGS, z0, z1, lane, uu, active, ch); break;")
+        A(f"    case {q}: bwd_group{q}<X1_IDX, G_IDX, ATOMIC_DX1>(BWD_ARGS, z0, z1, lane, sub, uu, active, ch); break;")
     A("  }")
     A("}")
     A(f"constexpr int kBwdWaves = {waves_per_eu};")
@@ -735,12 +780,12 @@ FWD_PARAMS = ("const TI* __restrict__ w, const TI* __restrict__ x1, const TI* __
               "const void* __restrict__ x1_index, int x1_idx64, const int64_t* __restrict__ csr_offsets, "
               "const int64_t* __restrict__ csr_perm")
 FWD_ARGS = "w, x1, x2, out, x1_index, x1_idx64, csr_offsets, csr_perm"
-BWD_ARGS = "w, x1, x2, g, dw, dx1, dx1_partial, dx2, dx2_partial, x1_index, x1_idx64, g_index, g_idx64, batch"
+BWD_ARGS = "w, x1, x2, g, dw, dx1, dx1_partial, dx2, dx2_partial, x1_index, x1_idx64, g_index, g_idx64, range, longer"
 # (dx1: sums by atomic additions, dx2_partial: partial rows - both in the arithmetic type; everything else holds TI)
 BWD_PARAMS = ("const TI* __restrict__ w, const TI* __restrict__ x1, const TI* __restrict__ x2, const TI* __restrict__ g, "
               "TI* __restrict__ dw, {T}* dx1, TI* __restrict__ dx1_partial, TI* __restrict__ dx2, "
               "{T}* __restrict__ dx2_partial, const void* __restrict__ x1_index, int x1_idx64, "
-              "const void* __restrict__ g_index, int g_idx64, int64_t batch")
+              "const void* __restrict__ g_index, int g_idx64, int64_t range, int64_t longer")
 
 
 IO_TYPES = {"bf16": ("bf16_t", "CUEQ_BF16"), "f16": ("f16_t", "CUEQ_F16")}
@@ -812,7 +857,7 @@ static int run_fwd(const SpecCall& c) {{
   TI* o = static_cast<TI*>(b[3].data);
   const int64_t* offs = out_idx ? b[3].csr_offsets : nullptr;
   const int64_t* perm = out_idx ? b[3].csr_perm : nullptr;
-  const int nparts = out_idx ? fwd_parts(grid, c.batch, rows, kFwdWaves, kFwdParts) : 1;
+  const int nparts = out_idx ? fwd_parts(grid, c.batch / kPacked, rows, kFwdWaves, kFwdParts) : 1;
   const dim3 g(static_cast<unsigned>(grid)), t(64 * nparts);
   const unsigned shared = nparts > 1 ? nparts * {FWD_FOLD * 64}u * sizeof({T}) : 0u;
   KernelTimer timer("{name}_fwd_{tag}", c.stream);
@@ -883,13 +928,14 @@ static int run_bwd(const SpecCall& c) {{
     // fp32: 32 ch l <= 2, 622 rows 24.3 / 13.2 / 5.4 / 4.4, 5 000 rows 30 / 17 / 12 / 12; 128 ch l <= 3, 1 000 rows 56 / 31 / 17 / 18,
     // 12 000 rows 100 / 104 / 103 / 103)
     int64_t nranges = wave_slots(kBwdWaves) / kBwdParts;
-    if (nranges > batch) nranges = batch;
+    if (nranges > (batch + kPacked - 1) / kPacked) nranges = (batch + kPacked - 1) / kPacked;
     if (nranges < 1) nranges = 1;
+    const int64_t range = batch / (nranges * kPacked), longer = batch % (nranges * kPacked);
     const int64_t grid = nranges * kBwdParts;
     const dim3 gd(static_cast<unsigned>(grid)), t(64);
     {{
     KernelTimer timer("{name}_bwd_{tag}", c.stream);
-#define LAUNCH_BWD(XI, GI, AT) hipLaunchKernelGGL((bwd_kernel<XI, GI, AT>), gd, t, 0, c.stream, w, x1, x2, g, dw, dx1_sums, dx1_partial, dx2, dx2_partial, b[1].index, b[1].index_is_64, b[3].index, b[3].index_is_64, batch)
+#define LAUNCH_BWD(XI, GI, AT) hipLaunchKernelGGL((bwd_kernel<XI, GI, AT>), gd, t, 0, c.stream, w, x1, x2, g, dw, dx1_sums, dx1_partial, dx2, dx2_partial, b[1].index, b[1].index_is_64, b[3].index, b[3].index_is_64, range, longer)
     if (x1_idx && g_idx && atomic) LAUNCH_BWD(true, true, true);
     else if (x1_idx && g_idx) LAUNCH_BWD(true, true, false);
     else if (x1_idx && atomic) LAUNCH_BWD(true, false, true);
