@@ -410,6 +410,7 @@ def emit_forward(st: ChannelwiseStructure, T: str, nsplit: int, waves_per_eu: in
         # registers to store: a segment each; with several batch rows per wavefront, the sums over them are halved among their
         # lanes, so that a register ends with a segment per group of lanes
         totals = [(f"acc{k}", [k]) for k in ks]
+        k_zero = [k for k in range(st.nseg_out) if q == 0 and not any(k in blk.k_list for blk in st.blocks)]  # (no path fills them)
         for bit in {1: (), 2: (32,), 4: (16, 32)}[P]:  # (segment n of a register ends in the lanes of group n)
             nxt = []
             for n in range(0, len(totals), 2):
@@ -430,6 +431,9 @@ def emit_forward(st: ChannelwiseStructure, T: str, nsplit: int, waves_per_eu: in
             guard += [f"sub != {n}" for n in missing]
             return f"if ({' && '.join(guard)}) io_stnt({value}, op + ({where}));"
 
+        for k in k_zero:
+            own = ["part == 0"] + (["sub == 0"] if P > 1 else []) + ["active"]
+            A(f"  if ({' && '.join(own)}) io_stnt({fp}(0), op + ({st.out_at(k)}));")
         A("  if (nparts == 1) {")
         for name, segs in totals:
             A(f"    {store(name, segs)}")

@@ -66,3 +66,35 @@ def test_lists_shared_by_wavefronts_128_channels(device, lists, dtype):
 def test_lists_shared_by_wavefronts_few_channels(device, jit_on, name, dtype, layout):
     for lists in ("one row", "eight parts", "four parts", "one batch row"):
         _case(device, name, LISTS[lists], dtype, layout, ordered=lists != "four parts")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("extent", [70, 32, 16])
+@pytest.mark.parametrize("degrees", [[1, 0, 3] * 30, [100, 0, 33, 1, 700]])
+def test_output_segments_that_no_path_fills_are_zero(device, jit_on, degrees, extent):
+    """w[u] x1[u] x2[] -> out[u] with one of twelve output segments in no path: zero, not what the memory held."""
+    from cuequivariance_amd import _lib
+    from cuequivariance_amd.cuet.uniform_1d import Uniform1dPlan, run_plan
+    from cuequivariance_amd.tables import U1dTables
+
+    E, Z, N = extent, sum(degrees), len(degrees)
+    paths = [(k % 3, (k + 1) % 2, k % 4, k if k < 5 else k + 1, 0.5 + k) for k in range(11)]
+    tables = U1dTables.make(E, 3, 1, [1, 1, 0, 1], [3, 2, 4, 12], [0, 1, 2, -1], [4], [0, 1, 2, 3], [11], [0], [0],
+                            [i for p in paths for i in p[:4]], [p[4] for p in paths])
+    plan = Uniform1dPlan(tables, torch.float32, name="unfilled")
+    g = torch.Generator().manual_seed(0)
+    rows = torch.repeat_interleave(torch.arange(N, dtype=torch.int32), torch.tensor(degrees))
+    args = [torch.randn(Z, n, generator=g).to(device) for n in (3 * E, 2 * E, 4)] + [rows.to(device)]
+    B, I = _lib.BATCH_DIM_BATCHED, _lib.BATCH_DIM_INDEXED
+
+    def run():
+        return run_plan(plan, [B, B, B, I], [-1, -1, -1, 0, N], Z, 1, args)[0]
+
+    want = run().clone()
+    assert plan.specialised(device)
+    full = [torch.full((N, 12 * E), float("nan"), device=device) for _ in range(4)]  # (the memory of the next output)
+    del full
+    got = run().reshape(N, 12, E)
+    assert (got[:, 5] == 0).all()
+    others = [k for k in range(12) if k != 5]
+    assert torch.equal(got[:, others], want.reshape(N, 12, E)[:, others])
