@@ -257,6 +257,22 @@ __device__ __forceinline__ T fold_sum(const T* p, int stride) {
   return v[0];
 }
 
+template <typename T>
+__device__ __forceinline__ T fold_sum_of(int n, const T* p, int stride) {  // n: 2, 4, 8 or 16
+  return n == 16 ? fold_sum<16>(p, stride) : n == 8 ? fold_sum<8>(p, stride) : n == 4 ? fold_sum<4>(p, stride) : fold_sum<2>(p, stride);
+}
+
+// Wavefronts of a block that share the list of an output row (general kernels: one load after the other, 2 us a batch element,
+// so more wavefronts help until the chip is full of them).  Second derivative of a channel-wise product, 64 ch l <= 1 with l <= 3, us
+// for 1 / 2 / 4 / 8 / 16 parts: 451 rows of 20 elements 44 / 26 / 17 / 16 / 18, 56 rows of 24 38 / 21 / 14 / 10 / 8, 1 500 rows of 13
+// 42 / 36 / 33 / 32 / 36; of a product basis (a row per chemical element), 10 rows of 150 267 / 136 / 71 / 41 / 37.
+inline int row_parts(int64_t grid, int64_t batch, int64_t rows, int most) {
+  const int64_t slots = wave_slots(8);
+  int n = 1;
+  while (n < most && grid * n * 2 <= slots && batch >= 2 * n * rows) n *= 2;
+  return n;
+}
+
 // Wavefronts of a block that share the list of an output row (forward of a channel-wise product; `grid` = blocks, `most` = 8, or 4
 // where a SIMD holds one wavefront).  A list is a serial chain of about 1 us an element, and few rows leave the chip idle:
 // eight parts while they all are resident together, four while the blocks are at most three quarters of the slots, and no part
