@@ -185,4 +185,5 @@ PYBIND11_MODULE(_host, m) {
   bind_triangle(m);
   bind_linear(m);
   bind_fully_connected(m);
+  bind_rows(m);
 }

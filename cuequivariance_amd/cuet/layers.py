@@ -19,7 +19,7 @@ from typing import Optional, Sequence, Union
 import torch
 from torch import nn
 
-from .. import cue
+from .. import _lib, cue
 from .operations import FullyConnectedTensorProduct, _assert_same_group, _default_irreps, _default_layout
 
 __all__ = ["BatchNorm", "FullyConnectedTensorProductConv"]
@@ -206,8 +206,13 @@ class FullyConnectedTensorProductConv(nn.Module):
             edge_sh = edge_sh * edge_envelope.view(-1, 1)
         out = self.tp(src_features, edge_sh, weights, indices_1=src, indices_out=dst, size_out=num_dst_nodes)
         if reduce == "mean":
-            degree = torch.bincount(dst.long(), minlength=num_dst_nodes).clamp(min=1)
-            out = out / degree.to(out.dtype).unsqueeze(1)
+            mean = None
+            if not (torch.compiler.is_compiling() or torch.jit.is_tracing()) and type(out) is torch.Tensor and type(dst) is torch.Tensor and out.is_cuda:
+                mean = _lib.host().rows_mean(out, dst)  # (the degrees are in the grouping that the product made of the same ids)
+            if mean is None:
+                degree = torch.bincount(dst.long(), minlength=num_dst_nodes).clamp(min=1)
+                mean = out / degree.to(out.dtype).unsqueeze(1)
+            out = mean
         if self.batch_norm is not None:
             out = self.batch_norm(out)
         return out

@@ -476,6 +476,10 @@ int cueq_linear_flex_dw(int32_t dtype, int64_t rows, const void* X, int64_t ldx,
 int cueq_sum_runs(const float* partial, int32_t per, int32_t nruns, const int32_t* first, const int64_t* w0, int32_t out_dtype,
                   void* out, void* stream);
 
+/* out[r, :] = in[r, :] / max(1, offsets[r + 1] - offsets[r]): the mean over the batch rows that the grouping `offsets` (rows + 1
+ * device integers, cueq_segment_csr_build) puts on every row.  Any CUEQ_* element type; float64 computes in float64. */
+int cueq_rows_mean(int32_t dtype, int64_t rows, int64_t width, const void* in, const int64_t* offsets, void* out, void* stream);
+
 /* Fully connected product with shared weights and a second operand of multiplicity one, table-driven, for batches that do not
  * fill the chip with the generated kernels and for extents those do not take.  gradient == 0: rows of x1 against the weights;
  * 1: rows of the cotangent against the weights read transposed - with X1, partial (column_tiles x rows x n2 floats) and dX2
