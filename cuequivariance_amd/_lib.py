@@ -80,6 +80,7 @@ EXPORTED_SYMBOLS = (
     "cueq_linear_flex_dw",
     "cueq_sum_runs",
     "cueq_rows_mean",
+    "cueq_normalize3",
     "cueq_fc_flex",
     "cueq_fc_flex_dw_chunks",
     "cueq_fc_flex_dw",
@@ -298,6 +299,8 @@ def load() -> C.CDLL:
         lib.cueq_sum_runs.restype = C.c_int
         lib.cueq_rows_mean.argtypes = [i32, i64, i64, ptr, ptr, ptr, ptr]
         lib.cueq_rows_mean.restype = C.c_int
+        lib.cueq_normalize3.argtypes = [i32, i32, i64, ptr, ptr, ptr, C.c_double, ptr, ptr, ptr]
+        lib.cueq_normalize3.restype = C.c_int
         lib.cueq_fc_flex.argtypes = [i32, i32, i32, i32, i64, ptr, i64, ptr, ptr, i64, ptr, i64, ptr, i64, ptr, i32, ptr, ptr, i32, i32, i32, ptr, ptr, ptr]
         lib.cueq_fc_flex.restype = C.c_int
         lib.cueq_fc_pack.argtypes = [i32, ptr, ptr, ptr, i32, i64, ptr]

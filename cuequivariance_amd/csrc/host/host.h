@@ -20,7 +20,7 @@ namespace cueq_host {
   X(cueq_trimul_saved_bytes) X(cueq_trimul_workspace_bytes) X(cueq_trimul_fwd)                                         \
   X(cueq_linear_flex) X(cueq_linear_flex_dw_chunks) X(cueq_linear_flex_dw) X(cueq_sum_runs) X(cueq_linear_rows) X(cueq_linear_rows_mul_ir) \
   X(cueq_linear_dw_mul_ir_items) X(cueq_linear_dw_mul_ir) X(cueq_gemm_tn_items) X(cueq_gemm_tn) X(cueq_gemm_table) \
-  X(cueq_fc_flex) X(cueq_fc_flex_dw_chunks) X(cueq_fc_flex_dw) X(cueq_fc_factors) X(cueq_fc_pack) X(cueq_rows_mean)
+  X(cueq_fc_flex) X(cueq_fc_flex_dw_chunks) X(cueq_fc_flex_dw) X(cueq_fc_factors) X(cueq_fc_pack) X(cueq_rows_mean) X(cueq_normalize3)
 
 // The library is the one the ctypes binding loaded (CUEQ_AMD_LIBRARY may name another build), so nothing is linked.
 struct Library {

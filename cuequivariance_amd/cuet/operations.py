@@ -710,9 +710,10 @@ class SphericalHarmonics(torch.nn.Module):
 
     def forward(self, vectors: torch.Tensor) -> torch.Tensor:
         torch._assert(vectors.ndim == 2, f"Input must have shape (batch, 3) - got {vectors.shape}")
-        if self.normalize:
-            vectors = torch.nn.functional.normalize(vectors, dim=1)
         op = _operator(self)
+        if self.normalize:
+            unit = _lib.host().normalize(vectors) if op is not None and type(vectors) is torch.Tensor and vectors.is_cuda else None
+            vectors = torch.nn.functional.normalize(vectors, dim=1) if unit is None else unit
         outs = op.call([vectors], [None], [None], [-1]) if op is not None and type(vectors) is torch.Tensor else None
         if outs is not None:
             return outs[0]

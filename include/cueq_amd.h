@@ -479,6 +479,10 @@ int cueq_sum_runs(const float* partial, int32_t per, int32_t nruns, const int32_
 /* out[r, :] = in[r, :] / max(1, offsets[r + 1] - offsets[r]): the mean over the batch rows that the grouping `offsets` (rows + 1
  * device integers, cueq_segment_csr_build) puts on every row.  Any CUEQ_* element type; float64 computes in float64. */
 int cueq_rows_mean(int32_t dtype, int64_t rows, int64_t width, const void* in, const int64_t* offsets, void* out, void* stream);
+/* Rows of three, float32 or float64, y = x / max(|x|, eps).  stage 0: out = y; 1: out = the gradient of g . y for x; 2: of v . (stage
+ * 1's result), out for g and out_x for x (either may be null).  Pointers a stage does not name are ignored. */
+int cueq_normalize3(int32_t dtype, int32_t stage, int64_t rows, const void* x, const void* g, const void* v, double eps, void* out,
+                    void* out_x, void* stream);
 
 /* Fully connected product with shared weights and a second operand of multiplicity one, table-driven, for batches that do not
  * fill the chip with the generated kernels and for extents those do not take.  gradient == 0: rows of x1 against the weights;
