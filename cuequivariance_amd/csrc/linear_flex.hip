@@ -5,14 +5,11 @@
 //
 //   out[z, c0 + v D + i] = sum over the parts p of the block  coeff_p sum_u A[z, a_p + u D + i] W_p[u, v]
 //
-// What bounds them: at a few thousand rows the latency of one wavefront's serial chain, so the unit of work is a tile of 32 rows
-// and 32 columns (the row-streaming kernels give a wavefront 32 x 128), without LDS and without barriers.  The products are
+// The unit of work is a tile of 32 rows and 32 columns (the row-streaming kernels give a wavefront 32 x 128).  The products are
 // issued as W-columns x rows: a lane then holds one row and, per accumulator, 4 adjacent columns of it (times D components in
-// mul_ir), and both its loads and its stores are whole 16-byte pieces; the k order inside a step is free, so a lane takes 4 (8)
-// adjacent channels of its row.  (Forward of 5 003 rows of 128x0e+128x1o+128x2e in mul_ir, float: 131 us in three row-streaming
-// launches, 40 us here.)  The wavefronts of a block share the rows and differ in the columns: the rows come from L1 for
-// all but the first.
+// mul_ir), both in whole 16-byte pieces; the k order inside a step is free, so a lane takes 4 (8) adjacent channels of its row.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 #include "cw_common.h"
@@ -32,161 +29,320 @@ struct FlexBlock {  // one block of the result
 };
 
 typedef float fx16 __attribute__((ext_vector_type(16)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-// one tile: rows z0 .. z0 + 32 ZT, columns n0 .. n0 + 32 of the block.  WT: the weights are read transposed (input gradient).
-// SK: wavefronts that share the tile, each with its part of every contraction; the first adds the others' sums, in order, through
-// LDS and stores (SK > 1: all SK wavefronts of the workgroup are here).
-template <typename TI, int D, int ZT, bool WT, int SK>
-__device__ __forceinline__ void flex_tile(const FlexBlock& blk, const FlexPart* __restrict__ parts, const TI* __restrict__ A, int64_t lda, const TI* __restrict__ W,
-                                          TI* __restrict__ C, int64_t ldc, int64_t Z, int64_t z0, int n0) {
-  constexpr int ES = sizeof(TI), EPV = 16 / ES, STEP = 2 * EPV;  // channels per step: 4 + 4 (float), 8 + 8
-  static_assert(SK == 1 || ZT == 1, "a shared tile has 32 rows");
+constexpr int kFlexStageBytes = 2 * 128 * (32 * 7 + 16);  // two buffers of 128 rows x 8 channels (float) x 7 components, the largest
+
+// The weights of a step of the contraction (STEP channels) as the matrix instructions take them, a column of W per lane (WT: a row of
+// W, read transposed for the input gradient).  2-byte weights read down a column are a word each until they are used.
+template <typename TI, bool WT>
+struct FlexWeights {
+  static constexpr int ES = sizeof(TI), EPV = 16 / ES, STEP = 2 * EPV;  // channels per step: 4 + 4 (float), 8 + 8
+  uint32_t v[WT || ES == 4 ? 4 : 8];
+  // lane: this lane's column n and half h: n K + EPV h (WT), EPV h N + n
+  static __device__ __forceinline__ uint32_t lane_of(int n, int h, int K, int N) {
+    return WT ? static_cast<uint32_t>(n) * K + EPV * h : static_cast<uint32_t>(EPV * h) * N + n;
+  }
+  __device__ __forceinline__ void load(const TI* __restrict__ w, int k0, int N, uint32_t lane) {
+    if constexpr (WT) {
+      const uint4 q = *reinterpret_cast<const uint4*>(w + k0 + lane);
+      v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
+    } else {
+      using Word = std::conditional_t<ES == 4, uint32_t, uint16_t>;
+#pragma unroll
+      for (int s = 0; s < EPV; ++s) v[s] = (reinterpret_cast<const Word*>(w) + static_cast<int64_t>(k0 + s) * N)[lane];
+    }
+  }
+  // acc[i] += W x for the D components of the lane's row, x as it lies: EPV channels of D components
+  template <int D>
+  __device__ __forceinline__ void multiply(const uint4 (&x)[D], fx16 (&acc)[D]) const {
+    if constexpr (ES == 4) {
+      const float* xf = reinterpret_cast<const float*>(&x[0]);
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int i = 0; i < D; ++i) acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(v[s]), xf[s * D + i], acc[i], 0, 0, 0);
+    } else {
+      uint4 w;
+      if constexpr (WT) w = make_uint4(v[0], v[1], v[2], v[3]);
+      else w = make_uint4(v[0] | v[1] << 16, v[2] | v[3] << 16, v[4] | v[5] << 16, v[6] | v[7] << 16);
+#pragma unroll
+      for (int i = 0; i < D; ++i) {
+        uint4 op;
+        if constexpr (D == 1) op = x[0];
+        else op = make_uint4(mm_pick(&x[0], i, D + i), mm_pick(&x[0], 2 * D + i, 3 * D + i), mm_pick(&x[0], 4 * D + i, 5 * D + i), mm_pick(&x[0], 6 * D + i, 7 * D + i));
+        acc[i] = mm_32x32x16<TI>(w, op, acc[i]);
+      }
+    }
+  }
+};
+
+// what is summed so far counts in units of the coefficient of the part before
+template <int D>
+__device__ __forceinline__ void flex_rescale(fx16 (&acc)[D], float& scale, float coeff, bool first) {
+  if (!first && coeff != scale) {
+    const float f = scale / coeff;
+#pragma unroll
+    for (int i = 0; i < D; ++i) acc[i] *= f;
+  }
+  scale = coeff;
+}
+
+// columns n0 .. n0 + 32 of row z: four adjacent columns of D components at a time
+template <typename TI, int D>
+__device__ __forceinline__ void flex_store(const FlexBlock& blk, TI* __restrict__ C, int64_t ldc, int64_t z, int n0, int h, const fx16 (&acc)[D], float scale) {
+  TI* out = C + z * ldc + blk.c0;
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+    const int m = n0 + 8 * a + 4 * h;
+    if (m >= blk.N) continue;
+    float v[4 * D];
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+      for (int i = 0; i < D; ++i) v[b * D + i] = scale * acc[i][4 * a + b];
+    if constexpr (sizeof(TI) == 4) {
+#pragma unroll
+      for (int i = 0; i < D; ++i) *reinterpret_cast<float4*>(out + m * D + 4 * i) = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < D; ++i)
+        *reinterpret_cast<uint2*>(out + m * D + 4 * i) = make_uint2(mm_pack<TI>(v[4 * i], v[4 * i + 1]), mm_pack<TI>(v[4 * i + 2], v[4 * i + 3]));
+    }
+  }
+}
+
+// ---- few tiles: the four wavefronts of a workgroup share a tile of 32 rows and 32 columns, each with its part of every contraction;
+// the first adds the others' sums, in order, through LDS and stores.  A lane reads its own row; the operands of PD steps are in
+// flight, as many as the registers beside the sums allow.
+template <typename TI, int D, bool WT>
+__device__ __forceinline__ void flex_shared_tile(const FlexBlock& blk, const FlexPart* __restrict__ parts, const TI* __restrict__ A, int64_t lda,
+                                                 const TI* __restrict__ W, TI* __restrict__ C, int64_t ldc, int64_t Z, int64_t z0, int n0) {
+  using Weights = FlexWeights<TI, WT>;
+  constexpr int EPV = Weights::EPV, STEP = Weights::STEP, PD = D == 1 ? 8 : D == 3 || (D == 5 && (WT || sizeof(TI) == 4)) ? 4 : 2;
   const int lane = threadIdx.x & 63, c = lane & 31, h = lane >> 5;
-  const int share = SK > 1 ? __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)) : 0;
+  const int share = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  fx16 acc[D];
+#pragma unroll
+  for (int i = 0; i < D; ++i) acc[i] = fx16{0};
+  const int n = min(n0 + c, blk.N - 1);
+  const TI* row = A + min(z0 + c, Z - 1) * lda;
+  float scale = 1.0f;
+  for (int p = 0; p < blk.parts; ++p) {
+    const FlexPart part = parts[blk.first + p];
+    flex_rescale(acc, scale, part.coeff, p == 0);
+    const int steps = part.K / STEP, first = steps * share / 4 * STEP, last = steps * (share + 1) / 4 * STEP;
+    if (first == last) continue;
+    uint4 x[PD][D];
+    Weights w[PD];
+    const uint32_t w_lane = Weights::lane_of(n, h, part.K, blk.N);
+    auto load = [&](int k0, uint4 (&xx)[D], Weights& ww) {
+#pragma unroll
+      for (int i = 0; i < D; ++i) xx[i] = *reinterpret_cast<const uint4*>(row + part.a0 + static_cast<int64_t>(k0 + EPV * h) * D + i * EPV);
+      ww.load(W + part.w0, k0, blk.N, w_lane);
+    };
+#pragma unroll
+    for (int j = 0; j < PD; ++j)
+      if (first + j * STEP < last) load(first + j * STEP, x[j], w[j]);
+    for (int k0 = first; k0 < last; k0 += PD * STEP)
+#pragma unroll
+      for (int j = 0; j < PD; ++j) {
+        if (k0 + j * STEP < last) {
+          w[j].multiply(x[j], acc);
+          if (k0 + (PD + j) * STEP < last) load(k0 + (PD + j) * STEP, x[j], w[j]);
+        }
+      }
+  }
+  __shared__ float others[3][16][64];
+#pragma unroll
+  for (int i = 0; i < D; ++i) {
+    if (share)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) others[share - 1][r][lane] = acc[i][r];
+    __syncthreads();
+    if (!share)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+#pragma unroll
+        for (int o = 0; o < 3; ++o) acc[i][r] += others[o][r][lane];
+    __syncthreads();
+  }
+  if (share == 0 && z0 + c < Z) flex_store(blk, C, ldc, z0 + c, n0, h, acc, scale);
+}
+
+// unit = (column tiles of the blocks one after the other) x (row tile)
+template <typename TI, bool WT>
+__global__ void __launch_bounds__(256, 2) flex_shared_kernel(const FlexBlock* __restrict__ blocks, const FlexPart* __restrict__ parts, int nblocks, int tiles_n,
+                                                             const TI* __restrict__ A, int64_t lda, const TI* __restrict__ W, TI* __restrict__ C, int64_t ldc,
+                                                             int64_t Z) {
+  const int64_t unit = blockIdx.x, zt = unit / tiles_n, z0 = 32 * zt;
+  int tile = static_cast<int>(unit - zt * tiles_n);
+  int b = 0;
+  while (b < nblocks && tile >= blocks[b].nt) tile -= blocks[b++].nt;
+  if (b == nblocks || z0 >= Z) return;
+  const FlexBlock blk = blocks[b];
+  switch (blk.D) {
+    case 1: flex_shared_tile<TI, 1, WT>(blk, parts, A, lda, W, C, ldc, Z, z0, tile * 32); break;
+    case 3: flex_shared_tile<TI, 3, WT>(blk, parts, A, lda, W, C, ldc, Z, z0, tile * 32); break;
+    case 5: flex_shared_tile<TI, 5, WT>(blk, parts, A, lda, W, C, ldc, Z, z0, tile * 32); break;
+    default: flex_shared_tile<TI, 7, WT>(blk, parts, A, lda, W, C, ldc, Z, z0, tile * 32);
+  }
+}
+
+// ---- more tiles: a workgroup stages its rows through LDS.  Bound by the matrix cores from some 10 000 rows of float on (20 000 rows of
+// 128x0e+128x1o+128x2e in mul_ir, forward: 131 -> 73 us, 80 TFLOP/s; 38 at the rate of a large product), below by the latency of the
+// first and last step of a tile (5 003 rows 37 -> 24 us), in 2-byte elements by bytes and latency (8 000 rows 25 -> 13 us).
+// A workgroup has RT row tiles of 32 and 4 / RT column tiles of a block, a wavefront each one of the four pairs.  The rows come in
+// chunks of 4 / RT steps, two buffers in turn, one barrier a chunk: 128 D / RT adjacent bytes of every row, whole lines of
+// memory where a lane's own row would be a line per lane and load (64 lines an instruction, four times over for the four
+// wavefronts).  16 bytes of padding per row put the lanes' reads on all banks.  The weights go straight to registers, four steps ahead.
+template <typename TI, int D, int RT, int ZT, bool WT>
+__device__ __forceinline__ void flex_stage_tile(const FlexBlock& blk, const FlexPart* __restrict__ parts, const TI* __restrict__ A, int64_t lda,
+                                                const TI* __restrict__ W, TI* __restrict__ C, int64_t ldc, int64_t Z, int64_t z0, int first_tile, char* lds) {
+  using Weights = FlexWeights<TI, WT>;
+  constexpr int ES = sizeof(TI), EPV = Weights::EPV, STEP = Weights::STEP;
+  constexpr int SPC = 4 / RT, KC = SPC * STEP;                       // steps and channels of a chunk
+  constexpr int PR = KC * D * ES / 16, RS = PR * 16 + 16, BUF = 32 * RT * ZT * RS;  // 16-byte pieces of a row, its stride, a buffer
+  constexpr int NP = D * ZT;                                                        // pieces a lane brings
+  static_assert(32 * RT * ZT * PR == 256 * NP && 2 * BUF <= kFlexStageBytes, "the rows of a chunk");
+  const int lane = threadIdx.x & 63, c = lane & 31, h = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)), rt = wave / (4 / RT), n0 = (first_tile + wave % (4 / RT)) * 32;
   fx16 acc[ZT][D];
 #pragma unroll
   for (int t = 0; t < ZT; ++t)
 #pragma unroll
     for (int i = 0; i < D; ++i) acc[t][i] = fx16{0};
   const int n = min(n0 + c, blk.N - 1);
-  const TI* row[ZT];
+  const TI* from[NP];  // this lane's pieces of a chunk
+  int into[NP], col[NP];
 #pragma unroll
-  for (int t = 0; t < ZT; ++t) row[t] = A + min(z0 + 32 * t + c, Z - 1) * lda;
+  for (int j = 0; j < NP; ++j) {
+    const int piece = j * 256 + threadIdx.x, r = piece / PR, q = piece % PR;
+    from[j] = A + min(z0 + r, Z - 1) * lda;
+    into[j] = r * RS + q * 16;
+    col[j] = q * EPV;
+  }
+  const char* mine = lds + (32 * rt * ZT + c) * RS + EPV * h * D * ES;
   float scale = 1.0f;
+  int turn = 0;
   for (int p = 0; p < blk.parts; ++p) {
     const FlexPart part = parts[blk.first + p];
-    if (p && part.coeff != scale) {  // (what is summed so far counts in units of the coefficient)
-      const float f = scale / part.coeff;
 #pragma unroll
-      for (int t = 0; t < ZT; ++t)
-#pragma unroll
-        for (int i = 0; i < D; ++i) acc[t][i] *= f;
+    for (int t = 0; t < ZT; ++t) {
+      float before = scale;
+      flex_rescale(acc[t], before, part.coeff, p == 0);
     }
     scale = part.coeff;
-    uint4 x[ZT][D], xn[ZT][D];
-    uint4 wv, wn;
-    auto load = [&](int k0, uint4 (&xx)[ZT][D], uint4& ww) {
-      const int k = k0 + EPV * h;
+    const int K = part.K, ends = K * D - EPV;  // (pieces past the row's channels repeat its last one and are not used)
+    u32x4 x[NP];  // (a vector type: an array of structs stays in memory here)
+    auto fetch = [&](int k0) {
 #pragma unroll
-      for (int t = 0; t < ZT; ++t)
+      for (int j = 0; j < NP; ++j) x[j] = *reinterpret_cast<const u32x4*>(from[j] + part.a0 + min(k0 * D + col[j], ends));
+    };
+    constexpr int WD = D == 7 && ES == 2 ? 2 : 4;  // (as the registers allow)
+    Weights w[WD];
+    const uint32_t w_lane = Weights::lane_of(n, h, K, blk.N);
+    fetch(0);
 #pragma unroll
-        for (int i = 0; i < D; ++i) xx[t][i] = *reinterpret_cast<const uint4*>(row[t] + part.a0 + static_cast<int64_t>(k) * D + i * EPV);
-      if constexpr (WT) {
-        ww = *reinterpret_cast<const uint4*>(W + part.w0 + static_cast<int64_t>(n) * part.K + k);
-      } else if constexpr (ES == 4) {
-        uint32_t e[4];
+    for (int s = 0; s < WD; ++s) w[s].load(W + part.w0, min(s * STEP, K - STEP), blk.N, w_lane);
+    // (whole groups of four steps without a condition: behind one the number of loads on the way is unknown, and every wait is for
+    // all of them)
+    auto four = [&](int k4, auto whole) {
 #pragma unroll
-        for (int s = 0; s < 4; ++s) e[s] = reinterpret_cast<const uint32_t*>(W)[part.w0 + static_cast<int64_t>(k + s) * blk.N + n];
-        ww = make_uint4(e[0], e[1], e[2], e[3]);
-      } else {
-        uint32_t e[8];
+      for (int ch = 0; ch < RT; ++ch) {
+        const int k0 = k4 + ch * KC;
+        if (!decltype(whole)::value && k0 >= K) continue;
+        char* buf = lds + turn * BUF;
 #pragma unroll
-        for (int s = 0; s < 8; ++s) e[s] = reinterpret_cast<const uint16_t*>(W)[part.w0 + static_cast<int64_t>(k + s) * blk.N + n];
-        ww = make_uint4(e[0] | e[1] << 16, e[2] | e[3] << 16, e[4] | e[5] << 16, e[6] | e[7] << 16);
+        for (int j = 0; j < NP; ++j) *reinterpret_cast<u32x4*>(buf + into[j]) = x[j];
+        __syncthreads();  // (the other buffer is no longer read once every wavefront is here)
+        fetch(k0 + KC);
+#pragma unroll
+        for (int s = 0; s < SPC; ++s) {
+          const int k = k0 + s * STEP;
+          if (!decltype(whole)::value && k >= K) continue;
+#pragma unroll
+          for (int t = 0; t < ZT; ++t) {
+            uint4 op[D];
+#pragma unroll
+            for (int i = 0; i < D; ++i) op[i] = *reinterpret_cast<const uint4*>(mine + turn * BUF + 32 * t * RS + s * STEP * D * ES + 16 * i);
+            w[(ch * SPC + s) % WD].multiply(op, acc[t]);
+          }
+          w[(ch * SPC + s) % WD].load(W + part.w0, min(k + WD * STEP, K - STEP), blk.N, w_lane);
+        }
+        turn ^= 1;
       }
     };
-    const int steps = part.K / STEP, first = SK > 1 ? steps * share / SK * STEP : 0, last = SK > 1 ? steps * (share + 1) / SK * STEP : part.K;
-    if (SK > 1 && first == last) continue;
-    load(first, x, wv);
-    for (int k0 = first; k0 < last; k0 += STEP) {
-      load(min(k0 + STEP, last - STEP), xn, wn);
-#pragma unroll
-      for (int t = 0; t < ZT; ++t) {
-        if constexpr (ES == 4) {
-          const float* xf = reinterpret_cast<const float*>(&x[t][0]);
-          const float* wf = reinterpret_cast<const float*>(&wv);
-#pragma unroll
-          for (int s = 0; s < 4; ++s)
-#pragma unroll
-            for (int i = 0; i < D; ++i) acc[t][i] = __builtin_amdgcn_mfma_f32_32x32x2f32(wf[s], xf[s * D + i], acc[t][i], 0, 0, 0);
-        } else {
-#pragma unroll
-          for (int i = 0; i < D; ++i) {
-            uint4 op;
-            if constexpr (D == 1) op = x[t][0];
-            else op = make_uint4(mm_pick(&x[t][0], i, D + i), mm_pick(&x[t][0], 2 * D + i, 3 * D + i), mm_pick(&x[t][0], 4 * D + i, 5 * D + i),
-                                 mm_pick(&x[t][0], 6 * D + i, 7 * D + i));
-            acc[t][i] = mm_32x32x16<TI>(wv, op, acc[t][i]);
-          }
-        }
-      }
-#pragma unroll
-      for (int t = 0; t < ZT; ++t)
-#pragma unroll
-        for (int i = 0; i < D; ++i) x[t][i] = xn[t][i];
-      wv = wn;
-    }
+    int k4 = 0;
+    for (; k4 + 4 * STEP <= K; k4 += 4 * STEP) four(k4, std::true_type{});
+    if (k4 < K) four(k4, std::false_type{});
   }
-  if constexpr (SK > 1) {
-    __shared__ float others[SK - 1][16][64];
+  // The tile goes out through LDS as well, 64 D bytes of every row at a time: a lane's own 16-byte pieces are a write request each
+  // (20 000 rows of 128x0e+128x1o+128x2e, float: 79 us with such stores, 60 without any).
+  constexpr int COLS = 64 / ES, OS = 64 * D + 16, OP = 4 * D;  // columns a turn; a row's stride and 16-byte pieces in LDS
+  static_assert(4 * 32 * OS <= kFlexStageBytes, "a turn of four wavefronts");
+  char* out_lds = lds + wave * 32 * OS;
+  __syncthreads();  // (no wavefront reads the rows any more)
 #pragma unroll
-    for (int i = 0; i < D; ++i) {
-      if (share)
+  for (int turn_z = 0; turn_z < ZT * (32 / COLS); ++turn_z) {
+    const int t = turn_z / (32 / COLS), turn_n = turn_z % (32 / COLS);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) others[share - 1][r][lane] = acc[0][i][r];
-      __syncthreads();
-      if (!share)
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-#pragma unroll
-          for (int o = 0; o < SK - 1; ++o) acc[0][i][r] += others[o][r][lane];
-      __syncthreads();
-    }
-    if (share) return;
-  }
-#pragma unroll
-  for (int t = 0; t < ZT; ++t) {
-    const int64_t z = z0 + 32 * t + c;
-    if (z >= Z) continue;
-    TI* out = C + z * ldc + blk.c0;
-#pragma unroll
-    for (int a = 0; a < 4; ++a) {
-      const int m = n0 + 8 * a + 4 * h;  // four adjacent columns, D components each
-      if (m >= blk.N) continue;
+    for (int a = 0; a < COLS / 8; ++a) {
       float v[4 * D];
 #pragma unroll
       for (int b = 0; b < 4; ++b)
 #pragma unroll
-        for (int i = 0; i < D; ++i) v[b * D + i] = scale * acc[t][i][4 * a + b];
-      if constexpr (ES == 4) {
+        for (int i = 0; i < D; ++i) v[b * D + i] = scale * acc[t][i][4 * (turn_n * (COLS / 8) + a) + b];
+      char* to = out_lds + c * OS + (8 * a + 4 * h) * D * ES;
 #pragma unroll
-        for (int i = 0; i < D; ++i) *reinterpret_cast<float4*>(out + m * D + 4 * i) = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
-      } else {
-#pragma unroll
-        for (int i = 0; i < D; ++i)
-          *reinterpret_cast<uint2*>(out + m * D + 4 * i) = make_uint2(mm_pack<TI>(v[4 * i], v[4 * i + 1]), mm_pack<TI>(v[4 * i + 2], v[4 * i + 3]));
+      for (int i = 0; i < D; ++i) {
+        if constexpr (ES == 4) *reinterpret_cast<float4*>(to + 16 * i) = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
+        else *reinterpret_cast<uint2*>(to + 8 * i) = make_uint2(mm_pack<TI>(v[4 * i], v[4 * i + 1]), mm_pack<TI>(v[4 * i + 2], v[4 * i + 3]));
       }
     }
+    __builtin_amdgcn_wave_barrier();
+    const int from_col = (n0 + turn_n * COLS) * D, ends_col = blk.N * D;
+#pragma unroll
+    for (int j = 0; j < 2 * D; ++j) {
+      const int piece = j * 64 + lane, r = piece / OP, q = piece % OP;
+      const int64_t z = z0 + 32 * (rt * ZT + t) + r;
+      const u32x4 value = *reinterpret_cast<const u32x4*>(out_lds + r * OS + 16 * q);
+      if (z < Z && from_col + q * EPV < ends_col) *reinterpret_cast<u32x4*>(C + z * ldc + blk.c0 + from_col + q * EPV) = value;
+    }
+    __builtin_amdgcn_wave_barrier();
   }
 }
 
-// unit = (column tiles of the blocks one after the other) x (row tile); the column tile runs fastest, so a block's wavefronts share rows
-// (SK > 1: a workgroup per unit)
-template <typename TI, bool WT, int ZBIG, int SK>
-__global__ void __launch_bounds__(256, 2) flex_rows_kernel(const FlexBlock* __restrict__ blocks, const FlexPart* __restrict__ parts, int nblocks, int tiles_n,
-                                                           const TI* __restrict__ A, int64_t lda, const TI* __restrict__ W, TI* __restrict__ C, int64_t ldc,
-                                                           int64_t Z) {
-  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-  const int64_t unit = SK > 1 ? static_cast<int64_t>(blockIdx.x) : static_cast<int64_t>(blockIdx.x) * 4 + wave;
-  const int64_t zt = unit / tiles_n;
-  int tile = static_cast<int>(unit - zt * tiles_n);
-  int b = 0;
-  while (b < nblocks && tile >= blocks[b].nt) tile -= blocks[b++].nt;
-  constexpr int RZ = 32 * ZBIG;
-  const int64_t z0 = zt * RZ;
-  if (b == nblocks || z0 >= Z) return;
+// A slab of 128 ZT rows and a block of nt column tiles are nt workgroups: four columns x one row tile for every whole four columns, the
+// rest two columns x two row tiles or one x four.  The last block first: the blocks of most components are the longest.  ZT > 1: row
+// tiles of a wavefront, where every block has one component (a tile of one is over before its first loads have paid).
+template <typename TI, bool WT, int ZT>
+__global__ void __launch_bounds__(256, 2) flex_stage_kernel(const FlexBlock* __restrict__ blocks, const FlexPart* __restrict__ parts, int nblocks,
+                                                            const TI* __restrict__ A, int64_t lda, const TI* __restrict__ W, TI* __restrict__ C, int64_t ldc,
+                                                            int64_t Z, int64_t slabs) {
+  __shared__ __align__(16) char lds[kFlexStageBytes];
+  int64_t unit = blockIdx.x;
+  int b = nblocks - 1;
+  while (b >= 0 && unit >= slabs * blocks[b].nt) unit -= slabs * blocks[b--].nt;
+  if (b < 0) return;
   const FlexBlock blk = blocks[b];
-  switch (blk.D) {
-    case 1: flex_tile<TI, 1, ZBIG, WT, SK>(blk, parts, A, lda, W, C, ldc, Z, z0, tile * 32); break;
-    case 3:
-      for (int t = 0; t < ZBIG && z0 + 32 * t < Z; ++t) flex_tile<TI, 3, 1, WT, SK>(blk, parts, A, lda, W, C, ldc, Z, z0 + 32 * t, tile * 32);
-      break;
-    case 5:
-      for (int t = 0; t < ZBIG && z0 + 32 * t < Z; ++t) flex_tile<TI, 5, 1, WT, SK>(blk, parts, A, lda, W, C, ldc, Z, z0 + 32 * t, tile * 32);
-      break;
-    default:
-      for (int t = 0; t < ZBIG && z0 + 32 * t < Z; ++t) flex_tile<TI, 7, 1, WT, SK>(blk, parts, A, lda, W, C, ldc, Z, z0 + 32 * t, tile * 32);
+  const int64_t slab = unit / blk.nt;
+  const int t = static_cast<int>(unit - slab * blk.nt), full = blk.nt & ~3, rest = blk.nt - full;
+  const int rt = t < full ? 1 : rest == 2 ? 2 : 4, tile = t < full ? t & ~3 : rest == 2 ? full : t;
+  const int64_t z0 = ZT * (slab * 128 + (t < full ? (t & 3) * 32 : rest == 2 ? (t - full) * 64 : 0));
+  if (z0 >= Z) return;
+#define STAGE(D)                                                                                                                do {                                                                                                                            if (rt == 1) flex_stage_tile<TI, D, 1, ZT, WT>(blk, parts, A, lda, W, C, ldc, Z, z0, tile, lds);                                  else if (rt == 2) flex_stage_tile<TI, D, 2, ZT, WT>(blk, parts, A, lda, W, C, ldc, Z, z0, tile, lds);                             else flex_stage_tile<TI, D, 4, ZT, WT>(blk, parts, A, lda, W, C, ldc, Z, z0, tile, lds);                                        } while (0)
+  if constexpr (ZT > 1) {
+    STAGE(1);
+  } else {
+    switch (blk.D) {
+      case 1: STAGE(1); break;
+      case 3: STAGE(3); break;
+      case 5: STAGE(5); break;
+      default: STAGE(7);
+    }
   }
+#undef STAGE
 }
 
 // Weight gradients: dW[w0 + u N + v] = coeff sum_z sum_i x[z, a0 + i sa + u D + i'] g[z, c0 + i sc + v D + i'] over a chunk of rows,
@@ -389,31 +545,35 @@ extern "C" int cueq_linear_flex(int32_t dtype, int32_t transposed_weights, int64
   const int64_t es = dtype == CUEQ_F32 ? 4 : 2, epv = 16 / es;
   CUEQ_REQUIRE(((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(C) | reinterpret_cast<uintptr_t>(W)) & 15) == 0 && lda % epv == 0 && ldc % epv == 0,
                CUEQ_ERR_UNSUPPORTED, "linear_flex: rows must be 16-byte aligned");
-  // two row tiles per wavefront halve the weight loads once there are units enough for two per SIMD
-  const int64_t zt1 = (rows + 31) / 32;
-  const bool big = zt1 * column_tiles >= 8 * 4ll * device_cus();
   // four wavefronts share a tile where all tiles, four wavefronts each, still run at once (two workgroups to a CU): 300 rows of
   // 128x0e+128x1o+128x2e in mul_ir, float, forward 21.8 -> 9.7 us, 1 000 rows 22.1 -> 12.6 (1 400 rows, past the line: 22.5 either way)
-  const bool shared = zt1 * column_tiles <= 2ll * device_cus();
-  const int64_t units = (big ? (rows + 63) / 64 : zt1) * column_tiles, grid = shared ? units : (units + 3) / 4;
+  const int64_t tiles = (rows + 31) / 32 * column_tiles;
+  const bool shared = tiles <= 2ll * device_cus();
+  // ir_mul rows (every block one component): four row tiles a wavefront once there are so many workgroups; us for one / four, 128 ch:
+  // float 4 000 rows (1 152 workgroups of one tile) 23 / 26, 8 000 38 / 38, 16 000 67 / 57, 32 000 147 / 113; bfloat16 2 000 9.8 / 9.7,
+  // 4 000 13.8 / 9.8, 32 000 73 / 35
+  const bool tall = !mul_ir && !shared && (rows + 127) / 128 * column_tiles >= (dtype == CUEQ_F32 ? 9ll : 4ll) * device_cus();
+  const int64_t slab_rows = tall ? 512 : 128, slabs = (rows + slab_rows - 1) / slab_rows;
+  const int64_t grid = shared ? tiles : slabs * column_tiles;
   CUEQ_REQUIRE(grid < (1ll << 31), CUEQ_ERR_TOO_LARGE, "linear_flex: too many rows");
   KernelTimer timer(mul_ir ? "linear_rows_mul_ir" : "linear_rows", stream);
-#define FLEX_ARGS(TI) static_cast<const FlexBlock*>(blocks), static_cast<const FlexPart*>(parts), nblocks, column_tiles, static_cast<const TI*>(A), lda, static_cast<const TI*>(W), static_cast<TI*>(C), ldc, rows
-#define FLEX(TI)                                                                                                                                                       \
-  do {                                                                                                                                                                 \
-    if (transposed_weights) {                                                                                                                                          \
-      if (shared) hipLaunchKernelGGL((flex_rows_kernel<TI, true, 1, 4>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, FLEX_ARGS(TI));                    \
-      else if (big) hipLaunchKernelGGL((flex_rows_kernel<TI, true, 2, 1>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, FLEX_ARGS(TI));                            \
-      else hipLaunchKernelGGL((flex_rows_kernel<TI, true, 1, 1>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, FLEX_ARGS(TI));                                \
-    } else {                                                                                                                                                           \
-      if (shared) hipLaunchKernelGGL((flex_rows_kernel<TI, false, 1, 4>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, FLEX_ARGS(TI));                    \
-      else if (big) hipLaunchKernelGGL((flex_rows_kernel<TI, false, 2, 1>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, FLEX_ARGS(TI));                           \
-      else hipLaunchKernelGGL((flex_rows_kernel<TI, false, 1, 1>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, FLEX_ARGS(TI));                               \
-    }                                                                                                                                                                  \
+#define FLEX_LAUNCH(KERNEL, ...)                                                                                                                         \
+  hipLaunchKernelGGL((KERNEL), dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, static_cast<const FlexBlock*>(blocks),                           \
+                     static_cast<const FlexPart*>(parts), nblocks, __VA_ARGS__)
+#define FLEX_OPERANDS(TI) static_cast<const TI*>(A), lda, static_cast<const TI*>(W), static_cast<TI*>(C), ldc, rows
+#define FLEX(TI)                                                                                                  \
+  do {                                                                                                            \
+    if (shared && transposed_weights) FLEX_LAUNCH((flex_shared_kernel<TI, true>), column_tiles, FLEX_OPERANDS(TI));  \
+    else if (shared) FLEX_LAUNCH((flex_shared_kernel<TI, false>), column_tiles, FLEX_OPERANDS(TI));                  \
+    else if (transposed_weights && tall) FLEX_LAUNCH((flex_stage_kernel<TI, true, 4>), FLEX_OPERANDS(TI), slabs);    \
+    else if (transposed_weights) FLEX_LAUNCH((flex_stage_kernel<TI, true, 1>), FLEX_OPERANDS(TI), slabs);            \
+    else if (tall) FLEX_LAUNCH((flex_stage_kernel<TI, false, 4>), FLEX_OPERANDS(TI), slabs);                         \
+    else FLEX_LAUNCH((flex_stage_kernel<TI, false, 1>), FLEX_OPERANDS(TI), slabs);                                   \
   } while (0)
   FLEX_DISPATCH(dtype, FLEX);
 #undef FLEX
-#undef FLEX_ARGS
+#undef FLEX_OPERANDS
+#undef FLEX_LAUNCH
   CUEQ_CHECK_HIP(hipGetLastError());
   return CUEQ_OK;
 }

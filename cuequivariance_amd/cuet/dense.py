@@ -273,12 +273,13 @@ def _rows_launches(mod: "SegmentedPolynomialDense", es: int):
 
 
 # Rows from which on the row-streaming launches (weights in LDS) are the faster ones for forward and input gradient, by (rows in
-# mul_ir, element size) and multiplicity (up to 32, up to 64, above): where the measured times of the two cross.  Below, a launch is
-# bound by the chain of one wavefront, above by what one CU keeps in flight (128x0e+128x1o+128x2e, 4 000 rows of float: 27 us
-# against 72; 200 000: 804 against 623).
+# mul_ir, element size) and multiplicity (up to 32, up to 64, above): where the measured times of the two cross.  Above, the weights are
+# read once per CU and not once per 128 rows (or 512); below, a launch per degree is bound by the chain of one wavefront.  Forward of
+# 0e+1o+2e blocks, us, streaming / staged: 128 ch float mul_ir 12 000 rows 93 / 43, 50 000 209 / 179, 60 000 204 / 206; ir_mul 30 000
+# 135 / 107, 64 000 192 / 213; bfloat16 mul_ir 12 000 38 / 13, 75 000 96 / 97, 100 000 118 / 127.
 _NEVER = 1 << 60
-_ROWS_FROM = {(False, 4): (15_000, 10_000, 35_000), (False, 2): (_NEVER, 3_000, 6_000), (True, 4): (60_000, 30_000, 22_000),
-              (True, 2): (_NEVER, 22_000, 15_000)}
+_ROWS_FROM = {(False, 4): (6_000, 3_000, 50_000), (False, 2): (20_000, 12_000, 40_000), (True, 4): (110_000, 75_000, 55_000),
+              (True, 2): (_NEVER, 120_000, 75_000)}
 # ... and for the weight gradient, whose row launches win from the first row on but for float in mul_ir and for up to 32 channels (their
 # 128 x 128 tiles are padding then: 200 000 rows of 32x0e+32x1o+32x2e, float: 485 us against 274)
 _GRADS_FROM = {(False, 4): (_NEVER, 0, 0), (False, 2): (15_000, 0, 0), (True, 4): (150_000, 5_000, 5_000), (True, 2): (0, 0, 0)}
