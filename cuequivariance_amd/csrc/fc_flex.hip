@@ -326,21 +326,23 @@ constexpr bool fc_couples(int i, int k) {
 // Bound by the issue of vector instructions (a product of 32 x 32 x K is scaled and added component by component); 12 501 rows of
 // 64x0e+64x1o (x) 16x0e+16x1o, bfloat16: forward 38.7 us, both input gradients 82 us (the tests in the loop: 45 / 172, x2 read from
 // memory: 46), where the products of the operands went through memory 160 and 340 us.
-template <typename TI, int DS, int DR, int D2, bool MI, bool DX2, int KT>
+// SK > 1 (few row tiles): the SK wavefronts of the workgroup share one row tile, each with every SK-th channel, its weights from memory.
+template <typename TI, int DS, int DR, int D2, bool MI, bool DX2, int KT, int SK>
 __device__ __forceinline__ void fc_part_channels(fx16 (&acc)[DR], const FcPart& part, const FcBlock& blk, const TI* __restrict__ row, const TI* __restrict__ W,
                                                  const float* __restrict__ coef, const TI* x2row, const TI* __restrict__ x1row, float* sums, uint4* wl,
                                                  int n0) {
-  constexpr int VC = 16 / KT;
-  const int lane = threadIdx.x & 63, h = lane >> 5, wave = threadIdx.x >> 6;
-  uint4 x[KT][DS], wn[4];
+  constexpr int VC = 16 / KT, WN = SK > 1 ? KT : 4;
+  const int lane = threadIdx.x & 63, h = lane >> 5, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  if (SK > 1 && wave >= part.V) return;
+  uint4 x[KT][DS], wn[WN];
   auto request = [&](int v0) {  // (fragments past K are packed as zeros; past the last channel the last one is read again)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int f = wave + 4 * e, v = min(v0 + f / KT, part.V - 1), t = f % KT;
+    for (int e = 0; e < WN; ++e) {
+      const int f = SK > 1 ? e : wave + 4 * e, v = min(v0 + f / KT, part.V - 1), t = f % KT;
       wn[e] = *reinterpret_cast<const uint4*>(W + part.w0 + static_cast<int64_t>(v) * part.wv + (t * part.stride + n0 / 32) * kFragment + lane * 8);
     }
   };
-  request(0);
+  request(SK > 1 ? wave : 0);
 #pragma unroll
   for (int t = 0; t < KT; ++t) {
     const int k = 16 * t + 8 * h, kk = min(k, part.K - 8);
@@ -361,22 +363,28 @@ __device__ __forceinline__ void fc_part_channels(fx16 (&acc)[DR], const FcPart& 
   }
   const FcCoefs cf(coef + part.coef, DS * DR * D2);
 #pragma unroll 1
-  for (int v0 = 0; v0 < part.V; v0 += VC) {
-    __syncthreads();
+  for (int v0 = SK > 1 ? wave : 0; v0 < part.V; v0 += SK > 1 ? SK : VC) {
+    uint4 wv[KT];
+    if constexpr (SK > 1) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) wl[(wave + 4 * e) * 64 + lane] = wn[e];
-    __syncthreads();
-    request(v0 + VC);
-    const int end = min(VC, part.V - v0);
+      for (int t = 0; t < KT; ++t) wv[t] = wn[t];
+    } else {
+      __syncthreads();
+#pragma unroll
+      for (int e = 0; e < 4; ++e) wl[(wave + 4 * e) * 64 + lane] = wn[e];
+      __syncthreads();
+    }
+    request(v0 + (SK > 1 ? SK : VC));
+    const int end = SK > 1 ? 1 : min(VC, part.V - v0);
 #pragma unroll 1
     for (int g = 0; g < end; ++g) {
       const int y0 = part.j0 + (v0 + g) * part.vs;
       float xj[D2];
 #pragma unroll
       for (int j = 0; j < D2; ++j) xj[j] = fc_widen(x2row + y0 + j * part.js);
-      uint4 wv[KT];
+      if constexpr (SK == 1)
 #pragma unroll
-      for (int t = 0; t < KT; ++t) wv[t] = wl[(g * KT + t) * 64 + lane];
+        for (int t = 0; t < KT; ++t) wv[t] = wl[(g * KT + t) * 64 + lane];
       fx16 T[DS];
 #pragma unroll
       for (int i = 0; i < DS; ++i) T[i] = fx16{0};
@@ -458,8 +466,9 @@ __device__ __forceinline__ void fc_part_channels(fx16 (&acc)[DR], const FcPart& 
 // 32-bit words from row to row of x2 in LDS
 __host__ __device__ constexpr int fc_x2_words(int n2) { return (n2 + 1) / 2 | 1; }
 
-// false: some result is not finite, nothing is stored
-template <typename TI, int DR, int WM, bool MI, bool DX2, int MAXD, int KT>
+// false: some result is not finite, nothing is stored.  SK > 1: the SK wavefronts of the workgroup share the tile, each with some of the
+// parts (or channels) of its sums; their sums are added in order, and each of the first four stores eight of the columns.
+template <typename TI, int DR, int WM, bool MI, bool DX2, int MAXD, int KT, int SK>
 __device__ __forceinline__ bool fc_tile(const FcBlock& blk, const FcPart* __restrict__ parts, const float* __restrict__ coef, const TI* __restrict__ A, int64_t lda,
                                         const TI* __restrict__ W, const TI* __restrict__ X2, int64_t ldx2, const TI* __restrict__ X1, int64_t ldx1,
                                         TI* __restrict__ C, int64_t ldc, float* __restrict__ partial, float* lsum, uint4* wl, int n2, int64_t Z, int64_t z0, int n0) {
@@ -479,6 +488,7 @@ __device__ __forceinline__ bool fc_tile(const FcBlock& blk, const FcPart* __rest
   if constexpr (KT > 0) {  // the rows of x2 are read channel by channel: from LDS, an odd number of words apart
     const int words = fc_x2_words(n2);
     uint32_t* x2l = reinterpret_cast<uint32_t*>(wl + 16 * 64) + (DX2 ? 4 * 32 * n2p : 0) + (threadIdx.x >> 6) * 32 * words;
+    static_assert(KT == 0 || SK == 1 || SK == 4, "four wavefronts' regions of LDS");
     const int used = (n2 + 1) / 2;
 #pragma unroll 8
     for (int e = lane; e < 32 * used; e += 64) {
@@ -492,7 +502,7 @@ __device__ __forceinline__ bool fc_tile(const FcBlock& blk, const FcPart* __rest
   float* sums = lsum + c * n2p;
   auto one = [&](auto ds, const FcPart& part) {
     constexpr int DS = decltype(ds)::value;
-    auto channels = [&](auto d2) { fc_part_channels<TI, DS, DR, decltype(d2)::value, MI, DX2, KT>(acc, part, blk, row, W, coef, x2row, x1row, sums, wl, n0); };
+    auto channels = [&](auto d2) { fc_part_channels<TI, DS, DR, decltype(d2)::value, MI, DX2, KT, SK>(acc, part, blk, row, W, coef, x2row, x1row, sums, wl, n0); };
     if constexpr (KT > 0 && DS == 3 && DR == 3) {
       if (part.d2 == 1) channels(std::integral_constant<int, 1>{});
       else if (part.d2 == 3) channels(std::integral_constant<int, 3>{});
@@ -503,7 +513,8 @@ __device__ __forceinline__ bool fc_tile(const FcBlock& blk, const FcPart* __rest
       fc_part<TI, DS, DR, WM, MI, DX2>(acc, part, blk, row, W, coef, x2row, x1row, sums, n0, n);
     }
   };
-  for (int p = 0; p < blk.parts; ++p) {
+  const int share = SK > 1 ? __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)) : 0;
+  for (int p = KT == 0 ? share : 0; p < blk.parts; p += KT == 0 ? SK : 1) {
     const FcPart part = parts[blk.first + p];
     switch (part.D) {
       case 1: one(std::integral_constant<int, 1>{}, part); break;
@@ -512,21 +523,59 @@ __device__ __forceinline__ bool fc_tile(const FcBlock& blk, const FcPart* __rest
         if constexpr (MAXD > 3) one(std::integral_constant<int, 5>{}, part);
     }
   }
+  // what this wavefront stores: the four groups of eight columns, or its own one of the shared tile
+  constexpr int GROUPS = SK > 1 ? 1 : 4;
+  if constexpr (SK > 1) {
+    float* fold = reinterpret_cast<float*>(wl);  // 4 KB a wavefront (KT > 0: the region of the weights, which go another way here)
+#pragma unroll
+    for (int k = 0; k < DR; ++k) {
+      __syncthreads();  // (what the region held before is no longer read)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) fold[(share * 16 + r) * 64 + lane] = acc[k][r];
+      __syncthreads();
+      if (share < 4)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          float sum = fold[(4 * share + e) * 64 + lane];
+#pragma unroll
+          for (int o = 1; o < SK; ++o) sum += fold[(o * 16 + 4 * share + e) * 64 + lane];
+          acc[k][e] = sum;
+        }
+    }
+  }
+  if constexpr (DX2 && SK > 1) {  // the row sums of all wavefronts into the first one's (complete: there was a barrier behind the last part)
+    float* first = lsum - share * 32 * n2p;
+    for (int e = threadIdx.x; e < 32 * n2p; e += 64 * SK) {
+      float sum = first[e];
+#pragma unroll
+      for (int o = 1; o < SK; ++o) sum += first[o * 32 * n2p + e];
+      first[e] = sum;
+    }
+    __syncthreads();
+    lsum = first;
+    sums = lsum + c * n2p;
+  }
   if constexpr (KT == 0) {  // (the straight kernels touch coupled components only)
     float probe = 0.f;
 #pragma unroll
-    for (int k = 0; k < DR; ++k) probe = fc_probe(acc[k], probe);
+    for (int k = 0; k < DR; ++k) {
+      if constexpr (SK == 1) probe = fc_probe(acc[k], probe);
+      else
+#pragma unroll
+        for (int e = 0; e < 4; ++e) probe = fmaf(share < 4 ? acc[k][e] : 0.f, 0.f, probe);
+    }
     if constexpr (DX2) {
       __builtin_amdgcn_wave_barrier();
       for (int e = h; e < n2; e += 2) probe = fmaf(sums[e], 0.f, probe);
     }
-    if (__any(!(probe == 0.f))) return false;
+    const bool odd = !(probe == 0.f);
+    if (SK > 1 ? __syncthreads_or(odd) : __any(odd)) return false;
   }
-  if (z0 + c < Z) {
+  if (z0 + c < Z && share < 4) {
     TI* out = C + z * ldc + blk.c0;
 #pragma unroll
-    for (int a = 0; a < 4; ++a) {
-      const int m = n0 + 8 * a + 4 * h;
+    for (int a = 0; a < GROUPS; ++a) {
+      const int m = n0 + 8 * (SK > 1 ? share : a) + 4 * h;
       if (m >= blk.N) continue;
 #pragma unroll
       for (int q = 0; q < DR; ++q) {
@@ -542,24 +591,29 @@ __device__ __forceinline__ bool fc_tile(const FcBlock& blk, const FcPart* __rest
   if constexpr (DX2) {
     __builtin_amdgcn_wave_barrier();
     const int64_t rows = min<int64_t>(32, Z - z0);
-    for (int e = lane; e < rows * n2; e += 64) partial[z0 * n2 + e] = lsum[e / n2 * n2p + e % n2];
+    for (int e = SK > 1 ? threadIdx.x : lane; e < rows * n2; e += 64 * SK) partial[z0 * n2 + e] = lsum[e / n2 * n2p + e % n2];
   }
   return true;
 }
 
 // MAXD: the most components of any block (3 or 5): what the register budget has to hold.
-template <typename TI, int WM, bool MI, bool DX2, int MAXD, int KT>
-__global__ void __launch_bounds__(256, (MAXD > 3 || KT > 0 ? 2 : 3)) fc_rows_kernel(const FcBlock* __restrict__ blocks, const FcPart* __restrict__ parts, const float* __restrict__ coef, int nblocks,
+// SK: wavefronts that share a tile.
+template <typename TI, int WM, bool MI, bool DX2, int MAXD, int KT, int SK>
+__global__ void __launch_bounds__(SK > 4 ? 64 * SK : 256, (MAXD > 3 || KT > 0 || SK > 1 ? 2 : 3)) fc_rows_kernel(const FcBlock* __restrict__ blocks, const FcPart* __restrict__ parts, const float* __restrict__ coef, int nblocks,
                                                          int tiles_n, const TI* __restrict__ A, int64_t lda, const TI* __restrict__ W, const TI* __restrict__ X2,
                                                          int64_t ldx2, const TI* __restrict__ X1, int64_t ldx1, TI* __restrict__ C, int64_t ldc,
                                                          float* __restrict__ partial, int n2, int64_t Z) {
-  extern __shared__ __align__(16) float fc_lsum[];  // 16 fragments of weights (KT > 0), the sums of every wavefront, its rows of x2 (KT > 0)
+  extern __shared__ __align__(16) float fc_lsum[];  // 16 fragments of weights (KT > 0) or the sums of SK wavefronts, the row sums of every wavefront, its
+                                                    // rows of x2 (KT > 0)
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
   // four tiles of one row of tiles to a workgroup; with packed weights four rows of tiles under one column: they read the same weights
   // at about the same time
   int64_t zt;
   int column;
-  if constexpr (WM == kPacked) {
+  if constexpr (SK > 1) {
+    zt = blockIdx.x / tiles_n;
+    column = static_cast<int>(blockIdx.x - zt * tiles_n);
+  } else if constexpr (WM == kPacked) {
     const int64_t group = blockIdx.x / tiles_n;
     column = static_cast<int>(blockIdx.x - group * tiles_n);
     zt = group * 4 + wave;
@@ -572,20 +626,20 @@ __global__ void __launch_bounds__(256, (MAXD > 3 || KT > 0 ? 2 : 3)) fc_rows_ker
   while (b < nblocks && tile >= blocks[b].nt) tile -= blocks[b++].nt;
   const int64_t z0 = zt * 32;
   // (with weights through LDS a wavefront past the last row stays for the barriers: it reads the last row and stores nothing)
-  if (b == nblocks || (KT == 0 && z0 >= Z)) return;
+  if (b == nblocks || ((KT == 0 || SK > 1) && z0 >= Z)) return;
   const FcBlock blk = blocks[b];
   uint4* wl = reinterpret_cast<uint4*>(fc_lsum);
-  float* lsum = fc_lsum + (KT > 0 ? 16 * 64 * 4 : 0) + wave * 32 * (n2 | 1);
+  float* lsum = fc_lsum + (KT > 0 ? 16 * 64 * 4 : SK > 1 ? SK * 16 * 64 : 0) + wave * 32 * (n2 | 1);
   float* part = DX2 ? partial + static_cast<int64_t>(column) * Z * n2 : nullptr;
   bool whole = true;
   switch (blk.D) {
-    case 1: whole = fc_tile<TI, 1, WM, MI, DX2, MAXD, KT>(blk, parts, coef, A, lda, W, X2, ldx2, X1, ldx1, C, ldc, part, lsum, wl, n2, Z, z0, tile * 32); break;
-    case 3: whole = fc_tile<TI, 3, WM, MI, DX2, MAXD, KT>(blk, parts, coef, A, lda, W, X2, ldx2, X1, ldx1, C, ldc, part, lsum, wl, n2, Z, z0, tile * 32); break;
+    case 1: whole = fc_tile<TI, 1, WM, MI, DX2, MAXD, KT, SK>(blk, parts, coef, A, lda, W, X2, ldx2, X1, ldx1, C, ldc, part, lsum, wl, n2, Z, z0, tile * 32); break;
+    case 3: whole = fc_tile<TI, 3, WM, MI, DX2, MAXD, KT, SK>(blk, parts, coef, A, lda, W, X2, ldx2, X1, ldx1, C, ldc, part, lsum, wl, n2, Z, z0, tile * 32); break;
     default:
-      if constexpr (MAXD > 3) whole = fc_tile<TI, 5, WM, MI, DX2, MAXD, KT>(blk, parts, coef, A, lda, W, X2, ldx2, X1, ldx1, C, ldc, part, lsum, wl, n2, Z, z0, tile * 32);
+      if constexpr (MAXD > 3) whole = fc_tile<TI, 5, WM, MI, DX2, MAXD, KT, SK>(blk, parts, coef, A, lda, W, X2, ldx2, X1, ldx1, C, ldc, part, lsum, wl, n2, Z, z0, tile * 32);
   }
   if constexpr (KT == 0) {
-    if (!whole) fc_tile_coupled<TI>(blocks + b, parts, coef, A, lda, W, X2, ldx2, DX2 ? X1 : nullptr, ldx1, C, ldc, part, lsum, WM, MI, n2, Z, z0, tile * 32);
+    if (!whole && (SK == 1 || wave == 0)) fc_tile_coupled<TI>(blocks + b, parts, coef, A, lda, W, X2, ldx2, DX2 ? X1 : nullptr, ldx1, C, ldc, part, lsum, WM, MI, n2, Z, z0, tile * 32);
   }
 }
 
@@ -1101,18 +1155,31 @@ extern "C" int cueq_fc_flex(int32_t dtype, int32_t gradient, int32_t mul_ir, int
                    lda % epv == 0 && ldc % epv == 0 && ldx1 % epv == 0,
                CUEQ_ERR_UNSUPPORTED, "fc_flex: rows must be 16-byte aligned");
   const int64_t row_tiles = (rows + 31) / 32;
-  const int64_t grid = packed ? (row_tiles + 3) / 4 * column_tiles : (row_tiles * column_tiles + 3) / 4;
+  const bool held = packed && packed <= 4 && most_components <= 3;  // (source blocks in registers, channel by channel)
+  // Few tiles: eight (four) wavefronts share one.  A tile is one serial chain over the paths and channels, 150 us for float and 16
+  // channels, and four times fewer rows took no less.  us for one / shared, forward + backward, 1 000, 4 000 and 8 000 rows of
+  // 0e+1o blocks: 64 ch (x) 16 float 463 / 133, 547 / 287, 661 / 542 (1 000 tiles); 64 (x) 4 float 129 / 59, 158 / 100, 186 / 180;
+  // 64 (x) 16 bfloat16 113 / 74, 121 / 90, 138 / 136; 64 (x) 4 bfloat16 56 / 54, 70 / 65, 77 / 92.
+  const int64_t tiles = row_tiles * column_tiles;
+  const int share = held ? (tiles <= 2 * device_cus() ? 4 : 1) : tiles <= 3 * device_cus() && n2 <= 64 ? 8 : 1;  // (n2: 100 KB of LDS)
+  const int64_t grid = share > 1 ? row_tiles * column_tiles : packed ? (row_tiles + 3) / 4 * column_tiles : (row_tiles * column_tiles + 3) / 4;
   CUEQ_REQUIRE(grid < (1ll << 31), CUEQ_ERR_TOO_LARGE, "fc_flex: too many rows");
-  const size_t lds = (dX2 ? 4 * 32 * (n2 | 1) * sizeof(float) : 0) + (packed && packed <= 4 && most_components <= 3 ? 16 * 1024 + 4 * 32 * fc_x2_words(n2) * sizeof(uint32_t) : 0);
+  const size_t lds = (dX2 ? std::max(4, share) * 32 * (n2 | 1) * sizeof(float) : 0) +
+                     (held ? 16 * 1024 + 4 * 32 * fc_x2_words(n2) * sizeof(uint32_t) : share > 1 ? share * 16 * 64 * sizeof(float) : 0);
   KernelTimer timer(gradient ? "fc_flex_dx" : "fc_flex_fwd", stream);
 #define FC_GD(TI, WM, MI, DX, MD, KT)                                                                                                            \
   do {                                                                                                                                         \
-    if (lds > 64 * 1024)                                                                                                                       \
-      CUEQ_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(fc_rows_kernel<TI, WM, MI, DX, MD, KT>),                                \
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));                                  \
-    FC_GL(TI, WM, MI, DX, MD, KT);                                                                                                             \
+    if (share > 1) FC_GE(TI, WM, MI, DX, MD, KT, (KT > 0 ? 4 : 8));                                                                            \
+    else FC_GE(TI, WM, MI, DX, MD, KT, 1);                                                                                                     \
   } while (0)
-#define FC_GL(TI, WM, MI, DX, MD, KT) hipLaunchKernelGGL((fc_rows_kernel<TI, WM, MI, DX, MD, KT>), dim3(static_cast<unsigned>(grid)), dim3(256), lds, stream, static_cast<const FcBlock*>(blocks), static_cast<const FcPart*>(parts), coef, nblocks, column_tiles, static_cast<const TI*>(A), lda, static_cast<const TI*>(W), static_cast<const TI*>(X2), ldx2, static_cast<const TI*>(X1), ldx1, static_cast<TI*>(C), ldc, partial, n2, rows)
+#define FC_GE(TI, WM, MI, DX, MD, KT, SK)                                                                                                            \
+  do {                                                                                                                                         \
+    if (lds > 64 * 1024)                                                                                                                       \
+      CUEQ_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(fc_rows_kernel<TI, WM, MI, DX, MD, KT, SK>),                                \
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));                                  \
+    FC_GL(TI, WM, MI, DX, MD, KT, SK);                                                                                                             \
+  } while (0)
+#define FC_GL(TI, WM, MI, DX, MD, KT, SK) hipLaunchKernelGGL((fc_rows_kernel<TI, WM, MI, DX, MD, KT, SK>), dim3(static_cast<unsigned>(grid)), dim3(SK > 4 ? 64 * SK : 256), lds, stream, static_cast<const FcBlock*>(blocks), static_cast<const FcPart*>(parts), coef, nblocks, column_tiles, static_cast<const TI*>(A), lda, static_cast<const TI*>(W), static_cast<const TI*>(X2), ldx2, static_cast<const TI*>(X1), ldx1, static_cast<TI*>(C), ldc, partial, n2, rows)
 #define FC_GK(TI, MI, DX)                                              \
   do {                                                                 \
     if constexpr (sizeof(TI) == 2) {                                   \
@@ -1139,6 +1206,7 @@ extern "C" int cueq_fc_flex(int32_t dtype, int32_t gradient, int32_t mul_ir, int
 #undef FC_GO
 #undef FC_GK
 #undef FC_GD
+#undef FC_GE
 #undef FC_GL
   CUEQ_CHECK_HIP(hipGetLastError());
   if (dX2) {
