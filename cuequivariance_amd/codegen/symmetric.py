@@ -312,13 +312,13 @@ def emit_unit(st: SymmetricStructure, T: str, name: str, fwd_hash: int, bwd_hash
     A("template <bool NEED_DW, bool NEED_DX>")
     A(f"__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu({bwd_waves}))) bwd_kernel(")
     A(f"    const TI* __restrict__ w, const TI* __restrict__ x, const TI* __restrict__ g, TI* __restrict__ dw, TI* __restrict__ dx,")
-    A(f"    {T}* __restrict__ part, const void* __restrict__ w_index, int idx64, const int64_t* __restrict__ csr_perm, int64_t batch) {{")
+    A(f"    {T}* __restrict__ part, const void* __restrict__ w_index, int idx64, const int64_t* __restrict__ csr_perm, int64_t range, int64_t longer) {{")
     A("  const int lane = threadIdx.x;")
-    A(f"  const int ch = blockIdx.x % {nch}; const int64_t slot = blockIdx.x / {nch}; const int64_t nslots = gridDim.x / {nch};")
+    A(f"  const int ch = blockIdx.x % {nch}; const int64_t slot = blockIdx.x / {nch}; ")
     A(lane_setup)
     if stage_decl:
         A(stage_decl)
-    A("  const int64_t p0 = slot * batch / nslots, p1 = (slot + 1) * batch / nslots;")
+    A("  const int64_t p0 = slot * range + (slot < longer ? slot : longer), p1 = p0 + range + (slot < longer ? 1 : 0);")
     A("  if (p0 >= p1) return;")
     for s in w_used:
         A(f"  {T} q{s} = 0, wv{s} = 0;")
@@ -398,38 +398,39 @@ def emit_unit(st: SymmetricStructure, T: str, name: str, fwd_hash: int, bwd_hash
     A("// dw[e] = head / tail partials of the slots that meet the index group e; groups stored directly by one slot are left")
     A("// alone, empty groups are zeroed.  Positions [a, b) of the grouped order hold exactly the rows of group e, so a slot")
     A("// [q0, q1) contributes its head partial when a <= q0 < b (e is its first group) and its tail partial when only its")
-    A("// last position lies in [a, b).  One block = 64 weight columns x 16 slot lanes; the 16 partial sums are added in lane")
+    A("// last position lies in [a, b).  One block = 64 weight columns x 8 slot lanes; the 8 partial sums are added in lane")
     A("// order (fixed, so the result does not change from run to run).")
-    A(f"__global__ void __launch_bounds__(1024) fold_kernel(const {T}* __restrict__ part, TI* __restrict__ dw,")
-    A("    const int64_t* __restrict__ csr_offsets, int64_t batch, int64_t nslots, int64_t row0) {")
-    A(f"  __shared__ {T} s_acc[16][64];")
-    A("  __shared__ int s_any[16];")
+    A(f"__global__ void __launch_bounds__(512) fold_kernel(const {T}* __restrict__ part, TI* __restrict__ dw,")
+    A("    const int64_t* __restrict__ csr_offsets, int64_t range, int64_t longer, int64_t row0) {")
+    A(f"  __shared__ {T} s_acc[8][64];")
+    A("  __shared__ int s_any[8];")
     A("  const int64_t e = row0 + blockIdx.y;")
     A("  const int jl = threadIdx.x & 63, sl = threadIdx.x >> 6;")
     A("  const int j = blockIdx.x * 64 + jl;")
     A(f"  const bool live = j < {W};")
     A("  const int64_t a = csr_offsets[e], b = csr_offsets[e + 1];")
     A(f"  if (a == b) {{ if (sl == 0 && live) io_st({T}(0), dw + e * {W}ll + j); return; }}")
-    A("  // slots whose range [s * batch / nslots, (s + 1) * batch / nslots) meets [a, b)")
-    A("  int64_t s_lo = a * nslots / batch, s_hi = (b - 1) * nslots / batch;")
-    A("  while (s_lo > 0 && (s_lo * batch / nslots) > a) --s_lo;")
-    A("  while ((s_lo + 1) * batch / nslots <= a) ++s_lo;")
-    A("  while (s_hi + 1 < nslots && ((s_hi + 1) * batch / nslots) < b) ++s_hi;")
-    A("  while (s_hi * batch / nslots >= b) --s_hi;")
+    A("  // slots whose range meets [a, b): range positions each, the first `longer` of them one more (two divisions a block: a slot's")
+    A("  // range as slot * batch / slots took two for every partial, most of the kernel's time: 20 011 nodes of 128 ch l <= 3 18.4 us")
+    A("  // with them and 16 slot lanes, 11.9 without)")
+    A("  const int64_t bound = longer * (range + 1);")
+    A("  const auto slot_of = [&](int64_t p) { return p < bound ? p / (range + 1) : longer + (p - bound) / range; };")
+    A("  const int64_t s_lo = slot_of(a), s_hi = slot_of(b - 1);")
     A(f"  {T} acc = 0; bool any = false;")
-    A("  for (int64_t s = s_lo + sl; s <= s_hi; s += 16) {")
-    A("    const int64_t q0 = s * batch / nslots, q1 = (s + 1) * batch / nslots;")
-    A("    if (q0 >= q1) continue;")
-    A("    int half = -1;")
-    A("    if (q0 >= a && q0 < b) half = 0; else if (q1 - 1 >= a && q1 - 1 < b) half = 1;")
-    A(f"    if (half >= 0) {{ any = true; if (live) acc += part[(s * 2 + half) * {W}ll + j]; }}")
+    A(f"  const {T}* __restrict__ column = part + (live ? j : 0);")
+    A("#pragma unroll 8")
+    A("  for (int64_t s = s_lo + sl; s <= s_hi; s += 8) {")
+    A("    const int64_t q0 = s * range + (s < longer ? s : longer), q1 = q0 + range + (s < longer ? 1 : 0);")
+    A("    const int half = q0 >= a && q0 < b ? 0 : q1 - 1 >= a && q1 - 1 < b ? 1 : -1;")
+    A(f"    const {T} v = column[(s * 2 + (half > 0 ? 1 : 0)) * {W}ll];  // (read either way, so that the reads do not wait for each other)")
+    A("    acc += half >= 0 ? v : 0; any = any || half >= 0;")
     A("  }")
     A("  s_acc[sl][jl] = acc;")
     A("  if (jl == 0) s_any[sl] = any ? 1 : 0;")
     A("  __syncthreads();")
     A("  if (sl == 0 && live) {")
     A(f"    {T} total = 0; int seen = 0;")
-    A("    for (int t = 0; t < 16; ++t) { total += s_acc[t][jl]; seen |= s_any[t]; }")
+    A("    for (int t = 0; t < 8; ++t) { total += s_acc[t][jl]; seen |= s_any[t]; }")
     A(f"    if (seen) io_st(total, dw + e * {W}ll + j);")
     A("  }")
     A("}")
@@ -501,15 +502,15 @@ static int run_bwd(const SpecCall& c) {{
     KernelTimer timer("{name}_bwd_{tag}", c.stream);
     hipLaunchKernelGGL((bwd_kernel<NEED_DW, NEED_DX>), dim3(static_cast<unsigned>(nslots * {nch})), dim3(64), 0, c.stream,
                        static_cast<const TI*>(b[0].data), static_cast<const TI*>(b[1].data), static_cast<const TI*>(b[2].data), dw,
-                       bdx ? static_cast<TI*>(bdx->data) : nullptr, part, b[0].index, b[0].index_is_64, perm, batch);
+                       bdx ? static_cast<TI*>(bdx->data) : nullptr, part, b[0].index, b[0].index_is_64, perm, batch / nslots, batch % nslots);
   }}
   CUEQ_CHECK_HIP(hipGetLastError());
   if (NEED_DW) {{
     // (the grid's y extent is the number of weight rows: at most 65535 of them per launch)
     for (int64_t r0 = 0; r0 < bdw->rows; r0 += 65535) {{
       const int64_t nr = bdw->rows - r0 < 65535 ? bdw->rows - r0 : 65535;
-      hipLaunchKernelGGL(fold_kernel, dim3(({W} + 63) / 64, static_cast<unsigned>(nr)), dim3(1024), 0, c.stream, part, dw, bdw->csr_offsets,
-                         batch, nslots, r0);
+      hipLaunchKernelGGL(fold_kernel, dim3(({W} + 63) / 64, static_cast<unsigned>(nr)), dim3(512), 0, c.stream, part, dw, bdw->csr_offsets,
+                         batch / nslots, batch % nslots, r0);
     }}
     CUEQ_CHECK_HIP(hipGetLastError());
   }}
