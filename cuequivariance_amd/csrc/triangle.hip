@@ -15,6 +15,7 @@
 // cuequivariance_torch/primitives/triangle.py:138-262 forwards to a closed kernel).
 
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 #include "cw_common.h"
@@ -240,10 +241,16 @@ __device__ __forceinline__ uint4 gemm_fragment(const char* tile, int base, int q
 
 // WM x WN wavefronts of 64 x 64 per block: 2 x 2 (a 128 x 128 tile) by default; 4 x 4 (256 x 256, 16 wavefronts) halves
 // the operand traffic between L2 and the CUs for products whose both extents are large.
+// EDGE: some tiles are partly filled.  A wavefront forms only those of its four subtiles that reach into C, and which wavefront has
+// which quarter goes round (the first ones of a partial tile have more to do, and a wavefront's number decides its SIMD); the bound on
+// registers keeps the accumulators of four wavefronts beside their operands and four (three) blocks on a CU.  128 products of n x n,
+// bfloat16, us with all subtiles always / with EDGE, both operands by rows: 480 55.7 / 48.6, 392 (4 x 4 tiles of 128, the last 8 wide)
+// 47.3 / 43.6, 264 23.0 / 21.4; by columns 47.5 / 45.2, 39.8 / 36.3, 20.7 / 19.4; whole tiles lose 1 - 3 % with it.  (Loads left
+// out as well, behind a condition, make every wait one for all loads: 392 47 us, 384 29 -> 38.)
 // KB: bytes of k per row and step; 128 makes every request of a contraction-contiguous operand a whole 128-byte line (with
 // 64 a line is fetched in two halves one step apart, and a 256 x 256 step turns over the whole L1 in between).
-template <typename TI, typename TO, bool TA, bool TB, int WM = 2, int WN = 2, int KB = 64>
-__global__ void __launch_bounds__(64 * WM * WN) gemm_kernel(const TI* __restrict__ A, int64_t lda, int64_t sA,
+template <typename TI, typename TO, bool TA, bool TB, int WM = 2, int WN = 2, int KB = 64, bool EDGE = false>
+__global__ void __launch_bounds__(64 * WM * WN, (!EDGE ? 1 : TA && !TB ? 3 : 4)) gemm_kernel(const TI* __restrict__ A, int64_t lda, int64_t sA,
                                                    const TI* __restrict__ B, int64_t ldb, int64_t sB,
                                                    TO* __restrict__ C, int64_t ldc, int64_t sC, int Mfull, int N, int Kfull,
                                                    float alpha, int accumulate, int vec_out, int64_t k_total, int nparts, int64_t pA,
@@ -261,9 +268,11 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_kernel(const TI* __restrict
   __shared__ __align__(16) char smem[2][ABYTES + BBYTES];
   const int tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63, c = lane & 31, h = lane >> 5;
-  const int wm = wave / WN, wn = wave % WN;
   int bx, by, bz;
   xcd_tile(bx, by, bz);
+  const int place = EDGE ? __builtin_amdgcn_readfirstlane(wave) ^ ((bx + by + bz) & 3) : wave;
+  static_assert(!EDGE || WM * WN == 4, "four wavefronts change places");
+  const int wm = place / WN, wn = place % WN;
   int m0 = by * TMR, M = Mfull;
   const int n0 = bx * TNC;
   // batch item = (chunk, part): strides s* between chunks, p* between parts (nparts == 1: a plain batch)
@@ -345,40 +354,59 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_kernel(const TI* __restrict
 
   const int nsteps = (K + BK - 1) / BK;
   if (nsteps > 0) load_step(0);
-  int buf = 0;
-  for (int ks = 0; ks < nsteps; ++ks) {
-    store_step(buf);
-    __syncthreads();
-    if (ks + 1 < nsteps) load_step(ks + 1);
-    uint4 fa[2][NQ], fb[2][NQ];
+  // NI x NJ of the wavefront's subtiles (the barriers are the same on every way)
+  auto steps = [&](auto ni, auto nj) {
+    constexpr int NI = decltype(ni)::value, NJ = decltype(nj)::value;
+    int buf = 0;
+    for (int ks = 0; ks < nsteps; ++ks) {
+      store_step(buf);
+      __syncthreads();
+      if (ks + 1 < nsteps) load_step(ks + 1);
+      if constexpr (NI > 0 && NJ > 0) {
+        uint4 fa[NI][NQ], fb[NJ][NQ];
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+        for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int q = 0; q < NQ; ++q) {
-        fa[t][q] = gemm_fragment<TI, TA, TMR, KB>(&smem[buf][0], wm * 64 + t * 32, q, lane);
-        fb[t][q] = gemm_fragment<TI, TB, TNC, KB>(&smem[buf][ABYTES], wn * 64 + t * 32, q, lane);
+          for (int q = 0; q < NQ; ++q) {
+            if (t < NI) fa[t < NI ? t : 0][q] = gemm_fragment<TI, TA, TMR, KB>(&smem[buf][0], wm * 64 + t * 32, q, lane);
+            if (t < NJ) fb[t < NJ ? t : 0][q] = gemm_fragment<TI, TB, TNC, KB>(&smem[buf][ABYTES], wn * 64 + t * 32, q, lane);
+          }
+        // consecutive MFMAs go to different accumulators: a dependent one would wait for its predecessor to drain
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+          if constexpr (sizeof(TI) == 2) {
+#pragma unroll
+            for (int i = 0; i < NI; ++i)
+#pragma unroll
+              for (int j = 0; j < NJ; ++j)
+                acc[i][j] = mm_32x32x16<F>(fa[i][q], fb[j][q], acc[i][j]);
+          } else {
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+              for (int i = 0; i < NI; ++i)
+#pragma unroll
+                for (int j = 0; j < NJ; ++j)
+                  acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(reinterpret_cast<const float*>(&fa[i][q])[s],
+                                                                   reinterpret_cast<const float*>(&fb[j][q])[s], acc[i][j], 0, 0, 0);
+          }
+        }
       }
-    // consecutive MFMAs go to different accumulators: a dependent one would wait for its predecessor to drain
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-      if constexpr (sizeof(TI) == 2) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-          for (int j = 0; j < 2; ++j)
-            acc[i][j] = mm_32x32x16<F>(fa[i][q], fb[j][q], acc[i][j]);
-      } else {
-#pragma unroll
-        for (int s = 0; s < 4; ++s)
-#pragma unroll
-          for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(reinterpret_cast<const float*>(&fa[i][q])[s],
-                                                               reinterpret_cast<const float*>(&fb[j][q])[s], acc[i][j], 0, 0, 0);
-      }
+      buf ^= 1;
     }
-    buf ^= 1;
+  };
+  constexpr std::integral_constant<int, 0> none;
+  constexpr std::integral_constant<int, 1> one;
+  constexpr std::integral_constant<int, 2> two;
+  const int mi = M - (m0 + wm * 64), nj = N - (n0 + wn * 64);  // rows and columns that exist
+  if constexpr (EDGE) {
+    if (mi > 32 && nj > 32) steps(two, two);
+    else if (mi <= 0 || nj <= 0) steps(none, none);
+    else if (mi > 32) steps(two, one);
+    else if (nj > 32) steps(one, two);
+    else steps(one, one);
+  } else {
+    steps(two, two);
   }
 
   // 2-byte results, whole wavefront tile inside C, 16-byte aligned rows: through LDS, 32 rows at a time (4-byte
@@ -2642,7 +2670,7 @@ extern "C" int cueq_gemm(int32_t in_dtype, int32_t out_dtype, int32_t trans_a, i
     const dim3 grid_big(static_cast<unsigned>(N / 256), static_cast<unsigned>(M / 256), static_cast<unsigned>(batch));
 #define GEMM_ARGS(TI, TO) static_cast<const TI*>(A), lda, stride_a, static_cast<const TI*>(B), ldb, stride_b, static_cast<TO*>(C), ldc, stride_c, m, n, k, al, accumulate, vec_out, 0, 1, 0, 0, 0, nullptr, 0, 0, 0, 0
 #define GEMM_LAUNCH(TI, TO, TA, TB) hipLaunchKernelGGL((gemm_kernel<TI, TO, TA, TB>), grid, dim3(256), 0, stream, GEMM_ARGS(TI, TO))
-#define GEMM_SZ(TI, TA, TB) do { if (big) hipLaunchKernelGGL((gemm_kernel<TI, TI, TA, TB, 4, 4, (sizeof(TI) == 2 ? 128 : 64)>), grid_big, dim3(1024), 0, stream, GEMM_ARGS(TI, TI)); else GEMM_LAUNCH(TI, TI, TA, TB); } while (0)
+#define GEMM_SZ(TI, TA, TB) do { if (big) hipLaunchKernelGGL((gemm_kernel<TI, TI, TA, TB, 4, 4, (sizeof(TI) == 2 ? 128 : 64)>), grid_big, dim3(1024), 0, stream, GEMM_ARGS(TI, TI)); else if (sizeof(TI) == 2 && (M % kTile || N % kTile) && (M > kTile || N > kTile)) hipLaunchKernelGGL((gemm_kernel<TI, TI, TA, TB, 2, 2, 64, sizeof(TI) == 2>), grid, dim3(256), 0, stream, GEMM_ARGS(TI, TI)); else GEMM_LAUNCH(TI, TI, TA, TB); } while (0)
 #define GEMM_TR(TI) do { if (trans_a && trans_b) GEMM_SZ(TI, true, true); else if (trans_a) GEMM_SZ(TI, true, false); else if (trans_b) GEMM_SZ(TI, false, true); else GEMM_SZ(TI, false, false); } while (0)
     if (in_dtype == CUEQ_F32 && out_dtype == CUEQ_F32) GEMM_TR(float);
     else if (in_dtype == CUEQ_F32 && out_dtype == CUEQ_F16) GEMM_LAUNCH(float, f16bits, false, false);
