@@ -2531,33 +2531,37 @@ __global__ void __launch_bounds__(1024) sum_rows_lds_kernel(const TI* __restrict
 }
 
 // the two halves of in (2 x R x Ccols) summed over their rows in one launch (grid.y = half; a null result is skipped): the
-// per-block partials of a LayerNorm's dgamma and dbeta.  (One thread per column over all rows took 243 us for 1024 rows of 128
-// columns - one load in flight at a time on one CU; sixteen row lanes with four loads each take 7.)
+// per-block partials of a LayerNorm's dgamma and dbeta.  Bound by the latency of a lane's chain of loads: 16 columns x 64 row lanes a
+// block, every lane adds rows r = lane, lane + 64, ... in order, eight loads in flight, and the 64 sums are added pairwise in a fixed
+// order (2 x 1 024 rows of 128 columns: one thread per column 243 us, 64 columns x 16 row lanes and four loads 6.9, this 4.7;
+// 2 048 rows: 10 and 5.2).
 __global__ void __launch_bounds__(1024) fold_two_kernel(const float* __restrict__ in, float* __restrict__ out0, float* __restrict__ out1, int64_t R,
                                                         int64_t Ccols) {
-  __shared__ float s_acc[16][64];
+  __shared__ float s_acc[64][17];
   float* out = blockIdx.y ? out1 : out0;
   if (!out) return;
   const float* p = in + static_cast<int64_t>(blockIdx.y) * R * Ccols;
-  const int cl = threadIdx.x & 63, rl = threadIdx.x >> 6;
-  const int64_t cc = static_cast<int64_t>(blockIdx.x) * 64 + cl;
+  const int cl = threadIdx.x & 15, rl = threadIdx.x >> 4;
+  const int64_t cc = static_cast<int64_t>(blockIdx.x) * 16 + cl;
   float s = 0;
   if (cc < Ccols) {
     int64_t r = rl;
-    for (; r + 48 < R; r += 64) {
-      const float v0 = p[r * Ccols + cc], v1 = p[(r + 16) * Ccols + cc], v2 = p[(r + 32) * Ccols + cc], v3 = p[(r + 48) * Ccols + cc];
-      s += v0; s += v1; s += v2; s += v3;
+    for (; r + 7 * 64 < R; r += 8 * 64) {
+      float v[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = p[(r + 64 * k) * Ccols + cc];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) s += v[k];
     }
-    for (; r < R; r += 16) s += p[r * Ccols + cc];
+    for (; r < R; r += 64) s += p[r * Ccols + cc];
   }
   s_acc[rl][cl] = s;
-  __syncthreads();
-  if (rl == 0 && cc < Ccols) {
-    float total = 0;
 #pragma unroll
-    for (int t = 0; t < 16; ++t) total += s_acc[t][cl];
-    out[cc] = total;
+  for (int half = 32; half > 0; half /= 2) {
+    __syncthreads();
+    if (rl < half) s_acc[rl][cl] += s_acc[rl + half][cl];
   }
+  if (rl == 0 && cc < Ccols) out[cc] = s_acc[0][cl];
 }
 
 // rows of a padded square from the caller's rows - the pair tensor and the mask (a null `in`: ones) as PairRows says, or with zeros
@@ -3215,7 +3219,7 @@ static int layer_norm_bwd_impl(int32_t dtype, int64_t rows, int64_t D, const voi
     }
   }
   CUEQ_CHECK_HIP(hipGetLastError());
-  if (dgamma || dbeta) hipLaunchKernelGGL(fold_two_kernel, dim3(static_cast<unsigned>((D + 63) / 64), 2), dim3(1024), 0, stream, part, dgamma, dbeta, nb, D);
+  if (dgamma || dbeta) hipLaunchKernelGGL(fold_two_kernel, dim3(static_cast<unsigned>((D + 15) / 16), 2), dim3(1024), 0, stream, part, dgamma, dbeta, nb, D);
   CUEQ_CHECK_HIP(hipGetLastError());
   return CUEQ_OK;
 }
@@ -3338,7 +3342,7 @@ extern "C" int cueq_layer_norm_t_bwd(int32_t dtype, int64_t M, int64_t D, const 
                  hipLaunchKernelGGL(ln_t_bwd_kernel<f16bits>, dim3(static_cast<unsigned>(nb)), dim3(256), bwd_lds, stream, static_cast<const f16bits*>(dy), static_cast<const f16bits*>(x_t), mean, rstd, static_cast<const f16bits*>(gamma), static_cast<f16bits*>(dx_t), part, M, static_cast<int>(D), ntiles, need_affine));
   }
   CUEQ_CHECK_HIP(hipGetLastError());
-  if (dgamma || dbeta) hipLaunchKernelGGL(fold_two_kernel, dim3(static_cast<unsigned>((D + 63) / 64), 2), dim3(1024), 0, stream, part, dgamma, dbeta, nb, D);
+  if (dgamma || dbeta) hipLaunchKernelGGL(fold_two_kernel, dim3(static_cast<unsigned>((D + 15) / 16), 2), dim3(1024), 0, stream, part, dgamma, dbeta, nb, D);
   CUEQ_CHECK_HIP(hipGetLastError());
   return CUEQ_OK;
 }
