@@ -1084,11 +1084,22 @@ __global__ void __launch_bounds__((SPLIT ? 256 : 512), (SPLIT ? 1 : 2))
   char* stage = reinterpret_cast<char*>(sb + 2 * C) + wave * (8 * SSTR);  // (two inputs only)
   float* sg = sb + 2 * C;                                                   // (LNB only) gamma[K]
 
-  for (int e = tid; e < C * VPR; e += NTH) {
-    const int r = e / VPR, part = e % VPR;
-    const int po = (part ^ swz(r)) << 4;
-    *reinterpret_cast<uint4*>(sw1 + r * WSTR + po) = *reinterpret_cast<const uint4*>(W1 + static_cast<int64_t>(r) * ldw + part * EPV);
-    *reinterpret_cast<uint4*>(sw2 + r * WSTR + po) = *reinterpret_cast<const uint4*>(W2 + static_cast<int64_t>(r) * ldw + part * EPV);
+  for (int e0 = tid; e0 < C * VPR; e0 += 4 * NTH) {
+    u32x4_t w1[4], w2[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {  // (eight requests in flight: 2 us less a launch than piece by piece; past the end the last one again)
+      const int e = min(e0 + i * NTH, C * VPR - 1);
+      const int64_t o = static_cast<int64_t>(e / VPR) * ldw + (e % VPR) * EPV;
+      w1[i] = *reinterpret_cast<const u32x4_t*>(W1 + o);
+      w2[i] = *reinterpret_cast<const u32x4_t*>(W2 + o);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int e = min(e0 + i * NTH, C * VPR - 1);
+      const int r = e / VPR, po = ((e % VPR) ^ swz(r)) << 4;
+      *reinterpret_cast<u32x4_t*>(sw1 + r * WSTR + po) = w1[i];
+      *reinterpret_cast<u32x4_t*>(sw2 + r * WSTR + po) = w2[i];
+    }
   }
   for (int i = tid; i < C; i += NTH) {
     sb[i] = bias1 ? tri_load(bias1, i) : 0.f;
@@ -1115,7 +1126,10 @@ __global__ void __launch_bounds__((SPLIT ? 256 : 512), (SPLIT ? 1 : 2))
     if constexpr (PAD && !DC_BY_ROW) mld = max(pairs.src(mld), 0);
     return DC_BY_ROW ? static_cast<uint32_t>(((4 * h + (lane & 1)) * ldc + (mld & ~1)) * ES) : static_cast<uint32_t>((mld * ldc + 4 * h) * ES);
   };
-  int64_t ptile = static_cast<int64_t>(blockIdx.x) * NWAVES + wave;
+  // (tiles dealt out wavefront-major, as in dual_gate_res_kernel; by rows, the two tiles of 64 bytes that share the lines of dC, dU
+  // and dV go to neighbouring wavefronts)
+  constexpr int kNear = DC_BY_ROW ? 2 : 1;
+  int64_t ptile = (static_cast<int64_t>(wave / kNear) * gridDim.x + blockIdx.x) * kNear + wave % kNear;
   int pci = 0;
   uint32_t pofs = ptile < ntiles ? dc_lane_offset(tile_row(ptile)) : 0u;
   auto request_dc = [&](uint32_t (&dst)[8]) {
@@ -1463,24 +1477,13 @@ __global__ void __launch_bounds__(512, 2)
   // (the wavefront's number as a scalar: tile indices and row bases derived from it stay in scalar registers)
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, c = lane & 31, h = lane >> 5;
 
-  for (int e = tid; e < C * VPR; e += NTH) {
-    const int r = e / VPR, part = e % VPR;
-    const int po = (part ^ swz(r)) << 4;
-    *reinterpret_cast<uint4*>(sw1 + r * WSTR + po) = *reinterpret_cast<const uint4*>(W1 + static_cast<int64_t>(r) * ldw + part * EPV);
-    *reinterpret_cast<uint4*>(sw2 + r * WSTR + po) = *reinterpret_cast<const uint4*>(W2 + static_cast<int64_t>(r) * ldw + part * EPV);
-  }
-  for (int i = tid; i < C; i += NTH) {
-    sb[i] = bias1 ? tri_load(bias1, i) : 0.f;
-    sb[C + i] = bias2 ? tri_load(bias2, i) : 0.f;
-  }
-  if constexpr (LN) {
-    for (int i = tid; i < K; i += NTH) {
-      sg[i] = gamma ? tri_load(gamma, i) : 1.f;
-      sg[K + i] = beta ? tri_load(beta, i) : 0.f;
-    }
-  }
-  __syncthreads();
-
+  // (few tiles: the weight rows are dealt out over grid.y as well, C of them each)
+  const int64_t row0 = static_cast<int64_t>(blockIdx.y) * C;
+  W1 += row0 * ldw;
+  W2 += row0 * ldw;
+  out += ROWS ? row0 : row0 * ldc;
+  if (bias1) bias1 += row0;
+  if (bias2) bias2 += row0;
   const int nchunks = C / 32;
   const int64_t ntiles = (static_cast<int64_t>(M) + 32 * NT - 1) / (32 * NT);
   const int64_t tstep = static_cast<int64_t>(gridDim.x) * NWAVES;
@@ -1510,6 +1513,35 @@ __global__ void __launch_bounds__(512, 2)
   // all CUs - 3 us less per launch than with the eight tiles of a block next to each other)
   const int64_t tile0 = static_cast<int64_t>(wave) * gridDim.x + blockIdx.x;
   if (tile0 < ntiles) request_x(tile0);
+  for (int e0 = tid; e0 < C * VPR; e0 += 4 * NTH) {
+    u32x4_t w1[4], w2[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {  // (eight requests in flight: 2 us less a launch than piece by piece; past the end the last one again)
+      const int e = min(e0 + i * NTH, C * VPR - 1);
+      const int64_t o = static_cast<int64_t>(e / VPR) * ldw + (e % VPR) * EPV;
+      w1[i] = *reinterpret_cast<const u32x4_t*>(W1 + o);
+      w2[i] = *reinterpret_cast<const u32x4_t*>(W2 + o);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int e = min(e0 + i * NTH, C * VPR - 1);
+      const int r = e / VPR, po = ((e % VPR) ^ swz(r)) << 4;
+      *reinterpret_cast<u32x4_t*>(sw1 + r * WSTR + po) = w1[i];
+      *reinterpret_cast<u32x4_t*>(sw2 + r * WSTR + po) = w2[i];
+    }
+  }
+  for (int i = tid; i < C; i += NTH) {
+    sb[i] = bias1 ? tri_load(bias1, i) : 0.f;
+    sb[C + i] = bias2 ? tri_load(bias2, i) : 0.f;
+  }
+  if constexpr (LN) {
+    for (int i = tid; i < K; i += NTH) {
+      sg[i] = gamma ? tri_load(gamma, i) : 1.f;
+      sg[K + i] = beta ? tri_load(beta, i) : 0.f;
+    }
+  }
+  __syncthreads();
+
   for (int64_t tile = tile0; tile < ntiles; tile += tstep) {
     uint4 xf[NT][NS][2], xf2[1][NS][2];
     float mk[NT];
@@ -1584,10 +1616,10 @@ __global__ void __launch_bounds__(512, 2)
               o[e] = pack16<F>(ln_affine(__fsub_rn(lo16<F>(w[e]), mu), rs, gm[2 * e], bt[2 * e]),
                                ln_affine(__fsub_rn(hi16<F>(w[e]), mu), rs, gm[2 * e + 1], bt[2 * e + 1]));
             xf[t][s2][q] = make_uint4(o[0], o[1], o[2], o[3]);
-            if (mcol[t] < M) *reinterpret_cast<uint4*>(xhat + static_cast<int64_t>(mld) * ldxh + (s2 * 64 + h * 32 + q * 16) / ES) = xf[t][s2][q];
+            if (mcol[t] < M && blockIdx.y == 0) *reinterpret_cast<uint4*>(xhat + static_cast<int64_t>(mld) * ldxh + (s2 * 64 + h * 32 + q * 16) / ES) = xf[t][s2][q];
             __builtin_amdgcn_sched_barrier(0);  // one piece at a time: its gamma / beta values die here
           }
-        if (h == 0 && mcol[t] < M) {
+        if (h == 0 && mcol[t] < M && blockIdx.y == 0) {
           mean[mld] = mu;
           rstd[mld] = rs;
         }
@@ -2830,13 +2862,19 @@ static int launch_dual_gate_res(int64_t C, int64_t M, int64_t K, const void* W1,
                                 const void* beta, float eps, void* xhat, int64_t ldxh, float* mean, float* rstd, bool half, hipStream_t stream,
                                 PairRows pairs = PairRows()) {
   const bool by_rows = X2 != nullptr;
-  const size_t lds = dual_gate_res_lds(C, K, xhat != nullptr);
   const int64_t ntiles = (M + (by_rows ? 31 : 63)) / (by_rows ? 32 : 64);
-  int64_t gx = (ntiles + 7) / 8;
-  if (gx > device_cus()) gx = device_cus();
+  // Tiles go to the CUs first, then to their wavefronts; where that leaves SIMDs idle, the weight rows are split over grid.y too, as
+  // long as the units then number no more than the SIMDs (each part repeats the LayerNorm, so more cost what they save).  The
+  // LayerNorm form, 256 weight rows: 64 x 64 rows took 35 us with eight tiles to a block, 25 with one, 16.6 in two parts, 15.0 in
+  // eight; 256 x 256 rows 39 with eight tiles to a block, 28.4 with four, 29.0 with eight halves.
+  int64_t parts = 1;
+  while (parts < 8 && (C / 32) % (2 * parts) == 0 && 2 * parts * ntiles <= 4 * device_cus()) parts *= 2;
+  C /= parts;
+  const size_t lds = dual_gate_res_lds(C, K, xhat != nullptr);
+  const int64_t gx = std::min<int64_t>(ntiles, std::max<int64_t>(1, device_cus() / parts));
 #define DGR_F(FT, KT, LN, RW, PD) do { auto kfn = dual_gate_res_kernel<FT, KT, LN, RW, PD>; \
     CUEQ_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kfn), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds))); \
-    hipLaunchKernelGGL(kfn, dim3(static_cast<unsigned>(gx)), dim3(512), lds, stream, static_cast<const FT*>(W1), static_cast<const FT*>(W2), ldw, static_cast<const FT*>(X), static_cast<const FT*>(X2), ldx, static_cast<const FT*>(bias1), static_cast<const FT*>(bias2), static_cast<const FT*>(mask), static_cast<FT*>(out), ldc, static_cast<int>(C), static_cast<int>(M), static_cast<const FT*>(gamma), static_cast<const FT*>(beta), eps, static_cast<FT*>(xhat), ldxh, mean, rstd, pairs); } while (0)
+    hipLaunchKernelGGL(kfn, dim3(static_cast<unsigned>(gx), static_cast<unsigned>(parts)), dim3(512), lds, stream, static_cast<const FT*>(W1), static_cast<const FT*>(W2), ldw, static_cast<const FT*>(X), static_cast<const FT*>(X2), ldx, static_cast<const FT*>(bias1), static_cast<const FT*>(bias2), static_cast<const FT*>(mask), static_cast<FT*>(out), ldc, static_cast<int>(C), static_cast<int>(M), static_cast<const FT*>(gamma), static_cast<const FT*>(beta), eps, static_cast<FT*>(xhat), ldxh, mean, rstd, pairs); } while (0)
 #define DGR(KT, LN, RW) do { if (half) DGR_F(f16bits, KT, LN, RW, false); else DGR_F(uint16_t, KT, LN, RW, false); } while (0)
 #define DGP(KT, LN, RW) do { if (half) DGR_F(f16bits, KT, LN, RW, true); else DGR_F(uint16_t, KT, LN, RW, true); } while (0)
 #define DGR_K(LN, RW) do { switch (K / 32) { case 1: DGR(1, LN, RW); break; case 2: DGR(2, LN, RW); break; case 3: DGR(3, LN, RW); break; default: DGR(4, LN, RW); break; } } while (0)
@@ -2976,8 +3014,9 @@ static int gate_bwd_input_impl(int32_t dtype, int64_t C, int64_t M, int64_t K, c
     const bool pairs_ok = !dc_by_row || (M % 2 == 0 && ldc % 2 == 0 && reinterpret_cast<uintptr_t>(dC) % 4 == 0);
     if (lds <= 160 * 1024 && pairs_ok) {
       const int64_t ntiles = (M + 31) / 32;
-      int64_t gx = (ntiles + nwaves - 1) / nwaves;
-      if (gx > device_cus()) gx = device_cus();
+      // (tiles to the CUs first: 392 x 392 rows, one input, 109 us with the tiles of a block next to each other, 94 so - the second
+      // round of 4 802 tiles on 2 048 wavefronts ran on a third of the CUs; 64 x 64 rows 30 and 21)
+      const int64_t gx = std::min<int64_t>(split ? ntiles : (ntiles + 1) / 2, device_cus());
 #define GBR_F(FT, KT, SP, PD) do { auto kfn = gate_bwd_input_res_kernel<FT, KT, SP, !SP, false, PD>; \
         CUEQ_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kfn), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds))); \
         hipLaunchKernelGGL(kfn, dim3(static_cast<unsigned>(gx)), dim3(SP ? 256 : 512), lds, stream, static_cast<const FT*>(W1), static_cast<const FT*>(W2), ldw, static_cast<const FT*>(X1), static_cast<const FT*>(X2), ldx, static_cast<const FT*>(bias1), static_cast<const FT*>(bias2), static_cast<const FT*>(mask), static_cast<const FT*>(dC), ldc, static_cast<FT*>(dX1), static_cast<FT*>(dX2), lddx, accumulate, static_cast<FT*>(dU), static_cast<FT*>(dV), static_cast<int>(C), static_cast<int>(M), static_cast<const FT*>(nullptr), int64_t(0), static_cast<const float*>(nullptr), static_cast<const float*>(nullptr), static_cast<const FT*>(nullptr), static_cast<FT*>(nullptr), pairs); } while (0)
