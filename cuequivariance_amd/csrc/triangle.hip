@@ -245,12 +245,13 @@ __device__ __forceinline__ uint4 gemm_fragment(const char* tile, int base, int q
 // which quarter goes round (the first ones of a partial tile have more to do, and a wavefront's number decides its SIMD); the bound on
 // registers keeps the accumulators of four wavefronts beside their operands and four (three) blocks on a CU.  128 products of n x n,
 // bfloat16, us with all subtiles always / with EDGE, both operands by rows: 480 55.7 / 48.6, 392 (4 x 4 tiles of 128, the last 8 wide)
-// 47.3 / 43.6, 264 23.0 / 21.4; by columns 47.5 / 45.2, 39.8 / 36.3, 20.7 / 19.4; whole tiles lose 1 - 3 % with it.  (Loads left
+// 47.3 / 43.6, 264 23.0 / 21.4; by columns 47.5 / 45.2, 39.8 / 36.3, 20.7 / 19.4; whole tiles lose 1 - 3 % with it.  float32, by
+// rows: 392 251 / 222, 320 138 / 114; by columns 231 / 220, 116 / 108, 200 37.5 / 37.1.  (Loads left
 // out as well, behind a condition, make every wait one for all loads: 392 47 us, 384 29 -> 38.)
 // KB: bytes of k per row and step; 128 makes every request of a contraction-contiguous operand a whole 128-byte line (with
 // 64 a line is fetched in two halves one step apart, and a 256 x 256 step turns over the whole L1 in between).
 template <typename TI, typename TO, bool TA, bool TB, int WM = 2, int WN = 2, int KB = 64, bool EDGE = false>
-__global__ void __launch_bounds__(64 * WM * WN, (!EDGE ? 1 : TA && !TB ? 3 : 4)) gemm_kernel(const TI* __restrict__ A, int64_t lda, int64_t sA,
+__global__ void __launch_bounds__(64 * WM * WN, (!EDGE ? 1 : TA && !TB && sizeof(TI) == 2 ? 3 : 4)) gemm_kernel(const TI* __restrict__ A, int64_t lda, int64_t sA,
                                                    const TI* __restrict__ B, int64_t ldb, int64_t sB,
                                                    TO* __restrict__ C, int64_t ldc, int64_t sC, int Mfull, int N, int Kfull,
                                                    float alpha, int accumulate, int vec_out, int64_t k_total, int nparts, int64_t pA,
@@ -2706,7 +2707,7 @@ extern "C" int cueq_gemm(int32_t in_dtype, int32_t out_dtype, int32_t trans_a, i
     const dim3 grid_big(static_cast<unsigned>(N / 256), static_cast<unsigned>(M / 256), static_cast<unsigned>(batch));
 #define GEMM_ARGS(TI, TO) static_cast<const TI*>(A), lda, stride_a, static_cast<const TI*>(B), ldb, stride_b, static_cast<TO*>(C), ldc, stride_c, m, n, k, al, accumulate, vec_out, 0, 1, 0, 0, 0, nullptr, 0, 0, 0, 0
 #define GEMM_LAUNCH(TI, TO, TA, TB) hipLaunchKernelGGL((gemm_kernel<TI, TO, TA, TB>), grid, dim3(256), 0, stream, GEMM_ARGS(TI, TO))
-#define GEMM_SZ(TI, TA, TB) do { if (big) hipLaunchKernelGGL((gemm_kernel<TI, TI, TA, TB, 4, 4, (sizeof(TI) == 2 ? 128 : 64)>), grid_big, dim3(1024), 0, stream, GEMM_ARGS(TI, TI)); else if (sizeof(TI) == 2 && (M % kTile || N % kTile) && (M > kTile || N > kTile)) hipLaunchKernelGGL((gemm_kernel<TI, TI, TA, TB, 2, 2, 64, sizeof(TI) == 2>), grid, dim3(256), 0, stream, GEMM_ARGS(TI, TI)); else GEMM_LAUNCH(TI, TI, TA, TB); } while (0)
+#define GEMM_SZ(TI, TA, TB) do { if (big) hipLaunchKernelGGL((gemm_kernel<TI, TI, TA, TB, 4, 4, (sizeof(TI) == 2 ? 128 : 64)>), grid_big, dim3(1024), 0, stream, GEMM_ARGS(TI, TI)); else if ((M % kTile || N % kTile) && (M > kTile || N > kTile)) hipLaunchKernelGGL((gemm_kernel<TI, TI, TA, TB, 2, 2, 64, true>), grid, dim3(256), 0, stream, GEMM_ARGS(TI, TI)); else GEMM_LAUNCH(TI, TI, TA, TB); } while (0)
 #define GEMM_TR(TI) do { if (trans_a && trans_b) GEMM_SZ(TI, true, true); else if (trans_a) GEMM_SZ(TI, true, false); else if (trans_b) GEMM_SZ(TI, false, true); else GEMM_SZ(TI, false, false); } while (0)
     if (in_dtype == CUEQ_F32 && out_dtype == CUEQ_F32) GEMM_TR(float);
     else if (in_dtype == CUEQ_F32 && out_dtype == CUEQ_F16) GEMM_LAUNCH(float, f16bits, false, false);
