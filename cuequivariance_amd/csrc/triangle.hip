@@ -959,11 +959,19 @@ __global__ void __launch_bounds__((gbi_threads<TI, SPLIT>()), (gbi_waves_per_sim
         const float duv = dvv * fmaf(-vv, sg, vv);          // du = d v s (1 - s)
         du[BF ? b : v] = duv;
         dv[BF ? b : v] = dvv;
-        if (dU != nullptr && mcol < M) {
+        if ((BF || DC_BY_ROW) && dU != nullptr && mcol < M) {
           const int row = c0 + 8 * a + 4 * h + b;
           const int64_t o = DC_BY_ROW ? static_cast<int64_t>(row) * ldc + mcol : static_cast<int64_t>(mcol) * ldc + row;
           tri_store(dU, o, duv);
           tri_store(dV, o, dvv);
+        }
+      }
+      if constexpr (!BF && !DC_BY_ROW) {
+        // four values next to each other, in whole 16-byte vectors (the host checks; one by one, 384 x 384 rows took 302 us, so 250)
+        if (dU != nullptr && mcol < M) {
+          const int64_t o = static_cast<int64_t>(mcol) * ldc + c0 + 8 * a + 4 * h;
+          *reinterpret_cast<float4*>(dU + o) = make_float4(du[4 * a], du[4 * a + 1], du[4 * a + 2], du[4 * a + 3]);
+          *reinterpret_cast<float4*>(dV + o) = make_float4(dv[4 * a], dv[4 * a + 1], dv[4 * a + 2], dv[4 * a + 3]);
         }
       }
       if constexpr (BF) {
