@@ -759,6 +759,11 @@ __device__ __forceinline__ V load_global(const char* uniform_base, uint32_t lane
   typedef const __attribute__((address_space(1))) V* gptr;
   return *reinterpret_cast<gptr>(reinterpret_cast<uint64_t>(uniform_base) + lane_offset);
 }
+template <typename V>
+__device__ __forceinline__ void store_global(const char* uniform_base, uint32_t lane_offset, V value) {
+  typedef __attribute__((address_space(1))) V* gptr;
+  *reinterpret_cast<gptr>(reinterpret_cast<uint64_t>(uniform_base) + lane_offset) = value;
+}
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 template <>
@@ -773,12 +778,16 @@ __device__ __forceinline__ uint2 load_global<uint2>(const char* uniform_base, ui
 }
 
 
-// 4 wavefronts (128 columns m) per block; the 2-byte single-input case fits 2 wavefronts per SIMD (two blocks per
-// CU, so one block's waits overlap the other's work), the others need more registers and run 1 per SIMD.
+// 4 wavefronts (128 columns m) per block; the single-input cases fit 2 wavefronts per SIMD (two blocks per CU, so one
+// block's waits and gate arithmetic overlap the other's products), the two-input ones need more registers and run 1 per SIMD.
+// float32, single input: bound by the matrix cores.  To fit, the cotangent and the next weights are requested in the
+// iteration that uses or stores them, behind one product each, and operands are read a few at a time (384 x 384 rows,
+// K = 128, C = 256: 457 us with one wavefront, 398 with two; 252 at the matrix rate, 280 for the five blocks of the
+// busiest CU).
 template <typename TI, bool SPLIT>
 constexpr int gbi_threads() { return 256; }
 template <typename TI, bool SPLIT>
-constexpr int gbi_waves_per_simd() { return (sizeof(TI) == 2 && !SPLIT) ? 2 : 1; }
+constexpr int gbi_waves_per_simd() { return !SPLIT ? 2 : 1; }
 
 // DC_BY_ROW: dC, dU, dV are C x M (else M x C).  Addresses inside the loop are a uniform 64-bit base plus a 32-bit
 // lane offset (the host checks the extents), which keeps them out of the vector registers.
@@ -823,7 +832,8 @@ __global__ void __launch_bounds__((gbi_threads<TI, SPLIT>()), (gbi_waves_per_sim
   const char* bptr = reinterpret_cast<const char*>(has_bias ? bsrc : W1);
   const uint32_t bofs = has_bias ? static_cast<uint32_t>((tid & 31) * ES) : 0u;
   TI stb;
-  // the next chunk and its biases are fetched at the top of an iteration and stored after the first product
+  // the next chunk and its biases are fetched at the top of an iteration and stored after the first product (kAhead), or fetched
+  // before the second product and stored behind it
   auto load_rows = [&](int c0) {
     stb = *reinterpret_cast<const TI*>(bptr + (has_bias ? static_cast<int64_t>(c0) * ES : 0) + bofs);  // bptr differs by lane
     const char* w1 = uniform_ptr(reinterpret_cast<const char*>(W1) + static_cast<int64_t>(c0) * ldw * ES);
@@ -871,9 +881,12 @@ __global__ void __launch_bounds__((gbi_threads<TI, SPLIT>()), (gbi_waves_per_sim
 #pragma unroll
   for (int t = 0; t < (SPLIT ? KT : 1); ++t) ax2[t] = floatx16{0};
 
-  // cotangent of a chunk: value v of the lane belongs to row c0 + 8 (v >> 2) + 4 h + (v & 3); fetched one chunk ahead
+  // cotangent of a chunk: value v of the lane belongs to row c0 + 8 (v >> 2) + 4 h + (v & 3); fetched one chunk ahead (kAhead)
   // (kept as loaded - one register per value, or packed pairs when read along c - and widened where it is used)
-  uint32_t dcr[16], dcn[16];
+  constexpr bool kAhead = BF || SPLIT;  // (registers to spare: everything a whole iteration ahead)
+  uint32_t dcb[kAhead ? 2 : 1][16];
+  uint32_t (&dcr)[16] = dcb[0];
+  uint32_t (&dcn)[16] = dcb[kAhead ? 1 : 0];
   const uint32_t dcofs = DC_BY_ROW ? static_cast<uint32_t>((4 * h * ldc + mld) * ES) : static_cast<uint32_t>((mld * ldc + 4 * h) * ES);
   auto load_dc = [&](int c0) {
     if constexpr (DC_BY_ROW) {
@@ -908,15 +921,18 @@ __global__ void __launch_bounds__((gbi_threads<TI, SPLIT>()), (gbi_waves_per_sim
 
   const int nchunks = C / 32;
   load_rows(0);
-  load_dc(0);
+  if constexpr (kAhead) load_dc(0);
   store_rows(0);
   __syncthreads();
   for (int ci = 0; ci < nchunks; ++ci) {
     const int c0 = ci * 32, buf = ci & 1;
     const bool more = ci + 1 < nchunks;
+    if constexpr (!kAhead) load_dc(c0);
+    if constexpr (kAhead) {
 #pragma unroll
-    for (int v = 0; v < 16; ++v) dcr[v] = dcn[v];
-    if (more) {
+      for (int v = 0; v < 16; ++v) dcr[v] = dcn[v];
+    }
+    if (kAhead && more) {
       load_rows(c0 + 32);
       load_dc(c0 + 32);  // a whole iteration ahead of its use
     }
@@ -940,10 +956,11 @@ __global__ void __launch_bounds__((gbi_threads<TI, SPLIT>()), (gbi_waves_per_sim
           const uint4 a2 = *reinterpret_cast<const uint4*>(w1 + WBYTES + s2 * 64 + q * 16);
           mma_step<TI>(au, a1, xf1[s2][q]);
           mma_step<TI>(av, a2, SPLIT ? xf2[s2][q] : xf1[s2][q]);
+          if constexpr (!kAhead) { if (q == 1) __builtin_amdgcn_sched_barrier(0); }
         }
     }
 
-    if (more) store_rows(buf ^ 1);  // the other buffer was last read before the previous barrier
+    if (kAhead && more) store_rows(buf ^ 1);  // the other buffer was last read before the previous barrier
 
     // gate backward in registers; du, dv are packed (2-byte types) as soon as they exist
     float du[BF ? 4 : 16], dv[BF ? 4 : 16];
@@ -959,7 +976,14 @@ __global__ void __launch_bounds__((gbi_threads<TI, SPLIT>()), (gbi_waves_per_sim
         const float duv = dvv * fmaf(-vv, sg, vv);          // du = d v s (1 - s)
         du[BF ? b : v] = duv;
         dv[BF ? b : v] = dvv;
-        if ((BF || DC_BY_ROW) && dU != nullptr && mcol < M) {
+        if constexpr (!BF && DC_BY_ROW) {
+          if (dU != nullptr && mcol < M) {
+            const int64_t r = static_cast<int64_t>(c0 + 8 * a + b) * ldc * ES;
+            store_global(uniform_ptr(reinterpret_cast<const char*>(dU) + r), dcofs, duv);
+            store_global(uniform_ptr(reinterpret_cast<const char*>(dV) + r), dcofs, dvv);
+          }
+        }
+        if (BF && dU != nullptr && mcol < M) {
           const int row = c0 + 8 * a + 4 * h + b;
           const int64_t o = DC_BY_ROW ? static_cast<int64_t>(row) * ldc + mcol : static_cast<int64_t>(mcol) * ldc + row;
           tri_store(dU, o, duv);
@@ -979,6 +1003,7 @@ __global__ void __launch_bounds__((gbi_threads<TI, SPLIT>()), (gbi_waves_per_sim
         pv[2 * a] = pack16<F>(dv[0], dv[1]); pv[2 * a + 1] = pack16<F>(dv[2], dv[3]);
       }
     }
+    if (!kAhead && more) load_rows(c0 + 32);
     // second product: rows m (lanes of the operand), contraction over the 32 rows c of the chunk
     if constexpr (BF) {
       // operand of the second product: for column d = 32 ds + (lane & 31), the 8 rows c that this lane's du / dv
@@ -1009,9 +1034,11 @@ __global__ void __launch_bounds__((gbi_threads<TI, SPLIT>()), (gbi_waves_per_sim
           ax1[ds] = __builtin_amdgcn_mfma_f32_32x32x2f32(du[v], w1, ax1[ds], 0, 0, 0);
           if constexpr (SPLIT) ax2[ds] = __builtin_amdgcn_mfma_f32_32x32x2f32(dv[v], w2, ax2[ds], 0, 0, 0);
           else ax1[ds] = __builtin_amdgcn_mfma_f32_32x32x2f32(dv[v], w2, ax1[ds], 0, 0, 0);
+          if constexpr (!kAhead) { if (v % 4 == 3) __builtin_amdgcn_sched_barrier(0); }
         }
     }
 
+    if (!kAhead && more) store_rows(buf ^ 1);
     __syncthreads();
   }
 
