@@ -76,7 +76,7 @@ struct NormalizeGrad : torch::autograd::Function<NormalizeGrad> {
     if (at::GradMode::is_enabled()) {
       if (want_g) dg = run(v, x);
       if (want_x) {
-        const at::Tensor length = at::linalg_vector_norm(x, 2, {1}, true), through = length.ge(kNormalizeEps);
+        const at::Tensor length = at::linalg_vector_norm(x, 2, {1}, true), through = length.lt(kNormalizeEps).logical_not();  // (a NaN stays one)
         const at::Tensor n = length.clamp_min(kNormalizeEps), y = x / n;
         const at::Tensor yv = (y * v).sum(1, true), yg = (y * g).sum(1, true), vg = (v * g).sum(1, true);
         dx = at::where(through, ((3 * yv * yg - vg) * y - yg * v - yv * g) / n / n, at::zeros({}, x.options()));

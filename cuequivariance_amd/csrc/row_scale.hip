@@ -57,7 +57,7 @@ __global__ void __launch_bounds__(64) normalize3_kernel(const T* __restrict__ x,
       y[a] = p[a] / n;
       yq = fma(y[a], q[a], yq);
     }
-    const bool through = length >= eps;
+    const bool through = !(length < eps);  // (a NaN stays one)
     if (out)
 #pragma unroll
       for (int a = 0; a < 3; ++a) out[3 * r + a] = static_cast<T>((q[a] - (through ? yq * y[a] : 0.0)) / n);

@@ -62,6 +62,16 @@ def test_short_zero_and_odd_vectors(device, dtype):
         assert torch.equal(out[0][k][4:].isnan(), out[1][k][4:].isnan())
 
 
+@pytest.mark.parametrize("graph", [False, True])
+def test_second_derivative_keeps_nan(device, graph):
+    """What no length divides has no second derivative either: NaN, with a graph (PyTorch's operations) and without (the kernel)."""
+    x = torch.tensor([[float("nan"), 1, 2], [float("inf"), 1, 2], [1, 2, 3]], device=device, requires_grad=True)
+    g = torch.ones_like(x).requires_grad_()
+    (dx,) = torch.autograd.grad(_lib.host().normalize(x), x, g, create_graph=True)
+    for second in torch.autograd.grad(dx, [g, x], torch.ones_like(x), create_graph=graph):
+        assert second[:2].isnan().all() and second[2].isfinite().all()
+
+
 def test_calls_that_are_not_plain_are_left_to_pytorch(device):
     normalize = _lib.host().normalize
     x = torch.randn(4, 3, device=device)
