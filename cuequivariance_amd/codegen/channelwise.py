@@ -8,8 +8,9 @@ tensor product takes after flattening the Clebsch-Gordan modes — i.e. for ever
 
 Output: HIP source with the path table unrolled into the instruction stream.
 
-Forward kernel (one wavefront = one output row x 64 channels, for 32 channels and fewer two or four batch rows at a time; where there are few rows, four or eight wavefronts of a block share
-the list of a row, ``fwd_parts`` in ``cw_common.h``, and add their sums in LDS):
+Forward kernel (one wavefront = one output row x 64 channels, for 32 channels and fewer two or four batch
+rows at a time; where there are few rows, four or eight wavefronts of a block share the list of a row,
+``fwd_parts`` in ``cw_common.h``, and add their sums in LDS):
   * channels across lanes, so every HBM access is a contiguous 256-byte (fp32) line;
   * the uniform factor ``c_p * x2[j_p]`` of each path lives in a table register: lane ``n`` of each
     16-lane row holds the factor of a path whose ``x2`` index is ``n``; the FMA reads it with the DPP
@@ -683,7 +684,8 @@ def emit_backward(st: ChannelwiseStructure, T: str, waves_per_eu: int, prefetch:
             A(f"{ind}}}")
             # dx2: reduced over the 64 lanes, the sums halved among them (16 sums over 64 lanes: 15 halving steps and 2 plain
             # ones, one store of 16 lanes, where 16 butterflies take 96 steps and one lane 16 stores; forward + backward, fp32:
-            # 32 ch l <= 2, 60 000 edges 124.5 -> 118.6 us, 128 ch l <= 3, 1 000 edges 102.2 -> 99.0 us); channel chunks and wavefronts of one batch row are folded afterwards
+            # 32 ch l <= 2, 60 000 edges 124.5 -> 118.6 us, 128 ch l <= 3, 1 000 edges 102.2 -> 99.0 us); channel chunks and
+            # wavefronts of one batch row are folded afterwards
             A(f"{ind}if (!active) {{" + " ".join(f"pj{j} = 0;" for j in j_used) + "}")
             if st.harmonics:
                 # dv[a] = sum_j pj[j] dY_j/dv[a] (this lane's share: the sums over channels and blocks are linear)
