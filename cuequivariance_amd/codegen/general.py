@@ -15,6 +15,7 @@ only when the extent fits one wavefront.  Anything else is declined and the tabl
 
 from __future__ import annotations
 
+import re
 from collections import defaultdict
 
 from ..tables import U1dTables
@@ -47,15 +48,51 @@ def supported(t: U1dTables) -> bool:
 FOLD = 8  # segments of the output that meet in LDS at a time (16 wavefronts, float64: 64 KB)
 
 
-def _most_parts(values: int, T: str) -> int:
-    """Most wavefronts that share the list of an output row: as many as a compute unit holds with registers for ``values`` values (the
-    inputs read once per batch element and the sums) and 30 more."""
-    registers = values * (2 if T == "double" else 1) + 30
-    return 16 if registers <= 110 else 8 if registers <= 230 else 4 if registers <= 480 else 1
+UNBOUND = 4  # wavefronts of a block that bound nothing: each may have all registers of its SIMD
 
 
-def emit_unit(t: U1dTables, T: str, name: str, table_hash: int, io=None) -> str:
-    """``io``: element type of the buffers when it is not the arithmetic type ``T`` ("bf16" / "f16" with ``T`` = float)."""
+def _most_parts(values: int, terms: int, T: str) -> int:
+    """Most wavefronts to try for the list of an output row.  Sixteen leave a wavefront 128 registers, eight 256, and a kernel that needs
+    more spills in every launch, a batched output's too.  What it needs is up to the compiler, which keeps products of operands
+    beside the ``values`` (inputs read once per batch element and sums): this is a guess that saves compiling twice, ``fewer_parts`` has the last
+    word.  (Registers of second derivatives, float: channel-wise product, 78 values and 116 terms, 65; 193 and 706, 167 - product
+    basis, 28 and 268, 86; 37 and 361, 157; 39 and 1 137, 246; 56 and 1 531, 279.  All gradients of that basis's gradients, 64 ch
+    l <= 2 -> l <= 1, us with sixteen wavefronts wherever the values fit / as here: float 451 rows 77 / 51, 20 000 rows
+    2 543 / 1 247; float64 3 000 rows 3 918 / 512.)"""
+    registers = (values + max(0, terms - 4 * values) // 4) * (2 if T == "double" else 1) + 30
+    return 16 if registers <= 110 else 8 if registers <= 320 else UNBOUND
+
+
+REPORT_FLAG = "-Rpass-analysis=kernel-resource-usage"
+
+
+def fewer_parts(parts: dict, report: str):
+    """``parts`` ({output buffer: most wavefronts that share a list}) after a look at what the compiler says of the unit emitted with them
+    (``REPORT_FLAG``): half as many where a kernel spills registers, ``UNBOUND`` where it says nothing; ``None`` when they may stay."""
+    spilled, kernel = {}, None
+    for line in report.splitlines():
+        if (m := re.search(r"Function Name: \S*out(\d+)_kernel", line)) is not None:
+            kernel = int(m.group(1))
+        elif kernel is not None and (m := re.search(r"ScratchSize \[bytes/lane\]: (\d+)", line)) is not None:
+            spilled[kernel] = int(m.group(1)) > 0
+    fewer = {ob: n if n <= UNBOUND or spilled.get(ob) is False else n // 2 if ob in spilled else UNBOUND for ob, n in parts.items()}
+    return None if fewer == parts else fewer
+
+
+def parts_of(t: U1dTables, T: str) -> dict:
+    """{output buffer: most wavefronts that share the list of one of its rows}, before the compiler was asked."""
+    terms = output_terms(t)
+
+    def values(tl):
+        return len({bs for _, ins, _ in tl for bs in ins}) + len({oseg for oseg, _, _ in tl})
+
+    return {ob: _most_parts(values(terms.get(ob, [])), len(terms.get(ob, [])), T) if t.operand_extent > 1 else 1
+            for ob in range(t.num_inputs, t.num_inputs + t.num_outputs)}
+
+
+def emit_unit(t: U1dTables, T: str, name: str, table_hash: int, io=None, parts=None) -> str:
+    """``io``: element type of the buffers when it is not the arithmetic type ``T`` ("bf16" / "f16" with ``T`` = float).  ``parts``: of
+    ``parts_of``, or what ``fewer_parts`` made of it."""
     TI, io_code, tag = io_type(T, io)
     E = t.operand_extent
     nin, nout = t.num_inputs, t.num_outputs
@@ -81,7 +118,7 @@ def emit_unit(t: U1dTables, T: str, name: str, table_hash: int, io=None) -> str:
     A("struct InBuf { const void* data; const void* index; int32_t mode; int32_t idx64; };")
     A(f"struct InTable {{ InBuf b[{max(nin, 1)}]; }};")
     A("")
-    most_parts = {}
+    most_parts = parts_of(t, T) if parts is None else parts
     for ob in range(nin, nin + nout):
         tl = terms.get(ob, [])
         used = sorted({bs for _, ins, _ in tl for bs in ins})
@@ -92,7 +129,7 @@ def emit_unit(t: U1dTables, T: str, name: str, table_hash: int, io=None) -> str:
         for oseg, ins, c in tl:
             by_seg[oseg].append((ins, c))
         A(f"// output buffer {ob}: {len(tl)} paths into {len(by_seg)} of {out_nseg} segments")
-        most = most_parts[ob] = _most_parts(len(used) + len(by_seg), T) if E > 1 else 1
+        most = most_parts[ob]
         A(f"__global__ void __launch_bounds__({64 * most}) out{ob}_kernel(const InTable tab, TI* __restrict__ out, int64_t rows, "
           "const int64_t* __restrict__ csr_offsets, const int64_t* __restrict__ csr_perm) {")
         if most > 1:

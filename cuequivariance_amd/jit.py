@@ -239,12 +239,21 @@ def _build_and_load(t: U1dTables, code: int, key: int, polynomial=None, origin=N
 
     T = "float" if code == _lib.F32 else "double"
     name = f"jit_{key:016x}"
+    revise = ()
     # the object's name carries a hash of the emitted source, so a changed generator (or tuning) never meets a stale object
     family = _family(t, polynomial, origin)
     if family is None:
         from .codegen import general as gen
 
-        src = gen.emit_unit(t, T, name, key, io=io)
+        parts = gen.parts_of(t, T)
+        src = gen.emit_unit(t, T, name, key, io=io, parts=parts)
+
+        def again(report):  # the same unit with fewer wavefronts to a list where the compiler could not give so many their registers
+            nonlocal parts
+            parts = gen.fewer_parts(parts, report)
+            return parts and gen.emit_unit(t, T, name, key, io=io, parts=parts)
+
+        revise = (gen.REPORT_FLAG, again)
         what = f"general plan, {sum(t.num_paths)} paths, extent {t.operand_extent}"
     elif family == "channelwise":
         _, paths = t.operation(0)
@@ -271,12 +280,14 @@ def _build_and_load(t: U1dTables, code: int, key: int, polynomial=None, origin=N
         what = f"symmetric contraction, {len(st.terms)} folded terms, extent {st.extent}"
     so = cache_dir() / f"u1d_{name}_{io or T}_{hashlib.sha1(src.encode()).hexdigest()[:10]}.so"
     if not so.exists():
-        _compile(src, so, f"descriptor {key:016x} ({T}{', buffers of ' + io if io else ''}, {what})")
+        _compile(src, so, f"descriptor {key:016x} ({T}{', buffers of ' + io if io else ''}, {what})", revise=revise)
     _lib.load()  # the library the object links against is already in the process
     return C.CDLL(str(so))
 
 
-def _compile(src: str, so: Path, what: str, link_library: bool = True) -> None:
+def _compile(src: str, so: Path, what: str, link_library: bool = True, revise: tuple = ()) -> None:
+    """``revise``: a flag that has the compiler say something, and what makes another source of what it says, or ``None`` when this one
+    may stay."""
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
     with tempfile.TemporaryDirectory(dir=so.parent) as tmp:
         hip = Path(tmp) / (so.stem + ".hip")
@@ -287,9 +298,14 @@ def _compile(src: str, so: Path, what: str, link_library: bool = True) -> None:
         if link_library:
             cmd += [f"-L{_lib.LIB_PATH.parent}", f"-l:{_lib.LIB_PATH.name}", f"-Wl,-rpath,{_lib.LIB_PATH.parent}"]
         print(f"[cueq_amd.jit] compiling kernels for {what} ...", file=sys.stderr, flush=True)
-        r = subprocess.run(cmd, capture_output=True, text=True)
-        if r.returncode != 0:
-            raise RuntimeError(f"hipcc failed:\n{r.stderr[-2000:]}")
+        while True:
+            r = subprocess.run([*cmd, *revise[:1]], capture_output=True, text=True)
+            if r.returncode != 0:
+                raise RuntimeError(f"hipcc failed:\n{r.stderr[-2000:]}")
+            src = revise[1](r.stderr) if revise else None
+            if src is None:
+                break
+            hip.write_text(src)
         os.replace(out, so)  # atomic: another process may be compiling the same descriptor
 
 
