@@ -31,6 +31,8 @@ struct FlexBlock {  // one block of the result
 typedef float fx16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
+constexpr int kFlexOneComponent = 2;  // `mul_ir` of a caller whose blocks all have one component
+
 constexpr int kFlexStageBytes = 2 * 128 * (32 * 7 + 16);  // two buffers of 128 rows x 8 channels (float) x 7 components, the largest
 
 // The weights of a step of the contraction (STEP channels) as the matrix instructions take them, a column of W per lane (WT: a row of
@@ -549,14 +551,14 @@ extern "C" int cueq_linear_flex(int32_t dtype, int32_t transposed_weights, int64
   // 128x0e+128x1o+128x2e in mul_ir, float, forward 21.8 -> 9.7 us, 1 000 rows 22.1 -> 12.6 (1 400 rows, past the line: 22.5 either way)
   const int64_t tiles = (rows + 31) / 32 * column_tiles;
   const bool shared = tiles <= 2ll * device_cus();
-  // ir_mul rows (every block one component): four row tiles a wavefront once there are so many workgroups; us for one / four, 128 ch:
+  // ir_mul rows (the caller says that every block has one component): four row tiles a wavefront once there are so many workgroups; us for one / four, 128 ch:
   // float 4 000 rows (1 152 workgroups of one tile) 23 / 26, 8 000 38 / 38, 16 000 67 / 57, 32 000 147 / 113; bfloat16 2 000 9.8 / 9.7,
   // 4 000 13.8 / 9.8, 32 000 73 / 35
-  const bool tall = !mul_ir && !shared && (rows + 127) / 128 * column_tiles >= (dtype == CUEQ_F32 ? 9ll : 4ll) * device_cus();
+  const bool tall = mul_ir == kFlexOneComponent && !shared && (rows + 127) / 128 * column_tiles >= (dtype == CUEQ_F32 ? 9ll : 4ll) * device_cus();
   const int64_t slab_rows = tall ? 512 : 128, slabs = (rows + slab_rows - 1) / slab_rows;
   const int64_t grid = shared ? tiles : slabs * column_tiles;
   CUEQ_REQUIRE(grid < (1ll << 31), CUEQ_ERR_TOO_LARGE, "linear_flex: too many rows");
-  KernelTimer timer(mul_ir ? "linear_rows_mul_ir" : "linear_rows", stream);
+  KernelTimer timer(mul_ir && mul_ir != kFlexOneComponent ? "linear_rows_mul_ir" : "linear_rows", stream);
 #define FLEX_LAUNCH(KERNEL, ...)                                                                                                                         \
   hipLaunchKernelGGL((KERNEL), dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, static_cast<const FlexBlock*>(blocks),                           \
                      static_cast<const FlexPart*>(parts), nblocks, __VA_ARGS__)
