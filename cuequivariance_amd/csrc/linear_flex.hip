@@ -309,7 +309,12 @@ __device__ __forceinline__ void flex_stage_tile(const FlexBlock& blk, const Flex
       const int piece = j * 64 + lane, r = piece / OP, q = piece % OP;
       const int64_t z = z0 + 32 * (rt * ZT + t) + r;
       const u32x4 value = *reinterpret_cast<const u32x4*>(out_lds + r * OS + 16 * q);
-      if (z < Z && from_col + q * EPV < ends_col) *reinterpret_cast<u32x4*>(C + z * ldc + blk.c0 + from_col + q * EPV) = value;
+      const int left = ends_col - (from_col + q * EPV);  // elements of the block from here on: multiples of 4, so half a piece of 2-byte ones may be
+      if (z < Z && left > 0) {
+        TI* to = C + z * ldc + blk.c0 + from_col + q * EPV;
+        if (ES == 4 || left >= EPV) *reinterpret_cast<u32x4*>(to) = value;
+        else *reinterpret_cast<uint2*>(to) = make_uint2(value[0], value[1]);
+      }
     }
     __builtin_amdgcn_wave_barrier();
   }

@@ -60,3 +60,11 @@ def test_many_rows_of_blocks_of_several_components(device, mul_ir, transposed, d
 @pytest.mark.parametrize("transposed", [False, True])
 def test_many_rows_of_blocks_of_one_component(device, transposed, dtype):
     _check(device, dtype, [(32, 1), (64, 1), (16, 1), (160, 1)], 48, 40_003, 2, transposed)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("mul_ir,blocks", [(1, [(4, 1), (20, 3), (36, 5), (68, 1), (12, 7)]), (2, [(4, 1), (36, 1), (132, 1)])])
+@pytest.mark.parametrize("rows", [700, 12_001, 40_003])
+def test_blocks_that_end_in_half_a_piece(device, rows, mul_ir, blocks, dtype):
+    """N of 4 in 2-byte elements: a block's last 8 bytes of a row are half of a 16-byte piece, and what lies behind them belongs to nobody."""
+    _check(device, dtype, blocks, 32, rows, mul_ir)
