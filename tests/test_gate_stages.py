@@ -52,3 +52,29 @@ def test_gated_projections(device, dtype, axis, aligned):
         assert a.dtype == s.dtype == dtype
         assert (a.cpu().double() - b.detach()).abs().max().item() <= TOL[dtype] * scale
         assert (s.cpu().double() - b.detach()).abs().max().item() <= TOL[dtype] * scale
+
+
+@pytest.mark.parametrize("K,C", [(32, 32), (64, 96), (96, 32), (128, 256)])
+@pytest.mark.parametrize("inputs,M", [(1, 4), (1, 36), (1, 128), (1, 132), (1, 3000), (2, 3), (2, 33), (2, 128), (2, 3001)])
+def test_input_gradients_of_float32(device, inputs, M, K, C):
+    """Down to the inputs in one kernel, 32 weight rows at a time (one, two, three and eight turns), 128 columns a block: with one input
+    the cotangent and the gate gradients are (C, M), and the input's gradient may be added to what is there; with two they are (M, C)."""
+    from cuequivariance_amd.cuet import triangle as T
+
+    g = torch.Generator().manual_seed(M + K)
+    r = lambda *shape: torch.randn(*shape, generator=g).double()
+    X1, X2, W1, W2, b1, b2, before = r(M, K), r(M, K), r(C, K) / K ** 0.5, r(C, K) / K ** 0.5, r(C), r(C), r(M, K)
+    mask, dout = (torch.rand(M, generator=g) < 0.8).double(), r(C, M)
+    x1, x2 = X1.clone().requires_grad_(), X2.clone().requires_grad_()
+    u, v = W1 @ x1.T, W2 @ (x1 if inputs == 1 else x2).T
+    ref = torch.sigmoid(u + b1[:, None]) * (v + b2[:, None]) * mask
+    dx1, du, dv, *dx2 = torch.autograd.grad(ref, [x1, u, v] + ([x2] if inputs == 2 else []), dout)
+    f = lambda t: t.float().to(device)
+    d = f(dout if inputs == 1 else dout.T.contiguous())
+    for add in (False, True) if inputs == 1 else (False,):
+        got = T.gate_bwd_input(d, inputs == 1, f(W1), f(W2), f(X1), f(X2) if inputs == 2 else None, f(b1), f(b2), f(mask), f(before) if add else None, True)
+        want = [dx1 + before if add else dx1, dx2[0] if dx2 else None, *(t if inputs == 1 else t.T for t in (du, dv))]
+        for a, b in zip(got, want):
+            assert (a is None) == (b is None)
+            # (float32 sums of up to 2 x 256 products)
+            assert a is None or (a.cpu().double() - b).abs().max().item() <= 1e-5 * b.abs().max().item()

@@ -1,6 +1,7 @@
 """How the gate kernels with resident weights deal out their tiles - over the CUs first and, for few of them, over the weight rows as
 well (four or eight parts of 64-row tiles up to 8 192 rows, two or four of 32-row tiles) - must not show in a result: every row has the
-bits it has among 70 008 rows, whose tiles fill the device.  (Against float64: tests/test_triangle.py.)"""
+bits it has among 70 008 rows, whose tiles fill the device.  (Against float64: tests/test_triangle.py, rows of padded
+squares, which take the same parts: tests/test_triangle_padded.py.)"""
 import pytest
 import torch
 
