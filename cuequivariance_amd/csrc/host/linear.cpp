@@ -73,8 +73,8 @@ at::Tensor apply_rows(LinearOp& op, const at::Tensor& w_, const at::Tensor& x_, 
     return out;
   }
   check(lib().cueq_linear_flex(code, forward ? 0 : 1, Z, x.data_ptr(), lda, w.data_ptr(), out.data_ptr(), width, tables.on(device, LinearOp::kBlocks),
-                               tables.count(LinearOp::kBlocks, 32), tables.on(device, LinearOp::kParts), forward ? op.fwd_tiles : op.dx_tiles, op.mul_ir ? 1 : 2, stream),
-        "cueq_linear_flex");  // (2: rows in ir_mul, a block per component)
+                               tables.count(LinearOp::kBlocks, 32), tables.on(device, LinearOp::kParts), forward ? op.fwd_tiles : op.dx_tiles, op.mul_ir ? 1 + 4 : 2 + 4, stream),
+        "cueq_linear_flex");  // (2: rows in ir_mul, a block per component; 4: extents of 8 columns in any element type)
   return out;
 }
 

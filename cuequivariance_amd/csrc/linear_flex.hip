@@ -31,7 +31,33 @@ struct FlexBlock {  // one block of the result
 typedef float fx16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kFlexOneComponent = 2;  // `mul_ir` of a caller whose blocks all have one component
+enum { kFlexMulIr = 1, kFlexOneComponent = 2, kFlexWholePieces = 4 };  // what a caller says of its blocks (cueq_linear_flex's last number)
+
+// The block of a column tile (`tile`: of all blocks, then of its own), nblocks past the last; the whole wavefront is here.  One after the other
+// the extents are a chain of loads (16 blocks of an l <= 3 row: 2 us of a kernel of 10), so the lanes read them at once where there are
+// more than a few; for three the sums over lanes take longer (0.5 us).
+// BACK: the blocks from the last to the first.
+template <bool BACK>
+__device__ __forceinline__ int flex_find_block(const FlexBlock* __restrict__ blocks, int nblocks, int& tile) {
+  if (nblocks <= 6) {
+    int b = 0;
+    while (b < nblocks && tile >= blocks[BACK ? nblocks - 1 - b : b].nt) tile -= blocks[BACK ? nblocks - 1 - b++ : b++].nt;
+    return b;
+  }
+  const int lane = threadIdx.x & 63;
+  for (int first = 0;; first += 64) {
+    const int i = first + lane;
+    int sum = i < nblocks ? blocks[BACK ? nblocks - 1 - i : i].nt : 1 << 24;
+#pragma unroll
+    for (int d = 1; d < 64; d *= 2) {
+      const int below = __shfl_up(sum, d, 64);
+      sum += lane >= d ? below : 0;
+    }
+    const int before = __builtin_amdgcn_readfirstlane(__popcll(__ballot(sum <= tile)));
+    if (before) tile -= __builtin_amdgcn_readlane(sum, before - 1);
+    if (before < 64) return first + before;
+  }
+}
 
 constexpr int kFlexStageBytes = 2 * 128 * (32 * 7 + 16);  // two buffers of 128 rows x 8 channels (float) x 7 components, the largest
 
@@ -114,6 +140,50 @@ __device__ __forceinline__ void flex_store(const FlexBlock& blk, TI* __restrict_
   }
 }
 
+// The same through LDS, 64 D bytes of every row at a time, by a wavefront for itself: a lane's own 16-byte pieces are a write request each
+// (20 000 rows of 128x0e+128x1o+128x2e in mul_ir, float: 79 us with such stores, 60 without any).
+template <int D>
+constexpr int kFlexLineBytes = 32 * (64 * D + 16);
+// WHOLE: no row of a block ends in half a piece (2-byte elements, N of 4).  What the ends take is 0.5 us of every kernel of 10 that has the code.
+template <bool WHOLE, typename TI, int D>
+__device__ __forceinline__ void flex_store_lines(const FlexBlock& blk, TI* __restrict__ C, int64_t ldc, int64_t Z, int64_t z0, int n0, const fx16 (&acc)[D],
+                                                 float scale, char* lds) {
+  constexpr int ES = sizeof(TI), EPV = 16 / ES, COLS = 64 / ES, OS = 64 * D + 16, OP = 4 * D;  // columns a turn; a row's stride and 16-byte pieces in LDS
+  const int lane = threadIdx.x & 63, c = lane & 31, h = lane >> 5;
+#pragma unroll
+  for (int turn = 0; turn < 32 / COLS; ++turn) {
+#pragma unroll
+    for (int a = 0; a < COLS / 8; ++a) {
+      float v[4 * D];
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+#pragma unroll
+        for (int i = 0; i < D; ++i) v[b * D + i] = scale * acc[i][4 * (turn * (COLS / 8) + a) + b];
+      char* to = lds + c * OS + (8 * a + 4 * h) * D * ES;
+#pragma unroll
+      for (int i = 0; i < D; ++i) {
+        if constexpr (ES == 4) *reinterpret_cast<float4*>(to + 16 * i) = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
+        else *reinterpret_cast<uint2*>(to + 8 * i) = make_uint2(mm_pack<TI>(v[4 * i], v[4 * i + 1]), mm_pack<TI>(v[4 * i + 2], v[4 * i + 3]));
+      }
+    }
+    __builtin_amdgcn_wave_barrier();
+    const int from_col = (n0 + turn * COLS) * D, ends_col = blk.N * D;
+#pragma unroll
+    for (int j = 0; j < 2 * D; ++j) {
+      const int piece = j * 64 + lane, r = piece / OP, q = piece % OP;
+      const int64_t z = z0 + r;
+      const u32x4 value = *reinterpret_cast<const u32x4*>(lds + r * OS + 16 * q);
+      if (z < Z && from_col + (WHOLE ? q * EPV : q * EPV + EPV - 1) < ends_col) *reinterpret_cast<u32x4*>(C + z * ldc + blk.c0 + from_col + q * EPV) = value;
+    }
+    if constexpr (!WHOLE) {
+      const int half = ends_col - 4 - from_col;
+      if (ends_col % EPV && half >= 0 && half < COLS * D && h == 0 && z0 + c < Z)
+        *reinterpret_cast<uint2*>(C + (z0 + c) * ldc + blk.c0 + from_col + half) = *reinterpret_cast<const uint2*>(lds + c * OS + half * ES);
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
 // ---- few tiles: the four wavefronts of a workgroup share a tile of 32 rows and 32 columns, each with its part of every contraction;
 // the first adds the others' sums, in order, through LDS and stores.  A lane reads its own row; the operands of PD steps are in
 // flight, as many as the registers beside the sums allow.
@@ -177,11 +247,11 @@ template <typename TI, bool WT>
 __global__ void __launch_bounds__(256, 2) flex_shared_kernel(const FlexBlock* __restrict__ blocks, const FlexPart* __restrict__ parts, int nblocks, int tiles_n,
                                                              const TI* __restrict__ A, int64_t lda, const TI* __restrict__ W, TI* __restrict__ C, int64_t ldc,
                                                              int64_t Z) {
-  const int64_t unit = blockIdx.x, zt = unit / tiles_n, z0 = 32 * zt;
-  int tile = static_cast<int>(unit - zt * tiles_n);
-  int b = 0;
-  while (b < nblocks && tile >= blocks[b].nt) tile -= blocks[b++].nt;
-  if (b == nblocks || z0 >= Z) return;
+  const uint32_t column = static_cast<uint32_t>(tiles_n), zt = blockIdx.x / column;
+  const int64_t z0 = static_cast<int64_t>(zt) * 32;
+  int tile = static_cast<int>(blockIdx.x - zt * column);
+  const int b = flex_find_block<false>(blocks, nblocks, tile);
+  if (b >= nblocks || z0 >= Z) return;
   const FlexBlock blk = blocks[b];
   switch (blk.D) {
     case 1: flex_shared_tile<TI, 1, WT>(blk, parts, A, lda, W, C, ldc, Z, z0, tile * 32); break;
@@ -191,24 +261,116 @@ __global__ void __launch_bounds__(256, 2) flex_shared_kernel(const FlexBlock* __
   }
 }
 
+// ---- blocks of few columns: a wavefront has ZT row tiles and a column tile to itself; the operands of two steps are in flight, and a lane
+// reads its own rows, whose lines the next steps and the neighbouring column tiles find in L1.  Bound by the latency of a tile's few
+// steps, so by how many wavefronts a SIMD holds (more steps in flight cost registers, and 1.05 to 1.3 times as long); the result leaves in
+// lines.  A workgroup that stages rows for one or two column tiles reads half or a quarter of a line of every row and step and
+// waits for all four wavefronts.  Forward of 0e+1o+2e rows in ir_mul, us, staged / this: float 16 ch 20 000 rows 17 / 9.7, 64 ch 9 000
+// 19.5 / 16.3, 96 ch 4 500 22.4 / 17.7; bfloat16 16 ch 20 000 15.3 / 7.3, 96 ch 4 500 14.6 / 10.6, l <= 3 48 ch 9 000 22.7 / 13.0.
+template <typename TI, int D, int ZT, bool WT>
+__device__ __forceinline__ void flex_direct_tile(const FlexBlock& blk, const FlexPart* __restrict__ parts, const TI* __restrict__ A, int64_t lda,
+                                                 const TI* __restrict__ W, TI* __restrict__ C, int64_t ldc, int64_t Z, int64_t z0, int n0, char* lds) {
+  using Weights = FlexWeights<TI, WT>;
+  constexpr int EPV = Weights::EPV, STEP = Weights::STEP, PD = 2;
+  const int lane = threadIdx.x & 63, c = lane & 31, h = lane >> 5;
+  fx16 acc[ZT][D];
+#pragma unroll
+  for (int t = 0; t < ZT; ++t)
+#pragma unroll
+    for (int i = 0; i < D; ++i) acc[t][i] = fx16{0};
+  const int n = min(n0 + c, blk.N - 1);
+  const TI* row[ZT];
+#pragma unroll
+  for (int t = 0; t < ZT; ++t) row[t] = A + min(z0 + 32 * t + c, Z - 1) * lda;
+  float scale = 1.0f;
+  for (int p = 0; p < blk.parts; ++p) {
+    const FlexPart part = parts[blk.first + p];
+#pragma unroll
+    for (int t = 0; t < ZT; ++t) {
+      float before = scale;
+      flex_rescale(acc[t], before, part.coeff, p == 0);
+    }
+    scale = part.coeff;
+    const int K = part.K;
+    uint4 x[PD][ZT][D];
+    Weights w[PD];
+    const uint32_t w_lane = Weights::lane_of(n, h, K, blk.N);
+    auto load = [&](int k0, uint4 (&xx)[ZT][D], Weights& ww) {  // (past the end the last step again: not used)
+      const int k = min(k0, K - STEP);
+#pragma unroll
+      for (int t = 0; t < ZT; ++t)
+#pragma unroll
+        for (int i = 0; i < D; ++i) xx[t][i] = *reinterpret_cast<const uint4*>(row[t] + part.a0 + static_cast<int64_t>(k + EPV * h) * D + i * EPV);
+      ww.load(W + part.w0, k, blk.N, w_lane);
+    };
+#pragma unroll
+    for (int j = 0; j < PD; ++j) load(j * STEP, x[j], w[j]);
+    int k0 = 0;
+    for (; k0 + PD * STEP <= K; k0 += PD * STEP)
+#pragma unroll
+      for (int j = 0; j < PD; ++j) {
+#pragma unroll
+        for (int t = 0; t < ZT; ++t) w[j].multiply(x[j][t], acc[t]);
+        load(k0 + (PD + j) * STEP, x[j], w[j]);
+      }
+#pragma unroll
+    for (int j = 0; j < PD - 1; ++j)
+      if (k0 + j * STEP < K)
+#pragma unroll
+        for (int t = 0; t < ZT; ++t) w[j].multiply(x[j][t], acc[t]);
+  }
+#pragma unroll
+  for (int t = 0; t < ZT; ++t) flex_store_lines<true>(blk, C, ldc, Z, z0 + 32 * t, n0, acc[t], scale, lds);
+}
+
+// unit = (column tiles of the blocks one after the other) x (ZT row tiles), four to a workgroup: its wavefronts share rows.  ONE: every
+// block has one component.
+template <typename TI, bool WT, bool ONE, int ZT>
+__global__ void __launch_bounds__(256, ONE ? (ZT == 1 ? 4 : 3) : 2) flex_direct_kernel(const FlexBlock* __restrict__ blocks, const FlexPart* __restrict__ parts, int nblocks,
+                                                                                      int tiles_n, const TI* __restrict__ A, int64_t lda, const TI* __restrict__ W,
+                                                                                      TI* __restrict__ C, int64_t ldc, int64_t Z) {
+  __shared__ __align__(16) char lines[4][ONE ? kFlexLineBytes<1> : kFlexLineBytes<7>];
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  const uint32_t column = static_cast<uint32_t>(tiles_n), unit = blockIdx.x * 4 + wave, zt = unit / column;  // (grid x 4 < 2^32)
+  const int64_t z0 = static_cast<int64_t>(zt) * (32 * ZT);
+  int tile = static_cast<int>(unit - zt * column);
+  const int b = flex_find_block<false>(blocks, nblocks, tile);
+  if (b >= nblocks || z0 >= Z) return;
+  const FlexBlock blk = blocks[b];
+  char* lds = lines[wave];
+  if constexpr (ONE) {
+    flex_direct_tile<TI, 1, ZT, WT>(blk, parts, A, lda, W, C, ldc, Z, z0, tile * 32, lds);
+  } else {
+    switch (blk.D) {
+      case 1: flex_direct_tile<TI, 1, ZT, WT>(blk, parts, A, lda, W, C, ldc, Z, z0, tile * 32, lds); break;
+      case 3: flex_direct_tile<TI, 3, ZT, WT>(blk, parts, A, lda, W, C, ldc, Z, z0, tile * 32, lds); break;
+      case 5: flex_direct_tile<TI, 5, ZT, WT>(blk, parts, A, lda, W, C, ldc, Z, z0, tile * 32, lds); break;
+      default: flex_direct_tile<TI, 7, ZT, WT>(blk, parts, A, lda, W, C, ldc, Z, z0, tile * 32, lds);
+    }
+  }
+}
+
 // ---- more tiles: a workgroup stages its rows through LDS.  Bound by the matrix cores from some 10 000 rows of float on (20 000 rows of
 // 128x0e+128x1o+128x2e in mul_ir, forward: 131 -> 73 us, 80 TFLOP/s; 38 at the rate of a large product), below by the latency of the
 // first and last step of a tile (5 003 rows 37 -> 24 us), in 2-byte elements by bytes and latency (8 000 rows 25 -> 13 us).
-// A workgroup has RT row tiles of 32 and 4 / RT column tiles of a block, a wavefront each one of the four pairs.  The rows come in
+// A workgroup has RT row tiles of 32 and 4 / RT column tiles of a block, a wavefront each one of the four pairs (MIXED, RT = 2: three have
+// the row tile at z0, the fourth that at z1 and a column tile of its own).  The rows come in
 // chunks of 4 / RT steps, two buffers in turn, one barrier a chunk: 128 D / RT adjacent bytes of every row, whole lines of
 // memory where a lane's own row would be a line per lane and load (64 lines an instruction, four times over for the four
 // wavefronts).  16 bytes of padding per row put the lanes' reads on all banks.  The weights go straight to registers, four steps ahead.
-template <typename TI, int D, int RT, int ZT, bool WT>
+template <typename TI, int D, int RT, int ZT, bool WT, bool WHOLE, bool MIXED = false>
 __device__ __forceinline__ void flex_stage_tile(const FlexBlock& blk, const FlexPart* __restrict__ parts, const TI* __restrict__ A, int64_t lda,
-                                                const TI* __restrict__ W, TI* __restrict__ C, int64_t ldc, int64_t Z, int64_t z0, int first_tile, char* lds) {
+                                                const TI* __restrict__ W, TI* __restrict__ C, int64_t ldc, int64_t Z, int64_t z0, int first_tile, char* lds, int64_t z1 = 0, int last_tile = 0) {
   using Weights = FlexWeights<TI, WT>;
   constexpr int ES = sizeof(TI), EPV = Weights::EPV, STEP = Weights::STEP;
   constexpr int SPC = 4 / RT, KC = SPC * STEP;                       // steps and channels of a chunk
   constexpr int PR = KC * D * ES / 16, RS = PR * 16 + 16, BUF = 32 * RT * ZT * RS;  // 16-byte pieces of a row, its stride, a buffer
   constexpr int NP = D * ZT;                                                        // pieces a lane brings
   static_assert(32 * RT * ZT * PR == 256 * NP && 2 * BUF <= kFlexStageBytes, "the rows of a chunk");
+  static_assert(4 * kFlexLineBytes<D> <= kFlexStageBytes, "the lines of four wavefronts");
   const int lane = threadIdx.x & 63, c = lane & 31, h = lane >> 5;
-  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)), rt = wave / (4 / RT), n0 = (first_tile + wave % (4 / RT)) * 32;
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  const int rt = MIXED ? wave == 3 : wave / (4 / RT), n0 = 32 * (!MIXED ? first_tile + wave % (4 / RT) : rt ? last_tile : first_tile + wave);
   fx16 acc[ZT][D];
 #pragma unroll
   for (int t = 0; t < ZT; ++t)
@@ -220,7 +382,7 @@ __device__ __forceinline__ void flex_stage_tile(const FlexBlock& blk, const Flex
 #pragma unroll
   for (int j = 0; j < NP; ++j) {
     const int piece = j * 256 + threadIdx.x, r = piece / PR, q = piece % PR;
-    from[j] = A + min(z0 + r, Z - 1) * lda;
+    from[j] = A + min(MIXED && r >= 32 * ZT ? z1 + (r - 32 * ZT) : z0 + r, Z - 1) * lda;
     into[j] = r * RS + q * 16;
     col[j] = q * EPV;
   }
@@ -266,6 +428,7 @@ __device__ __forceinline__ void flex_stage_tile(const FlexBlock& blk, const Flex
 #pragma unroll
           for (int t = 0; t < ZT; ++t) {
             uint4 op[D];
+            if constexpr (D == 7 && ES == 2 && WT) __builtin_amdgcn_sched_barrier(0);  // (a step at a time: 54 registers spilled, so 4)
 #pragma unroll
             for (int i = 0; i < D; ++i) op[i] = *reinterpret_cast<const uint4*>(mine + turn * BUF + 32 * t * RS + s * STEP * D * ES + 16 * i);
             w[(ch * SPC + s) % WD].multiply(op, acc[t]);
@@ -279,66 +442,45 @@ __device__ __forceinline__ void flex_stage_tile(const FlexBlock& blk, const Flex
     for (; k4 + 4 * STEP <= K; k4 += 4 * STEP) four(k4, std::true_type{});
     if (k4 < K) four(k4, std::false_type{});
   }
-  // The tile goes out through LDS as well, 64 D bytes of every row at a time: a lane's own 16-byte pieces are a write request each
-  // (20 000 rows of 128x0e+128x1o+128x2e, float: 79 us with such stores, 60 without any).
-  constexpr int COLS = 64 / ES, OS = 64 * D + 16, OP = 4 * D;  // columns a turn; a row's stride and 16-byte pieces in LDS
-  static_assert(4 * 32 * OS <= kFlexStageBytes, "a turn of four wavefronts");
-  char* out_lds = lds + wave * 32 * OS;
   __syncthreads();  // (no wavefront reads the rows any more)
 #pragma unroll
-  for (int turn_z = 0; turn_z < ZT * (32 / COLS); ++turn_z) {
-    const int t = turn_z / (32 / COLS), turn_n = turn_z % (32 / COLS);
-#pragma unroll
-    for (int a = 0; a < COLS / 8; ++a) {
-      float v[4 * D];
-#pragma unroll
-      for (int b = 0; b < 4; ++b)
-#pragma unroll
-        for (int i = 0; i < D; ++i) v[b * D + i] = scale * acc[t][i][4 * (turn_n * (COLS / 8) + a) + b];
-      char* to = out_lds + c * OS + (8 * a + 4 * h) * D * ES;
-#pragma unroll
-      for (int i = 0; i < D; ++i) {
-        if constexpr (ES == 4) *reinterpret_cast<float4*>(to + 16 * i) = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
-        else *reinterpret_cast<uint2*>(to + 8 * i) = make_uint2(mm_pack<TI>(v[4 * i], v[4 * i + 1]), mm_pack<TI>(v[4 * i + 2], v[4 * i + 3]));
-      }
-    }
-    __builtin_amdgcn_wave_barrier();
-    const int from_col = (n0 + turn_n * COLS) * D, ends_col = blk.N * D;
-#pragma unroll
-    for (int j = 0; j < 2 * D; ++j) {
-      const int piece = j * 64 + lane, r = piece / OP, q = piece % OP;
-      const int64_t z = z0 + 32 * (rt * ZT + t) + r;
-      const u32x4 value = *reinterpret_cast<const u32x4*>(out_lds + r * OS + 16 * q);
-      const int left = ends_col - (from_col + q * EPV);  // elements of the block from here on: multiples of 4, so half a piece of 2-byte ones may be
-      if (z < Z && left > 0) {
-        TI* to = C + z * ldc + blk.c0 + from_col + q * EPV;
-        if (ES == 4 || left >= EPV) *reinterpret_cast<u32x4*>(to) = value;
-        else *reinterpret_cast<uint2*>(to) = make_uint2(value[0], value[1]);
-      }
-    }
-    __builtin_amdgcn_wave_barrier();
-  }
+  for (int t = 0; t < ZT; ++t) flex_store_lines<WHOLE>(blk, C, ldc, Z, (MIXED && rt ? z1 : z0 + 32 * ZT * rt) + 32 * t, n0, acc[t], scale, lds + wave * kFlexLineBytes<D>);
 }
 
-// A slab of 128 ZT rows and a block of nt column tiles are nt workgroups: four columns x one row tile for every whole four columns, the
-// rest two columns x two row tiles or one x four.  The last block first: the blocks of most components are the longest.  ZT > 1: row
+// A slab of 128 ZT rows and a block of nt column tiles are nt workgroups: four columns x one row tile for every whole four columns.  Of
+// those that are left, one is four row tiles, two are two x two, and three are three workgroups of three columns x one row tile and,
+// by the fourth wavefront, one column of the last row tile (as three x four row tiles, rows staged three times over, 96 ch took twice
+// as long).  The last block first: the blocks of most components are the longest.  ZT > 1: row
 // tiles of a wavefront, where every block has one component (a tile of one is over before its first loads have paid).
-template <typename TI, bool WT, int ZT>
+template <typename TI, bool WT, int ZT, bool WHOLE>
 __global__ void __launch_bounds__(256, 2) flex_stage_kernel(const FlexBlock* __restrict__ blocks, const FlexPart* __restrict__ parts, int nblocks,
                                                             const TI* __restrict__ A, int64_t lda, const TI* __restrict__ W, TI* __restrict__ C, int64_t ldc,
                                                             int64_t Z, int64_t slabs) {
   __shared__ __align__(16) char lds[kFlexStageBytes];
-  int64_t unit = blockIdx.x;
-  int b = nblocks - 1;
-  while (b >= 0 && unit >= slabs * blocks[b].nt) unit -= slabs * blocks[b--].nt;
+  const uint32_t column = blockIdx.x / static_cast<uint32_t>(slabs);  // (slab and column tile of a block run over slabs x its extent)
+  int before = static_cast<int>(column);
+  const int b = nblocks - 1 - flex_find_block<true>(blocks, nblocks, before);
   if (b < 0) return;
   const FlexBlock blk = blocks[b];
-  const int64_t slab = unit / blk.nt;
-  const int t = static_cast<int>(unit - slab * blk.nt), full = blk.nt & ~3, rest = blk.nt - full;
-  const int rt = t < full ? 1 : rest == 2 ? 2 : 4, tile = t < full ? t & ~3 : rest == 2 ? full : t;
-  const int64_t z0 = ZT * (slab * 128 + (t < full ? (t & 3) * 32 : rest == 2 ? (t - full) * 64 : 0));
-  if (z0 >= Z) return;
-#define STAGE(D)                                                                                                                do {                                                                                                                            if (rt == 1) flex_stage_tile<TI, D, 1, ZT, WT>(blk, parts, A, lda, W, C, ldc, Z, z0, tile, lds);                                  else if (rt == 2) flex_stage_tile<TI, D, 2, ZT, WT>(blk, parts, A, lda, W, C, ldc, Z, z0, tile, lds);                             else flex_stage_tile<TI, D, 4, ZT, WT>(blk, parts, A, lda, W, C, ldc, Z, z0, tile, lds);                                        } while (0)
+  const uint32_t own = blockIdx.x - static_cast<uint32_t>(slabs) * (column - before), slab = own / static_cast<uint32_t>(blk.nt);
+  const int t = static_cast<int>(own - slab * blk.nt), full = blk.nt & ~3, rest = blk.nt - full;
+  const int64_t zs = static_cast<int64_t>(slab) * (128 * ZT);
+  constexpr int RZ = 32 * ZT;  // rows of a row tile
+#define STAGE(D)                                                                                                              \
+  do {                                                                                                                       \
+    if (t < full) {                                                                                                          \
+      const int64_t z0 = zs + (t & 3) * RZ;                                                                                   \
+      if (z0 < Z) flex_stage_tile<TI, D, 1, ZT, WT, WHOLE>(blk, parts, A, lda, W, C, ldc, Z, z0, t & ~3, lds);                  \
+    } else if (rest == 1) {                                                                                                  \
+      if (zs < Z) flex_stage_tile<TI, D, 4, ZT, WT, WHOLE>(blk, parts, A, lda, W, C, ldc, Z, zs, full, lds);                    \
+    } else if (rest == 2) {                                                                                                  \
+      const int64_t z0 = zs + 2 * (t - full) * RZ;                                                                            \
+      if (z0 < Z) flex_stage_tile<TI, D, 2, ZT, WT, WHOLE>(blk, parts, A, lda, W, C, ldc, Z, z0, full, lds);                    \
+    } else {                                                                                                                 \
+      const int64_t z0 = zs + (t - full) * RZ;                                                                                \
+      if (z0 < Z) flex_stage_tile<TI, D, 2, ZT, WT, WHOLE, true>(blk, parts, A, lda, W, C, ldc, Z, z0, full, lds, zs + 3 * RZ, t); \
+    }                                                                                                                        \
+  } while (0)
   if constexpr (ZT > 1) {
     STAGE(1);
   } else {
@@ -556,29 +698,43 @@ extern "C" int cueq_linear_flex(int32_t dtype, int32_t transposed_weights, int64
   // 128x0e+128x1o+128x2e in mul_ir, float, forward 21.8 -> 9.7 us, 1 000 rows 22.1 -> 12.6 (1 400 rows, past the line: 22.5 either way)
   const int64_t tiles = (rows + 31) / 32 * column_tiles;
   const bool shared = tiles <= 2ll * device_cus();
-  // ir_mul rows (the caller says that every block has one component): four row tiles a wavefront once there are so many workgroups; us for one / four, 128 ch:
-  // float 4 000 rows (1 152 workgroups of one tile) 23 / 26, 8 000 38 / 38, 16 000 67 / 57, 32 000 147 / 113; bfloat16 2 000 9.8 / 9.7,
-  // 4 000 13.8 / 9.8, 32 000 73 / 35
-  const bool tall = mul_ir == kFlexOneComponent && !shared && (rows + 127) / 128 * column_tiles >= (dtype == CUEQ_F32 ? 9ll : 4ll) * device_cus();
+  // Rows in ir_mul (the caller says that every block has one component).  Four staged row tiles a wavefront once there are so many
+  // workgroups; us for one / four, 128 ch l <= 2: float 4 000 rows (1 152 workgroups of one tile) 23 / 26, 8 000 38 / 38, 16 000 67 / 57,
+  // 32 000 147 / 113; bfloat16 2 000 9.8 / 9.7, 4 000 13.8 / 9.8, 32 000 73 / 35.  One where the columns are whole groups of four (or four
+  // and two: 192 ch, float, 1 000 rows 16 / 16.6, 3 000 53 / 51, so staged up to some 5 000 tiles).  Otherwise a wavefront has its tile to
+  // itself, and two row tiles from three column tiles a block on (their weights are read half as often: us for one / two, 96 ch l <= 2, float, input
+  // gradient 9 000 rows 34 / 29, bfloat16 9 000 18.6 / 16.0; 64 ch, float, forward 9 000 16.3 / 18.1).
+  // Rows in mul_ir: a component more is a longer step, and staging is the faster way but for one column tile of 2-byte elements
+  // and few rows (16 ch l <= 2, 6 500 rows, 7.6 / 7.0; 32 ch l <= 3, 20 000 13.3 / 16.0).
+  const bool whole = dtype == CUEQ_F32 || (mul_ir & kFlexWholePieces), one = (mul_ir & kFlexOneComponent) && whole;
+  const bool tall = one && !shared && column_tiles >= (dtype == CUEQ_F32 ? 4 : 3) * nblocks &&
+                    (rows + 127) / 128 * column_tiles >= (dtype == CUEQ_F32 ? 9ll : 4ll) * device_cus();
+  const bool even = column_tiles >= 4 * nblocks && column_tiles % (2 * nblocks) == 0;  // (on average: blocks of groups of four and two columns)
+  const bool direct = whole && !shared && !tall && (one ? !even || (dtype == CUEQ_F32 && column_tiles % (4 * nblocks) != 0 && tiles > 20ll * device_cus())
+                                                         : dtype != CUEQ_F32 && column_tiles == nblocks && tiles <= 4ll * device_cus());
+  const int zt = one && column_tiles >= 3 * nblocks && tiles >= 16ll * device_cus() ? 2 : 1;
   const int64_t slab_rows = tall ? 512 : 128, slabs = (rows + slab_rows - 1) / slab_rows;
-  const int64_t grid = shared ? tiles : slabs * column_tiles;
-  CUEQ_REQUIRE(grid < (1ll << 31), CUEQ_ERR_TOO_LARGE, "linear_flex: too many rows");
-  KernelTimer timer(mul_ir && mul_ir != kFlexOneComponent ? "linear_rows_mul_ir" : "linear_rows", stream);
+  const int64_t grid = shared ? tiles : direct ? ((rows + 32 * zt - 1) / (32 * zt) * column_tiles + 3) / 4 : slabs * column_tiles;
+  CUEQ_REQUIRE(grid < (1ll << 30), CUEQ_ERR_TOO_LARGE, "linear_flex: too many rows");
+  KernelTimer timer(mul_ir & kFlexMulIr ? "linear_rows_mul_ir" : "linear_rows", stream);
 #define FLEX_LAUNCH(KERNEL, ...)                                                                                                                         \
   hipLaunchKernelGGL((KERNEL), dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, static_cast<const FlexBlock*>(blocks),                           \
                      static_cast<const FlexPart*>(parts), nblocks, __VA_ARGS__)
 #define FLEX_OPERANDS(TI) static_cast<const TI*>(A), lda, static_cast<const TI*>(W), static_cast<TI*>(C), ldc, rows
-#define FLEX(TI)                                                                                                  \
-  do {                                                                                                            \
-    if (shared && transposed_weights) FLEX_LAUNCH((flex_shared_kernel<TI, true>), column_tiles, FLEX_OPERANDS(TI));  \
-    else if (shared) FLEX_LAUNCH((flex_shared_kernel<TI, false>), column_tiles, FLEX_OPERANDS(TI));                  \
-    else if (transposed_weights && tall) FLEX_LAUNCH((flex_stage_kernel<TI, true, 4>), FLEX_OPERANDS(TI), slabs);    \
-    else if (transposed_weights) FLEX_LAUNCH((flex_stage_kernel<TI, true, 1>), FLEX_OPERANDS(TI), slabs);            \
-    else if (tall) FLEX_LAUNCH((flex_stage_kernel<TI, false, 4>), FLEX_OPERANDS(TI), slabs);                         \
-    else FLEX_LAUNCH((flex_stage_kernel<TI, false, 1>), FLEX_OPERANDS(TI), slabs);                                   \
+#define FLEX_WT(TI, WT)                                                                                                    \
+  do {                                                                                                                      \
+    if (shared) FLEX_LAUNCH((flex_shared_kernel<TI, WT>), column_tiles, FLEX_OPERANDS(TI));                                   \
+    else if (direct && !one) FLEX_LAUNCH((flex_direct_kernel<TI, WT, false, 1>), column_tiles, FLEX_OPERANDS(TI));         \
+    else if (direct && zt == 1) FLEX_LAUNCH((flex_direct_kernel<TI, WT, true, 1>), column_tiles, FLEX_OPERANDS(TI));       \
+    else if (direct) FLEX_LAUNCH((flex_direct_kernel<TI, WT, true, 2>), column_tiles, FLEX_OPERANDS(TI));                  \
+    else if (tall) FLEX_LAUNCH((flex_stage_kernel<TI, WT, 4, true>), FLEX_OPERANDS(TI), slabs);                               \
+    else if (whole || sizeof(TI) == 4) FLEX_LAUNCH((flex_stage_kernel<TI, WT, 1, true>), FLEX_OPERANDS(TI), slabs);           \
+    else FLEX_LAUNCH((flex_stage_kernel<TI, WT, 1, sizeof(TI) == 4>), FLEX_OPERANDS(TI), slabs);                              \
   } while (0)
+#define FLEX(TI) do { if (transposed_weights) FLEX_WT(TI, true); else FLEX_WT(TI, false); } while (0)
   FLEX_DISPATCH(dtype, FLEX);
 #undef FLEX
+#undef FLEX_WT
 #undef FLEX_OPERANDS
 #undef FLEX_LAUNCH
   CUEQ_CHECK_HIP(hipGetLastError());

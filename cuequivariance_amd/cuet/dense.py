@@ -273,13 +273,25 @@ def _rows_launches(mod: "SegmentedPolynomialDense", es: int):
 
 
 # Rows from which on the row-streaming launches (weights in LDS) are the faster ones for forward and input gradient, by (rows in
-# mul_ir, element size) and multiplicity (up to 32, up to 64, above): where the measured times of the two cross.  Above, the weights are
-# read once per CU and not once per 128 rows (or 512); below, a launch per degree is bound by the chain of one wavefront.  Forward of
-# 0e+1o+2e blocks, us, streaming / staged: 128 ch float mul_ir 12 000 rows 93 / 43, 50 000 209 / 179, 60 000 204 / 206; ir_mul 30 000
-# 135 / 107, 64 000 192 / 213; bfloat16 mul_ir 12 000 38 / 13, 75 000 96 / 97, 100 000 118 / 127.
+# mul_ir, element size) and multiplicity (up to 32, 64, 96, above): where the measured times of the two cross.  Above, the weights are
+# read once per CU and not once per 32 rows (or 512); below, a launch per degree is bound by the chain of one wavefront.  Forward of
+# 0e+1o+2e blocks, us, row-streaming / tiles of csrc/linear_flex.hip: 128 ch float mul_ir 12 000 rows 93 / 43, 50 000 209 / 179,
+# 60 000 204 / 206; ir_mul 30 000 135 / 107, 64 000 192 / 213; bfloat16 mul_ir 12 000 38 / 13, 75 000 96 / 97, 100 000 118 / 127; 96 ch float ir_mul
+# 9 000 31 / 29, 13 000 36 / 39; mul_ir 40 000 111 / 103, 80 000 (l <= 1) 77 / 91; 64 ch bfloat16 ir_mul 2 000 8.5 / 7.4, 6 500 9.1 / 11;
+# mul_ir float 60 000 80 / 72, 97 500 115 / 121, bfloat16 96 000 56 / 47, 156 000 82 / 91; 32 ch float mul_ir (l <= 1) 130 000 36 / 33, 300 000
+# 66 / 80; bfloat16 ir_mul never (200 000 70 / 47).
 _NEVER = 1 << 60
-_ROWS_FROM = {(False, 4): (6_000, 3_000, 50_000), (False, 2): (20_000, 12_000, 40_000), (True, 4): (110_000, 75_000, 55_000),
-              (True, 2): (_NEVER, 120_000, 75_000)}
+_ROWS_FROM = {(False, 4): (_NEVER, _NEVER, 12_000, 50_000), (False, 2): (_NEVER, 3_000, _NEVER, 40_000), (True, 4): (170_000, 75_000, 45_000, 55_000),
+              (True, 2): (_NEVER, 120_000, 75_000, 75_000)}
+# ... where it is rows times components of a row that the crossing goes with (64 ch float 9 000 18 / 16, 13 000 21 / 22; l <= 3 6 500 20 / 20.6; 32 ch
+# 9 000 10.4 / 9.8, 13 000 11.8 / 11.2, 20 000 13.7 / 14.1; 96 ch bfloat16 20 000 26.7 / 25.3, 40 000 input gradient 42 / 45)
+_ROWS_COMPONENTS_FROM = {4: (80_000, 60_000, _NEVER, _NEVER), 2: (_NEVER, _NEVER, 250_000, _NEVER)}
+# ... and the same where some extents do not stream and take tiled launches, rows in ir_mul, up to 32, 64, 96, 192, above (256 ch float l <= 3
+# 2 000 47 / 53, 9 000 within 2 %; 160 ch never, 20 000 151 / 110, bfloat16 2 000 10.5 / 10.4, 4 500 13.7 / 17; 80 ch float 40 000 90 / 82, 80 000
+# 178 / 212, bfloat16 4 500 9.9 / 9.2, 6 500 11.1 / 11.4; 48 ch float 40 000 44 / 38, 80 000 80 / 90, bfloat16 40 000 25 / 22, but l <= 3
+# 9 000 11.6 / 13)
+_TILED_FROM = {4: (_NEVER, _NEVER, _NEVER, _NEVER, 2_000), 2: (_NEVER, _NEVER, _NEVER, 2_000, 2_000)}
+_TILED_COMPONENTS_FROM = {4: (_NEVER, 650_000, 450_000, _NEVER, _NEVER), 2: (_NEVER, _NEVER, 45_000, _NEVER, _NEVER)}
 # ... and for the weight gradient, whose row launches win from the first row on but for float in mul_ir and for up to 32 channels (their
 # 128 x 128 tiles are padding then: 200 000 rows of 32x0e+32x1o+32x2e, float: 485 us against 274)
 _GRADS_FROM = {(False, 4): (_NEVER, 0, 0), (False, 2): (15_000, 0, 0), (True, 4): (150_000, 5_000, 5_000), (True, 2): (0, 0, 0)}
@@ -294,21 +306,26 @@ def _linear_op(mod: "SegmentedPolynomialDense"):
         return None
     op = _lib.host().LinearOp(mod.input_sizes[1], mod.out_size, mod.input_sizes[0], mod.rows_mul_ir, mod.dx1_covers_input, mod.fwd_covers_output,
                               tables[2], tables[0], tables[1])
-    most = max(max(p.K, p.N) for p in mod.paths)
+    most, components = max(max(p.K, p.N) for p in mod.paths), sum(count for _, count, *_ in mod.fwd_groups)
     for es in (4, 2):
-        size = 0 if most <= 32 else 1 if most <= 64 else 2
-        rows_from, grads_from = _ROWS_FROM[(mod.rows_mul_ir, es)][size], _GRADS_FROM[(mod.rows_mul_ir, es)][size]
+        size = 0 if most <= 32 else 1 if most <= 64 else 2 if most <= 96 else 3
+        grads_from = _GRADS_FROM[(mod.rows_mul_ir, es)][min(size, 2)]
         if mod.rows_mul_ir:
             if mod.mul_ir is not None and mod.mul_ir.accepts({4: torch.float32, 2: torch.bfloat16}[es]):
                 fwd, dx, dw = mod.mul_ir.tables(es)
-                op.add_rows(es, rows_from, [(d, n, k, list(t), parts, c) for d, n, k, t, parts, c in fwd],
+                op.add_rows(es, _ROWS_FROM[True, es][size], [(d, n, k, list(t), parts, c) for d, n, k, t, parts, c in fwd],
                             [(d, n, k, list(t), parts, c) for d, n, k, t, parts, c in dx])
                 op.add_grads(es, grads_from, [(K, N, c, 0, 0, 0, 0, list(t), list(w), [1] * len(w)) for K, N, c, t, _, w in dw])
             continue
         launches = _rows_launches(mod, es)
         if launches is not None:
             fwd, dx, streaming = launches
-            op.add_rows(es, rows_from if streaming else 2_000, fwd, dx)
+            if streaming:
+                rows, product = _ROWS_FROM[False, es][size], _ROWS_COMPONENTS_FROM[es][size]
+            else:
+                wide = 4 if most > 192 else size
+                rows, product = _TILED_FROM[es][wide], _TILED_COMPONENTS_FROM[es][wide]
+            op.add_rows(es, min(rows, product // components), fwd, dx)
         merged = _merged_weight_gradient(mod)
         if merged is not None:
             K, N, coeff, a0, c0, da, dc, runs = merged

@@ -460,8 +460,8 @@ int cueq_sum_rows(int32_t dtype, int64_t rows, int64_t cols, const void* in, flo
  * of the result: C[z, c0 + v D + i] = sum over the block's parts of coeff sum_u A[z, a0 + u D + i] W[w0 + u N + v] - with
  * transposed_weights W[w0 + v K + u], K the contraction length.  `blocks` and `parts` are device tables (FlexBlock, FlexPart of csrc/linear_flex.hip:
  * {int64 c0; int32 N, D, first part, parts, column tiles of 32, unused} and {int64 a0, w0; int32 contraction length; float coeff});
- * contraction lengths multiples of 8 (float32) / 16, N of 4, D 1, 3, 5 or 7, offsets of 16 bytes.  mul_ir 0 or 1 only names the timer;
- * 2 (named as 0) says that D is 1 in every block, which many rows are then worked on for. */
+ * contraction lengths multiples of 8 (float32) / 16, N of 4, D 1, 3, 5 or 7, offsets of 16 bytes.  mul_ir: 1 names the timer; what else a caller
+ * may say of its tables chooses kernels: 2 that D is 1 in every block, 4 that every N is a multiple of 8. */
 int cueq_linear_flex(int32_t dtype, int32_t transposed_weights, int64_t rows, const void* A, int64_t lda, const void* W, void* C,
                      int64_t ldc, const void* blocks, int32_t nblocks, const void* parts, int32_t column_tiles, int32_t mul_ir,
                      void* stream);

@@ -49,7 +49,7 @@ def _check(device, dtype, blocks, K, rows, mul_ir, transposed=False):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("transposed", [False, True])
-@pytest.mark.parametrize("mul_ir", [0, 1])
+@pytest.mark.parametrize("mul_ir", [0, 1, 4, 1 + 4])
 def test_many_rows_of_blocks_of_several_components(device, mul_ir, transposed, dtype):
     """The row counts from which on blocks of one component take four row tiles a wavefront: whoever names the rows ``ir_mul`` (0) may
     have blocks of more all the same."""
@@ -58,13 +58,25 @@ def test_many_rows_of_blocks_of_several_components(device, mul_ir, transposed, d
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("transposed", [False, True])
-def test_many_rows_of_blocks_of_one_component(device, transposed, dtype):
-    _check(device, dtype, [(32, 1), (64, 1), (16, 1), (160, 1)], 48, 40_003, 2, transposed)
+@pytest.mark.parametrize("said", [2, 2 + 4])
+@pytest.mark.parametrize("rows,extents", [(40_003, (32, 64, 16, 160)), (40_003, (96, 224)), (9_001, (96, 16, 224)), (9_001, (32, 64)), (1_501, [32] * 70)])
+def test_many_rows_of_blocks_of_one_component(device, rows, extents, said, transposed, dtype):
+    """Tiles through LDS four rows high, tiles a wavefront has to itself, one and two rows high, and more blocks than lanes."""
+    _check(device, dtype, [(n, 1) for n in extents], 48, rows, said, transposed)
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("mul_ir,blocks", [(1, [(4, 1), (20, 3), (36, 5), (68, 1), (12, 7)]), (2, [(4, 1), (36, 1), (132, 1)])])
+@pytest.mark.parametrize("mul_ir,blocks", [(1, [(4, 1), (20, 3), (36, 5), (68, 1), (12, 7)]), (2, [(4, 1), (36, 1), (132, 1)]), (0, [(100, 3), (228, 1)])])
 @pytest.mark.parametrize("rows", [700, 12_001, 40_003])
 def test_blocks_that_end_in_half_a_piece(device, rows, mul_ir, blocks, dtype):
     """N of 4 in 2-byte elements: a block's last 8 bytes of a row are half of a 16-byte piece, and what lies behind them belongs to nobody."""
     _check(device, dtype, blocks, 32, rows, mul_ir)
+
+
+@pytest.mark.parametrize("transposed", [False, True])
+@pytest.mark.parametrize("rows", [2_049, 40_003])
+@pytest.mark.parametrize("blocks", [[(96, 3), (96, 1)], [(224, 1), (96, 5)], [(32, 7), (32, 5), (16, 3), (32, 1)]])
+def test_three_column_tiles_left_and_one(device, blocks, rows, transposed):
+    """Three column tiles beside a multiple of four (a workgroup's fourth wavefront has the last row tile), and blocks of one in 2-byte elements."""
+    for dtype in (torch.float32, torch.bfloat16):
+        _check(device, dtype, blocks, 48, rows, 1 + 4, transposed)

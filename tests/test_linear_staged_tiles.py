@@ -10,6 +10,14 @@ from cuequivariance_amd import cue
 pytestmark = pytest.mark.gpu
 
 
+@pytest.fixture(autouse=True)
+def tables_alone(monkeypatch):
+    """No row-streaming or tiled launches, whatever the number of rows (rows in mul_ir have theirs from 55 000 rows on, past all cases here)."""
+    from cuequivariance_amd.cuet import dense
+
+    monkeypatch.setattr(dense, "_rows_launches", lambda mod, es: None)
+
+
 def _check(device, irreps_in, irreps_out, rows, dtype, layout):
     from cuequivariance_amd import cuet
 
@@ -57,6 +65,13 @@ def test_against_64_bits(device, irreps_in, irreps_out, rows, layout, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("irreps_in,irreps_out,rows", [("144x0e+48x1o", "144x0e+48x1o", 40_001), ("80x0e+80x1o", "96x0e+32x1o", 33_000)])
+@pytest.mark.parametrize("irreps_in,irreps_out,rows", [
+    ("144x0e+48x1o", "144x0e+48x1o", 40_001),  # five and two column tiles of a block: groups of four, two and one
+    ("80x0e+80x1o", "96x0e+32x1o", 60_007),    # three and one
+])
 def test_taller_slabs(device, irreps_in, irreps_out, rows, dtype):
+    cus = torch.cuda.get_device_properties(device).multi_processor_count
+    for irreps in (irreps_in, irreps_out):  # (four row tiles a wavefront from so many workgroups of one on)
+        tiles = sum(-(-mul // 32) * ir.dim for mul, ir in cue.Irreps("O3", irreps))
+        assert -(-rows // 128) * tiles >= (9 if dtype == torch.float32 else 4) * cus
     _check(device, irreps_in, irreps_out, rows, dtype, cue.ir_mul)
