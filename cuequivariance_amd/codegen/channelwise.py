@@ -265,18 +265,19 @@ FWD_FOLD = 16   # registers of output sums that meet in LDS at a time
 
 
 def emit_lanes(A, st: ChannelwiseStructure):
-    """The lane's channel ``uu``, whether it has one (``active``), and which of the wavefront's batch rows it works on (``sub``)."""
+    """The lane's channel ``uu``, whether it has one (``active``; the others repeat the last channel, and may store what it stores), and
+    which of the wavefront's batch rows it works on (``sub``)."""
     if st.packed > 1:
         lanes = 64 // st.packed
         A(f"  const int sub = lane / {lanes};")
         if st.extent == lanes:
             A(f"  const int uu = lane & {lanes - 1}; constexpr bool active = true;")
         else:
-            A(f"  const int u = lane & {lanes - 1}; const bool active = u < {st.extent}; const int uu = active ? u : 0;")
+            A(f"  const int u = lane & {lanes - 1}; const bool active = u < {st.extent}; const int uu = active ? u : {st.extent - 1};")
     elif st.extent % 64 == 0:
         A("  constexpr int sub = 0; const int uu = ch * 64 + lane; constexpr bool active = true;")
     else:
-        A(f"  constexpr int sub = 0; const int u = ch * 64 + lane; const bool active = u < {st.extent}; const int uu = active ? u : 0;")
+        A(f"  constexpr int sub = 0; const int u = ch * 64 + lane; const bool active = u < {st.extent}; const int uu = active ? u : {st.extent - 1};")
 
 
 def emit_forward(st: ChannelwiseStructure, T: str, nsplit: int, waves_per_eu: int, ns: str, prefetch: bool = True) -> str:
@@ -648,13 +649,13 @@ def emit_backward(st: ChannelwiseStructure, T: str, waves_per_eu: int, prefetch:
                         A(f"{ind}    {{ const {fp} G = {expr}; D = fma(G, {S}_yv{j}, D); F{j} = fma(G, {S}_xv{i}, F{j}); }}")
                     A(f"{ind}    dwb = fma({S}_xv{i}, D, dwb); dxa{i} = fma(wb, D, dxa{i});")
                     A(f"{ind}  }}")
-                A(f"{ind}  if (active) io_stnt(dwb, dwp + {blk.b * st.extent} + uu);")
+                A(f"{ind}  io_stnt(dwb, dwp + {blk.b * st.extent} + uu);")
                 for j in blk.j_list:
                     A(f"{ind}  pj{j} = fma(wb, F{j}, pj{j});")
                 A(f"{ind}}}")
                 A(f"{ind}__builtin_amdgcn_sched_barrier(0);")
             for b_ in w_zero:
-                A(f"{ind}if (active) io_stnt({fp}(0), dwp + {b_ * st.extent} + uu);")
+                A(f"{ind}io_stnt({fp}(0), dwp + {b_ * st.extent} + uu);")
             # dx1: scatter.  Atomic adds are served per touched 32-byte sector, not per element: the components of a
             # channel-major group (a stride of d elements between lanes) go through LDS first, so that every atomic
             # instruction of the wavefront covers 64 consecutive elements as it does in the default layout.
@@ -670,23 +671,23 @@ def emit_backward(st: ChannelwiseStructure, T: str, waves_per_eu: int, prefetch:
                     guard = "" if st.extent % lanes == 0 else f"if (ch * {64 * d} + {k * lanes} + {own} < {st.extent * d}) "
                     A(f"{ind}  {guard}unsafeAtomicAdd(dp + {k * lanes} + {own}, dxs[{base}{k * lanes} + {own}]);")
                 A(f"{ind}}}")
-            A(f"{ind}if (active) {{")
-            A(f"{ind}  if (ATOMIC_DX1) {{")
-            A(f"{ind}    {fp}* dp = dx1 + {S}_srow * {st.nseg_x1 * st.extent}ll;")
+            A(f"{ind}if (ATOMIC_DX1) {{")
+            A(f"{ind}  {fp}* dp = dx1 + {S}_srow * {st.nseg_x1 * st.extent}ll;")
+            if st.extent % lanes:  # (where some lanes have no channel: no sum is put off until behind the branch, with all its operands)
+                for name in [f"dxa{i}" for i in i_used if i not in staged_segments] + [f"pj{j}" for j in j_used]:
+                    A(f'{ind}  asm volatile("" : "+v"({name}));')
+            A(f"{ind}  if (active) {{")
             for i in i_used:
                 if i not in staged_segments:
                     A(f"{ind}    unsafeAtomicAdd(dp + ({st.x1_at(i)}), dxa{i});")
-            A(f"{ind}  }} else {{")
-            A(f"{ind}    TI* __restrict__ dp = dx1_partial + z * {st.nseg_x1 * st.extent}ll;")
-            for i in sorted(i_used + i_zero):
-                A(f"{ind}    io_st(" + (f"dxa{i}" if i in i_used else f"{fp}(0)") + f", dp + ({st.x1_at(i)}));")
             A(f"{ind}  }}")
             A(f"{ind}}}")
             # dx2: reduced over the 64 lanes, the sums halved among them (16 sums over 64 lanes: 15 halving steps and 2 plain
             # ones, one store of 16 lanes, where 16 butterflies take 96 steps and one lane 16 stores; forward + backward, fp32:
             # 32 ch l <= 2, 60 000 edges 124.5 -> 118.6 us, 128 ch l <= 3, 1 000 edges 102.2 -> 99.0 us); channel chunks and
             # wavefronts of one batch row are folded afterwards
-            A(f"{ind}if (!active) {{" + " ".join(f"pj{j} = 0;" for j in j_used) + "}")
+            for j in j_used:
+                A(f"{ind}pj{j} = active ? pj{j} : {fp}(0);")
             if st.harmonics:
                 # dv[a] = sum_j pj[j] dY_j/dv[a] (this lane's share: the sums over channels and blocks are linear)
                 rests = set()
@@ -696,6 +697,10 @@ def emit_backward(st: ChannelwiseStructure, T: str, waves_per_eu: int, prefetch:
                             rest = list(vi)
                             rest.remove(a)
                             rests.add(tuple(rest))
+            A(f"{ind}}} else {{")
+            A(f"{ind}  TI* __restrict__ dp = dx1_partial + z * {st.nseg_x1 * st.extent}ll;")
+            for i in sorted(i_used + i_zero):
+                A(f"{ind}  io_st(" + (f"dxa{i}" if i in i_used else f"{fp}(0)") + f", dp + ({st.x1_at(i)}));")
                 A(f"{ind}{fp} dv0 = 0, dv1 = 0, dv2 = 0;")
                 A(f"{ind}{{")
                 _emit_monomials(A, ind + "  ", fp, _with_prefixes(rests), [f"{S}_v0", f"{S}_v1", f"{S}_v2"])
