@@ -369,8 +369,12 @@ def emit_forward(st: ChannelwiseStructure, T: str, nsplit: int, waves_per_eu: in
         for k in ks:
             A(f"  {fp} acc{k} = 0;")
         A("  int64_t z0, z1;")
-        A("  if (csr_offsets) { z0 = csr_offsets[r]; z1 = csr_offsets[r + 1]; } else { z0 = r; z1 = r + 1; }")
-        A("  if (nparts > 1) {" if P == 1 else "  {")
+        if P == 1:
+            A("  if (csr_offsets) { z0 = csr_offsets[r]; z1 = csr_offsets[r + 1]; } else { z0 = r; z1 = r + 1; }")
+            A("  if (nparts > 1) {")
+        else:  # a batched output: every group of lanes has an output row to itself
+            A(f"  if (csr_offsets) {{ z0 = csr_offsets[r]; z1 = csr_offsets[r + 1]; }} else {{ r = r * {P} + sub; z0 = r; z1 = r < rows ? r + 1 : r; }}")
+            A("  if (csr_offsets) {")
         A("    const int64_t first = z0, count = z1 - z0;")
         share = "part" if P == 1 else f"(part * {P} + sub)"
         A(f"    const int shift = 31 - __builtin_clz(nparts * {P});  // (a power of two)")
@@ -409,6 +413,17 @@ def emit_forward(st: ChannelwiseStructure, T: str, nsplit: int, waves_per_eu: in
             body("a", "    ")
             A("  }")
         A(f"  TI* __restrict__ op = out + r * {st.nseg_out * st.extent}ll;")
+        if P > 1:
+            A("  if (!csr_offsets) {")
+            A("    if (active && r < rows) {")
+            for k in range(st.nseg_out):
+                if k in ks:
+                    A(f"      io_stnt(acc{k}, op + ({st.out_at(k)}));")
+                elif q == 0 and not any(k in blk.k_list for blk in st.blocks):
+                    A(f"      io_stnt({fp}(0), op + ({st.out_at(k)}));")
+            A("    }")
+            A("    return;")
+            A("  }")
         # registers to store: a segment each; with several batch rows per wavefront, the sums over them are halved among their
         # lanes, so that a register ends with a segment per group of lanes
         totals = [(f"acc{k}", [k]) for k in ks]
@@ -681,6 +696,10 @@ def emit_backward(st: ChannelwiseStructure, T: str, waves_per_eu: int, prefetch:
                 if i not in staged_segments:
                     A(f"{ind}    unsafeAtomicAdd(dp + ({st.x1_at(i)}), dxa{i});")
             A(f"{ind}  }}")
+            A(f"{ind}}} else {{")
+            A(f"{ind}  TI* __restrict__ dp = dx1_partial + z * {st.nseg_x1 * st.extent}ll;")
+            for i in sorted(i_used + i_zero):
+                A(f"{ind}  io_st(" + (f"dxa{i}" if i in i_used else f"{fp}(0)") + f", dp + ({st.x1_at(i)}));")
             A(f"{ind}}}")
             # dx2: reduced over the 64 lanes, the sums halved among them (16 sums over 64 lanes: 15 halving steps and 2 plain
             # ones, one store of 16 lanes, where 16 butterflies take 96 steps and one lane 16 stores; forward + backward, fp32:
@@ -697,10 +716,6 @@ def emit_backward(st: ChannelwiseStructure, T: str, waves_per_eu: int, prefetch:
                             rest = list(vi)
                             rest.remove(a)
                             rests.add(tuple(rest))
-            A(f"{ind}}} else {{")
-            A(f"{ind}  TI* __restrict__ dp = dx1_partial + z * {st.nseg_x1 * st.extent}ll;")
-            for i in sorted(i_used + i_zero):
-                A(f"{ind}  io_st(" + (f"dxa{i}" if i in i_used else f"{fp}(0)") + f", dp + ({st.x1_at(i)}));")
                 A(f"{ind}{fp} dv0 = 0, dv1 = 0, dv2 = 0;")
                 A(f"{ind}{{")
                 _emit_monomials(A, ind + "  ", fp, _with_prefixes(rests), [f"{S}_v0", f"{S}_v1", f"{S}_v2"])
@@ -789,8 +804,8 @@ def emit_backward(st: ChannelwiseStructure, T: str, waves_per_eu: int, prefetch:
 # ---------------------------------------------------------------------------------------------
 FWD_PARAMS = ("const TI* __restrict__ w, const TI* __restrict__ x1, const TI* __restrict__ x2, TI* __restrict__ out, "
               "const void* __restrict__ x1_index, int x1_idx64, const int64_t* __restrict__ csr_offsets, "
-              "const int64_t* __restrict__ csr_perm")
-FWD_ARGS = "w, x1, x2, out, x1_index, x1_idx64, csr_offsets, csr_perm"
+              "const int64_t* __restrict__ csr_perm, int64_t rows")
+FWD_ARGS = "w, x1, x2, out, x1_index, x1_idx64, csr_offsets, csr_perm, rows"
 BWD_ARGS = "w, x1, x2, g, dw, dx1, dx1_partial, dx2, dx2_partial, x1_index, x1_idx64, g_index, g_idx64, range, longer"
 # (dx1: sums by atomic additions, dx2_partial: partial rows - both in the arithmetic type; everything else holds TI)
 BWD_PARAMS = ("const TI* __restrict__ w, const TI* __restrict__ x1, const TI* __restrict__ x2, const TI* __restrict__ g, "
@@ -860,7 +875,7 @@ static int run_fwd(const SpecCall& c) {{
   if (out_idx && (!b[3].csr_offsets || (!b[3].csr_perm && c.batch > 0))) return CUEQ_ERR_UNSUPPORTED;
   const int64_t rows = b[3].rows;
   if (rows == 0) return CUEQ_OK;
-  const int64_t grid = rows * {nch} * kFwdSplit;
+  const int64_t grid = (out_idx ? rows : (rows + kPacked - 1) / kPacked) * {nch} * kFwdSplit;
   CUEQ_REQUIRE(grid < (int64_t(1) << 31), CUEQ_ERR_TOO_LARGE, "too many output rows for one launch");
   const TI* w = static_cast<const TI*>(b[0].data);
   const TI* x1 = static_cast<const TI*>(b[1].data);
@@ -872,7 +887,7 @@ static int run_fwd(const SpecCall& c) {{
   const dim3 g(static_cast<unsigned>(grid)), t(64 * nparts);
   const unsigned shared = nparts > 1 ? nparts * {FWD_FOLD * 64}u * sizeof({T}) : 0u;
   KernelTimer timer("{name}_fwd_{tag}", c.stream);
-#define LAUNCH_FWD(XI, WS) hipLaunchKernelGGL((fwd_kernel<XI, WS>), g, t, shared, c.stream, w, x1, x2, o, b[1].index, b[1].index_is_64, offs, perm)
+#define LAUNCH_FWD(XI, WS) hipLaunchKernelGGL((fwd_kernel<XI, WS>), g, t, shared, c.stream, w, x1, x2, o, b[1].index, b[1].index_is_64, offs, perm, rows)
   if (x1_idx && w_shared) LAUNCH_FWD(true, true);
   else if (x1_idx) LAUNCH_FWD(true, false);
   else if (w_shared) LAUNCH_FWD(false, true);

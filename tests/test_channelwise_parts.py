@@ -98,3 +98,35 @@ def test_output_segments_that_no_path_fills_are_zero(device, jit_on, degrees, ex
     assert (got[:, 5] == 0).all()
     others = [k for k in range(12) if k != 5]
     assert torch.equal(got[:, others], want.reshape(N, 12, E)[:, others])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,dtype,layout", [("c32_l2", torch.float32, cue.ir_mul), ("c32_l2", torch.float64, cue.mul_ir), ("c16_l1", torch.float32, cue.mul_ir),
+                                               ("c24_l1", torch.float64, cue.ir_mul), ("c5_l1", torch.float32, cue.mul_ir), ("c5_l1", torch.float64, cue.ir_mul)])
+def test_a_row_of_the_output_per_batch_row(device, jit_on, name, dtype, layout):
+    """Two (four) output rows a wavefront where 32 (16) lanes hold every channel: a last wavefront with some of them, rows read by index."""
+    from cuequivariance_amd import cuet
+    from oracle.naive import naive_segmented_polynomial, spec_from_polynomial
+    from tests.test_mul_ir_addressing import assert_close, to_mul_ir
+
+    ir1, ir2, filt = DESCRIPTORS[name]
+    ir1, ir2 = cue.Irreps("O3", ir1), cue.Irreps("O3", ir2)
+    m = cuet.ChannelWiseTensorProduct(ir1, ir2, filt, layout=layout, shared_weights=False)
+    into1, into3 = [(lambda x, i=i: to_mul_ir(x, i)) if layout == cue.mul_ir else (lambda x: x) for i in (ir1, m.irreps_out)]
+    for Z, indexed in ((1, False), (2, True), (3, False), (7, True), (64, False), (1001, False)):
+        g = torch.Generator().manual_seed(Z)
+        rows = 5 if indexed else Z
+        w, x1, x2, cot = (torch.randn(*s, dtype=torch.float64, generator=g).to(dtype).double()
+                          for s in ((Z, m.weight_numel), (rows, ir1.dim), (Z, ir2.dim), (Z, m.irreps_out.dim)))
+        senders = torch.randint(0, rows, (Z,), generator=g, dtype=torch.int32)
+        a = [t.clone().requires_grad_(True) for t in (w, x1, x2)]
+        ref = naive_segmented_polynomial(spec_from_polynomial(m.f._polynomial_orig), a, {1: senders} if indexed else {}, {}, {})[0]
+        ref_grads = torch.autograd.grad(ref, a, cot)
+        b = [t.to(device, dtype).requires_grad_(True) for t in (w, into1(x1), x2)]
+        full = [torch.full((Z, m.irreps_out.dim), float("nan"), device=device, dtype=dtype) for _ in range(4)]  # (the memory of the output)
+        del full
+        out = m(b[1], b[2], b[0], indices_1=senders.to(device) if indexed else None)
+        grads = torch.autograd.grad(out, b, into3(cot).to(device, dtype))
+        assert m.f.m._plan(dtype).specialised(device)
+        for what, got, want in zip(("out", "dw", "dx1", "dx2"), (out, *grads), (into3(ref), ref_grads[0], into1(ref_grads[1]), ref_grads[2])):
+            assert_close(got, want, TOL[dtype], what)
