@@ -245,8 +245,8 @@ __device__ __forceinline__ uint4 gemm_fragment(const char* tile, int base, int q
 // which quarter goes round (the first ones of a partial tile have more to do, and a wavefront's number decides its SIMD); the bound on
 // registers keeps the accumulators of four wavefronts beside their operands and four (three) blocks on a CU.  128 products of n x n,
 // bfloat16, us with all subtiles always / with EDGE, both operands by rows: 480 55.7 / 48.6, 392 (4 x 4 tiles of 128, the last 8 wide)
-// 47.3 / 43.6, 264 23.0 / 21.4; by columns 47.5 / 45.2, 39.8 / 36.3, 20.7 / 19.4; whole tiles lose 1 - 3 % with it.  float32, by
-// rows: 392 251 / 222, 320 138 / 114; by columns 231 / 220, 116 / 108, 200 37.5 / 37.1.  (Loads left
+// 47.3 / 43.6, 264 23.0 / 21.4; by columns 47.5 / 45.2, 39.8 / 36.3, 20.7 / 19.4; one partial tile, 512 products: 64 6.1 / 5.9, float32
+// 16.5 / 12.6, 32 9.5 / 6.3.  float32, by rows: 392 251 / 222, 320 138 / 114; by columns 231 / 220, 116 / 108, 200 37.5 / 37.1.  (Loads left
 // out as well, behind a condition, make every wait one for all loads: 392 47 us, 384 29 -> 38.)
 // KB: bytes of k per row and step; 128 makes every request of a contraction-contiguous operand a whole 128-byte line (with
 // 64 a line is fetched in two halves one step apart, and a 256 x 256 step turns over the whole L1 in between).
@@ -2739,10 +2739,16 @@ extern "C" int cueq_gemm(int32_t in_dtype, int32_t out_dtype, int32_t trans_a, i
     const bool big = !mixed && M % 256 == 0 && N % 256 == 0 && (M / 256) * (N / 256) * batch >= 2 * static_cast<int64_t>(device_cus());
     // (the timing label names the tile size, so a test can tell which kernel a shape ran on)
     KernelTimer timer(in_dtype == CUEQ_F32 ? (big ? "gemm_nt_f32_256" : "gemm_nt_f32") : in_dtype == CUEQ_F16 ? (big ? "gemm_nt_f16_256" : "gemm_nt_f16") : (big ? "gemm_nt_bf16_256" : "gemm_nt_bf16"), stream);
+    // EDGE where some tile is partly filled, in float32 only where one in four is or there is one column of tiles: between whole tiles what is
+    // left is the bound on registers (us without / with, float32: 16 products of 1 032 x 1 032 x 128, 21 % of tiles partial, 64.6 / 70.5, 4 of
+    // 2 056 64.6 / 67.4, 64 of 520, 36 %, 76 / 71; 153 664 x 128 x 128, A by rows and B by columns, 64 / 57, both by columns 63 / 56, both
+    // by rows 66.6 / 70.2, 131 080 64.7 / 52.8; bfloat16 2 056 21.3 / 21.5, 1 032 22.5 / 22.3, 153 664 x 128 x 256 27.1 / 24.8)
+    const int64_t whole = (M / kTile) * (N / kTile), all = static_cast<int64_t>(grid.x) * grid.y;
+    const bool edge = whole < all && (in_dtype != CUEQ_F32 || grid.x == 1 || 4 * (all - whole) >= all);
     const dim3 grid_big(static_cast<unsigned>(N / 256), static_cast<unsigned>(M / 256), static_cast<unsigned>(batch));
 #define GEMM_ARGS(TI, TO) static_cast<const TI*>(A), lda, stride_a, static_cast<const TI*>(B), ldb, stride_b, static_cast<TO*>(C), ldc, stride_c, m, n, k, al, accumulate, vec_out, 0, 1, 0, 0, 0, nullptr, 0, 0, 0, 0
 #define GEMM_LAUNCH(TI, TO, TA, TB) hipLaunchKernelGGL((gemm_kernel<TI, TO, TA, TB>), grid, dim3(256), 0, stream, GEMM_ARGS(TI, TO))
-#define GEMM_SZ(TI, TA, TB) do { if (big) hipLaunchKernelGGL((gemm_kernel<TI, TI, TA, TB, 4, 4, (sizeof(TI) == 2 ? 128 : 64)>), grid_big, dim3(1024), 0, stream, GEMM_ARGS(TI, TI)); else if ((M % kTile || N % kTile) && (M > kTile || N > kTile)) hipLaunchKernelGGL((gemm_kernel<TI, TI, TA, TB, 2, 2, 64, true>), grid, dim3(256), 0, stream, GEMM_ARGS(TI, TI)); else GEMM_LAUNCH(TI, TI, TA, TB); } while (0)
+#define GEMM_SZ(TI, TA, TB) do { if (big) hipLaunchKernelGGL((gemm_kernel<TI, TI, TA, TB, 4, 4, (sizeof(TI) == 2 ? 128 : 64)>), grid_big, dim3(1024), 0, stream, GEMM_ARGS(TI, TI)); else if (edge) hipLaunchKernelGGL((gemm_kernel<TI, TI, TA, TB, 2, 2, 64, true>), grid, dim3(256), 0, stream, GEMM_ARGS(TI, TI)); else GEMM_LAUNCH(TI, TI, TA, TB); } while (0)
 #define GEMM_TR(TI) do { if (trans_a && trans_b) GEMM_SZ(TI, true, true); else if (trans_a) GEMM_SZ(TI, true, false); else if (trans_b) GEMM_SZ(TI, false, true); else GEMM_SZ(TI, false, false); } while (0)
     if (in_dtype == CUEQ_F32 && out_dtype == CUEQ_F32) GEMM_TR(float);
     else if (in_dtype == CUEQ_F32 && out_dtype == CUEQ_F16) GEMM_LAUNCH(float, f16bits, false, false);
