@@ -483,10 +483,10 @@ def emit_forward(st: ChannelwiseStructure, T: str, nsplit: int, waves_per_eu: in
     A(f"  {fp}* s_fold = reinterpret_cast<{fp}*>(fwd_shared);")
     A(f"  __shared__ {fp} s_c[{max(1, len(all_tables)) * 16}];")
     A("  const int lane = threadIdx.x & 63, nparts = blockDim.x >> 6, part = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);")
-    A(f"  for (int i = threadIdx.x; i < {len(all_tables) * 16}; i += blockDim.x) s_c[i] = fwd_ctab[i];")
+    A(f"  table_to_lds<{len(all_tables) * 16}>(fwd_ctab, s_c);")
     if st.harmonics:
         A(f"  __shared__ {fp} s_sh[{npad * NM}];")
-        A(f"  for (int i = threadIdx.x; i < {npad * NM}; i += blockDim.x) s_sh[i] = fwd_shtab[i];")
+        A(f"  table_to_lds<{npad * NM}>(fwd_shtab, s_sh);")
     else:
         A(f"  const {fp}* s_sh = nullptr;")
     A("  __syncthreads();")

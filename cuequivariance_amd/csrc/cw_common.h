@@ -246,6 +246,22 @@ inline int device_cus() {
 // Number of resident wavefront slots to fill: compute units x 4 SIMDs x waves per SIMD.
 inline int64_t wave_slots(int waves_per_simd) { return static_cast<int64_t>(device_cus()) * 4 * waves_per_simd; }
 
+// A table of N values into LDS by a block of one or more wavefronts.  All loads of a block of one are in flight together (one after the
+// other, 8 of them were 4 us of a kernel of 60); past the end the last value again.
+template <int N, typename T>
+__device__ __forceinline__ void table_to_lds(const T* __restrict__ from, T* to) {
+  if (blockDim.x == 64) {
+    constexpr int K = (N + 63) / 64;
+    T v[K > 0 ? K : 1];
+#pragma unroll
+    for (int k = 0; k < K; ++k) v[k] = from[min(static_cast<int>(threadIdx.x) + 64 * k, N - 1)];
+#pragma unroll
+    for (int k = 0; k < K; ++k) to[min(static_cast<int>(threadIdx.x) + 64 * k, N - 1)] = v[k];
+  } else {
+    for (int i = threadIdx.x; i < N; i += blockDim.x) to[i] = from[i];
+  }
+}
+
 // sum of N values `stride` elements apart, first to last
 template <int N, typename T>
 __device__ __forceinline__ T fold_sum(const T* p, int stride) {
