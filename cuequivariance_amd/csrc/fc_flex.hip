@@ -1156,17 +1156,28 @@ extern "C" int cueq_fc_flex(int32_t dtype, int32_t gradient, int32_t mul_ir, int
                CUEQ_ERR_UNSUPPORTED, "fc_flex: rows must be 16-byte aligned");
   const int64_t row_tiles = (rows + 31) / 32;
   const bool held = packed && packed <= 4 && most_components <= 3;  // (source blocks in registers, channel by channel)
-  // Few tiles: eight (four) wavefronts share one.  A tile is one serial chain over the paths and channels, 150 us for float and 16
-  // channels, and four times fewer rows took no less.  us for one / shared, forward + backward, 1 000, 4 000 and 8 000 rows of
-  // 0e+1o blocks: 64 ch (x) 16 float 463 / 133, 547 / 287, 661 / 542 (1 000 tiles); 64 (x) 4 float 129 / 59, 158 / 100, 186 / 180;
-  // 64 (x) 16 bfloat16 113 / 74, 121 / 90, 138 / 136; 64 (x) 4 bfloat16 56 / 54, 70 / 65, 77 / 92.
+  // Few tiles: eight (four) wavefronts share one, each with some of its parts (held: of the channels).  A tile is one serial chain over the
+  // paths and channels, 150 us for float and 16 channels, and four times fewer rows took no less.  Shared, a CU takes one tile at a time:
+  // how many rounds of that a chain is worth goes with its parts, and one part cannot be shared.  us for one / shared, 64 channels, forward +
+  // input gradients unless said otherwise, by parts of a block and tiles a CU:
+  //   0e+1o blocks, float: (x) 0e, 1 part, forward 1 10.7 / 12.2; 0e+1o, 2, forward 1 13.5 / 12.1, 2 14.4 / 20.6; l <= 2, 2.5, forward 1
+  //   19.9 / 13.4, 1.5 19.7 / 22.1; 2 channels, 4, 2 55 / 50, 3 57 / 69; 4 channels, 8, 3 103 / 84, 4 102 / 109; 8 channels, 16, 6 275 / 246, 8
+  //   293 / 321 (32 (x) 8 6 180 / 179); 16 channels, 32, 6 540 / 435, 8 575 / 575
+  //   0e+1o+2e blocks (a SIMD holds fewer tiles): (x) 0e, 1, 0.75 36 / 38; 0e+1o, 2.3, 0.75 56 / 41, 1.5 57 / 71; l <= 2, 3.7, 1.5 93 / 81, 3 103 / 123,
+  //   bfloat16 66 / 62, 3 68 / 94; l <= 3, 4.3, 2.2 118 / 112, 3 124 / 138; 2 channels l <= 2, 7.3, 3 186 / 150, 12 472 / 462, 18 651 / 674; 4
+  //   channels, 15, 12 925 / 719, bfloat16 575 / 487
+  //   held: 2 channels 2 37 / 35, 3 42 / 56; 16 channels 4 138 / 136; 4 channels 2 43 / 43, 3 47 / 70
   const int64_t tiles = row_tiles * column_tiles;
-  const int share = held ? (tiles <= 2 * device_cus() ? 4 : 1) : tiles <= 3 * device_cus() && n2 <= 64 ? 8 : 1;  // (n2: 100 KB of LDS)
+  const int said = mul_ir >> 1;
+  mul_ir &= 1;
+  const int rounds = held ? 2 : said == 0 ? 3 : said < 2 ? 0 : most_components > 3 ? (said < 3 ? 1 : said < 6 ? 2 : 12) : said < 4 ? 1 : said < 8 ? 2 : said < 16 ? 3 : 6;
+  const int share = tiles > static_cast<int64_t>(rounds) * device_cus() ? 1 : held ? 4 : n2 <= 64 ? 8 : 1;  // (n2: 100 KB of LDS)
   const int64_t grid = share > 1 ? row_tiles * column_tiles : packed ? (row_tiles + 3) / 4 * column_tiles : (row_tiles * column_tiles + 3) / 4;
   CUEQ_REQUIRE(grid < (1ll << 31), CUEQ_ERR_TOO_LARGE, "fc_flex: too many rows");
   const size_t lds = (dX2 ? std::max(4, share) * 32 * (n2 | 1) * sizeof(float) : 0) +
                      (held ? 16 * 1024 + 4 * 32 * fc_x2_words(n2) * sizeof(uint32_t) : share > 1 ? share * 16 * 64 * sizeof(float) : 0);
-  KernelTimer timer(gradient ? "fc_flex_dx" : "fc_flex_fwd", stream);
+  // (the timing label says whether tiles are shared, so a test can tell which kernel a shape ran on)
+  KernelTimer timer(gradient ? (share > 1 ? "fc_flex_dx_shared" : "fc_flex_dx") : share > 1 ? "fc_flex_fwd_shared" : "fc_flex_fwd", stream);
 #define FC_GD(TI, WM, MI, DX, MD, KT)                                                                                                            \
   do {                                                                                                                                         \
     if (share > 1) FC_GE(TI, WM, MI, DX, MD, KT, (KT > 0 ? 4 : 8));                                                                            \

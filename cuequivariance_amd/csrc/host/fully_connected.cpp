@@ -75,6 +75,9 @@ at::Tensor weights_for(FcOp& op, const at::Tensor& w, bool packed, bool gradient
   return out;
 }
 
+// cueq_fc_flex's word on the rows and on the tables
+int rows_layout(const FcOp& op, const DeviceTables& t) { return (op.mul_ir ? 1 : 0) + 2 * (t.count(FcOp::kParts, 56) / t.count(FcOp::kBlocks, 24)); }
+
 at::Tensor product(FcOp& op, const at::Tensor& w_, const at::Tensor& x1_, const at::Tensor& x2_, at::ScalarType dtype) {
   const at::Device device = x1_.device();
   const c10::DeviceGuard guard(device);
@@ -95,7 +98,7 @@ at::Tensor product(FcOp& op, const at::Tensor& w_, const at::Tensor& x1_, const 
   const bool packed = op.packed.any() && dtype != at::kFloat;
   const at::Tensor ww = weights_for(op, w, packed, false, code, stream);
   DeviceTables& t = packed ? op.packed.fwd : op.fwd;
-  check(lib().cueq_fc_flex(code, 0, op.mul_ir, packed ? op.packed.fwd_longest : 0, Z, x1.data_ptr(), op.width1, ww.data_ptr(), x2.data_ptr(), op.n2, nullptr, 0, out.data_ptr(), op.width_out,
+  check(lib().cueq_fc_flex(code, 0, rows_layout(op, t), packed ? op.packed.fwd_longest : 0, Z, x1.data_ptr(), op.width1, ww.data_ptr(), x2.data_ptr(), op.n2, nullptr, 0, out.data_ptr(), op.width_out,
                            t.on(device, FcOp::kBlocks), t.count(FcOp::kBlocks, 24), t.on(device, FcOp::kParts), t.on<float>(device, packed ? int(Packed::kCoef) : int(FcOp::kCoef)),
                            op.fwd_tiles, op.most, static_cast<int>(op.n2), nullptr, nullptr, stream),
         "cueq_fc_flex");
@@ -153,7 +156,7 @@ Grads gradients(FcOp& op, const at::Tensor& w_, const at::Tensor& x1_, const at:
       const bool packed = op.packed.any() && dtype != at::kFloat;
       const at::Tensor ww = weights_for(op, w, packed, true, code, stream);
       DeviceTables& t = packed ? op.packed.back : op.back;
-      check(lib().cueq_fc_flex(code, 1, op.mul_ir, packed ? op.packed.dx_longest : 0, Z, g.data_ptr(), op.width_out, ww.data_ptr(), second.data_ptr(), op.n2, need_2 ? x1.data_ptr() : nullptr,
+      check(lib().cueq_fc_flex(code, 1, rows_layout(op, t), packed ? op.packed.dx_longest : 0, Z, g.data_ptr(), op.width_out, ww.data_ptr(), second.data_ptr(), op.n2, need_2 ? x1.data_ptr() : nullptr,
                                need_2 ? op.width1 : 0, dx1.data_ptr(), op.width1, t.on(device, FcOp::kBlocks), t.count(FcOp::kBlocks, 24),
                                t.on(device, FcOp::kParts), t.on<float>(device, packed ? int(Packed::kCoef) : int(FcOp::kCoef)), op.dx_tiles, op.most, static_cast<int>(op.n2),
                                need_2 ? part.data_ptr<float>() : nullptr, need_2 ? r.x2.data_ptr() : nullptr, stream),

@@ -490,7 +490,8 @@ int cueq_normalize3(int32_t dtype, int32_t stage, int64_t rows, const void* x, c
  * 1: rows of the cotangent against the weights read transposed - with X1, partial (column_tiles x rows x n2 floats) and dX2
  * given also the gradient of x2 from the same products.  `blocks`, `parts`, `grads` are device tables (FcBlock, FcPart, FcGrad of
  * csrc/fc_flex.hip), `coef` the path coefficients; multiplicities multiples of 8 (float32) / 16, components 1, 3 or 5; blocks of x2
- * of any multiplicity, n2 <= 128.  packed (2-byte elements): W as cueq_fc_pack lays it, `packed` the steps
+ * of any multiplicity, n2 <= 128.  mul_ir: 1 for rows in mul_ir, plus - it chooses kernels - twice the parts a block has on average
+ * (rounded down; 0: not said).  packed (2-byte elements): W as cueq_fc_pack lays it, `packed` the steps
  * of 16 contracted values of every fragment group (2 or 4, zeros past the block), or 5: as many as the block has. */
 int cueq_fc_flex(int32_t dtype, int32_t gradient, int32_t mul_ir, int32_t packed, int64_t rows, const void* A, int64_t lda, const void* W,
                  const void* X2, int64_t ldx2, const void* X1, int64_t ldx1, void* C, int64_t ldc, const void* blocks,

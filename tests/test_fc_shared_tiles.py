@@ -53,3 +53,20 @@ def test_values_and_gradients(device, layout, i1, i2, rows, dtype, infinite):
         tol = {torch.float32: 1e-5, torch.bfloat16: 2e-2, torch.float16: 4e-3}[dtype]
         if keep.any():
             assert (a[keep] - b[keep]).abs().max().item() <= tol * b[keep].abs().max().item(), name
+
+
+# as many tiles as are shared, and one row more: no sharing of single parts, otherwise 1, 2 and 6 tiles a CU by 2, 6 and 32 parts of a block;
+# with blocks of five components 2 and 12 by 3 and 7 (256 CUs; two or three column tiles a row tile)
+@pytest.mark.parametrize("i1,i2,rows,most", [
+    ("32x0e+32x1o", "0e", 31, 0), ("32x0e+32x1o", "0e+1o", 4_097, 4_096), ("32x0e+32x1o", "3x0e+3x1o", 8_193, 8_192),
+    ("32x0e+32x1o", "16x0e+16x1o", 24_577, 24_576), ("32x0e+32x1o+32x2e", "0e+1o+2e", 5_441, 5_440), ("32x0e+32x1o+32x2e", "2x0e+2x1o+2x2e", 32_769, 32_768)])
+def test_which_tiles_are_shared(device, i1, i2, rows, most):
+    from cuequivariance_amd import _lib
+
+    for n in (rows, most) if most else (rows,):
+        _lib.timing_begin()
+        try:
+            test_values_and_gradients(device, cue.ir_mul, i1, i2, n, torch.float32, False)
+        finally:
+            labels = {k for k in _lib.timing_end() if k.startswith(("fc_flex_fwd", "fc_flex_dx"))}
+        assert labels == ({"fc_flex_fwd_shared", "fc_flex_dx_shared"} if n <= most else {"fc_flex_fwd", "fc_flex_dx"}), (n, labels)
