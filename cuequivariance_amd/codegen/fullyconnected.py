@@ -23,6 +23,9 @@ from collections import OrderedDict
 
 MAX_WIDTH = 256   # output / input columns held in accumulators (8 tiles of 32)
 MAX_LDS = 150 * 1024
+# 16-byte vectors of a four-byte mul_ir block that a lane holds at a time.  50 000 rows of 64x0e+64x1o (x) 0e+1o+2e -> the same, float,
+# mul_ir rows, us whole / in pieces: forward 71 (96 registers spilled) / 64 (7), both input gradients 93 (101) / 70 (none).
+PIECE = 12
 
 
 def supported(paths, n2: int, width_in: int, width_out: int, es: int) -> bool:
@@ -183,8 +186,8 @@ def _emit_staging(A, T: str, blocks, lds_off, transposed: bool, threads: int):
 
 
 def _operand_groups(A, prods, transposed: bool, in_blocks, es: int, single: bool = False):
-    """Declares the operand registers of a kernel and returns ``(groups, contraction, request, fragment)``: the products
-    grouped by the segment of the row operand ``IN`` they contract with, ``request(gi)`` emits the loads of group ``gi``
+    """Declares the operand registers of a kernel and returns ``(groups, request, fragment)``: the products
+    grouped by the segment of the row operand ``IN`` they contract with (in pieces of its channels), ``request(gi)`` emits the loads of group ``gi``
     (into one of two register sets, so that a group can be requested while the previous one is worked on) and
     ``fragment(gi, comp, s2, q)`` is the expression of one 16-byte MFMA operand.  ``single``: one register set only - a
     group is requested when the last product of the previous one has read its operands."""
@@ -207,38 +210,52 @@ def _operand_groups(A, prods, transposed: bool, in_blocks, es: int, single: bool
             groups[-1][1].append((in_off, pl, blk[3]))
         else:
             groups.append((blk, [(in_off, pl, blk[3] if blk else 0)]))
-    def nraw(g):  # 16-byte vectors a lane holds for the group
-        blk, members = g
-        C = contraction[members[0][0]]
-        return (C * es // 64) * 2 * (blk[2] if blk else 1)
+    # Pieces of a group: (block, members, first slice, end), a slice being 64 / es channels.  Four-byte rows of a mul_ir block are
+    # requested in pieces of at most PIECE vectors, each contracted on its own: the run of all channels with all components (96
+    # registers for 64 channels of three components) does not fit beside 128 accumulators.  Pieces of one block stand apart in the
+    # order where there is another group to work on, so that each is requested under the products of that one.
+    whole, parts = [], []
+    for blk, members in groups:
+        ns, per = contraction[members[0][0]] * es // 64, 2 * (blk[2] if blk else 1)
+        step = max(1, PIECE // per) if blk and es == 4 else ns
+        pieces = [(blk, members, s, min(ns, s + step)) for s in range(0, ns, step)]
+        (whole if len(pieces) == 1 else parts).extend(pieces)
+    order = []
+    while whole or parts:
+        order += parts[:1] + whole[:1]
+        whole, parts = whole[1:], parts[1:]
+    groups = order
+
+    def nraw(g):  # 16-byte vectors a lane holds for the piece
+        blk, members, lo, hi = g
+        return (hi - lo) * 2 * (blk[2] if blk else 1)
     if single:
         A(f"    uint4 rawa[{max(nraw(g) for g in groups)}];")
     else:
         A(f"    uint4 rawa[{max(nraw(g) for g in groups[0::2])}], rawb[{max([nraw(g) for g in groups[1::2]] or [1])}];")
 
     def request(gi):
-        blk, members = groups[gi]
-        C = contraction[members[0][0]]
+        blk, members, lo, hi = groups[gi]
         name = "rawa" if (gi % 2 == 0 or single) else "rawb"
         if blk is None:
             in_off = members[0][0]
-            for s2 in range(C * es // 64):
+            for s2 in range(lo, hi):
                 for q in range(2):
-                    A(f"    {name}[{2 * s2 + q}] = *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(IN + z * ldi + {in_off}) + {s2 * 64} + h * 32 + {q * 16});")
+                    A(f"    {name}[{2 * (s2 - lo) + q}] = *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(IN + z * ldi + {in_off}) + {s2 * 64} + h * 32 + {q * 16});")
         else:
             s0, mul, d, _ = blk
-            for s2 in range(C * es // 64):
+            for s2 in range(lo, hi):
                 for m in range(2 * d):
-                    A(f"    {name}[{2 * d * s2 + m}] = *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(IN + z * ldi + {s0}) + ({s2 * 64} + h * 32) * {d} + {16 * m});")
+                    A(f"    {name}[{2 * d * (s2 - lo) + m}] = *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(IN + z * ldi + {s0}) + ({s2 * 64} + h * 32) * {d} + {16 * m});")
 
     def fragment(gi, comp, s2, q):
-        """Expression of the MFMA operand (s2, q) of component ``comp`` of group ``gi``: 16 bytes of consecutive channels."""
-        blk, members = groups[gi]
+        """Expression of the MFMA operand (s2, q) of component ``comp`` of piece ``gi``: 16 bytes of consecutive channels."""
+        blk, members, lo, _ = groups[gi]
         name = "rawa" if (gi % 2 == 0 or single) else "rawb"
         if blk is None:
-            return f"{name}[{2 * s2 + q}]"
+            return f"{name}[{2 * (s2 - lo) + q}]"
         d = blk[2]
-        word = lambda e: f"{name}[{2 * d * s2 + (e // (4 if es == 4 else 8))}].{'xyzw'[(e // (1 if es == 4 else 2)) % 4]}"
+        word = lambda e: f"{name}[{2 * d * (s2 - lo) + (e // (4 if es == 4 else 8))}].{'xyzw'[(e // (1 if es == 4 else 2)) % 4]}"
         if es == 4:  # elements (4 q + e) * d + comp of the run, e < 4
             return "make_uint4(" + ", ".join(word((4 * q + e) * d + comp) for e in range(4)) + ")"
         parts = []
@@ -249,7 +266,7 @@ def _operand_groups(A, prods, transposed: bool, in_blocks, es: int, single: bool
             parts.append(f"__builtin_amdgcn_perm({word(e1)}, {word(e0)}, 0x{sel:08x}u)")
         return "make_uint4(" + ", ".join(parts) + ")"
 
-    return groups, contraction, request, fragment
+    return groups, request, fragment
 
 
 def _emit_kernel(A, name: str, T: str, paths, transposed: bool, rowdot: bool, width_res: int, n2: int, in_blocks=None, res_blocks=None):
@@ -319,16 +336,15 @@ def _emit_kernel(A, name: str, T: str, paths, transposed: bool, rowdot: bool, wi
     else:
         for t in range(ntiles):
             A(f"    floatx16 o{t} = floatx16{{0}};")
-    groups, contraction, request, fragment = _operand_groups(A, prods, transposed, in_blocks, es)
+    groups, request, fragment = _operand_groups(A, prods, transposed, in_blocks, es)
     request(0)
-    for gi, (blk, members) in enumerate(groups):
+    for gi, (blk, members, lo, hi) in enumerate(groups):
         # the operands of the next group are requested before the products of the current one are worked on
         if gi + 1 < len(groups):
             request(gi + 1)
         for in_off, plist, comp in members:
-            ns = contraction[in_off] * es // 64
             A("    {")
-            for s2 in range(ns):
+            for s2 in range(lo, hi):
                 for q in range(2):
                     A(f"      const uint4 xf_{s2}_{q} = {fragment(gi, comp, s2, q)};")
             for w_off, K, N, uses in plist:
@@ -337,7 +353,7 @@ def _emit_kernel(A, name: str, T: str, paths, transposed: bool, rowdot: bool, wi
                     A("      {")
                     A("        floatx16 T = floatx16{0};")
                     A(f"        const char* wr = smem + {o} + ({32 * t} + c) * {RS} + h * 32;")
-                    for s2 in range(ns):
+                    for s2 in range(lo, hi):
                         for q in range(2):
                             A(f"        mma_step<{T}>(T, *reinterpret_cast<const uint4*>(wr + {s2 * 64 + q * 16}), xf_{s2}_{q});")
                     for j, coeff, res_off in uses:
@@ -352,7 +368,8 @@ def _emit_kernel(A, name: str, T: str, paths, transposed: bool, rowdot: bool, wi
                         else:
                             A(f"        {{ const float sc = {coeff!r}f * s{j};")
                             A("#pragma unroll")
-                            A(f"          for (int v = 0; v < 16; ++v) o{res_off // 32 + t}[v] = fmaf(sc, T[v], o{res_off // 32 + t}[v]); }}")
+                            A(f"          for (int v = 0; v < 16; ++v) o{res_off // 32 + t}[v] = fmaf(sc, T[v], o{res_off // 32 + t}[v]);")
+                            A(f'          asm volatile("" : "+v"(o{res_off // 32 + t})); }}')
                     A("      }")
                     A("      __builtin_amdgcn_sched_barrier(0);  // keep the loads of later products from piling up ahead of this one")
             A("    }")
@@ -475,16 +492,17 @@ def _emit_dx12_kernel(A, T: str, paths, width_in: int, n2: int, g_blocks=None, x
                     for r in range(4):
                         A(f"      x_{s0 + kc * mul}_{tl}[{4 * a + r}] = gv[{r * d + kc}];")
                 A("    }")
+    # Every accumulator is written where its use stands ("+v" below): left to itself the compiler collects the uses of several products
+    # and keeps their results (52 registers spilled on ir_mul rows, 78 us; none, 67 us).
     # one set of operand registers (two do not fit beside the accumulators and the row of x1, and made no difference when
     # timed): the next group is requested as soon as the last product of the current one has issued its matrix
     # instructions, ahead of that product's uses
-    groups, contraction, request, fragment = _operand_groups(A, prods, False, g_blocks, es, single=True)
+    groups, request, fragment = _operand_groups(A, prods, False, g_blocks, es, single=True)
     request(0)
-    for gi, (blk, members) in enumerate(groups):
+    for gi, (blk, members, lo, hi) in enumerate(groups):
         for mi, (in_off, plist, comp) in enumerate(members):
-            ns = contraction[in_off] * es // 64
             A("    {")
-            for s2 in range(ns):
+            for s2 in range(lo, hi):
                 for q in range(2):
                     A(f"      const uint4 xf_{s2}_{q} = {fragment(gi, comp, s2, q)};")
             for pi, (w_off, K, N, uses) in enumerate(plist):
@@ -494,7 +512,7 @@ def _emit_dx12_kernel(A, T: str, paths, width_in: int, n2: int, g_blocks=None, x
                     A("      {")
                     A("        floatx16 T = floatx16{0};")
                     A(f"        const char* wr = smem + {o} + (32 * (hlf * {KH} + {tl}) + c) * {RS} + h * 32;")
-                    for s2 in range(ns):
+                    for s2 in range(lo, hi):
                         for q in range(2):
                             A(f"        mma_step<{T}>(T, *reinterpret_cast<const uint4*>(wr + {s2 * 64 + q * 16}), xf_{s2}_{q});")
                     if gi + 1 < len(groups) and mi == len(members) - 1 and pi == len(plist) - 1 and tl == KH - 1:
@@ -504,6 +522,7 @@ def _emit_dx12_kernel(A, T: str, paths, width_in: int, n2: int, g_blocks=None, x
                         A(f"        {{ const float sc = {coeff!r}f * s{j};")
                         A("#pragma unroll")
                         A(f"          for (int v = 0; v < 16; ++v) o_{a_off}_{tl}[v] = fmaf(sc, T[v], o_{a_off}_{tl}[v]);")
+                        A(f'          asm volatile("" : "+v"(o_{a_off}_{tl}));')
                         A("          float p = 0.f;")
                         A("#pragma unroll")
                         A(f"          for (int v = 0; v < 16; ++v) p = fmaf(T[v], x_{a_off}_{tl}[v], p);")

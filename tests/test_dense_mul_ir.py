@@ -182,3 +182,42 @@ def test_fully_connected_mul_ir_matches_oracle_without_transposition(device, ker
     assert rel_err(gx1, to_mul_ir(ref_gx1, i1)) <= tol
     assert rel_err(gx2, ref_gx2) <= tol
     assert rel_err(gw, ref_gw) <= tol
+
+
+@pytest.mark.parametrize("Z", [1, 33, 4129])
+@pytest.mark.parametrize(
+    "irreps_in1,irreps_in2,irreps_out",
+    [
+        ("64x0e+64x1o", "0e+1o+2e", "64x0e+64x1o"),  # pieces of one block around the other block
+        ("64x1o", "0e+1o+2e", "64x1o"),  # pieces of one block next to each other
+        ("32x0e+32x2e", "0e+2e", "64x0e+32x2e"),  # pieces of one slice of channels
+    ],
+)
+def test_fully_connected_mul_ir_pieces(device, kernels_at_first_use, irreps_in1, irreps_in2, irreps_out, Z):
+    """The generated float kernels read a block of several components in pieces of its channels; called directly, as the operator
+    takes other kernels for short batches.  Sums of up to 64 channels and a few paths in float32: 1e-5 of the largest value."""
+    i1, i2, i3 = (cue.Irreps("O3", s) for s in (irreps_in1, irreps_in2, irreps_out))
+    m = cuet.FullyConnectedTensorProduct(i1, i2, i3, layout=cue.mul_ir, internal_weights=False)
+    dense = next(x for x in m.modules() if type(x).__name__ == "SegmentedPolynomialDense" and x.rows_mul_ir)
+    g = torch.Generator().manual_seed(Z)
+    w, x1, x2, cot = (torch.randn(*s, generator=g) for s in ((1, m.weight_numel), (Z, i1.dim), (Z, i2.dim), (Z, i3.dim)))
+    a = [t.double().requires_grad_(True) for t in (w, to_ir_mul(x1, i1), x2)]
+    ref = naive_segmented_polynomial(spec_from_polynomial(m.f._polynomial_orig), a)[0]
+    ref_1, ref_2 = torch.autograd.grad(ref, a[1:], to_ir_mul(cot, i3).double())
+    wd, x1d, x2d, gd = (t.to(device) for t in (w, x1, x2, cot))
+    unit = dense.fused_unit(torch.float32, x1d, gd)
+    assert unit is not None
+    empty = lambda like: torch.full_like(like, float("nan"))
+    out, d1, d2, both1, both2 = empty(gd), empty(x1d), empty(x2d), empty(x1d), empty(x2d)
+    part = torch.empty(Z, 2 * i2.dim, device=device)
+    stream = torch.cuda.current_stream().cuda_stream
+    row = lambda t: (t.data_ptr(), t.stride(0))
+    assert unit.fcj_fwd(Z, wd.data_ptr(), *row(x1d), *row(x2d), *row(out), stream) == 0
+    assert unit.fcj_dx1(Z, wd.data_ptr(), *row(gd), *row(x2d), *row(d1), stream) == 0
+    assert unit.fcj_dx2(Z, wd.data_ptr(), *row(x1d), *row(x2d), *row(gd), *row(d2), stream) == 0
+    status = unit.fcj_dx12(Z, wd.data_ptr(), *row(gd), *row(x2d), *row(x1d), *row(both1), *row(both2), part.data_ptr(), stream)
+    assert status == (0 if all(mul % 64 == 0 for mul, _ in i1) else -2)
+    assert rel_err(out, to_mul_ir(ref, i3)) <= 1e-5
+    assert rel_err(d1, to_mul_ir(ref_1, i1)) <= 1e-5 and rel_err(d2, ref_2) <= 1e-5
+    if status == 0:
+        assert rel_err(both1, to_mul_ir(ref_1, i1)) <= 1e-5 and rel_err(both2, ref_2) <= 1e-5
