@@ -16,7 +16,11 @@ batch row at a time.  With ``S_p[k, u] = sum_ij C_p[i, j, k] x1[i, u] x2[j]`` (a
   per ``u`` - ``dx1[i, u] += sum_jk C_p[i, j, k] x2[j] R_p[k, u]`` and ``dx2[j] += sum_u sum_ik C_p[i, j, k] x1[i, u] R_p[k, u]``.
 
 The unit registers under the hashes of the flattened uniform-1d tables (forward, and backward for all three inputs), like
-the channel-wise units; buffers and batch modes are those of ``codegen/channelwise.py``.
+the channel-wise units; buffers and batch modes are those of ``codegen/channelwise.py``.  Rows of the first operand and of the output are
+addressed in either order (``Rows``): a lane's component of a ``mul_ir`` block lies as many elements from its neighbour's as the block has
+components, and the loads and stores of the components together cover the same whole lines.  Four transposition launches and their
+autograd functions less per step (forward and all gradients, float32: 3 001 edges of 48 channels 143 - 236 -> 90 us, nearly all of
+it host work; 12 007 edges of 64 channels 599 -> 583, forward 188 -> 178).
 """
 
 from __future__ import annotations
@@ -40,6 +44,16 @@ class Block:
     entries: List[Tuple[int, int, int, float]] = field(default_factory=list)  # (i, j, k, coefficient), non-zero
 
 
+@dataclass(frozen=True)
+class Rows:
+    """A fully connected product (``uvw,iu,jv,kw+ijk``) and whether the rows of its first operand and of its output keep the components
+    of a channel together (``mul_ir``: element (channel u, component i) of a segment at ``u d + i``; else at ``i U + u``)."""
+
+    polynomial: object
+    x1_mul_ir: bool = False
+    out_mul_ir: bool = False
+
+
 @dataclass
 class RowWeightStructure:
     U: int
@@ -49,10 +63,15 @@ class RowWeightStructure:
     width_x2: int
     width_out: int
     blocks: List[Block]
+    at_x1: List[Tuple[int, int]]   # (offset, distance between channels) of the components of a row of x1
+    at_out: List[Tuple[int, int]]  # ... and of the output
+    groups_out: Tuple[int, ...]    # the layout of the output buffer in the flattened tables
 
 
 def analyze(polynomial) -> Optional[RowWeightStructure]:
-    """The structure of ``uvw,iu,jv,kw+ijk`` with ``v = 1`` and one multiplicity per operand (at most 64), else None."""
+    """The structure of ``uvw,iu,jv,kw+ijk`` (or of its ``Rows``) with ``v = 1`` and one multiplicity per operand (at most 64), else None."""
+    rows = polynomial if isinstance(polynomial, Rows) else Rows(polynomial)
+    polynomial = rows.polynomial
     if polynomial is None or polynomial.num_inputs != 3 or polynomial.num_outputs != 1 or len(polynomial.operations) != 1:
         return None
     ope, stp = polynomial.operations[0]
@@ -95,7 +114,31 @@ def analyze(polynomial) -> Optional[RowWeightStructure]:
             blocks.append(blk)
     if not blocks:
         return None
-    return RowWeightStructure(U, Wd, nw, n1, n2, no, blocks)
+
+    def addresses(operand, offsets, mul_ir):
+        return [(off + i, d) if mul_ir else (off + i * U, 1) for off, (d, U) in zip(offsets, operand.segments) for i in range(d)]
+
+    dims = tuple(d for d, _ in oo.segments)
+    return RowWeightStructure(U, Wd, nw, n1, n2, no, blocks, addresses(o1, off1, rows.x1_mul_ir), addresses(oo, offo, rows.out_mul_ir),
+                              dims if rows.out_mul_ir and any(d > 1 for d in dims) else ())
+
+
+def flatten(rows: Rows):
+    """``(polynomial, segment groups)``: the product with every mode but the output's multiplicity flattened away, as the uniform-1d
+    kernels take it, over rows in the orders of ``rows``.  Channels of the first operand are scalar segments then: their order is that
+    of the row."""
+    q = rows.polynomial.flatten_coefficient_modes()
+    stp = q.operations[0][1]
+    keep = stp.subscripts.operands[-1][-1]
+    q = q.flatten_modes([m for m in stp.subscripts.modes() if m != keep])
+    if rows.x1_mul_ir:
+        order, off = [], 0
+        for d, U in rows.polynomial.operations[0][1].operands[1].segments:
+            order += [off + i * U + u for u in range(U) for i in range(d)]
+            off += d * U
+        q = q.apply_fn(lambda ope, stp: (ope, stp.permute_segments(1, order)))
+    dims = [d for d, _ in rows.polynomial.operations[0][1].operands[-1].segments]
+    return q, ({3: dims} if rows.out_mul_ir and any(d > 1 for d in dims) else {})
 
 
 def _lit(c: float, T: str) -> str:
@@ -116,6 +159,15 @@ def emit_unit(st: RowWeightStructure, T: str, name: str, fwd_hash: int, bwd_hash
     nx1 = st.width_x1 // U          # x1 components (each a vector over u)
     nout = st.width_out // Wd       # output components (each a vector over w)
     n2 = st.width_x2
+
+    def x1_at(i):
+        off, step = st.at_x1[i]
+        return f"{off} + lu" if step == 1 else f"{off} + lu * {step}"
+
+    def out_at(k):  # (lw is in the base address)
+        off, step = st.at_out[k]
+        return f"{off}" if step == 1 else f"{off} + lw * {step - 1}"
+
     TS = 65                         # row stride of the LDS tile in elements: column reads touch every bank once
     G = next(n for n in (32, 16, 8, 4, 2, 1) if n <= MAX_GROUP and U % n == 0)  # weight rows requested together, one group ahead of their use
     waves = 2 if T == "float" else 1
@@ -166,7 +218,7 @@ def emit_unit(st: RowWeightStructure, T: str, name: str, fwd_hash: int, bwd_hash
     A(f"    const {T}* __restrict__ x2p = x2 + z * {n2}ll;")
     A(f"    const {T}* __restrict__ wp = w + z * {st.width_w}ll + lw;")
     for i in range(nx1):
-        A(f"    const {T} xa{i} = act_u ? x1p[{i * U} + lu] : {T}(0);")
+        A(f"    const {T} xa{i} = act_u ? x1p[{x1_at(i)}] : {T}(0);")
     for j in range(n2):
         A(f"    const {T} xb{j} = x2p[{j}];")
     groups = [(b, g0) for b, blk in enumerate(st.blocks) for g0 in range(0, U, G)]
@@ -193,7 +245,8 @@ def emit_unit(st: RowWeightStructure, T: str, name: str, fwd_hash: int, bwd_hash
     A(f"  {T}* __restrict__ op = out + static_cast<int64_t>(blockIdx.x) * {st.width_out}ll + lw;  // (out = the partial rows when parts > 1)")
     A("  if (act_w) {")
     for k in range(nout):
-        A(f"    STREAM_STORE(acc{k}, op + {k * Wd});")
+        # (components that share their lines leave as ordinary stores, which meet in the cache)
+        A(f"    STREAM_STORE(acc{k}, op + {out_at(k)});" if st.at_out[k][1] == 1 else f"    op[{out_at(k)}] = acc{k};")
     A("  }")
     A("}")
     A("")
@@ -220,11 +273,11 @@ def emit_unit(st: RowWeightStructure, T: str, name: str, fwd_hash: int, bwd_hash
     A(f"    const {T}* __restrict__ wp = w + z * {st.width_w}ll + lw;")
     A(f"    {T}* __restrict__ dwp = dw + z * {st.width_w}ll + lw;")
     for i in range(nx1):
-        A(f"    const {T} xa{i} = act_u ? x1p[{i * U} + lu] : {T}(0);")
+        A(f"    const {T} xa{i} = act_u ? x1p[{x1_at(i)}] : {T}(0);")
     for j in range(n2):
         A(f"    const {T} xb{j} = x2p[{j}];")
     for k in range(nout):
-        A(f"    const {T} gv{k} = act_w ? gp[{k * Wd} + lw] : {T}(0);")
+        A(f"    const {T} gv{k} = act_w ? gp[lw + {out_at(k)}] : {T}(0);")
     for i in range(nx1):
         A(f"    {T} da{i} = 0;")
     for j in range(n2):
@@ -278,13 +331,13 @@ def emit_unit(st: RowWeightStructure, T: str, name: str, fwd_hash: int, bwd_hash
     # gradients of the row
     A("    if (act_u) {")
     A("      if (ATOMIC_DX1) {")
-    A(f"        {T}* dp = dx1 + srow * {st.width_x1}ll + lu;")
+    A(f"        {T}* dp = dx1 + srow * {st.width_x1}ll;")
     for i in range(nx1):
-        A(f"        unsafeAtomicAdd(dp + {i * U}, da{i});")
+        A(f"        unsafeAtomicAdd(dp + {x1_at(i)}, da{i});")
     A("      } else {")
-    A(f"        {T}* __restrict__ dp = dx1_partial + z * {st.width_x1}ll + lu;")
+    A(f"        {T}* __restrict__ dp = dx1_partial + z * {st.width_x1}ll;")
     for i in range(nx1):
-        A(f"        dp[{i * U}] = da{i};")
+        A(f"        dp[{x1_at(i)}] = da{i};")
     A("      }")
     A("    }")
     for j in range(n2):

@@ -22,6 +22,7 @@ from typing import Dict, List, Optional, Sequence
 import torch
 
 from .. import _lib, cue
+from ..codegen import fullyconnected_rows as fcr
 from ..cue import descriptors
 from .dense import GeneralFullyConnected, SegmentedPolynomialDense
 from .fused_tp import SegmentedPolynomialFusedTP, _FlattenedOperation, _MatrixWithElementwiseStage
@@ -405,6 +406,12 @@ class FullyConnectedTensorProduct(torch.nn.Module):
         )
         self.method = _method_from_fallback(method, use_fallback, "fused_tp")
         self.f_per_sample = _FlattenedUniform(e.polynomial, math_dtype)  # weights of shape (batch, weight_numel)
+        # the same on mul_ir rows as they lie, where kernels that stream a weight row per batch row are generated; built at first use
+        self._mul_ir_rows = None
+        if (self.transpose_in2.moves_nothing and not (self.transpose_in1.moves_nothing and self.transpose_out.moves_nothing)
+                and all(x.layout == cue.ir_mul for x in (e.inputs[1], e.outputs[0])) and fcr.analyze(e.polynomial) is not None):
+            self._mul_ir_rows = fcr.Rows(e.polynomial, self.transpose_in1.source == cue.mul_ir, self.transpose_out.target == cue.mul_ir)
+        self.per_sample_rows = None
         self.f = SegmentedPolynomial(e.polynomial, method=self.method, math_dtype=math_dtype)
         if getattr(self.f.m, "dense", True) is None and getattr(self.f.m, "composed", None) is None:
             # the matrix-core executor takes a second operand of multiplicity one directly, any other behind a stage that
@@ -463,6 +470,10 @@ class FullyConnectedTensorProduct(torch.nn.Module):
                 out = dense.fully_connected.direct(weight, x1, x2)
                 if out is not None:
                     return out
+        if getattr(self, "_mul_ir_rows", None) is not None and weight.shape[0] != 1 and not torch.compiler.is_compiling():
+            out = self._per_sample_as_they_lie(weight, x1, x2, indices_1, indices_out, size_out)
+            if out is not None:
+                return out
         if indices_1 is None and indices_out is None and self._rows_ready(x1, x2, weight):
             return self.f_rows([weight, x1, apply_layout(self.transpose_in2, x2)])[0]
         x1 = apply_layout(self.transpose_in1, x1)
@@ -478,6 +489,18 @@ class FullyConnectedTensorProduct(torch.nn.Module):
         if weight.shape[0] != 1 or self.f is None:
             return apply_layout(self.transpose_out, self.f_per_sample([weight, x1, x2])[0])
         return apply_layout(self.transpose_out, self.f([weight, x1, x2])[0])
+
+    def _per_sample_as_they_lie(self, weight, x1, x2, indices_1, indices_out, size_out):
+        """A plain call with a weight row per batch row of float32 or float64, rows in this module's layouts, in native code; ``None`` for
+        any other call (and every error), which takes the general way."""
+        if not (weight.is_cuda and weight.dtype == x1.dtype == x2.dtype and weight.dtype in (torch.float32, torch.float64)):
+            return None
+        if self.per_sample_rows is None:
+            q, groups = fcr.flatten(self._mul_ir_rows)
+            self.per_sample_rows = SegmentedPolynomial(q, method="uniform_1d", math_dtype=self.f_per_sample._math_dtype,
+                                                       options={"origin": self._mul_ir_rows, "segment_groups": groups})
+        m = _executor(self, "per_sample_rows", SegmentedPolynomialFromUniform1d)
+        return None if m is None else m.operator.product(weight, x1, x2, indices_1, None, indices_out, size_out)
 
     def _dense(self):
         """The executor of the 4-operand form for rows in this module's layouts, or ``None``."""

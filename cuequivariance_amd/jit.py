@@ -139,15 +139,15 @@ def is_symmetric_contraction(poly) -> bool:
 
 
 def is_row_weight_fully_connected(t: U1dTables, origin) -> bool:
-    """Tables flattened from a fully connected product ``origin`` (``uvw,iu,jv,kw+ijk``, second operand of multiplicity one,
-    one multiplicity per operand) - the form ``codegen/fullyconnected_rows.py`` generates kernels for when every batch row
+    """Tables flattened from a fully connected product ``origin`` (``uvw,iu,jv,kw+ijk``, or its ``fullyconnected_rows.Rows``; second operand of
+    multiplicity one, one multiplicity per operand) - the form ``codegen/fullyconnected_rows.py`` generates kernels for when every batch row
     brings its own weights."""
     from .codegen import fullyconnected_rows as fcr
 
-    if origin is None or t.layouts or t.num_inputs != 3 or t.num_outputs != 1 or tuple(t.buffer_dim) != (1, 0, 0, 1):
+    if origin is None or t.num_inputs != 3 or t.num_outputs != 1 or tuple(t.buffer_dim) != (1, 0, 0, 1):
         return False
     st = fcr.analyze(origin)
-    return (st is not None and t.operand_extent == st.Wd and
+    return (st is not None and t.operand_extent == st.Wd and [t.layout(b) for b in range(4)] == [(), (), (), st.groups_out] and
             list(t.buffer_num_segments) == [st.width_w // st.Wd, st.width_x1, st.width_x2, st.width_out // st.Wd])
 
 

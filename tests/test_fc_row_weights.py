@@ -127,3 +127,98 @@ def test_row_weights_without_batch_rows(device):
     g1, g2, gw = torch.autograd.grad(out, [x1, x2, w], torch.ones_like(out))
     assert g1.shape == x1.shape and float(g1.abs().sum()) == 0.0 and g2.shape == x2.shape and gw.shape == w.shape
     assert m.f_per_sample.f.m._plan(torch.float32).specialised(device)
+
+
+MUL_IR_ROWS = [("64x0e+64x1o", "0e+1o+2e", "64x0e+64x1o"), ("24x0e+24x1o+24x2e", "0e+1o", "40x0e+40x1o+40x2e"), ("8x1o", "0e+1o", "16x0e+16x1o")]
+
+
+@pytest.mark.parametrize("ir1,ir2,ir3", MUL_IR_ROWS[1:])
+@pytest.mark.parametrize("in_mul_ir,out_mul_ir", [(True, True), (True, False), (False, True)])
+def test_tables_of_mul_ir_rows(ir1, ir2, ir3, in_mul_ir, out_mul_ir):
+    """The flattened tables over mul_ir rows are those over ir_mul rows with every scalar of x1 and every segment of the output at the
+    place where such a row holds it."""
+    from cuequivariance_amd.codegen.registry import flattened_fully_connected_tables
+
+    e = descriptors.fully_connected_tensor_product(*(cue.Irreps("O3", s) for s in (ir1, ir2, ir3)))
+    plain, rows = flattened_tables(e.polynomial), fcr.Rows(e.polynomial, in_mul_ir, out_mul_ir)
+    t = flattened_fully_connected_tables(rows)
+    assert jit._family(t, None, rows) == "fc_rows" and jit._family(t, None, e.polynomial) == (None if out_mul_ir else "fc_rows")
+
+    def place(irreps, mul_ir):  # [(first, distance)] of the components of a row, in ir_mul order
+        out, off = [], 0
+        for mul, ir in irreps:
+            out += [(off + i, ir.dim) if mul_ir else (off + i * mul, 1) for i in range(ir.dim)]
+            off += mul * ir.dim
+        return out
+
+    U, st = e.inputs[1].irreps[0].mul, fcr.analyze(rows)
+    assert st.at_x1 == place(e.inputs[1].irreps, in_mul_ir) and st.at_out == place(e.outputs[0].irreps, out_mul_ir)
+    assert t.segment_addressing(3) == st.at_out
+    moved = [st.at_x1[c // U][0] + (c % U) * st.at_x1[c // U][1] for c in range(st.width_x1)]
+    (_, a), (_, b) = plain.operation(0), t.operation(0)
+    assert [((w, moved[x1], x2, out), c) for (w, x1, x2, out), c in a] == [(tuple(i), c) for i, c in b]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("indexed,deterministic", [(True, "0"), (True, "1"), (False, "0")])
+@pytest.mark.parametrize(
+    "ir1,ir2,ir3,layouts,dtype",
+    [(*MUL_IR_ROWS[0], ("mul_ir", "mul_ir"), torch.float32), (*MUL_IR_ROWS[0], ("mul_ir", "mul_ir"), torch.float64),
+     (*MUL_IR_ROWS[1], ("mul_ir", "ir_mul"), torch.float32), (*MUL_IR_ROWS[1], ("ir_mul", "mul_ir"), torch.float32),
+     (*MUL_IR_ROWS[2], ("mul_ir", "mul_ir"), torch.float32)],
+)
+def test_row_weights_on_mul_ir_rows(device, dtype, layouts, ir1, ir2, ir3, indexed, deterministic, jit_on, monkeypatch):
+    """Rows in mul_ir as they lie against the oracle on converted rows (float32 1e-5, float64 1e-12 of the largest value, as above), without a
+    transposition launch; a hook on the general executor takes the transposing way, with the same result."""
+    from cuequivariance_amd import _lib, cuet
+    from oracle.naive import naive_segmented_polynomial, spec_from_polynomial
+
+    monkeypatch.setenv("CUEQ_DETERMINISTIC", deterministic)
+    i1, i2, i3 = (cue.Irreps("O3", s) for s in (ir1, ir2, ir3))
+    m = cuet.FullyConnectedTensorProduct(i1, i2, i3, layout_in1=cue.IrrepsLayout.as_layout(layouts[0]), layout_in2=cue.mul_ir,
+                                         layout_out=cue.IrrepsLayout.as_layout(layouts[1]), shared_weights=False, internal_weights=False)
+    N, Z = 29, 301
+
+    def turned(x, irreps, layout):  # ir_mul rows in the given layout
+        if layout == "ir_mul":
+            return x
+        parts, off = [], 0
+        for mul, ir in irreps:
+            parts.append(x[:, off:off + mul * ir.dim].reshape(-1, ir.dim, mul).transpose(1, 2).reshape(-1, mul * ir.dim))
+            off += mul * ir.dim
+        return torch.cat(parts, 1)
+
+    g = torch.Generator().manual_seed(31)
+    x1, x2, w, cot = (torch.randn(*s, dtype=torch.float64, generator=g).to(dtype).double()
+                      for s in ((N if indexed else Z, i1.dim), (Z, i2.dim), (Z, m.weight_numel), (N if indexed else Z, i3.dim)))
+    snd, rcv = (torch.randint(0, N - 2, (Z,), generator=g, dtype=torch.int32) for _ in range(2))
+    a = [t.clone().requires_grad_(True) for t in (w, x1, x2)]
+    spec = spec_from_polynomial(descriptors.fully_connected_tensor_product(i1, i2, i3).polynomial)
+    ref = naive_segmented_polynomial(spec, a, {1: snd}, {0: N}, {0: rcv})[0] if indexed else naive_segmented_polynomial(spec, a)[0]
+    r_w, r_1, r_2 = torch.autograd.grad(ref, a, cot)
+    want = [turned(ref.detach(), i3, layouts[1]), r_w, turned(r_1, i1, layouts[0]), r_2]
+    b = [t.to(dtype).to(device).requires_grad_(True) for t in (w, turned(x1, i1, layouts[0]), x2)]
+    gd = turned(cot, i3, layouts[1]).to(dtype).to(device)
+    more = dict(indices_1=snd.to(device), indices_out=rcv.to(device), size_out=N) if indexed else {}
+
+    def step():
+        out = m(b[1], b[2], b[0], **more)
+        return (out, *torch.autograd.grad(out, b, gd))
+
+    _lib.load().cueq_timing_begin()
+    got = step()
+    torch.cuda.synchronize()
+    names = dict(_lib.timing_end())
+    assert "segmented_transpose" not in names, names
+    plan = m.per_sample_rows.m._plan(dtype)
+    assert plan.specialised(device) and plan.backward_plan((True, True, True)).specialised(device)
+    called = []
+    m.f_per_sample.register_forward_hook(lambda *_: called.append(1))
+    again = step()
+    assert called
+    tol = 1e-12 if dtype == torch.float64 else 1e-5
+    for what, p, q, r in zip(("out", "dw", "dx1", "dx2"), got, again, want):
+        assert p.shape == q.shape == r.shape
+        for t in (p, q):
+            err = (t.detach().cpu().double() - r).abs().max().item()
+            assert err <= tol * r.abs().max().item(), (what, err)
