@@ -42,7 +42,8 @@ __device__ __forceinline__ void tri_store(f16bits* p, int64_t i, float v) { p[i]
 // inside a step is free and every operand read is one or two ds_read_b128.
 // ------------------------------------------------------------------------------------------------
 constexpr int kTile = 128;
-constexpr int kRowBytes = 80;  // 64 bytes of data + 16 bytes of padding
+constexpr int kStepBytes = 64;  // of k per row and step
+constexpr int kRowBytes = kStepBytes + 16;  // padded: conflict-free 16-byte reads by 16 consecutive rows
 
 // Workgroups are handed to the 8 XCDs round-robin in launch order and every XCD has its own L2.  This maps the
 // launch-order index to a tile index so that each XCD works through one contiguous range of tiles (column tile
@@ -201,29 +202,28 @@ typedef short shortx4_t __attribute__((ext_vector_type(4)));
 // bytes between the k rows of a contraction-major tile of EXT columns: the row plus 64 (2-byte) / 128 (4-byte) bytes
 template <typename TI, int EXT>
 constexpr int trans_stride() { return EXT * static_cast<int>(sizeof(TI)) + (sizeof(TI) == 2 ? 64 : 128); }
-// LDS bytes of one operand tile of EXT rows (either layout); KB = bytes of k per row and step (64 or 128), rows of a
-// contraction-contiguous tile are KB + 16 bytes apart (conflict-free 16-byte reads by 16 consecutive rows for both)
-template <typename TI, int EXT, int KB = 64>
+// LDS bytes of one operand tile of EXT rows (either layout)
+template <typename TI, int EXT>
 constexpr int gemm_tile_bytes() {
-  constexpr int a = EXT * (KB + 16), b = (KB / static_cast<int>(sizeof(TI))) * trans_stride<TI, EXT>();
+  constexpr int a = EXT * kRowBytes, b = (kStepBytes / static_cast<int>(sizeof(TI))) * trans_stride<TI, EXT>();
   return a > b ? a : b;
 }
 
-template <typename TI, bool TR, int EXT, int KB = 64>
+template <typename TI, bool TR, int EXT>
 __device__ __forceinline__ void gemm_stage_offsets(int e, int& row, int& part) {
   constexpr int VPRN = EXT * sizeof(TI) / 16;  // vectors per k row of a contraction-major tile
   if constexpr (TR) { row = e / VPRN; part = e % VPRN; }
-  else { row = e / (KB / 16); part = e % (KB / 16); }
+  else { row = e / (kStepBytes / 16); part = e % (kStepBytes / 16); }
 }
 
-// fragment of subtile rows [base, base + 32) for MFMA slice q of the step (KB / 32 slices): 16 bytes of k per lane
-template <typename TI, bool TR, int EXT, int KB = 64>
+// fragment of subtile rows [base, base + 32) for MFMA slice q of the step (two slices): 16 bytes of k per lane
+template <typename TI, bool TR, int EXT>
 __device__ __forceinline__ uint4 gemm_fragment(const char* tile, int base, int q, int lane) {
   constexpr int kTransStride16 = trans_stride<uint16_t, EXT>(), kTransStride32 = trans_stride<float, EXT>();
-  constexpr int HK = KB / 2 / static_cast<int>(sizeof(TI));  // k rows of a contraction-major tile per half wavefront
+  constexpr int HK = kStepBytes / 2 / static_cast<int>(sizeof(TI));  // k rows of a contraction-major tile per half wavefront
   const int c = lane & 31, h = lane >> 5;
   if constexpr (!TR) {
-    return *reinterpret_cast<const uint4*>(tile + (base + c) * (KB + 16) + h * (KB / 2) + q * 16);
+    return *reinterpret_cast<const uint4*>(tile + (base + c) * kRowBytes + h * (kStepBytes / 2) + q * 16);
   } else if constexpr (sizeof(TI) == 2) {
     const int s = lane & 15, g16 = (lane >> 4) & 1;
     const char* p = tile + (HK * h + 8 * q + (s >> 2)) * kTransStride16 + (base + 16 * g16 + 4 * (s & 3)) * 2;  // k as in the other layout
@@ -243,15 +243,13 @@ __device__ __forceinline__ uint4 gemm_fragment(const char* tile, int base, int q
 // the operand traffic between L2 and the CUs for products whose both extents are large.
 // EDGE: some tiles are partly filled.  A wavefront forms only those of its four subtiles that reach into C, and which wavefront has
 // which quarter goes round (the first ones of a partial tile have more to do, and a wavefront's number decides its SIMD); the bound on
-// registers keeps the accumulators of four wavefronts beside their operands and four (three) blocks on a CU.  128 products of n x n,
-// bfloat16, us with all subtiles always / with EDGE, both operands by rows: 480 55.7 / 48.6, 392 (4 x 4 tiles of 128, the last 8 wide)
-// 47.3 / 43.6, 264 23.0 / 21.4; by columns 47.5 / 45.2, 39.8 / 36.3, 20.7 / 19.4; one partial tile, 512 products: 64 6.1 / 5.9, float32
-// 16.5 / 12.6, 32 9.5 / 6.3.  float32, by rows: 392 251 / 222, 320 138 / 114; by columns 231 / 220, 116 / 108, 200 37.5 / 37.1.  (Loads left
-// out as well, behind a condition, make every wait one for all loads: 392 47 us, 384 29 -> 38.)
-// KB: bytes of k per row and step; 128 makes every request of a contraction-contiguous operand a whole 128-byte line (with
-// 64 a line is fetched in two halves one step apart, and a 256 x 256 step turns over the whole L1 in between).
-template <typename TI, typename TO, bool TA, bool TB, int WM = 2, int WN = 2, int KB = 64, bool EDGE = false>
-__global__ void __launch_bounds__(64 * WM * WN, (!EDGE ? 1 : TA && !TB && sizeof(TI) == 2 ? 3 : 4)) gemm_kernel(const TI* __restrict__ A, int64_t lda, int64_t sA,
+// registers keeps the accumulators of four wavefronts beside their operands and four blocks on a CU.  128 products of n x n,
+// float32, us with all subtiles always / with EDGE, both operands by rows: 392 (4 x 4 tiles of 128, the last 8 wide) 251 / 222, 320
+// 138 / 114; by columns 231 / 220, 116 / 108, 200 37.5 / 37.1; one partial tile, 512 products: 64 16.5 / 12.6.  (Loads left out as well,
+// behind a condition, make every wait one for all loads.)
+// 2-byte operands come here where the result is float32, is added to, or does not lie in 16-byte pieces; see gemm_direct_kernel.
+template <typename TI, typename TO, bool TA, bool TB, int WM = 2, int WN = 2, bool EDGE = false>
+__global__ void __launch_bounds__(64 * WM * WN, (!EDGE ? 1 : 4)) gemm_kernel(const TI* __restrict__ A, int64_t lda, int64_t sA,
                                                    const TI* __restrict__ B, int64_t ldb, int64_t sB,
                                                    TO* __restrict__ C, int64_t ldc, int64_t sC, int Mfull, int N, int Kfull,
                                                    float alpha, int accumulate, int vec_out, int64_t k_total, int nparts, int64_t pA,
@@ -259,13 +257,13 @@ __global__ void __launch_bounds__(64 * WM * WN, (!EDGE ? 1 : TA && !TB && sizeof
                                                    int64_t gsB, int64_t gsC) {
   using F = TI;
   constexpr int EPV = 16 / sizeof(TI);  // elements per 16-byte vector
-  constexpr int BK = KB / sizeof(TI);   // k extent of one step
-  constexpr int RB = KB + 16;           // bytes between the rows of a contraction-contiguous tile
-  constexpr int NQ = KB / 32;           // 16-byte slices of k per half wavefront and step
+  constexpr int BK = kStepBytes / sizeof(TI);  // k extent of one step
+  constexpr int RB = kRowBytes;         // bytes between the rows of a contraction-contiguous tile
+  constexpr int NQ = kStepBytes / 32;   // 16-byte slices of k per half wavefront and step
   constexpr int TMR = 64 * WM, TNC = 64 * WN, NTH = 64 * WM * WN;  // tile rows, tile columns, threads
   constexpr int TSA = trans_stride<TI, TMR>(), TSB = trans_stride<TI, TNC>();
-  constexpr int ABYTES = gemm_tile_bytes<TI, TMR, KB>(), BBYTES = gemm_tile_bytes<TI, TNC, KB>();
-  constexpr int NVA = TMR * (KB / 16) / NTH, NVB = TNC * (KB / 16) / NTH;  // 16-byte vectors per thread and step
+  constexpr int ABYTES = gemm_tile_bytes<TI, TMR>(), BBYTES = gemm_tile_bytes<TI, TNC>();
+  constexpr int NVA = TMR * (kStepBytes / 16) / NTH, NVB = TNC * (kStepBytes / 16) / NTH;  // 16-byte vectors per thread and step
   __shared__ __align__(16) char smem[2][ABYTES + BBYTES];
   const int tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63, c = lane & 31, h = lane >> 5;
@@ -318,9 +316,9 @@ __global__ void __launch_bounds__(64 * WM * WN, (!EDGE ? 1 : TA && !TB && sizeof
   uint4 stA[NVA], stB[NVB];
   int arow[NVA], apart[NVA], brow[NVB], bpart[NVB];
 #pragma unroll
-  for (int q = 0; q < NVA; ++q) gemm_stage_offsets<TI, TA, TMR, KB>(tid + q * NTH, arow[q], apart[q]);
+  for (int q = 0; q < NVA; ++q) gemm_stage_offsets<TI, TA, TMR>(tid + q * NTH, arow[q], apart[q]);
 #pragma unroll
-  for (int q = 0; q < NVB; ++q) gemm_stage_offsets<TI, TB, TNC, KB>(tid + q * NTH, brow[q], bpart[q]);
+  for (int q = 0; q < NVB; ++q) gemm_stage_offsets<TI, TB, TNC>(tid + q * NTH, brow[q], bpart[q]);
   auto load_one = [&](const TI* __restrict__ P, int64_t ld, bool tr, int row, int part, int x0, int X, int ks) -> uint4 {
     if (tr) {  // row = k within the step, part = vector along the tile's columns (extent X is a multiple of EPV)
       const int k = ks * BK + row, x = x0 + part * EPV;
@@ -369,8 +367,8 @@ __global__ void __launch_bounds__(64 * WM * WN, (!EDGE ? 1 : TA && !TB && sizeof
         for (int t = 0; t < 2; ++t)
 #pragma unroll
           for (int q = 0; q < NQ; ++q) {
-            if (t < NI) fa[t < NI ? t : 0][q] = gemm_fragment<TI, TA, TMR, KB>(&smem[buf][0], wm * 64 + t * 32, q, lane);
-            if (t < NJ) fb[t < NJ ? t : 0][q] = gemm_fragment<TI, TB, TNC, KB>(&smem[buf][ABYTES], wn * 64 + t * 32, q, lane);
+            if (t < NI) fa[t < NI ? t : 0][q] = gemm_fragment<TI, TA, TMR>(&smem[buf][0], wm * 64 + t * 32, q, lane);
+            if (t < NJ) fb[t < NJ ? t : 0][q] = gemm_fragment<TI, TB, TNC>(&smem[buf][ABYTES], wn * 64 + t * 32, q, lane);
           }
         // consecutive MFMAs go to different accumulators: a dependent one would wait for its predecessor to drain
 #pragma unroll
@@ -448,6 +446,251 @@ __global__ void __launch_bounds__(64 * WM * WN, (!EDGE ? 1 : TA && !TB && sizeof
         }
       }
     }
+}
+
+// ------------------------------------------------------------------------------------------------
+// The same products of 2-byte operands with loads that go from memory straight into LDS (16 bytes a lane, 1 KB an instruction) and
+// blocks that stay: a block walks its tiles as one row of steps, ST step buffers in turn, and requests ST - 1 steps ahead, also
+// past the end of a tile - the first steps of the next one arrive while the results of this one leave.
+// What bounds it: memory traffic (128 products of 512 x 512 x 512 move 201 MB; without the fragment reads and products the same
+// launch takes 44 - 48 us, with operands from the L2 and one place for the results 36 - 38), for short rows the chain of a block's
+// first step and its results.
+// Tiles of one matrix are cut evenly (mstep x nstep, whole subtiles): 392 x 392 are four times 224 x 224, not 256 x 256 and three
+// rims.  A wavefront forms the subtiles that reach into its tile.
+// The places of the 16-byte units of a row are permuted by the row, so that both kinds of fragment read - 16 bytes of 16
+// consecutive rows, 8 bytes of 4 consecutive k rows - touch every bank once; the permutation is applied to the addresses of the
+// requests, as the places themselves are given by the lane.
+// Waits: loads and stores of a wavefront return in order, so "all but the youngest n" is exact: n counts the loads of the steps that
+// follow and, for the steps requested before them, the stores of a whole tile; after a partly filled one (whose stores are fewer) the
+// wait takes in the stores too.
+// us, 128 products of n x n x n in bfloat16 on rotating buffers, gemm_kernel / this one: both operands by rows 512 55 / 52, 480 67 / 49,
+// 392 56 / 40, 320 23 / 21, 256 13.2 / 11.4, 200 11.1 / 10.5, 128 6.2 / 5.1, 64 5.1 / 4.2; B by columns 53 / 50, 62 / 45, 51 / 38, 31 / 25,
+// 12.7 / 11.1, 10.7 / 9.9, 6.5 / 5.3; both by columns 52 / 48, 57 / 42, 45 / 32, 22 / 20, 12.2 / 10.7, 10.2 / 8.9, 6.4 / 5.3.
+// Without the steps that cross tiles 392 took 42, 41, 36; three buffers instead of two 512 52 instead of 57.
+// ------------------------------------------------------------------------------------------------
+__device__ __attribute__((aligned(16))) const uint32_t kZeros16[4] = {0, 0, 0, 0};
+
+// A wavefront-uniform address, pinned to scalar registers so that loads take the "scalar base + 32-bit lane offset" form
+// instead of one 64-bit vector address per access.
+__device__ __forceinline__ const char* uniform_ptr(const void* p) {
+  const uint64_t v = reinterpret_cast<uint64_t>(p);
+  const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v));
+  const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v >> 32));
+  return reinterpret_cast<const char*>((static_cast<uint64_t>(hi) << 32) | lo);
+}
+
+template <int N>
+__device__ __forceinline__ void wait_and_meet() {  // all but the N youngest memory accesses have returned, LDS reads are done; then everybody
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+// 16 bytes per lane from memory into LDS, at `lds` + 16 lane.  (As assembly: around the builtin the compiler waits for all loads in
+// flight before every LDS read.  The address may come fresh from a vector instruction, which takes five wait states; m0 takes one.)
+__device__ __forceinline__ void load_to_lds(const char* base, uint32_t off, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds) : "memory", "m0");
+}
+__device__ __forceinline__ void load_to_lds(const char* p, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(p), "s"(lds) : "memory", "m0");
+}
+// rows [half SR, half SR + SR) of a 32 x 32 accumulator into a staging tile (see stage_put)
+template <typename F, int SR>
+__device__ __forceinline__ void stage_rows(char* tile, int row_stride, int col, int h, const floatx16& acc, float alpha, int half) {
+#pragma unroll
+  for (int v = 0; v < 16; v += 2) {
+    const int r = 8 * (v >> 2) + (v & 3) - half * SR;
+    if (r < 0 || r >= SR) continue;
+    char* p = tile + (r + 4 * h) * row_stride + col * 2;
+    const uint32_t w = pack16<F>(alpha * acc[v], alpha * acc[v + 1]);
+    *reinterpret_cast<uint16_t*>(p) = static_cast<uint16_t>(w & 0xffffu);
+    *reinterpret_cast<uint16_t*>(p + row_stride) = static_cast<uint16_t>(w >> 16);
+  }
+}
+
+// SM x SN subtiles of 32 x 32 a wavefront, WM x WN wavefronts a block, KB bytes of k a row and step, SR staged rows at a time
+template <int SM_, int SN_, int WM_, int WN_, int KB_, int ST_, int SR_, int BLOCKS_>
+struct DirectShape {
+  static constexpr int SM = SM_, SN = SN_, WM = WM_, WN = WN_, KB = KB_, ST = ST_, SR = SR_, BLOCKS = BLOCKS_;  // BLOCKS: on a CU
+  static constexpr int TM = 32 * SM * WM, TN = 32 * SN * WN, RS = 64 * SN + 16;
+  static constexpr int kLds = ST * (TM + TN) * KB + WM * WN * SR * RS;
+};
+
+template <typename F, bool TA, bool TB, typename Shape>
+__global__ void __launch_bounds__(64 * Shape::WM * Shape::WN, 2)
+gemm_direct_kernel(const F* __restrict__ A, int64_t lda, int64_t sA, const F* __restrict__ B, int64_t ldb, int64_t sB, F* __restrict__ C, int64_t ldc,
+                   int64_t sC, int M, int N, int K, float alpha, int mstep, int nstep, uint32_t gx, uint32_t gy, uint32_t total) {
+  constexpr int SM = Shape::SM, SN = Shape::SN, WM = Shape::WM, WN = Shape::WN, KB = Shape::KB, ST = Shape::ST, SR = Shape::SR, RS = Shape::RS;
+  constexpr int TM = Shape::TM, TN = Shape::TN, NW = WM * WN, BK = KB / 2, NQ = KB / 32;
+  constexpr int AB = TM * KB, BB = TN * KB, SB = AB + BB;                          // bytes of a step of A, of B, of both
+  constexpr int NA = AB / (1024 * NW), NB = BB / (1024 * NW), NL = NA + NB;        // loads of a wavefront and step
+  constexpr int S = SM * 2 * SN;                                                   // stores of a wavefront and whole tile
+  static_assert(AB % (1024 * NW) == 0 && BB % (1024 * NW) == 0, "whole loads per wavefront");
+  static_assert(ST == 2 || ST == 3, "see arrive");
+  static_assert(NL + S < 64, "the counter of outstanding accesses has six bits");
+  extern __shared__ __align__(16) char smem[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = lane & 31, h = lane >> 5;
+  const int wm = wave / WN, wn = wave % WN;
+  const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)smem)) + wave * 1024;
+  const int64_t step_a = TA ? BK * lda * 2 : KB, step_b = TB ? BK * ldb * 2 : KB;
+  const int nsteps = (K + BK - 1) / BK;
+  auto tile_at = [&](uint32_t L, int& bx, int& by, int& bz) {  // (see xcd_tile)
+    const uint32_t q = total >> 3, r = total & 7, x = L & 7, P = x * q + (x < r ? x : r) + (L >> 3);
+    bx = static_cast<int>(P % gx);
+    by = static_cast<int>((P / gx) % gy);
+    bz = static_cast<int>(P / (gx * gy));
+  };
+  // the place of the unit that a lane fills in load i of a step, and which unit of the row belongs there
+  auto unit = [&](bool tr, int ext, int i, int& row, int& u) {
+    const int byte = (i * NW + wave) * 1024 + lane * 16, rb = tr ? ext * 2 : KB;
+    row = byte / rb;
+    u = (byte % rb) / 16;
+    if (tr) u ^= (row & 3) << 2;
+    else if (KB == 128) u ^= (row >> 1) & 7;
+    else u ^= (row >> 2) & 3;
+  };
+  auto offset = [&](bool tr, int ext, int64_t ld, int x0, int X, int i) -> uint32_t {  // rows and columns past the end: the last ones again
+    int row, u;
+    unit(tr, ext, i, row, u);
+    if (tr) return static_cast<uint32_t>(row * ld + min(x0 + u * 8, X - 8)) * 2;
+    return static_cast<uint32_t>(min(x0 + row, X - 1) * ld + u * 8) * 2;
+  };
+  auto first_k = [&](bool tr, int ext, int i) -> int {
+    int row, u;
+    unit(tr, ext, i, row, u);
+    return tr ? row : u * 8;
+  };
+  uint32_t next_tile = blockIdx.x;
+  int next_step = 0, next_buf = 0;
+  const char *pa = nullptr, *pb = nullptr;
+  uint32_t va[NA], vb[NB];
+  auto enter = [&](uint32_t t) {
+    int bx, by, bz;
+    tile_at(t, bx, by, bz);
+    pa = reinterpret_cast<const char*>(A + bz * sA);
+    pb = reinterpret_cast<const char*>(B + bz * sB);
+#pragma unroll
+    for (int i = 0; i < NA; ++i) va[i] = offset(TA, TM, lda, by * mstep, M, i);
+#pragma unroll
+    for (int i = 0; i < NB; ++i) vb[i] = offset(TB, TN, ldb, bx * nstep, N, i);
+  };
+  auto request = [&]() {  // the next step, if there is one
+    if (next_tile >= total) return;
+    const uint32_t d = __builtin_amdgcn_readfirstlane(lds0 + next_buf * SB);
+    const char *ua = uniform_ptr(pa), *ub = uniform_ptr(pb);
+    const int left = __builtin_amdgcn_readfirstlane(K - next_step * BK);
+    if (left >= BK) {
+#pragma unroll
+      for (int i = 0; i < NA; ++i) load_to_lds(ua, va[i], d + i * NW * 1024);
+#pragma unroll
+      for (int i = 0; i < NB; ++i) load_to_lds(ub, vb[i], d + AB + i * NW * 1024);
+    } else {  // zeros past the end of the contraction
+      const char* z = reinterpret_cast<const char*>(kZeros16);
+#pragma unroll
+      for (int i = 0; i < NA; ++i) load_to_lds(first_k(TA, TM, i) < left ? pa + va[i] : z, d + i * NW * 1024);
+#pragma unroll
+      for (int i = 0; i < NB; ++i) load_to_lds(first_k(TB, TN, i) < left ? pb + vb[i] : z, d + AB + i * NW * 1024);
+    }
+    next_buf = next_buf + 1 == ST ? 0 : next_buf + 1;
+    if (++next_step == nsteps) {
+      next_step = 0;
+      next_tile += gridDim.x;
+      if (next_tile < total) enter(next_tile);
+    } else {
+      pa += step_a;
+      pb += step_b;
+    }
+  };
+  auto fragment = [&](bool tr, int ext, const char* tile, int base, int q) -> uint4 {  // k = 16 q + 8 h + (0 .. 7)
+    if (!tr) {
+      const int row = base + c, u = 2 * q + h;
+      return *reinterpret_cast<const uint4*>(tile + row * KB + (u ^ (KB == 128 ? (row >> 1) & 7 : (row >> 2) & 3)) * 16);
+    }
+    const int s = lane & 15, g16 = (lane >> 4) & 1, row = 16 * q + 8 * h + (s >> 2), col = base + 16 * g16 + 4 * (s & 3);
+    const char* p = tile + row * ext * 2 + ((col * 2) ^ ((row & 3) << 6));
+    typedef shortx4_t __attribute__((address_space(3))) * lptr;
+    const uint2 x = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lptr)(p)));
+    const uint2 y = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lptr)(p + 4 * ext * 2)));
+    return make_uint4(x.x, x.y, y.x, y.y);
+  };
+
+  enter(next_tile);
+#pragma unroll
+  for (int s = 0; s < ST - 1; ++s) request();
+  int buf = 0;
+  bool stores = false;  // the tile before was a whole one of this wavefront: S stores are younger than the requests made ahead of them
+  char* const tile = smem + ST * SB + wave * (SR * RS);
+  for (uint32_t t = blockIdx.x; t < total; t += gridDim.x) {
+    int bx, by, bz;
+    tile_at(t, bx, by, bz);
+    const int m0 = by * mstep, n0 = bx * nstep;
+    const int mi = min(M, m0 + mstep) - (m0 + wm * 32 * SM), nj = min(N, n0 + nstep) - (n0 + wn * 32 * SN);  // rows and columns that exist
+    const int follow = static_cast<int>((total - 1 - t) / gridDim.x) * nsteps + nsteps - 1;  // steps after the tile's first
+    floatx16 acc[SM][SN];
+#pragma unroll
+    for (int i = 0; i < SM; ++i)
+#pragma unroll
+      for (int j = 0; j < SN; ++j) acc[i][j] = floatx16{0};
+    auto arrive = [&](int ks) {
+      const bool st = ks < ST - 1 && stores;
+      if (ST == 3 && follow > ks) {
+        if (st) wait_and_meet<(ST - 2) * NL + S>();
+        else wait_and_meet<(ST - 2) * NL>();
+      } else {
+        if (st) wait_and_meet<S>();
+        else wait_and_meet<0>();
+      }
+    };
+    auto steps = [&](auto ni, auto njs) {  // NI x NJ of the wavefront's subtiles (the barriers are the same on every way)
+      constexpr int NI = decltype(ni)::value, NJ = decltype(njs)::value;
+      for (int ks = 0; ks < nsteps; ++ks) {
+        arrive(ks);
+        request();  // (into the buffer that everybody has just left)
+        if constexpr (NI > 0 && NJ > 0) {
+          const char* ta = smem + buf * SB;
+          const char* tb = ta + AB;
+#pragma unroll
+          for (int q = 0; q < NQ; ++q) {
+            uint4 fa[NI], fb[NJ];
+#pragma unroll
+            for (int i = 0; i < NI; ++i) fa[i] = fragment(TA, TM, ta, (wm * SM + i) * 32, q);
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) fb[j] = fragment(TB, TN, tb, (wn * SN + j) * 32, q);
+#pragma unroll
+            for (int i = 0; i < NI; ++i)
+#pragma unroll
+              for (int j = 0; j < NJ; ++j) acc[i][j] = mm_32x32x16<F>(fa[i], fb[j], acc[i][j]);
+          }
+        }
+        buf = buf + 1 == ST ? 0 : buf + 1;
+      }
+    };
+    static_assert(SN == 2 && (SM == 2 || SM == 4), "the ways below");
+    constexpr std::integral_constant<int, 0> none;
+    constexpr std::integral_constant<int, 1> one;
+    constexpr std::integral_constant<int, 2> two;
+    constexpr std::integral_constant<int, SM == 4 ? 3 : 2> three;
+    constexpr std::integral_constant<int, SM> all;
+    auto rows = [&](auto n) {
+      if (nj > 32) steps(n, two);
+      else steps(n, one);
+    };
+    if (mi <= 0 || nj <= 0) steps(none, none);
+    else if (mi > 32 * (SM - 1)) rows(all);
+    else if (SM == 4 && mi > 64) rows(three);
+    else if (SM == 4 && mi > 32) rows(two);
+    else rows(one);
+    F* out = C + bz * sC + static_cast<int64_t>(m0 + wm * SM * 32) * ldc + n0 + wn * 32 * SN;
+#pragma unroll
+    for (int i = 0; i < SM; ++i)
+#pragma unroll
+      for (int half = 0; half < 32 / SR; ++half) {
+        const int r0 = 32 * i + half * SR;
+#pragma unroll
+        for (int j = 0; j < SN; ++j) stage_rows<F, SR>(tile, RS, 32 * j + c, h, acc[i][j], alpha, half);
+        __builtin_amdgcn_wave_barrier();
+        stage_flush<F, 32 * SN>(tile, RS, min(SR, mi - r0), out + static_cast<int64_t>(r0) * ldc, ldc, lane, 64, false, nj);
+        __builtin_amdgcn_wave_barrier();
+      }
+    stores = mi >= 32 * SM && nj >= 32 * SN;
+  }
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -743,15 +986,6 @@ __device__ __forceinline__ void mma_step(floatx16& acc, const uint4& a, const ui
 #pragma unroll
     for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(pa[e], pb[e], acc, 0, 0, 0);
   }
-}
-
-// A wavefront-uniform address, pinned to scalar registers so that loads take the "scalar base + 32-bit lane offset" form
-// instead of one 64-bit vector address per access.
-__device__ __forceinline__ const char* uniform_ptr(const void* p) {
-  const uint64_t v = reinterpret_cast<uint64_t>(p);
-  const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v));
-  const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v >> 32));
-  return reinterpret_cast<const char*>((static_cast<uint64_t>(hi) << 32) | lo);
 }
 
 template <typename V>
@@ -2690,6 +2924,62 @@ using namespace cueq;
     if ((dt) == CUEQ_F32) { CALL_F32; } else if ((dt) == CUEQ_F16) { CALL_F16; } else { CALL_BF16; } \
   } while (0)
 
+// A kernel's limit of dynamic LDS, raised once per device.
+template <auto Kernel>
+static int raise_lds(int bytes) {
+  static uint64_t done = 0;  // one bit per device
+  int dev = 0;
+  CUEQ_CHECK_HIP(hipGetDevice(&dev));
+  if (dev < 64 && (__atomic_load_n(&done, __ATOMIC_ACQUIRE) >> dev & 1)) return CUEQ_OK;
+  CUEQ_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(Kernel), hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
+  if (dev < 64) __atomic_fetch_or(&done, uint64_t(1) << dev, __ATOMIC_RELEASE);
+  return CUEQ_OK;
+}
+
+// Wide: 256 x 256 tiles, eight wavefronts of 128 x 64, from one tile per compute unit on, and where the tile is not mostly empty (128
+// products, us wide / narrow: 512 48 - 52 / 57 - 63, 384 30 - 33 / 32 - 35, 264 19 / 20; 64 products of 264 11 - 12 / 13 - 14, of 256 - 64
+// tiles - 11.6 / 7.6; 256 products of 256 21 / 24, of 144 10 / 12, of 104 7.7 / 6.2).  Operands that both lie by rows of k take 128 bytes of
+// a row a step and two buffers, whole lines (128 products of 392 39.5 / 42.2, 768 141 / 164); by columns a step's rows are whole lines
+// already, and three buffers of half the depth are faster (392 36.4 / 32.0, 480 45.6 / 42.3).
+template <bool ROWS>
+using DirectWide = DirectShape<4, 2, 2, 4, ROWS ? 128 : 64, ROWS ? 2 : 3, ROWS ? 16 : 32, 1>;
+using DirectNarrow = DirectShape<2, 2, 2, 2, 64, 3, 16, 2>;  // 128 x 128 tiles, four wavefronts of 64 x 64
+
+template <typename F, bool TA, bool TB, typename Shape>
+static int launch_gemm_direct(int64_t M, int64_t N, int64_t K, const F* A, int64_t lda, int64_t sA, const F* B, int64_t ldb, int64_t sB, F* C, int64_t ldc,
+                              int64_t sC, int64_t batch, float alpha, hipStream_t stream) {
+  static_assert(Shape::kLds <= 160 * 1024, "");
+  auto cut = [](int64_t n, int64_t tile, int64_t& count) {  // as many tiles as there must be, all but the last of one size
+    count = (n + tile - 1) / tile;
+    return static_cast<int>(((n + count - 1) / count + 31) & ~int64_t(31));
+  };
+  int64_t gx, gy;
+  const int mstep = cut(M, Shape::TM, gy), nstep = cut(N, Shape::TN, gx);
+  const int64_t total = gx * gy * batch;
+  constexpr auto kernel = gemm_direct_kernel<F, TA, TB, Shape>;
+  const int rc = raise_lds<kernel>(Shape::kLds);
+  if (rc != CUEQ_OK) return rc;
+  const int64_t grid = std::min<int64_t>(total, static_cast<int64_t>(device_cus()) * Shape::BLOCKS);
+  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(64 * Shape::WM * Shape::WN), Shape::kLds, stream, A, lda, sA, B, ldb, sB, C, ldc, sC,
+                     static_cast<int>(M), static_cast<int>(N), static_cast<int>(K), alpha, mstep, nstep, static_cast<uint32_t>(gx), static_cast<uint32_t>(gy),
+                     static_cast<uint32_t>(total));
+  CUEQ_CHECK_HIP(hipGetLastError());
+  return CUEQ_OK;
+}
+template <typename F>
+static int gemm_direct(bool ta, bool tb, int64_t M, int64_t N, int64_t K, const void* A, int64_t lda, int64_t sA, const void* B, int64_t ldb, int64_t sB, void* C,
+                       int64_t ldc, int64_t sC, int64_t batch, float alpha, hipStream_t stream) {
+  const bool wide = M > 128 && N > 128 && ((M + 255) / 256) * ((N + 255) / 256) * batch >= device_cus();
+  auto go = [&](auto a, auto b) {
+    constexpr bool TA = decltype(a)::value, TB = decltype(b)::value;
+    const F *pa = static_cast<const F*>(A), *pb = static_cast<const F*>(B);
+    return wide ? launch_gemm_direct<F, TA, TB, DirectWide<!TA && !TB>>(M, N, K, pa, lda, sA, pb, ldb, sB, static_cast<F*>(C), ldc, sC, batch, alpha, stream)
+                : launch_gemm_direct<F, TA, TB, DirectNarrow>(M, N, K, pa, lda, sA, pb, ldb, sB, static_cast<F*>(C), ldc, sC, batch, alpha, stream);
+  };
+  if (ta) return tb ? go(std::true_type{}, std::true_type{}) : go(std::true_type{}, std::false_type{});
+  return tb ? go(std::false_type{}, std::true_type{}) : go(std::false_type{}, std::false_type{});
+}
+
 extern "C" int cueq_gemm(int32_t in_dtype, int32_t out_dtype, int32_t trans_a, int32_t trans_b, int64_t M, int64_t N, int64_t K,
                          const void* A, int64_t lda, int64_t stride_a, const void* B, int64_t ldb, int64_t stride_b, void* C,
                          int64_t ldc, int64_t stride_c, int64_t batch, double alpha, int32_t accumulate, void* stream_) {
@@ -2737,18 +3027,35 @@ extern "C" int cueq_gemm(int32_t in_dtype, int32_t out_dtype, int32_t trans_a, i
     const int vec_out = (reinterpret_cast<uintptr_t>(C) % 16 == 0 && (ldc * out_es) % 16 == 0 && (stride_c * out_es) % 16 == 0) ? 1 : 0;
     // 256 x 256 tiles when both extents are multiples of 256 and there are enough of them to fill the chip
     const bool big = !mixed && M % 256 == 0 && N % 256 == 0 && (M / 256) * (N / 256) * batch >= 2 * static_cast<int64_t>(device_cus());
-    // (the timing label names the tile size, so a test can tell which kernel a shape ran on)
+    // (the timing label says whether 256 x 256 tiles fill the chip twice, so a test can tell which kernel a shape ran on)
     KernelTimer timer(in_dtype == CUEQ_F32 ? (big ? "gemm_nt_f32_256" : "gemm_nt_f32") : in_dtype == CUEQ_F16 ? (big ? "gemm_nt_f16_256" : "gemm_nt_f16") : (big ? "gemm_nt_bf16_256" : "gemm_nt_bf16"), stream);
-    // EDGE where some tile is partly filled, in float32 only where one in four is or there is one column of tiles: between whole tiles what is
-    // left is the bound on registers (us without / with, float32: 16 products of 1 032 x 1 032 x 128, 21 % of tiles partial, 64.6 / 70.5, 4 of
-    // 2 056 64.6 / 67.4, 64 of 520, 36 %, 76 / 71; 153 664 x 128 x 128, A by rows and B by columns, 64 / 57, both by columns 63 / 56, both
-    // by rows 66.6 / 70.2, 131 080 64.7 / 52.8; bfloat16 2 056 21.3 / 21.5, 1 032 22.5 / 22.3, 153 664 x 128 x 256 27.1 / 24.8)
+    // 2-byte operands and results of one type: straight into LDS, unless results are added to or their rows are not 16-byte pieces
+    // (byte offsets inside an operand are 32 bits, tile numbers 31)
+    const int64_t far = int64_t(1) << 31;
+    if (!mixed && in_dtype != CUEQ_F32 && !accumulate && vec_out && n % 8 == 0 && (trans_a ? 64 : M) * lda < far && (trans_b ? 64 : N) * ldb < far &&
+        (M / 128 + 1) * (N / 128 + 1) * batch < far) {
+      if (in_dtype == CUEQ_F16) return gemm_direct<f16bits>(trans_a != 0, trans_b != 0, M, N, K, A, lda, stride_a, B, ldb, stride_b, C, ldc, stride_c, batch, al, stream);
+      return gemm_direct<uint16_t>(trans_a != 0, trans_b != 0, M, N, K, A, lda, stride_a, B, ldb, stride_b, C, ldc, stride_c, batch, al, stream);
+    }
+    // EDGE (float32) where one tile in four is partly filled or there is one column of tiles: between whole tiles what is left is the
+    // bound on registers (us without / with: 16 products of 1 032 x 1 032 x 128, 21 % of tiles partial, 64.6 / 70.5, 4 of 2 056
+    // 64.6 / 67.4, 64 of 520, 36 %, 76 / 71; 153 664 x 128 x 128, A by rows and B by columns, 64 / 57, both by columns 63 / 56, both by
+    // rows 66.6 / 70.2, 131 080 64.7 / 52.8)
     const int64_t whole = (M / kTile) * (N / kTile), all = static_cast<int64_t>(grid.x) * grid.y;
-    const bool edge = whole < all && (in_dtype != CUEQ_F32 || grid.x == 1 || 4 * (all - whole) >= all);
+    const bool edge = whole < all && (grid.x == 1 || 4 * (all - whole) >= all);
     const dim3 grid_big(static_cast<unsigned>(N / 256), static_cast<unsigned>(M / 256), static_cast<unsigned>(batch));
 #define GEMM_ARGS(TI, TO) static_cast<const TI*>(A), lda, stride_a, static_cast<const TI*>(B), ldb, stride_b, static_cast<TO*>(C), ldc, stride_c, m, n, k, al, accumulate, vec_out, 0, 1, 0, 0, 0, nullptr, 0, 0, 0, 0
 #define GEMM_LAUNCH(TI, TO, TA, TB) hipLaunchKernelGGL((gemm_kernel<TI, TO, TA, TB>), grid, dim3(256), 0, stream, GEMM_ARGS(TI, TO))
-#define GEMM_SZ(TI, TA, TB) do { if (big) hipLaunchKernelGGL((gemm_kernel<TI, TI, TA, TB, 4, 4, (sizeof(TI) == 2 ? 128 : 64)>), grid_big, dim3(1024), 0, stream, GEMM_ARGS(TI, TI)); else if (edge) hipLaunchKernelGGL((gemm_kernel<TI, TI, TA, TB, 2, 2, 64, true>), grid, dim3(256), 0, stream, GEMM_ARGS(TI, TI)); else GEMM_LAUNCH(TI, TI, TA, TB); } while (0)
+#define GEMM_SZ(TI, TA, TB)                                                                                                                      \
+  do {                                                                                                                                       \
+    if constexpr (sizeof(TI) == 4) {                                                                                                         \
+      if (big) hipLaunchKernelGGL((gemm_kernel<TI, TI, TA, TB, 4, 4>), grid_big, dim3(1024), 0, stream, GEMM_ARGS(TI, TI));                  \
+      else if (edge) hipLaunchKernelGGL((gemm_kernel<TI, TI, TA, TB, 2, 2, true>), grid, dim3(256), 0, stream, GEMM_ARGS(TI, TI));          \
+      else GEMM_LAUNCH(TI, TI, TA, TB);                                                                                                      \
+    } else {                                                                                                                                 \
+      GEMM_LAUNCH(TI, TI, TA, TB);                                                                                                           \
+    }                                                                                                                                        \
+  } while (0)
 #define GEMM_TR(TI) do { if (trans_a && trans_b) GEMM_SZ(TI, true, true); else if (trans_a) GEMM_SZ(TI, true, false); else if (trans_b) GEMM_SZ(TI, false, true); else GEMM_SZ(TI, false, false); } while (0)
     if (in_dtype == CUEQ_F32 && out_dtype == CUEQ_F32) GEMM_TR(float);
     else if (in_dtype == CUEQ_F32 && out_dtype == CUEQ_F16) GEMM_LAUNCH(float, f16bits, false, false);

@@ -186,6 +186,51 @@ def test_layer_norm_fused_into_the_gated_projection(device, M, K, C, affine, bia
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("trans_a,trans_b", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize(
+    "batch,M,N,K",
+    [
+        (700, 72, 40, 8),  # more 128 x 128 tiles than stay on the chip, one step each
+        (1, 8, 8, 24),  # the smallest
+        (3, 200, 136, 1000),  # tiles cut unevenly, the last step a quarter full
+        (300, 264, 136, 40),  # 256 x 256 tiles, two a matrix and more than one a compute unit, partly filled ones between whole ones
+        (130, 392, 520, 104),
+    ],
+)
+def test_gemm_two_byte_tiles(device, dtype, trans_a, trans_b, batch, M, N, K):
+    """The tiles of the 2-byte products at their edges, against float64: rounding of one result (2^-8 / 2^-11) and float32 sums; an
+    infinity in the last row of A and in the last column of B stays in its row and column; nothing is written between the rows of C."""
+    import ctypes as C
+
+    from cuequivariance_amd import _lib
+
+    g = torch.Generator(device=device).manual_seed(M + N + K)
+    A = torch.randn((batch, K, M) if trans_a else (batch, M, K), generator=g, device=device).to(dtype)
+    B = torch.randn((batch, K, N) if trans_b else (batch, N, K), generator=g, device=device).to(dtype)
+    A64 = A.double().transpose(1, 2).contiguous() if trans_a else A.double()
+    B64 = B.double() if trans_b else B.double().transpose(1, 2).contiguous()
+    ref = A64 @ B64
+    (A[-1, K - 1, M - 1:] if trans_a else A[-1, M - 1, K - 1:]).fill_(float("inf"))
+    (B[0, K - 1, N - 1:] if trans_b else B[0, N - 1, K - 1:]).fill_(float("inf"))
+    out = torch.full((batch, M, N + 8), -7.0, dtype=dtype, device=device)
+    lib = _lib.load()
+    code = {torch.bfloat16: _lib.BF16, torch.float16: _lib.F16}[dtype]
+    p = lambda t: C.c_void_p(t.data_ptr())
+    _lib.check(lib.cueq_gemm(code, code, int(trans_a), int(trans_b), M, N, K, p(A), A.shape[2], A[0].numel(), p(B), B.shape[2], B[0].numel(), p(out), N + 8,
+                             M * (N + 8), batch, C.c_double(1.0), 0, torch.cuda.current_stream().cuda_stream), "cueq_gemm")
+    assert bool((out[:, :, N:] == -7.0).all())
+    got = out[:, :, :N].double()
+    bad = torch.zeros_like(got, dtype=torch.bool)
+    bad[-1, M - 1, :] = True
+    bad[0, :, N - 1] = True
+    assert torch.equal(~torch.isfinite(got), bad)
+    unit = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    bound = unit * ref.abs() + 2.0 ** -22 * K * (A64.abs().amax() * B64.abs().amax())
+    assert bool(((got - ref).abs() <= bound + 2.0 ** -24)[~bad].all())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("trans_a,trans_b", [(False, False), (False, True), (True, False), (True, True)])
 @pytest.mark.parametrize("dims", [(3, 256, 128, 192), (2, 136, 200, 72), (1, 33, 47, 21), (160, 512, 256, 96),
