@@ -510,33 +510,51 @@ template <int SM_, int SN_, int WM_, int WN_, int KB_, int ST_, int SR_, int BLO
 struct DirectShape {
   static constexpr int SM = SM_, SN = SN_, WM = WM_, WN = WN_, KB = KB_, ST = ST_, SR = SR_, BLOCKS = BLOCKS_;  // BLOCKS: on a CU
   static constexpr int TM = 32 * SM * WM, TN = 32 * SN * WN, RS = 64 * SN + 16;
-  static constexpr int kLds = ST * (TM + TN) * KB + WM * WN * SR * RS;
+  static constexpr int kLds = ST * (TM + TN) * KB + WM * WN * SR * RS;  // (SR = 0: float32 results, which need no staging)
 };
 
-template <typename F, bool TA, bool TB, typename Shape>
+// The pieces of a long contraction: item = (chunk, part) of the batch covers k in [chunk K, (chunk + 1) K) of k_total (the last ones may
+// be short or empty), operands and result `p*` elements apart from part to part.
+struct DirectParts {
+  int64_t k_total, pA, pB, pC;
+  int nparts;
+};
+
+// TO = F: a batch of products, blocks that stay.  TO = float (F two bytes): the pieces of a long contraction, a block each.
+template <typename F, typename TO, bool TA, bool TB, typename Shape>
 __global__ void __launch_bounds__(64 * Shape::WM * Shape::WN, 2)
-gemm_direct_kernel(const F* __restrict__ A, int64_t lda, int64_t sA, const F* __restrict__ B, int64_t ldb, int64_t sB, F* __restrict__ C, int64_t ldc,
-                   int64_t sC, int M, int N, int K, float alpha, int mstep, int nstep, uint32_t gx, uint32_t gy, uint32_t total) {
+gemm_direct_kernel(const F* __restrict__ A, int64_t lda, int64_t sA, const F* __restrict__ B, int64_t ldb, int64_t sB, TO* __restrict__ C, int64_t ldc,
+                   int64_t sC, int M, int N, int K, float alpha, int mstep, int nstep, uint32_t gx, uint32_t gy, uint32_t total, DirectParts parts) {
+  constexpr bool PARTS = std::is_same_v<TO, float>;
   constexpr int SM = Shape::SM, SN = Shape::SN, WM = Shape::WM, WN = Shape::WN, KB = Shape::KB, ST = Shape::ST, SR = Shape::SR, RS = Shape::RS;
   constexpr int TM = Shape::TM, TN = Shape::TN, NW = WM * WN, BK = KB / 2, NQ = KB / 32;
   constexpr int AB = TM * KB, BB = TN * KB, SB = AB + BB;                          // bytes of a step of A, of B, of both
   constexpr int NA = AB / (1024 * NW), NB = BB / (1024 * NW), NL = NA + NB;        // loads of a wavefront and step
-  constexpr int S = SM * 2 * SN;                                                   // stores of a wavefront and whole tile
+  constexpr int S = PARTS ? 0 : SM * 2 * SN;                                       // stores of a wavefront and whole tile
   static_assert(AB % (1024 * NW) == 0 && BB % (1024 * NW) == 0, "whole loads per wavefront");
-  static_assert(ST == 2 || ST == 3, "see arrive");
-  static_assert(NL + S < 64, "the counter of outstanding accesses has six bits");
+  static_assert(ST >= 2 && ST <= 4, "see arrive");
+  static_assert((ST - 2) * NL + S < 64, "the counter of outstanding accesses has six bits");
   extern __shared__ __align__(16) char smem[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = lane & 31, h = lane >> 5;
   const int wm = wave / WN, wn = wave % WN;
   const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)smem)) + wave * 1024;
   const int64_t step_a = TA ? BK * lda * 2 : KB, step_b = TB ? BK * ldb * 2 : KB;
-  const int nsteps = (K + BK - 1) / BK;
   auto tile_at = [&](uint32_t L, int& bx, int& by, int& bz) {  // (see xcd_tile)
     const uint32_t q = total >> 3, r = total & 7, x = L & 7, P = x * q + (x < r ? x : r) + (L >> 3);
     bx = static_cast<int>(P % gx);
     by = static_cast<int>((P / gx) % gy);
     bz = static_cast<int>(P / (gx * gy));
   };
+  if constexpr (PARTS) {
+    int bx, by, bz;
+    tile_at(blockIdx.x, bx, by, bz);
+    const int chunk = bz / parts.nparts, part = bz - chunk * parts.nparts;
+    A += (chunk - bz) * sA + part * parts.pA;
+    B += (chunk - bz) * sB + part * parts.pB;
+    C += (chunk - bz) * sC + part * parts.pC;
+    K = static_cast<int>(max<int64_t>(0, min<int64_t>(K, parts.k_total - static_cast<int64_t>(chunk) * K)));
+  }
+  const int nsteps = (K + BK - 1) / BK;
   // the place of the unit that a lane fills in load i of a step, and which unit of the row belongs there
   auto unit = [&](bool tr, int ext, int i, int& row, int& u) {
     const int byte = (i * NW + wave) * 1024 + lane * 16, rb = tr ? ext * 2 : KB;
@@ -613,7 +631,8 @@ gemm_direct_kernel(const F* __restrict__ A, int64_t lda, int64_t sA, const F* __
 
   enter(next_tile);
 #pragma unroll
-  for (int s = 0; s < ST - 1; ++s) request();
+  for (int s = 0; s < ST - 1; ++s)
+    if (!PARTS || s < nsteps) request();
   int buf = 0;
   bool stores = false;  // the tile before was a whole one of this wavefront: S stores are younger than the requests made ahead of them
   char* const tile = smem + ST * SB + wave * (SR * RS);
@@ -630,13 +649,15 @@ gemm_direct_kernel(const F* __restrict__ A, int64_t lda, int64_t sA, const F* __
       for (int j = 0; j < SN; ++j) acc[i][j] = floatx16{0};
     auto arrive = [&](int ks) {
       const bool st = ks < ST - 1 && stores;
-      if (ST == 3 && follow > ks) {
-        if (st) wait_and_meet<(ST - 2) * NL + S>();
-        else wait_and_meet<(ST - 2) * NL>();
-      } else {
-        if (st) wait_and_meet<S>();
-        else wait_and_meet<0>();
-      }
+      const int ahead = min(follow - ks, ST - 2);  // younger steps
+      auto wait = [&](auto n) {
+        constexpr int younger = decltype(n)::value * NL;
+        if (st) wait_and_meet<younger + S>();
+        else wait_and_meet<younger>();
+      };
+      if (ST >= 4 && ahead == 2) wait(std::integral_constant<int, ST >= 4 ? 2 : 0>{});
+      else if (ST >= 3 && ahead == 1) wait(std::integral_constant<int, ST >= 3 ? 1 : 0>{});
+      else wait(std::integral_constant<int, 0>{});
     };
     auto steps = [&](auto ni, auto njs) {  // NI x NJ of the wavefront's subtiles (the barriers are the same on every way)
       constexpr int NI = decltype(ni)::value, NJ = decltype(njs)::value;
@@ -677,18 +698,31 @@ gemm_direct_kernel(const F* __restrict__ A, int64_t lda, int64_t sA, const F* __
     else if (SM == 4 && mi > 64) rows(three);
     else if (SM == 4 && mi > 32) rows(two);
     else rows(one);
-    F* out = C + bz * sC + static_cast<int64_t>(m0 + wm * SM * 32) * ldc + n0 + wn * 32 * SN;
+    TO* out = C + bz * sC + static_cast<int64_t>(m0 + wm * SM * 32) * ldc + n0 + wn * 32 * SN;
+    if constexpr (PARTS) {  // 128 contiguous bytes a store as they are
 #pragma unroll
-    for (int i = 0; i < SM; ++i)
+      for (int i = 0; i < SM; ++i)
 #pragma unroll
-      for (int half = 0; half < 32 / SR; ++half) {
-        const int r0 = 32 * i + half * SR;
+        for (int j = 0; j < SN; ++j)
 #pragma unroll
-        for (int j = 0; j < SN; ++j) stage_rows<F, SR>(tile, RS, 32 * j + c, h, acc[i][j], alpha, half);
-        __builtin_amdgcn_wave_barrier();
-        stage_flush<F, 32 * SN>(tile, RS, min(SR, mi - r0), out + static_cast<int64_t>(r0) * ldc, ldc, lane, 64, false, nj);
-        __builtin_amdgcn_wave_barrier();
-      }
+          for (int v = 0; v < 16; ++v) {
+            const int row = 32 * i + 8 * (v >> 2) + 4 * h + (v & 3), col = 32 * j + c;
+            if (row < mi && col < nj) out[row * ldc + col] = alpha * acc[i][j][v];
+          }
+      return;
+    } else {
+#pragma unroll
+      for (int i = 0; i < SM; ++i)
+#pragma unroll
+        for (int half = 0; half < 32 / SR; ++half) {
+          const int r0 = 32 * i + half * SR;
+#pragma unroll
+          for (int j = 0; j < SN; ++j) stage_rows<F, SR>(tile, RS, 32 * j + c, h, acc[i][j], alpha, half);
+          __builtin_amdgcn_wave_barrier();
+          stage_flush<F, 32 * SN>(tile, RS, min(SR, mi - r0), out + static_cast<int64_t>(r0) * ldc, ldc, lane, 64, false, nj);
+          __builtin_amdgcn_wave_barrier();
+        }
+    }
     stores = mi >= 32 * SM && nj >= 32 * SN;
   }
 }
@@ -2956,13 +2990,13 @@ static int launch_gemm_direct(int64_t M, int64_t N, int64_t K, const F* A, int64
   int64_t gx, gy;
   const int mstep = cut(M, Shape::TM, gy), nstep = cut(N, Shape::TN, gx);
   const int64_t total = gx * gy * batch;
-  constexpr auto kernel = gemm_direct_kernel<F, TA, TB, Shape>;
+  constexpr auto kernel = gemm_direct_kernel<F, F, TA, TB, Shape>;
   const int rc = raise_lds<kernel>(Shape::kLds);
   if (rc != CUEQ_OK) return rc;
   const int64_t grid = std::min<int64_t>(total, static_cast<int64_t>(device_cus()) * Shape::BLOCKS);
   hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(64 * Shape::WM * Shape::WN), Shape::kLds, stream, A, lda, sA, B, ldb, sB, C, ldc, sC,
                      static_cast<int>(M), static_cast<int>(N), static_cast<int>(K), alpha, mstep, nstep, static_cast<uint32_t>(gx), static_cast<uint32_t>(gy),
-                     static_cast<uint32_t>(total));
+                     static_cast<uint32_t>(total), DirectParts{});
   CUEQ_CHECK_HIP(hipGetLastError());
   return CUEQ_OK;
 }
@@ -2978,6 +3012,27 @@ static int gemm_direct(bool ta, bool tb, int64_t M, int64_t N, int64_t K, const 
   };
   if (ta) return tb ? go(std::true_type{}, std::true_type{}) : go(std::true_type{}, std::false_type{});
   return tb ? go(std::false_type{}, std::true_type{}) : go(std::false_type{}, std::false_type{});
+}
+
+// 128 x 128 float32 partial products of a long contraction (chunks x parts of them), B contraction-major: bound by the operands' bytes,
+// which are read once.  One block on a CU with 64 KB in flight and half as many partial results (us, 512 x 128 over 153 664 / 262 144
+// columns, A by rows: this 35 / 67, two blocks a CU of 64 bytes a step and four buffers 37 / 78, three 36 / 79), or two of them where
+// the number of pieces is given (PieceShape: 128 x 128 x 9 parts over 200 000 rows 171, gemm_kernel 174; 64 x 64 x 16 over 150 000 126 / 148).
+using DirectLong = DirectShape<2, 2, 2, 2, 128, 3, 0, 1>;
+using PieceShape = DirectShape<2, 2, 2, 2, 64, 3, 0, 2>;
+template <typename F, bool TA, typename Shape>
+static int gemm_direct_long(int64_t M, int64_t N, int64_t kc, const void* A, int64_t lda, int64_t sA, const void* B, int64_t ldb, int64_t sB, float* C, int64_t sC,
+                            int64_t chunks, const DirectParts& parts, float alpha, hipStream_t stream) {
+  const int64_t gy = (M + Shape::TM - 1) / Shape::TM, gx = (N + Shape::TN - 1) / Shape::TN, total = gx * gy * chunks * parts.nparts;
+  CUEQ_REQUIRE(total < (int64_t(1) << 31), CUEQ_ERR_TOO_LARGE, "gemm: too many tiles");
+  constexpr auto kernel = gemm_direct_kernel<F, float, TA, true, Shape>;
+  const int rc = raise_lds<kernel>(Shape::kLds);
+  if (rc != CUEQ_OK) return rc;
+  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(total)), dim3(64 * Shape::WM * Shape::WN), Shape::kLds, stream, static_cast<const F*>(A), lda,
+                     sA, static_cast<const F*>(B), ldb, sB, C, N, sC, static_cast<int>(M), static_cast<int>(N), static_cast<int>(kc), alpha, Shape::TM,
+                     Shape::TN, static_cast<uint32_t>(gx), static_cast<uint32_t>(gy), static_cast<uint32_t>(total), parts);
+  CUEQ_CHECK_HIP(hipGetLastError());
+  return CUEQ_OK;
 }
 
 extern "C" int cueq_gemm(int32_t in_dtype, int32_t out_dtype, int32_t trans_a, int32_t trans_b, int64_t M, int64_t N, int64_t K,
@@ -3429,18 +3484,26 @@ extern "C" int cueq_gate_bwd_input_ln(int32_t dtype, int64_t C, int64_t M, int64
 // Partial products of a long contraction in the input type's matrix instructions: chunk i of `chunks` covers k in
 // [i kc, (i + 1) kc), kc = long_k_chunk(...); partials[i][part] (float32, M x N) = A_part[:, chunk] B_part[:, chunk]^T.  A is M x K, or
 // K x M with trans_a; B is K x N; part p of A / B starts p * stride_a / stride_b elements further.  The caller sums the chunks.
-static int64_t long_k_chunk(int64_t K, int64_t M, int64_t N, int64_t nparts) {
+static int64_t long_k_chunk(int32_t dtype, int64_t K, int64_t M, int64_t N, int64_t nparts) {
   const int64_t tiles = ((M + kTile - 1) / kTile) * ((N + kTile - 1) / kTile) * nparts;
-  int64_t chunks = std::max<int64_t>(1, 2 * device_cus() / tiles);
+  int64_t chunks = std::max<int64_t>(1, (dtype == CUEQ_F32 ? 2 : 1) * device_cus() / tiles);
   chunks = std::min(chunks, std::max<int64_t>(1, K / 512));
   return ((K + chunks - 1) / chunks + 63) & ~int64_t(63);
 }
 static int gemm_long_k(int32_t dtype, bool trans_a, int64_t M, int64_t N, int64_t K, const void* A, int64_t lda, int64_t stride_a, const void* B,
                        int64_t ldb, int64_t stride_b, int64_t nparts, float* partials, hipStream_t stream) {
-  const int64_t kc = long_k_chunk(K, M, N, nparts), chunks = (K + kc - 1) / kc;
+  const int64_t kc = long_k_chunk(dtype, K, M, N, nparts), chunks = (K + kc - 1) / kc;
   CUEQ_REQUIRE(chunks * nparts < 65536 && M < (1 << 20) && N < (1 << 20), CUEQ_ERR_TOO_LARGE, "gemm_long_k: too many parts");
   const dim3 grid(static_cast<unsigned>((N + kTile - 1) / kTile), static_cast<unsigned>((M + kTile - 1) / kTile), static_cast<unsigned>(chunks * nparts));
   KernelTimer timer("gemm_long_k", stream);
+  // (offsets inside a tile are 32 bits: 64 rows of k, or M rows with the contraction inside)
+  if (dtype != CUEQ_F32 && (trans_a ? 64 : M) * lda < (int64_t(1) << 31) && 64 * ldb < (int64_t(1) << 31)) {
+    const DirectParts parts{K, stride_a, stride_b, M * N, static_cast<int>(nparts)};
+#define LKD(F) (trans_a ? gemm_direct_long<F, true, DirectLong>(M, N, kc, A, lda, kc * lda, B, ldb, kc * ldb, partials, nparts * M * N, chunks, parts, 1.0f, stream) \
+                        : gemm_direct_long<F, false, DirectLong>(M, N, kc, A, lda, kc, B, ldb, kc * ldb, partials, nparts * M * N, chunks, parts, 1.0f, stream))
+    return dtype == CUEQ_F16 ? LKD(f16bits) : LKD(uint16_t);
+#undef LKD
+  }
 #define LK(TI, TA) hipLaunchKernelGGL((gemm_kernel<TI, float, TA, true>), grid, dim3(256), 0, stream, static_cast<const TI*>(A), lda, TA ? kc * lda : kc, static_cast<const TI*>(B), ldb, kc * ldb, partials, N, nparts * M * N, static_cast<int>(M), static_cast<int>(N), static_cast<int>(kc), 1.0f, 0, 0, K, static_cast<int>(nparts), stride_a, stride_b, M * N, nullptr, 0, 0, 0, 0)
 #define LK_T(TI) do { if (trans_a) LK(TI, true); else LK(TI, false); } while (0)
   TRI_DISPATCH(dtype, LK_T(float), LK_T(uint16_t), LK_T(f16bits));
@@ -3477,6 +3540,13 @@ extern "C" int cueq_gemm_tn(int32_t in_dtype, int64_t M, int64_t N, int64_t rows
   if (in_dtype != CUEQ_F32 && vec && rows > 0) {
     // 2-byte inputs: MFMA on contraction-major tiles (transposing LDS reads); batch items = (row chunk, part)
     const int64_t rpc32 = (((rows + chunks - 1) / chunks + 31) / 32) * 32;
+    // (whole 128 x 128 results: the other kernel, 163 us / 172 inside a step of the 200 000 rows above)
+    if ((M % kTile || N % kTile) && 64 * lda < (int64_t(1) << 31) && 64 * ldb < (int64_t(1) << 31)) {
+      const DirectParts parts{rows, stride_a, stride_b, chunks * M * N, nparts};
+#define TND(F) gemm_direct_long<F, true, PieceShape>(M, N, rpc32, A, lda, rpc32 * lda, B, ldb, rpc32 * ldb, partials, M * N, chunks, parts, static_cast<float>(alpha), stream)
+      return in_dtype == CUEQ_F16 ? TND(f16bits) : TND(uint16_t);
+#undef TND
+    }
 #define TN2(FT) hipLaunchKernelGGL((gemm_kernel<FT, float, true, true>), grid, dim3(256), 0, stream, static_cast<const FT*>(A), lda, \
                        rpc32 * lda, static_cast<const FT*>(B), ldb, rpc32 * ldb, partials, N, static_cast<int64_t>(M) * N, \
                        static_cast<int>(M), static_cast<int>(N), static_cast<int>(rpc32), static_cast<float>(alpha), 0, 0, rows, nparts, \
@@ -3934,7 +4004,7 @@ struct TriBwdWork {
     du2 = weights || !fused_out ? c.take(2 * p.M * p.Do * p.es) : nullptr;
     du1 = weights || !fused_in ? c.take(4 * rows) : nullptr;
     auto partial = [&](int64_t m, int64_t n, int64_t parts) {
-      const int64_t kc = long_k_chunk(p.M, m, n, parts), chunks = (p.M + kc - 1) / kc;
+      const int64_t kc = long_k_chunk(p.dt, p.M, m, n, parts), chunks = (p.M + kc - 1) / kc;
       return chunks * parts * m * n * 4 + 256 + cueq_sum_rows_workspace(chunks, parts * m * n);
     };
     part_bytes = weights ? std::max({partial(4 * p.D, p.D, 1), partial(p.Do, p.D, 2), cueq_sum_rows_workspace(p.M, p.Do)}) : 0;
@@ -4094,7 +4164,7 @@ extern "C" int cueq_trimul_bwd_parts(int32_t dtype, int64_t B, int64_t N, int64_
   const int64_t epv = 16 / es;
   // sums of the partial products of a long contraction straight into the gradient
   auto long_k = [&](bool trans_a, int64_t m, const char* A, int64_t lda, int64_t sa, const char* Bm, int64_t sb, int64_t parts, float* to) -> int {
-    const int64_t kc = long_k_chunk(M, m, D, parts), chunks = (M + kc - 1) / kc;
+    const int64_t kc = long_k_chunk(dtype, M, m, D, parts), chunks = (M + kc - 1) / kc;
     float* part = reinterpret_cast<float*>(k.part);
     TRI_STEP(gemm_long_k(dtype, trans_a, m, D, M, A, lda, sa, Bm, D, sb, parts, part, stream));
     char* ws = k.part + ((chunks * parts * m * D * 4 + 255) & ~int64_t(255));

@@ -231,6 +231,27 @@ def test_gemm_two_byte_tiles(device, dtype, trans_a, trans_b, batch, M, N, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,parts,M,N", [(1, 1, 8, 8), (40, 3, 64, 32), (65, 2, 136, 40), (5000, 16, 32, 64), (20_011, 9, 64, 96), (4097, 1, 128, 128)])
+def test_gemm_tn_two_byte_pieces(device, dtype, rows, parts, M, N):
+    """The pieces of long 2-byte contractions, those without rows among them, against float64: float32 sums of exact products."""
+    from cuequivariance_amd import _lib
+
+    g = torch.Generator(device=device).manual_seed(rows)
+    A, B = (torch.randn(rows, parts * n, generator=g, device=device).to(dtype) for n in (M, N))
+    lib = _lib.load()
+    items = lib.cueq_gemm_tn_items(rows, parts)
+    part = torch.full((items, M, N), float("nan"), device=device)
+    code = {torch.bfloat16: _lib.BF16, torch.float16: _lib.F16}[dtype]
+    _lib.check(lib.cueq_gemm_tn(code, M, N, rows, A.data_ptr(), parts * M, M, B.data_ptr(), parts * N, N, parts, part.data_ptr(), 0.5,
+                                torch.cuda.current_stream().cuda_stream), "cueq_gemm_tn")
+    got = part.view(parts, items // parts, M, N).double().sum(1)
+    a, b = A.double().view(rows, parts, M).permute(1, 2, 0).contiguous(), B.double().view(rows, parts, N).transpose(0, 1).contiguous()
+    ref = 0.5 * a @ b
+    assert (got - ref).abs().max().item() <= 2.0 ** -22 * (a.abs() @ b.abs()).max().item()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("trans_a,trans_b", [(False, False), (False, True), (True, False), (True, True)])
 @pytest.mark.parametrize("dims", [(3, 256, 128, 192), (2, 136, 200, 72), (1, 33, 47, 21), (160, 512, 256, 96),
