@@ -1603,7 +1603,7 @@ __global__ void __launch_bounds__((SPLIT ? 256 : 512), (SPLIT ? 1 : 2))
     // the rows of the next tile (past the end: the last tile again, so that the request is unconditional)
     request_x(tile_row(min(tile + tstep, ntiles - 1)));
     if constexpr (SPLIT) {
-      // Results of the two-input form (one wavefront per SIMD, nothing to add to): 8 rows (one value group a) at a time
+      // Results of the two-input form (one wavefront per SIMD, C other than K; nothing to add to): 8 rows (one value group a) at a time
       // through the wave-private staging tile, whole rows out as 16-byte vectors.  (The stores from registers of the
       // other form, 32 bytes per row and instruction, measure 5 % slower here.)
 #pragma unroll
@@ -1734,6 +1734,200 @@ __global__ void __launch_bounds__((SPLIT ? 256 : 512), (SPLIT ? 1 : 2))
           for (int j = 0; j < 2; ++j) *reinterpret_cast<uint4*>(dX1 + orow + (ds * 64 + j * 32) / ES) = val[ds][j];
       }
       __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+}
+
+// ------------------------------------------------------------------------------------------------
+// The two-input form for as many weight rows as there are columns (C = K = 32 KT, the output stage of the triangle update), eight
+// wavefronts to a compute unit instead of four.  What kept one wavefront to a SIMD above is 2 KT accumulators beside both rows of X
+// and the chunk in work.  Here the gate gradients of all chunks are formed first and kept packed (8 KT registers each) - the rows of
+// X are done with then -, and the two products follow one after the other with KT accumulators each, the next tile's rows already on
+// their way.  Results pass through a tile of LDS private to the wavefront and leave as whole rows.
+// Bound by its bytes (x, y, the cotangent, two gradients): 512 x 512 rows of 128, bfloat16, 111 -> 77 us = 4.4 TB/s; 392 x 392 rows of a
+// padded square with the gate gradients written out, 81 -> 59 us.
+// ------------------------------------------------------------------------------------------------
+template <typename F, int KT, bool PAD>
+__global__ void __launch_bounds__(512, 2)
+    gate_bwd_two_kernel(const F* __restrict__ W1, const F* __restrict__ W2, int64_t ldw, const F* __restrict__ X1, const F* __restrict__ X2,
+                        int64_t ldx, const F* __restrict__ bias1, const F* __restrict__ bias2, const F* __restrict__ mask,
+                        const F* __restrict__ dC, int64_t ldc, F* __restrict__ dX1, F* __restrict__ dX2, int64_t lddx, F* __restrict__ dU,
+                        F* __restrict__ dV, int M, PairRows pairs) {
+  constexpr int C = 32 * KT, K = 32 * KT, ROWB = 2 * K, NS = ROWB / 64, VPR = ROWB / 16;
+  constexpr bool SWZ = KT == 4;  // (same layout of the weight rows as gate_bwd_input_res_kernel)
+  constexpr int WSTR = SWZ ? ROWB : ROWB + 16, SSTR = ROWB + 16;
+  auto swz = [](int row) -> int { return SWZ ? (((row & 3) << 2) | ((row >> 2) & 3)) : 0; };
+  constexpr int NTH = 512, NWAVES = 8;
+  extern __shared__ __align__(16) char gbi_dsm[];
+  char* sw1 = gbi_dsm;
+  char* sw2 = gbi_dsm + C * WSTR;
+  float* sb = reinterpret_cast<float*>(gbi_dsm + 2 * C * WSTR);  // bias1[C], bias2[C]
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, c = lane & 31, h = lane >> 5;
+  char* stage = reinterpret_cast<char*>(sb + 2 * C) + wave * (32 * SSTR);
+
+  for (int e0 = tid; e0 < C * VPR; e0 += 4 * NTH) {
+    u32x4_t w1[4], w2[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {  // (eight requests in flight: 2 us less a launch than piece by piece; past the end the last one again)
+      const int e = min(e0 + i * NTH, C * VPR - 1);
+      const int64_t o = static_cast<int64_t>(e / VPR) * ldw + (e % VPR) * 8;
+      w1[i] = *reinterpret_cast<const u32x4_t*>(W1 + o);
+      w2[i] = *reinterpret_cast<const u32x4_t*>(W2 + o);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int e = min(e0 + i * NTH, C * VPR - 1);
+      const int r = e / VPR, po = ((e % VPR) ^ swz(r)) << 4;
+      *reinterpret_cast<u32x4_t*>(sw1 + r * WSTR + po) = w1[i];
+      *reinterpret_cast<u32x4_t*>(sw2 + r * WSTR + po) = w2[i];
+    }
+  }
+  for (int i = tid; i < C; i += NTH) {
+    sb[i] = bias1 ? tri_load(bias1, i) : 0.f;
+    sb[C + i] = bias2 ? tri_load(bias2, i) : 0.f;
+  }
+  __syncthreads();
+
+  const int64_t ntiles = (static_cast<int64_t>(M) + 31) / 32;
+  const int64_t tstep = static_cast<int64_t>(gridDim.x) * NWAVES;
+  auto tile_row = [&](int64_t t) -> int { return static_cast<int>(min(t * 32 + c, static_cast<int64_t>(M) - 1)); };
+  // the cotangents of a chunk, four adjacent ones a register pair (rows 8 a + 4 h .. + 3), requested a chunk ahead across tiles
+  uint32_t dcr[8], dcn[8], pofs = 0;
+  auto dc_lane_offset = [&](int mld) -> uint32_t {
+    if constexpr (PAD) mld = max(pairs.src(mld), 0);
+    return static_cast<uint32_t>((mld * ldc + 4 * h) * 2);
+  };
+  auto request_dc = [&](int ci) {
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+      const char* base = uniform_ptr(reinterpret_cast<const char*>(dC) + static_cast<int64_t>(ci * 32 + 8 * a) * 2);
+      const uint2 w = load_global<uint2>(base, pofs);
+      dcn[2 * a] = w.x; dcn[2 * a + 1] = w.y;
+    }
+  };
+  uint4 xf1[NS][2], xf2[NS][2];
+  uint32_t mraw = 0;
+  auto request_x = [&](int mld) {
+#pragma unroll
+    for (int s2 = 0; s2 < NS; ++s2)
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const int64_t o = static_cast<int64_t>(mld) * ldx + (s2 * 64 + h * 32 + q * 16) / 2;
+        xf1[s2][q] = *reinterpret_cast<const uint4*>(X1 + o);
+        xf2[s2][q] = *reinterpret_cast<const uint4*>(X2 + o);
+      }
+    bool live;
+    if (mask) mraw = raw16(mask[PAD ? pairs.near(mld, live) : mld]);
+  };
+  // (tiles dealt out wavefront-major: the last round of a ragged number of them runs on all compute units)
+  int64_t tile = static_cast<int64_t>(wave) * gridDim.x + blockIdx.x;
+  if (tile >= ntiles) return;
+  request_x(tile_row(tile));
+  pofs = dc_lane_offset(tile_row(tile));
+  request_dc(0);
+
+  for (; tile < ntiles; tile += tstep) {
+    const int mrow0 = static_cast<int>(tile * 32), mcol = mrow0 + c;
+    const int next = tile_row(min(tile + tstep, ntiles - 1));  // (past the end: the last tile again, so that requests are unconditional)
+    const float mk = mask ? lo16<F>(mraw) : 1.0f;
+    const uint32_t real = (PAD && pairs.src(min(mcol, M - 1)) < 0) ? 0u : ~0u;  // (padding has no cotangent)
+    uint32_t pu[KT][8], pv[KT][8];
+#pragma unroll
+    for (int ci = 0; ci < KT; ++ci) {
+      const int c0 = ci * 32;
+#pragma unroll
+      for (int v = 0; v < 8; ++v) dcr[v] = PAD ? (dcn[v] & real) : dcn[v];
+      if (ci == KT - 1) pofs = dc_lane_offset(next);
+      request_dc((ci + 1) % KT);
+
+      floatx16 au, av;
+#pragma unroll
+      for (int a = 0; a < 4; ++a) {
+        const float4 b1 = *reinterpret_cast<const float4*>(sb + c0 + 8 * a + 4 * h);
+        const float4 b2 = *reinterpret_cast<const float4*>(sb + C + c0 + 8 * a + 4 * h);
+        au[4 * a] = b1.x; au[4 * a + 1] = b1.y; au[4 * a + 2] = b1.z; au[4 * a + 3] = b1.w;
+        av[4 * a] = b2.x; av[4 * a + 1] = b2.y; av[4 * a + 2] = b2.z; av[4 * a + 3] = b2.w;
+      }
+      const int wrow = (c0 + c) * WSTR;
+#pragma unroll
+      for (int s2 = 0; s2 < NS; ++s2)
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          const int wo = wrow + ((((2 * h + q) ^ swz(c)) << 4) ^ (s2 << 6));
+          mma_step<F>(au, *reinterpret_cast<const uint4*>(sw1 + wo), xf1[s2][q]);
+          mma_step<F>(av, *reinterpret_cast<const uint4*>(sw2 + wo), xf2[s2][q]);
+        }
+#pragma unroll
+      for (int a = 0; a < 4; ++a) {
+        float du[4], dv[4];
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+          const int v = 4 * a + b;
+          const float sg = __builtin_amdgcn_rcpf(1.0f + __expf(-au[v]));
+          const uint32_t w = dcr[v >> 1];
+          dv[b] = ((v & 1) ? hi16<F>(w) : lo16<F>(w)) * mk * sg;
+          du[b] = dv[b] * fmaf(-av[v], sg, av[v]);
+        }
+        pu[ci][2 * a] = pack16<F>(du[0], du[1]); pu[ci][2 * a + 1] = pack16<F>(du[2], du[3]);
+        pv[ci][2 * a] = pack16<F>(dv[0], dv[1]); pv[ci][2 * a + 1] = pack16<F>(dv[2], dv[3]);
+      }
+      __builtin_amdgcn_sched_barrier(0);  // one chunk at a time
+    }
+
+    // whole rows of what the wavefront has staged
+    auto flush = [&](F* to, int64_t ld) {
+      __builtin_amdgcn_wave_barrier();
+      stage_flush<F, K>(stage, SSTR, min(32, M - mrow0), to + static_cast<int64_t>(mrow0) * ld, ld, lane, 64, false);
+      __builtin_amdgcn_wave_barrier();
+    };
+    if (dU != nullptr) {
+#pragma unroll
+      for (int which = 0; which < 2; ++which) {
+#pragma unroll
+        for (int ci = 0; ci < KT; ++ci)
+#pragma unroll
+          for (int a = 0; a < 4; ++a) {
+            const uint32_t* w = which == 0 ? pu[ci] : pv[ci];
+            *reinterpret_cast<uint2*>(stage + c * SSTR + (ci * 32 + 8 * a + 4 * h) * 2) = make_uint2(w[2 * a], w[2 * a + 1]);
+          }
+        flush(which == 0 ? dU : dV, ldc);
+      }
+    }
+    request_x(next);
+#pragma unroll
+    for (int which = 0; which < 2; ++which) {
+      const char* sw = which == 0 ? sw1 : sw2;
+      floatx16 ax[KT];
+#pragma unroll
+      for (int t = 0; t < KT; ++t) ax[t] = floatx16{0};
+      typedef shortx4_t __attribute__((address_space(3))) * lptr;
+      const int s16 = lane & 15, g16 = (lane >> 4) & 1;
+      // rows 4 h + (s16 >> 2) (+ 8, + 16 t): a row 8 further flips bit 1 of the swizzle, 16 further leaves it
+      const int trow = 4 * h + (s16 >> 2), tunit = 2 * g16 + ((s16 & 3) >> 1);
+      const int ulo = (tunit ^ swz(trow)) << 4, uhi = SWZ ? (ulo ^ 32) : ulo;
+#pragma unroll
+      for (int ci = 0; ci < KT; ++ci) {
+        const int off = (ci * 32 + trow) * WSTR + 8 * (s16 & 1);
+        const uint32_t* w = which == 0 ? pu[ci] : pv[ci];
+#pragma unroll
+        for (int ds = 0; ds < KT; ++ds)
+#pragma unroll
+          for (int t = 0; t < 2; ++t) {
+            const uint2 lo = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lptr)(sw + off + t * 16 * WSTR + (ulo ^ (ds << 6)))));
+            const uint2 hi = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lptr)(sw + off + (t * 16 + 8) * WSTR + (uhi ^ (ds << 6)))));
+            // the weight columns are the rows of the product: a lane holds its own m and 16 values of k
+            mma_step<F>(ax[ds], make_uint4(lo.x, lo.y, hi.x, hi.y), make_uint4(w[4 * t], w[4 * t + 1], w[4 * t + 2], w[4 * t + 3]));
+          }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int ds = 0; ds < KT; ++ds)
+#pragma unroll
+        for (int a = 0; a < 4; ++a)
+          *reinterpret_cast<uint2*>(stage + c * SSTR + (ds * 32 + 8 * a + 4 * h) * 2) =
+              make_uint2(pack16<F>(ax[ds][4 * a], ax[ds][4 * a + 1]), pack16<F>(ax[ds][4 * a + 2], ax[ds][4 * a + 3]));
+      flush(which == 0 ? dX1 : dX2, lddx);
     }
   }
 }
@@ -3418,6 +3612,22 @@ static int gate_bwd_input_impl(int32_t dtype, int64_t C, int64_t M, int64_t K, c
     const bool pairs_ok = !dc_by_row || (M % 2 == 0 && ldc % 2 == 0 && reinterpret_cast<uintptr_t>(dC) % 4 == 0);
     if (lds <= 160 * 1024 && pairs_ok) {
       const int64_t ntiles = (M + 31) / 32;
+      // (as many weight rows as columns: two wavefronts to a SIMD, 77 us where one takes 111; the gate gradients of more rows than columns
+      // would not stay in the registers)
+      if (split && C == K) {
+        const size_t two = static_cast<size_t>(2 * C * (K == 128 ? 2 * K : 2 * K + 16) + 8 * C + 8 * 32 * (2 * K + 16));
+        const int64_t gt = std::min<int64_t>(ntiles, device_cus());
+#define GBT_F(FT, KT, PD) do { auto kfn = gate_bwd_two_kernel<FT, KT, PD>; \
+        CUEQ_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kfn), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(two))); \
+        hipLaunchKernelGGL(kfn, dim3(static_cast<unsigned>(gt)), dim3(512), two, stream, static_cast<const FT*>(W1), static_cast<const FT*>(W2), ldw, static_cast<const FT*>(X1), static_cast<const FT*>(X2), ldx, static_cast<const FT*>(bias1), static_cast<const FT*>(bias2), static_cast<const FT*>(mask), static_cast<const FT*>(dC), ldc, static_cast<FT*>(dX1), static_cast<FT*>(dX2), lddx, static_cast<FT*>(dU), static_cast<FT*>(dV), static_cast<int>(M), pairs); } while (0)
+#define GBT(KT, PD) do { if (half) GBT_F(f16bits, KT, PD); else GBT_F(uint16_t, KT, PD); } while (0)
+        if (pairs.np) { if (K == 64) GBT(2, true); else GBT(4, true); }
+        else switch (K / 32) { case 1: GBT(1, false); break; case 2: GBT(2, false); break; case 3: GBT(3, false); break; default: GBT(4, false); break; }
+#undef GBT
+#undef GBT_F
+        CUEQ_CHECK_HIP(hipGetLastError());
+        return CUEQ_OK;
+      }
       // (tiles to the CUs first: 392 x 392 rows, one input, 109 us with the tiles of a block next to each other, 94 so - the second
       // round of 4 802 tiles on 2 048 wavefronts ran on a third of the CUs; 64 x 64 rows 30 and 21)
       const int64_t gx = std::min<int64_t>(split ? ntiles : (ntiles + 1) / 2, device_cus());

@@ -78,3 +78,28 @@ def test_input_gradients_of_float32(device, inputs, M, K, C):
             assert (a is None) == (b is None)
             # (float32 sums of up to 2 x 256 products)
             assert a is None or (a.cpu().double() - b).abs().max().item() <= 1e-5 * b.abs().max().item()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("K", [32, 64, 96, 128])
+@pytest.mark.parametrize("M", [1, 31, 33, 8191, 65_569])
+def test_two_inputs_with_as_many_weight_rows_as_columns(device, M, K, dtype):
+    """The output stage in 2-byte types: parts of a tile of 32 rows, and one wavefront with a second tile (65 569 rows are 2 050 tiles for
+    2 048 wavefronts); with and without gate gradients, mask and biases."""
+    from cuequivariance_amd.cuet import triangle as T
+
+    g = torch.Generator().manual_seed(M + K)
+    r = lambda *shape: torch.randn(*shape, generator=g).to(dtype).float().to(device)
+    X1, X2, W1, W2, b1, b2, dout = r(M, K), r(M, K), r(K, K) / 8, r(K, K) / 8, r(K), r(K), r(M, K)
+    mask = (torch.rand(M, generator=g) < 0.8).float().to(device)
+    f = lambda t: t.to(dtype)
+    for plain in (False, True):
+        x1, x2 = X1.clone().requires_grad_(), X2.clone().requires_grad_()
+        u, v = x1 @ W1.T + (0 if plain else b1), x2 @ W2.T + (0 if plain else b2)
+        want = torch.autograd.grad(torch.sigmoid(u) * v * (1 if plain else mask[:, None]), [x1, x2, u, v], dout)
+        few = (None, None, None) if plain else (f(b1), f(b2), f(mask))
+        got = T.gate_bwd_input(f(dout), False, f(W1), f(W2), f(X1), f(X2), *few, None, not plain)
+        for a, b in zip(got, want):
+            # (the gate gradients are rounded once and so is the result: with unit roundoff e, e (sum |du w| / max |dx| + 1) of the largest
+            # value, the sum of K random products about twice the largest result)
+            assert (plain and a is None) or (a.float() - b).abs().max().item() <= TOL[dtype] * b.abs().max().item()
