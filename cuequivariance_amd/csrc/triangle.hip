@@ -1747,17 +1747,43 @@ __global__ void __launch_bounds__((SPLIT ? 256 : 512), (SPLIT ? 1 : 2))
 // Bound by its bytes (x, y, the cotangent, two gradients): 512 x 512 rows of 128, bfloat16, 111 -> 77 us = 4.4 TB/s; 392 x 392 rows of a
 // padded square with the gate gradients written out, 81 -> 59 us.
 // ------------------------------------------------------------------------------------------------
-template <typename F, int KT, bool PAD>
+// sums of v[0 .. 15] over the lanes of each half of a wavefront: lane c of a half returns that of v[c >> 1]
+__device__ __forceinline__ float half_wave_sums16(float (&v)[16], int lane) {
+#pragma unroll
+  for (int i = 0; i < 8; ++i) v[i] = lane_fold<16>(v[i], v[i + 8], lane);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v[i] = lane_fold<8>(v[i], v[i + 4], lane);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) v[i] = lane_fold<4>(v[i], v[i + 2], lane);
+  return lane_fold<1>(lane_fold<2>(v[0], v[1], lane));
+}
+
+// The LayerNorm across d whose rows are X2, for the backward that goes on through it: its input (D x M, D = K), statistics and weight,
+// where the gradient of the input goes (D x M), and, where those of its weight and bias are wanted, partial sums of a block
+// ([2][blocks][K]).
+template <typename F>
+struct NormAcross {
+  const F* x = nullptr;
+  const float* mean = nullptr;
+  const float* rstd = nullptr;
+  const F* gamma = nullptr;
+  F* dx = nullptr;
+  float* part = nullptr;
+};
+
+// NORM: 0 none, 1 the backward goes on through the norm, 2 and forms the sums for its weight and bias.
+template <typename F, int KT, bool PAD, int NORM>
 __global__ void __launch_bounds__(512, 2)
     gate_bwd_two_kernel(const F* __restrict__ W1, const F* __restrict__ W2, int64_t ldw, const F* __restrict__ X1, const F* __restrict__ X2,
                         int64_t ldx, const F* __restrict__ bias1, const F* __restrict__ bias2, const F* __restrict__ mask,
                         const F* __restrict__ dC, int64_t ldc, F* __restrict__ dX1, F* __restrict__ dX2, int64_t lddx, F* __restrict__ dU,
-                        F* __restrict__ dV, int M, PairRows pairs) {
+                        F* __restrict__ dV, int M, PairRows pairs, NormAcross<F> norm) {
   constexpr int C = 32 * KT, K = 32 * KT, ROWB = 2 * K, NS = ROWB / 64, VPR = ROWB / 16;
   constexpr bool SWZ = KT == 4;  // (same layout of the weight rows as gate_bwd_input_res_kernel)
   constexpr int WSTR = SWZ ? ROWB : ROWB + 16, SSTR = ROWB + 16;
   auto swz = [](int row) -> int { return SWZ ? (((row & 3) << 2) | ((row >> 2) & 3)) : 0; };
   constexpr int NTH = 512, NWAVES = 8;
+  constexpr bool LNT = NORM > 0;
   extern __shared__ __align__(16) char gbi_dsm[];
   char* sw1 = gbi_dsm;
   char* sw2 = gbi_dsm + C * WSTR;
@@ -1765,6 +1791,7 @@ __global__ void __launch_bounds__(512, 2)
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, c = lane & 31, h = lane >> 5;
   char* stage = reinterpret_cast<char*>(sb + 2 * C) + wave * (32 * SSTR);
+  float* sg = reinterpret_cast<float*>(gbi_dsm + 2 * C * WSTR + 8 * C + NWAVES * 32 * SSTR);  // (LNT only) gamma[K]
 
   for (int e0 = tid; e0 < C * VPR; e0 += 4 * NTH) {
     u32x4_t w1[4], w2[4];
@@ -1786,6 +1813,9 @@ __global__ void __launch_bounds__(512, 2)
   for (int i = tid; i < C; i += NTH) {
     sb[i] = bias1 ? tri_load(bias1, i) : 0.f;
     sb[C + i] = bias2 ? tri_load(bias2, i) : 0.f;
+  }
+  if constexpr (LNT) {
+    for (int i = tid; i < K; i += NTH) sg[i] = norm.gamma ? tri_load(norm.gamma, i) : 1.f;
   }
   __syncthreads();
 
@@ -1818,19 +1848,27 @@ __global__ void __launch_bounds__(512, 2)
         xf2[s2][q] = *reinterpret_cast<const uint4*>(X2 + o);
       }
     bool live;
-    if (mask) mraw = raw16(mask[PAD ? pairs.near(mld, live) : mld]);
+    if (!LNT && mask) mraw = raw16(mask[PAD ? pairs.near(mld, live) : mld]);
   };
-  // (tiles dealt out wavefront-major: the last round of a ragged number of them runs on all compute units)
-  int64_t tile = static_cast<int64_t>(wave) * gridDim.x + blockIdx.x;
-  if (tile >= ntiles) return;
-  request_x(tile_row(tile));
-  pofs = dc_lane_offset(tile_row(tile));
-  request_dc(0);
+  // (tiles dealt out wavefront-major: the last round of a ragged number of them runs on all compute units; across d, the two tiles of
+  // 64 bytes that share the lines of the norm's input and its gradient go to neighbouring wavefronts)
+  constexpr int kNear = LNT ? 2 : 1;
+  int64_t tile = (static_cast<int64_t>(wave / kNear) * gridDim.x + blockIdx.x) * kNear + wave % kNear;
+  if (tile < ntiles) {
+    request_x(tile_row(tile));
+    pofs = dc_lane_offset(tile_row(tile));
+    request_dc(0);
+  }
+  const uint32_t pair_sel = (lane & 1) ? 0x03020706u : 0x05040100u;  // (as in gate_bwd_input_res_kernel)
+  auto of_pair = [&](uint32_t own) -> uint32_t {
+    return __builtin_amdgcn_perm(static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(own), 0xB1, 0xF, 0xF, true)), own, pair_sel);
+  };
+  float sum_g[KT] = {}, sum_b[KT] = {};  // (NORM == 2) of value 32 ds + 8 (c >> 3) + 4 h + ((c >> 1) & 3), over the tiles of the wavefront
 
   for (; tile < ntiles; tile += tstep) {
     const int mrow0 = static_cast<int>(tile * 32), mcol = mrow0 + c;
     const int next = tile_row(min(tile + tstep, ntiles - 1));  // (past the end: the last tile again, so that requests are unconditional)
-    const float mk = mask ? lo16<F>(mraw) : 1.0f;
+    const float mk = !LNT && mask ? lo16<F>(mraw) : 1.0f;  // (LNT: the output stage has none)
     const uint32_t real = (PAD && pairs.src(min(mcol, M - 1)) < 0) ? 0u : ~0u;  // (padding has no cotangent)
     uint32_t pu[KT][8], pv[KT][8];
 #pragma unroll
@@ -1849,12 +1887,14 @@ __global__ void __launch_bounds__(512, 2)
         au[4 * a] = b1.x; au[4 * a + 1] = b1.y; au[4 * a + 2] = b1.z; au[4 * a + 3] = b1.w;
         av[4 * a] = b2.x; av[4 * a + 1] = b2.y; av[4 * a + 2] = b2.z; av[4 * a + 3] = b2.w;
       }
-      const int wrow = (c0 + c) * WSTR;
+      // (addresses within the local data share are formed where they are used: kept over the tiles they would take the registers)
+      const int lw = static_cast<int>(again(static_cast<uint32_t>(lane))), cw = lw & 31, hw = lw >> 5;
+      const int wrow = (c0 + cw) * WSTR;
 #pragma unroll
       for (int s2 = 0; s2 < NS; ++s2)
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
-          const int wo = wrow + ((((2 * h + q) ^ swz(c)) << 4) ^ (s2 << 6));
+          const int wo = wrow + ((((2 * hw + q) ^ swz(cw)) << 4) ^ (s2 << 6));
           mma_step<F>(au, *reinterpret_cast<const uint4*>(sw1 + wo), xf1[s2][q]);
           mma_step<F>(av, *reinterpret_cast<const uint4*>(sw2 + wo), xf2[s2][q]);
         }
@@ -1878,7 +1918,26 @@ __global__ void __launch_bounds__(512, 2)
     // whole rows of what the wavefront has staged
     auto flush = [&](F* to, int64_t ld) {
       __builtin_amdgcn_wave_barrier();
-      stage_flush<F, K>(stage, SSTR, min(32, M - mrow0), to + static_cast<int64_t>(mrow0) * ld, ld, lane, 64, false);
+      F* rows = to + static_cast<int64_t>(mrow0) * ld;
+      if (64 % VPR == 0 && mrow0 + 32 <= M) {  // (whole rows to an instruction)
+        const int lf = static_cast<int>(again(static_cast<uint32_t>(lane)));
+        uint4 val[VPR / 2];
+#pragma unroll
+        for (int i = 0; i < VPR / 2; ++i) {
+          const int idx = lf + 64 * i;
+          val[i] = *reinterpret_cast<const uint4*>(stage + idx / VPR * SSTR + idx % VPR * 16);
+        }
+        // (one scalar base that walks down the rows, one offset a lane)
+        const char* base = uniform_ptr(rows);
+        const uint32_t ofs = static_cast<uint32_t>(lf / VPR * ld * 2 + lf % VPR * 16);
+#pragma unroll
+        for (int i = 0; i < VPR / 2; ++i) {
+          store_global(base, ofs, u32x4_t{val[i].x, val[i].y, val[i].z, val[i].w});
+          base += 64 / VPR * ld * 2;
+        }
+      } else {
+        stage_flush<F, K>(stage, SSTR, min(32, M - mrow0), rows, ld, lane, 64, false);
+      }
       __builtin_amdgcn_wave_barrier();
     };
     if (dU != nullptr) {
@@ -1894,17 +1953,38 @@ __global__ void __launch_bounds__(512, 2)
         flush(which == 0 ? dU : dV, ldc);
       }
     }
-    request_x(next);
+    if constexpr (NORM < 2) request_x(next);
 #pragma unroll
     for (int which = 0; which < 2; ++which) {
       const char* sw = which == 0 ? sw1 : sw2;
+      // the norm's input, four rows of a column pair a request: the even lane of row 2 j, the odd lane of row 2 j + 1
+      uint32_t tr[LNT ? KT : 1][8];
+      float mu = 0.f, rs = 0.f;
+      const uint32_t pair_ofs = static_cast<uint32_t>(((4 * h + (lane & 1)) * static_cast<int64_t>(M) + (min(c, M - 1 - mrow0) & ~1)) * 2);
+      const int64_t rows2 = 4 * static_cast<int64_t>(M);  // bytes of two rows
+      if constexpr (LNT) {
+        if (which == 1) {
+          // (one scalar base that starts at the tile and walks down the rows: bases of their own would not fit the scalar registers)
+          const char* from = uniform_ptr(norm.x + mrow0);
+#pragma unroll
+          for (int ds = 0; ds < KT; ++ds)
+#pragma unroll
+            for (int v = 0; v < 8; ++v) {
+              tr[ds][v] = load_global<uint32_t>(from, pair_ofs);
+              from += v % 2 ? 3 * rows2 : rows2;
+              __builtin_amdgcn_sched_barrier(0);
+            }
+          mu = norm.mean[min(mcol, M - 1)];
+          rs = norm.rstd[min(mcol, M - 1)];
+        }
+      }
       floatx16 ax[KT];
 #pragma unroll
       for (int t = 0; t < KT; ++t) ax[t] = floatx16{0};
       typedef shortx4_t __attribute__((address_space(3))) * lptr;
-      const int s16 = lane & 15, g16 = (lane >> 4) & 1;
+      const int lt = static_cast<int>(again(static_cast<uint32_t>(lane))), s16 = lt & 15, g16 = (lt >> 4) & 1;
       // rows 4 h + (s16 >> 2) (+ 8, + 16 t): a row 8 further flips bit 1 of the swizzle, 16 further leaves it
-      const int trow = 4 * h + (s16 >> 2), tunit = 2 * g16 + ((s16 & 3) >> 1);
+      const int trow = 4 * (lt >> 5) + (s16 >> 2), tunit = 2 * g16 + ((s16 & 3) >> 1);
       const int ulo = (tunit ^ swz(trow)) << 4, uhi = SWZ ? (ulo ^ 32) : ulo;
 #pragma unroll
       for (int ci = 0; ci < KT; ++ci) {
@@ -1921,6 +2001,63 @@ __global__ void __launch_bounds__(512, 2)
           }
         __builtin_amdgcn_sched_barrier(0);
       }
+      if constexpr (LNT) {
+        if (which == 1) {
+          // dx = rstd (g - mean(g) - xn mean(g xn)) with g = dy gamma, xn = (x - mean) rstd, over the K values of the column
+          float s1 = 0.f, s2 = 0.f;
+#pragma unroll
+          for (int ds = 0; ds < KT; ++ds) {
+            float xn[16];
+#pragma unroll
+            for (int v = 0; v < 16; v += 2) {
+              const uint32_t w = tr[ds][v >> 1] = of_pair(tr[ds][v >> 1]);
+              xn[v] = (lo16<F>(w) - mu) * rs;
+              xn[v + 1] = (hi16<F>(w) - mu) * rs;
+            }
+            if constexpr (NORM == 2) {  // (past the end: the last column again, left out)
+              float sum[16];
+#pragma unroll
+              for (int v = 0; v < 16; ++v) sum[v] = mcol < M ? ax[ds][v] * xn[v] : 0.f;
+              sum_g[ds] += half_wave_sums16(sum, lane);
+              __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+              for (int v = 0; v < 16; ++v) sum[v] = mcol < M ? ax[ds][v] : 0.f;
+              sum_b[ds] += half_wave_sums16(sum, lane);
+              __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int a = 0; a < 4; ++a) {
+              const float4 g4 = *reinterpret_cast<const float4*>(sg + ds * 32 + 8 * a + 4 * h);
+              const float gm[4] = {g4.x, g4.y, g4.z, g4.w};
+#pragma unroll
+              for (int b = 0; b < 4; ++b) {
+                const float g = ax[ds][4 * a + b] * gm[b];
+                s1 += g;
+                s2 = fmaf(g, xn[4 * a + b], s2);
+                ax[ds][4 * a + b] = g;
+              }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          if constexpr (NORM == 2) request_x(next);  // (no registers are left for them before)
+          s1 = (s1 + __shfl_xor(s1, 32, 64)) * (1.0f / K);
+          s2 = (s2 + __shfl_xor(s2, 32, 64)) * (1.0f / K);
+          if (mcol < M) {  // (M is even: a column pair is in or out as a whole)
+            const char* to = uniform_ptr(norm.dx + mrow0);
+#pragma unroll
+            for (int ds = 0; ds < KT; ++ds)
+#pragma unroll
+              for (int v = 0; v < 16; v += 2) {
+                const uint32_t w = again(tr[ds][v >> 1]);
+                const float x0 = (lo16<F>(w) - mu) * rs, x1 = (hi16<F>(w) - mu) * rs;
+                store_global(to, pair_ofs, of_pair(pack16<F>(rs * (ax[ds][v] - s1 - x0 * s2), rs * (ax[ds][v + 1] - s1 - x1 * s2))));
+                to += v % 4 ? 3 * rows2 : rows2;
+                __builtin_amdgcn_sched_barrier(0);
+              }
+          }
+          continue;
+        }
+      }
 #pragma unroll
       for (int ds = 0; ds < KT; ++ds)
 #pragma unroll
@@ -1928,6 +2065,25 @@ __global__ void __launch_bounds__(512, 2)
           *reinterpret_cast<uint2*>(stage + c * SSTR + (ds * 32 + 8 * a + 4 * h) * 2) =
               make_uint2(pack16<F>(ax[ds][4 * a], ax[ds][4 * a + 1]), pack16<F>(ax[ds][4 * a + 2], ax[ds][4 * a + 3]));
       flush(which == 0 ? dX1 : dX2, lddx);
+    }
+  }
+  if constexpr (NORM == 2) {
+    // the wavefronts' sums, in order, through the staging tiles
+    float* mine = reinterpret_cast<float*>(stage);
+    if ((lane & 1) == 0) {
+#pragma unroll
+      for (int ds = 0; ds < KT; ++ds) {
+        const int k = ds * 32 + 8 * (c >> 3) + 4 * h + ((c >> 1) & 3);
+        mine[k] = sum_g[ds];
+        mine[K + k] = sum_b[ds];
+      }
+    }
+    __syncthreads();
+    for (int i = tid; i < 2 * K; i += NTH) {
+      float s = 0.f;
+#pragma unroll
+      for (int w = 0; w < NWAVES; ++w) s += reinterpret_cast<const float*>(reinterpret_cast<char*>(sb + 2 * C) + w * (32 * SSTR))[i];
+      norm.part[(static_cast<int64_t>(i / K) * gridDim.x + blockIdx.x) * K + i % K] = s;
     }
   }
 }
@@ -3559,12 +3715,22 @@ extern "C" int cueq_ln_dual_gate(int32_t dtype, int64_t C, int64_t M, int64_t K,
 }
 
 // ln_x != NULL: the LayerNorm backward in the same kernel (cueq_gate_bwd_input_ln)
+// the LayerNorm across d (its weight may be null) that a two-input call with C = K goes on through; the gradients of its weight and
+// bias, where wanted, in float32 through partial sums of a block ([2][(M + 63) / 64 or as many as there are compute units][K])
+struct GateNorm {
+  const void* x;
+  const float *mean, *rstd;
+  const void* gamma;
+  void* dx;
+  float *dgamma, *dbeta, *part;
+};
+
 static int gate_bwd_input_impl(int32_t dtype, int64_t C, int64_t M, int64_t K, const void* W1, const void* W2, int64_t ldw,
                                const void* X1, const void* X2, int64_t ldx,
                                const void* bias1, const void* bias2, const void* mask, const void* dC, int64_t ldc,
                                int32_t dc_by_row, void* dX1, void* dX2, int64_t lddx, int32_t accumulate, void* dU, void* dV,
                                const void* ln_x, int64_t ldlx, const float* ln_mean, const float* ln_rstd, const void* ln_gamma, void* stream_,
-                               void* dres = nullptr, PairRows pairs = PairRows()) {
+                               void* dres = nullptr, PairRows pairs = PairRows(), const GateNorm* norm = nullptr) {
   hipStream_t stream = static_cast<hipStream_t>(stream_);
   CUEQ_REQUIRE(is_io(dtype), CUEQ_ERR_UNSUPPORTED, "gate_bwd_input: dtype must be float32 or bfloat16");
   CUEQ_REQUIRE(C >= 0 && M >= 0 && K > 0, CUEQ_ERR_INVALID, "gate_bwd_input: bad extents");
@@ -3588,6 +3754,7 @@ static int gate_bwd_input_impl(int32_t dtype, int64_t C, int64_t M, int64_t K, c
   const int64_t es = bf ? 2 : 4;
   if (!dc_by_row && ldc > 0 && (M * ldc + 8) * es >= (1ll << 32)) {
     // dC (M x C) is addressed with 32-bit byte offsets from a uniform base: more rows go in slabs (rows are independent)
+    CUEQ_REQUIRE(!norm, CUEQ_ERR_TOO_LARGE, "gate_bwd_input: too many rows to go on through the LayerNorm across d");
     const int64_t slab = (((1ll << 32) / es - 8) / ldc) & ~int64_t(255);
     CUEQ_REQUIRE(slab > 0, CUEQ_ERR_TOO_LARGE, "gate_bwd_input: row stride of dC too large");
     auto rows = [&](const void* p, int64_t ld, int64_t r0) { return p ? static_cast<const void*>(static_cast<const char*>(p) + r0 * ld * es) : nullptr; };
@@ -3615,14 +3782,22 @@ static int gate_bwd_input_impl(int32_t dtype, int64_t C, int64_t M, int64_t K, c
       // (as many weight rows as columns: two wavefronts to a SIMD, 77 us where one takes 111; the gate gradients of more rows than columns
       // would not stay in the registers)
       if (split && C == K) {
-        const size_t two = static_cast<size_t>(2 * C * (K == 128 ? 2 * K : 2 * K + 16) + 8 * C + 8 * 32 * (2 * K + 16));
-        const int64_t gt = std::min<int64_t>(ntiles, device_cus());
-#define GBT_F(FT, KT, PD) do { auto kfn = gate_bwd_two_kernel<FT, KT, PD>; \
+        const size_t two = static_cast<size_t>(2 * C * (K == 128 ? 2 * K : 2 * K + 16) + 8 * C + 8 * 32 * (2 * K + 16) + 4 * K);
+        const int64_t gt = std::min<int64_t>(norm ? (ntiles + 1) / 2 : ntiles, device_cus());
+#define GBT_F(FT, KT, PD, NA) do { auto kfn = gate_bwd_two_kernel<FT, KT, PD, NA>; \
+        NormAcross<FT> na; \
+        if (norm) na = {static_cast<const FT*>(norm->x), norm->mean, norm->rstd, static_cast<const FT*>(norm->gamma), static_cast<FT*>(norm->dx), norm->part}; \
         CUEQ_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kfn), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(two))); \
-        hipLaunchKernelGGL(kfn, dim3(static_cast<unsigned>(gt)), dim3(512), two, stream, static_cast<const FT*>(W1), static_cast<const FT*>(W2), ldw, static_cast<const FT*>(X1), static_cast<const FT*>(X2), ldx, static_cast<const FT*>(bias1), static_cast<const FT*>(bias2), static_cast<const FT*>(mask), static_cast<const FT*>(dC), ldc, static_cast<FT*>(dX1), static_cast<FT*>(dX2), lddx, static_cast<FT*>(dU), static_cast<FT*>(dV), static_cast<int>(M), pairs); } while (0)
-#define GBT(KT, PD) do { if (half) GBT_F(f16bits, KT, PD); else GBT_F(uint16_t, KT, PD); } while (0)
-        if (pairs.np) { if (K == 64) GBT(2, true); else GBT(4, true); }
-        else switch (K / 32) { case 1: GBT(1, false); break; case 2: GBT(2, false); break; case 3: GBT(3, false); break; default: GBT(4, false); break; }
+        hipLaunchKernelGGL(kfn, dim3(static_cast<unsigned>(gt)), dim3(512), two, stream, static_cast<const FT*>(W1), static_cast<const FT*>(W2), ldw, static_cast<const FT*>(X1), static_cast<const FT*>(X2), ldx, static_cast<const FT*>(bias1), static_cast<const FT*>(bias2), static_cast<const FT*>(mask), static_cast<const FT*>(dC), ldc, static_cast<FT*>(dX1), static_cast<FT*>(dX2), lddx, static_cast<FT*>(dU), static_cast<FT*>(dV), static_cast<int>(M), pairs, na); } while (0)
+#define GBT(KT, PD, NA) do { if (half) GBT_F(f16bits, KT, PD, NA); else GBT_F(uint16_t, KT, PD, NA); } while (0)
+#define GBN(NA) do { if (pairs.np) { if (K == 64) GBT(2, true, NA); else GBT(4, true, NA); } else { if (K == 64) GBT(2, false, NA); else GBT(4, false, NA); } } while (0)
+        if (norm && (norm->dgamma || norm->dbeta)) {  // (K = 64 or 128, no mask: the caller checks)
+          GBN(2);
+          hipLaunchKernelGGL(fold_two_kernel, dim3(static_cast<unsigned>((K + 15) / 16), 2), dim3(1024), 0, stream, norm->part, norm->dgamma, norm->dbeta, gt, K);
+        } else if (norm) { GBN(1);
+        } else if (pairs.np) { if (K == 64) GBT(2, true, 0); else GBT(4, true, 0); }
+        else switch (K / 32) { case 1: GBT(1, false, 0); break; case 2: GBT(2, false, 0); break; case 3: GBT(3, false, 0); break; default: GBT(4, false, 0); break; }
+#undef GBN
 #undef GBT
 #undef GBT_F
         CUEQ_CHECK_HIP(hipGetLastError());
@@ -3658,6 +3833,7 @@ static int gate_bwd_input_impl(int32_t dtype, int64_t C, int64_t M, int64_t K, c
     }
   }
   CUEQ_REQUIRE(!pairs.np, CUEQ_ERR_UNSUPPORTED, "gate_bwd_input: padded rows need the resident weights");
+  CUEQ_REQUIRE(!norm, CUEQ_ERR_UNSUPPORTED, "gate_bwd_input: the LayerNorm across d needs the resident weights");
   CUEQ_REQUIRE(!ln_x, CUEQ_ERR_UNSUPPORTED, "gate_bwd_input_ln: needs bfloat16, the weights fitting the local data share, an even M and ldc (compose cueq_gate_bwd_input and cueq_layer_norm_bwd otherwise)");
 #define GBI(TI, KT, SP) hipLaunchKernelGGL((gate_bwd_input_kernel<TI, KT, SP, !SP>), dim3(static_cast<unsigned>((M + gbi_threads<TI, SP>() / 2 - 1) / (gbi_threads<TI, SP>() / 2))), dim3(gbi_threads<TI, SP>()), 0, stream, static_cast<const TI*>(W1), static_cast<const TI*>(W2), ldw, static_cast<const TI*>(X1), static_cast<const TI*>(X2), ldx, static_cast<const TI*>(bias1), static_cast<const TI*>(bias2), static_cast<const TI*>(mask), static_cast<const TI*>(dC), ldc, static_cast<TI*>(dX1), static_cast<TI*>(dX2), lddx, accumulate, static_cast<TI*>(dU), static_cast<TI*>(dV), static_cast<int>(C), static_cast<int>(M))
 #define GBI_K(TI, SP) do { switch (K / 32) { case 1: GBI(TI, 1, SP); break; case 2: GBI(TI, 2, SP); break; case 3: GBI(TI, 3, SP); break; default: GBI(TI, 4, SP); break; } } while (0)
@@ -4363,7 +4539,15 @@ extern "C" int cueq_trimul_bwd_parts(int32_t dtype, int64_t B, int64_t N, int64_
 
   // output gate
   char *du2 = k.du2, *dv2 = k.du2 ? k.du2 + M * Do * es : nullptr;
-  if (D <= 128 && Do % 32 == 0) {
+  float *dgo = wants(kNoutW) ? g_nout : nullptr, *dbo = wants(kNoutB) ? g_nout + D : nullptr;
+  // and, where the result is as wide as the input, the LayerNorm across d in the same kernel (the gradient of its rows is not stored;
+  // 512 x 512 x 128, bfloat16: the two kernels 77 + 44 us, the one 108; 391 x 391 with all gradients 59 + 49 and 78)
+  const bool norm_fused = dtype != CUEQ_F32 && Do == D && (D == 64 || D == 128) && (M * D + 8) * es < (1ll << 32) && 6 * M * es < (1ll << 32);
+  if (norm_fused) {
+    const GateNorm norm{s.t, s.mean2, s.rstd2, w[kNoutW], k.dt, dgo, dbo, reinterpret_cast<float*>(k.ln)};
+    TRI_STEP(gate_bwd_input_impl(dtype, Do, M, D, w[kGoutW], w[kPoutW], D, s.xh, s.y, D, w[kGoutB], w[kPoutB], nullptr, dout, Do, 0, k.dxh, k.dy, D, 0,
+                                 w_out ? du2 : nullptr, w_out ? dv2 : nullptr, nullptr, 0, nullptr, nullptr, nullptr, stream_, nullptr, pairs, &norm));
+  } else if (D <= 128 && Do % 32 == 0) {
     TRI_STEP(gate_bwd_input_impl(dtype, Do, M, D, w[kGoutW], w[kPoutW], D, s.xh, s.y, D, w[kGoutB], w[kPoutB], nullptr, dout, Do, 0, k.dxh, k.dy, D, 0,
                                  w_out ? du2 : nullptr, w_out ? dv2 : nullptr, nullptr, 0, nullptr, nullptr, nullptr, stream_, nullptr, pairs));
   } else {
@@ -4392,8 +4576,9 @@ extern "C" int cueq_trimul_bwd_parts(int32_t dtype, int64_t B, int64_t N, int64_
   if (wants(kPoutB)) TRI_STEP(cueq_sum_rows(dtype, M, Do, dv2, g_out_b + Do, k.part, k.part_bytes, stream_));
 
   // LayerNorm across d
-  float *dgo = wants(kNoutW) ? g_nout : nullptr, *dbo = wants(kNoutB) ? g_nout + D : nullptr;
-  if (D <= kLnTMaxD) {
+  if (norm_fused) {
+    // (done with the gate)
+  } else if (D <= kLnTMaxD) {
     TRI_STEP(cueq_layer_norm_t_bwd(dtype, M, D, k.dy, s.t, s.mean2, s.rstd2, w[kNoutW], k.dt, dgo, dbo, k.ln, k.ln_bytes, stream_));
   } else {
     char* dtT = k.tT + M * D * es;

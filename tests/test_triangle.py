@@ -332,6 +332,24 @@ def test_defaults_shapes_and_errors(device):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("wanted", [(), ("norm_out_weight",), ("norm_out_bias", "g_out_weight")])
+@pytest.mark.parametrize("Bsz,N,D", [(1, 1, 64), (1, 4, 128), (1, 8, 64), (3, 24, 128), (1, 75, 128), (1, 264, 64)])
+def test_output_stage_backward_goes_on_through_its_norm(device, dtype, wanted, Bsz, N, D):
+    """D = 64 / 128 in 2-byte types: one tile of 32 rows of which some are padding, whole ones, and more tiles than wavefronts (264 x 264
+    rows are 2 178 for 2 048); with and without the sums for the norm's weight and bias and the gate gradients."""
+    from cuequivariance_amd import cuet
+
+    p, cot = make_case(Bsz, N, D, dtype, 1)
+    names = ["x", *wanted]
+    pr = {k: v.to(device).requires_grad_(k in names) for k, v in p.items()}
+    ref = torch.autograd.grad(oracle_trimul(direction="incoming", **pr), [pr[k] for k in names], cot.to(device))
+    pg = {k: v.detach().to(dtype).to(device).requires_grad_(k in names) for k, v in p.items()}
+    out = cuet.triangle_multiplicative_update(direction="incoming", **pg)
+    for k, got, want in zip(names, torch.autograd.grad(out, [pg[k] for k in names], cot.to(dtype).to(device)), ref):
+        assert got.shape == want.shape and rel_err(got, want.cpu()) <= TOL[dtype], (k, rel_err(got, want.cpu()))
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 def test_benchmark_size_against_oracle(device, dtype):
     """The benchmarked case itself (one 512 x 512 pair tensor, 128 channels, bfloat16 - and the same in half -, outgoing,
