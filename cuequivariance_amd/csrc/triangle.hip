@@ -1345,6 +1345,17 @@ __global__ void __launch_bounds__((gbi_threads<TI, SPLIT>()), (gbi_waves_per_sim
   }
 }
 
+// sums of v[0 .. 15] over the lanes of each half of a wavefront: lane c of a half returns that of v[c >> 1]
+__device__ __forceinline__ float half_wave_sums16(float (&v)[16], int lane) {
+#pragma unroll
+  for (int i = 0; i < 8; ++i) v[i] = lane_fold<16>(v[i], v[i + 8], lane);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v[i] = lane_fold<8>(v[i], v[i + 4], lane);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) v[i] = lane_fold<4>(v[i], v[i + 2], lane);
+  return lane_fold<1>(lane_fold<2>(v[0], v[1], lane));
+}
+
 // ------------------------------------------------------------------------------------------------
 // The same computation for 2-byte types with the weights resident in LDS: one block per CU loads W1, W2 (C rows)
 // and the biases once, then its wavefronts walk 32-column tiles of m independently - no barrier and no weight
@@ -1353,12 +1364,14 @@ __global__ void __launch_bounds__((gbi_threads<TI, SPLIT>()), (gbi_waves_per_sim
 //
 // LNB (one-input form): X1 holds the rows of a LayerNorm whose input rows, mean and 1 / std are given, and the kernel
 // goes on to the gradient with respect to those input rows - the lane has half of the gradient row in registers, so the two
-// row sums of the LayerNorm backward are sums over its own values completed by one exchange - and writes that to dX1.
+// row sums of the LayerNorm backward are sums over its own values completed by one exchange - and writes that to `dres`.  LNB = 2 also
+// forms a block's sums for the gradients of the norm's weight and bias (`ln_part`, [2][blocks][K]): the rows of a tile are lanes, added
+// by halving exchanges.
 //
 // PAD: the rows are those of a padded square (PairRows).  X and the gradients stay padded; dC by columns (the cotangent of
 // the update), the mask, the LayerNorm's input rows and, with LNB, the result `dres` are the caller's rows.
 // ------------------------------------------------------------------------------------------------
-template <typename F, int KT, bool SPLIT, bool DC_BY_ROW, bool LNB = false, bool PAD = false>
+template <typename F, int KT, bool SPLIT, bool DC_BY_ROW, int LNB = 0, bool PAD = false>
 __global__ void __launch_bounds__((SPLIT ? 256 : 512), (SPLIT ? 1 : 2))
     gate_bwd_input_res_kernel(const F* __restrict__ W1, const F* __restrict__ W2, int64_t ldw, const F* __restrict__ X1,
                               const F* __restrict__ X2, int64_t ldx, const F* __restrict__ bias1,
@@ -1366,8 +1379,9 @@ __global__ void __launch_bounds__((SPLIT ? 256 : 512), (SPLIT ? 1 : 2))
                               int64_t ldc, F* __restrict__ dX1, F* __restrict__ dX2, int64_t lddx, int accumulate,
                               F* __restrict__ dU, F* __restrict__ dV, int C, int M, const F* __restrict__ ln_x = nullptr,
                               int64_t ldlx = 0, const float* __restrict__ ln_mean = nullptr, const float* __restrict__ ln_rstd = nullptr,
-                              const F* __restrict__ ln_gamma = nullptr, F* __restrict__ dres = nullptr, PairRows pairs = PairRows()) {
-  static_assert(!(LNB && SPLIT), "the LayerNorm backward goes with the one-input form");
+                              const F* __restrict__ ln_gamma = nullptr, F* __restrict__ dres = nullptr, PairRows pairs = PairRows(),
+                              float* __restrict__ ln_part = nullptr) {
+  static_assert(LNB == 0 || !SPLIT, "the LayerNorm backward goes with the one-input form");
   using TI = F;
   constexpr int ES = 2, EPV = 8;
   constexpr int K = 32 * KT, ROWB = K * ES, NS = ROWB / 64, VPR = ROWB / 16;
@@ -1409,7 +1423,7 @@ __global__ void __launch_bounds__((SPLIT ? 256 : 512), (SPLIT ? 1 : 2))
     sb[i] = bias1 ? tri_load(bias1, i) : 0.f;
     sb[C + i] = bias2 ? tri_load(bias2, i) : 0.f;
   }
-  if constexpr (LNB) {
+  if constexpr (LNB > 0) {
     for (int i = tid; i < K; i += NTH) sg[i] = ln_gamma ? tri_load(ln_gamma, i) : 1.f;
   }
   __syncthreads();
@@ -1419,6 +1433,7 @@ __global__ void __launch_bounds__((SPLIT ? 256 : 512), (SPLIT ? 1 : 2))
   // v_perm_b32 selectors (bytes 0-3 = own register, 4-7 = the neighbour's): even lane (own.lo, other.lo), odd lane (other.hi, own.hi)
   const uint32_t pair_sel = (lane & 1) ? 0x03020706u : 0x05040100u;
   const int64_t tstep = static_cast<int64_t>(gridDim.x) * NWAVES;
+  const uint32_t du_ofs = DC_BY_ROW ? static_cast<uint32_t>(((4 * h + (lane & 1)) * ldc + (c & ~1)) * ES) : 0u;
   auto tile_row = [&](int64_t t) -> int { return static_cast<int>(min(t * 32 + c, static_cast<int64_t>(M) - 1)); };
 
   // cotangent values of a chunk, packed: register 2 a + j holds rows 8 a + 4 h + 2 j, + 1 of this lane's column.
@@ -1478,8 +1493,11 @@ __global__ void __launch_bounds__((SPLIT ? 256 : 512), (SPLIT ? 1 : 2))
         if constexpr (SPLIT) xf2[s2][q] = *reinterpret_cast<const uint4*>(X2 + o);
       }
     bool live;  // (padding: its cotangent is zero)
-    if (mask) mraw = raw16(mask[PAD ? pairs.near(mld, live) : mld]);
+    // (without a mask the first value of X, not used: a branch here would let the sums in front of it move behind it, into more registers)
+    const F* ms = mask ? mask : X1;
+    mraw = raw16(ms[again(static_cast<uint32_t>(PAD ? pairs.near(mld, live) : mld)) & (mask ? ~0u : 0u)]);
   };
+  float sum_g[KT] = {}, sum_b[KT] = {};  // (LNB = 2) of value 32 ds + 16 (c >> 4) + 8 h + ((c >> 1) & 7), over the tiles of the wavefront
   int64_t tile = ptile;
   if (tile < ntiles) request_x(tile_row(tile));
   request_dc(dcn);
@@ -1542,29 +1560,28 @@ __global__ void __launch_bounds__((SPLIT ? 256 : 512), (SPLIT ? 1 : 2))
         }
         pu[2 * a] = pack16<F>(du[0], du[1]); pu[2 * a + 1] = pack16<F>(du[2], du[3]);
         pv[2 * a] = pack16<F>(dv[0], dv[1]); pv[2 * a + 1] = pack16<F>(dv[2], dv[3]);
-        if (dU != nullptr) {
+      }
+      if (dU != nullptr && mcol < M) {
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
           const int row = c0 + 8 * a + 4 * h;
           if constexpr (!DC_BY_ROW) {
             // the lane's four rows are adjacent elements of its m row: one 8-byte store per array
-            if (mcol < M) {
-              const int64_t o = static_cast<int64_t>(mcol) * ldc + row;
-              *reinterpret_cast<uint2*>(dU + o) = make_uint2(pu[2 * a], pu[2 * a + 1]);
-              *reinterpret_cast<uint2*>(dV + o) = make_uint2(pv[2 * a], pv[2 * a + 1]);
-            }
+            const int64_t o = static_cast<int64_t>(mcol) * ldc + row;
+            *reinterpret_cast<uint2*>(dU + o) = make_uint2(pu[2 * a], pu[2 * a + 1]);
+            *reinterpret_cast<uint2*>(dV + o) = make_uint2(pv[2 * a], pv[2 * a + 1]);
           } else {
             // neighbouring lanes swap halves: the even lane stores rows 0 and 2 for columns (m, m + 1), the odd
-            // lane rows 1 and 3 for columns (m - 1, m) - 4-byte stores, 128 contiguous bytes per half-wave
+            // lane rows 1 and 3 for columns (m - 1, m) - 4-byte stores, 64 contiguous bytes per half-wave (M is even: a column pair
+            // is in or out as a whole)
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
               const uint32_t ou = pu[2 * a + j], ov = pv[2 * a + j];
               const uint32_t ru = static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(ou), 0xB1, 0xF, 0xF, true));
               const uint32_t rv = static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(ov), 0xB1, 0xF, 0xF, true));
-              const uint32_t wu = __builtin_amdgcn_perm(ru, ou, pair_sel), wv = __builtin_amdgcn_perm(rv, ov, pair_sel);
-              if (mcol < M) {
-                const int64_t o = static_cast<int64_t>(row + 2 * j + (lane & 1)) * ldc + (mcol & ~1);
-                *reinterpret_cast<uint32_t*>(dU + o) = wu;
-                *reinterpret_cast<uint32_t*>(dV + o) = wv;
-              }
+              const int64_t r = static_cast<int64_t>(c0 + 8 * a + 2 * j) * ldc * ES;
+              store_global(uniform_ptr(reinterpret_cast<const char*>(dU + mrow0) + r), du_ofs, __builtin_amdgcn_perm(ru, ou, pair_sel));
+              store_global(uniform_ptr(reinterpret_cast<const char*>(dV + mrow0) + r), du_ofs, __builtin_amdgcn_perm(rv, ov, pair_sel));
             }
           }
         }
@@ -1601,7 +1618,8 @@ __global__ void __launch_bounds__((SPLIT ? 256 : 512), (SPLIT ? 1 : 2))
     }
 
     // the rows of the next tile (past the end: the last tile again, so that the request is unconditional)
-    request_x(tile_row(min(tile + tstep, ntiles - 1)));
+    const int next = tile_row(min(tile + tstep, ntiles - 1));
+    if constexpr (LNB < 2) request_x(next);
     if constexpr (SPLIT) {
       // Results of the two-input form (one wavefront per SIMD, C other than K; nothing to add to): 8 rows (one value group a) at a time
       // through the wave-private staging tile, whole rows out as 16-byte vectors.  (The stores from registers of the
@@ -1636,7 +1654,7 @@ __global__ void __launch_bounds__((SPLIT ? 256 : 512), (SPLIT ? 1 : 2))
       // first, in the same shape, all of it at once.  All vectors are formed before the first of them is stored.
       const int mrow = mrow0 + c;
       const int64_t orow = static_cast<int64_t>(min(mrow, M - 1)) * lddx + (h * 16) / ES;
-      uint4 old[KT][2];
+      uint4 old[KT][2] = {};
       if (accumulate) {
 #pragma unroll
         for (int ds = 0; ds < KT; ++ds)
@@ -1644,7 +1662,7 @@ __global__ void __launch_bounds__((SPLIT ? 256 : 512), (SPLIT ? 1 : 2))
           for (int j = 0; j < 2; ++j) old[ds][j] = *reinterpret_cast<const uint4*>(dX1 + orow + (ds * 64 + j * 32) / ES);
       }
       uint4 val[KT][2];
-      if constexpr (LNB) {
+      if constexpr (LNB > 0) {
         // dx = rstd (g - mean(g) - xn mean(g xn)) with g = dy gamma, xn = (x - mean) rstd, over the K elements of the row.
         // The float accumulators are swapped into row order (k = 16 j + 8 h + e per 32 columns), what is added to them
         // and the LayerNorm's input rows arrive in the same order.
@@ -1668,23 +1686,48 @@ __global__ void __launch_bounds__((SPLIT ? 256 : 512), (SPLIT ? 1 : 2))
               acc[8 * j + i] = __uint_as_float(sw[0]);
               acc[8 * j + 4 + i] = __uint_as_float(sw[1]);
             }
+            const uint32_t ow[4] = {old[ds][j].x, old[ds][j].y, old[ds][j].z, old[ds][j].w};
+#pragma unroll
+            for (int e = 0; e < 8; ++e) acc[8 * j + e] += (e & 1) ? hi16<F>(ow[e >> 1]) : lo16<F>(ow[e >> 1]);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);  // (what was added is done with)
+#pragma unroll
+        for (int ds = 0; ds < KT; ++ds) {
+          floatx16& acc = ax1[ds];
+          auto xn = [&](int v) -> float {
+            const uint4 x = xr[ds][v >> 3];
+            const uint32_t w = (v >> 1 & 3) == 0 ? x.x : (v >> 1 & 3) == 1 ? x.y : (v >> 1 & 3) == 2 ? x.z : x.w;
+            return (((v & 1) ? hi16<F>(again(w)) : lo16<F>(again(w))) - mu) * rs;
+          };
+          if constexpr (LNB == 2) {
+            // (as a mask of bits: the compiler makes a branch of every conditional sum)
+            const uint32_t counts = mrow < M && (!PAD || xsrc >= 0) ? ~0u : 0u;
+            float sum[16];
+#pragma unroll
+            for (int v = 0; v < 16; ++v) sum[v] = __uint_as_float(__float_as_uint(acc[v] * xn(v)) & counts);
+            sum_g[ds] += half_wave_sums16(sum, lane);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int v = 0; v < 16; ++v) sum[v] = __uint_as_float(__float_as_uint(acc[v]) & counts);
+            sum_b[ds] += half_wave_sums16(sum, lane);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
             const int k0 = ds * 32 + j * 16 + h * 8;
             const float4 g0 = *reinterpret_cast<const float4*>(sg + k0), g1 = *reinterpret_cast<const float4*>(sg + k0 + 4);
             const float gm[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
-            const uint32_t ow[4] = {old[ds][j].x, old[ds][j].y, old[ds][j].z, old[ds][j].w};
-            const uint32_t xw[4] = {xr[ds][j].x, xr[ds][j].y, xr[ds][j].z, xr[ds][j].w};
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-              float d = acc[8 * j + e];
-              if (accumulate) d += (e & 1) ? hi16<F>(ow[e >> 1]) : lo16<F>(ow[e >> 1]);
-              const float g = d * gm[e];
-              const float xn = (((e & 1) ? hi16<F>(xw[e >> 1]) : lo16<F>(xw[e >> 1])) - mu) * rs;
+              const float g = acc[8 * j + e] * gm[e];
               s1 += g;
-              s2 = fmaf(g, xn, s2);
+              s2 = fmaf(g, xn(8 * j + e), s2);
               acc[8 * j + e] = g;
             }
           }
         }
+        if constexpr (LNB == 2) request_x(next);  // (no registers are left for them before)
         s1 = (s1 + __shfl_xor(s1, 32, 64)) * (1.0f / K);
         s2 = (s2 + __shfl_xor(s2, 32, 64)) * (1.0f / K);
 #pragma unroll
@@ -1718,7 +1761,7 @@ __global__ void __launch_bounds__((SPLIT ? 256 : 512), (SPLIT ? 1 : 2))
       }
       }
       __builtin_amdgcn_sched_barrier(0);
-      if constexpr (LNB) {
+      if constexpr (LNB > 0) {
         const int dst = mrow < M ? (PAD ? pairs.src(mrow) : mrow) : -1;
         if (dst >= 0) {
           F* to = dres + static_cast<int64_t>(dst) * lddx + (h * 16) / ES;
@@ -1736,6 +1779,26 @@ __global__ void __launch_bounds__((SPLIT ? 256 : 512), (SPLIT ? 1 : 2))
       __builtin_amdgcn_sched_barrier(0);
     }
   }
+  if constexpr (LNB == 2) {
+    // the wavefronts' sums, in order, where the weights were
+    __syncthreads();
+    float* sums = reinterpret_cast<float*>(gbi_dsm);
+    if ((lane & 1) == 0) {
+#pragma unroll
+      for (int ds = 0; ds < KT; ++ds) {
+        const int k = ds * 32 + 16 * (c >> 4) + 8 * h + ((c >> 1) & 7);
+        sums[wave * 2 * K + k] = sum_g[ds];
+        sums[wave * 2 * K + K + k] = sum_b[ds];
+      }
+    }
+    __syncthreads();
+    for (int i = tid; i < 2 * K; i += NTH) {
+      float s = 0.f;
+#pragma unroll
+      for (int w = 0; w < NWAVES; ++w) s += sums[w * 2 * K + i];
+      ln_part[(static_cast<int64_t>(i / K) * gridDim.x + blockIdx.x) * K + i % K] = s;
+    }
+  }
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1747,17 +1810,6 @@ __global__ void __launch_bounds__((SPLIT ? 256 : 512), (SPLIT ? 1 : 2))
 // Bound by its bytes (x, y, the cotangent, two gradients): 512 x 512 rows of 128, bfloat16, 111 -> 77 us = 4.4 TB/s; 392 x 392 rows of a
 // padded square with the gate gradients written out, 81 -> 59 us.
 // ------------------------------------------------------------------------------------------------
-// sums of v[0 .. 15] over the lanes of each half of a wavefront: lane c of a half returns that of v[c >> 1]
-__device__ __forceinline__ float half_wave_sums16(float (&v)[16], int lane) {
-#pragma unroll
-  for (int i = 0; i < 8; ++i) v[i] = lane_fold<16>(v[i], v[i + 8], lane);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) v[i] = lane_fold<8>(v[i], v[i + 4], lane);
-#pragma unroll
-  for (int i = 0; i < 2; ++i) v[i] = lane_fold<4>(v[i], v[i + 2], lane);
-  return lane_fold<1>(lane_fold<2>(v[0], v[1], lane));
-}
-
 // The LayerNorm across d whose rows are X2, for the backward that goes on through it: its input (D x M, D = K), statistics and weight,
 // where the gradient of the input goes (D x M), and, where those of its weight and bias are wanted, partial sums of a block
 // ([2][blocks][K]).
@@ -3725,12 +3777,19 @@ struct GateNorm {
   float *dgamma, *dbeta, *part;
 };
 
+// gradients of the weight and bias of the LayerNorm that a one-input call goes on through (either may be null), in float32, and room
+// for a block's partial sums ([2][ln_bwd_blocks or fewer][K])
+struct LnSums {
+  float *dgamma, *dbeta, *part;
+};
+
 static int gate_bwd_input_impl(int32_t dtype, int64_t C, int64_t M, int64_t K, const void* W1, const void* W2, int64_t ldw,
                                const void* X1, const void* X2, int64_t ldx,
                                const void* bias1, const void* bias2, const void* mask, const void* dC, int64_t ldc,
                                int32_t dc_by_row, void* dX1, void* dX2, int64_t lddx, int32_t accumulate, void* dU, void* dV,
                                const void* ln_x, int64_t ldlx, const float* ln_mean, const float* ln_rstd, const void* ln_gamma, void* stream_,
-                               void* dres = nullptr, PairRows pairs = PairRows(), const GateNorm* norm = nullptr) {
+                               void* dres = nullptr, PairRows pairs = PairRows(), const GateNorm* norm = nullptr,
+                               const LnSums* sums = nullptr) {
   hipStream_t stream = static_cast<hipStream_t>(stream_);
   CUEQ_REQUIRE(is_io(dtype), CUEQ_ERR_UNSUPPORTED, "gate_bwd_input: dtype must be float32 or bfloat16");
   CUEQ_REQUIRE(C >= 0 && M >= 0 && K > 0, CUEQ_ERR_INVALID, "gate_bwd_input: bad extents");
@@ -3806,23 +3865,27 @@ static int gate_bwd_input_impl(int32_t dtype, int64_t C, int64_t M, int64_t K, c
       // (tiles to the CUs first: 392 x 392 rows, one input, 109 us with the tiles of a block next to each other, 94 so - the second
       // round of 4 802 tiles on 2 048 wavefronts ran on a third of the CUs; 64 x 64 rows 30 and 21)
       const int64_t gx = std::min<int64_t>(split ? ntiles : (ntiles + 1) / 2, device_cus());
-#define GBR_F(FT, KT, SP, PD) do { auto kfn = gate_bwd_input_res_kernel<FT, KT, SP, !SP, false, PD>; \
+#define GBR_F(FT, KT, SP, PD) do { auto kfn = gate_bwd_input_res_kernel<FT, KT, SP, !SP, 0, PD>; \
         CUEQ_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kfn), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds))); \
-        hipLaunchKernelGGL(kfn, dim3(static_cast<unsigned>(gx)), dim3(SP ? 256 : 512), lds, stream, static_cast<const FT*>(W1), static_cast<const FT*>(W2), ldw, static_cast<const FT*>(X1), static_cast<const FT*>(X2), ldx, static_cast<const FT*>(bias1), static_cast<const FT*>(bias2), static_cast<const FT*>(mask), static_cast<const FT*>(dC), ldc, static_cast<FT*>(dX1), static_cast<FT*>(dX2), lddx, accumulate, static_cast<FT*>(dU), static_cast<FT*>(dV), static_cast<int>(C), static_cast<int>(M), static_cast<const FT*>(nullptr), int64_t(0), static_cast<const float*>(nullptr), static_cast<const float*>(nullptr), static_cast<const FT*>(nullptr), static_cast<FT*>(nullptr), pairs); } while (0)
+        hipLaunchKernelGGL(kfn, dim3(static_cast<unsigned>(gx)), dim3(SP ? 256 : 512), lds, stream, static_cast<const FT*>(W1), static_cast<const FT*>(W2), ldw, static_cast<const FT*>(X1), static_cast<const FT*>(X2), ldx, static_cast<const FT*>(bias1), static_cast<const FT*>(bias2), static_cast<const FT*>(mask), static_cast<const FT*>(dC), ldc, static_cast<FT*>(dX1), static_cast<FT*>(dX2), lddx, accumulate, static_cast<FT*>(dU), static_cast<FT*>(dV), static_cast<int>(C), static_cast<int>(M), static_cast<const FT*>(nullptr), int64_t(0), static_cast<const float*>(nullptr), static_cast<const float*>(nullptr), static_cast<const FT*>(nullptr), static_cast<FT*>(nullptr), pairs, nullptr); } while (0)
 #define GBR(KT, SP) do { if (half) GBR_F(f16bits, KT, SP, false); else GBR_F(uint16_t, KT, SP, false); } while (0)
 #define GBP(KT, SP) do { if (half) GBR_F(f16bits, KT, SP, true); else GBR_F(uint16_t, KT, SP, true); } while (0)
 #define GBR_K(SP) do { switch (K / 32) { case 1: GBR(1, SP); break; case 2: GBR(2, SP); break; case 3: GBR(3, SP); break; default: GBR(4, SP); break; } } while (0)
-#define GBL_F(FT, KT, PD) do { auto kfn = gate_bwd_input_res_kernel<FT, KT, false, true, true, PD>; \
+#define GBL_F(FT, KT, PD, SUMS) do { auto kfn = gate_bwd_input_res_kernel<FT, KT, false, true, SUMS, PD>; \
         CUEQ_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kfn), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds))); \
-        hipLaunchKernelGGL(kfn, dim3(static_cast<unsigned>(gx)), dim3(512), lds, stream, static_cast<const FT*>(W1), static_cast<const FT*>(W2), ldw, static_cast<const FT*>(X1), static_cast<const FT*>(X2), ldx, static_cast<const FT*>(bias1), static_cast<const FT*>(bias2), static_cast<const FT*>(mask), static_cast<const FT*>(dC), ldc, static_cast<FT*>(dX1), static_cast<FT*>(dX2), lddx, accumulate, static_cast<FT*>(dU), static_cast<FT*>(dV), static_cast<int>(C), static_cast<int>(M), static_cast<const FT*>(ln_x), ldlx, ln_mean, ln_rstd, static_cast<const FT*>(ln_gamma), static_cast<FT*>(dres), pairs); } while (0)
-#define GBL(KT, PD) do { if (half) GBL_F(f16bits, KT, PD); else GBL_F(uint16_t, KT, PD); } while (0)
+        hipLaunchKernelGGL(kfn, dim3(static_cast<unsigned>(gx)), dim3(512), lds, stream, static_cast<const FT*>(W1), static_cast<const FT*>(W2), ldw, static_cast<const FT*>(X1), static_cast<const FT*>(X2), ldx, static_cast<const FT*>(bias1), static_cast<const FT*>(bias2), static_cast<const FT*>(mask), static_cast<const FT*>(dC), ldc, static_cast<FT*>(dX1), static_cast<FT*>(dX2), lddx, accumulate, static_cast<FT*>(dU), static_cast<FT*>(dV), static_cast<int>(C), static_cast<int>(M), static_cast<const FT*>(ln_x), ldlx, ln_mean, ln_rstd, static_cast<const FT*>(ln_gamma), static_cast<FT*>(dres), pairs, sums ? sums->part : nullptr); } while (0)
+#define GBL_S(KT, PD, SUMS) do { if (half) GBL_F(f16bits, KT, PD, SUMS); else GBL_F(uint16_t, KT, PD, SUMS); } while (0)
+#define GBL(KT, PD) do { if (sums) GBL_S(KT, PD, 2); else GBL_S(KT, PD, 1); } while (0)
       if (pairs.np) {  // (K = 64 or 128: the caller checks)
         if (ln_x) { if (K == 64) GBL(2, true); else GBL(4, true); }
         else if (split) { if (K == 64) GBP(2, true); else GBP(4, true); }
         else { if (K == 64) GBP(2, false); else GBP(4, false); }
       } else if (ln_x) { switch (K / 32) { case 1: GBL(1, false); break; case 2: GBL(2, false); break; case 3: GBL(3, false); break; default: GBL(4, false); break; } }
       else if (split) GBR_K(true); else GBR_K(false);
+      if (sums)
+        hipLaunchKernelGGL(fold_two_kernel, dim3(static_cast<unsigned>((K + 15) / 16), 2), dim3(1024), 0, stream, sums->part, sums->dgamma, sums->dbeta, gx, K);
 #undef GBL
+#undef GBL_S
 #undef GBL_F
 #undef GBR_K
 #undef GBP
@@ -4597,15 +4660,26 @@ extern "C" int cueq_trimul_bwd_parts(int32_t dtype, int64_t B, int64_t N, int64_
     TRI_STEP(cueq_gemm(dtype, dtype, 0, 1, np, np, np, a, np, sq, k.dt, np, sq, db, np, sq, D * B, 1.0, 0, stream_));
   }
 
-  // input gate and projections - and, when neither their weights nor the LayerNorm's ask for a gradient, the input LayerNorm in
-  // the same kernel
+  // input gate and projections and the input LayerNorm, in one kernel where the weights fit the local data share: no gradient of the
+  // norm's rows is stored and read again (391 x 391 x 128, bfloat16, all gradients: 94 + 26 us apart, 107 so)
   const bool affine_in = wants(kNinW) || wants(kNinB);
   char *du1 = k.du1, *dv1 = k.du1 ? k.du1 + 2 * M * D * es : nullptr;
   const bool ln_fused = dtype != CUEQ_F32 && D <= 128 && M % 2 == 0 && (4 * M + M) * es < (1ll << 32) &&
                         4 * D * (D == 128 ? 2 * D : 2 * D + 16) + 20 * D <= 160 * 1024;  // (what cueq_gate_bwd_input_ln takes, however many rows)
-  if (!w_in && !affine_in && ln_fused) {
-    TRI_STEP(gate_bwd_input_impl(dtype, 2 * D, M, D, w[kGinW], w[kPinW], D, s.xh, nullptr, D, w[kGinB], w[kPinB], mask, k.dab, M, 1,
-                                 k.dxh, nullptr, D, 1, nullptr, nullptr, x, D, s.mean1, s.rstd1, w[kNinW], stream_, dxt, pairs));
+  auto projections = [&]() -> int {  // their gradients
+    if (wants(kGinW) || wants(kPinW)) TRI_STEP(long_k(false, 4 * D, du1, M, 0, s.xh, 0, 1, g_in));  // (gate rows, then value rows)
+    if (wants(kGinB)) TRI_STEP(cueq_sum_cols(dtype, 2 * D, M, du1, g_in_b, stream_));
+    if (wants(kPinB)) TRI_STEP(cueq_sum_cols(dtype, 2 * D, M, dv1, g_in_b + 2 * D, stream_));
+    return CUEQ_OK;
+  };
+  // (rows that are not 16-byte aligned and ask for the norm's or the weights' gradients: a kernel of their own for the norm)
+  const bool x_aligned = ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(dxt)) & 15) == 0;
+  if (ln_fused && (x_aligned || !(w_in || affine_in))) {
+    const LnSums sums{wants(kNinW) ? g_nin : nullptr, wants(kNinB) ? g_nin + D : nullptr, reinterpret_cast<float*>(k.ln)};
+    TRI_STEP(gate_bwd_input_impl(dtype, 2 * D, M, D, w[kGinW], w[kPinW], D, s.xh, nullptr, D, w[kGinB], w[kPinB], mask, k.dab, M, 1, k.dxh, nullptr, D, 1,
+                                 w_in ? du1 : nullptr, w_in ? dv1 : nullptr, x, D, s.mean1, s.rstd1, w[kNinW], stream_, dxt, pairs, nullptr,
+                                 affine_in ? &sums : nullptr));
+    TRI_STEP(projections());
     if (p.copies) TRI_STEP(pair_copy(p, dxt, dx, D, kPairBack, stream));
   } else {
     if (D <= 128) {
@@ -4616,9 +4690,7 @@ extern "C" int cueq_trimul_bwd_parts(int32_t dtype, int64_t B, int64_t N, int64_
       TRI_STEP(cueq_gemm(dtype, dtype, 1, 1, M, D, 2 * D, du1, M, 0, w[kGinW], D, 0, k.dxh, D, 0, 1, 1.0, 1, stream_));
       TRI_STEP(cueq_gemm(dtype, dtype, 1, 1, M, D, 2 * D, dv1, M, 0, w[kPinW], D, 0, k.dxh, D, 0, 1, 1.0, 1, stream_));
     }
-    if (wants(kGinW) || wants(kPinW)) TRI_STEP(long_k(false, 4 * D, du1, M, 0, s.xh, 0, 1, g_in));  // (gate rows, then value rows)
-    if (wants(kGinB)) TRI_STEP(cueq_sum_cols(dtype, 2 * D, M, du1, g_in_b, stream_));
-    if (wants(kPinB)) TRI_STEP(cueq_sum_cols(dtype, 2 * D, M, dv1, g_in_b + 2 * D, stream_));
+    TRI_STEP(projections());
     TRI_STEP(layer_norm_bwd_impl(dtype, M, D, k.dxh, x, s.mean1, s.rstd1, w[kNinW], dxt, wants(kNinW) ? g_nin : nullptr, wants(kNinB) ? g_nin + D : nullptr,
                                  k.ln, k.ln_bytes, stream_, pairs));
     if (p.copies) TRI_STEP(pair_copy(p, dxt, dx, D, kPairBack, stream));

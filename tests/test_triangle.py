@@ -333,11 +333,11 @@ def test_defaults_shapes_and_errors(device):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("wanted", [(), ("norm_out_weight",), ("norm_out_bias", "g_out_weight")])
-@pytest.mark.parametrize("Bsz,N,D", [(1, 1, 64), (1, 4, 128), (1, 8, 64), (3, 24, 128), (1, 75, 128), (1, 264, 64)])
-def test_output_stage_backward_goes_on_through_its_norm(device, dtype, wanted, Bsz, N, D):
+@pytest.mark.parametrize("wanted", [(), ("norm_out_weight",), ("norm_out_bias", "g_out_weight"), ("norm_in_weight",), ("norm_in_bias", "p_in_weight")])
+@pytest.mark.parametrize("Bsz,N,D", [(1, 1, 64), (1, 4, 128), (1, 8, 64), (3, 24, 128), (1, 70, 96), (1, 75, 128), (1, 264, 64)])
+def test_backward_stages_go_on_through_their_norms(device, dtype, wanted, Bsz, N, D):
     """D = 64 / 128 in 2-byte types: one tile of 32 rows of which some are padding, whole ones, and more tiles than wavefronts (264 x 264
-    rows are 2 178 for 2 048); with and without the sums for the norm's weight and bias and the gate gradients."""
+    rows are 2 178 for 2 048); with and without the sums for a norm's weight and bias and the gate gradients."""
     from cuequivariance_amd import cuet
 
     p, cot = make_case(Bsz, N, D, dtype, 1)
