@@ -2157,13 +2157,19 @@ __global__ void __launch_bounds__(512, 2)
 // PAD: the rows are those of a padded square (PairRows).  LN: X and the mask are the caller's rows, padding takes the nearest one,
 // and its result is zero where the contraction runs over it.  ROWS: X and X2 are padded, the result goes to the caller's rows.
 // ------------------------------------------------------------------------------------------------
-template <typename F, int KT, bool LN, bool ROWS, bool PAD = false>
+// NORMT (with ROWS): X2 is the input of a LayerNorm across d, K x M.  A lane reads four-byte column pairs, the even one of a pair row
+// 2 j and the odd one row 2 j + 1; exchanged, they are the words of the operand.  The statistics are sums over the lane's own half of the
+// column completed by one exchange; the normalised rows are rounded, become the operand, and are stored (xhat, mean, rstd) for the
+// backward.  Rows of 128, bfloat16: the norm's kernel and this one 25 + 32 us for 392 x 392, the one 43; 32 + 56 and 86 for 512 x 512, where
+// all rows of x2 start on the same memory channels.
+template <typename F, int KT, bool LN, bool ROWS, bool PAD = false, bool NORMT = false>
 __global__ void __launch_bounds__(512, 2)
     dual_gate_res_kernel(const F* __restrict__ W1, const F* __restrict__ W2, int64_t ldw, const F* __restrict__ X,
                          const F* __restrict__ X2, int64_t ldx, const F* __restrict__ bias1, const F* __restrict__ bias2, const F* __restrict__ mask,
                          F* __restrict__ out, int64_t ldc, int C, int M, const F* __restrict__ gamma,
                          const F* __restrict__ beta, float eps, F* __restrict__ xhat, int64_t ldxh, float* __restrict__ mean,
                          float* __restrict__ rstd, PairRows pairs = PairRows()) {
+  static_assert(!NORMT || ROWS, "the LayerNorm across d is that of the second input");
   static_assert(!PAD || LN || ROWS, "padded rows go with the two stages of the triangle update");
   using TI = F;
   constexpr int ES = 2, EPV = 8;
@@ -2210,14 +2216,35 @@ __global__ void __launch_bounds__(512, 2)
         for (int q = 0; q < 2; ++q) {
           const int64_t o = static_cast<int64_t>(mld) * ldx + (s2 * 64 + h * 32 + q * 16) / ES;
           xn[t][s2][q] = *reinterpret_cast<const uint4*>(X + o);
-          if constexpr (ROWS) xn2[t][s2][q] = *reinterpret_cast<const uint4*>(X2 + o);
+          if constexpr (ROWS && !NORMT) xn2[t][s2][q] = *reinterpret_cast<const uint4*>(X2 + o);
         }
+      if constexpr (NORMT) {
+        const int m0 = static_cast<int>(tl * 32);
+        const uint32_t ofs = static_cast<uint32_t>(((16 * h + (lane & 1)) * static_cast<int64_t>(M) + (min(c, M - 1 - m0) & ~1)) * ES);
+        const int64_t rows2 = 2 * static_cast<int64_t>(M) * ES;
+        const char* from = uniform_ptr(X2 + m0);
+#pragma unroll
+        for (int s2 = 0; s2 < NS; ++s2) {
+#pragma unroll
+          for (int q = 0; q < 2; ++q) {
+            uint32_t w[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              w[e] = load_global<uint32_t>(from, ofs);
+              from += rows2;
+            }
+            xn2[t][s2][q] = make_uint4(w[0], w[1], w[2], w[3]);
+          }
+          from += 8 * rows2;  // (16 rows of the other half)
+        }
+      }
       if (mask) mraw[t] = raw16(mask[mld]);
     }
   };
   // (tiles dealt out wavefront-major: the tiles worked on at one time lie next to each other in memory and are spread over
   // all CUs - 3 us less per launch than with the eight tiles of a block next to each other)
-  const int64_t tile0 = static_cast<int64_t>(wave) * gridDim.x + blockIdx.x;
+  constexpr int kNear = NORMT ? 2 : 1;  // (the two tiles of 64 bytes that share the lines of a K x M operand go to neighbouring wavefronts)
+  const int64_t tile0 = (static_cast<int64_t>(wave / kNear) * gridDim.x + blockIdx.x) * kNear + wave % kNear;
   if (tile0 < ntiles) request_x(tile0);
   for (int e0 = tid; e0 < C * VPR; e0 += 4 * NTH) {
     u32x4_t w1[4], w2[4];
@@ -2240,7 +2267,7 @@ __global__ void __launch_bounds__(512, 2)
     sb[i] = bias1 ? tri_load(bias1, i) : 0.f;
     sb[C + i] = bias2 ? tri_load(bias2, i) : 0.f;
   }
-  if constexpr (LN) {
+  if constexpr (LN || NORMT) {
     for (int i = tid; i < K; i += NTH) {
       sg[i] = gamma ? tri_load(gamma, i) : 1.f;
       sg[K + i] = beta ? tri_load(beta, i) : 0.f;
@@ -2268,6 +2295,76 @@ __global__ void __launch_bounds__(512, 2)
       }
     }
     request_x(min(tile + tstep, ntiles - 1));  // (past the end: the last tile again, so that the request is unconditional)
+    if constexpr (NORMT) {
+      // (in the order of ln_t_fwd_cols_kernel: 16 values in sequence, pairs of these - the other one is in the lane 32 further -, pairs of pairs)
+      float part[NS];
+      auto total = [&]() -> float {
+        float p[NS];
+#pragma unroll
+        for (int s2 = 0; s2 < NS; ++s2) p[s2] = part[s2] + __shfl_xor(part[s2], 32, 64);
+        if constexpr (NS == 4) return (p[0] + p[1]) + (p[2] + p[3]);
+        else return p[0] + p[NS - 1];
+      };
+#pragma unroll
+      for (int s2 = 0; s2 < NS; ++s2) {
+        part[s2] = 0.f;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          uint32_t w[4] = {xf2[0][s2][q].x, xf2[0][s2][q].y, xf2[0][s2][q].z, xf2[0][s2][q].w};
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            w[e] = __builtin_amdgcn_perm(static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(w[e]), 0xB1, 0xF, 0xF, true)), w[e], pair_sel);
+            part[s2] += lo16<F>(w[e]);
+            part[s2] += hi16<F>(w[e]);
+          }
+          xf2[0][s2][q] = make_uint4(w[0], w[1], w[2], w[3]);
+        }
+      }
+      const float mu = total() * (1.0f / K);
+#pragma unroll
+      for (int s2 = 0; s2 < NS; ++s2) {
+        part[s2] = 0.f;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          const uint32_t w[4] = {again(xf2[0][s2][q].x), again(xf2[0][s2][q].y), again(xf2[0][s2][q].z), again(xf2[0][s2][q].w)};
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float c0 = lo16<F>(w[e]) - mu, c1 = hi16<F>(w[e]) - mu;
+            part[s2] = fmaf(c0, c0, part[s2]);
+            part[s2] = fmaf(c1, c1, part[s2]);
+          }
+        }
+      }
+      const float rs = rsqrtf(total() * (1.0f / K) + eps);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int s2 = 0; s2 < NS; ++s2)
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          const int k0 = s2 * 32 + h * 16 + q * 8;
+          const float4 g0 = *reinterpret_cast<const float4*>(sg + k0), g1 = *reinterpret_cast<const float4*>(sg + k0 + 4);
+          const float4 b0 = *reinterpret_cast<const float4*>(sg + K + k0), b1 = *reinterpret_cast<const float4*>(sg + K + k0 + 4);
+          const float gm[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w}, bt[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
+          const uint32_t w[4] = {again(xf2[0][s2][q].x), again(xf2[0][s2][q].y), again(xf2[0][s2][q].z), again(xf2[0][s2][q].w)};
+          uint32_t o[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            o[e] = pack16<F>((lo16<F>(w[e]) - mu) * rs * gm[2 * e] + bt[2 * e], (hi16<F>(w[e]) - mu) * rs * gm[2 * e + 1] + bt[2 * e + 1]);
+          xf2[0][s2][q] = make_uint4(o[0], o[1], o[2], o[3]);
+          __builtin_amdgcn_sched_barrier(0);  // one piece at a time: its gamma / beta values die here
+        }
+      if (mcol[0] < M && blockIdx.y == 0) {
+        F* to = xhat + static_cast<int64_t>(mcol[0]) * ldxh + h * 16;
+#pragma unroll
+        for (int s2 = 0; s2 < NS; ++s2)
+#pragma unroll
+          for (int q = 0; q < 2; ++q) *reinterpret_cast<uint4*>(to + s2 * 32 + q * 8) = xf2[0][s2][q];
+        if (h == 0) {
+          mean[mcol[0]] = mu;
+          rstd[mcol[0]] = rs;
+        }
+      }
+    }
     if constexpr (LN) {
       // The sums are formed in the order of the row kernel ln_fwd_rows8 - groups of eight elements summed in sequence,
       // then pairs, fours, eights of groups - so that both give the same bits: a group pair lives in one lane, the
@@ -3011,20 +3108,29 @@ __global__ void __launch_bounds__(256, 2) ln_t_fwd_cols_kernel(const F* __restri
   auto work = [&](const uint32_t (&xv)[H], int64_t tile) {
     asm volatile("" ::: "memory");  // gamma / beta are read from LDS again for every tile, not kept in 2 D registers
     const int64_t m0 = tile * 64;
-    float s0 = 0.f, s1 = 0.f;
+    // (sums of 16 values in sequence, then pairs of them, then pairs of pairs: the output gate, which takes large batches, has every
+    // other 16 in a lane and gives the same bits)
+    float p0[H / 16] = {}, p1[H / 16] = {};
+    auto tree = [](const float (&p)[H / 16]) -> float {
+      if constexpr (H == 64) return (p[0] + p[1]) + (p[2] + p[3]);
+      else return p[0] + p[1];
+    };
 #pragma unroll
-    for (int i = 0; i < H; ++i) { s0 += lo16<F>(xv[i]); s1 += hi16<F>(xv[i]); }
+    for (int i = 0; i < H; ++i) { p0[i / 16] += lo16<F>(xv[i]); p1[i / 16] += hi16<F>(xv[i]); }
+    float s0 = tree(p0), s1 = tree(p1);
     s0 += __shfl_xor(s0, 32, 64);
     s1 += __shfl_xor(s1, 32, 64);
     const float mu0 = s0 * (1.0f / D), mu1 = s1 * (1.0f / D);
-    float q0 = 0.f, q1 = 0.f;
+#pragma unroll
+    for (int b = 0; b < H / 16; ++b) { p0[b] = 0.f; p1[b] = 0.f; }
 #pragma unroll
     for (int i = 0; i < H; ++i) {
       const uint32_t w = again(xv[i]);
       const float c0 = lo16<F>(w) - mu0, c1 = hi16<F>(w) - mu1;
-      q0 = fmaf(c0, c0, q0);
-      q1 = fmaf(c1, c1, q1);
+      p0[i / 16] = fmaf(c0, c0, p0[i / 16]);
+      p1[i / 16] = fmaf(c1, c1, p1[i / 16]);
     }
+    float q0 = tree(p0), q1 = tree(p1);
     q0 += __shfl_xor(q0, 32, 64);
     q1 += __shfl_xor(q1, 32, 64);
     const float r0 = rsqrtf(q0 * (1.0f / D) + eps), r1 = rsqrtf(q1 * (1.0f / D) + eps);
@@ -3678,17 +3784,21 @@ static int launch_dual_gate_res(int64_t C, int64_t M, int64_t K, const void* W1,
   C /= parts;
   const size_t lds = dual_gate_res_lds(C, K, xhat != nullptr);
   const int64_t gx = std::min<int64_t>(ntiles, std::max<int64_t>(1, device_cus() / parts));
-#define DGR_F(FT, KT, LN, RW, PD) do { auto kfn = dual_gate_res_kernel<FT, KT, LN, RW, PD>; \
+#define DGR_F(FT, KT, LN, RW, ...) do { auto kfn = dual_gate_res_kernel<FT, KT, LN, RW, __VA_ARGS__>; \
     CUEQ_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kfn), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds))); \
     hipLaunchKernelGGL(kfn, dim3(static_cast<unsigned>(gx), static_cast<unsigned>(parts)), dim3(512), lds, stream, static_cast<const FT*>(W1), static_cast<const FT*>(W2), ldw, static_cast<const FT*>(X), static_cast<const FT*>(X2), ldx, static_cast<const FT*>(bias1), static_cast<const FT*>(bias2), static_cast<const FT*>(mask), static_cast<FT*>(out), ldc, static_cast<int>(C), static_cast<int>(M), static_cast<const FT*>(gamma), static_cast<const FT*>(beta), eps, static_cast<FT*>(xhat), ldxh, mean, rstd, pairs); } while (0)
 #define DGR(KT, LN, RW) do { if (half) DGR_F(f16bits, KT, LN, RW, false); else DGR_F(uint16_t, KT, LN, RW, false); } while (0)
 #define DGP(KT, LN, RW) do { if (half) DGR_F(f16bits, KT, LN, RW, true); else DGR_F(uint16_t, KT, LN, RW, true); } while (0)
 #define DGR_K(LN, RW) do { switch (K / 32) { case 1: DGR(1, LN, RW); break; case 2: DGR(2, LN, RW); break; case 3: DGR(3, LN, RW); break; default: DGR(4, LN, RW); break; } } while (0)
-  if (pairs.np) {  // (K = 64 or 128: the caller checks)
+#define DGN(KT, PD) do { if (half) DGR_F(f16bits, KT, false, true, PD, true); else DGR_F(uint16_t, KT, false, true, PD, true); } while (0)
+  if (by_rows && xhat) {  // (the LayerNorm across d; K = 64 or 128: the caller checks)
+    if (pairs.np) { if (K == 64) DGN(2, true); else DGN(4, true); } else { if (K == 64) DGN(2, false); else DGN(4, false); }
+  } else if (pairs.np) {  // (K = 64 or 128: the caller checks)
     if (by_rows) { if (K == 64) DGP(2, false, true); else DGP(4, false, true); }
     else { if (K == 64) DGP(2, true, false); else DGP(4, true, false); }
   } else if (by_rows) DGR_K(false, true); else if (xhat) DGR_K(true, false); else DGR_K(false, false);
 #undef DGR_K
+#undef DGN
 #undef DGP
 #undef DGR
 #undef DGR_F
@@ -4544,6 +4654,15 @@ extern "C" int cueq_trimul_fwd(int32_t dtype, int64_t B, int64_t N, int64_t D, i
   char* b = s.ab + M * D * p.es;
   // t[i, j] = sum_k a[i, k] b[j, k]  /  sum_k a[k, i] b[k, j]
   TRI_STEP(cueq_gemm(dtype, dtype, outgoing ? 0 : 1, outgoing ? 0 : 1, np, np, np, s.ab, np, sq, b, np, sq, s.t, np, sq, D * B, 1.0, 0, stream_));
+  void* to = p.copies ? k.outp : out;
+  // the LayerNorm across d: inside the output gate where the weights stay in the local data share
+  if (p.resident && (D == 64 || D == 128) && dual_gate_res_fits(Do, M, D, to, Do, true, true)) {
+    KernelTimer timer("dual_gate_fwd", stream);
+    TRI_STEP(launch_dual_gate_res(Do, M, D, w[kGoutW], w[kPoutW], D, s.xh, s.t, D, w[kGoutB], w[kPoutB], nullptr, to, Do, w[kNoutW], w[kNoutB],
+                                  static_cast<float>(eps), s.y, D, s.mean2, s.rstd2, dtype == CUEQ_F16, stream, p.mapped ? p.pairs : PairRows()));
+    if (p.copies) TRI_STEP(pair_copy(p, to, out, Do, kPairBack, stream));
+    return CUEQ_OK;
+  }
   if (D <= kLnTMaxD) {
     TRI_STEP(cueq_layer_norm_t_fwd(dtype, M, D, s.t, w[kNoutW], w[kNoutB], eps, s.y, s.mean2, s.rstd2, stream_));
   } else {
@@ -4556,7 +4675,6 @@ extern "C" int cueq_trimul_fwd(int32_t dtype, int64_t B, int64_t N, int64_t D, i
                                   nullptr, nullptr, dtype == CUEQ_F16, stream, p.pairs));
     return CUEQ_OK;
   }
-  void* to = p.copies ? k.outp : out;
   TRI_STEP(cueq_dual_gate(dtype, 0, M, Do, D, s.xh, s.y, D, w[kGoutW], w[kPoutW], D, w[kGoutB], w[kPoutB], 1, nullptr, 0, nullptr, to, nullptr, Do, stream_));
   if (p.copies) TRI_STEP(pair_copy(p, to, out, Do, kPairBack, stream));
   return CUEQ_OK;

@@ -333,6 +333,24 @@ def test_defaults_shapes_and_errors(device):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("Bsz,N,D,Do", [(1, 64, 128, 128), (1, 64, 64, 32), (2, 48, 128, 128), (1, 65, 64, 64), (1, 70, 128, 32), (1, 264, 128, 96)])
+def test_output_gate_normalises_across_d(device, dtype, Bsz, N, D, Do):
+    """From 4 096 rows on the norm across d runs in the output gate: the least number, tiles of padded squares, results narrower than the
+    input (with weight rows over several blocks), more tiles than wavefronts; what it keeps for the backward through the gradients."""
+    from cuequivariance_amd import cuet
+
+    p, cot = make_case(Bsz, N, D, dtype, 1, Do=Do)
+    names = ["x", "norm_out_weight", "p_out_weight"]
+    pr = {k: v.to(device).requires_grad_(k in names) for k, v in p.items()}
+    ref = oracle_trimul(direction="outgoing", **pr)
+    want = [ref, *torch.autograd.grad(ref, [pr[k] for k in names], cot.to(device))]
+    pg = {k: v.detach().to(dtype).to(device).requires_grad_(k in names) for k, v in p.items()}
+    out = cuet.triangle_multiplicative_update(direction="outgoing", **pg)
+    for k, got, w in zip(["out", *names], [out, *torch.autograd.grad(out, [pg[k] for k in names], cot.to(dtype).to(device))], want):
+        assert got.shape == w.shape and rel_err(got, w.detach().cpu()) <= TOL[dtype], (k, rel_err(got, w.detach().cpu()))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("wanted", [(), ("norm_out_weight",), ("norm_out_bias", "g_out_weight"), ("norm_in_weight",), ("norm_in_bias", "p_in_weight")])
 @pytest.mark.parametrize("Bsz,N,D", [(1, 1, 64), (1, 4, 128), (1, 8, 64), (3, 24, 128), (1, 70, 96), (1, 75, 128), (1, 264, 64)])
 def test_backward_stages_go_on_through_their_norms(device, dtype, wanted, Bsz, N, D):
