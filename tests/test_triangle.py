@@ -350,6 +350,7 @@ def test_output_gate_normalises_across_d(device, dtype, Bsz, N, D, Do):
         assert got.shape == w.shape and rel_err(got, w.detach().cpu()) <= TOL[dtype], (k, rel_err(got, w.detach().cpu()))
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("wanted", [(), ("norm_out_weight",), ("norm_out_bias", "g_out_weight"), ("norm_in_weight",), ("norm_in_bias", "p_in_weight")])
 @pytest.mark.parametrize("Bsz,N,D", [(1, 1, 64), (1, 4, 128), (1, 8, 64), (3, 24, 128), (1, 70, 96), (1, 75, 128), (1, 264, 64)])
@@ -368,6 +369,7 @@ def test_backward_stages_go_on_through_their_norms(device, dtype, wanted, Bsz, N
         assert got.shape == want.shape and rel_err(got, want.cpu()) <= TOL[dtype], (k, rel_err(got, want.cpu()))
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 def test_benchmark_size_against_oracle(device, dtype):
     """The benchmarked case itself (one 512 x 512 pair tensor, 128 channels, bfloat16 - and the same in half -, outgoing,
