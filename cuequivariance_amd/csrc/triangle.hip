@@ -3944,8 +3944,9 @@ static int gate_bwd_input_impl(int32_t dtype, int64_t C, int64_t M, int64_t K, c
     // weights resident in LDS when they fit (2 C rows of 2 K + 16 bytes, biases, with two inputs the staging tiles)
     const int nwaves = split ? 4 : 8;
     const size_t lds = static_cast<size_t>(2 * C * (K == 128 ? 2 * K : 2 * K + 16) + 8 * C + (split ? nwaves * 8 * (2 * K + 16) : 0) + (ln_x ? 4 * K : 0));
-    // (dC by rows is read, and the gate gradients written, as 4-byte column pairs)
-    const bool pairs_ok = !dc_by_row || (M % 2 == 0 && ldc % 2 == 0 && reinterpret_cast<uintptr_t>(dC) % 4 == 0);
+    // (dC by rows is read, and the gate gradients written, as 4-byte column pairs at lane offsets of up to five rows and a column - the
+    // other kernel's reach four rows and a column, which is what the check above admits)
+    const bool pairs_ok = !dc_by_row || (M % 2 == 0 && ldc % 2 == 0 && reinterpret_cast<uintptr_t>(dC) % 4 == 0 && (5 * ldc + M) * es < (1ll << 32));
     if (lds <= 160 * 1024 && pairs_ok) {
       const int64_t ntiles = (M + 31) / 32;
       // (as many weight rows as columns: two wavefronts to a SIMD, 77 us where one takes 111; the gate gradients of more rows than columns
@@ -4492,7 +4493,7 @@ struct TriPlan {
     const size_t bwd_out = static_cast<size_t>(2 * Do * (D == 128 ? 2 * D : 2 * D + 16) + 8 * Do + 32 * (2 * D + 16));
     const size_t bwd_in = static_cast<size_t>(4 * D * (D == 128 ? 2 * D : 2 * D + 16) + 16 * D + 4 * D);
     mapped = Np != N && resident && (D == 64 || D == 128) && Do % 32 == 0 && dual_gate_res_lds(Do, D, false) <= 160 * 1024 && bwd_out <= 160 * 1024 &&
-             bwd_in <= 160 * 1024 && (M * Do + 8) * es < (1ll << 32) && 5 * M * es < (1ll << 32);
+             bwd_in <= 160 * 1024 && (M * Do + 8) * es < (1ll << 32) && 6 * M * es < (1ll << 32);
     copies = Np != N && !mapped;
     if (Np != N && M < (1ll << 31)) pairs = PairRows::make(static_cast<int>(N), static_cast<int>(Np), !outgoing);
   }
@@ -4782,7 +4783,7 @@ extern "C" int cueq_trimul_bwd_parts(int32_t dtype, int64_t B, int64_t N, int64_
   // norm's rows is stored and read again (391 x 391 x 128, bfloat16, all gradients: 94 + 26 us apart, 107 so)
   const bool affine_in = wants(kNinW) || wants(kNinB);
   char *du1 = k.du1, *dv1 = k.du1 ? k.du1 + 2 * M * D * es : nullptr;
-  const bool ln_fused = dtype != CUEQ_F32 && D <= 128 && M % 2 == 0 && (4 * M + M) * es < (1ll << 32) &&
+  const bool ln_fused = dtype != CUEQ_F32 && D <= 128 && M % 2 == 0 && 6 * M * es < (1ll << 32) &&
                         4 * D * (D == 128 ? 2 * D : 2 * D + 16) + 20 * D <= 160 * 1024;  // (what cueq_gate_bwd_input_ln takes, however many rows)
   auto projections = [&]() -> int {  // their gradients
     if (wants(kGinW) || wants(kPinW)) TRI_STEP(long_k(false, 4 * D, du1, M, 0, s.xh, 0, 1, g_in));  // (gate rows, then value rows)

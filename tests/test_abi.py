@@ -96,6 +96,10 @@ def test_dense_entries_refuse_bad_arguments_before_any_launch():
     lnb = lambda dtype, lx, ldlx: lib.cueq_gate_bwd_input_ln(dtype, 256, 8192, 128, p, p, 128, p, 128, None, None, None, p, 8192, p, 128, 0, lx, ldlx, p, p,
                                                              None, None)
     assert lnb(F32, p, 128) == -2 and lnb(BF16, None, 128) == -1 and lnb(BF16, p + 8, 128) == -2 and lnb(BF16, p, 100) == -2
+    # ... and its lane offsets, up to five rows of dC and a column, within 32 bits (450 000 000: four rows of 2-byte elements are, five are not)
+    far = 450_000_000
+    assert lib.cueq_gate_bwd_input_ln(BF16, 64, 64, 64, p, p, 64, p, 64, None, None, None, p, far, p, 64, 0, p, 64, p, p, None, None) == -2
+    assert b"compose cueq_gate_bwd_input" in lib.cueq_last_error()
 
 
 
