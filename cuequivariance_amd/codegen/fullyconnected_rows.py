@@ -130,13 +130,12 @@ def flatten(rows: Rows):
     q = rows.polynomial.flatten_coefficient_modes()
     stp = q.operations[0][1]
     keep = stp.subscripts.operands[-1][-1]
-    q = q.flatten_modes([m for m in stp.subscripts.modes() if m != keep])
-    if rows.x1_mul_ir:
-        order, off = [], 0
-        for d, U in rows.polynomial.operations[0][1].operands[1].segments:
-            order += [off + i * U + u for u in range(U) for i in range(d)]
-            off += d * U
-        q = q.apply_fn(lambda ope, stp: (ope, stp.permute_segments(1, order)))
+    modes = [m for m in stp.subscripts.modes() if m != keep]
+    order, off = [], 0
+    for d, U in rows.polynomial.operations[0][1].operands[1].segments:
+        order += [off + i * U + u for u in range(U) for i in range(d)] if rows.x1_mul_ir else range(off, off + d * U)
+        off += d * U
+    q = q.apply_fn(lambda ope, stp: (ope, stp.flatten_modes(modes).permute_segments(1, order)))
     dims = [d for d, _ in rows.polynomial.operations[0][1].operands[-1].segments]
     return q, ({3: dims} if rows.out_mul_ir and any(d > 1 for d in dims) else {})
 

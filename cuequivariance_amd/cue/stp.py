@@ -179,6 +179,13 @@ class Path:
         c.setflags(write=False)
         self.coefficients = c
 
+    def renumbered(self, operand: int, where) -> "Path":
+        """Its segment ``s`` of ``operand`` is ``where[s]`` now (the coefficients, which are never written, are shared)."""
+        p = object.__new__(Path)
+        p.indices = self.indices[:operand] + (where[self.indices[operand]],) + self.indices[operand + 1:]
+        p.coefficients = self.coefficients
+        return p
+
     def __repr__(self):
         return f"Path({self.indices}, c.shape={self.coefficients.shape})"
 
@@ -506,6 +513,8 @@ class SegmentedTensorProduct:
 
     # ---------------------------------------------------------------- functional transforms
     def permute_operands(self, perm) -> "SegmentedTensorProduct":
+        if list(perm) == list(range(self.num_operands)):
+            return self.copy()  # (paths do not change once they are made)
         return self._replace(
             operands_and_subscripts=[self.operands_and_subscripts[i] for i in perm],
             paths=[p.permute_operands(perm) for p in self.paths],
@@ -530,14 +539,13 @@ class SegmentedTensorProduct:
         """New segment ``n`` is old segment ``perm[n]``; paths are relabelled, their order is kept."""
         operand = _canon(operand, self.num_operands, "operand")
         perm = list(perm)
+        if perm == list(range(self.operands[operand].num_segments)):
+            return self
         where = {old: new for new, old in enumerate(perm)}
         ops = list(self.operands_and_subscripts)
         ope, ss = ops[operand]
         ops[operand] = (ope.with_segments([ope[i] for i in perm]), ss)
-        paths = [
-            Path([s if o != operand else where[s] for o, s in enumerate(p.indices)], p.coefficients)
-            for p in self.paths
-        ]
+        paths = [p.renumbered(operand, where) for p in self.paths]
         return self._replace(operands_and_subscripts=ops, paths=paths)
 
     def sort_paths(self, operands_ordering=None) -> "SegmentedTensorProduct":

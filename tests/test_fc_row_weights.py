@@ -159,6 +159,28 @@ def test_tables_of_mul_ir_rows(ir1, ir2, ir3, in_mul_ir, out_mul_ir):
     assert [((w, moved[x1], x2, out), c) for (w, x1, x2, out), c in a] == [(tuple(i), c) for i, c in b]
 
 
+@pytest.mark.parametrize("ir1,ir2,ir3", MUL_IR_ROWS)
+def test_mul_ir_rows_are_flattened_at_the_cost_of_ir_mul_rows(ir1, ir2, ir3, monkeypatch):
+    """What the first call of a module pays for, one object per scalar path and pass over them, is the same in either order of the rows."""
+    from cuequivariance_amd.cue import stp
+
+    poly = descriptors.fully_connected_tensor_product(*(cue.Irreps("O3", s) for s in (ir1, ir2, ir3))).polynomial
+    made, init = [], stp.Path.__init__
+
+    def counted(self, indices, coefficients):
+        made.append(1)
+        init(self, indices, coefficients)
+
+    monkeypatch.setattr(stp.Path, "__init__", counted)
+
+    def count(rows):
+        made.clear()
+        fcr.flatten(rows)
+        return len(made)
+
+    assert count(fcr.Rows(poly, True, True)) == count(fcr.Rows(poly))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("indexed,deterministic", [(True, "0"), (True, "1"), (False, "0")])
 @pytest.mark.parametrize(
