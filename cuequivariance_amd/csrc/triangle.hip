@@ -3512,6 +3512,8 @@ template <typename F>
 static int gemm_direct(bool ta, bool tb, int64_t M, int64_t N, int64_t K, const void* A, int64_t lda, int64_t sA, const void* B, int64_t ldb, int64_t sB, void* C,
                        int64_t ldc, int64_t sC, int64_t batch, float alpha, hipStream_t stream) {
   const bool wide = M > 128 && N > 128 && ((M + 255) / 256) * ((N + 255) / 256) * batch >= device_cus();
+  constexpr bool half = std::is_same_v<F, f16bits>;
+  KernelTimer timer(wide ? (half ? "gemm_direct_f16_256" : "gemm_direct_bf16_256") : (half ? "gemm_direct_f16" : "gemm_direct_bf16"), stream);
   auto go = [&](auto a, auto b) {
     constexpr bool TA = decltype(a)::value, TB = decltype(b)::value;
     const F *pa = static_cast<const F*>(A), *pb = static_cast<const F*>(B);
@@ -3589,9 +3591,7 @@ extern "C" int cueq_gemm(int32_t in_dtype, int32_t out_dtype, int32_t trans_a, i
     const int64_t out_es = out_dtype == CUEQ_F32 ? 4 : 2;
     const int vec_out = (reinterpret_cast<uintptr_t>(C) % 16 == 0 && (ldc * out_es) % 16 == 0 && (stride_c * out_es) % 16 == 0) ? 1 : 0;
     // 256 x 256 tiles when both extents are multiples of 256 and there are enough of them to fill the chip
-    const bool big = !mixed && M % 256 == 0 && N % 256 == 0 && (M / 256) * (N / 256) * batch >= 2 * static_cast<int64_t>(device_cus());
-    // (the timing label says whether 256 x 256 tiles fill the chip twice, so a test can tell which kernel a shape ran on)
-    KernelTimer timer(in_dtype == CUEQ_F32 ? (big ? "gemm_nt_f32_256" : "gemm_nt_f32") : in_dtype == CUEQ_F16 ? (big ? "gemm_nt_f16_256" : "gemm_nt_f16") : (big ? "gemm_nt_bf16_256" : "gemm_nt_bf16"), stream);
+    const bool big = in_dtype == CUEQ_F32 && !mixed && M % 256 == 0 && N % 256 == 0 && (M / 256) * (N / 256) * batch >= 2 * static_cast<int64_t>(device_cus());
     // 2-byte operands and results of one type: straight into LDS, unless results are added to or their rows are not 16-byte pieces
     // (byte offsets inside an operand are 32 bits, tile numbers 31)
     const int64_t far = int64_t(1) << 31;
@@ -3600,6 +3600,8 @@ extern "C" int cueq_gemm(int32_t in_dtype, int32_t out_dtype, int32_t trans_a, i
       if (in_dtype == CUEQ_F16) return gemm_direct<f16bits>(trans_a != 0, trans_b != 0, M, N, K, A, lda, stride_a, B, ldb, stride_b, C, ldc, stride_c, batch, al, stream);
       return gemm_direct<uint16_t>(trans_a != 0, trans_b != 0, M, N, K, A, lda, stride_a, B, ldb, stride_b, C, ldc, stride_c, batch, al, stream);
     }
+    // (a timing label names the kernel and its tiles, so a test can tell which one a shape ran on)
+    KernelTimer timer(in_dtype == CUEQ_F32 ? (big ? "gemm_nt_f32_256" : "gemm_nt_f32") : in_dtype == CUEQ_F16 ? "gemm_nt_f16" : "gemm_nt_bf16", stream);
     // EDGE (float32) where one tile in four is partly filled or there is one column of tiles: between whole tiles what is left is the
     // bound on registers (us without / with: 16 products of 1 032 x 1 032 x 128, 21 % of tiles partial, 64.6 / 70.5, 4 of 2 056
     // 64.6 / 67.4, 64 of 520, 36 %, 76 / 71; 153 664 x 128 x 128, A by rows and B by columns, 64 / 57, both by columns 63 / 56, both by

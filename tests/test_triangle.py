@@ -258,8 +258,9 @@ def test_gemm_tn_two_byte_pieces(device, dtype, rows, parts, M, N):
                                   (128, 512, 512, 512)])
 def test_gemm_operand_orders(device, dtype, trans_a, trans_b, dims):
     """cueq_gemm against torch.matmul in float64 for the four operand orders: tiled MFMA path (aligned extents,
-    partial tiles included), the 256 x 256 tiles (both extents multiples of 256 and at least two tiles per compute
-    unit: the last case, which is the contraction of the N = 512, D = 128 update and of its two gradients) and the
+    partial tiles included), the 256 x 256 tiles (float32: both extents multiples of 256 and at least two tiles per compute
+    unit: the last case, which is the contraction of the N = 512, D = 128 update and of its two gradients; 2-byte types, which load
+    straight into the local data share: extents above 128 and a tile per compute unit) and the
     element-wise path (odd extents).  The kernel each case ran on is read back from the library's timing labels."""
     from cuequivariance_amd import _lib
     from cuequivariance_amd.cuet import triangle as tri
@@ -268,9 +269,11 @@ def test_gemm_operand_orders(device, dtype, trans_a, trans_b, dims):
     cus = torch.cuda.get_device_properties(device).multi_processor_count
     aligned = all(v % 8 == 0 for v in (M, N, K))
     big = M % 256 == 0 and N % 256 == 0 and (M // 256) * (N // 256) * batch >= 2 * cus
+    if dtype != torch.float32:
+        big = M > 128 and N > 128 and -(-M // 256) * -(-N // 256) * batch >= cus
     if dims == (128, 512, 512, 512):
         assert big or cus > 256, "the benchmark's contraction shape must run on the 256 x 256 tiles"
-    label = {torch.float32: "gemm_nt_f32", torch.bfloat16: "gemm_nt_bf16", torch.float16: "gemm_nt_f16"}[dtype] + ("_256" if big else "") if aligned else "gemm_nt_simple"
+    label = {torch.float32: "gemm_nt_f32", torch.bfloat16: "gemm_direct_bf16", torch.float16: "gemm_direct_f16"}[dtype] + ("_256" if big else "") if aligned else "gemm_nt_simple"
     g = torch.Generator().manual_seed(M * 7 + N)
     A = torch.randn((batch, K, M) if trans_a else (batch, M, K), generator=g).to(dtype)
     B = torch.randn((batch, K, N) if trans_b else (batch, N, K), generator=g).to(dtype)
@@ -391,7 +394,7 @@ def test_benchmark_size_against_oracle(device, dtype):
     (got,) = torch.autograd.grad(out, [pg["x"]], cot.to(dtype).to(device))
     ran = _lib.timing_end()
     if torch.cuda.get_device_properties(device).multi_processor_count <= 256:
-        label = {torch.bfloat16: "gemm_nt_bf16_256", torch.float16: "gemm_nt_f16_256", torch.float32: "gemm_nt_f32_256"}[dtype]
+        label = {torch.bfloat16: "gemm_direct_bf16_256", torch.float16: "gemm_direct_f16_256", torch.float32: "gemm_nt_f32_256"}[dtype]
         assert ran.get(label, (0, 0))[0] == 3, ran  # the contraction and its two gradients
     if dtype != torch.float32:  # the stages with the weights resident in the local data share serve both 2-byte formats
         assert "ln_dual_gate_fwd" in ran and "gate_bwd_input_ln" in ran, ran
