@@ -42,8 +42,7 @@ __device__ __forceinline__ void tri_store(f16bits* p, int64_t i, float v) { p[i]
 // inside a step is free and every operand read is one or two ds_read_b128.
 // ------------------------------------------------------------------------------------------------
 constexpr int kTile = 128;
-constexpr int kStepBytes = 64;  // of k per row and step
-constexpr int kRowBytes = kStepBytes + 16;  // padded: conflict-free 16-byte reads by 16 consecutive rows
+constexpr int kRowBytes = 80;  // 64 bytes of data + 16 bytes of padding
 
 // Workgroups are handed to the 8 XCDs round-robin in launch order and every XCD has its own L2.  This maps the
 // launch-order index to a tile index so that each XCD works through one contiguous range of tiles (column tile
@@ -202,28 +201,29 @@ typedef short shortx4_t __attribute__((ext_vector_type(4)));
 // bytes between the k rows of a contraction-major tile of EXT columns: the row plus 64 (2-byte) / 128 (4-byte) bytes
 template <typename TI, int EXT>
 constexpr int trans_stride() { return EXT * static_cast<int>(sizeof(TI)) + (sizeof(TI) == 2 ? 64 : 128); }
-// LDS bytes of one operand tile of EXT rows (either layout)
-template <typename TI, int EXT>
+// LDS bytes of one operand tile of EXT rows (either layout); KB = bytes of k per row and step (64 or 128), rows of a
+// contraction-contiguous tile are KB + 16 bytes apart (conflict-free 16-byte reads by 16 consecutive rows for both)
+template <typename TI, int EXT, int KB = 64>
 constexpr int gemm_tile_bytes() {
-  constexpr int a = EXT * kRowBytes, b = (kStepBytes / static_cast<int>(sizeof(TI))) * trans_stride<TI, EXT>();
+  constexpr int a = EXT * (KB + 16), b = (KB / static_cast<int>(sizeof(TI))) * trans_stride<TI, EXT>();
   return a > b ? a : b;
 }
 
-template <typename TI, bool TR, int EXT>
+template <typename TI, bool TR, int EXT, int KB = 64>
 __device__ __forceinline__ void gemm_stage_offsets(int e, int& row, int& part) {
   constexpr int VPRN = EXT * sizeof(TI) / 16;  // vectors per k row of a contraction-major tile
   if constexpr (TR) { row = e / VPRN; part = e % VPRN; }
-  else { row = e / (kStepBytes / 16); part = e % (kStepBytes / 16); }
+  else { row = e / (KB / 16); part = e % (KB / 16); }
 }
 
-// fragment of subtile rows [base, base + 32) for MFMA slice q of the step (two slices): 16 bytes of k per lane
-template <typename TI, bool TR, int EXT>
+// fragment of subtile rows [base, base + 32) for MFMA slice q of the step (KB / 32 slices): 16 bytes of k per lane
+template <typename TI, bool TR, int EXT, int KB = 64>
 __device__ __forceinline__ uint4 gemm_fragment(const char* tile, int base, int q, int lane) {
   constexpr int kTransStride16 = trans_stride<uint16_t, EXT>(), kTransStride32 = trans_stride<float, EXT>();
-  constexpr int HK = kStepBytes / 2 / static_cast<int>(sizeof(TI));  // k rows of a contraction-major tile per half wavefront
+  constexpr int HK = KB / 2 / static_cast<int>(sizeof(TI));  // k rows of a contraction-major tile per half wavefront
   const int c = lane & 31, h = lane >> 5;
   if constexpr (!TR) {
-    return *reinterpret_cast<const uint4*>(tile + (base + c) * kRowBytes + h * (kStepBytes / 2) + q * 16);
+    return *reinterpret_cast<const uint4*>(tile + (base + c) * (KB + 16) + h * (KB / 2) + q * 16);
   } else if constexpr (sizeof(TI) == 2) {
     const int s = lane & 15, g16 = (lane >> 4) & 1;
     const char* p = tile + (HK * h + 8 * q + (s >> 2)) * kTransStride16 + (base + 16 * g16 + 4 * (s & 3)) * 2;  // k as in the other layout
@@ -243,13 +243,18 @@ __device__ __forceinline__ uint4 gemm_fragment(const char* tile, int base, int q
 // the operand traffic between L2 and the CUs for products whose both extents are large.
 // EDGE: some tiles are partly filled.  A wavefront forms only those of its four subtiles that reach into C, and which wavefront has
 // which quarter goes round (the first ones of a partial tile have more to do, and a wavefront's number decides its SIMD); the bound on
-// registers keeps the accumulators of four wavefronts beside their operands and four blocks on a CU.  128 products of n x n,
-// float32, us with all subtiles always / with EDGE, both operands by rows: 392 (4 x 4 tiles of 128, the last 8 wide) 251 / 222, 320
+// registers keeps the accumulators of four wavefronts beside their operands and four (three) blocks on a CU.  128 products of n x n,
+// us with all subtiles always / with EDGE, float32, both operands by rows: 392 (4 x 4 tiles of 128, the last 8 wide) 251 / 222, 320
 // 138 / 114; by columns 231 / 220, 116 / 108, 200 37.5 / 37.1; one partial tile, 512 products: 64 16.5 / 12.6.  (Loads left out as well,
 // behind a condition, make every wait one for all loads.)
-// 2-byte operands come here where the result is float32, is added to, or does not lie in 16-byte pieces; see gemm_direct_kernel.
-template <typename TI, typename TO, bool TA, bool TB, int WM = 2, int WN = 2, bool EDGE = false>
-__global__ void __launch_bounds__(64 * WM * WN, (!EDGE ? 1 : 4)) gemm_kernel(const TI* __restrict__ A, int64_t lda, int64_t sA,
+// KB: bytes of k per row and step; 128 (2-byte operands, 256 x 256) makes every request of a contraction-contiguous operand a whole
+// 128-byte line (with 64 a line is fetched in two halves one step apart, and a 256 x 256 step turns over the whole L1 in between).
+// 2-byte operands come here where the result is float32, is added to, does not lie in 16-byte pieces, or an operand reaches 4 GiB; see
+// gemm_direct_kernel.  It would be slower for the first of these: what is added to is read in the middle of its row of steps, and each
+// such wait takes in the loads ahead (us, this kernel / that one with 256 x 256 tiles: added to, 128 products of 512 54.4 / 79.0, of 392
+// 43.6 / 55.6, 147 456 x 192 x 384 48.3 / 81.8, 4 of 2 056 x 2 056 x 128 21.7 / 40.9; rows of 513 elements, 128 of 512 58.6 / 107).
+template <typename TI, typename TO, bool TA, bool TB, int WM = 2, int WN = 2, int KB = 64, bool EDGE = false>
+__global__ void __launch_bounds__(64 * WM * WN, (!EDGE ? 1 : TA && !TB && sizeof(TI) == 2 ? 3 : 4)) gemm_kernel(const TI* __restrict__ A, int64_t lda, int64_t sA,
                                                    const TI* __restrict__ B, int64_t ldb, int64_t sB,
                                                    TO* __restrict__ C, int64_t ldc, int64_t sC, int Mfull, int N, int Kfull,
                                                    float alpha, int accumulate, int vec_out, int64_t k_total, int nparts, int64_t pA,
@@ -257,13 +262,13 @@ __global__ void __launch_bounds__(64 * WM * WN, (!EDGE ? 1 : 4)) gemm_kernel(con
                                                    int64_t gsB, int64_t gsC) {
   using F = TI;
   constexpr int EPV = 16 / sizeof(TI);  // elements per 16-byte vector
-  constexpr int BK = kStepBytes / sizeof(TI);  // k extent of one step
-  constexpr int RB = kRowBytes;         // bytes between the rows of a contraction-contiguous tile
-  constexpr int NQ = kStepBytes / 32;   // 16-byte slices of k per half wavefront and step
+  constexpr int BK = KB / sizeof(TI);   // k extent of one step
+  constexpr int RB = KB + 16;           // bytes between the rows of a contraction-contiguous tile
+  constexpr int NQ = KB / 32;           // 16-byte slices of k per half wavefront and step
   constexpr int TMR = 64 * WM, TNC = 64 * WN, NTH = 64 * WM * WN;  // tile rows, tile columns, threads
   constexpr int TSA = trans_stride<TI, TMR>(), TSB = trans_stride<TI, TNC>();
-  constexpr int ABYTES = gemm_tile_bytes<TI, TMR>(), BBYTES = gemm_tile_bytes<TI, TNC>();
-  constexpr int NVA = TMR * (kStepBytes / 16) / NTH, NVB = TNC * (kStepBytes / 16) / NTH;  // 16-byte vectors per thread and step
+  constexpr int ABYTES = gemm_tile_bytes<TI, TMR, KB>(), BBYTES = gemm_tile_bytes<TI, TNC, KB>();
+  constexpr int NVA = TMR * (KB / 16) / NTH, NVB = TNC * (KB / 16) / NTH;  // 16-byte vectors per thread and step
   __shared__ __align__(16) char smem[2][ABYTES + BBYTES];
   const int tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63, c = lane & 31, h = lane >> 5;
@@ -316,9 +321,9 @@ __global__ void __launch_bounds__(64 * WM * WN, (!EDGE ? 1 : 4)) gemm_kernel(con
   uint4 stA[NVA], stB[NVB];
   int arow[NVA], apart[NVA], brow[NVB], bpart[NVB];
 #pragma unroll
-  for (int q = 0; q < NVA; ++q) gemm_stage_offsets<TI, TA, TMR>(tid + q * NTH, arow[q], apart[q]);
+  for (int q = 0; q < NVA; ++q) gemm_stage_offsets<TI, TA, TMR, KB>(tid + q * NTH, arow[q], apart[q]);
 #pragma unroll
-  for (int q = 0; q < NVB; ++q) gemm_stage_offsets<TI, TB, TNC>(tid + q * NTH, brow[q], bpart[q]);
+  for (int q = 0; q < NVB; ++q) gemm_stage_offsets<TI, TB, TNC, KB>(tid + q * NTH, brow[q], bpart[q]);
   auto load_one = [&](const TI* __restrict__ P, int64_t ld, bool tr, int row, int part, int x0, int X, int ks) -> uint4 {
     if (tr) {  // row = k within the step, part = vector along the tile's columns (extent X is a multiple of EPV)
       const int k = ks * BK + row, x = x0 + part * EPV;
@@ -367,8 +372,8 @@ __global__ void __launch_bounds__(64 * WM * WN, (!EDGE ? 1 : 4)) gemm_kernel(con
         for (int t = 0; t < 2; ++t)
 #pragma unroll
           for (int q = 0; q < NQ; ++q) {
-            if (t < NI) fa[t < NI ? t : 0][q] = gemm_fragment<TI, TA, TMR>(&smem[buf][0], wm * 64 + t * 32, q, lane);
-            if (t < NJ) fb[t < NJ ? t : 0][q] = gemm_fragment<TI, TB, TNC>(&smem[buf][ABYTES], wn * 64 + t * 32, q, lane);
+            if (t < NI) fa[t < NI ? t : 0][q] = gemm_fragment<TI, TA, TMR, KB>(&smem[buf][0], wm * 64 + t * 32, q, lane);
+            if (t < NJ) fb[t < NJ ? t : 0][q] = gemm_fragment<TI, TB, TNC, KB>(&smem[buf][ABYTES], wn * 64 + t * 32, q, lane);
           }
         // consecutive MFMAs go to different accumulators: a dependent one would wait for its predecessor to drain
 #pragma unroll
@@ -3590,8 +3595,6 @@ extern "C" int cueq_gemm(int32_t in_dtype, int32_t out_dtype, int32_t trans_a, i
     CUEQ_REQUIRE(grid.y < 65536, CUEQ_ERR_TOO_LARGE, "gemm: too many row tiles (M <= 8388480)");
     const int64_t out_es = out_dtype == CUEQ_F32 ? 4 : 2;
     const int vec_out = (reinterpret_cast<uintptr_t>(C) % 16 == 0 && (ldc * out_es) % 16 == 0 && (stride_c * out_es) % 16 == 0) ? 1 : 0;
-    // 256 x 256 tiles when both extents are multiples of 256 and there are enough of them to fill the chip
-    const bool big = in_dtype == CUEQ_F32 && !mixed && M % 256 == 0 && N % 256 == 0 && (M / 256) * (N / 256) * batch >= 2 * static_cast<int64_t>(device_cus());
     // 2-byte operands and results of one type: straight into LDS, unless results are added to or their rows are not 16-byte pieces
     // (byte offsets inside an operand are 32 bits, tile numbers 31)
     const int64_t far = int64_t(1) << 31;
@@ -3600,26 +3603,26 @@ extern "C" int cueq_gemm(int32_t in_dtype, int32_t out_dtype, int32_t trans_a, i
       if (in_dtype == CUEQ_F16) return gemm_direct<f16bits>(trans_a != 0, trans_b != 0, M, N, K, A, lda, stride_a, B, ldb, stride_b, C, ldc, stride_c, batch, al, stream);
       return gemm_direct<uint16_t>(trans_a != 0, trans_b != 0, M, N, K, A, lda, stride_a, B, ldb, stride_b, C, ldc, stride_c, batch, al, stream);
     }
+    // 256 x 256 tiles when both extents are multiples of 256 and there are enough of them to fill the chip twice (2-byte, added to, 128
+    // products of 512, both operands by columns 54.4 us, with 128 x 128 tiles 60.5; by rows 55.5 / 66.2)
+    const bool big = !mixed && M % 256 == 0 && N % 256 == 0 && (M / 256) * (N / 256) * batch >= 2 * static_cast<int64_t>(device_cus());
     // (a timing label names the kernel and its tiles, so a test can tell which one a shape ran on)
-    KernelTimer timer(in_dtype == CUEQ_F32 ? (big ? "gemm_nt_f32_256" : "gemm_nt_f32") : in_dtype == CUEQ_F16 ? "gemm_nt_f16" : "gemm_nt_bf16", stream);
-    // EDGE (float32) where one tile in four is partly filled or there is one column of tiles: between whole tiles what is left is the
-    // bound on registers (us without / with: 16 products of 1 032 x 1 032 x 128, 21 % of tiles partial, 64.6 / 70.5, 4 of 2 056
-    // 64.6 / 67.4, 64 of 520, 36 %, 76 / 71; 153 664 x 128 x 128, A by rows and B by columns, 64 / 57, both by columns 63 / 56, both by
-    // rows 66.6 / 70.2, 131 080 64.7 / 52.8)
+    KernelTimer timer(in_dtype == CUEQ_F32 ? (big ? "gemm_nt_f32_256" : "gemm_nt_f32") : in_dtype == CUEQ_F16 ? (big ? "gemm_nt_f16_256" : "gemm_nt_f16") : (big ? "gemm_nt_bf16_256" : "gemm_nt_bf16"), stream);
+    // EDGE where some tile is partly filled, in float32 only where one in four is or there is one column of tiles: between whole tiles what is
+    // left is the bound on registers (us without / with, float32: 16 products of 1 032 x 1 032 x 128, 21 % of tiles partial, 64.6 / 70.5, 4
+    // of 2 056 64.6 / 67.4, 64 of 520, 36 %, 76 / 71; 153 664 x 128 x 128, A by rows and B by columns, 64 / 57, both by columns 63 / 56, both by
+    // rows 66.6 / 70.2, 131 080 64.7 / 52.8; bfloat16, added to: 65 536 x 160 x 320 26.1 / 21.3, 147 456 x 192 x 384 53.0 / 48.2, 128 of 392
+    // 48.6 / 42.8, 4 of 2 056 21.2 / 21.7; into rows that are no 16-byte pieces: 100 000 x 100 x 128 21.4 / 17.1, 128 of 392 56.7 / 50.1)
     const int64_t whole = (M / kTile) * (N / kTile), all = static_cast<int64_t>(grid.x) * grid.y;
-    const bool edge = whole < all && (grid.x == 1 || 4 * (all - whole) >= all);
+    const bool edge = whole < all && (in_dtype != CUEQ_F32 || grid.x == 1 || 4 * (all - whole) >= all);
     const dim3 grid_big(static_cast<unsigned>(N / 256), static_cast<unsigned>(M / 256), static_cast<unsigned>(batch));
 #define GEMM_ARGS(TI, TO) static_cast<const TI*>(A), lda, stride_a, static_cast<const TI*>(B), ldb, stride_b, static_cast<TO*>(C), ldc, stride_c, m, n, k, al, accumulate, vec_out, 0, 1, 0, 0, 0, nullptr, 0, 0, 0, 0
 #define GEMM_LAUNCH(TI, TO, TA, TB) hipLaunchKernelGGL((gemm_kernel<TI, TO, TA, TB>), grid, dim3(256), 0, stream, GEMM_ARGS(TI, TO))
 #define GEMM_SZ(TI, TA, TB)                                                                                                                      \
   do {                                                                                                                                       \
-    if constexpr (sizeof(TI) == 4) {                                                                                                         \
-      if (big) hipLaunchKernelGGL((gemm_kernel<TI, TI, TA, TB, 4, 4>), grid_big, dim3(1024), 0, stream, GEMM_ARGS(TI, TI));                  \
-      else if (edge) hipLaunchKernelGGL((gemm_kernel<TI, TI, TA, TB, 2, 2, true>), grid, dim3(256), 0, stream, GEMM_ARGS(TI, TI));          \
-      else GEMM_LAUNCH(TI, TI, TA, TB);                                                                                                      \
-    } else {                                                                                                                                 \
-      GEMM_LAUNCH(TI, TI, TA, TB);                                                                                                           \
-    }                                                                                                                                        \
+    if (big) hipLaunchKernelGGL((gemm_kernel<TI, TI, TA, TB, 4, 4, (sizeof(TI) == 2 ? 128 : 64)>), grid_big, dim3(1024), 0, stream, GEMM_ARGS(TI, TI)); \
+    else if (edge) hipLaunchKernelGGL((gemm_kernel<TI, TI, TA, TB, 2, 2, 64, true>), grid, dim3(256), 0, stream, GEMM_ARGS(TI, TI));          \
+    else GEMM_LAUNCH(TI, TI, TA, TB);                                                                                                        \
   } while (0)
 #define GEMM_TR(TI) do { if (trans_a && trans_b) GEMM_SZ(TI, true, true); else if (trans_a) GEMM_SZ(TI, true, false); else if (trans_b) GEMM_SZ(TI, false, true); else GEMM_SZ(TI, false, false); } while (0)
     if (in_dtype == CUEQ_F32 && out_dtype == CUEQ_F32) GEMM_TR(float);

@@ -252,6 +252,46 @@ def test_gemm_tn_two_byte_pieces(device, dtype, rows, parts, M, N):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("trans_a,trans_b", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("batch,M,N,K,pad,shift", [(3, 200, 136, 72, 1, 0), (2, 72, 40, 8, 0, 1), (300, 136, 144, 40, 0, 0), (300, 144, 136, 136, 3, 1),
+                                                   (70, 264, 392, 64, 8, 0), (70, 264, 392, 96, 2, 0), (1, 512, 48, 1024, 0, 0), (130, 512, 512, 72, 0, 0),
+                                                   (130, 512, 512, 64, 1, 0)])
+def test_two_byte_products_into_rows_of_any_length(device, dtype, trans_a, trans_b, batch, M, N, K, pad, shift):
+    """2-byte products that are added to what is there, and whose rows are longer than the result, start at any element or are no whole
+    16-byte pieces: parts of tiles, 256 x 256 tiles, one step and many.  Against float64 on the rounded operands:
+    the product is rounded at most once, and so is the sum; what lies between the rows stays."""
+    from cuequivariance_amd import _lib
+
+    g = torch.Generator(device=device).manual_seed(M + N + K)
+    r = lambda *s: torch.randn(*s, generator=g, device=device).to(dtype)
+    A, B = r(batch, *((K, M) if trans_a else (M, K))), r(batch, *((K, N) if trans_b else (N, K)))
+    A64 = (A.transpose(1, 2) if trans_a else A).double()
+    ref = 0.5 * A64 @ (B if trans_b else B.transpose(1, 2)).double().contiguous()
+    ldc, lib = N + pad, _lib.load()
+    before = r(batch * M * ldc + shift)
+    code = {torch.bfloat16: _lib.BF16, torch.float16: _lib.F16}[dtype]
+    for accumulate in (0, 1):
+        C = before.clone()
+        _lib.timing_begin()
+        _lib.check(lib.cueq_gemm(code, code, int(trans_a), int(trans_b), M, N, K, A.data_ptr(), A.stride(1), A.stride(0), B.data_ptr(), B.stride(1),
+                                 B.stride(0), C[shift:].data_ptr(), ldc, M * ldc, batch, 0.5, accumulate, torch.cuda.current_stream().cuda_stream), "cueq_gemm")
+        ran = list(_lib.timing_end())
+        pieces = ldc % 8 == 0 and N % 8 == 0 and shift == 0
+        big = M == 512 and N == 512 and 4 * batch >= 2 * torch.cuda.get_device_properties(device).multi_processor_count
+        if accumulate or not pieces:
+            assert ran == [f"gemm_nt_{'bf16' if dtype == torch.bfloat16 else 'f16'}" + ("_256" if big else "")], ran
+        else:
+            assert len(ran) == 1 and ran[0].startswith("gemm_direct"), ran
+        got, was = (t[shift:].view(batch, M, ldc) for t in (C, before))
+        assert torch.equal(got[:, :, N:], was[:, :, N:]) and torch.equal(C[:shift], before[:shift])
+        unit = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+        want = ref + (was[:, :, :N].double() if accumulate else 0)
+        bound = unit * (want.abs() + accumulate * ref.abs()) * (1 + unit) + 2.0 ** -22 * K * (A.double().abs().amax() * B.double().abs().amax())
+        assert bool(((got[:, :, :N].double() - want).abs() <= bound + 2.0 ** -24).all())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("trans_a,trans_b", [(False, False), (False, True), (True, False), (True, True)])
 @pytest.mark.parametrize("dims", [(3, 256, 128, 192), (2, 136, 200, 72), (1, 33, 47, 21), (160, 512, 256, 96),
