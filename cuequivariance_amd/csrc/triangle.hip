@@ -249,8 +249,8 @@ __device__ __forceinline__ uint4 gemm_fragment(const char* tile, int base, int q
 // behind a condition, make every wait one for all loads.)
 // KB: bytes of k per row and step; 128 (2-byte operands, 256 x 256) makes every request of a contraction-contiguous operand a whole
 // 128-byte line (with 64 a line is fetched in two halves one step apart, and a 256 x 256 step turns over the whole L1 in between).
-// 2-byte operands come here where the result is float32, is added to, does not lie in 16-byte pieces, or an operand reaches 4 GiB; see
-// gemm_direct_kernel.  It would be slower for the first of these: what is added to is read in the middle of its row of steps, and each
+// 2-byte operands come here where the result is float32, is added to, does not lie in 16-byte pieces, or an operand reaches 4 GiB, and
+// where gemm_direct_kernel is the slower one (direct_tiles).  It would be slower for what is added to: what is added to is read in the middle of its row of steps, and each
 // such wait takes in the loads ahead (us, this kernel / that one with 256 x 256 tiles: added to, 128 products of 512 54.4 / 79.0, of 392
 // 43.6 / 55.6, 147 456 x 192 x 384 48.3 / 81.8, 4 of 2 056 x 2 056 x 128 21.7 / 40.9; rows of 513 elements, 128 of 512 58.6 / 107).
 template <typename TI, typename TO, bool TA, bool TB, int WM = 2, int WN = 2, int KB = 64, bool EDGE = false>
@@ -3483,11 +3483,10 @@ static int raise_lds(int bytes) {
   return CUEQ_OK;
 }
 
-// Wide: 256 x 256 tiles, eight wavefronts of 128 x 64, from one tile per compute unit on, and where the tile is not mostly empty (128
-// products, us wide / narrow: 512 48 - 52 / 57 - 63, 384 30 - 33 / 32 - 35, 264 19 / 20; 64 products of 264 11 - 12 / 13 - 14, of 256 - 64
-// tiles - 11.6 / 7.6; 256 products of 256 21 / 24, of 144 10 / 12, of 104 7.7 / 6.2).  Operands that both lie by rows of k take 128 bytes of
-// a row a step and two buffers, whole lines (128 products of 392 39.5 / 42.2, 768 141 / 164); by columns a step's rows are whole lines
-// already, and three buffers of half the depth are faster (392 36.4 / 32.0, 480 45.6 / 42.3).
+// Wide: 256 x 256 tiles, eight wavefronts of 128 x 64, one block on a compute unit.  Narrow: 128 x 128, four of 64 x 64, two blocks.
+// Operands that both lie by rows of k take 128 bytes of a row a step and two buffers in the wide form, whole lines (128 products of 392
+// 39.5 / 42.2, 768 141 / 164); by columns a step's rows are whole lines already, and three buffers of half the depth are faster (392
+// 36.4 / 32.0, 480 45.6 / 42.3).
 template <bool ROWS>
 using DirectWide = DirectShape<4, 2, 2, 4, ROWS ? 128 : 64, ROWS ? 2 : 3, ROWS ? 16 : 32, 1>;
 using DirectNarrow = DirectShape<2, 2, 2, 2, 64, 3, 16, 2>;  // 128 x 128 tiles, four wavefronts of 64 x 64
@@ -3513,10 +3512,39 @@ static int launch_gemm_direct(int64_t M, int64_t N, int64_t K, const F* A, int64
   CUEQ_CHECK_HIP(hipGetLastError());
   return CUEQ_OK;
 }
+// Blocks stay, so a round of tiles ends with its last one, and a short contraction ends before its results have left: gemm_kernel, with
+// four blocks a compute unit that come and go, is the better one where the last round is poorly filled or the tiles are.  Taken from 3 600
+// timings (squares of 48 to 512 in batches of 32 to 320, 4 096 to 262 144 rows by 32 to 512 columns over 8 to 512; every order of operands,
+// operands not in the L2), us, wide / narrow / gemm_kernel: the rule is within 1 % of the best of them on average and 2.6 % faster than
+// wide from one tile a compute unit on, narrow before.
+//   wide, rounds at least 95 % full: 128 products of 512 51.5 / 68.5 / 56.3, 64 of 264 12.3 / 14.6 / 13.2, 256 of 136 10.9 / 12.6 / 13.1; not
+//     where the shorter side leaves much of its two or more tiles empty (192 of 264 30.7 / 26.7 / 28.1, 153 664 x 264 x 192
+//     53.3 / 52.8 / 48.6), unless a long contraction stands against few rounds, and not rows of fewer than the 64 values a step has
+//     (65 536 x 384 x 32 15.4 / 12.9 / 12.6);
+//   wide, rounds less full: large whole tiles only (96 of 392 30.6 / 32.5 / 36.3, 160 of 480 60.4 / 70.5 / 72.0, 160 of 264 27.3 / 21.5 / 21.6,
+//     66 000 x 264 x 128 23.9 / 18.1 / 17.1, 66 000 x 320 x 8 19.7 / 14.0 / 12.3);
+//   narrow: one round (20 000 x 192 x 128 9.2 / 6.8 / 7.6, x 512 17.9 / 11.5 / 15.0), or well filled ones of three steps and more (200 000 x 128
+//     x 8 24.8 / 14.3 / 12.7, 66 000 x 128 x 64 13.5 / 9.2 / 8.5).
+enum class Direct { kNo, kNarrow, kWide };
+static Direct direct_tiles(bool by_rows, int64_t M, int64_t N, int64_t K, int64_t batch) {
+  const int64_t cus = device_cus();
+  const auto tiles = [&](int64_t side) { return ((M + side - 1) / side) * ((N + side - 1) / side) * batch; };
+  const int64_t wide = tiles(256), narrow = tiles(128);
+  if (M > 128 && N > 128 && wide >= cus) {
+    const int64_t rounds = (wide + cus - 1) / cus, side = std::min(M, N), room = (side + 255) / 256 * 256;
+    const bool square = K >= side;
+    const bool take = 20 * wide >= 19 * rounds * cus
+                          ? ((side <= 256 || 10 * side >= 7 * room) && (K >= 64 || !by_rows)) || (square && (20 * side >= 13 * room || rounds <= 2))
+                          : K >= 128 && side >= 384 && (square || 10 * side >= 8 * room);
+    return take ? Direct::kWide : Direct::kNo;
+  }
+  const int64_t rounds = (narrow + 2 * cus - 1) / (2 * cus);
+  return rounds <= 1 || (K >= 96 && 4 * narrow >= 3 * rounds * 2 * cus) ? Direct::kNarrow : Direct::kNo;
+}
 template <typename F>
-static int gemm_direct(bool ta, bool tb, int64_t M, int64_t N, int64_t K, const void* A, int64_t lda, int64_t sA, const void* B, int64_t ldb, int64_t sB, void* C,
+static int gemm_direct(Direct tiles, bool ta, bool tb, int64_t M, int64_t N, int64_t K, const void* A, int64_t lda, int64_t sA, const void* B, int64_t ldb, int64_t sB, void* C,
                        int64_t ldc, int64_t sC, int64_t batch, float alpha, hipStream_t stream) {
-  const bool wide = M > 128 && N > 128 && ((M + 255) / 256) * ((N + 255) / 256) * batch >= device_cus();
+  const bool wide = tiles == Direct::kWide;
   constexpr bool half = std::is_same_v<F, f16bits>;
   KernelTimer timer(wide ? (half ? "gemm_direct_f16_256" : "gemm_direct_bf16_256") : (half ? "gemm_direct_f16" : "gemm_direct_bf16"), stream);
   auto go = [&](auto a, auto b) {
@@ -3598,10 +3626,12 @@ extern "C" int cueq_gemm(int32_t in_dtype, int32_t out_dtype, int32_t trans_a, i
     // 2-byte operands and results of one type: straight into LDS, unless results are added to or their rows are not 16-byte pieces
     // (byte offsets inside an operand are 32 bits, tile numbers 31)
     const int64_t far = int64_t(1) << 31;
-    if (!mixed && in_dtype != CUEQ_F32 && !accumulate && vec_out && n % 8 == 0 && (trans_a ? 64 : M) * lda < far && (trans_b ? 64 : N) * ldb < far &&
-        (M / 128 + 1) * (N / 128 + 1) * batch < far) {
-      if (in_dtype == CUEQ_F16) return gemm_direct<f16bits>(trans_a != 0, trans_b != 0, M, N, K, A, lda, stride_a, B, ldb, stride_b, C, ldc, stride_c, batch, al, stream);
-      return gemm_direct<uint16_t>(trans_a != 0, trans_b != 0, M, N, K, A, lda, stride_a, B, ldb, stride_b, C, ldc, stride_c, batch, al, stream);
+    const bool direct_ok = !mixed && in_dtype != CUEQ_F32 && !accumulate && vec_out && n % 8 == 0 && (trans_a ? 64 : M) * lda < far &&
+                           (trans_b ? 64 : N) * ldb < far && (M / 128 + 1) * (N / 128 + 1) * batch < far;
+    const Direct direct = direct_ok ? direct_tiles(!trans_a && !trans_b, M, N, K, batch) : Direct::kNo;
+    if (direct != Direct::kNo) {
+      if (in_dtype == CUEQ_F16) return gemm_direct<f16bits>(direct, trans_a != 0, trans_b != 0, M, N, K, A, lda, stride_a, B, ldb, stride_b, C, ldc, stride_c, batch, al, stream);
+      return gemm_direct<uint16_t>(direct, trans_a != 0, trans_b != 0, M, N, K, A, lda, stride_a, B, ldb, stride_b, C, ldc, stride_c, batch, al, stream);
     }
     // 256 x 256 tiles when both extents are multiples of 256 and there are enough of them to fill the chip twice (2-byte, added to, 128
     // products of 512, both operands by columns 54.4 us, with 128 x 128 tiles 60.5; by rows 55.5 / 66.2)

@@ -185,6 +185,27 @@ def test_layer_norm_fused_into_the_gated_projection(device, M, K, C, affine, bia
         assert (out.float() - out2.float()).abs().max().item() <= 2.0 ** -6 * out2.float().abs().max().item()
 
 
+def two_byte_kernel(dtype, by_rows, M, N, K, batch, plain=True):
+    """The timing label of the kernel a 2-byte product runs on: straight into LDS where whole rounds of its tiles are well filled, unless it
+    is added to or its rows are no 16-byte pieces (not ``plain``)."""
+    name, cus = {torch.bfloat16: "bf16", torch.float16: "f16"}[dtype], torch.cuda.get_device_properties(0).multi_processor_count
+    up = lambda a, b: -(-a // b)
+    wide, narrow, side = up(M, 256) * up(N, 256) * batch, up(M, 128) * up(N, 128) * batch, min(M, N)
+    room, rounds = 256 * up(side, 256), up(wide, cus)
+    if plain and M > 128 and N > 128 and wide >= cus:
+        if 20 * wide >= 19 * rounds * cus:
+            take = (side <= 256 or 10 * side >= 7 * room) and (K >= 64 or not by_rows) or K >= side and (20 * side >= 13 * room or rounds <= 2)
+        else:
+            take = K >= 128 and side >= 384 and (K >= side or 10 * side >= 8 * room)
+        if take:
+            return f"gemm_direct_{name}_256"
+    elif plain:
+        rounds = up(narrow, 2 * cus)
+        if rounds <= 1 or K >= 96 and 4 * narrow >= 3 * rounds * 2 * cus:
+            return f"gemm_direct_{name}"
+    return f"gemm_nt_{name}" + ("_256" if M % 256 == N % 256 == 0 and wide >= 2 * cus else "")
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("trans_a,trans_b", [(False, False), (False, True), (True, False), (True, True)])
@@ -196,6 +217,10 @@ def test_layer_norm_fused_into_the_gated_projection(device, M, K, C, affine, bia
         (3, 200, 136, 1000),  # tiles cut unevenly, the last step a quarter full
         (300, 264, 136, 40),  # 256 x 256 tiles, two a matrix and more than one a compute unit, partly filled ones between whole ones
         (130, 392, 520, 104),
+        (1000, 72, 40, 104),  # the same where loads go straight into LDS: rounds of tiles that are well filled (on 256 compute units)
+        (252, 264, 136, 72),
+        (252, 264, 136, 40),
+        (168, 392, 520, 104),
     ],
 )
 def test_gemm_two_byte_tiles(device, dtype, trans_a, trans_b, batch, M, N, K):
@@ -217,8 +242,10 @@ def test_gemm_two_byte_tiles(device, dtype, trans_a, trans_b, batch, M, N, K):
     lib = _lib.load()
     code = {torch.bfloat16: _lib.BF16, torch.float16: _lib.F16}[dtype]
     p = lambda t: C.c_void_p(t.data_ptr())
+    _lib.timing_begin()
     _lib.check(lib.cueq_gemm(code, code, int(trans_a), int(trans_b), M, N, K, p(A), A.shape[2], A[0].numel(), p(B), B.shape[2], B[0].numel(), p(out), N + 8,
                              M * (N + 8), batch, C.c_double(1.0), 0, torch.cuda.current_stream().cuda_stream), "cueq_gemm")
+    assert list(_lib.timing_end()) == [two_byte_kernel(dtype, not trans_a and not trans_b, M, N, K, batch)]
     assert bool((out[:, :, N:] == -7.0).all())
     got = out[:, :, :N].double()
     bad = torch.zeros_like(got, dtype=torch.bool)
@@ -277,12 +304,8 @@ def test_two_byte_products_into_rows_of_any_length(device, dtype, trans_a, trans
         _lib.check(lib.cueq_gemm(code, code, int(trans_a), int(trans_b), M, N, K, A.data_ptr(), A.stride(1), A.stride(0), B.data_ptr(), B.stride(1),
                                  B.stride(0), C[shift:].data_ptr(), ldc, M * ldc, batch, 0.5, accumulate, torch.cuda.current_stream().cuda_stream), "cueq_gemm")
         ran = list(_lib.timing_end())
-        pieces = ldc % 8 == 0 and N % 8 == 0 and shift == 0
-        big = M == 512 and N == 512 and 4 * batch >= 2 * torch.cuda.get_device_properties(device).multi_processor_count
-        if accumulate or not pieces:
-            assert ran == [f"gemm_nt_{'bf16' if dtype == torch.bfloat16 else 'f16'}" + ("_256" if big else "")], ran
-        else:
-            assert len(ran) == 1 and ran[0].startswith("gemm_direct"), ran
+        plain = not accumulate and ldc % 8 == 0 and N % 8 == 0 and shift == 0
+        assert ran == [two_byte_kernel(dtype, not trans_a and not trans_b, M, N, K, batch, plain)], ran
         got, was = (t[shift:].view(batch, M, ldc) for t in (C, before))
         assert torch.equal(got[:, :, N:], was[:, :, N:]) and torch.equal(C[:shift], before[:shift])
         unit = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
@@ -298,9 +321,8 @@ def test_two_byte_products_into_rows_of_any_length(device, dtype, trans_a, trans
                                   (128, 512, 512, 512)])
 def test_gemm_operand_orders(device, dtype, trans_a, trans_b, dims):
     """cueq_gemm against torch.matmul in float64 for the four operand orders: tiled MFMA path (aligned extents,
-    partial tiles included), the 256 x 256 tiles (float32: both extents multiples of 256 and at least two tiles per compute
-    unit: the last case, which is the contraction of the N = 512, D = 128 update and of its two gradients; 2-byte types, which load
-    straight into the local data share: extents above 128 and a tile per compute unit) and the
+    partial tiles included), the 256 x 256 tiles (float32, and 2-byte results that are added to: both extents multiples of 256 and at least
+    two tiles per compute unit: the last case, which is the contraction of the N = 512, D = 128 update and of its two gradients) and the
     element-wise path (odd extents).  The kernel each case ran on is read back from the library's timing labels."""
     from cuequivariance_amd import _lib
     from cuequivariance_amd.cuet import triangle as tri
@@ -309,11 +331,11 @@ def test_gemm_operand_orders(device, dtype, trans_a, trans_b, dims):
     cus = torch.cuda.get_device_properties(device).multi_processor_count
     aligned = all(v % 8 == 0 for v in (M, N, K))
     big = M % 256 == 0 and N % 256 == 0 and (M // 256) * (N // 256) * batch >= 2 * cus
-    if dtype != torch.float32:
-        big = M > 128 and N > 128 and -(-M // 256) * -(-N // 256) * batch >= cus
     if dims == (128, 512, 512, 512):
         assert big or cus > 256, "the benchmark's contraction shape must run on the 256 x 256 tiles"
-    label = {torch.float32: "gemm_nt_f32", torch.bfloat16: "gemm_direct_bf16", torch.float16: "gemm_direct_f16"}[dtype] + ("_256" if big else "") if aligned else "gemm_nt_simple"
+    labels = ["gemm_nt_f32" + ("_256" if big else "")] * 2 if aligned else ["gemm_nt_simple"] * 2
+    if aligned and dtype != torch.float32:
+        labels = [two_byte_kernel(dtype, not trans_a and not trans_b, M, N, K, batch, plain) for plain in (True, False)]
     g = torch.Generator().manual_seed(M * 7 + N)
     A = torch.randn((batch, K, M) if trans_a else (batch, M, K), generator=g).to(dtype)
     B = torch.randn((batch, K, N) if trans_b else (batch, N, K), generator=g).to(dtype)
@@ -323,10 +345,13 @@ def test_gemm_operand_orders(device, dtype, trans_a, trans_b, dims):
     _lib.timing_begin()
     got = tri.gemm_nt(A.to(device), B.to(device), dtype, alpha=0.5, trans_a=trans_a, trans_b=trans_b)
     ran = _lib.timing_end()
-    assert list(ran) == [label], (ran, label)
+    assert list(ran) == labels[:1], (ran, labels)
     assert rel_err(got, ref) <= TOL[dtype], rel_err(got, ref)
     prev = torch.randn(batch, M, N, generator=g).to(dtype)
+    _lib.timing_begin()
     got2 = tri.gemm_nt(A.to(device), B.to(device), dtype, out=prev.to(device).clone(), accumulate=True, trans_a=trans_a, trans_b=trans_b)
+    ran = _lib.timing_end()
+    assert list(ran) == labels[1:], (ran, labels)
     assert rel_err(got2, 2 * ref + prev.double()) <= TOL[dtype]
 
 
