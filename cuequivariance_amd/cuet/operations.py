@@ -22,6 +22,7 @@ from typing import Dict, List, Optional, Sequence
 import torch
 
 from .. import _lib, cue
+from .. import jit as _jit
 from ..codegen import fullyconnected_rows as fcr
 from ..cue import descriptors
 from .dense import GeneralFullyConnected, SegmentedPolynomialDense
@@ -106,6 +107,10 @@ class _FlattenedUniform(torch.nn.Module):
 
     def forward(self, inputs: List[torch.Tensor], input_indices: Optional[Dict[int, torch.Tensor]] = None,
                 output_shapes: Optional[Dict[int, torch.Tensor]] = None, output_indices: Optional[Dict[int, torch.Tensor]] = None):
+        return self.built()(inputs, input_indices=input_indices or {}, output_shapes=output_shapes or {},
+                            output_indices=output_indices or {})
+
+    def built(self) -> SegmentedPolynomial:
         if self.f is None:
             q = self._polynomial.flatten_coefficient_modes()
             stp = q.operations[0][1]
@@ -115,8 +120,7 @@ class _FlattenedUniform(torch.nn.Module):
             if len(extents) > 1:
                 q = q.split_mode(keep, math.gcd(*extents))
             self.f = SegmentedPolynomial(q, method="uniform_1d", math_dtype=self._math_dtype, options={"origin": self._polynomial})
-        return self.f(inputs, input_indices=input_indices or {}, output_shapes=output_shapes or {},
-                      output_indices=output_indices or {})
+        return self.f
 
 
 _BUILT = frozenset([SegmentedPolynomial, SegmentedPolynomialFromUniform1d, SegmentedPolynomialFusedTP, SegmentedPolynomialDense,
@@ -500,7 +504,20 @@ class FullyConnectedTensorProduct(torch.nn.Module):
             self.per_sample_rows = SegmentedPolynomial(q, method="uniform_1d", math_dtype=self.f_per_sample._math_dtype,
                                                        options={"origin": self._mul_ir_rows, "segment_groups": groups})
         m = _executor(self, "per_sample_rows", SegmentedPolynomialFromUniform1d)
-        return None if m is None else m.operator.product(weight, x1, x2, indices_1, None, indices_out, size_out)
+        if m is None or not self._rows_are_served(m._plan(m.math_dtype or weight.dtype)):
+            return None
+        return m.operator.product(weight, x1, x2, indices_1, None, indices_out, size_out)
+
+    def _rows_are_served(self, plan) -> bool:
+        """Whether there are kernels for the rows as they lie, in the library or compiled before, or they are to be compiled at first use:
+        not where the library has those of ir_mul rows (a transposition on either side costs microseconds, a compilation seconds), and
+        without compilation a transposition costs far less than the table-driven kernels."""
+        compiles = _jit.enabled()
+        if compiles not in plan.served:
+            flat = None if plan.registered() or not compiles else getattr(self.f_per_sample.built(), "m", None)
+            plan.served[compiles] = plan.registered() or (isinstance(flat, SegmentedPolynomialFromUniform1d)
+                                                          and not flat._plan(plan.math_dtype).registered(linked=True))
+        return plan.served[compiles]
 
     def _dense(self):
         """The executor of the 4-operand form for rows in this module's layouts, or ``None``."""

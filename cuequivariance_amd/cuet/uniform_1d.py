@@ -93,6 +93,7 @@ class Uniform1dPlan:
         self.jit_root = None  # for a backward plan: the forward plan, whose translation unit holds its kernels
         self.polynomial = None  # the flattened polynomial the tables came from, when the caller has it
         self.origin = None      # the polynomial that one was flattened from (a fully connected product's descriptor)
+        self.served: dict = {}  # for the rows of a module that has another way too: whether it takes this plan, by whether compilation is on
         self._lock = threading.Lock()
         # under this text a traced graph (torch.compile, torch.export, torch.jit.trace) names the plan: operator name,
         # arithmetic type and the packed tables, so that a saved graph stays valid where this object does not exist
@@ -128,6 +129,10 @@ class Uniform1dPlan:
         """True when kernels generated for exactly these tables are linked into the library."""
         h = self.handle(device)
         return bool(_lib.load().cueq_u1d_plan_info(h, None))
+
+    def registered(self, linked: bool = False) -> bool:
+        """Whether such kernels are there without a compilation; ``linked``: in the library itself, not compiled at first use."""
+        return _jit.has_kernels(self.tables, _DTYPE_CODE[self.math_dtype], linked)
 
     # ------------------------------------------------------------------ device plan
     def handle(self, device: torch.device) -> int:

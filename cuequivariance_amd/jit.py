@@ -123,6 +123,14 @@ def _has_spec(t: U1dTables, code: int, io_code: Optional[int] = None) -> bool:
     return bool(_lib.load().cueq_u1d_desc_serves(C.byref(desc), io_code))
 
 
+def has_kernels(t: U1dTables, code: int, linked: bool = False) -> bool:
+    """Whether kernels generated for these tables (and buffers of the arithmetic type) are registered with the library; ``linked``: by the
+    library itself, not by an object that was compiled at first use."""
+    desc, keep = _lib.make_desc(t, code)
+    key = C.c_uint64()
+    return bool(_lib.load().cueq_u1d_desc_info(C.byref(desc), C.byref(key))) and not (linked and key.value in _loaded)
+
+
 def is_symmetric_contraction(poly) -> bool:
     """``w[u], x[u] (one to three times) -> out[u]`` in every operation, one uniform extent: the form
     ``codegen/symmetric.py`` generates kernels for."""

@@ -181,6 +181,70 @@ def test_mul_ir_rows_are_flattened_at_the_cost_of_ir_mul_rows(ir1, ir2, ir3, mon
     assert count(fcr.Rows(poly, True, True)) == count(fcr.Rows(poly))
 
 
+@pytest.mark.parametrize("compiles", [False, True])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("which,layouts,served", [
+    (0, ("mul_ir", "mul_ir"), (True, True)),    # in the library
+    (0, ("mul_ir", "ir_mul"), (False, False)),  # the library has ir_mul rows, one transposition away
+    (0, ("ir_mul", "mul_ir"), (False, False)),
+    (1, ("mul_ir", "mul_ir"), (False, True)),   # compiled at first use or not at all
+    (1, ("mul_ir", "ir_mul"), (False, True)),
+])
+def test_which_mul_ir_rows_are_taken_as_they_lie(which, layouts, served, dtype, compiles, monkeypatch):
+    from cuequivariance_amd import cuet
+
+    i1, i2, i3 = (cue.Irreps("O3", s) for s in (MUL_IR_ROWS[0] if which == 0 else ("20x0e+20x1o", "0e+1o", "12x0e+12x1o")))
+    m = cuet.FullyConnectedTensorProduct(i1, i2, i3, layout_in1=cue.IrrepsLayout.as_layout(layouts[0]), layout_in2=cue.mul_ir,
+                                         layout_out=cue.IrrepsLayout.as_layout(layouts[1]), shared_weights=False, internal_weights=False)
+    monkeypatch.setattr(jit, "_enabled", compiles)
+    q, groups = fcr.flatten(m._mul_ir_rows)
+    rows = cuet.SegmentedPolynomial(q, method="uniform_1d", options={"origin": m._mul_ir_rows, "segment_groups": groups})
+    plan = rows.m._plan(dtype)
+    assert m._rows_are_served(plan) == m._rows_are_served(plan) == served[compiles]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layouts", [("mul_ir", "ir_mul"), ("ir_mul", "mul_ir")])
+def test_mixed_row_orders_without_compilation_keep_to_the_library(device, layouts, monkeypatch):
+    """One side is transposed and the linked kernels run, forward and backward."""
+    from cuequivariance_amd import _lib, cuet
+
+    monkeypatch.setattr(jit, "_enabled", False)
+    i1, i2, i3 = (cue.Irreps("O3", s) for s in MUL_IR_ROWS[0])
+    more = dict(shared_weights=False, internal_weights=False)
+    m = cuet.FullyConnectedTensorProduct(i1, i2, i3, layout_in1=cue.IrrepsLayout.as_layout(layouts[0]), layout_in2=cue.mul_ir,
+                                         layout_out=cue.IrrepsLayout.as_layout(layouts[1]), **more)
+    same = cuet.FullyConnectedTensorProduct(i1, i2, i3, layout=cue.mul_ir, **more)
+    g = torch.Generator(device=device).manual_seed(3)
+    x1, x2, w, cot = (torch.randn(77, d, generator=g, device=device) for d in (i1.dim, i2.dim, m.weight_numel, i3.dim))
+
+    def turned(x, irreps, layout, back=False):  # mul_ir rows in the given layout, or back
+        if layout == "mul_ir":
+            return x
+        parts, off = [], 0
+        for mul, ir in irreps:
+            shape = (-1, ir.dim, mul) if back else (-1, mul, ir.dim)
+            parts.append(x[:, off:off + mul * ir.dim].reshape(shape).transpose(1, 2).reshape(-1, mul * ir.dim))
+            off += mul * ir.dim
+        return torch.cat(parts, 1)
+
+    def step(f, x, c):
+        args = [t.clone().requires_grad_() for t in (x, x2, w)]
+        out = f(*args)
+        return [out.detach(), *torch.autograd.grad(out, args, c)]
+
+    want = step(same, x1, cot)
+    _lib.timing_begin()
+    got = step(m, turned(x1, i1, layouts[0]).contiguous(), turned(cot, i3, layouts[1]).contiguous())
+    names = list(_lib.timing_end())
+    assert "segmented_transpose" in names and all(any(n.startswith("fcr_") and f"_{way}_" in n for n in names) for way in ("fwd", "bwd")), names
+    plan = m.f_per_sample.f.m._plan(torch.float32)
+    assert plan.specialised(device) and plan.backward_plan((True, True, True)).specialised(device)
+    got = [turned(got[0], i3, layouts[1], True), turned(got[1], i1, layouts[0], True), got[2], got[3]]
+    for a, b in zip(got, want):  # (the same kernels but for the addresses)
+        assert (a - b).abs().max().item() <= 1e-6 * b.abs().max().item()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("indexed,deterministic", [(True, "0"), (True, "1"), (False, "0")])
 @pytest.mark.parametrize(
