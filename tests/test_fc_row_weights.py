@@ -308,3 +308,75 @@ def test_row_weights_on_mul_ir_rows(device, dtype, layouts, ir1, ir2, ir3, index
         for t in (p, q):
             err = (t.detach().cpu().double() - r).abs().max().item()
             assert err <= tol * r.abs().max().item(), (what, err)
+
+
+@pytest.mark.gpu
+def test_mul_ir_rows_without_batch_rows(device):
+    """No edges at all on the default layout: the output rows are zeros, the gradients have their shapes (the build's unit)."""
+    from cuequivariance_amd import cuet
+
+    i1, i2 = cue.Irreps("O3", "64x0e+64x1o"), cue.Irreps("O3", "0e+1o+2e")
+    m = cuet.FullyConnectedTensorProduct(i1, i2, i1, layout=cue.mul_ir, shared_weights=False, internal_weights=False)
+    x1 = torch.randn(5, i1.dim, device=device, requires_grad=True)
+    x2 = torch.randn(0, i2.dim, device=device, requires_grad=True)
+    w = torch.randn(0, m.weight_numel, device=device, requires_grad=True)
+    idx = torch.zeros(0, dtype=torch.int32, device=device)
+    out = m(x1, x2, w, indices_1=idx, indices_out=idx, size_out=5)
+    assert out.shape == (5, i1.dim) and float(out.detach().abs().sum()) == 0.0
+    g1, g2, gw = torch.autograd.grad(out, [x1, x2, w], torch.ones_like(out))
+    assert g1.shape == x1.shape and float(g1.abs().sum()) == 0.0 and g2.shape == x2.shape and gw.shape == w.shape
+    assert m.f_per_sample.f is None  # (the rows were taken as they lie)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("product,compiles,taken", [
+    (MUL_IR_ROWS[0], False, True), (MUL_IR_ROWS[0], True, True),
+    (("4x1o", "0e+1o", "12x0e+12x1o"), False, False),  # (not in the library: without compilation its rows are transposed)
+    (MUL_IR_ROWS[2], True, True),
+])
+def test_second_derivatives_on_mul_ir_rows(device, product, compiles, taken, dtype, jit_on, monkeypatch):
+    """Gradients of a function of the output and of its first gradients, against the oracle in float64 (float32: sums over 64 x 64 and
+    over 11 products of three random factors, 2e-5 of the largest value)."""
+    from cuequivariance_amd import _lib, cuet
+    from oracle.naive import naive_segmented_polynomial, spec_from_polynomial
+
+    monkeypatch.setattr(jit, "_enabled", compiles)
+    i1, i2, i3 = (cue.Irreps("O3", s) for s in product)
+    m = cuet.FullyConnectedTensorProduct(i1, i2, i3, layout=cue.mul_ir, shared_weights=False, internal_weights=False)
+    N, Z = 4, 9
+    g = torch.Generator().manual_seed(8)
+    r = lambda *s: torch.randn(*s, dtype=torch.float64, generator=g).to(dtype).double()
+    x1, x2, w, cot = r(N, i1.dim), r(Z, i2.dim), r(Z, m.weight_numel), r(N, i3.dim)
+    snd, rcv = (torch.randint(0, N, (Z,), generator=g, dtype=torch.int32) for _ in range(2))
+    inner = [r(*t.shape) for t in (w, x1, x2)]
+
+    def swapped(x, irreps, back):  # mul_ir rows as ir_mul rows, or back
+        parts, off = [], 0
+        for mul, ir in irreps:
+            shape = (-1, ir.dim, mul) if back else (-1, mul, ir.dim)
+            parts.append(x[:, off:off + mul * ir.dim].reshape(shape).transpose(1, 2).reshape(-1, mul * ir.dim))
+            off += mul * ir.dim
+        return torch.cat(parts, 1)
+
+    spec = spec_from_polynomial(descriptors.fully_connected_tensor_product(i1, i2, i3).polynomial)
+
+    def oracle(w, x1, x2):
+        return swapped(naive_segmented_polynomial(spec, [w, swapped(x1, i1, False), x2], {1: snd}, {0: N}, {0: rcv})[0], i3, True)
+
+    def ours(w, x1, x2):
+        return m(x1, x2, w, indices_1=snd.to(device), indices_out=rcv.to(device), size_out=N)
+
+    def step(f, args, c, inner):
+        args = [t.clone().requires_grad_() for t in args]
+        first = torch.autograd.grad(f(*args), args, c, create_graph=True)
+        return torch.autograd.grad(first, args, inner)
+
+    want = step(oracle, (w, x1, x2), cot, inner)
+    to = lambda t: t.to(dtype).to(device)
+    _lib.timing_begin()
+    got = step(ours, tuple(map(to, (w, x1, x2))), to(cot), list(map(to, inner)))
+    assert ("segmented_transpose" in _lib.timing_end()) == (not taken)
+    tol = 1e-12 if dtype == torch.float64 else 2e-5
+    for a, b in zip(got, want):
+        assert (a.cpu().double() - b).abs().max().item() <= tol * b.abs().max().item()
