@@ -23,8 +23,11 @@ from collections import OrderedDict
 
 MAX_WIDTH = 256   # output / input columns held in accumulators (8 tiles of 32)
 MAX_LDS = 150 * 1024
-# 16-byte vectors of a four-byte mul_ir block that a lane holds at a time.  50 000 rows of 64x0e+64x1o (x) 0e+1o+2e -> the same, float,
-# mul_ir rows, us whole / in pieces: forward 71 (96 registers spilled) / 64 (7), both input gradients 93 (101) / 70 (none).
+# 16-byte vectors of a four-byte mul_ir block that a lane holds at a time, where there is another group of products to request a piece
+# under.  50 000 rows, float, mul_ir rows, us of the module's calls (forward / both input gradients and the weights' / the first / the
+# second alone) whole and in pieces: 64x0e+64x1o (x) 0e+1o+2e -> the same 68.6 / 217 / 130 / 129 and 61.0 / 187 / 115 / 115; (x) 0e+1o
+# 48.6 / 162 / 89.0 / 93.9 and 49.4 / 154 / 90.9 / 87.9; one group, 64x1o (x) 0e+1o+2e -> 64x0e+64x1o, whose two pieces fill both register
+# sets: 52.0 / 159 / 87.6 / 99.8 and 54.5 / 161 / 93.5 / 104 (so one group is requested whole, as far as two pieces go).
 PIECE = 12
 
 
@@ -217,7 +220,7 @@ def _operand_groups(A, prods, transposed: bool, in_blocks, es: int, single: bool
     whole, parts = [], []
     for blk, members in groups:
         ns, per = contraction[members[0][0]] * es // 64, 2 * (blk[2] if blk else 1)
-        step = max(1, PIECE // per) if blk and es == 4 else ns
+        step = max(1, PIECE // per) if blk and es == 4 and (len(groups) > 1 or ns * per > 2 * PIECE) else ns
         pieces = [(blk, members, s, min(ns, s + step)) for s in range(0, ns, step)]
         (whole if len(pieces) == 1 else parts).extend(pieces)
     order = []
@@ -368,8 +371,7 @@ def _emit_kernel(A, name: str, T: str, paths, transposed: bool, rowdot: bool, wi
                         else:
                             A(f"        {{ const float sc = {coeff!r}f * s{j};")
                             A("#pragma unroll")
-                            A(f"          for (int v = 0; v < 16; ++v) o{res_off // 32 + t}[v] = fmaf(sc, T[v], o{res_off // 32 + t}[v]);")
-                            A(f'          asm volatile("" : "+v"(o{res_off // 32 + t})); }}')
+                            A(f"          for (int v = 0; v < 16; ++v) o{res_off // 32 + t}[v] = fmaf(sc, T[v], o{res_off // 32 + t}[v]); }}")
                     A("      }")
                     A("      __builtin_amdgcn_sched_barrier(0);  // keep the loads of later products from piling up ahead of this one")
             A("    }")

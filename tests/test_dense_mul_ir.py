@@ -189,7 +189,9 @@ def test_fully_connected_mul_ir_matches_oracle_without_transposition(device, ker
     "irreps_in1,irreps_in2,irreps_out",
     [
         ("64x0e+64x1o", "0e+1o+2e", "64x0e+64x1o"),  # pieces of one block around the other block
-        ("64x1o", "0e+1o+2e", "64x1o"),  # pieces of one block next to each other
+        ("64x1o", "0e+1o+2e", "64x1o"),  # one block, whole
+        ("32x3o", "0e+2e", "32x1o"),  # one block that two pieces do not hold
+        ("32x1o+32x2e", "0e+1o", "32x1o+32x2e"),  # two blocks, whole pieces apart from each other
         ("32x0e+32x2e", "0e+2e", "64x0e+32x2e"),  # pieces of one slice of channels
     ],
 )

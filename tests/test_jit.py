@@ -386,3 +386,20 @@ def test_scalar_output_mixing_contracting_and_scalar_paths(device, jit_on, on):
     got = run_plan(plan, [B] * 5, [-1] * 5, Z, 0, [v.to(device) for v in (x, gy, sc, gt)])[0]
     assert plan.specialised(device) == on
     assert (got.cpu() - want).abs().max().item() <= 1e-12 * want.abs().max().item()
+
+
+def test_a_mul_ir_block_is_requested_in_pieces_where_there_is_another():
+    """A piece leaves room for another group of products to be requested under; the kernels of one block ask for it whole."""
+    from cuequivariance_amd import cuet
+    from cuequivariance_amd.codegen import fullyconnected as fc
+
+    def forward(i1, i2, i3):
+        i1, i2, i3 = (cue.Irreps("O3", s) for s in (i1, i2, i3))
+        m = cuet.FullyConnectedTensorProduct(i1, i2, i3, layout=cue.mul_ir, internal_weights=False)
+        dense = next(x for x in m.modules() if type(x).__name__ == "SegmentedPolynomialDense" and x.rows_mul_ir)
+        text = fc.emit_unit(dense.paths, dense.input_sizes[2], dense.input_sizes[1], dense.out_size, "float", *dense.fc_blocks)
+        return text.split("fwd_kernel(")[1].split("__global__")[0]
+
+    assert "uint4 rawa[24]" in forward("64x1o", "0e+1o+2e", "64x0e+64x1o")
+    assert "uint4 rawa[12], rawb[8]" in forward("64x0e+64x1o", "0e+1o+2e", "64x0e+64x1o")
+    assert "uint4 rawa[14], rawb[14]" in forward("32x3o", "0e+2e", "32x1o")
