@@ -3911,8 +3911,7 @@ extern "C" int cueq_ln_dual_gate(int32_t dtype, int64_t C, int64_t M, int64_t K,
   return launch_dual_gate_res(C, M, K, W1, W2, ldw, X, nullptr, ldx, bias1, bias2, mask, out, ldc, gamma, beta, static_cast<float>(eps), xhat, ldxh, mean, rstd, dtype == CUEQ_F16, stream);
 }
 
-// ln_x != NULL: the LayerNorm backward in the same kernel (cueq_gate_bwd_input_ln)
-// the LayerNorm across d (its weight may be null) that a two-input call with C = K goes on through; the gradients of its weight and
+// The LayerNorm across d (its weight may be null) that a two-input call with C = K goes on through; the gradients of its weight and
 // bias, where wanted, in float32 through partial sums of a block ([2][(M + 63) / 64 or as many as there are compute units][K])
 struct GateNorm {
   const void* x;
@@ -3922,12 +3921,14 @@ struct GateNorm {
   float *dgamma, *dbeta, *part;
 };
 
-// gradients of the weight and bias of the LayerNorm that a one-input call goes on through (either may be null), in float32, and room
+// Gradients of the weight and bias of the LayerNorm that a one-input call goes on through (either may be null), in float32, and room
 // for a block's partial sums ([2][ln_bwd_blocks or fewer][K])
 struct LnSums {
   float *dgamma, *dbeta, *part;
 };
 
+// ln_x != NULL: the LayerNorm backward in the same kernel (cueq_gate_bwd_input_ln).  norm != NULL: that across d in the two-input one, which
+// takes the place of dX2.
 static int gate_bwd_input_impl(int32_t dtype, int64_t C, int64_t M, int64_t K, const void* W1, const void* W2, int64_t ldw,
                                const void* X1, const void* X2, int64_t ldx,
                                const void* bias1, const void* bias2, const void* mask, const void* dC, int64_t ldc,
@@ -3946,7 +3947,7 @@ static int gate_bwd_input_impl(int32_t dtype, int64_t C, int64_t M, int64_t K, c
   if (ln_x && !dres) dres = dX1;  // (in place)
   const bool bf = dtype != CUEQ_F32, half = dtype == CUEQ_F16;
   const bool split = X2 != nullptr && X2 != X1;
-  CUEQ_REQUIRE(!split || dX2, CUEQ_ERR_INVALID, "gate_bwd_input: two inputs need two gradients");
+  CUEQ_REQUIRE(!split || dX2 || norm, CUEQ_ERR_INVALID, "gate_bwd_input: two inputs need two gradients");
   CUEQ_REQUIRE(!(split && accumulate), CUEQ_ERR_UNSUPPORTED, "gate_bwd_input: accumulate needs a single input");
   const int epv = bf ? 8 : 4;
   const uintptr_t ptrs = reinterpret_cast<uintptr_t>(W1) | reinterpret_cast<uintptr_t>(W2) | reinterpret_cast<uintptr_t>(X1) | reinterpret_cast<uintptr_t>(X2) |
@@ -4515,7 +4516,7 @@ enum { kNinW, kNinB, kPinW, kPinB, kGinW, kGinB, kNoutW, kNoutB, kPoutW, kPoutB,
 struct TriPlan {
   int32_t dt;
   int64_t B, N, Np, D, Do, M, es;
-  bool resident, mapped, copies;
+  bool resident, mapped, copies, norm_fused;
   PairRows pairs;
 
   TriPlan(int32_t dt_, int64_t B_, int64_t N_, int64_t D_, int64_t Do_, bool outgoing = true) : dt(dt_), B(B_), N(N_), D(D_), Do(Do_) {
@@ -4530,6 +4531,10 @@ struct TriPlan {
     mapped = Np != N && resident && (D == 64 || D == 128) && Do % 32 == 0 && dual_gate_res_lds(Do, D, false) <= 160 * 1024 && bwd_out <= 160 * 1024 &&
              bwd_in <= 160 * 1024 && (M * Do + 8) * es < (1ll << 32) && 6 * M * es < (1ll << 32);
     copies = Np != N && !mapped;
+    // the backward of the LayerNorm across d in the output stage's kernel, where the result is as wide as the input: the gradient of the
+    // norm's rows is not stored (bfloat16, 512 x 512 x 128: the two kernels 77 + 44 us, the one 108; 391 x 391 with all gradients 59 + 49
+    // and 78; down to 16 x 16 x 64 no size is slower, see the whole backward there: 28.0 and 21.3)
+    norm_fused = dt != CUEQ_F32 && Do == D && (D == 64 || D == 128) && (M * D + 8) * es < (1ll << 32) && 6 * M * es < (1ll << 32);
     if (Np != N && M < (1ll << 31)) pairs = PairRows::make(static_cast<int>(N), static_cast<int>(Np), !outgoing);
   }
 };
@@ -4588,7 +4593,7 @@ struct TriBwdWork {
     Carve c(buf);
     const int64_t rows = p.M * p.D * p.es;
     dxh = c.take(rows);
-    dy = c.take(rows);
+    dy = p.norm_fused ? nullptr : c.take(rows);
     dt = c.take(rows);
     dab = c.take(2 * rows);
     doutp = p.copies ? c.take(p.M * p.Do * p.es) : nullptr;
@@ -4757,12 +4762,9 @@ extern "C" int cueq_trimul_bwd_parts(int32_t dtype, int64_t B, int64_t N, int64_
   // output gate
   char *du2 = k.du2, *dv2 = k.du2 ? k.du2 + M * Do * es : nullptr;
   float *dgo = wants(kNoutW) ? g_nout : nullptr, *dbo = wants(kNoutB) ? g_nout + D : nullptr;
-  // and, where the result is as wide as the input, the LayerNorm across d in the same kernel (the gradient of its rows is not stored;
-  // 512 x 512 x 128, bfloat16: the two kernels 77 + 44 us, the one 108; 391 x 391 with all gradients 59 + 49 and 78)
-  const bool norm_fused = dtype != CUEQ_F32 && Do == D && (D == 64 || D == 128) && (M * D + 8) * es < (1ll << 32) && 6 * M * es < (1ll << 32);
-  if (norm_fused) {
+  if (p.norm_fused) {
     const GateNorm norm{s.t, s.mean2, s.rstd2, w[kNoutW], k.dt, dgo, dbo, reinterpret_cast<float*>(k.ln)};
-    TRI_STEP(gate_bwd_input_impl(dtype, Do, M, D, w[kGoutW], w[kPoutW], D, s.xh, s.y, D, w[kGoutB], w[kPoutB], nullptr, dout, Do, 0, k.dxh, k.dy, D, 0,
+    TRI_STEP(gate_bwd_input_impl(dtype, Do, M, D, w[kGoutW], w[kPoutW], D, s.xh, s.y, D, w[kGoutB], w[kPoutB], nullptr, dout, Do, 0, k.dxh, nullptr, D, 0,
                                  w_out ? du2 : nullptr, w_out ? dv2 : nullptr, nullptr, 0, nullptr, nullptr, nullptr, stream_, nullptr, pairs, &norm));
   } else if (D <= 128 && Do % 32 == 0) {
     TRI_STEP(gate_bwd_input_impl(dtype, Do, M, D, w[kGoutW], w[kPoutW], D, s.xh, s.y, D, w[kGoutB], w[kPoutB], nullptr, dout, Do, 0, k.dxh, k.dy, D, 0,
@@ -4793,7 +4795,7 @@ extern "C" int cueq_trimul_bwd_parts(int32_t dtype, int64_t B, int64_t N, int64_
   if (wants(kPoutB)) TRI_STEP(cueq_sum_rows(dtype, M, Do, dv2, g_out_b + Do, k.part, k.part_bytes, stream_));
 
   // LayerNorm across d
-  if (norm_fused) {
+  if (p.norm_fused) {
     // (done with the gate)
   } else if (D <= kLnTMaxD) {
     TRI_STEP(cueq_layer_norm_t_bwd(dtype, M, D, k.dy, s.t, s.mean2, s.rstd2, w[kNoutW], k.dt, dgo, dbo, k.ln, k.ln_bytes, stream_));

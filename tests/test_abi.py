@@ -127,3 +127,14 @@ def test_option_set_by_the_program_survives_the_environment_sync(monkeypatch):
     finally:
         lib.cueq_set_option(b"deterministic", 0)
         _lib._env_seen["CUEQ_DETERMINISTIC"] = None
+
+
+@pytest.mark.parametrize("n,B", [(512, 1), (391, 1), (24, 3)])
+def test_workspace_of_the_triangle_backward(n, B):
+    """Where the output stage goes on through its norm (2-byte types, as wide a result as the input, 64 or 128) the gradient of the norm's
+    rows takes no memory: those of dx_hat, dt, da and db are left, four of five, and partial sums."""
+    lib, np_ = _lib.load(), -(-n // 8) * 8
+    for D in (64, 128):
+        rows = B * np_ * np_ * D * 2
+        fused, apart = (lib.cueq_trimul_workspace_bytes(_lib.BF16, B, n, D, Do, 1, 0) for Do in (D, D - 32))
+        assert 4 * rows <= fused < 4.5 * rows < 5 * rows <= apart
