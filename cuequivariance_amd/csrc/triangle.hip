@@ -216,17 +216,19 @@ __device__ __forceinline__ void gemm_stage_offsets(int e, int& row, int& part) {
   else { row = e / (KB / 16); part = e % (KB / 16); }
 }
 
-// fragment of subtile rows [base, base + 32) for MFMA slice q of the step (KB / 32 slices): 16 bytes of k per lane
-template <typename TI, bool TR, int EXT, int KB = 64>
+// fragment of subtile rows [base, base + 32) for MFMA slice q of the step (KB / 32 slices): 16 bytes of k per lane.  SEQ (2-byte types): slice
+// q is the values 16 q .. 16 q + 15 of k, in the order of gemm_direct_kernel; else half a wavefront has one half of the step
+template <typename TI, bool TR, int EXT, int KB = 64, bool SEQ = false>
 __device__ __forceinline__ uint4 gemm_fragment(const char* tile, int base, int q, int lane) {
   constexpr int kTransStride16 = trans_stride<uint16_t, EXT>(), kTransStride32 = trans_stride<float, EXT>();
   constexpr int HK = KB / 2 / static_cast<int>(sizeof(TI));  // k rows of a contraction-major tile per half wavefront
+  static_assert(!SEQ || sizeof(TI) == 2, "");
   const int c = lane & 31, h = lane >> 5;
   if constexpr (!TR) {
-    return *reinterpret_cast<const uint4*>(tile + (base + c) * (KB + 16) + h * (KB / 2) + q * 16);
+    return *reinterpret_cast<const uint4*>(tile + (base + c) * (KB + 16) + (SEQ ? (2 * q + h) * 16 : h * (KB / 2) + q * 16));
   } else if constexpr (sizeof(TI) == 2) {
     const int s = lane & 15, g16 = (lane >> 4) & 1;
-    const char* p = tile + (HK * h + 8 * q + (s >> 2)) * kTransStride16 + (base + 16 * g16 + 4 * (s & 3)) * 2;  // k as in the other layout
+    const char* p = tile + ((SEQ ? 16 * q + 8 * h : HK * h + 8 * q) + (s >> 2)) * kTransStride16 + (base + 16 * g16 + 4 * (s & 3)) * 2;  // k as in the other layout
     typedef shortx4_t __attribute__((address_space(3))) * lptr;
     const shortx4_t r0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lptr)(p));
     const shortx4_t r1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lptr)(p + 4 * kTransStride16));
@@ -253,7 +255,8 @@ __device__ __forceinline__ uint4 gemm_fragment(const char* tile, int base, int q
 // where gemm_direct_kernel is the slower one (direct_tiles).  It would be slower for what is added to: what is added to is read in the middle of its row of steps, and each
 // such wait takes in the loads ahead (us, this kernel / that one with 256 x 256 tiles: added to, 128 products of 512 54.4 / 79.0, of 392
 // 43.6 / 55.6, 147 456 x 192 x 384 48.3 / 81.8, 4 of 2 056 x 2 056 x 128 21.7 / 40.9; rows of 513 elements, 128 of 512 58.6 / 107).
-template <typename TI, typename TO, bool TA, bool TB, int WM = 2, int WN = 2, int KB = 64, bool EDGE = false>
+// SEQ: sums in the order of gemm_direct_kernel, so that a 2-byte product has the same bits whichever kernel its batch or its rows take it to.
+template <typename TI, typename TO, bool TA, bool TB, int WM = 2, int WN = 2, int KB = 64, bool EDGE = false, bool SEQ = false>
 __global__ void __launch_bounds__(64 * WM * WN, (!EDGE ? 1 : TA && !TB && sizeof(TI) == 2 ? 3 : 4)) gemm_kernel(const TI* __restrict__ A, int64_t lda, int64_t sA,
                                                    const TI* __restrict__ B, int64_t ldb, int64_t sB,
                                                    TO* __restrict__ C, int64_t ldc, int64_t sC, int Mfull, int N, int Kfull,
@@ -372,8 +375,8 @@ __global__ void __launch_bounds__(64 * WM * WN, (!EDGE ? 1 : TA && !TB && sizeof
         for (int t = 0; t < 2; ++t)
 #pragma unroll
           for (int q = 0; q < NQ; ++q) {
-            if (t < NI) fa[t < NI ? t : 0][q] = gemm_fragment<TI, TA, TMR, KB>(&smem[buf][0], wm * 64 + t * 32, q, lane);
-            if (t < NJ) fb[t < NJ ? t : 0][q] = gemm_fragment<TI, TB, TNC, KB>(&smem[buf][ABYTES], wn * 64 + t * 32, q, lane);
+            if (t < NI) fa[t < NI ? t : 0][q] = gemm_fragment<TI, TA, TMR, KB, SEQ>(&smem[buf][0], wm * 64 + t * 32, q, lane);
+            if (t < NJ) fb[t < NJ ? t : 0][q] = gemm_fragment<TI, TB, TNC, KB, SEQ>(&smem[buf][ABYTES], wn * 64 + t * 32, q, lane);
           }
         // consecutive MFMAs go to different accumulators: a dependent one would wait for its predecessor to drain
 #pragma unroll
@@ -3650,9 +3653,10 @@ extern "C" int cueq_gemm(int32_t in_dtype, int32_t out_dtype, int32_t trans_a, i
 #define GEMM_LAUNCH(TI, TO, TA, TB) hipLaunchKernelGGL((gemm_kernel<TI, TO, TA, TB>), grid, dim3(256), 0, stream, GEMM_ARGS(TI, TO))
 #define GEMM_SZ(TI, TA, TB)                                                                                                                      \
   do {                                                                                                                                       \
-    if (big) hipLaunchKernelGGL((gemm_kernel<TI, TI, TA, TB, 4, 4, (sizeof(TI) == 2 ? 128 : 64)>), grid_big, dim3(1024), 0, stream, GEMM_ARGS(TI, TI)); \
-    else if (edge) hipLaunchKernelGGL((gemm_kernel<TI, TI, TA, TB, 2, 2, 64, true>), grid, dim3(256), 0, stream, GEMM_ARGS(TI, TI));          \
-    else GEMM_LAUNCH(TI, TI, TA, TB);                                                                                                        \
+    constexpr bool two = sizeof(TI) == 2;                                                                                                    \
+    if (big) hipLaunchKernelGGL((gemm_kernel<TI, TI, TA, TB, 4, 4, (two ? 128 : 64), false, two>), grid_big, dim3(1024), 0, stream, GEMM_ARGS(TI, TI)); \
+    else if (edge) hipLaunchKernelGGL((gemm_kernel<TI, TI, TA, TB, 2, 2, 64, true, two>), grid, dim3(256), 0, stream, GEMM_ARGS(TI, TI));    \
+    else hipLaunchKernelGGL((gemm_kernel<TI, TI, TA, TB, 2, 2, 64, false, two>), grid, dim3(256), 0, stream, GEMM_ARGS(TI, TI));             \
   } while (0)
 #define GEMM_TR(TI) do { if (trans_a && trans_b) GEMM_SZ(TI, true, true); else if (trans_a) GEMM_SZ(TI, true, false); else if (trans_b) GEMM_SZ(TI, false, true); else GEMM_SZ(TI, false, false); } while (0)
     if (in_dtype == CUEQ_F32 && out_dtype == CUEQ_F32) GEMM_TR(float);

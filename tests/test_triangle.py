@@ -281,6 +281,31 @@ def test_gemm_tn_two_byte_pieces(device, dtype, rows, parts, M, N):
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("trans_a,trans_b", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("M,N,K,batches", [(264, 264, 264, (1, 64, 160)), (32, 32, 32, (384, 640)), (512, 512, 200, (2, 128))])
+def test_two_byte_products_have_the_same_bits_on_every_kernel(device, dtype, trans_a, trans_b, M, N, K, batches):
+    """Which kernel a product runs on depends on how many there are and on where its rows go; its sums have one order."""
+    from cuequivariance_amd import _lib
+
+    g = torch.Generator(device=device).manual_seed(K)
+    A, B = (torch.randn(batches[-1], *(s[::-1] if t else s), generator=g, device=device).to(dtype) for s, t in (((M, K), trans_a), ((N, K), trans_b)))
+    lib, code = _lib.load(), {torch.bfloat16: _lib.BF16, torch.float16: _lib.F16}[dtype]
+    first, ran = None, set()
+    for batch in batches:
+        for ldc in (N, N + 1):
+            C = torch.zeros(batch, M, ldc, dtype=dtype, device=device)
+            _lib.timing_begin()
+            _lib.check(lib.cueq_gemm(code, code, int(trans_a), int(trans_b), M, N, K, A.data_ptr(), A.stride(1), A.stride(0), B.data_ptr(), B.stride(1),
+                                     B.stride(0), C.data_ptr(), ldc, M * ldc, batch, 1.0, 0, torch.cuda.current_stream().cuda_stream), "cueq_gemm")
+            ran |= set(_lib.timing_end())
+            got = C[:batches[0], :, :N].contiguous()
+            first = got if first is None else first
+            assert torch.equal(got, first), (batch, ldc, ran)
+    assert len(ran) >= 2
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("trans_a,trans_b", [(False, False), (False, True), (True, False), (True, True)])
 @pytest.mark.parametrize("batch,M,N,K,pad,shift", [(3, 200, 136, 72, 1, 0), (2, 72, 40, 8, 0, 1), (300, 136, 144, 40, 0, 0), (300, 144, 136, 136, 3, 1),
                                                    (70, 264, 392, 64, 8, 0), (70, 264, 392, 96, 2, 0), (1, 512, 48, 1024, 0, 0), (130, 512, 512, 72, 0, 0),
                                                    (130, 512, 512, 64, 1, 0)])
@@ -405,7 +430,7 @@ def test_defaults_shapes_and_errors(device):
 def test_output_gate_normalises_across_d(device, dtype, Bsz, N, D, Do):
     """From 4 096 rows on the norm across d runs in the output gate: the least number, tiles of padded squares, results narrower than the
     input (with weight rows over several blocks), more tiles than wavefronts; what it keeps for the backward through the gradients."""
-    from cuequivariance_amd import cuet
+    from cuequivariance_amd import _lib, cuet
 
     p, cot = make_case(Bsz, N, D, dtype, 1, Do=Do)
     names = ["x", "norm_out_weight", "p_out_weight"]
@@ -413,9 +438,37 @@ def test_output_gate_normalises_across_d(device, dtype, Bsz, N, D, Do):
     ref = oracle_trimul(direction="outgoing", **pr)
     want = [ref, *torch.autograd.grad(ref, [pr[k] for k in names], cot.to(device))]
     pg = {k: v.detach().to(dtype).to(device).requires_grad_(k in names) for k, v in p.items()}
+    _lib.timing_begin()
     out = cuet.triangle_multiplicative_update(direction="outgoing", **pg)
-    for k, got, w in zip(["out", *names], [out, *torch.autograd.grad(out, [pg[k] for k in names], cot.to(dtype).to(device))], want):
+    forward = _lib.timing_end()
+    assert "dual_gate_fwd" in forward and "layer_norm_t_fwd" not in forward, forward
+    _lib.timing_begin()
+    grads = torch.autograd.grad(out, [pg[k] for k in names], cot.to(dtype).to(device))
+    backward = _lib.timing_end()
+    assert ("layer_norm_t_bwd" in backward) == (Do != D) and "layer_norm_bwd" not in backward, backward
+    for k, got, w in zip(["out", *names], [out, *grads], want):
         assert got.shape == w.shape and rel_err(got, w.detach().cpu()) <= TOL[dtype], (k, rel_err(got, w.detach().cpu()))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("N,alone,together", [(40, 2, 3), (32, 3, 5)])
+def test_a_batch_above_4096_rows_gives_the_bits_of_one_below(device, D, N, alone, together):
+    """Below 4 096 rows the norm across d has a kernel of its own (``layer_norm_t_fwd``), from there on the output gate forms it: sums in
+    one order, so the items of a batch in bfloat16 do not depend on how many there are.  (In half the two gate kernels round apart.)"""
+    from cuequivariance_amd import _lib, cuet
+
+    dtype = torch.bfloat16
+    p, _ = make_case(together, N, D, dtype, 5)
+    pg = {k: v.to(dtype).to(device) for k, v in p.items()}
+    assert alone * N * N < 4096 <= together * N * N
+    outs = []
+    for n in (alone, together):
+        part = dict(pg, x=pg["x"][:n].contiguous(), mask=pg["mask"][:n].contiguous())
+        _lib.timing_begin()
+        outs.append(cuet.triangle_multiplicative_update(direction="outgoing", **part))
+        assert ("layer_norm_t_fwd" in _lib.timing_end()) == (n == alone)
+    assert torch.equal(outs[0], outs[1][:alone])
 
 
 @pytest.mark.gpu
@@ -425,7 +478,7 @@ def test_output_gate_normalises_across_d(device, dtype, Bsz, N, D, Do):
 def test_backward_stages_go_on_through_their_norms(device, dtype, wanted, Bsz, N, D):
     """D = 64 / 128 in 2-byte types: one tile of 32 rows of which some are padding, whole ones, and more tiles than wavefronts (264 x 264
     rows are 2 178 for 2 048); with and without the sums for a norm's weight and bias and the gate gradients."""
-    from cuequivariance_amd import cuet
+    from cuequivariance_amd import _lib, cuet
 
     p, cot = make_case(Bsz, N, D, dtype, 1)
     names = ["x", *wanted]
@@ -433,7 +486,12 @@ def test_backward_stages_go_on_through_their_norms(device, dtype, wanted, Bsz, N
     ref = torch.autograd.grad(oracle_trimul(direction="incoming", **pr), [pr[k] for k in names], cot.to(device))
     pg = {k: v.detach().to(dtype).to(device).requires_grad_(k in names) for k, v in p.items()}
     out = cuet.triangle_multiplicative_update(direction="incoming", **pg)
-    for k, got, want in zip(names, torch.autograd.grad(out, [pg[k] for k in names], cot.to(dtype).to(device)), ref):
+    _lib.timing_begin()
+    grads = torch.autograd.grad(out, [pg[k] for k in names], cot.to(dtype).to(device))
+    ran = _lib.timing_end()
+    # (96 wide: the norm across d has a kernel of its own)
+    assert ("layer_norm_t_bwd" in ran) == (D == 96) and "gate_bwd_input_ln" in ran and "layer_norm_bwd" not in ran, ran
+    for k, got, want in zip(names, grads, ref):
         assert got.shape == want.shape and rel_err(got, want.cpu()) <= TOL[dtype], (k, rel_err(got, want.cpu()))
 
 
