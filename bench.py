@@ -352,10 +352,10 @@ def secondary(torch, cue, cuet, _lib, dev, wl: str, dtype_name, steps: int, warm
         desc = "configs[4]: triangle multiplicative update, outgoing, z [1,512,512,128], mask Bernoulli(0.9), fwd + bwd w.r.t. z"
         # What the stages of this decomposition move at the least (the normalised input, a, b, t, y and their cotangents live
         # in HBM between the launches): per pair row and channel, in elements - forward: x read, x-hat written, a|b (2)
-        # written and read, t written and read, y written, x-hat and y read, out written = 12; backward: dout, x-hat, y read,
-        # dx-hat and dy written, dy and t read, dt written, dt read twice with a and b, da|db (2) written and read, x and
-        # x-hat and dx-hat read, dx written = 20.
-        extra = {"decomposition_traffic_bytes": (12 + 20) * n * n * D * es}
+        # written and read, t written and read, y written, x-hat read, out written = 11; backward: dout, x-hat, y and t read,
+        # dx-hat and dt written, dt read twice with a and b, da|db (2) written and read, x and x-hat and dx-hat read, dx
+        # written = 18.  In float32 the norm across d has launches of its own: y is read again, dy written and read, 12 and 20.
+        extra = {"decomposition_traffic_bytes": (11 + 18 if es == 2 else 12 + 20) * n * n * D * es}
     else:
         raise ValueError(wl)
     if graph:
