@@ -3563,7 +3563,7 @@ static int gemm_direct(Direct tiles, bool ta, bool tb, int64_t M, int64_t N, int
 // 128 x 128 float32 partial products of a long contraction (chunks x parts of them), B contraction-major: bound by the operands' bytes,
 // which are read once.  One block on a CU with 64 KB in flight and half as many partial results (us, 512 x 128 over 153 664 / 262 144
 // columns, A by rows: this 35 / 67, two blocks a CU of 64 bytes a step and four buffers 37 / 78, three 36 / 79), or two of them where
-// the number of pieces is given (PieceShape: 128 x 128 x 9 parts over 200 000 rows 171, gemm_kernel 174; 64 x 64 x 16 over 150 000 126 / 148).
+// the number of pieces is given (PieceShape: 64 x 64 x 16 parts over 150 000 rows 126, gemm_kernel 148; cueq_gemm_tn has the rule).
 using DirectLong = DirectShape<2, 2, 2, 2, 128, 3, 0, 1>;
 using PieceShape = DirectShape<2, 2, 2, 2, 64, 3, 0, 2>;
 template <typename F, bool TA, typename Shape>
@@ -4140,7 +4140,10 @@ extern "C" int cueq_gemm_tn(int32_t in_dtype, int64_t M, int64_t N, int64_t rows
   if (in_dtype != CUEQ_F32 && vec && rows > 0) {
     // 2-byte inputs: MFMA on contraction-major tiles (transposing LDS reads); batch items = (row chunk, part)
     const int64_t rpc32 = (((rows + chunks - 1) / chunks + 31) / 32) * 32;
-    // (whole 128 x 128 results: the other kernel, 163 us / 172 inside a step of the 200 000 rows above)
+    // (results of whole 128 x 128 tiles stay with gemm_kernel.  Over many rows both are bound by the rows' bytes, and which one is ahead
+    // changes with the shape and with where the operands lie, by 8 % either way; us, direct / gemm_kernel, rows x parts: 128 x 128 50 001 x 9
+    // 47.3 / 45.2, 100 000 x 16 163 / 154, 200 000 x 2 47.1 / 48.0; 384 x 128 12 501 x 9 41.7 / 39.5; 512 x 512 200 000 x 1 225 / 251.  Operands of a
+    // few MB would gain: 5 003 x 9 of 128 x 128 10.8 / 12.3)
     if ((M % kTile || N % kTile) && 64 * lda < (int64_t(1) << 31) && 64 * ldb < (int64_t(1) << 31)) {
       const DirectParts parts{rows, stride_a, stride_b, chunks * M * N, nparts};
 #define TND(F) gemm_direct_long<F, true, PieceShape>(M, N, rpc32, A, lda, rpc32 * lda, B, ldb, rpc32 * ldb, partials, M * N, chunks, parts, static_cast<float>(alpha), stream)

@@ -259,7 +259,7 @@ def test_gemm_two_byte_tiles(device, dtype, trans_a, trans_b, batch, M, N, K):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("rows,parts,M,N", [(1, 1, 8, 8), (40, 3, 64, 32), (65, 2, 136, 40), (5000, 16, 32, 64), (20_011, 9, 64, 96), (4097, 1, 128, 128)])
+@pytest.mark.parametrize("rows,parts,M,N", [(1, 1, 8, 8), (40, 3, 64, 32), (65, 2, 136, 40), (5000, 16, 32, 64), (20_011, 9, 64, 96), (4097, 1, 128, 128), (3001, 2, 256, 384)])
 def test_gemm_tn_two_byte_pieces(device, dtype, rows, parts, M, N):
     """The pieces of long 2-byte contractions, those without rows among them, against float64: float32 sums of exact products."""
     from cuequivariance_amd import _lib
