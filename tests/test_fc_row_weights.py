@@ -335,13 +335,13 @@ def test_mul_ir_rows_without_batch_rows(device):
     (("4x1o", "0e+1o", "12x0e+12x1o"), False, False),  # (not in the library: without compilation its rows are transposed)
     (MUL_IR_ROWS[2], True, True),
 ])
-def test_second_derivatives_on_mul_ir_rows(device, product, compiles, taken, dtype, jit_on, monkeypatch):
+def test_second_derivatives_on_mul_ir_rows(device, product, compiles, taken, dtype, jit_on):
     """Gradients of a function of the output and of its first gradients, against the oracle in float64 (float32: sums over 64 x 64 and
     over 11 products of three random factors, 2e-5 of the largest value)."""
     from cuequivariance_amd import _lib, cuet
     from oracle.naive import naive_segmented_polynomial, spec_from_polynomial
 
-    monkeypatch.setattr(jit, "_enabled", compiles)
+    jit.enable(compiles)  # (the fixture brings the previous state back)
     i1, i2, i3 = (cue.Irreps("O3", s) for s in product)
     m = cuet.FullyConnectedTensorProduct(i1, i2, i3, layout=cue.mul_ir, shared_weights=False, internal_weights=False)
     N, Z = 4, 9
