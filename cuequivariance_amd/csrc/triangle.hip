@@ -3989,8 +3989,8 @@ static int gate_bwd_input_impl(int32_t dtype, int64_t C, int64_t M, int64_t K, c
     const bool pairs_ok = !dc_by_row || (M % 2 == 0 && ldc % 2 == 0 && reinterpret_cast<uintptr_t>(dC) % 4 == 0 && (5 * ldc + M) * es < (1ll << 32));
     if (lds <= 160 * 1024 && pairs_ok) {
       const int64_t ntiles = (M + 31) / 32;
-      // (as many weight rows as columns: two wavefronts to a SIMD, 77 us where one takes 111; the gate gradients of more rows than columns
-      // would not stay in the registers)
+      // (as many weight rows as columns: two wavefronts to a SIMD, 262 144 rows of 32 / 64 / 96 / 128 14 / 31 / 48 / 75 us where one takes 21 / 38 /
+      // 63 / 99, 64 rows 7.9 / 8.0 / 7.9 / 8.1 and 8.3 / 8.1 / 8.8 / 11.0; the gate gradients of more rows than columns would not stay in the registers)
       if (split && C == K) {
         const size_t two = static_cast<size_t>(2 * C * (K == 128 ? 2 * K : 2 * K + 16) + 8 * C + 8 * 32 * (2 * K + 16) + 4 * K);
         const int64_t gt = std::min<int64_t>(norm ? (ntiles + 1) / 2 : ntiles, device_cus());

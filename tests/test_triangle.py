@@ -212,12 +212,12 @@ def two_byte_kernel(dtype, by_rows, M, N, K, batch, plain=True):
 @pytest.mark.parametrize(
     "batch,M,N,K",
     [
-        (700, 72, 40, 8),  # more 128 x 128 tiles than stay on the chip, one step each
+        (700, 72, 40, 8),  # a poorly filled second round of 128 x 128 tiles, one step each
         (1, 8, 8, 24),  # the smallest
         (3, 200, 136, 1000),  # tiles cut unevenly, the last step a quarter full
-        (300, 264, 136, 40),  # 256 x 256 tiles, two a matrix and more than one a compute unit, partly filled ones between whole ones
+        (300, 264, 136, 40),  # the same of 256 x 256 tiles, two a matrix, partly filled ones between whole ones
         (130, 392, 520, 104),
-        (1000, 72, 40, 104),  # the same where loads go straight into LDS: rounds of tiles that are well filled (on 256 compute units)
+        (1000, 72, 40, 104),  # well filled rounds (on 256 compute units): loads straight into LDS, more tiles than stay on the chip
         (252, 264, 136, 72),
         (252, 264, 136, 40),
         (168, 392, 520, 104),
